@@ -179,6 +179,12 @@ typedef struct mvit_gemm_args {
  * (merger), with the element-wise ops of :204, :256, :784, :791 fused as epilogues. */
 int mvit_gemm(const mvit_gemm_args* args, mvit_stream_t stream);
 
+/* Host-only: the split_k to ask for when C[out_rows, out_cols] is a weight gradient contracted over k tokens (bf16). */
+int mvit_gemm_wgrad_split_k(int64_t out_rows, int64_t out_cols, int64_t k);
+/* Host-only: 1 when a bf16 MVIT_EPI_SWIGLU_BWD product of this shape is fastest on the kernel that can hand back column sums
+ * of C, 0 when it is faster without a workspace (mvit_colsum then takes the sums). */
+int mvit_gemm_swiglu_bwd_sums_columns(int64_t M, int64_t N, int64_t K);
+
 /* ---------------------------------------------------------------- varlen attention */
 
 /* Per segment [cu[i], cu[i+1]) and head: O = softmax(Q K^T * scale) V, non-causal, fp32 softmax;

@@ -51,7 +51,7 @@ BwdWorkspace plan_bwd_workspace(const mvit_block_args* a, void* base) {
   const int64_t S = a->S, C = a->C, I = a->I, Ipad = a->Ipad;
   Bump b{static_cast<char*>(base), 0, 0};
   BwdWorkspace w;
-  w.colsum = static_cast<float*>(b.take(64 * 3 * C * 4));
+  w.colsum = static_cast<float*>(b.take(64 * (3 * C > 2 * Ipad ? 3 * C : 2 * Ipad) * 4));
   w.swiglu_cols = static_cast<float*>(b.take((S + 255) / 256 * 2 * Ipad * 4));
   w.rms = static_cast<float*>(b.take((int64_t)RMS_PARTIALS * C * 4));
   w.delta_elems = mvit_attn_bwd_delta_elems(a->max_seqlen, S, a->nheads, a->head_dim, a->dtype);
@@ -189,18 +189,24 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
     STEP(bias_grad(a->dx2, C, C, a->g_bdown, st));
     STEP(weight_grad(a->dx2, C, C, a->h, Ipad, I, a->g_wdown, a->split_k_down, st));
   }
-  {  // dgu = (dx2 . Wdown) through the SwiGLU derivative; per-tile column sums of dgu come back with it
+  // dgu = (dx2 . Wdown) through the SwiGLU derivative.  With many rows the per-tile column sums of dgu come back with it;
+  // with few the product runs on smaller tiles and the sums are taken beside the chain
+  const bool fused_cols = dt != MVIT_BF16 || mvit_gemm_swiglu_bwd_sums_columns(S, Ipad, C);
+  {
     mvit_gemm_args g = gemm_args(dt, dt);
     g.trans_b = 1; g.epilogue = MVIT_EPI_SWIGLU_BWD;
     g.M = S; g.N = Ipad; g.K = C;
     g.A = a->dx2; g.lda = C; g.B = a->wdown; g.ldb = Ipad; g.C = a->dgu; g.ldc = 2 * Ipad; g.R = a->gu; g.ldr = 2 * Ipad; g.aux_off = Ipad;
-    g.workspace = w.swiglu_cols; g.workspace_bytes = (S + 255) / 256 * 2 * Ipad * 4;
+    if (fused_cols) {
+      g.workspace = w.swiglu_cols; g.workspace_bytes = (S + 255) / 256 * 2 * Ipad * 4;
+    }
     STEP(mvit_gemm(&g, stream));
   }
   {
     mvit_stream_t st = fork(1);
     if (!st && two) return MVIT_ERR_LAUNCH;
-    STEP(mvit_reduce_partials(w.swiglu_cols, (int)((S + 255) / 256), 2 * Ipad, a->g_bgu, gdt, st));
+    if (fused_cols) STEP(mvit_reduce_partials(w.swiglu_cols, (int)((S + 255) / 256), 2 * Ipad, a->g_bgu, gdt, st));
+    else STEP(bias_grad(a->dgu, 2 * Ipad, 2 * Ipad, a->g_bgu, st));
     STEP(weight_grad(a->dgu, 2 * Ipad, 2 * Ipad, a->n2, C, C, a->g_wgu, a->split_k_gate_up, st));
   }
   {  // dn2 = dgu . Wgu

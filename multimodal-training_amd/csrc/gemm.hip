@@ -1,8 +1,11 @@
 // MFMA GEMM for gfx950 with fused epilogues:  C[M,N] = epi( sum_k A[m,k] * B[n,k] ).
 //
 // Main loops:
-//   bf16: 256x256 tile, 8 waves of 128x64 (4x2 MFMA 32x32x16 tiles each), BK = 32, four LDS stages filled by direct
-//      global -> LDS loads (see gemm_dl_kernel).
+//   bf16, the products of the vision tower: gemm_pp_kernel (gemm_pingpong.hip) and, where its 256x256 tiles are too few,
+//      gemm_small_kernel (gemm_small.hip); choose_tile() below picks.
+//   bf16, the rest (SwiGLU backward of many rows, patch embedding from frames, fp32 outputs, accumulation): 256x256 tile, 8
+//      waves of 128x64 (4x2 MFMA 32x32x16 tiles each), BK = 32, four LDS stages filled by direct global -> LDS loads (see
+//      gemm_dl_kernel).
 //   fp32 (the parity path, v_mfma_f32_32x32x2_f32), and bf16 operands whose row pitch exceeds 2^22 elements (the
 //      direct loads use 32-bit lane offsets): 256x256 tile, 8 waves, BK = 64 (fp32: 16), global -> registers -> LDS,
 //      double-buffered LDS, one barrier per K step (gemm_kernel).
@@ -13,7 +16,7 @@
 // The epilogue stages the accumulators through LDS (fp32) so that bias / residual / activation inputs are
 // read and results written as 16-byte vectors along N.
 // Work-group ids are remapped so that the tiles a single XCD (one L2) works on are neighbours in N.
-#include "mvit_common.h"
+#include "gemm_common.h"
 #include <math.h>
 #include <stdlib.h>
 #include <string.h>
@@ -21,54 +24,6 @@
 
 namespace {
 
-
-struct GemmParams {
-  int64_t M, N, K;
-  const void* A;
-  int64_t lda;
-  const void* B;
-  const void* B2;
-  int64_t ldb;
-  const void* bias;
-  const void* bias2;
-  void* C;
-  int64_t ldc;
-  const void* R;
-  int64_t ldr;
-  void* aux;
-  int64_t ldaux;
-  int64_t aux_off;
-  int reduce_epi;  // split_k > 1: the epilogue that the reduction over the K slices applies (none, bias, bias + residual)
-  int tiles_m, tiles_n;
-  int split_k;        // K slices (1 = none)
-  int64_t k_chunk;    // K extent of one slice (multiple of BK)
-  float* workspace;   // [split_k][M][N] fp32 partial sums when split_k > 1
-  int vec_ok;         // every epilogue pointer / stride allows 16-byte accesses
-  float* colsum;      // SWIGLU_BWD: per-tile-row column sums of the output, [tiles_m][ldc] (null: not wanted)
-  int panel_w;        // tiles are walked in panels of this many tile columns (M fastest across a panel's rows)
-  // A operand made from decoded frames (gemm_dl_kernel<..., PIX = true>): image table and the affine form of the
-  // rescale / normalise step, value = byte * px_a[channel] + px_c[channel]
-  const mvit_image* px_images;
-  int px_n_images;
-  float px_a[3], px_c[3];
-};
-
-// Tile order inside one K slice: panels of panel_w tile columns; within a panel row by row.  Work-groups that run
-// at the same time on one XCD (consecutive tile indices) then cover a compact block of the output, e.g. 8 x 4
-// tiles, so the A and B panels they stream through that XCD's L2 are shared as widely as possible.
-__device__ __forceinline__ void tile_coords(const GemmParams& p, int tile, int& tm, int& tn) {
-  const int pw = p.panel_w;
-  const int full_panels = p.tiles_n / pw, per_panel = p.tiles_m * pw;
-  if (tile < full_panels * per_panel) {
-    const int r = tile % per_panel;
-    tm = r / pw;
-    tn = (tile / per_panel) * pw + r % pw;
-  } else {
-    const int r = tile - full_panels * per_panel, w = p.tiles_n - full_panels * pw;
-    tm = r / w;
-    tn = full_panels * pw + r % w;
-  }
-}
 
 template <typename T>
 struct Cfg;
@@ -91,71 +46,6 @@ template <>
 struct Waves<1> {  // 256x256 tile, 8 waves of 128x64, double-buffered LDS, one work-group per CU
   static constexpr int BM = 256, BN = 256, WM = 128, WN = 64, NTHREADS = 512, MIN_WAVES = 2;
 };
-
-__device__ __forceinline__ float gelu_erf(float z) { return 0.5f * z * (1.f + erff(z * 0.70710678118654752440f)); }
-__device__ __forceinline__ float gelu_erf_grad(float z) {
-  const float cdf = 0.5f * (1.f + erff(z * 0.70710678118654752440f));
-  const float pdf = 0.39894228040143267794f * __expf(-0.5f * z * z);
-  return cdf + z * pdf;
-}
-// 1 / (1 + e^-z) with the hardware reciprocal (1 ulp) instead of the IEEE division sequence
-__device__ __forceinline__ float sigmoidf_(float z) { return __builtin_amdgcn_rcpf(1.f + __expf(-z)); }
-
-// 8 consecutive elements <-> fp32 registers
-__device__ __forceinline__ void load8(const bf16_t* p, float* v) {
-  const bf16x8 x = *reinterpret_cast<const bf16x8*>(p);
-#pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = (float)x[e];
-}
-__device__ __forceinline__ void load8(const float* p, float* v) {
-  const f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    v[e] = a[e];
-    v[4 + e] = b[e];
-  }
-}
-template <typename T>
-__device__ __forceinline__ void unpack8(const T __attribute__((ext_vector_type(8))) & x, float* v) {
-#pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = (float)x[e];
-}
-// Epilogue outputs and per-element epilogue inputs are touched once per launch: they are stored / loaded with the
-// non-temporal hint, so that they do not push the operand panels of the tiles in flight out of the XCD's L2 (a round of
-// 32 output tiles is as large as that L2; with plain stores the main loop after an epilogue ran 18 % slower).
-typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void store8(bf16_t* p, const float* v) {
-  bf16x8 x;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] = (bf16_t)v[e];
-  __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, x), reinterpret_cast<u32x4_t*>(p));
-}
-__device__ __forceinline__ void store8(float* p, const float* v) {
-  __builtin_nontemporal_store(f32x4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f32x4*>(p));
-  __builtin_nontemporal_store(f32x4{v[4], v[5], v[6], v[7]}, reinterpret_cast<f32x4*>(p + 4));
-}
-// split-K partial tiles are read back by the reduction kernel right away: they stay cacheable
-__device__ __forceinline__ void store8_cached(float* p, const float* v) {
-  *reinterpret_cast<f32x4*>(p) = f32x4{v[0], v[1], v[2], v[3]};
-  *reinterpret_cast<f32x4*>(p + 4) = f32x4{v[4], v[5], v[6], v[7]};
-}
-template <typename T>
-__device__ __forceinline__ T __attribute__((ext_vector_type(8))) load8_stream(const void* p) {
-  typedef T raw8 __attribute__((ext_vector_type(8)));
-  if constexpr (sizeof(T) == 2) {
-    return __builtin_bit_cast(raw8, __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p)));
-  } else {
-    raw8 r;
-    const f32x4 a = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
-    const f32x4 b = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p) + 1);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      r[e] = a[e];
-      r[4 + e] = b[e];
-    }
-    return r;
-  }
-}
 
 // Stage one operand tile (ROWS rows of the output dimension x BK of the contraction) global -> registers -> LDS.
 // TR = false: memory is [row][k];  TR = true: memory is [k][row].
@@ -348,154 +238,6 @@ __device__ __forceinline__ float frag_f32(const float* lds, int row, int k) {
     return lds[(row + (l & 31)) * C::PITCH_K + k + (l >> 5)];
   else
     return lds[(k + (l >> 5)) * (ROWS + C::PAD_T) + row + (l & 31)];
-}
-
-// Epilogue on 8 consecutive output columns n..n+7 of row m.  v: accumulators (gate half for SWIGLU), u: up half.
-// FULL: all 8 columns exist and every pointer allows 16-byte accesses (compile-time trip counts, vector memory
-// operations); otherwise a scalar path bounded by the matrix edge.
-// PRE: the epilogue's per-element inputs (residual / saved activations) were fetched earlier into pre[0..1].
-// hb / hb2: the 8 bias values of columns n .. n+7, already in registers (null: loaded here)
-template <typename T, typename TO, int EPI, bool FULL, bool PRE = false>
-__device__ __forceinline__ void emit8_impl(const GemmParams& p, int64_t m, int64_t n, float* v, const float* u,
-                                           const T __attribute__((ext_vector_type(8))) * pre, float (&cs)[16], bool do_cs,
-                                           const float* hb = nullptr, const float* hb2 = nullptr) {
-  TO* Cp = static_cast<TO*>(p.C);
-  const T* Rp = static_cast<const T*>(p.R);
-  T* auxp = static_cast<T*>(p.aux);
-  const T* bias = static_cast<const T*>(p.bias);
-  const T* bias2 = static_cast<const T*>(p.bias2);
-  const int cnt = FULL ? 8 : ((p.N - n) < 8 ? (int)(p.N - n) : 8);
-  constexpr bool vec = FULL;
-
-  if constexpr (EPI == MVIT_EPI_BIAS || EPI == MVIT_EPI_BIAS_RES || EPI == MVIT_EPI_BIAS_GELU || EPI == MVIT_EPI_SWIGLU) {
-    if (hb) {
-      for (int e = 0; e < 8; ++e) v[e] += hb[e];
-    } else if (bias) {
-      float b[8];
-      if (vec) load8(bias + n, b);
-      else
-        for (int e = 0; e < cnt; ++e) b[e] = to_f32(bias[n + e]);
-      for (int e = 0; e < cnt; ++e) v[e] += b[e];
-    }
-  }
-  if constexpr (EPI == MVIT_EPI_SWIGLU) {
-    float uu[8], h[8];
-    for (int e = 0; e < 8; ++e) uu[e] = u[e];
-    if (hb2) {
-      for (int e = 0; e < 8; ++e) uu[e] += hb2[e];
-    } else if (bias2) {
-      float b[8];
-      if (vec) load8(bias2 + n, b);
-      else
-        for (int e = 0; e < cnt; ++e) b[e] = to_f32(bias2[n + e]);
-      for (int e = 0; e < cnt; ++e) uu[e] += b[e];
-    }
-    // round g and u to the storage type first: the backward recomputes from those stored values
-    for (int e = 0; e < 8; ++e) {
-      v[e] = to_f32(from_f32<T>(v[e]));
-      uu[e] = to_f32(from_f32<T>(uu[e]));
-      h[e] = v[e] * sigmoidf_(v[e]) * uu[e];
-    }
-    TO* h_out = Cp + m * p.ldc + n;
-    if (auxp) {  // a caller that will not differentiate passes no aux and gets the product alone
-      T* g_out = auxp + m * p.ldaux + n;
-      T* u_out = g_out + p.aux_off;
-      if (vec) {
-        store8(g_out, v);
-        store8(u_out, uu);
-      } else {
-        for (int e = 0; e < cnt; ++e) {
-          g_out[e] = from_f32<T>(v[e]);
-          u_out[e] = from_f32<T>(uu[e]);
-        }
-      }
-    }
-    if (vec) store8(h_out, h);
-    else
-      for (int e = 0; e < cnt; ++e) h_out[e] = from_f32<TO>(h[e]);
-    return;
-  }
-  if constexpr (EPI == MVIT_EPI_SWIGLU_BWD) {
-    const T* g_in = Rp + m * p.ldr + n;
-    const T* u_in = g_in + p.aux_off;
-    float g[8], uu[8], dg[8], du[8];
-    if (PRE) {
-      unpack8<T>(pre[0], g);
-      unpack8<T>(pre[1], uu);
-    } else if (vec) {
-      load8(g_in, g);
-      load8(u_in, uu);
-    } else {
-      for (int e = 0; e < 8; ++e) {
-        g[e] = e < cnt ? to_f32(g_in[e]) : 0.f;
-        uu[e] = e < cnt ? to_f32(u_in[e]) : 0.f;
-      }
-    }
-    for (int e = 0; e < 8; ++e) {
-      const float sg = sigmoidf_(g[e]);
-      const float silu = g[e] * sg;
-      dg[e] = v[e] * uu[e] * (sg + silu * (1.f - sg));
-      du[e] = v[e] * silu;
-    }
-    if (do_cs) {  // running column sums of this thread's 8 columns (the gate / up bias gradient)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        if (e < cnt) {
-          cs[e] += dg[e];
-          cs[8 + e] += du[e];
-        }
-      }
-    }
-    TO* dg_out = Cp + m * p.ldc + n;
-    TO* du_out = dg_out + p.aux_off;
-    if (vec) {
-      store8(dg_out, dg);
-      store8(du_out, du);
-    } else {
-      for (int e = 0; e < cnt; ++e) {
-        dg_out[e] = from_f32<TO>(dg[e]);
-        du_out[e] = from_f32<TO>(du[e]);
-      }
-    }
-    return;
-  }
-  if constexpr (EPI == MVIT_EPI_BIAS_RES || EPI == MVIT_EPI_GELU_BWD) {
-    float r[8];
-    if (PRE) unpack8<T>(pre[0], r);
-    else if (vec) load8(Rp + m * p.ldr + n, r);
-    else
-      for (int e = 0; e < 8; ++e) r[e] = e < cnt ? to_f32(Rp[m * p.ldr + n + e]) : 0.f;
-    for (int e = 0; e < 8; ++e) {
-      if constexpr (EPI == MVIT_EPI_BIAS_RES) v[e] += r[e];
-      else v[e] *= gelu_erf_grad(r[e]);
-    }
-  }
-  if constexpr (EPI == MVIT_EPI_BIAS_GELU) {
-    T* z_out = auxp + m * p.ldaux + n;
-    for (int e = 0; e < 8; ++e) v[e] = to_f32(from_f32<T>(v[e]));  // gelu of the stored pre-activation
-    if (vec) store8(z_out, v);
-    else
-      for (int e = 0; e < cnt; ++e) z_out[e] = from_f32<T>(v[e]);
-    for (int e = 0; e < 8; ++e) v[e] = gelu_erf(v[e]);
-  }
-  TO* c_out = Cp + m * p.ldc + n;
-  if constexpr (EPI == MVIT_EPI_ACCUM) {
-    float c[8];
-    if (vec) load8(c_out, c);
-    else
-      for (int e = 0; e < 8; ++e) c[e] = e < cnt ? to_f32(c_out[e]) : 0.f;
-    for (int e = 0; e < 8; ++e) v[e] += c[e];
-  }
-  if (vec) store8(c_out, v);
-  else
-    for (int e = 0; e < cnt; ++e) c_out[e] = from_f32<TO>(v[e]);
-}
-
-template <typename T, typename TO, int EPI>
-__device__ __forceinline__ void emit8(const GemmParams& p, int64_t m, int64_t n, float* v, const float* u, bool vec,
-                                      float (&cs)[16], bool do_cs) {
-  if (vec && n + 8 <= p.N) emit8_impl<T, TO, EPI, true>(p, m, n, v, u, nullptr, cs, do_cs);
-  else emit8_impl<T, TO, EPI, false>(p, m, n, v, u, nullptr, cs, do_cs);
 }
 
 // Per-element epilogue inputs (residual / saved activations) of an interior tile, fetched ahead of their use.
@@ -855,17 +597,12 @@ __global__ __launch_bounds__(Waves<VAR>::NTHREADS, Waves<VAR>::MIN_WAVES) void g
 // Rows past the matrix edge are clamped to valid rows (they only feed outputs that are never stored).  A partial
 // last K tile (K not a multiple of 32) is loaded through registers with zeros past the end of K.
 // The compiler does not see these loads: s_waitcnt vmcnt is placed by hand (loads return in order).
-// waves per work-group: 8 -> each owns 128x64 (two waves per SIMD), 4 -> 128x128 (one per SIMD).  BM_ = 128: an output
-// tile of half the height for products whose 256-row tiles would leave most compute units idle: the eight waves own
-// 64x64 each, the A stage holds 128 rows (in the first half of its 16 KiB slot), everything an output element sees
-// (K order, MFMA form, epilogue arithmetic) is unchanged, so results are bit-identical to the 256-row tile's.
-template <int NW, int BM_ = 256>
+// waves per work-group: 8 -> each owns 128x64 (two waves per SIMD), 4 -> 128x128 (one per SIMD).
+template <int NW>
 struct DL {
-  static_assert(BM_ == 256 || (BM_ == 128 && NW == 8), "tile heights built: 256, and 128 with eight waves");
-  static constexpr int BM = BM_, BN = 256, BK = 32, WM = BM_ / 2, WN = NW == 8 ? 64 : 128, NTHREADS = 64 * NW;
+  static constexpr int BM = 256, BN = 256, BK = 32, WM = 128, WN = NW == 8 ? 64 : 128, NTHREADS = 64 * NW;
   static constexpr int TILE_BYTES = 256 * BK * 2;
-  static constexpr int CPT = 16 / NW;          // 1 KiB load instructions per wave and K tile for a 256-row operand stage
-  static constexpr int CPT_A = BM_ / 16 / NW;  // ... for the A stage of this tile height
+  static constexpr int CPT = 16 / NW;  // 1 KiB load instructions per wave and K tile and operand
 };
 constexpr int DL_BK = 32, DL_TILE_BYTES = 256 * DL_BK * 2;
 
@@ -877,10 +614,9 @@ __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
 }
 
-template <bool TR, bool DUAL, int NW, bool MI16 = false, int ROWS = 256>
+template <bool TR, bool DUAL, int NW, bool MI16 = false>
 struct DlOperand {
-  static_assert(ROWS == 256 || !TR, "a [k][row] stage is always 256 rows wide");
-  static constexpr int CPT = ROWS / 16 / NW, WN = DL<NW>::WN;
+  static constexpr int CPT = DL<NW>::CPT, WN = DL<NW>::WN;
   unsigned voff[CPT];  // byte offset of this lane's 16-byte chunks from `base`
   const char* base;    // wave-uniform, advanced by `step` every K tile (DUAL: odd waves read the second matrix)
   int64_t step;
@@ -1066,13 +802,12 @@ __device__ __forceinline__ void wait_tiles(int n) {
 }
 
 // PIX: the A operand is made from decoded frames (DlPixelOperand)
-template <typename TO, bool TA, bool TB, int EPI, int NSTAGE, int NW, bool MI16 = false, bool PIX = false, int BM_ = 256>
+template <typename TO, bool TA, bool TB, int EPI, int NSTAGE, int NW, bool MI16 = false, bool PIX = false>
 __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_dl_kernel(const GemmParams p) {
   static_assert(!PIX || (!TA && !MI16 && !dl_prefetches(EPI, TA)), "frames as the A operand: [row][k] layout, 32x32x16 fragments, no early loads");
-  static_assert(BM_ == 256 || (!TA && !PIX && EPI != MVIT_EPI_SWIGLU_BWD), "half-height tiles: A in [row][k] layout, no per-256-row column sums");
   using T = bf16_t;
-  using D = DL<NW, BM_>;
-  constexpr int BM = D::BM, BN = D::BN, WM = D::WM, WN = D::WN, TILE = D::TILE_BYTES, SLICE = D::CPT * 1024, SLICE_A = D::CPT_A * 1024;
+  using D = DL<NW>;
+  constexpr int BM = D::BM, BN = D::BN, WM = D::WM, WN = D::WN, TILE = D::TILE_BYTES, SLICE = D::CPT * 1024;
   constexpr int MT = WM / 32, NT = WN / 32, WGN = BN / WN;
   constexpr bool DUAL = (EPI == MVIT_EPI_SWIGLU);
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -1087,8 +822,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_dl_kernel(const GemmPara
   ra.init(wm * WM, 0);
   rb.init(wn * WN, NSTAGE * TILE);
   typedef __attribute__((address_space(3))) unsigned char lds_byte;
-  const unsigned lds0 = (unsigned)(__UINTPTR_TYPE__)(lds_byte*)smem_raw + wv * SLICE;      // this wave's slice of a B stage
-  const unsigned lds0a = (unsigned)(__UINTPTR_TYPE__)(lds_byte*)smem_raw + wv * SLICE_A;   // ... of an A stage
+  const unsigned lds0 = (unsigned)(__UINTPTR_TYPE__)(lds_byte*)smem_raw + wv * SLICE;  // this wave's slice of a stage
 
   // Persistent work-groups: the grid has at most one work-group per CU; work-group (xcd, slot) walks that XCD's
   // tile range with stride slots-per-XCD, the order a one-tile-per-work-group grid would be dispatched in.
@@ -1098,7 +832,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_dl_kernel(const GemmPara
   constexpr bool PREFETCH = dl_prefetches(EPI, TA);
   constexpr int EARLY = PREFETCH ? (NSTAGE - 1 < 2 ? NSTAGE - 1 : 2) : NSTAGE - 1;  // K tiles requested by start_tile
   constexpr int STAGING_OFF = PREFETCH ? (NSTAGE + EARLY) * TILE : 0;
-  typename std::conditional<PIX, DlPixelOperand<NW>, DlOperand<TA, false, NW, MI16, BM>>::type la;
+  typename std::conditional<PIX, DlPixelOperand<NW>, DlOperand<TA, false, NW, MI16>>::type la;
   DlOperand<TB, DUAL, NW, MI16> lb;
   int T_ = 0, k_tail = 0;  // of the tile whose operands are being loaded
   [[maybe_unused]] int px_pending = -1;  // PIX: stage whose A bytes are in registers, requested by the previous issue()
@@ -1108,7 +842,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_dl_kernel(const GemmPara
     if constexpr (PIX) {
       // the A bytes requested one call ago are converted and written now (their K tile is read two barriers from here),
       // then K tile t is requested: B straight into LDS, A into registers
-      if (px_pending >= 0) la.flush(smem_raw + px_pending * TILE + wv * SLICE_A, px_norm);
+      if (px_pending >= 0) la.flush(smem_raw + px_pending * TILE + wv * SLICE, px_norm);
       px_pending = -1;
       if (t >= T_) return;
       lb.issue(lds0 + (NSTAGE + s) * TILE);
@@ -1117,10 +851,10 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_dl_kernel(const GemmPara
     } else {
       if (t >= T_) return;
       if (k_tail != 0 && t == T_ - 1) {
-        la.issue_tail(smem_raw + s * TILE + wv * SLICE_A, k_tail, wv);
+        la.issue_tail(smem_raw + s * TILE + wv * SLICE, k_tail, wv);
         lb.issue_tail(smem_raw + (NSTAGE + s) * TILE + wv * SLICE, k_tail, wv);
       } else {
-        la.issue(lds0a + s * TILE);
+        la.issue(lds0 + s * TILE);
         lb.issue(lds0 + (NSTAGE + s) * TILE);
       }
     }
@@ -1183,7 +917,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_dl_kernel(const GemmPara
       // tile t has landed once only the tiles issued after it are pending
       const int rem = T_ - 1 - t;
       constexpr int AHEAD = NSTAGE - 2;
-      wait_tiles<D::CPT_A + D::CPT>(rem < 0 ? 0 : (rem < AHEAD ? rem : AHEAD));
+      wait_tiles<2 * D::CPT>(rem < 0 ? 0 : (rem < AHEAD ? rem : AHEAD));
       __builtin_amdgcn_s_barrier();  // every wave's share of that tile is in LDS; stage (s-1) has been consumed
       // PIX: the conversion of the A bytes is vector work of about the length of a K tile's MFMAs.  The two waves of a
       // SIMD (w and w + NW/2) do it at opposite ends of the step, one before its MFMAs and one after, so that one
@@ -1350,16 +1084,16 @@ int device_cu_count(int dev) {
   return n_cu;
 }
 
-template <typename TO, bool TA, bool TB, int EPI, int NSTAGE, int NW, bool MI16 = false, bool PIX = false, int BM_ = 256>
+template <typename TO, bool TA, bool TB, int EPI, int NSTAGE, int NW, bool MI16 = false, bool PIX = false>
 int launch_dl(const GemmParams& p, hipStream_t stream) {
-  using D = DL<NW, BM_>;
+  using D = DL<NW>;
   constexpr size_t operands = 2 * (size_t)NSTAGE * D::TILE_BYTES;
   constexpr size_t staging = (size_t)(D::BM / D::WM) * 32 * D::BN * sizeof(float);
   // with prefetching the staging area starts behind the B stages that the next tile's first two K tiles arrive in
   constexpr size_t staging_end = dl_prefetches(EPI, TA) ? (NSTAGE + (NSTAGE - 1 < 2 ? NSTAGE - 1 : 2)) * D::TILE_BYTES + staging : staging;
   constexpr size_t lds = staging_end > operands ? staging_end : operands;
   static_assert(lds <= 160 * 1024, "operand stages plus the epilogue staging area exceed the LDS of a CU");
-  auto kern = gemm_dl_kernel<TO, TA, TB, EPI, NSTAGE, NW, MI16, PIX, BM_>;
+  auto kern = gemm_dl_kernel<TO, TA, TB, EPI, NSTAGE, NW, MI16, PIX>;
   static bool attr_set_on[MVIT_MAX_DEVICES] = {};  // once per kernel and device
   const int dev = mvit_current_device("gemm");
   if (dev < 0) return MVIT_ERR_LAUNCH;
@@ -1433,6 +1167,64 @@ int dispatch_trans(int ta, int tb, int epi, int var, const GemmParams& p, hipStr
 
 inline bool vec16(const void* ptr, int64_t ld, size_t esize) {
   return ptr == nullptr || (mvit_aligned16(ptr) && (ld * (int64_t)esize) % 16 == 0);
+}
+
+// ---- which bf16 kernel and tile
+GemmTiledKind tiled_kind(int dtype, int out_dtype, int ta, int tb, int epi, const GemmParams& p) {
+  if (dtype != MVIT_BF16) return TILED_NONE;
+  if (out_dtype != MVIT_BF16) return ta && tb && epi == MVIT_EPI_NONE ? TT_NONE_F32 : TILED_NONE;
+  const bool even = p.N % 2 == 0 && (reinterpret_cast<uintptr_t>(p.bias) | reinterpret_cast<uintptr_t>(p.bias2)) % 4 == 0;  // biases travel in pairs
+  if (!ta && !tb) {
+    switch (epi) {
+      case MVIT_EPI_NONE: return NN_NONE;
+      case MVIT_EPI_BIAS: return p.bias && even ? NN_BIAS : TILED_NONE;
+      case MVIT_EPI_BIAS_RES: return p.bias && even ? NN_BIAS_RES : TILED_NONE;
+      case MVIT_EPI_BIAS_GELU: return p.bias && even ? NN_BIAS_GELU : TILED_NONE;
+      case MVIT_EPI_SWIGLU: return p.bias && p.bias2 && even ? NN_SWIGLU : TILED_NONE;
+      default: return TILED_NONE;
+    }
+  }
+  if (!ta && tb) return epi == MVIT_EPI_NONE ? NT_NONE : (epi == MVIT_EPI_GELU_BWD ? NT_GELU_BWD : (epi == MVIT_EPI_SWIGLU_BWD ? NT_SWIGLU_BWD : TILED_NONE));
+  return ta && tb && epi == MVIT_EPI_NONE ? TT_NONE : TILED_NONE;
+}
+
+bool pp_takes(GemmTiledKind kind, int64_t k_chunk, int64_t k_last) {  // at least three K tiles of 64 in every slice
+  return kind != NT_SWIGLU_BWD && k_chunk > 128 && k_last > 128;
+}
+
+// Modelled times (us) of the tiles on one MI355X, measured at 64 ... 8,192 rows over the tower's products: a step of 64 along
+// K takes 1.2 us in a 256 x 256 tile (one work-group per compute unit; 1.35 with both operands behind the transposing LDS
+// read), and in the smaller ones `one` us while every unit has at most one work-group and `two` us once it has two.  A
+// fuller last round, a shorter step and more units at work all lower the estimate; the epilogue of a 256 x 256 tile is the
+// longest.  The line between the tiles follows from these numbers and not from any shape: e.g. 1280 columns, K = 3840 are
+// fastest on 64 x 64 up to 1,500 rows, on 64 x 128 to 2,600, on 128 x 128 to 6,500 and on 256 x 256 above (us at 256 / 1,040 /
+// 2,048 / 4,096 / 8,192 rows: 19 / 26 / 35 / 51 / 70, with 256 x 256 tiles alone 69 / 69 / 69 / 69 / 70).
+struct TileChoice {
+  int bm, bn;
+  double us;
+};
+TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk, int64_t k_last, int64_t slices, int n_cu) {
+  const bool tt = kind == TT_NONE || kind == TT_NONE_F32;
+  const double steps = (double)((k_chunk + 63) / 64);
+  const int64_t n_mul = kind == NN_SWIGLU ? 2 : 1;
+  TileChoice best{0, 0, 1e30};
+  auto consider = [&](int bm, int bn, double one, double two, double per_tile) {
+    const int64_t items = ((M + bm - 1) / bm) * ((N * n_mul + bn - 1) / bn) * slices;
+    const int64_t slots = two > 0. ? 2 * (int64_t)n_cu : n_cu, full = items / slots, rest = items % slots;
+    double us = 4. + full * (steps * (two > 0. ? two : one) + per_tile);
+    if (rest > 0) us += steps * (two > 0. && rest > n_cu ? two : one) + per_tile;
+    if (us < best.us) best = TileChoice{bm, bn, us};
+  };
+  if (pp_takes(kind, k_chunk, k_last)) consider(256, 256, tt ? 1.35 : 1.2, 0., kind == NN_SWIGLU ? 6. : 5.);
+  if (kind != NN_SWIGLU) consider(64, 64, 0.30, 0.43, 2.);
+  consider(64, 128, 0.46, 0.57, 2.);
+  if (kind != NT_SWIGLU_BWD) consider(128, 128, 0.64, tt ? 1.0 : 0.84, 2.5);
+  // SwiGLU backward of many rows: the 256-row kernel, which also sums the columns of its result
+  if (kind == NT_SWIGLU_BWD) {
+    const double tiles = (double)(((M + 255) / 256) * ((N + 255) / 256)), us = 4. + ceil(tiles / n_cu) * (steps * 1.6 + 16.);
+    if (us < best.us + (double)M * (double)N * 4. / 4e6) best = TileChoice{0, 0, us};
+  }
+  return best;
 }
 
 // packed[n][line * 48 + b] = w[n][channel * 392 + frame * 196 + y * 14 + x] for b = x * 3 + channel < 42, else 0
@@ -1546,6 +1338,7 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
   const size_t es = a->dtype == MVIT_BF16 ? 2 : 4, eo = a->out_dtype == MVIT_BF16 ? 2 : 4;
   p.vec_ok = vec16(a->C, a->ldc, eo) && vec16(a->R, a->ldr, es) && vec16(a->aux, a->ldaux, es) && vec16(a->bias, 0, es) &&
              vec16(a->bias2, 0, es) && (a->aux_off * (int64_t)(es < eo ? es : eo)) % 16 == 0;
+  p.half_vec_ok = a->ldc % 4 == 0 && reinterpret_cast<uintptr_t>(a->C) % 8 == 0;
   const int var = (a->lda > (1ll << 22) || a->ldb > (1ll << 22)) ? 1 : 3;  // 3: direct-to-LDS loads (32-bit lane offsets); 1: register-staged
   const int BM = 256, BN = 256;
   const int n_per_block = (epi == MVIT_EPI_SWIGLU) ? BN / 2 : BN;
@@ -1578,21 +1371,28 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
     }
   }
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  // Half-height tiles (128 x 256) for the two products that have few tile columns (N = hidden size): when the 256-row
-  // tiles would fill the last round of one-tile-per-unit work poorly and the 128-row tiles fill theirs better.  The
-  // result does not depend on the choice (same arithmetic per output element), so it may follow M.
-  if (a->dtype == MVIT_BF16 && a->out_dtype == MVIT_BF16 && var == 3 && !a->trans_a && p.split_k == 1 && getenv("MVIT_GEMM_NO_HALF_TILES") == nullptr &&
-      ((!a->trans_b && epi == MVIT_EPI_BIAS_RES) || (a->trans_b && epi == MVIT_EPI_NONE))) {
+  const GemmTiledKind kind = var == 3 ? tiled_kind(a->dtype, a->out_dtype, a->trans_a, a->trans_b, epi, p) : TILED_NONE;
+  if (kind != TILED_NONE) {
     const int dev = mvit_current_device("gemm");
     if (dev < 0) return MVIT_ERR_LAUNCH;
-    const double n_cu = device_cu_count(dev);
-    const int64_t tm_half = (a->M + 127) / 128;
-    const double r_full = (double)(tm * tn) / n_cu, r_half = (double)(tm_half * tn) / n_cu;
-    const double fill_full = r_full / ceil(r_full), fill_half = r_half / ceil(r_half);
-    if (fill_full < 0.75 && fill_half > fill_full + 0.1 && tm_half * tn < (1ll << 30)) {
-      p.tiles_m = (int)tm_half;
-      if (!a->trans_b) return launch_dl<bf16_t, false, false, MVIT_EPI_BIAS_RES, 4, 8, false, false, 128>(p, s);
-      return launch_dl<bf16_t, false, true, MVIT_EPI_NONE, 4, 8, true, false, 128>(p, s);
+    const int n_cu = device_cu_count(dev);
+    TileChoice c = choose_tile(kind, p.M, p.N, p.k_chunk, p.K - (p.split_k - 1) * p.k_chunk, p.split_k, n_cu);
+    if (getenv("MVIT_GEMM_NO_HALF_TILES") != nullptr && c.bm != 256 && pp_takes(kind, p.k_chunk, p.K - (p.split_k - 1) * p.k_chunk)) c = TileChoice{256, 256, 0.};
+    if (kind == NT_SWIGLU_BWD && p.colsum != nullptr) c.bm = 0;  // per-256-row column sums: the 256-row kernel makes them
+    if (c.bm != 0) {
+      p.tiles_m = (int)((p.M + c.bm - 1) / c.bm);
+      const int n_cols = kind == NN_SWIGLU ? c.bn / 2 : c.bn;
+      p.tiles_n = (int)((p.N + n_cols - 1) / n_cols);
+      MVIT_REQUIRE((int64_t)p.tiles_m * p.tiles_n * p.split_k < (1ll << 30), "gemm: too many tiles");
+      p.panel_w = p.tiles_n <= 6 ? p.tiles_n : 4;
+      const int rc = c.bm == 256 ? mvit_gemm_pp(kind, p, n_cu, s) : mvit_gemm_small(kind, c.bm, c.bn, p, s);
+      if (rc != MVIT_OK) return rc;
+      if (p.split_k > 1) {
+        if (kind == TT_NONE_F32) launch_splitk_reduce<bf16_t, float>(p, s);
+        else launch_splitk_reduce<bf16_t, bf16_t>(p, s);
+        MVIT_CHECK_LAUNCH("gemm split-k reduce");
+      }
+      return MVIT_OK;
     }
   }
   if (a->dtype == MVIT_BF16) {
@@ -1601,4 +1401,27 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
   }
   MVIT_REQUIRE(a->out_dtype == MVIT_F32, "gemm: fp32 operands need fp32 output");
   return dispatch_trans<float, float>(a->trans_a, a->trans_b, epi, var, p, s);
+}
+
+extern "C" int mvit_gemm_wgrad_split_k(int64_t out_rows, int64_t out_cols, int64_t k) {
+  // Slices along the contraction for a product with few output tiles and a long contraction (a weight gradient, contracted
+  // over the tokens): the count with the lowest modelled time.  Every slice costs an fp32 partial tile written and read back
+  // (3.5 TB/s) and one more launch sums them.
+  if (out_rows <= 0 || out_cols <= 0 || k <= 0) return 1;
+  int best = 1;
+  double best_us = 1e30;
+  for (int sk = 1; sk <= 16 && (sk == 1 || k / sk >= 512); ++sk) {
+    const int64_t chunk = ((k + sk - 1) / sk + 63) / 64 * 64, slices = (k + chunk - 1) / chunk;
+    double us = choose_tile(TT_NONE, out_rows, out_cols, chunk, k - (slices - 1) * chunk, slices, 256).us;
+    if (slices > 1) us += 5. + (double)slices * (double)out_rows * (double)out_cols * 4. / 3.5e6;
+    if (us < best_us) {
+      best_us = us;
+      best = sk;
+    }
+  }
+  return best;
+}
+
+extern "C" int mvit_gemm_swiglu_bwd_sums_columns(int64_t M, int64_t N, int64_t K) {
+  return choose_tile(NT_SWIGLU_BWD, M, N, K, K, 1, 256).bm == 0 ? 1 : 0;
 }

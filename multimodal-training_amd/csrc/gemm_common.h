@@ -1,0 +1,284 @@
+// What the GEMM kernels share: launch parameters, tile order, and the epilogue arithmetic on eight consecutive columns.
+// Included by gemm.hip inside its anonymous namespace's translation unit only.
+#pragma once
+#include "mvit_common.h"
+#include <type_traits>
+
+struct GemmParams {
+  int64_t M, N, K;
+  const void* A;
+  int64_t lda;
+  const void* B;
+  const void* B2;
+  int64_t ldb;
+  const void* bias;
+  const void* bias2;
+  void* C;
+  int64_t ldc;
+  const void* R;
+  int64_t ldr;
+  void* aux;
+  int64_t ldaux;
+  int64_t aux_off;
+  int reduce_epi;  // split_k > 1: the epilogue that the reduction over the K slices applies (none, bias, bias + residual)
+  int tiles_m, tiles_n;
+  int split_k;        // K slices (1 = none)
+  int64_t k_chunk;    // K extent of one slice (multiple of BK)
+  float* workspace;   // [split_k][M][N] fp32 partial sums when split_k > 1
+  int vec_ok;         // every epilogue pointer / stride allows 16-byte accesses
+  int half_vec_ok;    // the output allows 8-byte stores of bf16 (a row pitch that is a multiple of 4 elements only)
+  float* colsum;      // SWIGLU_BWD: per-tile-row column sums of the output, [tiles_m][ldc] (null: not wanted)
+  int panel_w;        // tiles are walked in panels of this many tile columns (M fastest across a panel's rows)
+  // A operand made from decoded frames (gemm_dl_kernel<..., PIX = true>): image table and the affine form of the
+  // rescale / normalise step, value = byte * px_a[channel] + px_c[channel]
+  const mvit_image* px_images;
+  int px_n_images;
+  float px_a[3], px_c[3];
+};
+
+// bf16 kernels behind mvit_gemm that live in translation units of their own; gemm.hip chooses (the K slices of a split
+// product are reduced there too).  They cover the products of the vision tower, see mvit_gemm_tiled_kind.
+enum GemmTiledKind { TILED_NONE = -1, NN_NONE, NN_BIAS, NN_BIAS_RES, NN_BIAS_GELU, NN_SWIGLU, NT_NONE, NT_GELU_BWD, NT_SWIGLU_BWD, TT_NONE, TT_NONE_F32 };
+int mvit_gemm_pp(GemmTiledKind kind, const GemmParams& p, int n_cu, hipStream_t stream);                  // gemm_pingpong.hip
+int mvit_gemm_small(GemmTiledKind kind, int bm, int bn, const GemmParams& p, hipStream_t stream);         // gemm_small.hip
+
+namespace {
+
+// Tile order inside one K slice: panels of panel_w tile columns; within a panel row by row.  Work-groups that run
+// at the same time on one XCD (consecutive tile indices) then cover a compact block of the output, e.g. 8 x 4
+// tiles, so the A and B panels they stream through that XCD's L2 are shared as widely as possible.
+__device__ __forceinline__ void tile_coords(const GemmParams& p, int tile, int& tm, int& tn) {
+  const int pw = p.panel_w;
+  const int full_panels = p.tiles_n / pw, per_panel = p.tiles_m * pw;
+  if (tile < full_panels * per_panel) {
+    const int r = tile % per_panel;
+    tm = r / pw;
+    tn = (tile / per_panel) * pw + r % pw;
+  } else {
+    const int r = tile - full_panels * per_panel, w = p.tiles_n - full_panels * pw;
+    tm = r / w;
+    tn = full_panels * pw + r % w;
+  }
+}
+
+__device__ __forceinline__ float gelu_erf(float z) { return 0.5f * z * (1.f + erff(z * 0.70710678118654752440f)); }
+__device__ __forceinline__ float gelu_erf_grad(float z) {
+  const float cdf = 0.5f * (1.f + erff(z * 0.70710678118654752440f));
+  const float pdf = 0.39894228040143267794f * __expf(-0.5f * z * z);
+  return cdf + z * pdf;
+}
+// 1 / (1 + e^-z) with the hardware reciprocal (1 ulp) instead of the IEEE division sequence
+__device__ __forceinline__ float sigmoidf_(float z) { return __builtin_amdgcn_rcpf(1.f + __expf(-z)); }
+
+// 8 consecutive elements <-> fp32 registers
+__device__ __forceinline__ void load8(const bf16_t* p, float* v) {
+  const bf16x8 x = *reinterpret_cast<const bf16x8*>(p);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = (float)x[e];
+}
+__device__ __forceinline__ void load8(const float* p, float* v) {
+  const f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    v[e] = a[e];
+    v[4 + e] = b[e];
+  }
+}
+template <typename T>
+__device__ __forceinline__ void unpack8(const T __attribute__((ext_vector_type(8))) & x, float* v) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = (float)x[e];
+}
+// Epilogue outputs and per-element epilogue inputs are touched once per launch: they are stored / loaded with the
+// non-temporal hint, so that they do not push the operand panels of the tiles in flight out of the XCD's L2 (a round of
+// 32 output tiles is as large as that L2; with plain stores the main loop after an epilogue ran 18 % slower).
+typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void store8(bf16_t* p, const float* v) {
+  bf16x8 x;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = (bf16_t)v[e];
+  __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, x), reinterpret_cast<u32x4_t*>(p));
+}
+__device__ __forceinline__ void store8(float* p, const float* v) {
+  __builtin_nontemporal_store(f32x4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f32x4*>(p));
+  __builtin_nontemporal_store(f32x4{v[4], v[5], v[6], v[7]}, reinterpret_cast<f32x4*>(p + 4));
+}
+// split-K partial tiles are read back by the reduction kernel right away: they stay cacheable
+__device__ __forceinline__ void store8_cached(float* p, const float* v) {
+  *reinterpret_cast<f32x4*>(p) = f32x4{v[0], v[1], v[2], v[3]};
+  *reinterpret_cast<f32x4*>(p + 4) = f32x4{v[4], v[5], v[6], v[7]};
+}
+template <typename T>
+__device__ __forceinline__ T __attribute__((ext_vector_type(8))) load8_stream(const void* p) {
+  typedef T raw8 __attribute__((ext_vector_type(8)));
+  if constexpr (sizeof(T) == 2) {
+    return __builtin_bit_cast(raw8, __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p)));
+  } else {
+    raw8 r;
+    const f32x4 a = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
+    const f32x4 b = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p) + 1);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      r[e] = a[e];
+      r[4 + e] = b[e];
+    }
+    return r;
+  }
+}
+
+// Epilogue on 8 consecutive output columns n..n+7 of row m.  v: accumulators (gate half for SWIGLU), u: up half.
+// FULL: all 8 columns exist and every pointer allows 16-byte accesses (compile-time trip counts, vector memory
+// operations); otherwise a scalar path bounded by the matrix edge.
+// PRE: the epilogue's per-element inputs (residual / saved activations) were fetched earlier into pre[0..1].
+// hb / hb2: the 8 bias values of columns n .. n+7, already in registers (null: loaded here)
+template <typename T, typename TO, int EPI, bool FULL, bool PRE = false>
+__device__ __forceinline__ void emit8_impl(const GemmParams& p, int64_t m, int64_t n, float* v, const float* u,
+                                           const T __attribute__((ext_vector_type(8))) * pre, float (&cs)[16], bool do_cs,
+                                           const float* hb = nullptr, const float* hb2 = nullptr) {
+  TO* Cp = static_cast<TO*>(p.C);
+  const T* Rp = static_cast<const T*>(p.R);
+  T* auxp = static_cast<T*>(p.aux);
+  const T* bias = static_cast<const T*>(p.bias);
+  const T* bias2 = static_cast<const T*>(p.bias2);
+  const int cnt = FULL ? 8 : ((p.N - n) < 8 ? (int)(p.N - n) : 8);
+  constexpr bool vec = FULL;
+
+  if constexpr (EPI == MVIT_EPI_BIAS || EPI == MVIT_EPI_BIAS_RES || EPI == MVIT_EPI_BIAS_GELU || EPI == MVIT_EPI_SWIGLU) {
+    if (hb) {
+      for (int e = 0; e < 8; ++e) v[e] += hb[e];
+    } else if (bias) {
+      float b[8];
+      if (vec) load8(bias + n, b);
+      else
+        for (int e = 0; e < cnt; ++e) b[e] = to_f32(bias[n + e]);
+      for (int e = 0; e < cnt; ++e) v[e] += b[e];
+    }
+  }
+  if constexpr (EPI == MVIT_EPI_SWIGLU) {
+    float uu[8], h[8];
+    for (int e = 0; e < 8; ++e) uu[e] = u[e];
+    if (hb2) {
+      for (int e = 0; e < 8; ++e) uu[e] += hb2[e];
+    } else if (bias2) {
+      float b[8];
+      if (vec) load8(bias2 + n, b);
+      else
+        for (int e = 0; e < cnt; ++e) b[e] = to_f32(bias2[n + e]);
+      for (int e = 0; e < cnt; ++e) uu[e] += b[e];
+    }
+    // round g and u to the storage type first: the backward recomputes from those stored values
+    for (int e = 0; e < 8; ++e) {
+      v[e] = to_f32(from_f32<T>(v[e]));
+      uu[e] = to_f32(from_f32<T>(uu[e]));
+      h[e] = v[e] * sigmoidf_(v[e]) * uu[e];
+    }
+    TO* h_out = Cp + m * p.ldc + n;
+    if (auxp) {  // a caller that will not differentiate passes no aux and gets the product alone
+      T* g_out = auxp + m * p.ldaux + n;
+      T* u_out = g_out + p.aux_off;
+      if (vec) {
+        store8(g_out, v);
+        store8(u_out, uu);
+      } else {
+        for (int e = 0; e < cnt; ++e) {
+          g_out[e] = from_f32<T>(v[e]);
+          u_out[e] = from_f32<T>(uu[e]);
+        }
+      }
+    }
+    if (vec) store8(h_out, h);
+    else
+      for (int e = 0; e < cnt; ++e) h_out[e] = from_f32<TO>(h[e]);
+    return;
+  }
+  if constexpr (EPI == MVIT_EPI_SWIGLU_BWD) {
+    const T* g_in = Rp + m * p.ldr + n;
+    const T* u_in = g_in + p.aux_off;
+    float g[8], uu[8], dg[8], du[8];
+    if (PRE) {
+      unpack8<T>(pre[0], g);
+      unpack8<T>(pre[1], uu);
+    } else if (vec) {
+      load8(g_in, g);
+      load8(u_in, uu);
+    } else {
+      for (int e = 0; e < 8; ++e) {
+        g[e] = e < cnt ? to_f32(g_in[e]) : 0.f;
+        uu[e] = e < cnt ? to_f32(u_in[e]) : 0.f;
+      }
+    }
+    for (int e = 0; e < 8; ++e) {
+      const float sg = sigmoidf_(g[e]);
+      const float silu = g[e] * sg;
+      dg[e] = v[e] * uu[e] * (sg + silu * (1.f - sg));
+      du[e] = v[e] * silu;
+    }
+    if (do_cs) {  // running column sums of this thread's 8 columns (the gate / up bias gradient)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if (e < cnt) {
+          cs[e] += dg[e];
+          cs[8 + e] += du[e];
+        }
+      }
+    }
+    TO* dg_out = Cp + m * p.ldc + n;
+    TO* du_out = dg_out + p.aux_off;
+    if (vec) {
+      store8(dg_out, dg);
+      store8(du_out, du);
+    } else {
+      for (int e = 0; e < cnt; ++e) {
+        dg_out[e] = from_f32<TO>(dg[e]);
+        du_out[e] = from_f32<TO>(du[e]);
+      }
+    }
+    return;
+  }
+  if constexpr (EPI == MVIT_EPI_BIAS_RES || EPI == MVIT_EPI_GELU_BWD) {
+    float r[8];
+    if (PRE) unpack8<T>(pre[0], r);
+    else if (vec) load8(Rp + m * p.ldr + n, r);
+    else
+      for (int e = 0; e < 8; ++e) r[e] = e < cnt ? to_f32(Rp[m * p.ldr + n + e]) : 0.f;
+    for (int e = 0; e < 8; ++e) {
+      if constexpr (EPI == MVIT_EPI_BIAS_RES) v[e] += r[e];
+      else v[e] *= gelu_erf_grad(r[e]);
+    }
+  }
+  if constexpr (EPI == MVIT_EPI_BIAS_GELU) {
+    T* z_out = auxp + m * p.ldaux + n;
+    for (int e = 0; e < 8; ++e) v[e] = to_f32(from_f32<T>(v[e]));  // gelu of the stored pre-activation
+    if (vec) store8(z_out, v);
+    else
+      for (int e = 0; e < cnt; ++e) z_out[e] = from_f32<T>(v[e]);
+    for (int e = 0; e < 8; ++e) v[e] = gelu_erf(v[e]);
+  }
+  TO* c_out = Cp + m * p.ldc + n;
+  if constexpr (EPI == MVIT_EPI_ACCUM) {
+    float c[8];
+    if (vec) load8(c_out, c);
+    else
+      for (int e = 0; e < 8; ++e) c[e] = e < cnt ? to_f32(c_out[e]) : 0.f;
+    for (int e = 0; e < 8; ++e) v[e] += c[e];
+  }
+  if (vec) store8(c_out, v);
+  else
+    for (int e = 0; e < cnt; ++e) c_out[e] = from_f32<TO>(v[e]);
+}
+
+template <typename T, typename TO, int EPI>
+__device__ __forceinline__ void emit8(const GemmParams& p, int64_t m, int64_t n, float* v, const float* u, bool vec,
+                                      float (&cs)[16], bool do_cs) {
+  if (vec && n + 8 <= p.N) emit8_impl<T, TO, EPI, true>(p, m, n, v, u, nullptr, cs, do_cs);
+  else if (EPI == MVIT_EPI_NONE && sizeof(TO) == 2 && p.half_vec_ok && n + 4 <= p.N) {
+    TO* c = static_cast<TO*>(p.C) + m * p.ldc + n;
+    *reinterpret_cast<bf16x4*>(c) = bf16x4{(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
+    if (n + 8 <= p.N) *reinterpret_cast<bf16x4*>(c + 4) = bf16x4{(bf16_t)v[4], (bf16_t)v[5], (bf16_t)v[6], (bf16_t)v[7]};
+    else
+      for (int e = 4; n + e < p.N; ++e) c[e] = from_f32<TO>(v[e]);
+  }
+  else emit8_impl<T, TO, EPI, false>(p, m, n, v, u, nullptr, cs, do_cs);
+}
+
+}  // namespace

@@ -1,0 +1,39 @@
+// Direct global -> LDS loads, hand-placed waits and the transposing LDS read, as the bf16 GEMM kernels use them.
+// The compiler does not see these loads: waits for them are placed by hand (a wave's memory instructions complete in order).
+#pragma once
+#include "gemm_common.h"
+
+namespace {
+
+template <int N>
+__device__ __forceinline__ void pp_wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
+}
+__device__ __forceinline__ void pp_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+__device__ __forceinline__ void pp_load(unsigned lds_addr, unsigned voff, const char* base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds_addr), "v"(voff), "s"(base) : "memory");
+}
+// the same for the lanes with k < limit only; the instruction is issued (and counted by vmcnt) even when no lane takes part
+__device__ __forceinline__ void pp_load_below(unsigned lds_addr, unsigned voff, const char* base, int k, int limit) {
+  unsigned long long saved;
+  asm volatile(
+      "s_mov_b32 m0, %1\n\tv_cmp_gt_i32 vcc, %5, %4\n\ts_mov_b64 %0, exec\n\ts_and_b64 exec, exec, vcc\n\ts_nop 0\n\t"
+      "global_load_lds_dwordx4 %2, %3\n\ts_mov_b64 exec, %0"
+      : "=&s"(saved) : "s"(lds_addr), "v"(voff), "s"(base), "v"(k), "s"(limit) : "memory", "vcc", "scc");
+}
+__device__ __forceinline__ void pp_load_dword_at(unsigned lds_addr, const char* addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(lds_addr), "v"(addr) : "memory");
+}
+__device__ __forceinline__ bf16x8 pp_read_tr(const unsigned char* p, int second) {
+  typedef s16x4 __attribute__((address_space(3))) * lds_ptr_t;
+  s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr_t)(p));
+  s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr_t)(p + second));
+  typedef short s16x8 __attribute__((ext_vector_type(8)));
+  return __builtin_bit_cast(bf16x8, (s16x8){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+}
+
+}  // namespace

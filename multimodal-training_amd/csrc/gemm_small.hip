@@ -1,0 +1,310 @@
+// bf16 GEMM for products with too few 256 x 256 tiles to fill the chip: one work-group per BM x BN tile, NW waves of
+// WM x WN, K tiles of 64 in a ring of NST LDS stages filled by direct global -> LDS loads up to NST - 1 K tiles ahead.
+// Two work-groups share a compute unit: one multiplies while the other waits for LDS or memory (reading the next K tile's
+// fragments ahead inside one work-group, and deeper rings with one work-group per unit, measured no better).
+// What bounds it is the chain of K steps of one tile, not the matrix pipe: small tiles make the step short (a 64 x 64 tile's
+// step moves 16 KiB into LDS, the 256 x 256 tile's 64 KiB) and put more compute units to work.
+// Fragment layouts, K order, MFMA form and epilogue arithmetic are those of gemm_pp_kernel (gemm_pingpong.hip), so the results
+// are the same bits whichever of the two computed them.
+// A work-group computes one tile, so bias, residual and saved activations are fetched into registers before the main loop.
+#include "gemm_direct.h"
+
+namespace {
+
+template <int BM_, int BN_, int WGM_, int WGN_, int NST_>
+struct SmallCfg {
+  static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, NST = NST_, BK = 64;
+  static constexpr int NW = WGM * WGN, NTHREADS = 64 * NW, WM = BM / WGM, WN = BN / WGN;
+  static constexpr int A_BYTES = BM * BK * 2, STAGE = (BM + BN) * BK * 2, LDS = NST * STAGE;
+  static constexpr int PER_A = BM / 8 / NW, PER_B = BN / 8 / NW, PER = PER_A + PER_B;  // 1 KiB loads per wave and K tile
+  static_assert(NST >= 2 && NST <= 4 && (BM == 64 || BM == 128) && (BN == 64 || BN == 128), "ring depths and swizzles built");
+  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0 && WM % 16 == 0 && WN % 32 == 0, "whole load instructions and MFMA blocks per wave");
+};
+
+// chunk (16 bytes) swizzle of a staged operand: [row][k] tiles by row, [k][row] tiles of ROWS rows by k
+template <bool TR, bool IS_A, int ROWS>
+__device__ __forceinline__ int small_swizzle(int major) {
+  if (!TR) return IS_A ? (major >> 1) & 7 : ((major >> 1) & 1) | (((major >> 3) & 3) << 1);
+  if (ROWS == 64) return IS_A ? (((major >> 1) & 1) << 1) | (((major >> 3) & 1) << 2) : ((major >> 1) & 1) << 2;
+  return IS_A ? ((major & 3) << 1) | (((major >> 3) & 1) << 3) : (major & 3) << 2;
+}
+
+template <typename TO, bool TA, bool TB, int EPI, typename S>
+__global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(const GemmParams p) {  // two work-groups fit a compute unit
+  using T = bf16_t;
+  constexpr int BM = S::BM, BN = S::BN, BK = S::BK, NST = S::NST;
+  constexpr bool DUAL = (EPI == MVIT_EPI_SWIGLU);
+  constexpr bool HAS_IN = EPI == MVIT_EPI_BIAS_RES || EPI == MVIT_EPI_GELU_BWD || EPI == MVIT_EPI_SWIGLU_BWD;
+  constexpr bool HAS_BIAS = EPI == MVIT_EPI_BIAS || EPI == MVIT_EPI_BIAS_RES || EPI == MVIT_EPI_BIAS_GELU || EPI == MVIT_EPI_SWIGLU;
+  constexpr int NA = S::WM / 16, NB = S::WN / 16, NGB = NB / 2;  // row blocks, column blocks, groups of 32 columns of a wave
+  static_assert(!DUAL || (!TB && NGB == 2), "SWIGLU: a gate group and an up group per wave");
+  constexpr int NG = DUAL ? 1 : NGB, NCOLS = DUAL ? BN / 2 : BN, ITEMS = NA * NG;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+
+  const unsigned tiles = (unsigned)(p.tiles_m * p.tiles_n), total = tiles * (unsigned)p.split_k, per_xcd = (total + 7) / 8;
+  const unsigned work = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if ((blockIdx.x >> 3) >= per_xcd || work >= total) return;
+  const unsigned slice = p.split_k > 1 ? work / tiles : 0;
+  int tm, tn;
+  tile_coords(p, (int)(work - slice * tiles), tm, tn);
+  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * NCOLS;
+  const int64_t k_begin = (int64_t)slice * p.k_chunk;
+  const int64_t k_end = p.split_k > 1 ? (k_begin + p.k_chunk < p.K ? k_begin + p.k_chunk : p.K) : p.K;
+  const int klen = (int)(k_end - k_begin), n_kt = (klen + BK - 1) / BK, k_tail = klen % BK;
+
+  const int l = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wv / S::WGN, wn = wv % S::WGN;
+  const int i16 = l & 15, g4 = l >> 4;
+  typedef __attribute__((address_space(3))) unsigned char lds_byte;
+  const unsigned lds_base = (unsigned)(__UINTPTR_TYPE__)(lds_byte*)smem_raw;
+
+  // ---- loader
+  constexpr int A_CH = BM / 8, B_CH = BN / 8;  // chunks of a [k][row] operand's k-row
+  unsigned va[S::PER_A], vb[S::PER_B];
+  const char *ba, *bb;
+  const int64_t step_a = TA ? 2ll * BK * p.lda : 2 * BK, step_b = TB ? 2ll * BK * p.ldb : 2 * BK;
+  const int m_left = (int)(p.M - m0 < BM ? p.M - m0 : BM), n_left = (int)(p.N - n0 < NCOLS ? p.N - n0 : NCOLS);
+  {
+    const T* A = static_cast<const T*>(p.A);
+    const T* B = static_cast<const T*>(DUAL && ((wv * S::PER_B * 8) >> 5 & 1) ? p.B2 : p.B);  // a wave loads rows of one 32-row group
+    static_assert(!DUAL || S::PER_B * 8 <= 32, "one matrix per wave");
+    ba = reinterpret_cast<const char*>(TA ? A + k_begin * p.lda + m0 : A + m0 * p.lda + k_begin);
+    bb = reinterpret_cast<const char*>(TB ? B + k_begin * p.ldb + n0 : B + n0 * p.ldb + k_begin);
+#pragma unroll
+    for (int j = 0; j < S::PER_A; ++j) {
+      const int q = wv * S::PER_A + j;
+      if constexpr (!TA) {
+        const int row = q * 8 + (l >> 3), c = (l & 7) ^ small_swizzle<TA, true, BM>(row);
+        const int r = row < m_left ? row : m_left - 1;  // rows past the edge repeat the last row: their results are not stored
+        va[j] = (unsigned)((r * p.lda + c * 8) * 2);
+      } else {
+        const int k = (q * 64 + l) / A_CH, c = ((q * 64 + l) % A_CH) ^ small_swizzle<TA, true, BM>(k);
+        va[j] = (unsigned)((k * p.lda + (c * 8 < m_left ? c * 8 : 0)) * 2);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < S::PER_B; ++j) {
+      const int q = wv * S::PER_B + j;
+      if constexpr (!TB) {
+        const int row = q * 8 + (l >> 3), c = (l & 7) ^ small_swizzle<TB, false, BN>(row);
+        int r = DUAL ? (row >> 6) * 32 + (row & 31) : row;
+        if (r >= n_left) r = n_left - 1;
+        vb[j] = (unsigned)((r * p.ldb + c * 8) * 2);
+      } else {
+        const int k = (q * 64 + l) / B_CH, c = ((q * 64 + l) % B_CH) ^ small_swizzle<TB, false, BN>(k);
+        vb[j] = (unsigned)((k * p.ldb + (c * 8 < n_left ? c * 8 : 0)) * 2);
+      }
+    }
+  }
+  auto issue = [&](int t, unsigned stage_off) {
+    const unsigned da = lds_base + stage_off + wv * S::PER_A * 1024, db = lds_base + stage_off + S::A_BYTES + wv * S::PER_B * 1024;
+    if (k_tail != 0 && t == n_kt - 1) {  // partial K tile: chunks past the end of K are zeros
+#pragma unroll
+      for (int j = 0; j < S::PER_A; ++j) {
+        const int q = wv * S::PER_A + j, row = q * 8 + (l >> 3);
+        const int k = TA ? (q * 64 + l) / A_CH : 8 * ((l & 7) ^ small_swizzle<TA, true, BM>(row));
+        pp_load_below(da + j * 1024, va[j], ba, k, k_tail);
+        if (k >= k_tail) *reinterpret_cast<u32x4*>(smem_raw + (da - lds_base) + j * 1024 + l * 16) = u32x4{0u, 0u, 0u, 0u};
+      }
+#pragma unroll
+      for (int j = 0; j < S::PER_B; ++j) {
+        const int q = wv * S::PER_B + j, row = q * 8 + (l >> 3);
+        const int k = TB ? (q * 64 + l) / B_CH : 8 * ((l & 7) ^ small_swizzle<TB, false, BN>(row));
+        pp_load_below(db + j * 1024, vb[j], bb, k, k_tail);
+        if (k >= k_tail) *reinterpret_cast<u32x4*>(smem_raw + (db - lds_base) + j * 1024 + l * 16) = u32x4{0u, 0u, 0u, 0u};
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    } else {
+#pragma unroll
+      for (int j = 0; j < S::PER_A; ++j) pp_load(da + j * 1024, va[j], ba);
+#pragma unroll
+      for (int j = 0; j < S::PER_B; ++j) pp_load(db + j * 1024, vb[j], bb);
+    }
+    ba += step_a;
+    bb += step_b;
+  };
+#pragma unroll
+  for (int t = 0; t < NST - 1; ++t)
+    if (t < n_kt) issue(t, t * S::STAGE);
+
+  // ---- fragment addresses (stage 0)
+  unsigned ra[TA ? NA : 2], rb[TB ? 2 * NGB : 2];
+  if constexpr (!TA) {
+    const int row = wm * S::WM + i16, f = small_swizzle<TA, true, BM>(row);
+    ra[0] = row * 128 + ((g4 ^ f) << 4);
+    ra[1] = row * 128 + (((4 + g4) ^ f) << 4);
+  } else {
+    const int k = 8 * g4 + (i16 >> 2), sw = small_swizzle<TA, true, BM>(k);
+#pragma unroll
+    for (int a = 0; a < NA; ++a) ra[a] = k * (BM * 2) + ((((wm * S::WM + a * 16) / 8 + ((i16 & 3) >> 1)) ^ sw) << 4) + (i16 & 1) * 8;
+  }
+  if constexpr (!TB) {
+    const int row = wn * S::WN + 8 * (i16 >> 2) + (i16 & 3), f = small_swizzle<TB, false, BN>(row);
+    rb[0] = S::A_BYTES + row * 128 + ((g4 ^ f) << 4);
+    rb[1] = S::A_BYTES + row * 128 + (((4 + g4) ^ f) << 4);
+  } else {
+    const int k = 8 * g4 + (i16 >> 2), sw = small_swizzle<TB, false, BN>(k);
+#pragma unroll
+    for (int b = 0; b < 2 * NGB; ++b) rb[b] = S::A_BYTES + k * (BN * 2) + ((((wn * S::WN + (b >> 1) * 32) / 8 + (i16 & 3)) ^ sw) << 4) + (b & 1) * 8;
+  }
+
+  // ---- epilogue inputs of this lane: row l % 16 of each row block, columns 8 * (l / 16) .. of each 32-column group
+  const bool to_ws = (EPI == MVIT_EPI_NONE) && p.split_k > 1;
+  const bool vec = to_ws ? (p.N % 4 == 0) : p.vec_ok != 0;
+  const bool interior = vec && m0 + BM <= p.M && n0 + NCOLS <= p.N;
+  int64_t n_lane[NG];
+#pragma unroll
+  for (int g = 0; g < NG; ++g) n_lane[g] = n0 + (DUAL ? wn * 32 : wn * S::WN + g * 32) + 8 * g4;
+  auto row_of = [&](int it) { return m0 + wm * S::WM + (it / NG) * 16 + i16; };
+  constexpr int NLOAD = EPI == MVIT_EPI_SWIGLU_BWD ? 2 : 1;
+  [[maybe_unused]] bf16x8 pre[HAS_IN ? ITEMS : 1][NLOAD];
+  [[maybe_unused]] bf16x8 bias_g[HAS_BIAS ? NG : 1], bias_u;
+  if (interior) {
+    if constexpr (HAS_IN) {
+#pragma unroll
+      for (int it = 0; it < ITEMS; ++it) {
+        const T* r = static_cast<const T*>(p.R) + row_of(it) * p.ldr + n_lane[it % NG];
+        pre[it][0] = *reinterpret_cast<const bf16x8*>(r);
+        if (NLOAD == 2) pre[it][NLOAD - 1] = *reinterpret_cast<const bf16x8*>(r + p.aux_off);
+      }
+    }
+    if constexpr (HAS_BIAS) {
+#pragma unroll
+      for (int g = 0; g < NG; ++g) bias_g[g] = *reinterpret_cast<const bf16x8*>(static_cast<const T*>(p.bias) + n_lane[g]);
+      if (DUAL) bias_u = *reinterpret_cast<const bf16x8*>(static_cast<const T*>(p.bias2) + n_lane[0]);
+    }
+  }
+
+  // ---- main loop
+  f32x4 acc[NA][NB];
+#pragma unroll
+  for (int a = 0; a < NA; ++a)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  unsigned st = 0, st_in = (NST - 1) * S::STAGE;  // stage consumed, stage filled
+  for (int t = 0; t < n_kt; ++t) {
+    // K tile t has landed once only tiles requested after it are in flight
+    const int newer = n_kt - 1 - t;
+    if (newer >= NST - 2) pp_wait_vm<(NST - 2) * S::PER>();
+    else if (NST > 3 && newer == 1) pp_wait_vm<S::PER>();
+    else pp_wait_vm<0>();
+    pp_barrier();  // every wave's share of K tile t is in LDS; K tile t - 1 has been consumed
+    if (t + NST - 1 < n_kt) issue(t + NST - 1, st_in);
+    const unsigned char* at = smem_raw + st;
+    bf16x8 fa[NA][2], fb[NB][2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        if constexpr (!TB) fb[b][ks] = *reinterpret_cast<const bf16x8*>(at + rb[ks] + (b >> 1) * 4096 + (b & 1) * 512);
+        else fb[b][ks] = pp_read_tr(at + rb[b] + ks * 32 * (BN * 2), 4 * (BN * 2));
+      }
+#pragma unroll
+      for (int a = 0; a < NA; ++a) {
+        if constexpr (!TA) fa[a][ks] = *reinterpret_cast<const bf16x8*>(at + ra[ks] + a * 2048);
+        else fa[a][ks] = pp_read_tr(at + ra[a] + ks * 32 * (BM * 2), 4 * (BM * 2));
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[b][ks], fa[a][ks], acc[a][b], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    st = st + S::STAGE == S::LDS ? 0 : st + S::STAGE;
+    st_in = st_in + S::STAGE == S::LDS ? 0 : st_in + S::STAGE;
+  }
+
+  // ---- epilogue
+  float* ws = to_ws ? p.workspace + (int64_t)slice * p.M * p.N : nullptr;
+  float no_cs[16];
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    const int a = it / NG, g = it % NG;
+    const int64_t m = row_of(it), n = n_lane[g];
+    float v[8], u[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[e] = acc[a][2 * g][e];
+      v[4 + e] = acc[a][2 * g + 1][e];
+      if (DUAL) {
+        u[e] = acc[a][NB - 2][e];
+        u[4 + e] = acc[a][NB - 1][e];
+      }
+    }
+    if (interior) {
+      float hb[8], hb2[8];
+      if (HAS_BIAS) unpack8<T>(bias_g[g], hb);
+      if (HAS_BIAS && DUAL) unpack8<T>(bias_u, hb2);
+      if (to_ws) store8_cached(ws + m * p.N + n, v);
+      else emit8_impl<T, TO, EPI, true, HAS_IN>(p, m, n, v, u, HAS_IN ? pre[it] : nullptr, no_cs, false, HAS_BIAS ? hb : nullptr, HAS_BIAS && DUAL ? hb2 : nullptr);
+    } else {
+      if (m >= p.M || n >= p.N) continue;
+      if (to_ws) {
+        float* w = ws + m * p.N + n;
+        if (vec && n + 8 <= p.N) store8_cached(w, v);
+        else
+          for (int e = 0; e < 8 && n + e < p.N; ++e) w[e] = v[e];
+      } else {
+        emit8<T, TO, EPI>(p, m, n, v, u, vec, no_cs, false);
+      }
+    }
+  }
+}
+
+}  // namespace
+
+namespace {
+
+using Small64 = SmallCfg<64, 64, 2, 2, 4>;      // 64 KiB of LDS
+using Small64x128 = SmallCfg<64, 128, 2, 2, 3>;  // 72 KiB
+using Small128 = SmallCfg<128, 128, 4, 2, 2>;    // 64 KiB
+
+template <typename TO, bool TA, bool TB, int EPI, typename S>
+int launch_small(const GemmParams& p, hipStream_t stream) {
+  auto kern = gemm_small_kernel<TO, TA, TB, EPI, S>;
+  static bool attr_set_on[MVIT_MAX_DEVICES] = {};
+  const int dev = mvit_current_device("gemm");
+  if (dev < 0) return MVIT_ERR_LAUNCH;
+  if (!attr_set_on[dev] && S::LDS > 64 * 1024) {  // dynamic LDS above 64 KiB is opted into once per kernel and device
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
+    if (e != hipSuccess) return mvit_set_error(MVIT_ERR_LAUNCH, "gemm: hipFuncSetAttribute(%d B LDS): %s", S::LDS, hipGetErrorString(e));
+    attr_set_on[dev] = true;
+  }
+  hipLaunchKernelGGL(kern, (p.tiles_m * p.tiles_n * p.split_k + 7) / 8 * 8, S::NTHREADS, S::LDS, stream, p);
+  MVIT_CHECK_LAUNCH("gemm");
+  return MVIT_OK;
+}
+
+template <typename S>
+int dispatch_small(GemmTiledKind kind, const GemmParams& p, hipStream_t s) {
+  switch (kind) {
+    case NN_NONE: return launch_small<bf16_t, false, false, MVIT_EPI_NONE, S>(p, s);
+    case NN_BIAS: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS, S>(p, s);
+    case NN_BIAS_RES: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_RES, S>(p, s);
+    case NN_BIAS_GELU: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_GELU, S>(p, s);
+    case NN_SWIGLU:
+      if constexpr (S::WN == 64) return launch_small<bf16_t, false, false, MVIT_EPI_SWIGLU, S>(p, s);
+      break;
+    case NT_NONE: return launch_small<bf16_t, false, true, MVIT_EPI_NONE, S>(p, s);
+    case NT_GELU_BWD: return launch_small<bf16_t, false, true, MVIT_EPI_GELU_BWD, S>(p, s);
+    case NT_SWIGLU_BWD:  // 128 x 128 with two inputs per element would not leave registers for two work-groups per unit
+      if constexpr (S::BM == 64) return launch_small<bf16_t, false, true, MVIT_EPI_SWIGLU_BWD, S>(p, s);
+      break;
+    case TT_NONE: return launch_small<bf16_t, true, true, MVIT_EPI_NONE, S>(p, s);
+    case TT_NONE_F32: return launch_small<float, true, true, MVIT_EPI_NONE, S>(p, s);
+    default: break;
+  }
+  return mvit_set_error(MVIT_ERR_UNSUPPORTED, "gemm: product kind %d has no %d x %d kernel", (int)kind, S::BM, S::BN);
+}
+
+}  // namespace
+
+int mvit_gemm_small(GemmTiledKind kind, int bm, int bn, const GemmParams& p, hipStream_t stream) {
+  if (bm == 128) return dispatch_small<Small128>(kind, p, stream);
+  if (bn == 128) return dispatch_small<Small64x128>(kind, p, stream);
+  return dispatch_small<Small64>(kind, p, stream);
+}

@@ -298,11 +298,13 @@ def _block_backward(dx2: torch.Tensor, x: torch.Tensor, saved: tuple, W: BlockWe
     g_wd = torch.empty(C, I, dtype=gdt["mlp.down_proj.weight"], device=dev)
     g_bd = off_chain(lambda: (ops.colsum(dx2, gdt["mlp.down_proj.bias"]), wgrad(dx2, h, g_wd, n=I))[0])
     dgu = torch.empty(S, 2 * Ipad, dtype=x.dtype, device=dev)
-    # the epilogue also hands back per-tile column sums of dgu: the gate / up bias gradient without re-reading dgu
-    part = torch.empty(-(-S // 256), 2 * Ipad, dtype=torch.float32, device=dev)
+    # with many rows the epilogue also hands back per-tile column sums of dgu: the gate / up bias gradient without re-reading dgu
+    fused = x.dtype != torch.bfloat16 or ops.swiglu_bwd_sums_columns(S, Ipad, C)
+    part = torch.empty(-(-S // 256), 2 * Ipad, dtype=torch.float32, device=dev) if fused else None
     ops.gemm(dx2, W.wdown, dgu, trans_b=True, epilogue=E.EPI_SWIGLU_BWD, residual=gu, aux_off=Ipad, colsum_partial=part)
     g_wgu = torch.empty(2 * Ipad, C, dtype=gdt["mlp.gate_proj.weight"], device=dev)
-    g_bgu = off_chain(lambda: (ops.reduce_partials(part, gdt["mlp.gate_proj.bias"]), wgrad(dgu, n2, g_wgu))[0])
+    bgrad = (lambda: ops.reduce_partials(part, gdt["mlp.gate_proj.bias"])) if fused else (lambda: ops.colsum(dgu, gdt["mlp.gate_proj.bias"]))
+    g_bgu = off_chain(lambda: (bgrad(), wgrad(dgu, n2, g_wgu))[0])
     dn2 = torch.empty_like(x)
     ops.gemm(dgu, W.wgu, dn2, trans_b=True)
     dx1, g_n2 = ops.rmsnorm_bwd(dn2, x1, W.norm2.view(-1), rstd2, dx_add=dx2, w_grad_dtype=gdt["norm2.weight"])

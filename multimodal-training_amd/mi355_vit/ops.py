@@ -362,34 +362,18 @@ def gemm(
     return out
 
 
-_N_CU = 256  # MI355X compute units; one 256x256 GEMM work-group runs per CU
+@functools.lru_cache(maxsize=None)
+def wgrad_split_k(out_rows: int, out_cols: int, k: int) -> int:
+    """K slices for a GEMM with few output tiles and a long contraction: the weight gradients (contraction over the
+    tokens).  The model uses it for those only: on a forward or input-gradient GEMM a slice count chosen from the batch
+    size would make a row's result depend on how many rows share its batch."""
+    return _lib.load().mvit_gemm_wgrad_split_k(out_rows, out_cols, k)
 
 
 @functools.lru_cache(maxsize=None)
-def wgrad_split_k(out_rows: int, out_cols: int, k: int) -> int:
-    """K slices for a GEMM with few output tiles (256x256) and a long contraction: the weight gradients (contraction
-    over the tokens).  The model uses it for those only: on a forward or input-gradient GEMM a slice count chosen
-    from the batch size would make a row's result depend on how many rows share its batch.
-
-    Picks the slice count with the lowest modelled time.  Work items (tiles x slices) run in rounds of one per
-    CU, so the count should fill whole rounds; every slice costs an fp32 partial tile that a second kernel
-    re-reads.  Constants are microseconds measured on MI355X (a 32-deep K step takes 0.6 us on a lightly loaded
-    chip, 0.95 us when every CU is busy; ~8 us per tile epilogue; ~3.5 TB/s for the partial-sum traffic)."""
-    tiles = -(-out_rows // 256) * -(-out_cols // 256)
-    best, best_t = 1, None
-    for sk in range(1, 17):
-        if sk > 1 and k // sk < 512:
-            break
-        items = tiles * sk
-        rounds = -(-items // _N_CU)
-        load = items / (rounds * _N_CU)
-        steps = -(-(-(-k // sk)) // 64) * 2
-        t = rounds * (steps * (0.6 + 0.35 * load) + 8.0)
-        if sk > 1:
-            t += 5.0 + sk * out_rows * out_cols * 4 / 3.5e6
-        if best_t is None or t < best_t:
-            best, best_t = sk, t
-    return best
+def swiglu_bwd_sums_columns(rows: int, cols: int, k: int) -> bool:
+    """Whether the bf16 SwiGLU-backward product of this shape hands back the column sums of its result (many rows)."""
+    return bool(_lib.load().mvit_gemm_swiglu_bwd_sums_columns(rows, cols, k))
 
 
 # ------------------------------------------------------------------------------ attention
