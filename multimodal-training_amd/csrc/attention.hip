@@ -11,8 +11,8 @@
 // registers; row reductions are two cross-lane exchanges (lanes l, l^16, l^32, l^48 share a query).
 // The backward is split in two kernels (dK/dV, then dQ), which keeps it free of atomics and bit-reproducible.
 //
-// fp32 path (parity mode): one lane per query (or key) row, K/V (or Q/dO) tiles broadcast from LDS.
-#include "mvit_common.h"
+// fp32 path (parity mode): attention_f32.hip.
+#include "attention_common.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -22,47 +22,6 @@ namespace {
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float LN2 = 0.6931471805599453f;
 
-struct AttnParams {
-  const void *q, *k, *v, *o, *d_o;
-  void *out, *dq, *dk, *dv;
-  float* lse;
-  float* delta;
-  const int32_t* cu;
-  int64_t total;
-  int nheads;
-  int64_t q_stride, k_stride, v_stride, o_stride, do_stride, dq_stride, dk_stride, dv_stride;
-  float scale;
-  const void* q_scaled;  // wide backward: bf16(Q * scale * log2(e)), row stride qs_stride
-  int64_t qs_stride;
-  const float *nlse2, *ndelta;  // wide backward: - lse * log2(e) and - delta, [nheads, total]
-  const int32_t* order;  // optional: the segment scheduled at grid position i is order[i] (null: i)
-  int seg_major;         // 0: grid (x, segment, head); 1: grid (x, head, segment), all heads of a segment together
-};
-
-// Which segment and head this work-group serves.  Work per work-group grows with its segment's length, so
-// callers list long segments first: the short ones then fill the tail of the launch.
-//
-// seg_major = 2 (short segments, grid (1, n_seg, heads) with n_seg * heads a multiple of 8): a head's slice of a
-// token row is 160 bytes at head_dim 80, so the heads of one segment share their 128-byte lines.  Work-group ids
-// are dealt round-robin to the 8 XCDs; id i therefore takes work item (i % 8) * (total / 8) + i / 8 of the
-// head-fastest list, which puts all heads of a segment on one XCD at about the same time and lets its L2 serve
-// the shared lines (the natural order reads them from memory once per head).
-__device__ __forceinline__ void seg_and_head(const AttnParams& p, int& seg, int& h) {
-  int pos = p.seg_major == 1 ? blockIdx.z : blockIdx.y;
-  h = p.seg_major == 1 ? blockIdx.y : blockIdx.z;
-  const int n_seg = p.seg_major == 1 ? gridDim.z : gridDim.y;
-  if (p.seg_major == 2) {
-    const int nh = gridDim.z, lin = blockIdx.y + n_seg * blockIdx.z;
-    const int w = (lin & 7) * ((n_seg * nh) >> 3) + (lin >> 3);
-    pos = w / nh;
-    h = w % nh;
-  }
-  seg = pos;
-  if (p.order) {
-    const int listed = p.order[pos];
-    if ((unsigned)listed < (unsigned)n_seg) seg = listed;  // an entry outside the list never becomes an address
-  }
-}
 
 typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr;
 typedef short s16x8 __attribute__((ext_vector_type(8)));
@@ -2001,191 +1960,6 @@ __global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const Attn
   }
 }
 
-// ================================================================================================
-// fp32 parity kernels: one lane per row, 32-row tiles of the other side broadcast from LDS.
-template <int HD>
-__global__ __launch_bounds__(64) void attn_fwd_f32(const AttnParams p) {
-  constexpr int TB = 32;
-  __shared__ float sk[TB * HD];
-  __shared__ float sv[TB * HD];
-  int seg, h;
-  seg_and_head(p, seg, h);
-  const int s0 = p.cu[seg], L = p.cu[seg + 1] - s0;
-  const int q0 = blockIdx.x * 64;
-  if (q0 >= L) return;
-  const int qi = q0 + threadIdx.x;
-  const bool valid = qi < L;
-  const float* Q = static_cast<const float*>(p.q) + (int64_t)s0 * p.q_stride + (int64_t)h * HD;
-  const float* K = static_cast<const float*>(p.k) + (int64_t)s0 * p.k_stride + (int64_t)h * HD;
-  const float* V = static_cast<const float*>(p.v) + (int64_t)s0 * p.v_stride + (int64_t)h * HD;
-  float qr[HD], acc[HD];
-#pragma unroll
-  for (int j = 0; j < HD; ++j) {
-    qr[j] = valid ? Q[(int64_t)qi * p.q_stride + j] : 0.f;
-    acc[j] = 0.f;
-  }
-  float m = -INFINITY, lsum = 0.f;
-  for (int k0 = 0; k0 < L; k0 += TB) {
-    const int nk = min(TB, L - k0);
-    __syncthreads();
-    for (int i = threadIdx.x; i < TB * HD; i += 64) {
-      const int rr = i / HD, j = i % HD;
-      sk[i] = rr < nk ? K[(int64_t)(k0 + rr) * p.k_stride + j] : 0.f;
-      sv[i] = rr < nk ? V[(int64_t)(k0 + rr) * p.v_stride + j] : 0.f;
-    }
-    __syncthreads();
-    float s[TB];
-    float mx = m;
-#pragma unroll
-    for (int t = 0; t < TB; ++t) {
-      float d = 0.f;
-#pragma unroll
-      for (int j = 0; j < HD; ++j) d += qr[j] * sk[t * HD + j];
-      s[t] = t < nk ? d * p.scale : -INFINITY;
-      mx = fmaxf(mx, s[t]);
-    }
-    const float alpha = expf(m - mx);
-    m = mx;
-    lsum *= alpha;
-#pragma unroll
-    for (int j = 0; j < HD; ++j) acc[j] *= alpha;
-#pragma unroll
-    for (int t = 0; t < TB; ++t) {
-      const float e = expf(s[t] - mx);
-      lsum += e;
-#pragma unroll
-      for (int j = 0; j < HD; ++j) acc[j] += e * sv[t * HD + j];
-    }
-  }
-  if (valid) {
-    float* O = static_cast<float*>(p.out) + (int64_t)(s0 + qi) * p.o_stride + (int64_t)h * HD;
-    const float inv = 1.f / lsum;
-#pragma unroll
-    for (int j = 0; j < HD; ++j) O[j] = acc[j] * inv;
-    p.lse[(int64_t)h * p.total + s0 + qi] = m + logf(lsum);
-  }
-}
-
-template <int HD>
-__global__ __launch_bounds__(64) void attn_bwd_dq_f32(const AttnParams p) {
-  constexpr int TB = 32;
-  __shared__ float sk[TB * HD];
-  __shared__ float sv[TB * HD];
-  int seg, h;
-  seg_and_head(p, seg, h);
-  const int s0 = p.cu[seg], L = p.cu[seg + 1] - s0;
-  const int q0 = blockIdx.x * 64;
-  if (q0 >= L) return;
-  const int qi = q0 + threadIdx.x;
-  const bool valid = qi < L;
-  const float* Q = static_cast<const float*>(p.q) + (int64_t)s0 * p.q_stride + (int64_t)h * HD;
-  const float* K = static_cast<const float*>(p.k) + (int64_t)s0 * p.k_stride + (int64_t)h * HD;
-  const float* V = static_cast<const float*>(p.v) + (int64_t)s0 * p.v_stride + (int64_t)h * HD;
-  const float* DO = static_cast<const float*>(p.d_o) + (int64_t)s0 * p.do_stride + (int64_t)h * HD;
-  float qr[HD], dor[HD], acc[HD];
-#pragma unroll
-  for (int j = 0; j < HD; ++j) {
-    qr[j] = valid ? Q[(int64_t)qi * p.q_stride + j] : 0.f;
-    dor[j] = valid ? DO[(int64_t)qi * p.do_stride + j] : 0.f;
-    acc[j] = 0.f;
-  }
-  const float lse = valid ? p.lse[(int64_t)h * p.total + s0 + qi] : INFINITY;
-  const float dl = valid ? p.delta[(int64_t)h * p.total + s0 + qi] : 0.f;
-  for (int k0 = 0; k0 < L; k0 += TB) {
-    const int nk = min(TB, L - k0);
-    __syncthreads();
-    for (int i = threadIdx.x; i < TB * HD; i += 64) {
-      const int rr = i / HD, j = i % HD;
-      sk[i] = rr < nk ? K[(int64_t)(k0 + rr) * p.k_stride + j] : 0.f;
-      sv[i] = rr < nk ? V[(int64_t)(k0 + rr) * p.v_stride + j] : 0.f;
-    }
-    __syncthreads();
-    for (int t = 0; t < nk; ++t) {
-      float d = 0.f, dp = 0.f;
-#pragma unroll
-      for (int j = 0; j < HD; ++j) {
-        d += qr[j] * sk[t * HD + j];
-        dp += dor[j] * sv[t * HD + j];
-      }
-      const float ds = expf(d * p.scale - lse) * (dp - dl);
-#pragma unroll
-      for (int j = 0; j < HD; ++j) acc[j] += ds * sk[t * HD + j];
-    }
-  }
-  if (valid) {
-    float* DQ = static_cast<float*>(p.dq) + (int64_t)(s0 + qi) * p.dq_stride + (int64_t)h * HD;
-#pragma unroll
-    for (int j = 0; j < HD; ++j) DQ[j] = acc[j] * p.scale;
-  }
-}
-
-template <int HD>
-__global__ __launch_bounds__(64) void attn_bwd_dkdv_f32(const AttnParams p) {
-  constexpr int TB = 32;
-  __shared__ float sq[TB * HD];
-  __shared__ float sdo[TB * HD];
-  __shared__ float slse[TB];
-  __shared__ float sdl[TB];
-  int seg, h;
-  seg_and_head(p, seg, h);
-  const int s0 = p.cu[seg], L = p.cu[seg + 1] - s0;
-  const int kb0 = blockIdx.x * 64;
-  if (kb0 >= L) return;
-  const int ki = kb0 + threadIdx.x;
-  const bool valid = ki < L;
-  const float* Q = static_cast<const float*>(p.q) + (int64_t)s0 * p.q_stride + (int64_t)h * HD;
-  const float* K = static_cast<const float*>(p.k) + (int64_t)s0 * p.k_stride + (int64_t)h * HD;
-  const float* V = static_cast<const float*>(p.v) + (int64_t)s0 * p.v_stride + (int64_t)h * HD;
-  const float* DO = static_cast<const float*>(p.d_o) + (int64_t)s0 * p.do_stride + (int64_t)h * HD;
-  float kr[HD], vr[HD], dk[HD], dv[HD];
-#pragma unroll
-  for (int j = 0; j < HD; ++j) {
-    kr[j] = valid ? K[(int64_t)ki * p.k_stride + j] : 0.f;
-    vr[j] = valid ? V[(int64_t)ki * p.v_stride + j] : 0.f;
-    dk[j] = 0.f;
-    dv[j] = 0.f;
-  }
-  for (int qs = 0; qs < L; qs += TB) {
-    const int nq = min(TB, L - qs);
-    __syncthreads();
-    for (int i = threadIdx.x; i < TB * HD; i += 64) {
-      const int rr = i / HD, j = i % HD;
-      sq[i] = rr < nq ? Q[(int64_t)(qs + rr) * p.q_stride + j] : 0.f;
-      sdo[i] = rr < nq ? DO[(int64_t)(qs + rr) * p.do_stride + j] : 0.f;
-    }
-    if (threadIdx.x < TB) {
-      const bool ok = (int)threadIdx.x < nq;
-      slse[threadIdx.x] = ok ? p.lse[(int64_t)h * p.total + s0 + qs + threadIdx.x] : INFINITY;
-      sdl[threadIdx.x] = ok ? p.delta[(int64_t)h * p.total + s0 + qs + threadIdx.x] : 0.f;
-    }
-    __syncthreads();
-    for (int t = 0; t < nq; ++t) {
-      float d = 0.f, dp = 0.f;
-#pragma unroll
-      for (int j = 0; j < HD; ++j) {
-        d += sq[t * HD + j] * kr[j];
-        dp += sdo[t * HD + j] * vr[j];
-      }
-      const float e = expf(d * p.scale - slse[t]);
-      const float ds = e * (dp - sdl[t]);
-#pragma unroll
-      for (int j = 0; j < HD; ++j) {
-        dv[j] += e * sdo[t * HD + j];
-        dk[j] += ds * sq[t * HD + j];
-      }
-    }
-  }
-  if (valid) {
-    float* DK = static_cast<float*>(p.dk) + (int64_t)(s0 + ki) * p.dk_stride + (int64_t)h * HD;
-    float* DV = static_cast<float*>(p.dv) + (int64_t)(s0 + ki) * p.dv_stride + (int64_t)h * HD;
-#pragma unroll
-    for (int j = 0; j < HD; ++j) {
-      DK[j] = dk[j] * p.scale;
-      DV[j] = dv[j];
-    }
-  }
-}
-
 // ------------------------------------------------------------------------------------------------
 constexpr int WIDE_MIN_SEQLEN = 512;  // from here on the 64-rows-per-wave kernels fill their work-groups well enough
 inline int pick_waves(int max_seqlen) { return max_seqlen <= 64 ? 1 : (max_seqlen <= 128 ? 2 : 4); }
@@ -2271,19 +2045,6 @@ int launch_bwd_mfma(const AttnParams& p, int n_seg, int max_seqlen, hipStream_t 
   MVIT_CHECK_LAUNCH("attn_bwd");
   return MVIT_OK;
 }
-template <int HD>
-int launch_f32(const AttnParams& p, int n_seg, int max_seqlen, bool bwd, hipStream_t s) {
-  dim3 grid((unsigned)((max_seqlen + 63) / 64), (unsigned)n_seg, (unsigned)p.nheads);
-  if (!bwd) {
-    hipLaunchKernelGGL((attn_fwd_f32<HD>), grid, 64, 0, s, p);
-  } else {
-    hipLaunchKernelGGL((attn_bwd_dkdv_f32<HD>), grid, 64, 0, s, p);
-    hipLaunchKernelGGL((attn_bwd_dq_f32<HD>), grid, 64, 0, s, p);
-  }
-  MVIT_CHECK_LAUNCH("attn_f32");
-  return MVIT_OK;
-}
-
 int check_common(const char* who, const int32_t* cu, int n_seg, int max_seqlen, int64_t total, int nheads, int head_dim,
                  int dtype, std::initializer_list<int64_t> strides, std::initializer_list<const void*> ptrs) {
   MVIT_REQUIRE(cu && n_seg >= 0 && max_seqlen >= 0 && total >= 0 && nheads > 0 && nheads <= 65535 && n_seg <= 65535,
@@ -2341,12 +2102,7 @@ int mvit_attn_fwd(const void* q, const void* k, const void* v, void* o, float* l
       default: return launch_fwd_mfma<8>(p, n_seg, max_seqlen, s);
     }
   }
-  switch (head_dim) {
-    case 32: return launch_f32<32>(p, n_seg, max_seqlen, false, s);
-    case 64: return launch_f32<64>(p, n_seg, max_seqlen, false, s);
-    case 80: return launch_f32<80>(p, n_seg, max_seqlen, false, s);
-    default: return launch_f32<128>(p, n_seg, max_seqlen, false, s);
-  }
+  return mvit_attn_f32(p, head_dim, n_seg, max_seqlen, false, s);
 }
 
 int mvit_attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, void* dq,
@@ -2407,12 +2163,7 @@ int mvit_attn_bwd(const void* q, const void* k, const void* v, const void* o, co
       default: return launch_bwd_mfma<8>(p, n_seg, max_seqlen, s);
     }
   }
-  switch (head_dim) {
-    case 32: return launch_f32<32>(p, n_seg, max_seqlen, true, s);
-    case 64: return launch_f32<64>(p, n_seg, max_seqlen, true, s);
-    case 80: return launch_f32<80>(p, n_seg, max_seqlen, true, s);
-    default: return launch_f32<128>(p, n_seg, max_seqlen, true, s);
-  }
+  return mvit_attn_f32(p, head_dim, n_seg, max_seqlen, true, s);
 }
 
 }  // extern "C"

@@ -191,7 +191,7 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   }
   // dgu = (dx2 . Wdown) through the SwiGLU derivative.  With many rows the per-tile column sums of dgu come back with it;
   // with few the product runs on smaller tiles and the sums are taken beside the chain
-  const bool fused_cols = dt != MVIT_BF16 || mvit_gemm_swiglu_bwd_sums_columns(S, Ipad, C);
+  const bool fused_cols = dt == MVIT_BF16 && mvit_gemm_swiglu_bwd_sums_columns(S, Ipad, C);
   {
     mvit_gemm_args g = gemm_args(dt, dt);
     g.trans_b = 1; g.epilogue = MVIT_EPI_SWIGLU_BWD;

@@ -6,9 +6,9 @@
 //   bf16, the rest (SwiGLU backward of many rows, patch embedding from frames, fp32 outputs, accumulation): 256x256 tile, 8
 //      waves of 128x64 (4x2 MFMA 32x32x16 tiles each), BK = 32, four LDS stages filled by direct global -> LDS loads (see
 //      gemm_dl_kernel).
-//   fp32 (the parity path, v_mfma_f32_32x32x2_f32), and bf16 operands whose row pitch exceeds 2^22 elements (the
-//      direct loads use 32-bit lane offsets): 256x256 tile, 8 waves, BK = 64 (fp32: 16), global -> registers -> LDS,
-//      double-buffered LDS, one barrier per K step (gemm_kernel).
+//   bf16 operands whose row pitch exceeds 2^22 elements (the direct loads use 32-bit lane offsets): 256x256 tile, 8 waves,
+//      BK = 64, global -> registers -> LDS, double-buffered LDS, one barrier per K step (gemm_kernel).
+//   fp32 (the parity path): gemm_f32_kernel (gemm_f32.hip).
 // Operands whose contraction index is contiguous in memory are staged as [row][k] and read with 16-byte LDS
 // loads; operands whose contraction index is the slow dimension (dgrad's weight, both operands of wgrad) are
 // staged as [k][row] exactly as they lie in memory and read with ds_read_b64_tr_b16, which hands each lane 4
@@ -32,12 +32,6 @@ struct Cfg<bf16_t> {
   static constexpr int BK = 64, VEC = 8;
   static constexpr int PITCH_K = BK + 8;  // [row][k] staging: 144-byte rows, conflict-free 16-byte reads
   static constexpr int PAD_T = 32;        // [k][row] staging: row pitch = rows + 32 elements
-};
-template <>
-struct Cfg<float> {
-  static constexpr int BK = 16, VEC = 4;
-  static constexpr int PITCH_K = BK + 4;
-  static constexpr int PAD_T = 4;
 };
 
 template <int VAR>
@@ -228,16 +222,6 @@ __device__ __forceinline__ bf16x8 frag_bf16(const bf16_t* lds, int row, int k) {
     s16x8 both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     return __builtin_bit_cast(bf16x8, both);
   }
-}
-
-template <bool TR, int ROWS>
-__device__ __forceinline__ float frag_f32(const float* lds, int row, int k) {
-  using C = Cfg<float>;
-  const int l = threadIdx.x & 63;
-  if (!TR)
-    return lds[(row + (l & 31)) * C::PITCH_K + k + (l >> 5)];
-  else
-    return lds[(k + (l >> 5)) * (ROWS + C::PAD_T) + row + (l & 31)];
 }
 
 // Per-element epilogue inputs (residual / saved activations) of an interior tile, fetched ahead of their use.
@@ -532,7 +516,7 @@ __global__ __launch_bounds__(Waves<VAR>::NTHREADS, Waves<VAR>::MIN_WAVES) void g
     }
     const T* lds_a = lds + buf * STAGE_ELEMS;
     const T* lds_b = lds_a + LoaderA::LDS_ELEMS;
-    if constexpr (sizeof(T) == 2) {
+    {
       // operand fragments are fetched one 16-wide step ahead of the MFMAs that consume them
       const bf16_t* la_ = reinterpret_cast<const bf16_t*>(lds_a);
       const bf16_t* lb_ = reinterpret_cast<const bf16_t*>(lds_b);
@@ -557,19 +541,6 @@ __global__ __launch_bounds__(Waves<VAR>::NTHREADS, Waves<VAR>::MIN_WAVES) void g
           for (int b = 0; b < NT; ++b)
             acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[cur][a], fb[cur][b], acc[a][b], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
-      }
-    } else {
-#pragma unroll
-      for (int ks = 0; ks < BK; ks += 2) {
-        float fa[MT], fb[NT];
-#pragma unroll
-        for (int a = 0; a < MT; ++a) fa[a] = frag_f32<TA, BM>(reinterpret_cast<const float*>(lds_a), wm * WM + a * 32, ks);
-#pragma unroll
-        for (int b = 0; b < NT; ++b) fb[b] = frag_f32<TB, BN>(reinterpret_cast<const float*>(lds_b), wn * WN + b * 32, ks);
-#pragma unroll
-        for (int a = 0; a < MT; ++a)
-#pragma unroll
-          for (int b = 0; b < NT; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[a], fb[b], acc[a][b], 0, 0, 0);
       }
     }
     if (has_next) {
@@ -1072,6 +1043,17 @@ int launch(const GemmParams& p, hipStream_t stream) {
   return MVIT_OK;
 }
 
+// Column sums of C per 256 rows, columns [0, N) and [aux_off, aux_off + N): what the bf16 SwiGLU-backward epilogue hands back
+// from its tiles, for the fp32 product whose tiles are smaller.
+__global__ __launch_bounds__(256) void tile_colsum_kernel(const float* __restrict__ C, int64_t ldc, int64_t M, int64_t N, int64_t aux_off, float* __restrict__ out) {
+  const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x, m0 = (int64_t)blockIdx.y * 256, m1 = m0 + 256 < M ? m0 + 256 : M;
+  if (n >= N) return;
+  const int64_t col = n + blockIdx.z * aux_off;
+  float s = 0.f;
+  for (int64_t m = m0; m < m1; ++m) s += C[m * ldc + col];
+  out[blockIdx.y * ldc + col] = s;
+}
+
 // Compute units of the device (rounded down to a multiple of the 8 XCDs): persistent GEMM work-groups run one per unit.
 int device_cu_count(int dev) {
   static int n_cu_on[MVIT_MAX_DEVICES] = {};
@@ -1119,14 +1101,14 @@ int launch_dl(const GemmParams& p, hipStream_t stream) {
 
 template <typename T, typename TO, bool TA, bool TB, int EPI>
 int launch_var(int var, const GemmParams& p, hipStream_t s) {
-  if constexpr (sizeof(T) == 2) {
+  {
     // direct-to-LDS main loop: v_mfma_f32_16x16x32_bf16 for the plain GEMMs with an operand behind the transposing
     // LDS read (weight gradients +6 %, input gradients +1 % on real data), v_mfma_f32_32x32x16_bf16 for the forward
     // GEMMs (both operands row-major: 3-5 % faster that way) and for the fused backward epilogues
     constexpr int NS = 4;
     if (var == 3) return (TB && EPI == MVIT_EPI_NONE) ? launch_dl<TO, TA, TB, EPI, NS, 8, true>(p, s) : launch_dl<TO, TA, TB, EPI, NS, 8>(p, s);
   }
-  return launch<T, TO, TA, TB, EPI, 1>(p, s);  // register-staged main loop: fp32, and bf16 operands whose row pitch exceeds 32-bit lane offsets
+  return launch<T, TO, TA, TB, EPI, 1>(p, s);  // register-staged main loop: operands whose row pitch exceeds 32-bit lane offsets
 }
 
 template <typename T, typename TO, bool TA, bool TB>
@@ -1400,7 +1382,17 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
     return dispatch_trans<bf16_t, float>(a->trans_a, a->trans_b, epi, var, p, s);
   }
   MVIT_REQUIRE(a->out_dtype == MVIT_F32, "gemm: fp32 operands need fp32 output");
-  return dispatch_trans<float, float>(a->trans_a, a->trans_b, epi, var, p, s);
+  const int rc = mvit_gemm_f32(a->trans_a, a->trans_b, epi, p, s);
+  if (rc != MVIT_OK) return rc;
+  if (p.split_k > 1) {
+    launch_splitk_reduce<float, float>(p, s);
+    MVIT_CHECK_LAUNCH("gemm split-k reduce");
+  }
+  if (p.colsum != nullptr) {
+    hipLaunchKernelGGL(tile_colsum_kernel, dim3((unsigned)((p.N + 255) / 256), (unsigned)tm, 2), 256, 0, s, static_cast<const float*>(p.C), p.ldc, p.M, p.N, p.aux_off, p.colsum);
+    MVIT_CHECK_LAUNCH("gemm column sums");
+  }
+  return MVIT_OK;
 }
 
 extern "C" int mvit_gemm_wgrad_split_k(int64_t out_rows, int64_t out_cols, int64_t k) {

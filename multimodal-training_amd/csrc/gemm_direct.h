@@ -25,6 +25,17 @@ __device__ __forceinline__ void pp_load_below(unsigned lds_addr, unsigned voff, 
       "global_load_lds_dwordx4 %2, %3\n\ts_mov_b64 exec, %0"
       : "=&s"(saved) : "s"(lds_addr), "v"(voff), "s"(base), "v"(k), "s"(limit) : "memory", "vcc", "scc");
 }
+// per-lane 64-bit addresses: 16 bytes per lane, and the same for the lanes with k < limit only
+__device__ __forceinline__ void pp_load_at(unsigned lds_addr, const char* addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_addr), "v"(addr) : "memory");
+}
+__device__ __forceinline__ void pp_load_at_below(unsigned lds_addr, const char* addr, int k, int limit) {
+  unsigned long long saved;
+  asm volatile(
+      "s_mov_b32 m0, %1\n\tv_cmp_gt_i32 vcc, %4, %3\n\ts_mov_b64 %0, exec\n\ts_and_b64 exec, exec, vcc\n\ts_nop 0\n\t"
+      "global_load_lds_dwordx4 %2, off\n\ts_mov_b64 exec, %0"
+      : "=&s"(saved) : "s"(lds_addr), "v"(addr), "v"(k), "s"(limit) : "memory", "vcc", "scc");
+}
 __device__ __forceinline__ void pp_load_dword_at(unsigned lds_addr, const char* addr) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(lds_addr), "v"(addr) : "memory");
 }

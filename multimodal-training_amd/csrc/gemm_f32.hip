@@ -1,0 +1,261 @@
+// fp32 GEMM (the parity path) on v_mfma_f32_16x16x4_f32:  C[M,N] = epi( sum_k A[m,k] * B[n,k] ).
+//
+// What bounds it is the fp32 matrix rate (157 TFLOP/s, a sixteenth of bf16's) once enough compute units have work: a
+// 64 x 64 tile per work-group of four waves keeps the matrix pipes of its unit busy (a K tile of 32 is 1,024 cycles of MFMA
+// and 16 KiB of operands), and 512 rows of the tower already give 160 to 1,700 of them.
+// K tiles of 32 floats (128-byte rows) in a ring of four LDS stages filled by direct global -> LDS loads, two work-groups
+// per compute unit.  MFMA (s, j) of a K tile contracts k = 16 s + 4 g + j over the lane groups g = 0..3, so one 16-byte read
+// of a [row][k] operand feeds four of them; a [k][row] operand is read as two neighbouring rows (8 bytes) per k, and the two
+// row blocks of a wave are its even and its odd rows.
+// The products are computed transposed (B's fragment first), so a lane ends with eight consecutive columns of a row and
+// stores them from registers.  One tile shape for every size: a row's result does not depend on its batch.
+#include "gemm_direct.h"
+
+namespace {
+
+template <int WGM_, int WGN_>
+struct F32Cfg {
+  static constexpr int BM = 64, BN = 64, BK = 32, NST = 4, NTHREADS = 256, WGM = WGM_, WGN = WGN_, WM = BM / WGM, WN = BN / WGN;
+  static constexpr int OPERAND = 64 * 128, STAGE = 2 * OPERAND, LDS = NST * STAGE;
+};
+
+// slot of chunk c (16 bytes) of row `major` ([row][k]: eight chunks) or k-row `major` ([k][row]: sixteen chunks)
+template <bool TR, bool IS_A>
+__device__ __forceinline__ int f32_swizzle(int major) {
+  if (TR) return ((major >> 2) & 1) << 3;
+  return IS_A ? (major >> 1) & 7 : ((major >> 1) & 1) | (((major >> 3) & 3) << 1);
+}
+
+template <bool TA, bool TB, int EPI>
+__global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmParams p) {
+  constexpr bool DUAL = (EPI == MVIT_EPI_SWIGLU);
+  using S = F32Cfg<DUAL ? 4 : 2, DUAL ? 1 : 2>;
+  constexpr int BK = S::BK, NST = S::NST, NA = S::WM / 16, NB = S::WN / 16, NG = DUAL ? 1 : NB / 2, NCOLS = DUAL ? 32 : 64;
+  static_assert(!(TA || TB) || (NA == 2 && NB == 2), "[k][row] operands are read as pairs of rows");
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+
+  const unsigned tiles = (unsigned)(p.tiles_m * p.tiles_n), total = tiles * (unsigned)p.split_k, per_xcd = (total + 7) / 8;
+  const unsigned work = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if ((blockIdx.x >> 3) >= per_xcd || work >= total) return;
+  const unsigned slice = p.split_k > 1 ? work / tiles : 0;
+  int tm, tn;
+  tile_coords(p, (int)(work - slice * tiles), tm, tn);
+  const int64_t m0 = (int64_t)tm * S::BM, n0 = (int64_t)tn * NCOLS;
+  const int64_t k_begin = (int64_t)slice * p.k_chunk;
+  const int64_t k_end = p.split_k > 1 ? (k_begin + p.k_chunk < p.K ? k_begin + p.k_chunk : p.K) : p.K;
+  const int klen = (int)(k_end - k_begin), n_kt = (klen + BK - 1) / BK, k_tail = klen % BK;
+
+  const int l = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wv / S::WGN, wn = wv % S::WGN;
+  const int i16 = l & 15, g4 = l >> 4;
+  typedef __attribute__((address_space(3))) unsigned char lds_byte;
+  const unsigned lds_base = (unsigned)(__UINTPTR_TYPE__)(lds_byte*)smem_raw;
+
+  // ---- loader: two 1 KiB loads per wave, operand and K tile
+  const char *pa[2], *pb[2];
+  int ka[2], kb[2];  // first k of the lane's chunk inside a K tile
+  const int64_t step_a = TA ? 4ll * BK * p.lda : 4 * BK, step_b = TB ? 4ll * BK * p.ldb : 4 * BK;
+  const int m_left = (int)(p.M - m0 < S::BM ? p.M - m0 : S::BM), n_left = (int)(p.N - n0 < NCOLS ? p.N - n0 : NCOLS);
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int q = wv * 2 + j;
+    auto place = [&](auto TR, auto IS_A, const void* X, int64_t ld, int64_t row0, int left, int row_of_tile, const char*& ptr, int& k) {
+      const float* x = static_cast<const float*>(X);
+      if (!decltype(TR)::value) {
+        const int c = (l & 7) ^ f32_swizzle<false, decltype(IS_A)::value>(q * 8 + (l >> 3));
+        const int r = row_of_tile < left ? row_of_tile : left - 1;  // rows past the edge repeat the last row: their results are not stored
+        k = c * 4;
+        ptr = reinterpret_cast<const char*>(x + (row0 + r) * ld + k_begin + k);
+      } else {
+        k = q * 4 + (l >> 4);
+        const int c = (l & 15) ^ f32_swizzle<true, decltype(IS_A)::value>(k);
+        ptr = reinterpret_cast<const char*>(x + (k_begin + k) * ld + row0 + (c * 4 < left ? c * 4 : 0));
+      }
+    };
+    const int row = q * 8 + (l >> 3);
+    place(std::bool_constant<TA>{}, std::true_type{}, p.A, p.lda, m0, m_left, row, pa[j], ka[j]);
+    // SWIGLU: tile rows 0-31 are gate rows, 32-63 up rows
+    place(std::bool_constant<TB>{}, std::false_type{}, DUAL && q >= 4 ? p.B2 : p.B, p.ldb, n0, n_left, DUAL ? row & 31 : row, pb[j], kb[j]);
+  }
+  auto issue = [&](int t, unsigned stage_off) {
+    const unsigned da = lds_base + stage_off + wv * 2048, db = da + S::OPERAND;
+    const bool partial = k_tail != 0 && t == n_kt - 1;  // chunks past the end of K are zeros
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if (partial) {
+        pp_load_at_below(da + j * 1024, pa[j], ka[j], k_tail);
+        pp_load_at_below(db + j * 1024, pb[j], kb[j], k_tail);
+        unsigned char* at = smem_raw + (da - lds_base) + j * 1024 + l * 16;
+        if (ka[j] >= k_tail) *reinterpret_cast<u32x4*>(at) = u32x4{0u, 0u, 0u, 0u};
+        if (kb[j] >= k_tail) *reinterpret_cast<u32x4*>(at + S::OPERAND) = u32x4{0u, 0u, 0u, 0u};
+      } else {
+        pp_load_at(da + j * 1024, pa[j]);
+        pp_load_at(db + j * 1024, pb[j]);
+      }
+      pa[j] += step_a;
+      pb[j] += step_b;
+    }
+    if (partial) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  };
+#pragma unroll
+  for (int t = 0; t < NST - 1; ++t)
+    if (t < n_kt) issue(t, t * S::STAGE);
+
+  // ---- fragment addresses (stage 0)
+  unsigned ra[2], rb[2];  // [row][k]: chunk 4 s + g of the lane's row; [k][row]: entry 0, k-row 4 g
+  if constexpr (!TA) {
+    const int row = wm * S::WM + i16, f = f32_swizzle<false, true>(row);
+    ra[0] = row * 128 + ((g4 ^ f) << 4);
+    ra[1] = row * 128 + (((4 + g4) ^ f) << 4);
+  } else {
+    const int r = wm * S::WM + 2 * i16;
+    ra[0] = ra[1] = 4 * g4 * 256 + (((r >> 2) ^ f32_swizzle<true, true>(4 * g4)) << 4) + (r & 3) * 4;
+  }
+  if constexpr (!TB) {
+    const int row = wn * S::WN + 8 * (i16 >> 2) + (i16 & 3), f = f32_swizzle<false, false>(row);
+    rb[0] = S::OPERAND + row * 128 + ((g4 ^ f) << 4);
+    rb[1] = S::OPERAND + row * 128 + (((4 + g4) ^ f) << 4);
+  } else {
+    const int r = wn * S::WN + 2 * i16;
+    rb[0] = rb[1] = S::OPERAND + 4 * g4 * 256 + (((r >> 2) ^ f32_swizzle<true, false>(4 * g4)) << 4) + (r & 3) * 4;
+  }
+
+  f32x4 acc[NA][NB];
+#pragma unroll
+  for (int a = 0; a < NA; ++a)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  unsigned st = 0, st_in = (NST - 1) * S::STAGE;  // stage consumed, stage filled
+  for (int t = 0; t < n_kt; ++t) {
+    const int newer = n_kt - 1 - t;  // K tiles that may still be in flight
+    if (newer >= 2) pp_wait_vm<8>();
+    else if (newer == 1) pp_wait_vm<4>();
+    else pp_wait_vm<0>();
+    pp_barrier();  // every wave's share of K tile t is in LDS; K tile t - 1 has been consumed
+    if (t + NST - 1 < n_kt) issue(t + NST - 1, st_in);
+    const unsigned char* at = smem_raw + st;
+    float fa[NA][8], fb[NB][8];  // [block][4 s + j]
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      if constexpr (!TA) {
+#pragma unroll
+        for (int a = 0; a < NA; ++a) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(at + ra[s] + a * 2048);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) fa[a][4 * s + j] = v[j];
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const f32x2 v = *reinterpret_cast<const f32x2*>(at + ra[0] + (16 * s + j) * 256);
+          fa[0][4 * s + j] = v[0];
+          fa[NA - 1][4 * s + j] = v[1];
+        }
+      }
+      if constexpr (!TB) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(at + rb[s] + (b >> 1) * 4096 + (b & 1) * 512);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) fb[b][4 * s + j] = v[j];
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const f32x2 v = *reinterpret_cast<const f32x2*>(at + rb[0] + (16 * s + j) * 256);
+          fb[0][4 * s + j] = v[0];
+          fb[NB - 1][4 * s + j] = v[1];
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+#pragma unroll
+      for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[b][k], fa[a][k], acc[a][b], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    st = st + S::STAGE == S::LDS ? 0 : st + S::STAGE;
+    st_in = st_in + S::STAGE == S::LDS ? 0 : st_in + S::STAGE;
+  }
+
+  // ---- epilogue: the lane holds columns 8 g .. 8 g + 7 of each 32-column group, one row per row block
+  const bool to_ws = (EPI == MVIT_EPI_NONE) && p.split_k > 1;
+  const bool vec = to_ws ? (p.N % 4 == 0) : p.vec_ok != 0;
+  float* ws = to_ws ? p.workspace + (int64_t)slice * p.M * p.N : nullptr;
+  float no_cs[16];
+#pragma unroll
+  for (int a = 0; a < NA; ++a)
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const int64_t m = m0 + wm * S::WM + (TA ? 2 * i16 + a : a * 16 + i16), n = n0 + (DUAL ? 0 : wn * S::WN) + g * 32 + 8 * g4;
+      if (m >= p.M || n >= p.N) continue;
+      float v[8], u[8];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        v[TB ? 2 * r : r] = acc[a][2 * g][r];
+        v[TB ? 2 * r + 1 : 4 + r] = acc[a][2 * g + 1][r];
+        if (DUAL) {
+          u[r] = acc[a][NB - 2][r];
+          u[4 + r] = acc[a][NB - 1][r];
+        }
+      }
+      if (to_ws) {
+        float* w = ws + m * p.N + n;
+        if (vec && n + 8 <= p.N) store8_cached(w, v);
+        else
+          for (int e = 0; e < 8 && n + e < p.N; ++e) w[e] = v[e];
+      } else {
+        emit8<float, float, EPI>(p, m, n, v, u, vec, no_cs, false);
+      }
+    }
+}
+
+template <bool TA, bool TB, int EPI>
+int launch_f32(GemmParams p, hipStream_t stream) {
+  constexpr int NCOLS = EPI == MVIT_EPI_SWIGLU ? 32 : 64;
+  const int64_t tm = (p.M + 63) / 64, tn = (p.N + NCOLS - 1) / NCOLS;
+  MVIT_REQUIRE(tm * tn * p.split_k < (1ll << 30), "gemm: too many tiles");
+  p.tiles_m = (int)tm; p.tiles_n = (int)tn;
+  p.panel_w = tn <= 6 ? (int)tn : 4;
+  hipLaunchKernelGGL((gemm_f32_kernel<TA, TB, EPI>), (p.tiles_m * p.tiles_n * p.split_k + 7) / 8 * 8, 256, (F32Cfg<2, 2>::LDS), stream, p);
+  MVIT_CHECK_LAUNCH("gemm");
+  return MVIT_OK;
+}
+
+}  // namespace
+
+int mvit_gemm_f32(int ta, int tb, int epi, const GemmParams& p, hipStream_t s) {
+  if (!ta && !tb) {
+    switch (epi) {
+      case MVIT_EPI_NONE: return launch_f32<false, false, MVIT_EPI_NONE>(p, s);
+      case MVIT_EPI_BIAS: return launch_f32<false, false, MVIT_EPI_BIAS>(p, s);
+      case MVIT_EPI_BIAS_RES: return launch_f32<false, false, MVIT_EPI_BIAS_RES>(p, s);
+      case MVIT_EPI_BIAS_GELU: return launch_f32<false, false, MVIT_EPI_BIAS_GELU>(p, s);
+      case MVIT_EPI_SWIGLU: return launch_f32<false, false, MVIT_EPI_SWIGLU>(p, s);
+      case MVIT_EPI_ACCUM: return launch_f32<false, false, MVIT_EPI_ACCUM>(p, s);
+      default: break;
+    }
+  } else if (!ta && tb) {
+    switch (epi) {
+      case MVIT_EPI_NONE: return launch_f32<false, true, MVIT_EPI_NONE>(p, s);
+      case MVIT_EPI_BIAS: return launch_f32<false, true, MVIT_EPI_BIAS>(p, s);
+      case MVIT_EPI_SWIGLU_BWD: return launch_f32<false, true, MVIT_EPI_SWIGLU_BWD>(p, s);
+      case MVIT_EPI_GELU_BWD: return launch_f32<false, true, MVIT_EPI_GELU_BWD>(p, s);
+      case MVIT_EPI_ACCUM: return launch_f32<false, true, MVIT_EPI_ACCUM>(p, s);
+      default: break;
+    }
+  } else if (ta && tb) {
+    switch (epi) {
+      case MVIT_EPI_NONE: return launch_f32<true, true, MVIT_EPI_NONE>(p, s);
+      case MVIT_EPI_BIAS: return launch_f32<true, true, MVIT_EPI_BIAS>(p, s);
+      case MVIT_EPI_ACCUM: return launch_f32<true, true, MVIT_EPI_ACCUM>(p, s);
+      default: break;
+    }
+  } else {
+    return mvit_set_error(MVIT_ERR_UNSUPPORTED, "gemm: trans_a=1, trans_b=0 is not built");
+  }
+  return mvit_set_error(MVIT_ERR_UNSUPPORTED, "gemm: epilogue %d not built for trans_a=%d trans_b=%d", epi, ta, tb);
+}

@@ -299,7 +299,7 @@ def _block_backward(dx2: torch.Tensor, x: torch.Tensor, saved: tuple, W: BlockWe
     g_bd = off_chain(lambda: (ops.colsum(dx2, gdt["mlp.down_proj.bias"]), wgrad(dx2, h, g_wd, n=I))[0])
     dgu = torch.empty(S, 2 * Ipad, dtype=x.dtype, device=dev)
     # with many rows the epilogue also hands back per-tile column sums of dgu: the gate / up bias gradient without re-reading dgu
-    fused = x.dtype != torch.bfloat16 or ops.swiglu_bwd_sums_columns(S, Ipad, C)
+    fused = x.dtype == torch.bfloat16 and ops.swiglu_bwd_sums_columns(S, Ipad, C)
     part = torch.empty(-(-S // 256), 2 * Ipad, dtype=torch.float32, device=dev) if fused else None
     ops.gemm(dx2, W.wdown, dgu, trans_b=True, epilogue=E.EPI_SWIGLU_BWD, residual=gu, aux_off=Ipad, colsum_partial=part)
     g_wgu = torch.empty(2 * Ipad, C, dtype=gdt["mlp.gate_proj.weight"], device=dev)
