@@ -111,6 +111,16 @@ int mvit_gather_rows(const void* src, const int64_t* index, void* dst, int64_t n
 int mvit_segment_copy(const void* src, void* dst, const int64_t* desc, int64_t nseg, int64_t max_seg_rows,
                       int64_t row_bytes, mvit_stream_t stream);
 
+/* Copies of contiguous byte ranges on the device, all in one launch (the list is in host memory and travels with it; ranges
+ * must not overlap).  Bit-exact.  The same replacements as mvit_segment_copy, whose segments are such ranges, for callers
+ * that hold the list on the host; ranges may have different sources and destinations. */
+typedef struct mvit_copy_range {
+  const void* src;
+  void* dst;
+  int64_t bytes;
+} mvit_copy_range;
+int mvit_copy_ranges(const mvit_copy_range* ranges, int n_ranges, mvit_stream_t stream);
+
 /* pack [sum len, row] -> padded [B, pad_len, row] filled with `pad_value` past each sample's length,
  * plus mask [B, pad_len] (uint8 0/1).  lens, offsets: device int64 [B].  elem_size 2 or 4; pad_bits is
  * the bit pattern of the pad value in that element type.  Replaces pad_pack_to_batch, spu:300-327. */
@@ -266,7 +276,8 @@ int mvit_block_bwd(const mvit_block_args* args, mvit_stream_t stream);
 /* Ranks the image placeholders of a token sequence: rank[t] = k (0-based) if input_ids[t] is the k-th entry equal
  * to image_token_id, else -1; positions[k] = t; counts[0] = number of placeholders; counts[1] = number of
  * placeholders whose label differs from ignore_label (0 when labels is null).  All device pointers; rank
- * [n_tokens] int32, positions [n_tokens] int64 (first counts[0] entries written), counts [2] int64.
+ * [n_tokens] int32, positions [n_tokens] int64 (first counts[0] entries written; may be null), counts [2] int64 (device
+ * memory, or pinned host memory that the device can write).
  * Replaces the mask building and the counting guards of TextTrainer's forward, python/ray/text.py:883-910. */
 int mvit_image_token_ranks(const int64_t* input_ids, const int64_t* labels, int64_t n_tokens, int64_t image_token_id,
                            int64_t ignore_label, int32_t* rank, int64_t* positions, int64_t* counts,
@@ -279,6 +290,11 @@ int mvit_image_token_ranks(const int64_t* input_ids, const int64_t* labels, int6
  * (text.py:1000-1019) is mvit_gather_rows(grad, positions, ...). */
 int mvit_merge_rows(const void* embeds, const void* vision, const int32_t* rank, void* merged, int64_t n_tokens,
                     int64_t n_vision, int64_t row_bytes, mvit_stream_t stream);
+
+/* Both gradients of that merge in one pass over grad [n_tokens]: rows with 0 <= rank < n_vision go to vision[rank] and leave a
+ * zero row in text, the others go to text.  Either output may be null.  (text.py:1000-1019 and the autograd of :913.) */
+int mvit_split_rows(const void* grad, const int32_t* rank, void* text, void* vision, int64_t n_tokens, int64_t n_vision,
+                    int64_t row_bytes, mvit_stream_t stream);
 
 /* ---------------------------------------------------------------- optimizer step (multi-tensor) */
 
@@ -368,6 +384,9 @@ typedef struct mvit_image {
  * model dtype is the one of the tower's first line (modeling_qwen2_5_vl.py, patch_embed input). */
 int mvit_patchify(const mvit_image* images, int n_images, int64_t total_rows, void* out, double rescale, float mean_r,
                   float mean_g, float mean_b, float std_r, float std_g, float std_b, int dtype, mvit_stream_t stream);
+/* The same with the table in host memory, at most 64 images (MVIT_ERR_UNSUPPORTED beyond): it travels with the launch. */
+int mvit_patchify_host_table(const mvit_image* images, int n_images, int64_t total_rows, void* out, double rescale, float mean_r,
+                             float mean_g, float mean_b, float std_r, float std_g, float std_b, int dtype, mvit_stream_t stream);
 
 /* The patch embedding straight from decoded frames: out[r, :] = row r of pixel_values (exactly the bf16 rows that
  * mvit_patchify makes for the same table and constants) x weight^T, bf16 MFMA with fp32 accumulation, without the
@@ -403,6 +422,16 @@ int mvit_patch_embed_frames(const mvit_image* images, int n_images, int64_t tota
  * own fixed-size BILINEAR resize (python/data/preprocessing.py:126-131) and the BICUBIC resize to the smart_resize
  * target inside the image processor (transformers 4.57.0 Qwen2VLImageProcessor, reached through
  * processor.apply_chat_template, python/data/preprocessing.py:134). */
+typedef struct mvit_resample_job { /* one pass: the arguments of mvit_resample_u8 */
+  const uint8_t* src;
+  uint8_t* dst;
+  const int32_t *bounds, *kk;
+  int64_t outer, in_len, out_len, inner;
+  int32_t ksize, reserved;
+} mvit_resample_job;
+/* Independent passes together (`jobs` in host memory): the horizontal passes of all images of a batch in one launch, and
+ * their vertical passes in another. */
+int mvit_resample_u8_batch(const mvit_resample_job* jobs, int n_jobs, mvit_stream_t stream);
 int mvit_resample_u8(const uint8_t* src, uint8_t* dst, int64_t outer, int64_t in_len, int64_t out_len, int64_t inner,
                      const int32_t* bounds, const int32_t* kk, int ksize, mvit_stream_t stream);
 

@@ -9,6 +9,7 @@
 // Qwen2VLImageProcessor._preprocess: rescale in float64 rounded to float32, then (x - mean) / std in float32
 // with an IEEE division), so fp32 results can be compared bit for bit with a numpy restatement.
 #include "mvit_common.h"
+#include <string.h>
 
 namespace {
 
@@ -42,9 +43,13 @@ constexpr int SQ = 2 * PATCH;          // a merge block is a square of 28 x 28 p
 constexpr int SQ_LINE = SQ * 3;        // 84 bytes (21 dwords) per line of the square
 constexpr int SQ_DWORDS = SQ * SQ_LINE / 4;  // 588
 
+// The image table travels as a kernel argument when it is short (no copy to the device in front of the launch).
+constexpr int TABLE_ARG_IMAGES = 64;
+struct TableArg {
+  mvit_image im[TABLE_ARG_IMAGES + 1];
+};
 template <typename TO>
-__global__ __launch_bounds__(256) void patchify_kernel(const mvit_image* __restrict__ images, int n_images, TO* __restrict__ out,
-                                                       int64_t total_rows, Norm nm) {
+__device__ __forceinline__ void patchify_block(const mvit_image* images, int n_images, TO* __restrict__ out, int64_t total_rows, const Norm& nm) {
 #pragma clang fp contract(off)
   // a byte has 256 values: the work-group computes the result for each of them and each channel once (exact
   // arithmetic, three divisions per thread) and every element of its rows is then a byte read and a table lookup
@@ -105,6 +110,14 @@ __global__ __launch_bounds__(256) void patchify_kernel(const mvit_image* __restr
     store4(dst + (c * TPS + 1) * PLANE + 4 * q, v1);
   }
 }
+template <typename TO>
+__global__ __launch_bounds__(256) void patchify_kernel(const mvit_image* __restrict__ images, int n_images, TO* __restrict__ out, int64_t total_rows, Norm nm) {
+  patchify_block<TO>(images, n_images, out, total_rows, nm);
+}
+template <typename TO>
+__global__ __launch_bounds__(256) void patchify_arg_kernel(const TableArg images, int n_images, TO* __restrict__ out, int64_t total_rows, Norm nm) {
+  patchify_block<TO>(images.im, n_images, out, total_rows, nm);
+}
 
 }  // namespace
 // A window as the kernels use it: first tap and tap count forced into the table's row (ksize entries) and into the
@@ -125,187 +138,175 @@ __device__ __forceinline__ TapWindow tap_window(const int32_t* __restrict__ boun
 // Pillow's 8-bit arithmetic (libImaging/Resample.c, ImagingResampleHorizontal_8bpc / Vertical_8bpc): per output
 // coordinate a window of `bounds[2*x + 1]` input coordinates starting at `bounds[2*x]`, 22-bit fixed-point weights
 // kk[x * ksize + i], an accumulator that starts at one half, an arithmetic shift and a clamp to 0..255.
-// A thread makes four consecutive output bytes of one output coordinate (inner is the contiguous dimension: pixels
-// times channels for the vertical pass, 3 channels for the horizontal one) or, when inner is not a multiple of four,
-// four consecutive bytes of the flattened [out_len * inner] row, each with its own window.
+// inner is the contiguous dimension: pixels times channels for the vertical pass, 3 channels for the horizontal one.  The
+// kernels for those two follow; this one, a thread per output byte, takes everything else.
 constexpr int RESAMPLE_PRECISION_BITS = 22;
 __device__ __forceinline__ unsigned clip8(int v) {
   v >>= RESAMPLE_PRECISION_BITS;
+  // keeps the compiler from pairing shift and clamp into v_ashr_pk_u8_i32: it takes the upper half of that instruction's result
+  // for zero, and the hardware leaves the old bits there
+  asm("" : "+v"(v));
   return (unsigned)(v < 0 ? 0 : (v > 255 ? 255 : v));
 }
-template <bool WIDE>  // WIDE: inner % 4 == 0 and 4-byte aligned rows, the four bytes share one window
 __global__ __launch_bounds__(256) void resample_pass_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, int64_t outer,
                                                             int64_t in_len, int64_t out_len, int64_t inner,
                                                             const int32_t* __restrict__ bounds, const int32_t* __restrict__ kk, int ksize) {
   const int64_t row_out = out_len * inner, row_in = in_len * inner;
-  const int64_t quads = (row_out + 3) / 4;
-  const int64_t total = outer * quads;
+  const int64_t total = outer * row_out;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-    const int64_t o = i / quads, q = i % quads;
-    const uint8_t* s = src + o * row_in;
-    uint8_t* d = dst + o * row_out + 4 * q;
-    if (WIDE) {
-      const int64_t x = (4 * q) / inner, c = (4 * q) % inner;
-      const TapWindow tw = tap_window(bounds, x, ksize, in_len);
-      const int xmin = tw.xmin, n = tw.n;
-      const int32_t* k = kk + x * ksize;
-      int a0 = 1 << (RESAMPLE_PRECISION_BITS - 1), a1 = a0, a2 = a0, a3 = a0;
-      for (int t = 0; t < n; ++t) {
-        const unsigned w = *reinterpret_cast<const unsigned*>(s + (int64_t)(xmin + t) * inner + c);
-        const int kt = k[t];
-        a0 += (int)(w & 0xff) * kt;
-        a1 += (int)((w >> 8) & 0xff) * kt;
-        a2 += (int)((w >> 16) & 0xff) * kt;
-        a3 += (int)(w >> 24) * kt;
-      }
-      *reinterpret_cast<unsigned*>(d) = clip8(a0) | (clip8(a1) << 8) | (clip8(a2) << 16) | (clip8(a3) << 24);
-    } else {
-      for (int b = 0; b < 4; ++b) {
-        const int64_t e = 4 * q + b;
-        if (e >= row_out) break;
-        const int64_t x = e / inner, c = e % inner;
-        const TapWindow tw = tap_window(bounds, x, ksize, in_len);
-      const int xmin = tw.xmin, n = tw.n;
-        const int32_t* k = kk + x * ksize;
-        int a = 1 << (RESAMPLE_PRECISION_BITS - 1);
-        for (int t = 0; t < n; ++t) a += (int)s[(int64_t)(xmin + t) * inner + c] * k[t];
-        d[b] = (uint8_t)clip8(a);
-      }
-    }
+    const int64_t o = i / row_out, e = i % row_out, x = e / inner, c = e % inner;
+    const TapWindow tw = tap_window(bounds, x, ksize, in_len);
+    const int32_t* k = kk + x * ksize;
+    int a = 1 << (RESAMPLE_PRECISION_BITS - 1);
+    for (int t = 0; t < tw.n; ++t) a += (int)src[o * row_in + (int64_t)(tw.xmin + t) * inner + c] * k[t];
+    dst[i] = (uint8_t)clip8(a);
   }
 }
 
-// The same pass for a short contiguous dimension (the horizontal pass: inner = channels): neighbouring output bytes have
-// different windows and every tap is a single byte, so a work-group first copies its input row into LDS with aligned
-// 4-byte loads and then reads the taps from there.  One work-group per row of the outer dimension; a thread makes whole
-// pixels (up to four channels).
-constexpr int RESAMPLE_LDS_BYTES = 60 * 1024, RESAMPLE_MAX_CHANNELS = 4;
-__global__ __launch_bounds__(256) void resample_rows_lds_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, int64_t outer,
-                                                                int64_t in_len, int64_t out_len, int inner,
-                                                                const int32_t* __restrict__ bounds, const int32_t* __restrict__ kk, int ksize) {
-  __shared__ __attribute__((aligned(16))) uint8_t row[RESAMPLE_LDS_BYTES + 8];
-  const int64_t row_in = in_len * inner, row_out = out_len * inner;
-  const uint8_t* src_end = src + outer * row_in;
-  for (int64_t o = blockIdx.x; o < outer; o += gridDim.x) {
-    const uint8_t* b = src + o * row_in;
-    const int lead = (int)((uintptr_t)b & 3);  // the row starts `lead` bytes into an aligned word
-    const uint8_t* a = b - lead;
-    const int words = (int)((lead + row_in + 3) / 4);
-    __syncthreads();  // the previous row has been consumed
-    for (int j = threadIdx.x; j < words; j += 256) {
-      const uint8_t* g = a + 4 * j;
-      unsigned w;
-      if (g >= src && g + 4 <= src_end) {
-        w = *reinterpret_cast<const unsigned*>(g);
-      } else {  // first / last word of the array: only the bytes that belong to it
-        w = 0;
+// ---- several passes in one launch
+constexpr int RESAMPLE_MAX_JOBS = 32;
+struct ResampleJobs {
+  int n;
+  int first_block[RESAMPLE_MAX_JOBS];
+  mvit_resample_job job[RESAMPLE_MAX_JOBS];
+};
+__device__ __forceinline__ int resample_job_of(const ResampleJobs& jobs, int block) {
+  int j = 0;
+  while (j + 1 < jobs.n && block >= jobs.first_block[j + 1]) ++j;
+  return j;
+}
+// A weight that fits 24 bits is multiplied with one full-rate multiply-add (v_mad_i32_i24); the 22-bit weights of a
+// resampling always do, tables of the caller's own need not.  The low 32 bits are the same either way.
+__device__ __forceinline__ bool fits24(int k) { return k < (1 << 23) && k >= -(1 << 23); }
+template <bool FAST>
+__device__ __forceinline__ int tap(int acc, unsigned byte, int k) {
+  return acc + (int)byte * (FAST ? (int)((unsigned)k << 8) >> 8 : k);  // the shifts tell the compiler that 24 bits suffice
+}
+
+// The pass for a short contiguous dimension (the horizontal pass: inner = channels).  A wave makes 64 consecutive output
+// coordinates of RESAMPLE_ROWS rows: a thread holds 16 weights of its window in registers at a time and applies them to every
+// row, whose 16 taps are INNER unaligned 16-byte loads (neighbouring windows overlap and are served by the L1), so there is no
+// staging and no barrier.  Bound by the multiply-adds and by the L1; with full-width multiplies (16 cycles each) and single
+// bytes from LDS the four photographs of 1080 x 1920 ... 2448 x 3264 took 300 us.
+constexpr int RESAMPLE_ROWS = 8, RESAMPLE_TAPS = 16, RESAMPLE_MAX_CHANNELS = 4;
+template <int INNER, bool FAST>
+__device__ __forceinline__ void resample_narrow_rows(const uint8_t* p, int64_t row_in, int rows, const uint8_t* src_end, const int (&k)[RESAMPLE_TAPS],
+                                                     int (&acc)[RESAMPLE_ROWS][INNER]) {
+  typedef __attribute__((address_space(1))) const uint8_t* global_bytes;
+#pragma unroll
+  for (int r = 0; r < RESAMPLE_ROWS; ++r) {
+    if (r >= rows) break;
+    const uint8_t* q = p + r * row_in;
+    unsigned w[4 * INNER];
+    if (q + RESAMPLE_TAPS * INNER <= src_end) {
+#pragma unroll
+      for (int i = 0; i < INNER; ++i) __builtin_memcpy(w + 4 * i, (global_bytes)(uintptr_t)(q + 16 * i), 16);
+    } else {  // the end of the array: only the bytes that belong to it
+#pragma unroll
+      for (int i = 0; i < 4 * INNER; ++i) {
+        w[i] = 0;
+#pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (g + e >= src && g + e < src_end) w |= (unsigned)g[e] << (8 * e);
+          if (q + 4 * i + e < src_end) w[i] |= (unsigned)q[4 * i + e] << (8 * e);
       }
-      *reinterpret_cast<unsigned*>(row + 4 * j) = w;
     }
-    __syncthreads();
-    const uint8_t* r = row + lead;
-    uint8_t* d = dst + o * row_out;
-    // a thread makes whole pixels: the channels of a pixel share its window and its weights
-    for (int x = threadIdx.x; x < (int)out_len; x += 256) {
-      const TapWindow tw = tap_window(bounds, x, ksize, in_len);
-      const int xmin = tw.xmin, n = tw.n;
-      const int32_t* k = kk + (int64_t)x * ksize;
-      int acc[RESAMPLE_MAX_CHANNELS];
 #pragma unroll
-      for (int c = 0; c < RESAMPLE_MAX_CHANNELS; ++c) acc[c] = 1 << (RESAMPLE_PRECISION_BITS - 1);
-      const uint8_t* px = r + xmin * inner;
-      for (int t = 0; t < n; ++t) {
-        const int kt = k[t];
+    for (int t = 0; t < RESAMPLE_TAPS; ++t)
 #pragma unroll
-        for (int c = 0; c < RESAMPLE_MAX_CHANNELS; ++c)
-          if (c < inner) acc[c] += (int)px[c] * kt;
-        px += inner;
-      }
+      for (int c = 0; c < INNER; ++c) acc[r][c] = tap<FAST>(acc[r][c], (w[(t * INNER + c) / 4] >> (8 * ((t * INNER + c) & 3))) & 0xffu, k[t]);
+  }
+}
+template <int INNER>
+__global__ __launch_bounds__(256) void resample_narrow_kernel(const ResampleJobs jobs) {
+  const int j = resample_job_of(jobs, blockIdx.x);
+  const mvit_resample_job& jb = jobs.job[j];
+  const int block = blockIdx.x - jobs.first_block[j], lane = threadIdx.x & 63;
+  const int in_len = (int)jb.in_len, out_len = (int)jb.out_len, ksize = jb.ksize;
+  const int xblocks = (out_len + 63) / 64, xb = block % xblocks;
+  const int64_t o0 = ((int64_t)(block / xblocks) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * RESAMPLE_ROWS;
+  if (o0 >= jb.outer) return;
+  const int rows = jb.outer - o0 < RESAMPLE_ROWS ? (int)(jb.outer - o0) : RESAMPLE_ROWS;
+  const bool mine = xb * 64 + lane < out_len;
+  const int x = mine ? xb * 64 + lane : out_len - 1;
+  const int64_t row_in = (int64_t)in_len * INNER, row_out = (int64_t)out_len * INNER;
+  const uint8_t* src_end = jb.src + jb.outer * row_in;
+  const TapWindow tw = tap_window(jb.bounds, x, ksize, in_len);
+  int acc[RESAMPLE_ROWS][INNER];
 #pragma unroll
-      for (int c = 0; c < RESAMPLE_MAX_CHANNELS; ++c)
-        if (c < inner) d[x * inner + c] = (uint8_t)clip8(acc[c]);
+  for (int r = 0; r < RESAMPLE_ROWS; ++r)
+#pragma unroll
+    for (int c = 0; c < INNER; ++c) acc[r][c] = 1 << (RESAMPLE_PRECISION_BITS - 1);
+  for (int t0 = 0; t0 < ksize; t0 += RESAMPLE_TAPS) {
+    if (!__any(t0 < tw.n)) break;
+    int k[RESAMPLE_TAPS];
+    bool narrow = true;
+#pragma unroll
+    for (int t = 0; t < RESAMPLE_TAPS; ++t) {
+      k[t] = t0 + t < tw.n ? jb.kk[(int64_t)x * ksize + t0 + t] : 0;  // taps past the window have weight 0
+      narrow = narrow && fits24(k[t]);
+    }
+    const uint8_t* p = jb.src + o0 * row_in + (int64_t)(tw.xmin + (t0 < tw.n ? t0 : 0)) * INNER;
+    if (__all(narrow)) resample_narrow_rows<INNER, true>(p, row_in, rows, src_end, k, acc);
+    else resample_narrow_rows<INNER, false>(p, row_in, rows, src_end, k, acc);
+  }
+  // four pixels of three channels leave as three words, each made by one lane from its own and its neighbour's bytes
+  const bool words = INNER == 3 && out_len % 4 == 0 && (reinterpret_cast<uintptr_t>(jb.dst) & 3u) == 0;
+#pragma unroll
+  for (int r = 0; r < RESAMPLE_ROWS; ++r) {
+    if (r >= rows) break;
+    uint8_t* d = jb.dst + (o0 + r) * row_out;
+    if (words) {
+      const unsigned v = clip8(acc[r][0]) | (clip8(acc[r][INNER > 1 ? 1 : 0]) << 8) | (clip8(acc[r][INNER > 2 ? 2 : 0]) << 16);
+      const unsigned next = __shfl_down(v, 1, 64);
+      const int q = lane & 3;
+      if (mine && q < 3) *reinterpret_cast<unsigned*>(d + (x - q) * 3 + 4 * q) = (v >> (8 * q)) | (next << (24 - 8 * q));
+    } else if (mine) {
+#pragma unroll
+      for (int c = 0; c < INNER; ++c) d[(int64_t)x * INNER + c] = (uint8_t)clip8(acc[r][c]);
     }
   }
 }
 
-// The horizontal pass again, for windows of at most RESAMPLE_KMAX taps: a work-group owns 256 consecutive output
-// coordinates and a strip of rows.  A thread keeps its coordinate's window and weights in registers for the whole strip
-// (they are the same for every row, and fetching them per row was most of the row kernel's time); per row the
-// work-group stages just the input bytes its 256 windows cover (two LDS buffers, one barrier per row) and every thread
-// makes one pixel.  A work-group whose windows cover more than the LDS buffer (windows are the caller's) reads its taps
-// from global memory instead.
-constexpr int RESAMPLE_KMAX = 16, RESAMPLE_SPAN_BYTES = 8 * 1024;
-__global__ __launch_bounds__(256) void resample_cols_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, int64_t outer,
-                                                            int64_t in_len, int64_t out_len, int inner, const int32_t* __restrict__ bounds,
-                                                            const int32_t* __restrict__ kk, int ksize, int rows_per_group) {
-  __shared__ __attribute__((aligned(16))) uint8_t buf[2][RESAMPLE_SPAN_BYTES + 8];
-  const int64_t row_in = in_len * inner, row_out = out_len * inner;
-  const uint8_t* src_end = src + outer * row_in;
-  const int x_first = blockIdx.x * 256, x_last = min(x_first + 255, (int)out_len - 1);
-  const bool mine = x_first + (int)threadIdx.x <= x_last;
-  const int x = mine ? x_first + (int)threadIdx.x : x_last;
-  const TapWindow tw = tap_window(bounds, x, ksize, in_len);
-      const int xmin = tw.xmin, n = tw.n;
-  int k[RESAMPLE_KMAX];
+// The pass for a long contiguous dimension of whole words (the vertical pass): the window and its weights are the same for a
+// whole output row, so they are read once per work-group, and a thread makes four consecutive bytes.
+template <bool FAST>
+__device__ __forceinline__ unsigned resample_wide_word(const uint8_t* p, int64_t inner, int n, const int32_t* __restrict__ k) {
+  int a[4];
 #pragma unroll
-  for (int t = 0; t < RESAMPLE_KMAX; ++t) k[t] = t < n ? kk[(int64_t)x * ksize + t] : 0;
-  // bytes of a row that the work-group's windows cover (window starts and ends do not decrease with the coordinate
-  // for a resampling; anything else shows up as a span that does not fit and takes the global path)
-  int lo = bounds[2 * x_first] * inner, hi = (bounds[2 * x_last] + bounds[2 * x_last + 1]) * inner;
-  bool fits = hi - lo + 4 <= RESAMPLE_SPAN_BYTES && xmin * inner >= lo && (xmin + n) * inner <= hi;
-  fits = __syncthreads_and(fits);
-  const int64_t o_begin = (int64_t)blockIdx.y * rows_per_group, o_end = min(o_begin + rows_per_group, outer);
-  for (int64_t o = o_begin; o < o_end; ++o) {
-    int acc[RESAMPLE_MAX_CHANNELS];
+  for (int e = 0; e < 4; ++e) a[e] = 1 << (RESAMPLE_PRECISION_BITS - 1);
+  int t = 0;
+  for (; t + 4 <= n; t += 4) {
+    unsigned w[4];
 #pragma unroll
-    for (int c = 0; c < RESAMPLE_MAX_CHANNELS; ++c) acc[c] = 1 << (RESAMPLE_PRECISION_BITS - 1);
-    if (fits) {
-      const uint8_t* b = src + o * row_in + lo;
-      const int lead = (int)((uintptr_t)b & 3);
-      const uint8_t* a = b - lead;
-      const int words = (lead + (hi - lo) + 3) / 4;
-      uint8_t* stage = buf[o & 1];
-      for (int j = threadIdx.x; j < words; j += 256) {
-        const uint8_t* g = a + 4 * j;
-        unsigned w;
-        if (g >= src && g + 4 <= src_end) {
-          w = *reinterpret_cast<const unsigned*>(g);
-        } else {  // first / last word of the array: only the bytes that belong to it
-          w = 0;
-          for (int e = 0; e < 4; ++e)
-            if (g + e >= src && g + e < src_end) w |= (unsigned)g[e] << (8 * e);
-        }
-        *reinterpret_cast<unsigned*>(stage + 4 * j) = w;
-      }
-      __syncthreads();  // also: every thread is done with the buffer of two rows ago
-      const uint8_t* px = stage + lead + (xmin * inner - lo);
+    for (int i = 0; i < 4; ++i) w[i] = *reinterpret_cast<const unsigned*>(p + (int64_t)(t + i) * inner);
 #pragma unroll
-      for (int t = 0; t < RESAMPLE_KMAX; ++t) {
-        if (t >= ksize) break;
-        const uint8_t* q = px + max(min(t, n - 1), 0) * inner;  // taps past the window have weight 0 and re-read its last one
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int c = 0; c < RESAMPLE_MAX_CHANNELS; ++c)
-          if (c < inner) acc[c] += (int)q[c] * k[t];
-      }
-    } else {
-      const uint8_t* px = src + o * row_in + (int64_t)xmin * inner;
-#pragma unroll
-      for (int t = 0; t < RESAMPLE_KMAX; ++t) {
-        if (t >= n) break;
-#pragma unroll
-        for (int c = 0; c < RESAMPLE_MAX_CHANNELS; ++c)
-          if (c < inner) acc[c] += (int)px[t * inner + c] * k[t];
-      }
-    }
-    if (mine) {
-      uint8_t* d = dst + o * row_out + (int64_t)x * inner;
-#pragma unroll
-      for (int c = 0; c < RESAMPLE_MAX_CHANNELS; ++c)
-        if (c < inner) d[c] = (uint8_t)clip8(acc[c]);
-    }
+      for (int e = 0; e < 4; ++e) a[e] = tap<FAST>(a[e], (w[i] >> (8 * e)) & 0xffu, k[t + i]);
   }
+  for (; t < n; ++t) {
+    const unsigned w = *reinterpret_cast<const unsigned*>(p + (int64_t)t * inner);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) a[e] = tap<FAST>(a[e], (w >> (8 * e)) & 0xffu, k[t]);
+  }
+  return clip8(a[0]) | (clip8(a[1]) << 8) | (clip8(a[2]) << 16) | (clip8(a[3]) << 24);
+}
+__global__ __launch_bounds__(256) void resample_wide_kernel(const ResampleJobs jobs) {
+  const int j = resample_job_of(jobs, blockIdx.x);
+  const mvit_resample_job& jb = jobs.job[j];
+  const int block = blockIdx.x - jobs.first_block[j];
+  const int64_t words = jb.inner / 4;
+  const int wblocks = (int)((words + 255) / 256);
+  const int64_t row = block / wblocks, o = row / jb.out_len, x = row % jb.out_len;
+  const TapWindow tw = tap_window(jb.bounds, x, jb.ksize, jb.in_len);
+  const int32_t* k = jb.kk + x * jb.ksize;
+  bool narrow = true;
+  for (int t = 0; t < tw.n; ++t) narrow = narrow && fits24(k[t]);
+  const int64_t w = (int64_t)(block % wblocks) * 256 + threadIdx.x;
+  if (w >= words) return;
+  const uint8_t* p = jb.src + (o * jb.in_len + tw.xmin) * jb.inner + 4 * w;
+  const unsigned v = narrow ? resample_wide_word<true>(p, jb.inner, tw.n, k) : resample_wide_word<false>(p, jb.inner, tw.n, k);
+  *reinterpret_cast<unsigned*>(jb.dst + row * jb.inner + 4 * w) = v;
 }
 
 extern "C" {
@@ -330,29 +331,93 @@ int mvit_patchify(const mvit_image* images, int n_images, int64_t total_rows, vo
   return MVIT_OK;
 }
 
+int mvit_patchify_host_table(const mvit_image* images, int n_images, int64_t total_rows, void* out, double rescale, float mean_r,
+                             float mean_g, float mean_b, float std_r, float std_g, float std_b, int dtype, mvit_stream_t stream) {
+  MVIT_REQUIRE(images != nullptr && n_images > 0, "patchify: empty image table");
+  if (n_images > TABLE_ARG_IMAGES) return mvit_set_error(MVIT_ERR_UNSUPPORTED, "patchify: %d images; a host table holds at most %d", n_images, TABLE_ARG_IMAGES);
+  MVIT_REQUIRE(total_rows >= 0 && total_rows % 4 == 0 && total_rows / 4 <= 0x7fffffffLL,
+               "patchify: total_rows %lld must be a multiple of 4 (2x2 merge blocks) below 2^33", (long long)total_rows);
+  MVIT_REQUIRE(dtype == MVIT_BF16 || dtype == MVIT_F32, "patchify: dtype %d", dtype);
+  MVIT_REQUIRE(std_r != 0.f && std_g != 0.f && std_b != 0.f, "patchify: zero std");
+  if (total_rows == 0) return MVIT_OK;
+  MVIT_REQUIRE(out != nullptr && mvit_aligned16(out), "patchify: output must be a 16-byte aligned device pointer");
+  TableArg table;
+  memset(&table, 0, sizeof(table));
+  memcpy(table.im, images, sizeof(mvit_image) * ((size_t)n_images + 1));
+  Norm nm{rescale, {mean_r, mean_g, mean_b}, {std_r, std_g, std_b}};
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const unsigned grid = (unsigned)(total_rows / 4);
+  if (dtype == MVIT_BF16)
+    hipLaunchKernelGGL((patchify_arg_kernel<bf16_t>), dim3(grid), 256, 0, s, table, n_images, static_cast<bf16_t*>(out), total_rows, nm);
+  else
+    hipLaunchKernelGGL((patchify_arg_kernel<float>), dim3(grid), 256, 0, s, table, n_images, static_cast<float*>(out), total_rows, nm);
+  MVIT_CHECK_LAUNCH("patchify");
+  return MVIT_OK;
+}
+
+int mvit_resample_u8_batch(const mvit_resample_job* list, int n_jobs, mvit_stream_t stream) {
+  MVIT_REQUIRE(n_jobs >= 0 && (n_jobs == 0 || list), "resample_u8: null job list");
+  for (int i = 0; i < n_jobs; ++i) {
+    const mvit_resample_job& j = list[i];
+    MVIT_REQUIRE(j.src && j.dst && j.bounds && j.kk, "resample_u8: null pointer");
+    MVIT_REQUIRE(j.outer >= 0 && j.in_len > 0 && j.out_len > 0 && j.inner > 0 && j.ksize > 0, "resample_u8: bad sizes (outer=%lld in=%lld out=%lld inner=%lld ksize=%d)",
+                 (long long)j.outer, (long long)j.in_len, (long long)j.out_len, (long long)j.inner, j.ksize);
+    MVIT_REQUIRE(j.in_len < (1 << 24) && j.out_len < (1 << 24) && j.in_len * j.inner < (1ll << 40) && j.out_len * j.inner < (1ll << 40) && j.outer < (1ll << 40) / (j.in_len + j.out_len),
+                 "resample_u8: axis too long");
+  }
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  // jobs of one kind (wide words; 1 .. 4 bytes) share launches; 0: everything else, a launch each
+  auto kind_of = [](const mvit_resample_job& j) {
+    if (j.inner % 4 == 0 && j.inner > RESAMPLE_MAX_CHANNELS && reinterpret_cast<uintptr_t>(j.src) % 4 == 0 && reinterpret_cast<uintptr_t>(j.dst) % 4 == 0) return 5;
+    return j.inner <= RESAMPLE_MAX_CHANNELS ? (int)j.inner : 0;
+  };
+  for (int kind = 0; kind <= 5; ++kind) {
+    ResampleJobs jobs;
+    memset(&jobs, 0, sizeof(jobs));
+    int64_t blocks = 0;
+    auto flush = [&]() -> int {
+      if (jobs.n == 0) return MVIT_OK;
+      const dim3 grid((unsigned)blocks);
+      switch (kind) {
+        case 1: hipLaunchKernelGGL((resample_narrow_kernel<1>), grid, 256, 0, s, jobs); break;
+        case 2: hipLaunchKernelGGL((resample_narrow_kernel<2>), grid, 256, 0, s, jobs); break;
+        case 3: hipLaunchKernelGGL((resample_narrow_kernel<3>), grid, 256, 0, s, jobs); break;
+        case 4: hipLaunchKernelGGL((resample_narrow_kernel<4>), grid, 256, 0, s, jobs); break;
+        default: hipLaunchKernelGGL(resample_wide_kernel, grid, 256, 0, s, jobs); break;
+      }
+      MVIT_CHECK_LAUNCH("resample_u8");
+      jobs.n = 0;
+      blocks = 0;
+      return MVIT_OK;
+    };
+    for (int i = 0; i < n_jobs; ++i) {
+      const mvit_resample_job& j = list[i];
+      if (j.outer == 0 || kind_of(j) != kind) continue;
+      if (kind == 0) {
+        const int64_t total = j.outer * j.out_len * j.inner;
+        hipLaunchKernelGGL(resample_pass_kernel, dim3((unsigned)((total + 255) / 256 < 65535 * 16 ? (total + 255) / 256 : 65535 * 16)), 256, 0, s,
+                           j.src, j.dst, j.outer, j.in_len, j.out_len, j.inner, j.bounds, j.kk, j.ksize);
+        MVIT_CHECK_LAUNCH("resample_u8");
+        continue;
+      }
+      const int64_t need = kind == 5 ? j.outer * j.out_len * ((j.inner / 4 + 255) / 256)
+                                     : (j.out_len + 63) / 64 * ((j.outer + 4 * RESAMPLE_ROWS - 1) / (4 * RESAMPLE_ROWS));
+      MVIT_REQUIRE(need < (1ll << 31), "resample_u8: too many rows for one launch");
+      if (jobs.n == RESAMPLE_MAX_JOBS || blocks + need >= (1ll << 31))
+        if (int rc = flush()) return rc;
+      jobs.first_block[jobs.n] = (int)blocks;
+      jobs.job[jobs.n++] = j;
+      blocks += need;
+    }
+    if (int rc = flush()) return rc;
+  }
+  return MVIT_OK;
+}
+
 int mvit_resample_u8(const uint8_t* src, uint8_t* dst, int64_t outer, int64_t in_len, int64_t out_len, int64_t inner,
                      const int32_t* bounds, const int32_t* kk, int ksize, mvit_stream_t stream) {
-  MVIT_REQUIRE(src && dst && bounds && kk, "resample_u8: null pointer");
-  MVIT_REQUIRE(outer >= 0 && in_len > 0 && out_len > 0 && inner > 0 && ksize > 0, "resample_u8: bad sizes (outer=%lld in=%lld out=%lld inner=%lld ksize=%d)",
-               (long long)outer, (long long)in_len, (long long)out_len, (long long)inner, ksize);
-  MVIT_REQUIRE(in_len < (1 << 24) && out_len < (1 << 24) && in_len * inner < (1ll << 40) && out_len * inner < (1ll << 40), "resample_u8: axis too long");
-  if (outer == 0) return MVIT_OK;
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const int64_t quads = (out_len * inner + 3) / 4, total = outer * quads;
-  const unsigned grid = (unsigned)((total + 255) / 256 < 65535 * 16 ? (total + 255) / 256 : 65535 * 16);
-  const bool wide = inner % 4 == 0 && ((uintptr_t)src % 4 == 0) && ((uintptr_t)dst % 4 == 0);
-  if (!wide && inner <= RESAMPLE_MAX_CHANNELS && ksize <= RESAMPLE_KMAX) {
-    const int rows_per_group = 32;
-    const dim3 g((unsigned)((out_len + 255) / 256), (unsigned)((outer + rows_per_group - 1) / rows_per_group));
-    MVIT_REQUIRE(g.y <= 65535, "resample_u8: outer=%lld too large for a short inner dimension", (long long)outer);
-    hipLaunchKernelGGL(resample_cols_kernel, g, 256, 0, s, src, dst, outer, in_len, out_len, (int)inner, bounds, kk, ksize, rows_per_group);
-  } else if (!wide && inner <= RESAMPLE_MAX_CHANNELS && in_len * inner + 4 <= RESAMPLE_LDS_BYTES) {
-    const unsigned rows = (unsigned)(outer < 65535 * 16 ? outer : 65535 * 16);
-    hipLaunchKernelGGL(resample_rows_lds_kernel, dim3(rows), 256, 0, s, src, dst, outer, in_len, out_len, (int)inner, bounds, kk, ksize);
-  } else if (wide) hipLaunchKernelGGL((resample_pass_kernel<true>), dim3(grid), 256, 0, s, src, dst, outer, in_len, out_len, inner, bounds, kk, ksize);
-  else hipLaunchKernelGGL((resample_pass_kernel<false>), dim3(grid), 256, 0, s, src, dst, outer, in_len, out_len, inner, bounds, kk, ksize);
-  MVIT_CHECK_LAUNCH("resample_u8");
-  return MVIT_OK;
+  const mvit_resample_job job = {src, dst, bounds, kk, outer, in_len, out_len, inner, ksize, 0};
+  return mvit_resample_u8_batch(&job, 1, stream);
 }
 
 }  // extern "C"

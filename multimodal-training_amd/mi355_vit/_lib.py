@@ -94,11 +94,15 @@ PROTOTYPES = {
     "mvit_gemm_swiglu_bwd_sums_columns": [_i64, _i64, _i64],
     "mvit_attn_fwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i64, _i32, _i32, _i64, _i64, _i64, _i64, _f32, _i32, _vp],
     "mvit_image_token_ranks": [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp],
+    "mvit_split_rows": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp],
+    "mvit_copy_ranges": [_vp, _i32, _vp],
     "mvit_merge_rows": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp],
     "mvit_adam_step": [_vp, _i32, _i64, C.c_double, C.c_double, C.c_double, C.c_double, _i32, _i32, _vp],
     "mvit_grad_sumsq": [_vp, _i32, _i64, _vp, _vp, _i32, _vp],
     "mvit_grad_sumsq_static": [_vp, _i32, _i64, _vp, _i32, _vp],
     "mvit_patchify": [_vp, _i32, _i64, _vp, C.c_double] + [_f32] * 6 + [_i32, _vp],
+    "mvit_patchify_host_table": [_vp, _i32, _i64, _vp, C.c_double] + [_f32] * 6 + [_i32, _vp],
+    "mvit_resample_u8_batch": [_vp, _i32, _vp],
     "mvit_resample_u8": [_vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _i32, _vp],
     "mvit_patch_embed_pack_weight": [_vp, _i32, _i64, _i64, _vp, _vp],
     "mvit_patch_embed_frames": [_vp, _i32, _i64, _vp, _i64, _vp, _i64, _i32, C.c_double] + [_f32] * 6 + [_vp],

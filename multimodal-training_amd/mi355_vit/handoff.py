@@ -8,7 +8,7 @@ Mirrors the text actor's side of the exchange in the reference, python/ray/text.
   * ``extract_vision_grad``        text.py:1000-1019 (gradient of the leaf, batch dimension removed, detached copy)
 
 One ranking kernel and one row-merge kernel replace the expanded boolean mask, three reductions with host
-read-backs and ``masked_scatter``; the backward is one row gather and one zero-filling merge.
+read-backs and ``masked_scatter``; the backward is one pass over the gradient.
 """
 
 from __future__ import annotations
@@ -18,56 +18,62 @@ from typing import Optional
 import torch
 
 from . import _lib
-from .ops import _stream, gather_rows
+from .ops import _p, _stream
 
 IMAGE_TOKEN_ID = 151655  # text.py:884
 
 
+def _int64_row(t: torch.Tensor) -> torch.Tensor:
+    t = t.reshape(-1)
+    return t if t.dtype == torch.int64 and t.is_contiguous() else t.to(torch.int64).contiguous()
+
+
 def _ranks(input_ids: torch.Tensor, labels: Optional[torch.Tensor], image_token_id: int):
-    ids = input_ids.reshape(-1)
-    if ids.dtype != torch.int64 or not ids.is_contiguous():
-        ids = ids.to(torch.int64).contiguous()
+    """(rank of every token, pinned counts, event after which the host may read them)."""
+    ids = _int64_row(input_ids)
     lab = None
     if labels is not None:
-        lab = labels.reshape(-1)
-        if lab.numel() != ids.numel():
+        if labels.numel() != ids.numel():
             raise ValueError("labels and input_ids differ in size")
-        if lab.dtype != torch.int64 or not lab.is_contiguous():
-            lab = lab.to(torch.int64).contiguous()
+        lab = _int64_row(labels)
     n = ids.numel()
     rank = torch.empty(n, dtype=torch.int32, device=ids.device)
-    positions = torch.empty(n, dtype=torch.int64, device=ids.device)
-    counts = torch.empty(2, dtype=torch.int64, device=ids.device)
+    counts = torch.empty(2, dtype=torch.int64, pin_memory=True)  # the kernel writes them where the host reads them
     rc = _lib.load().mvit_image_token_ranks(ids.data_ptr(), None if lab is None else lab.data_ptr(), n, image_token_id, -100,
-                                            rank.data_ptr(), positions.data_ptr(), counts.data_ptr(), _stream(ids))
+                                            rank.data_ptr(), None, counts.data_ptr(), _stream(ids))
     _lib.check(rc, "mvit_image_token_ranks")
-    n_image, n_bad_labels = counts.tolist()  # the one host read-back (the reference has three)
-    return rank, positions[:n_image], n_image, n_bad_labels
-
-
-def _merge(embeds2d: torch.Tensor, vision2d: Optional[torch.Tensor], rank: torch.Tensor, n_vision: int) -> torch.Tensor:
-    out = torch.empty_like(embeds2d)
-    rc = _lib.load().mvit_merge_rows(embeds2d.data_ptr(), None if vision2d is None else vision2d.data_ptr(), rank.data_ptr(),
-                                     out.data_ptr(), embeds2d.shape[0], n_vision, embeds2d.shape[1] * embeds2d.element_size(),
-                                     _stream(embeds2d))
-    _lib.check(rc, "mvit_merge_rows")
-    return out
+    ready = torch.cuda.Event()
+    ready.record(torch.cuda.current_stream(ids.device))
+    return rank, counts, ready
 
 
 class _MergeRowsFn(torch.autograd.Function):
+    """Row merge over the last dimension of embeds [..., O] and vision [..., O]; the gradients keep those shapes."""
+
     @staticmethod
-    def forward(ctx, embeds2d, vision2d, rank, positions):
-        ctx.save_for_backward(rank, positions)
-        ctx.n_vision = vision2d.shape[0]
-        return _merge(embeds2d, vision2d, rank, vision2d.shape[0])
+    def forward(ctx, embeds, vision, rank):
+        embeds, vision = embeds.contiguous(), vision.contiguous()
+        hidden = embeds.shape[-1]
+        n_vision = vision.numel() // hidden
+        out = torch.empty_like(embeds)
+        rc = _lib.load().mvit_merge_rows(embeds.data_ptr(), vision.data_ptr(), rank.data_ptr(), out.data_ptr(), rank.numel(), n_vision,
+                                         hidden * embeds.element_size(), _stream(embeds))
+        _lib.check(rc, "mvit_merge_rows")
+        ctx.save_for_backward(rank)
+        ctx.vision_shape = vision.shape
+        return out
 
     @staticmethod
     def backward(ctx, grad):
-        rank, positions = ctx.saved_tensors
+        (rank,) = ctx.saved_tensors
         grad = grad.contiguous()
-        d_embeds = _merge(grad, None, rank, ctx.n_vision) if ctx.needs_input_grad[0] else None
-        d_vision = gather_rows(grad, positions, 1) if ctx.needs_input_grad[1] else None
-        return d_embeds, d_vision, None, None
+        hidden = grad.shape[-1]
+        d_embeds = torch.empty_like(grad) if ctx.needs_input_grad[0] else None
+        d_vision = torch.empty(ctx.vision_shape, dtype=grad.dtype, device=grad.device) if ctx.needs_input_grad[1] else None
+        rc = _lib.load().mvit_split_rows(grad.data_ptr(), rank.data_ptr(), _p(d_embeds), _p(d_vision), rank.numel(),
+                                         ctx.vision_shape.numel() // hidden, hidden * grad.element_size(), _stream(grad))
+        _lib.check(rc, "mvit_split_rows")
+        return d_embeds, d_vision, None
 
 
 def prepare_vision_embeddings(vision_embeddings: torch.Tensor) -> torch.Tensor:
@@ -89,25 +95,29 @@ def merge_vision_embeddings(inputs_embeds: torch.Tensor, input_ids: torch.Tensor
     if tuple(inputs_embeds.shape[:-1]) != tuple(input_ids.shape):
         raise ValueError(f"inputs_embeds {tuple(inputs_embeds.shape)} does not match input_ids {tuple(input_ids.shape)}")
     hidden = inputs_embeds.shape[-1]
-    vision_flat = vision_embeddings.reshape(-1, vision_embeddings.shape[-1])
-    if vision_flat.shape[1] != hidden or vision_flat.dtype != inputs_embeds.dtype or vision_flat.device != inputs_embeds.device:
+    n_vision = vision_embeddings.numel() // hidden if hidden else 0
+    if vision_embeddings.shape[-1] != hidden or vision_embeddings.dtype != inputs_embeds.dtype or vision_embeddings.device != inputs_embeds.device:
         raise ValueError("vision embeddings must share hidden size, dtype and device with inputs_embeds")
-    ranks, positions, n_image, n_bad = _ranks(input_ids, labels, image_token_id)
+    ranks, counts, ready = _ranks(input_ids, labels, image_token_id)
+    # the merge is queued before the host waits for the counts: it stays inside its arrays whatever they are, and its result
+    # is dropped when one of the checks below refuses the call
+    merged = _MergeRowsFn.apply(inputs_embeds, vision_embeddings, ranks)
+    ready.synchronize()  # the one host wait (the reference has three)
+    n_image, n_bad = counts.tolist()
     if n_image == 0:
         raise RuntimeError(
             f"[r{rank}] No <image> tokens (ID={image_token_id}) found in input_ids! "
             f"This likely means modality filter is wrong. input_ids shape: {input_ids.shape}")
-    if vision_flat.shape[0] != n_image:
+    if n_vision != n_image:
         raise RuntimeError(
-            f"[r{rank}] Mismatch: {vision_flat.shape[0]} vision embeddings but "
+            f"[r{rank}] Mismatch: {n_vision} vision embeddings but "
             f"{n_image} <image> tokens in input_ids! "
             f"Vision and text trainers are out of sync.")
     if n_bad:
         raise RuntimeError(
             f"[r{rank}] Labels should be -100 at <image> positions, but found {n_bad} "
             f"positions with other values. This indicates incorrect label preprocessing.")
-    merged = _MergeRowsFn.apply(inputs_embeds.reshape(-1, hidden).contiguous(), vision_flat.contiguous(), ranks, positions)
-    return merged.view(inputs_embeds.shape)
+    return merged
 
 
 def extract_vision_grad(vision_embeddings: Optional[torch.Tensor], rank: int = 0) -> torch.Tensor:

@@ -226,23 +226,32 @@ def gather_rows(src: torch.Tensor, index: torch.Tensor, rows_per_index: int = 1)
     return out
 
 
+def segment_copies(copies: Sequence[Tuple[torch.Tensor, torch.Tensor, Sequence[Tuple[int, int, int]]]]) -> None:
+    """Copy rows: for every (src, dst, segments) and every (src_row, dst_row, n_rows) of its segments, all in one launch.
+    The host validates bounds; the kernel moves bytes."""
+    ranges, at = [], None
+    for src, dst, segments in copies:
+        if src.dim() != 2 or dst.dim() != 2 or not (src.is_contiguous() and dst.is_contiguous()):
+            raise ValueError("segment_copy: src and dst must be contiguous 2-D")
+        if src.shape[1] != dst.shape[1] or src.dtype != dst.dtype:
+            raise ValueError("segment_copy: column count / dtype mismatch")
+        n_src, n_dst, row = src.shape[0], dst.shape[0], src.shape[1] * src.element_size()
+        p_src, p_dst = src.data_ptr(), dst.data_ptr()
+        for a, b, n in segments:
+            if n <= 0:
+                continue
+            if a < 0 or b < 0 or a + n > n_src or b + n > n_dst:
+                raise ValueError(f"segment_copy: segment ({a},{b},{n}) out of bounds for {n_src} -> {n_dst} rows")
+            ranges += (p_src + a * row, p_dst + b * row, n * row)
+        at = src
+    if ranges:
+        flat = (C.c_uint64 * len(ranges))(*ranges)
+        _lib.check(_lib.load().mvit_copy_ranges(C.addressof(flat), len(ranges) // 3, _stream(at)), "mvit_copy_ranges")
+
+
 def segment_copy(src: torch.Tensor, dst: torch.Tensor, segments: Sequence[Tuple[int, int, int]]) -> torch.Tensor:
-    """Copy rows: for (src_row, dst_row, n_rows) in segments.  Host validates bounds; the kernel moves bytes."""
-    if src.dim() != 2 or dst.dim() != 2 or not (src.is_contiguous() and dst.is_contiguous()):
-        raise ValueError("segment_copy: src and dst must be contiguous 2-D")
-    if src.shape[1] != dst.shape[1] or src.dtype != dst.dtype:
-        raise ValueError("segment_copy: column count / dtype mismatch")
-    segs = [(int(a), int(b), int(n)) for a, b, n in segments if n > 0]
-    for a, b, n in segs:
-        if a < 0 or b < 0 or a + n > src.shape[0] or b + n > dst.shape[0]:
-            raise ValueError(f"segment_copy: segment ({a},{b},{n}) out of bounds for {src.shape[0]} -> {dst.shape[0]} rows")
-    if not segs:
-        return dst
-    # pinned staging + asynchronous copy: the launch below is ordered behind it on the same stream, the host does not wait
-    desc = torch.tensor(segs, dtype=torch.int64).pin_memory().to(src.device, non_blocking=True)
-    row_bytes = src.shape[1] * src.element_size()
-    rc = _lib.load().mvit_segment_copy(src.data_ptr(), dst.data_ptr(), desc.data_ptr(), len(segs), max(n for _, _, n in segs), row_bytes, _stream(src))
-    _lib.check(rc, "mvit_segment_copy")
+    """Copy rows: for (src_row, dst_row, n_rows) in segments."""
+    segment_copies([(src, dst, segments)])
     return dst
 
 

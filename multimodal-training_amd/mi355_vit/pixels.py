@@ -36,6 +36,7 @@ PATCH_SIZE, TEMPORAL_PATCH_SIZE, MERGE_SIZE = 14, 2, 2
 _TABLE_DTYPE = np.dtype([("pixels", "<u8"), ("frames", "<i4"), ("height", "<i4"), ("width", "<i4"), ("reserved", "<i4"),
                          ("first_row", "<i8")])
 assert _TABLE_DTYPE.itemsize == C.sizeof(_lib.Image) == 32
+_HOST_TABLE_IMAGES = 64  # image tables up to this length travel with the launch
 
 
 def grid_thw_of(frames: Sequence[torch.Tensor]) -> torch.Tensor:
@@ -54,8 +55,8 @@ def grid_thw_of(frames: Sequence[torch.Tensor]) -> torch.Tensor:
 
 
 def _image_table(frames: Sequence[torch.Tensor], what: str):
-    """Checks the frame stacks and builds the device table of ``mvit_image`` entries (32 bytes per image, one
-    synchronous copy).  Returns (frames as a list, image_grid_thw, device table, total rows)."""
+    """Checks the frame stacks and builds the table of ``mvit_image`` entries (32 bytes per image).  Returns (frames as a
+    list, image_grid_thw, table on the host, total rows)."""
     frames = list(frames)
     if not frames:
         raise ValueError(f"{what}: no images")
@@ -66,16 +67,16 @@ def _image_table(frames: Sequence[torch.Tensor], what: str):
             raise RuntimeError(f"image {i} on {f.device}: frames must be on one GPU (there is no CPU path)")
         if not f.is_contiguous():
             raise RuntimeError(f"image {i}: frames must be contiguous")
-    counts = (grid[:, 0] * grid[:, 1] * grid[:, 2]).numpy()
-    n = len(frames)
-    table = np.zeros(n + 1, dtype=_TABLE_DTYPE)
-    table["pixels"][:n] = [f.data_ptr() for f in frames]
-    table["frames"][:n] = [f.shape[0] for f in frames]
-    table["height"][:n] = [f.shape[1] for f in frames]
-    table["width"][:n] = [f.shape[2] for f in frames]
-    table["first_row"][1:] = np.cumsum(counts)
-    total = int(table["first_row"][n])
-    return frames, grid, torch.from_numpy(table.view(np.uint8)).to(device), total
+    rows, total = [], 0
+    for f, (t, gh, gw) in zip(frames, grid.tolist()):
+        rows.append((f.data_ptr(), f.shape[0], f.shape[1], f.shape[2], 0, total))
+        total += t * gh * gw
+    rows.append((0, 0, 0, 0, 0, total))
+    return frames, grid, np.array(rows, dtype=_TABLE_DTYPE), total
+
+
+def _on_device(table: np.ndarray, device: torch.device) -> torch.Tensor:
+    return torch.from_numpy(table.view(np.uint8)).to(device)  # a few tens of bytes per image, one synchronous copy
 
 
 def patchify(frames: Sequence[torch.Tensor], dtype: torch.dtype = torch.float32,
@@ -92,7 +93,7 @@ def patchify(frames: Sequence[torch.Tensor], dtype: torch.dtype = torch.float32,
         code = _lib.BF16
     else:
         raise TypeError(f"unsupported dtype {dtype} (float32 and bfloat16 only)")
-    frames, grid, dev_table, total = _image_table(frames, "patchify")
+    frames, grid, table, total = _image_table(frames, "patchify")
     n, device = len(frames), frames[0].device
     if out is None:
         out = torch.empty((total, _lib.PIXEL_ROW), dtype=dtype, device=device)
@@ -103,7 +104,11 @@ def patchify(frames: Sequence[torch.Tensor], dtype: torch.dtype = torch.float32,
     lib = _lib.load()
     with torch.cuda.device(device):
         stream = torch.cuda.current_stream(device).cuda_stream
-        rc = lib.mvit_patchify(dev_table.data_ptr(), n, total, out.data_ptr(), float(rescale_factor), *mean, *std, code, stream)
+        if n <= _HOST_TABLE_IMAGES:
+            rc = lib.mvit_patchify_host_table(table.ctypes.data, n, total, out.data_ptr(), float(rescale_factor), *mean, *std, code, stream)
+        else:
+            dev_table = _on_device(table, device)
+            rc = lib.mvit_patchify(dev_table.data_ptr(), n, total, out.data_ptr(), float(rescale_factor), *mean, *std, code, stream)
     _lib.check(rc, "mvit_patchify")
     return out, grid
 
@@ -142,7 +147,7 @@ def patch_embed_frames(frames: Sequence[torch.Tensor], packed_weight: torch.Tens
     one multiply-add per byte without changing a bfloat16 value (the caller then uses ``patchify`` and a GEMM)."""
     if dtype not in (torch.float32, torch.bfloat16):
         raise TypeError(f"unsupported dtype {dtype} (float32 and bfloat16 only)")
-    frames, grid, dev_table, total = _image_table(frames, "patch_embed_frames")
+    frames, grid, table, total = _image_table(frames, "patch_embed_frames")
     device = frames[0].device
     if not frames_fit_fused_patch_embed(frames):
         raise RuntimeError("patch_embed_frames: frame buffers must be 4-byte aligned and smaller than 2 GiB")
@@ -150,6 +155,7 @@ def patch_embed_frames(frames: Sequence[torch.Tensor], packed_weight: torch.Tens
             or packed_weight.device != device or not packed_weight.is_contiguous()):
         raise ValueError("patch_embed_frames: packed_weight must be the contiguous bfloat16 [embed_dim, 1344] result of pack_patch_embed_weight on the frames' GPU")
     out = torch.empty((total, packed_weight.shape[0]), dtype=dtype, device=device)
+    dev_table = _on_device(table, device)
     mean = [float(np.float32(m)) for m in image_mean]
     std = [float(np.float32(s)) for s in image_std]
     lib = _lib.load()
@@ -231,47 +237,74 @@ def _device_coefficients(in_size: int, out_size: int, resample: str, device_inde
     return torch.from_numpy(bounds).to(dev), torch.from_numpy(kk).to(dev), kk.shape[1]
 
 
-def resize_frames(frames: torch.Tensor, out_height: int, out_width: int, resample: str = BICUBIC) -> torch.Tensor:
-    """``PIL.Image.resize((out_width, out_height), resample)`` applied to every frame of a contiguous uint8 GPU tensor
-    ``[frames, height, width, 3]``, bit for bit: a horizontal pass into an 8-bit intermediate image, then a vertical
-    pass (a pass whose size does not change is skipped, as Pillow does)."""
+def _check_resizable(frames: torch.Tensor) -> None:
     if frames.dim() != 4 or frames.dtype != torch.uint8 or frames.shape[0] < 1:
         raise ValueError(f"resize_frames: expected uint8 [frames, height, width, channels], got {frames.dtype} {tuple(frames.shape)}")
     if not frames.is_cuda:
         raise RuntimeError("resize_frames: frames must be on the GPU (there is no CPU path)")
     if not frames.is_contiguous():
         raise RuntimeError("resize_frames: frames must be contiguous")
+
+
+def resize_frames(frames: torch.Tensor, out_height: int, out_width: int, resample: str = BICUBIC) -> torch.Tensor:
+    """``PIL.Image.resize((out_width, out_height), resample)`` applied to every frame of a contiguous uint8 GPU tensor
+    ``[frames, height, width, 3]``, bit for bit: a horizontal pass into an 8-bit intermediate image, then a vertical
+    pass (a pass whose size does not change is skipped, as Pillow does)."""
+    _check_resizable(frames)
     if out_height < 1 or out_width < 1:
         raise ValueError(f"resize_frames: target {out_height}x{out_width}")
-    n, h, w, ch = frames.shape
-    lib = _lib.load()
-    device = frames.device
-    cur = frames
+    return _resize_batch([frames], [(out_height, out_width)], resample, frames.device, copy_unchanged=True)[0]
+
+
+_JOB_DTYPE = np.dtype([("src", "<u8"), ("dst", "<u8"), ("bounds", "<u8"), ("kk", "<u8"), ("outer", "<i8"), ("in_len", "<i8"), ("out_len", "<i8"),
+                       ("inner", "<i8"), ("ksize", "<i4"), ("reserved", "<i4")])
+
+
+def _resample_passes(jobs: list, device: torch.device) -> None:
+    if jobs:
+        table = np.array(jobs, dtype=_JOB_DTYPE)
+        _lib.check(_lib.load().mvit_resample_u8_batch(table.ctypes.data, len(jobs), torch.cuda.current_stream(device).cuda_stream), "mvit_resample_u8_batch")
+
+
+def _resize_batch(frames: Sequence[torch.Tensor], sizes: Sequence[Tuple[int, int]], resample: str, device: torch.device,
+                  copy_unchanged: bool) -> list:
+    """Every frame stack resized to its (height, width): the horizontal passes of all of them in one launch, then the
+    vertical ones in another.  A stack that already has its size is returned as it is (copied if asked)."""
+    index = device.index or 0
+    out, across, down = [], [], []
+    for f, (oh, ow) in zip(frames, sizes):
+        n, h, w, ch = f.shape
+        cur = f
+        if w != ow:
+            bounds, kk, ksize = _device_coefficients(w, ow, resample, index)
+            nxt = torch.empty((n, h, ow, ch), dtype=torch.uint8, device=device)
+            across.append((cur.data_ptr(), nxt.data_ptr(), bounds.data_ptr(), kk.data_ptr(), n * h, w, ow, ch, ksize, 0))
+            cur = nxt
+        if h != oh:
+            bounds, kk, ksize = _device_coefficients(h, oh, resample, index)
+            nxt = torch.empty((n, oh, ow, ch), dtype=torch.uint8, device=device)
+            down.append((cur.data_ptr(), nxt.data_ptr(), bounds.data_ptr(), kk.data_ptr(), n, h, oh, ow * ch, ksize, 0))
+            out.append((nxt, cur))  # the intermediate image lives until both launches are queued
+        else:
+            out.append((cur, None))
     with torch.cuda.device(device):
-        stream = torch.cuda.current_stream(device).cuda_stream
-        if w != out_width:
-            bounds, kk, ksize = _device_coefficients(w, out_width, resample, device.index or 0)
-            nxt = torch.empty((n, h, out_width, ch), dtype=torch.uint8, device=device)
-            _lib.check(lib.mvit_resample_u8(cur.data_ptr(), nxt.data_ptr(), n * h, w, out_width, ch, bounds.data_ptr(), kk.data_ptr(),
-                                            ksize, stream), "mvit_resample_u8")
-            cur = nxt
-        if h != out_height:
-            bounds, kk, ksize = _device_coefficients(h, out_height, resample, device.index or 0)
-            nxt = torch.empty((n, out_height, out_width, ch), dtype=torch.uint8, device=device)
-            _lib.check(lib.mvit_resample_u8(cur.data_ptr(), nxt.data_ptr(), n, h, out_height, out_width * ch, bounds.data_ptr(),
-                                            kk.data_ptr(), ksize, stream), "mvit_resample_u8")
-            cur = nxt
-    return cur.clone() if cur is frames else cur
+        _resample_passes(across, device)
+        _resample_passes(down, device)
+    return [o.clone() if copy_unchanged and o is f else o for (o, _), f in zip(out, frames)]
 
 
 def preprocess(images: Sequence[torch.Tensor], dtype: torch.dtype = torch.float32, min_pixels: int = 56 * 56,
                max_pixels: int = 14 * 14 * 4 * 1280, resample: str = BICUBIC) -> Tuple[torch.Tensor, torch.Tensor]:
     """Decoded still images (uint8 GPU tensors ``[1, height, width, 3]`` of any size) -> (``pixel_values``,
     ``image_grid_thw``): the image processor's smart_resize + resize + rescale + normalise + patchify, on the GPU."""
-    resized = []
+    images, sizes = list(images), []
     for i, f in enumerate(images):
         if f.dim() != 4 or f.shape[0] != 1 or f.shape[3] != 3:
             raise ValueError(f"image {i}: expected uint8 [1, height, width, 3], got {tuple(f.shape)}")
-        th, tw = smart_resize(int(f.shape[1]), int(f.shape[2]), min_pixels=min_pixels, max_pixels=max_pixels)
-        resized.append(resize_frames(f, th, tw, resample))
-    return patchify(resized, dtype=dtype)
+        sizes.append(smart_resize(int(f.shape[1]), int(f.shape[2]), min_pixels=min_pixels, max_pixels=max_pixels))
+        _check_resizable(f)
+        if f.device != images[0].device:
+            raise RuntimeError(f"image {i} on {f.device}: frames must be on one GPU (there is no CPU path)")
+    if not images:
+        raise ValueError("patchify: no images")
+    return patchify(_resize_batch(images, sizes, resample, images[0].device, copy_unchanged=False), dtype=dtype)

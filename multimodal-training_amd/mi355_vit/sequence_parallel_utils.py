@@ -5,7 +5,7 @@ python/models/qwen2_5_vl/sequence_parallel_utils.py, split in two layers:
 
 * planning (pure host integers, done by the C planners ``mvit_sp_token_cuts`` / ``mvit_sp_window_cuts``)
   produces a ``RaggedSequenceMeta`` -- usable without a GPU;
-* data movement (``mvit_segment_copy`` / ``mvit_pad_pack``) turns a plan into one kernel launch instead of
+* data movement (``mvit_copy_ranges`` / ``mvit_pad_pack``) turns a plan into one kernel launch instead of
   a Python loop of slices and ``torch.cat``.  Copies are bit-exact.
 
 The collectives of the reference (all-gather / all-to-all) are outside this build; ``gather_rank_packs``
@@ -183,10 +183,9 @@ def rebuild_local_cu_seqlens(meta: RaggedSequenceMeta, *, use_windows: bool = Fa
 def build_local_rope(meta: RaggedSequenceMeta, global_pos_emb_cos: torch.Tensor, global_pos_emb_sin: torch.Tensor,
                      pad_to: Optional[int] = None):
     segs = [(a, lo, b - a) for (a, b), (lo, _) in zip(meta.sample_global_slices, meta.local_token_offsets)]
-    outs = []
-    for src in (global_pos_emb_cos, global_pos_emb_sin):
-        dst = torch.empty(meta.total_local_len, src.shape[-1], dtype=src.dtype, device=src.device)
-        outs.append(ops.segment_copy(src.contiguous(), dst, segs))
+    srcs = (global_pos_emb_cos, global_pos_emb_sin)
+    outs = [torch.empty(meta.total_local_len, src.shape[-1], dtype=src.dtype, device=src.device) for src in srcs]
+    ops.segment_copies([(src.contiguous(), dst, segs) for src, dst in zip(srcs, outs)])
     if pad_to is None:
         return outs[0], outs[1], None
     cos_p, mask = ops.pad_pack(outs[0], meta.local_lengths, pad_to, 0.0)
@@ -208,8 +207,7 @@ def gather_rank_packs(rank_packs: Sequence[torch.Tensor], lengths_matrix: Sequen
                 segs[r].append((cursor[r], o, n))
                 cursor[r] += n
                 o += n
-    for r, pack in enumerate(rank_packs):
-        ops.segment_copy(pack.contiguous(), out, segs[r])
+    ops.segment_copies([(pack.contiguous(), out, segs[r]) for r, pack in enumerate(rank_packs)])
     return out
 
 
