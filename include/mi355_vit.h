@@ -33,10 +33,11 @@ typedef void* mvit_stream_t; /* hipStream_t */
 enum { MVIT_F32 = 0, MVIT_BF16 = 1 };
 enum { MVIT_OK = 0, MVIT_ERR_ARG = -1, MVIT_ERR_LAUNCH = -2, MVIT_ERR_UNSUPPORTED = -3 };
 
-/* 200: mvit_attn_bwd takes the size of its workspace (delta_elems) and checks that outputs and inputs are disjoint;
+/* 201: mvit_gemm_args has row_sums at its end.
+ * 200: mvit_attn_bwd takes the size of its workspace (delta_elems) and checks that outputs and inputs are disjoint;
  *      mvit_adam_tensor rows are 96 bytes (shadow copy fields).  A caller built against an older header must be
  *      rebuilt: compare mvit_version() with the value the header was written for. */
-#define MVIT_VERSION 200
+#define MVIT_VERSION 201
 int mvit_version(void);
 const char* mvit_last_error(void);
 
@@ -181,6 +182,9 @@ typedef struct mvit_gemm_args {
                     order and applies the epilogue (few output tiles, long contraction).  Available to any caller; the
                     vision tower uses it for weight gradients only, because a slice count chosen from M would make a
                     row's result depend on how many rows share its batch */
+  void* row_sums; /* optional, bf16 operands with trans_a = trans_b = 1 and EPI_NONE only: receives sum_k A[m,k], [M], in
+                     out_dtype.  For a weight gradient dW = dY^T X this is the bias gradient.  With split_k > 1 the
+                     workspace holds split_k * M more floats */
 } mvit_gemm_args;
 
 /* C[M,N] = epilogue(sum_k A[m,k] * B[n,k]).  Operands must be 16-byte aligned with lda/ldb multiples of
@@ -192,7 +196,7 @@ int mvit_gemm(const mvit_gemm_args* args, mvit_stream_t stream);
 /* Host-only: the split_k to ask for when C[out_rows, out_cols] is a weight gradient contracted over k tokens (bf16). */
 int mvit_gemm_wgrad_split_k(int64_t out_rows, int64_t out_cols, int64_t k);
 /* Host-only: 1 when a bf16 MVIT_EPI_SWIGLU_BWD product of this shape is fastest on the kernel that can hand back column sums
- * of C, 0 when it is faster without a workspace (mvit_colsum then takes the sums). */
+ * of C (of its fp32 values), 0 when it is faster without a workspace (the weight gradient's row_sums then take the sums). */
 int mvit_gemm_swiglu_bwd_sums_columns(int64_t M, int64_t N, int64_t K);
 
 /* ---------------------------------------------------------------- varlen attention */

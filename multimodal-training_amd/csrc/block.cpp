@@ -51,14 +51,18 @@ BwdWorkspace plan_bwd_workspace(const mvit_block_args* a, void* base) {
   const int64_t S = a->S, C = a->C, I = a->I, Ipad = a->Ipad;
   Bump b{static_cast<char*>(base), 0, 0};
   BwdWorkspace w;
-  w.colsum = static_cast<float*>(b.take(64 * (3 * C > 2 * Ipad ? 3 * C : 2 * Ipad) * 4));
+  w.colsum = static_cast<float*>(b.take(a->dtype == MVIT_BF16 ? 0 : 64 * (3 * C > 2 * Ipad ? 3 * C : 2 * Ipad) * 4));
   w.swiglu_cols = static_cast<float*>(b.take((S + 255) / 256 * 2 * Ipad * 4));
   w.rms = static_cast<float*>(b.take((int64_t)RMS_PARTIALS * C * 4));
   w.delta_elems = mvit_attn_bwd_delta_elems(a->max_seqlen, S, a->nheads, a->head_dim, a->dtype);
   w.delta = static_cast<float*>(b.take(w.delta_elems * 4));
   const int64_t sk[4] = {a->split_k_down * C * I, a->split_k_gate_up * 2 * Ipad * C, a->split_k_proj * C * C, a->split_k_qkv * 3 * C * C};
   w.splitk_bytes = 0;
-  for (int64_t n : sk) w.splitk_bytes = n * 4 > w.splitk_bytes ? n * 4 : w.splitk_bytes;
+  const int64_t rows[4] = {a->split_k_down * C, a->split_k_gate_up * 2 * Ipad, a->split_k_proj * C, a->split_k_qkv * 3 * C};  // bias gradients
+  for (int i = 0; i < 4; ++i) {
+    const int64_t n = sk[i] + rows[i];
+    w.splitk_bytes = n * 4 > w.splitk_bytes ? n * 4 : w.splitk_bytes;
+  }
   w.splitk = static_cast<float*>(b.take(w.splitk_bytes));
   w.total = b.used;
   return w;
@@ -170,15 +174,17 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
     STEP(mvit_colsum(dy, ld, S, cols, w.colsum, np, dt, st));
     return mvit_reduce_partials(w.colsum, np, cols, out, gdt, st);
   };
-  // dW[M, N] = dY^T . X over the S rows
-  auto weight_grad = [&](const void* dy, int64_t ldy, int64_t M, const void* x, int64_t ldx, int64_t N, void* out, int split_k, mvit_stream_t st) -> int {
+  // dW[M, N] = dY^T . X over the S rows and db[M], the column sums of dY: bf16 products sum them from the operand they read
+  auto weight_grad = [&](const void* dy, int64_t ldy, int64_t M, const void* x, int64_t ldx, int64_t N, void* out, void* bias, int split_k, mvit_stream_t st) -> int {
+    if (bias && dt != MVIT_BF16) STEP(bias_grad(dy, ldy, M, bias, st));
     mvit_gemm_args g = gemm_args(dt, gdt);
     g.trans_a = 1; g.trans_b = 1;
     g.M = M; g.N = N; g.K = S;
     g.A = dy; g.lda = ldy; g.B = x; g.ldb = ldx; g.C = out; g.ldc = N;
     if (split_k > 1) {
-      g.split_k = split_k; g.workspace = w.splitk; g.workspace_bytes = (int64_t)split_k * M * N * 4;
+      g.split_k = split_k; g.workspace = w.splitk; g.workspace_bytes = (int64_t)split_k * M * (N + 1) * 4;
     }
+    if (dt == MVIT_BF16) g.row_sums = bias;
     return mvit_gemm(&g, st);
   };
 
@@ -186,11 +192,10 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   {
     mvit_stream_t st = fork(0);
     if (!st && two) return MVIT_ERR_LAUNCH;
-    STEP(bias_grad(a->dx2, C, C, a->g_bdown, st));
-    STEP(weight_grad(a->dx2, C, C, a->h, Ipad, I, a->g_wdown, a->split_k_down, st));
+    STEP(weight_grad(a->dx2, C, C, a->h, Ipad, I, a->g_wdown, a->g_bdown, a->split_k_down, st));
   }
-  // dgu = (dx2 . Wdown) through the SwiGLU derivative.  With many rows the per-tile column sums of dgu come back with it;
-  // with few the product runs on smaller tiles and the sums are taken beside the chain
+  // dgu = (dx2 . Wdown) through the SwiGLU derivative.  With many rows the per-tile column sums of dgu come back with it, from
+  // its fp32 values; with few the product runs on smaller tiles and the weight gradient sums the operand it reads
   const bool fused_cols = dt == MVIT_BF16 && mvit_gemm_swiglu_bwd_sums_columns(S, Ipad, C);
   {
     mvit_gemm_args g = gemm_args(dt, dt);
@@ -206,8 +211,7 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
     mvit_stream_t st = fork(1);
     if (!st && two) return MVIT_ERR_LAUNCH;
     if (fused_cols) STEP(mvit_reduce_partials(w.swiglu_cols, (int)((S + 255) / 256), 2 * Ipad, a->g_bgu, gdt, st));
-    else STEP(bias_grad(a->dgu, 2 * Ipad, 2 * Ipad, a->g_bgu, st));
-    STEP(weight_grad(a->dgu, 2 * Ipad, 2 * Ipad, a->n2, C, C, a->g_wgu, a->split_k_gate_up, st));
+    STEP(weight_grad(a->dgu, 2 * Ipad, 2 * Ipad, a->n2, C, C, a->g_wgu, fused_cols ? nullptr : a->g_bgu, a->split_k_gate_up, st));
   }
   {  // dn2 = dgu . Wgu
     mvit_gemm_args g = gemm_args(dt, dt);
@@ -223,8 +227,7 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   {
     mvit_stream_t st = fork(2);
     if (!st && two) return MVIT_ERR_LAUNCH;
-    STEP(bias_grad(a->dx1, C, C, a->g_bproj, st));
-    STEP(weight_grad(a->dx1, C, C, a->o, C, C, a->g_wproj, a->split_k_proj, st));
+    STEP(weight_grad(a->dx1, C, C, a->o, C, C, a->g_wproj, a->g_bproj, a->split_k_proj, st));
   }
   {  // d_o = dx1 . Wproj  (into the dn buffer, whose contents the norm backward above has consumed)
     mvit_gemm_args g = gemm_args(dt, dt);
@@ -240,8 +243,7 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   {
     mvit_stream_t st = fork(3);
     if (!st && two) return MVIT_ERR_LAUNCH;
-    STEP(bias_grad(a->dqkv, 3 * C, 3 * C, a->g_bqkv, st));
-    STEP(weight_grad(a->dqkv, 3 * C, 3 * C, a->n1, C, C, a->g_wqkv, a->split_k_qkv, st));
+    STEP(weight_grad(a->dqkv, 3 * C, 3 * C, a->n1, C, C, a->g_wqkv, a->g_bqkv, a->split_k_qkv, st));
   }
   {  // dn1 = dqkv . Wqkv
     mvit_gemm_args g = gemm_args(dt, dt);

@@ -963,8 +963,15 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_dl_kernel(const GemmPara
 template <typename T, typename TO, bool VEC>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ ws, int split_k, int64_t M, int64_t N,
                                                             TO* __restrict__ C, int64_t ldc, int epi, const T* __restrict__ bias,
-                                                            const T* __restrict__ R, int64_t ldr) {
+                                                            const T* __restrict__ R, int64_t ldr, const float* __restrict__ row_ws,
+                                                            TO* __restrict__ row_sums) {
   const int64_t total = M * N;
+  if (row_ws != nullptr)
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < M; i += (int64_t)gridDim.x * 256) {
+      float s = 0.f;
+      for (int k = 0; k < split_k; ++k) s += row_ws[(int64_t)k * M + i];
+      row_sums[i] = from_f32<TO>(s);
+    }
   if constexpr (VEC) {
     const int64_t quads = total / 4, nq = N / 4;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < quads; i += (int64_t)gridDim.x * 256) {
@@ -1008,8 +1015,8 @@ void launch_splitk_reduce(const GemmParams& p, hipStream_t stream) {
   if (epi == MVIT_EPI_BIAS_RES) vec = vec && p.ldr % 4 == 0 && reinterpret_cast<uintptr_t>(R) % (4 * sizeof(T)) == 0;
   const int64_t items = vec ? elems / 4 : elems;
   const int rgrid = (int)((items + 255) / 256 < 8192 ? (items + 255) / 256 : 8192);
-  if (vec) hipLaunchKernelGGL((splitk_reduce_kernel<T, TO, true>), rgrid, 256, 0, stream, p.workspace, p.split_k, p.M, p.N, static_cast<TO*>(p.C), p.ldc, epi, bias, R, p.ldr);
-  else hipLaunchKernelGGL((splitk_reduce_kernel<T, TO, false>), rgrid, 256, 0, stream, p.workspace, p.split_k, p.M, p.N, static_cast<TO*>(p.C), p.ldc, epi, bias, R, p.ldr);
+  if (vec) hipLaunchKernelGGL((splitk_reduce_kernel<T, TO, true>), rgrid, 256, 0, stream, p.workspace, p.split_k, p.M, p.N, static_cast<TO*>(p.C), p.ldc, epi, bias, R, p.ldr, p.row_ws, static_cast<TO*>(p.row_sums));
+  else hipLaunchKernelGGL((splitk_reduce_kernel<T, TO, false>), rgrid, 256, 0, stream, p.workspace, p.split_k, p.M, p.N, static_cast<TO*>(p.C), p.ldc, epi, bias, R, p.ldr, p.row_ws, static_cast<TO*>(p.row_sums));
 }
 
 template <typename T, typename TO, bool TA, bool TB, int EPI, int VAR>
@@ -1330,6 +1337,10 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
   p.panel_w = tn <= 6 ? (int)tn : 4;
   p.split_k = 1; p.k_chunk = a->K; p.workspace = nullptr; p.reduce_epi = MVIT_EPI_NONE;
   p.colsum = nullptr;
+  p.row_sums = a->row_sums; p.row_ws = nullptr;
+  if (a->row_sums)
+    MVIT_REQUIRE(a->dtype == MVIT_BF16 && a->trans_a && a->trans_b && epi == MVIT_EPI_NONE && var == 3,
+                 "gemm: row sums come with a plain bf16 product of two transposed operands");
   if (epi == MVIT_EPI_SWIGLU_BWD && a->workspace) {
     MVIT_REQUIRE(mvit_aligned16(a->workspace) && a->workspace_bytes >= (int64_t)sizeof(float) * tm * a->ldc,
                  "gemm: SWIGLU_BWD column sums need a workspace of %lld bytes", (long long)(sizeof(float) * tm * a->ldc));
@@ -1342,13 +1353,14 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
     MVIT_REQUIRE(epi == MVIT_EPI_NONE || epi == MVIT_EPI_BIAS || epi == MVIT_EPI_BIAS_RES,
                  "gemm: split_k is available with the plain, bias and bias + residual epilogues (got %d)", epi);
     if (epi != MVIT_EPI_NONE) MVIT_REQUIRE(a->bias, "gemm: split_k with epilogue %d needs bias", epi);
-    MVIT_REQUIRE(a->workspace && mvit_aligned16(a->workspace) && a->workspace_bytes >= (int64_t)sizeof(float) * slices * a->M * a->N,
-                 "gemm: split_k=%d needs a 16-byte aligned workspace of %lld bytes", a->split_k, (long long)(sizeof(float) * slices * a->M * a->N));
+    MVIT_REQUIRE(a->workspace && mvit_aligned16(a->workspace) && a->workspace_bytes >= (int64_t)sizeof(float) * slices * a->M * (a->N + (a->row_sums ? 1 : 0)),
+                 "gemm: split_k=%d needs a 16-byte aligned workspace of %lld bytes", a->split_k, (long long)(sizeof(float) * slices * a->M * (a->N + (a->row_sums ? 1 : 0))));
     MVIT_REQUIRE(tm * tn * slices < (1ll << 30), "gemm: too many tiles");
     if (slices > 1) {
       // the main kernel leaves fp32 partial tiles; the reduction over the slices applies the epilogue
       p.split_k = (int)slices; p.k_chunk = chunk; p.workspace = static_cast<float*>(a->workspace);
       p.reduce_epi = epi;
+      if (a->row_sums) p.row_ws = p.workspace + slices * a->M * a->N;
       epi = MVIT_EPI_NONE;
     }
   }

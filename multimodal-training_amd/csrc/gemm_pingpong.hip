@@ -44,6 +44,11 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
   constexpr bool HAS_IN = EPI == MVIT_EPI_BIAS_RES || EPI == MVIT_EPI_GELU_BWD;
   constexpr bool HAS_BIAS = EPI == MVIT_EPI_BIAS || EPI == MVIT_EPI_BIAS_RES || EPI == MVIT_EPI_BIAS_GELU || EPI == MVIT_EPI_SWIGLU;
   constexpr int NCOLS = DUAL ? 128 : 256;
+  // sums of A's rows over k (the bias gradient of a weight-gradient product) from the fragments that are in registers anyway:
+  // in the tiles of the first tile column the four waves of a group take one row block of each A half, 4 MFMAs with a vector
+  // of ones beside 64.  In passes of their own the column sums of the gradients took 211 us and six launches per block of the
+  // tower at 65,536 rows, 30 us and eight launches at 256 (forward + backward of the 32 blocks: 672 -> 666 ms and 15.4 -> 13.3).
+  constexpr bool ROW_SUMS = TA && TB && EPI == MVIT_EPI_NONE;
   static_assert(!DUAL || !TB, "SWIGLU takes untransposed operands");
   // stores of an interior tile's epilogue that are issued after the next tile's first loads (memory instructions of a wave
   // complete in order, so a wait for those loads may leave this many more in flight)
@@ -227,6 +232,26 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
         }
     __builtin_amdgcn_s_setprio(0);
   };
+  bool do_rs = false;  // this output tile also sums A's rows
+  // row block wn of the group's four in each A half: the ones stand in rows 0-7 of the first operand for half 0 and in rows
+  // 8-15 for half 1, so that lanes 0-31 end up with the sums of half 0 and lanes 32-63 with those of half 1 (row l % 16)
+  [[maybe_unused]] f32x4 rs;
+  auto row_sums = [&](auto H) {
+    if constexpr (ROW_SUMS) {
+      if (do_rs) {
+        int lane = l;
+        asm volatile("" : "+v"(lane));  // made where it is used rather than held in registers
+        const unsigned o = ((lane >> 3) & 1) == decltype(H)::value ? 0x3f803f80u : 0u;
+        const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{o, o, o, o});
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+          if (wn == a) {
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) rs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, fa[a][ks], rs, 0, 0, 0);
+          }
+      }
+    }
+  };
   // K tile t.  MODE 0: steady, 1: first of the output tile, 2: last but one, 3: last
   auto ktile = [&](auto MODE_, int t) {
     constexpr int MODE = decltype(MODE_)::value;
@@ -248,6 +273,7 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
     pp_wait_vm<MODE == 3 ? 0 : W>();
     pp_barrier();
     mfma(X0{}, X1{}, fb[1], F{});
+    row_sums(X0{});
     pp_barrier();
     // phase 2
     read_a(fa, 1);
@@ -261,6 +287,7 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
     if constexpr (MODE != 3) pp_wait_vm<MODE == 2 ? 4 : W>();
     pp_barrier();
     mfma(X1{}, X0{}, fb[0], F{});
+    row_sums(X1{});
     pp_barrier();
     st = other;
   };
@@ -275,6 +302,10 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
     const int slice = next_slice, bias_now = bias_buf;
     n_kt = T_;
     st = 0;
+    if constexpr (ROW_SUMS) {
+      do_rs = p.row_sums != nullptr && n0 == 0;
+      rs = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     pp_wait_vm<(8 + TRAILING < 63 ? 8 + TRAILING : 63)>();
     pp_barrier();
     pp_barrier();
@@ -319,6 +350,15 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
         }
       }
     };
+    if constexpr (ROW_SUMS) {
+      if (do_rs) {
+        const int64_t m = m_lane + (g4 >> 1) * 128 + wn * 16;
+        if ((g4 & 1) == 0 && m < p.M) {  // stores that the next tile's waits do not count only make them wait for more
+          if (to_ws) p.row_ws[(int64_t)slice * p.M + m] = rs[0];
+          else static_cast<TO*>(p.row_sums)[m] = from_f32<TO>(rs[0]);
+        }
+      }
+    }
     if (interior) {
       if constexpr (HAS_IN) {
         // the input was written a few launches ago and is often still in the memory-side cache: a plain load finds it there

@@ -176,6 +176,12 @@ __global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(cons
     }
   }
 
+  // sums of A's rows over k, see gemm_pingpong.hip: wave wn of a row group takes row block wn, 2 MFMAs more per K tile
+  constexpr bool ROW_SUMS = TA && TB && EPI == MVIT_EPI_NONE;
+  static_assert(!ROW_SUMS || NA == S::WGN, "one row block per wave of a row group");
+  const bool do_rs = ROW_SUMS && p.row_sums != nullptr && tn == 0;
+  [[maybe_unused]] f32x4 rs = {0.f, 0.f, 0.f, 0.f};
+
   // ---- main loop
   f32x4 acc[NA][NB];
 #pragma unroll
@@ -213,6 +219,18 @@ __global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(cons
       for (int a = 0; a < NA; ++a)
 #pragma unroll
         for (int b = 0; b < NB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[b][ks], fa[a][ks], acc[a][b], 0, 0, 0);
+    if constexpr (ROW_SUMS) {
+      if (do_rs) {
+        const bf16_t one = (bf16_t)1.f;
+        const bf16x8 ones = {one, one, one, one, one, one, one, one};
+#pragma unroll
+        for (int a = 0; a < NA; ++a)
+          if (wn == a) {
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) rs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, fa[a][ks], rs, 0, 0, 0);
+          }
+      }
+    }
     __builtin_amdgcn_sched_barrier(0);
     st = st + S::STAGE == S::LDS ? 0 : st + S::STAGE;
     st_in = st_in + S::STAGE == S::LDS ? 0 : st_in + S::STAGE;
@@ -221,6 +239,13 @@ __global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(cons
   // ---- epilogue
   float* ws = to_ws ? p.workspace + (int64_t)slice * p.M * p.N : nullptr;
   float no_cs[16];
+  if constexpr (ROW_SUMS) {
+    const int64_t m = m0 + wm * S::WM + wn * 16 + i16;
+    if (do_rs && g4 == 0 && m < p.M) {
+      if (to_ws) p.row_ws[(int64_t)slice * p.M + m] = rs[0];
+      else static_cast<TO*>(p.row_sums)[m] = from_f32<TO>(rs[0]);
+    }
+  }
 #pragma unroll
   for (int it = 0; it < ITEMS; ++it) {
     const int a = it / NG, g = it % NG;

@@ -291,27 +291,24 @@ def _block_backward(dx2: torch.Tensor, x: torch.Tensor, saved: tuple, W: BlockWe
             side.wait_event(ev)
             return fn()
 
-    def wgrad(dy, act, out, **kw):
-        ops.gemm(dy, act, out, trans_a=True, trans_b=True, split_k=ops.wgrad_split_k(out.shape[0], out.shape[1], S), **kw)
-
     # ---- MLP: x2 = x1 + down(silu(g) * u)
     g_wd = torch.empty(C, I, dtype=gdt["mlp.down_proj.weight"], device=dev)
-    g_bd = off_chain(lambda: (ops.colsum(dx2, gdt["mlp.down_proj.bias"]), wgrad(dx2, h, g_wd, n=I))[0])
+    g_bd = off_chain(lambda: ops.weight_grad(dx2, h, g_wd, gdt["mlp.down_proj.bias"], n=I))
     dgu = torch.empty(S, 2 * Ipad, dtype=x.dtype, device=dev)
-    # with many rows the epilogue also hands back per-tile column sums of dgu: the gate / up bias gradient without re-reading dgu
+    # with many rows the epilogue also hands back per-tile column sums of dgu in fp32: the gate / up bias gradient
     fused = x.dtype == torch.bfloat16 and ops.swiglu_bwd_sums_columns(S, Ipad, C)
     part = torch.empty(-(-S // 256), 2 * Ipad, dtype=torch.float32, device=dev) if fused else None
     ops.gemm(dx2, W.wdown, dgu, trans_b=True, epilogue=E.EPI_SWIGLU_BWD, residual=gu, aux_off=Ipad, colsum_partial=part)
     g_wgu = torch.empty(2 * Ipad, C, dtype=gdt["mlp.gate_proj.weight"], device=dev)
-    bgrad = (lambda: ops.reduce_partials(part, gdt["mlp.gate_proj.bias"])) if fused else (lambda: ops.colsum(dgu, gdt["mlp.gate_proj.bias"]))
-    g_bgu = off_chain(lambda: (bgrad(), wgrad(dgu, n2, g_wgu))[0])
+    b_gu = gdt["mlp.gate_proj.bias"]
+    g_bgu = off_chain(lambda: (ops.reduce_partials(part, b_gu), ops.weight_grad(dgu, n2, g_wgu, None))[0] if fused else ops.weight_grad(dgu, n2, g_wgu, b_gu))
     dn2 = torch.empty_like(x)
     ops.gemm(dgu, W.wgu, dn2, trans_b=True)
     dx1, g_n2 = ops.rmsnorm_bwd(dn2, x1, W.norm2.view(-1), rstd2, dx_add=dx2, w_grad_dtype=gdt["norm2.weight"])
 
     # ---- attention: x1 = x + proj(attn(rope(qkv(norm1(x)))))
     g_wp = torch.empty(C, C, dtype=gdt["attn.proj.weight"], device=dev)
-    g_bp = off_chain(lambda: (ops.colsum(dx1, gdt["attn.proj.bias"]), wgrad(dx1, o, g_wp))[0])
+    g_bp = off_chain(lambda: ops.weight_grad(dx1, o, g_wp, gdt["attn.proj.bias"]))
     d_o = dn2  # reuse the buffer
     ops.gemm(dx1, W.wproj, d_o, trans_b=True)
     dqkv = torch.empty_like(qkv)
@@ -320,7 +317,7 @@ def _block_backward(dx2: torch.Tensor, x: torch.Tensor, saved: tuple, W: BlockWe
     # dq arrives as the gradient with respect to the scaled, rotated queries: the same factor on the way back
     ops.rope_(dqkv, geo.cos, geo.sin, 2 * H, hd, backward=True, lead_heads=H, lead_scale=hd**-0.5 * LOG2E)
     g_wqkv = torch.empty(3 * C, C, dtype=gdt["attn.q_proj.weight"], device=dev)
-    g_bqkv = off_chain(lambda: (ops.colsum(dqkv, gdt["attn.q_proj.bias"]), wgrad(dqkv, n1, g_wqkv))[0])
+    g_bqkv = off_chain(lambda: ops.weight_grad(dqkv, n1, g_wqkv, gdt["attn.q_proj.bias"]))
     dn1 = d_o
     ops.gemm(dqkv, W.wqkv, dn1, trans_b=True)
     dx, g_n1 = ops.rmsnorm_bwd(dn1, x, W.norm1.view(-1), rstd1, dx_add=dx1, w_grad_dtype=gdt["norm1.weight"])
@@ -479,14 +476,12 @@ class MergerFn(torch.autograd.Function):
         ctx.saved = None
         dy = dy.contiguous()
         dev = x.device
-        g_b2 = ops.colsum(dy, ctx.gdt[4])
         g_w2 = torch.empty(W2.shape, dtype=ctx.gdt[3], device=dev)
-        ops.gemm(dy, y1, g_w2, trans_a=True, trans_b=True, split_k=ops.wgrad_split_k(g_w2.shape[0], g_w2.shape[1], dy.shape[0]))
+        g_b2 = ops.weight_grad(dy, y1, g_w2, ctx.gdt[4])
         dz = torch.empty_like(z)
         ops.gemm(dy, W2, dz, trans_b=True, epilogue=E.EPI_GELU_BWD, residual=z)
-        g_b0 = ops.colsum(dz, ctx.gdt[2])
         g_w0 = torch.empty(W0.shape, dtype=ctx.gdt[1], device=dev)
-        ops.gemm(dz, ln2, g_w0, trans_a=True, trans_b=True, split_k=ops.wgrad_split_k(g_w0.shape[0], g_w0.shape[1], dz.shape[0]))
+        g_b0 = ops.weight_grad(dz, ln2, g_w0, ctx.gdt[2])
         dln = torch.empty_like(ln2)
         ops.gemm(dz, W0, dln, trans_b=True)
         dx, g_ln = ops.rmsnorm_bwd(dln.view(x.shape), x, lw, rstd, w_grad_dtype=ctx.gdt[0])

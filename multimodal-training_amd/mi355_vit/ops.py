@@ -305,12 +305,14 @@ def gemm(
     n: Optional[int] = None,
     split_k: int = 1,
     colsum_partial: Optional[torch.Tensor] = None,
+    row_sums: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
     """out[M, N] = epilogue(A . B^T) with A = a (or a^T if trans_a) and B = b (or b^T if trans_b), see include/mi355_vit.h.
 
     Shapes: a [M,K] (or [K,M]); b [N,K] (or [K,N]); all 2-D with unit column stride (row strides free).
     ``n`` narrows the logical N (columns of B / out) below b's extent.
     ``colsum_partial`` (EPI_SWIGLU_BWD only): fp32 [ceil(M/256), out.stride(0)] receiving per-tile column sums of out.
+    ``row_sums`` (bf16, both operands transposed, plain epilogue): [M] of out's dtype, receives the sums of op(A) over k.
     """
     for t, nm in ((a, "a"), (b, "b"), (out, "out")):
         _rowmajor(t, f"gemm {nm}")
@@ -356,8 +358,12 @@ def gemm(
     if split_k > 1:
         if epilogue not in (_lib.EPI_NONE, _lib.EPI_BIAS, _lib.EPI_BIAS_RES):
             raise ValueError("gemm: split_k needs the plain, the bias or the bias + residual epilogue")
-        ws = torch.empty(split_k * M * N, dtype=torch.float32, device=a.device)
+        ws = torch.empty(split_k * M * (N + (row_sums is not None)), dtype=torch.float32, device=a.device)
         args.workspace, args.workspace_bytes, args.split_k = ws.data_ptr(), ws.numel() * 4, split_k
+    if row_sums is not None:
+        if row_sums.dtype != out.dtype or row_sums.shape != (M,) or not row_sums.is_contiguous() or row_sums.device != a.device:
+            raise ValueError(f"gemm: row_sums must be contiguous [{M}] of out's dtype")
+        args.row_sums = row_sums.data_ptr()
     if colsum_partial is not None:
         if epilogue != _lib.EPI_SWIGLU_BWD:
             raise ValueError("gemm: colsum_partial is an output of the SwiGLU-backward epilogue only")
@@ -383,6 +389,17 @@ def wgrad_split_k(out_rows: int, out_cols: int, k: int) -> int:
 def swiglu_bwd_sums_columns(rows: int, cols: int, k: int) -> bool:
     """Whether the bf16 SwiGLU-backward product of this shape hands back the column sums of its result (many rows)."""
     return bool(_lib.load().mvit_gemm_swiglu_bwd_sums_columns(rows, cols, k))
+
+
+def weight_grad(dy: torch.Tensor, act: torch.Tensor, out: torch.Tensor, bias_dtype: Optional[torch.dtype], n: Optional[int] = None) -> Optional[torch.Tensor]:
+    """Gradients of a Linear layer's weight (``out`` = dy^T act) and, with ``bias_dtype``, bias (returned: the column sums of
+    dy).  In bf16 the product sums the operand it reads anyway."""
+    fused = dy.dtype == torch.bfloat16 and bias_dtype == out.dtype
+    bias = None
+    if bias_dtype is not None:
+        bias = torch.empty(dy.shape[1], dtype=bias_dtype, device=dy.device) if fused else colsum(dy, bias_dtype)
+    gemm(dy, act, out, trans_a=True, trans_b=True, n=n, split_k=wgrad_split_k(out.shape[0], out.shape[1], dy.shape[0]), row_sums=bias if fused else None)
+    return bias
 
 
 # ------------------------------------------------------------------------------ attention

@@ -421,6 +421,28 @@ def test_gemm_wgrad_layout(dtype, odt, S, No, Ni):
     assert max_rel_err(out, dy.double().t() @ x.double()[:, :Ni]) < TOL[dtype]
 
 
+@pytest.mark.parametrize("odt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("split_k", [1, 3])
+@pytest.mark.parametrize("S,No,Ni", [(1, 8, 8), (63, 130, 72), (1000, 1280, 1280), (515, 3840, 256), (2052, 1280, 3420), (4100, 264, 4096), (20011, 3840, 1280)])
+def test_gemm_wgrad_row_sums(odt, split_k, S, No, Ni):
+    """The bias gradient that comes with a weight gradient: fp32 sums of bf16 values, whatever tile computed them."""
+    _announce(f"gemm row sums {odt} S={S} No={No} Ni={Ni} split_k={split_k}")
+    ops = _ops()
+    ld = -(-No // 8) * 8
+    dy, act = _rand((S, ld), torch.bfloat16, 0)[:, :No], _rand((S, -(-Ni // 8) * 8), torch.bfloat16, 1)[:, :Ni]
+    dy_dev, act_dev = dy.to(DEV), act.to(DEV)
+    dy_dev, act_dev = (torch.nn.functional.pad(t, (0, -t.shape[1] % 8))[:, : t.shape[1]] for t in (dy_dev, act_dev))
+    out, plain = (torch.full((No, Ni), float("nan"), dtype=odt, device=DEV) for _ in range(2))
+    sums = torch.full((No,), float("nan"), dtype=odt, device=DEV)
+    ops.gemm(dy_dev, act_dev, out, trans_a=True, trans_b=True, split_k=split_k, row_sums=sums)
+    ops.gemm(dy_dev, act_dev, plain, trans_a=True, trans_b=True, split_k=split_k)
+    assert torch.equal(out, plain)  # the product itself is not touched
+    want, size = dy.double().sum(0), dy.double().abs().sum(0)
+    # S - 1 fp32 additions in some order, then one rounding to the output type
+    bound = size * (S * 2.0**-24) + want.abs() * (2.0**-8 if odt == torch.bfloat16 else 2.0**-23)
+    assert bool(((sums.cpu().double() - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_gemm_gelu_and_swiglu_epilogues(dtype):
     ops = _ops()
