@@ -2,6 +2,9 @@
 // WM x WN, K tiles of 64 in a ring of NST LDS stages filled by direct global -> LDS loads up to NST - 1 K tiles ahead.
 // Two work-groups share a compute unit: one multiplies while the other waits for LDS or memory (reading the next K tile's
 // fragments ahead inside one work-group, and deeper rings with one work-group per unit, measured no better).
+// A wave's tile is as square as its registers allow, because LDS reads are the next limit: 128 x 128 split in eight waves of
+// 32 x 64 read 96 KiB per K tile, in four of 64 x 64 64 KiB (4,096 rows, two transposed-layout operands, K = 6848: 84 -> 77 us;
+// K contiguous in both, K = 3424: 55 -> 52; weight gradient of 3840 x 1280 over 2,048 rows: 32 -> 27).
 // What bounds it is the chain of K steps of one tile, not the matrix pipe: small tiles make the step short (a 64 x 64 tile's
 // step moves 16 KiB into LDS, the 256 x 256 tile's 64 KiB) and put more compute units to work.
 // Fragment layouts, K order, MFMA form and epilogue arithmetic are those of gemm_pp_kernel (gemm_pingpong.hip), so the results
@@ -176,11 +179,14 @@ __global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(cons
     }
   }
 
-  // sums of A's rows over k, see gemm_pingpong.hip: wave wn of a row group takes row block wn, 2 MFMAs more per K tile
+  // sums of A's rows over k, see gemm_pingpong.hip: wave wn of a row group takes NRS row blocks, two MFMAs more each per K tile
   constexpr bool ROW_SUMS = TA && TB && EPI == MVIT_EPI_NONE;
-  static_assert(!ROW_SUMS || NA == S::WGN, "one row block per wave of a row group");
+  constexpr int NRS = NA / S::WGN;  // row blocks that a wave sums
+  static_assert(!ROW_SUMS || NA % S::WGN == 0, "the waves of a row group share its row blocks");
   const bool do_rs = ROW_SUMS && p.row_sums != nullptr && tn == 0;
-  [[maybe_unused]] f32x4 rs = {0.f, 0.f, 0.f, 0.f};
+  [[maybe_unused]] f32x4 rs[ROW_SUMS ? NRS : 1];
+#pragma unroll
+  for (int i = 0; i < (ROW_SUMS ? NRS : 1); ++i) rs[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // ---- main loop
   f32x4 acc[NA][NB];
@@ -225,9 +231,9 @@ __global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(cons
         const bf16x8 ones = {one, one, one, one, one, one, one, one};
 #pragma unroll
         for (int a = 0; a < NA; ++a)
-          if (wn == a) {
+          if (wn == a / NRS) {
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) rs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, fa[a][ks], rs, 0, 0, 0);
+            for (int ks = 0; ks < 2; ++ks) rs[a % NRS] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, fa[a][ks], rs[a % NRS], 0, 0, 0);
           }
       }
     }
@@ -240,10 +246,13 @@ __global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(cons
   float* ws = to_ws ? p.workspace + (int64_t)slice * p.M * p.N : nullptr;
   float no_cs[16];
   if constexpr (ROW_SUMS) {
-    const int64_t m = m0 + wm * S::WM + wn * 16 + i16;
-    if (do_rs && g4 == 0 && m < p.M) {
-      if (to_ws) p.row_ws[(int64_t)slice * p.M + m] = rs[0];
-      else static_cast<TO*>(p.row_sums)[m] = from_f32<TO>(rs[0]);
+#pragma unroll
+    for (int i = 0; i < NRS; ++i) {
+      const int64_t m = m0 + wm * S::WM + (wn * NRS + i) * 16 + i16;
+      if (do_rs && g4 == 0 && m < p.M) {
+        if (to_ws) p.row_ws[(int64_t)slice * p.M + m] = rs[i][0];
+        else static_cast<TO*>(p.row_sums)[m] = from_f32<TO>(rs[i][0]);
+      }
     }
   }
 #pragma unroll
@@ -286,7 +295,7 @@ namespace {
 
 using Small64 = SmallCfg<64, 64, 2, 2, 4>;      // 64 KiB of LDS
 using Small64x128 = SmallCfg<64, 128, 2, 2, 3>;  // 72 KiB
-using Small128 = SmallCfg<128, 128, 4, 2, 2>;    // 64 KiB
+using Small128 = SmallCfg<128, 128, 2, 2, 2>;    // 64 KiB
 
 template <typename TO, bool TA, bool TB, int EPI, typename S>
 int launch_small(const GemmParams& p, hipStream_t stream) {
