@@ -1184,12 +1184,12 @@ bool pp_takes(GemmTiledKind kind, int64_t k_chunk, int64_t k_last) {  // at leas
 // Modelled times (us) of the tiles on one MI355X, fitted to every tile's time at 256 ... 16,384 rows of the tower's products: a
 // step of 64 along K takes 1.15 us in a 256 x 256 tile (one work-group per compute unit; 1.2 with both operands behind the
 // transposing LDS read), and in the smaller ones `one` us while every unit has at most one work-group and `two` us once it has
-// two; operands with k contiguous (no transposing read) are slower there.  A fuller last round, a shorter step and more units
-// at work all lower the estimate; the epilogue of a 256 x 256 tile is the longest.  The line between the tiles follows from
-// these numbers and not from any shape: e.g. input gradients of 1280 columns, K = 3840, are fastest on 64 x 64 up to 1,500 rows,
-// on 64 x 128 to 3,100, on 128 x 128 to 6,500 and on 256 x 256 at 8,192 (us at 256 / 1,024 / 2,048 / 4,096 / 8,192 rows: 19 / 26 /
-// 35 / 47 / 80, with 256 x 256 tiles alone 69 / 69 / 69 / 70 / 80); weight gradients of 3840 x 1280 over 4,096 rows take 49 us
-// in one slice on 128 x 128 and 57 in three on 256 x 256, over 8,192 rows 93 and 87.
+// two.  A fuller last round, a shorter step and more units at work all lower the estimate; the epilogue of a 256 x 256 tile is
+// the longest.  The line between the tiles follows from these numbers and not from any shape: e.g. input gradients of 1280
+// columns, K = 3840, are fastest on 64 x 64 up to 1,500 rows, on 64 x 128 to 3,100, on 128 x 128 to 6,500 and on 256 x 256 at
+// 8,192 (us at 256 / 1,024 / 2,048 / 4,096 / 8,192 rows: 19 / 26 / 35 / 47 / 80, with 256 x 256 tiles alone 69 / 69 / 69 / 70 / 80);
+// weight gradients of 3840 x 1280 over 4,096 rows take 49 us in one slice on 128 x 128 and 57 in three on 256 x 256, over 8,192
+// rows 93 and 87.
 struct TileChoice {
   int bm, bn;
   double us;
@@ -1206,15 +1206,15 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
     if (rest > 0) us += steps * (two > 0. && rest > n_cu ? two : one) + per_tile;
     if (us < best.us) best = TileChoice{bm, bn, us};
   };
-  const bool nn = kind <= NN_SWIGLU, swiglu = kind == NN_SWIGLU;
+  const bool swiglu = kind == NN_SWIGLU;
   if (pp_takes(kind, k_chunk, k_last)) consider(256, 256, tt ? 1.2 : 1.15, 0., swiglu ? 11. : 7.);
   if (kind == NT_SWIGLU_BWD) {  // two inputs and two outputs per element lengthen its epilogue
     consider(64, 64, 0.30, 0.43, 2.);
     consider(64, 128, 0.46, 0.57, 2.);
   } else {
-    if (!swiglu) consider(64, 64, 0.23, nn ? 0.40 : 0.36, 2.);
-    consider(64, 128, nn ? 0.35 : 0.40, nn ? 0.66 : 0.52, 2.);
-    consider(128, 128, nn ? 0.66 : 0.60, nn ? 0.88 : 0.72, swiglu ? 4.5 : 2.5);
+    if (!swiglu) consider(64, 64, 0.23, 0.36, 2.);
+    consider(64, 128, 0.37, 0.52, 2.);
+    consider(128, 128, 0.60, 0.72, swiglu ? 6. : 2.5);
   }
   // SwiGLU backward of many rows: the 256-row kernel, which also sums the columns of its result
   if (kind == NT_SWIGLU_BWD) {

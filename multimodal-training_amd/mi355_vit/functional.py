@@ -26,6 +26,16 @@ def round_up(v: int, m: int) -> int:
     return (v + m - 1) // m * m
 
 
+def padded_inner(inner: int) -> int:
+    """Columns that a block's gate, up and hidden activations are laid out in: whole 128-byte cache lines of bf16 for MLPs wide
+    enough that the padding is small, else the 8 columns that 16-byte accesses need.  Rows of 3,424 columns (3,420 rounded up
+    to 8) begin in the middle of a line every other time, and a K tile of the down projection, 128 bytes of each row, then
+    touches two (us at 4,096 / 16,384 / 65,536 rows: 53 / 162 / 479 with 3,424 columns, 43 / 138 / 460 with 3,456; SwiGLU
+    backward 61 / 225 / 779 and 59 / 219 / 760; the products that grow with the padding, gate/up forward and input gradient,
+    take 1 % more)."""
+    return round_up(inner, 64 if inner >= 512 else 8)
+
+
 @dataclass
 class BlockWeights:
     """Compute-dtype operands of one block, laid out for the fused GEMMs.
@@ -76,7 +86,7 @@ def pack_block_weights(params: List[torch.Tensor], dtype: torch.dtype, into: Opt
     (n1, n2, wq, bq, wk, bk, wv, bv, wp, bp, wg, bg, wu, bu, wd, bd) = params
     C = wq.shape[1]
     I = wg.shape[0]
-    Ipad = round_up(I, 8)
+    Ipad = padded_inner(I)
     dev = wq.device
     alias = all(p.dtype == dtype and p.is_contiguous() for p in (n1, n2, wp, bp, bd))
     if into is None or into.wqkv.dtype != dtype or into.wqkv.device != dev or into.alias != alias:
