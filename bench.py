@@ -129,15 +129,15 @@ def measured_traffic_bytes(workload: str, tag: str):
 
 
 KERNEL_NAMES = {
-    "gemm_nn_epi0": "gemm_dl_kernel<TO, TA=false, TB=false, EPI=NONE>",
-    "gemm_nn_epi1": "gemm_dl_kernel<TO, TA=false, TB=false, EPI=BIAS>",
-    "gemm_nn_epi2": "gemm_dl_kernel<TO, TA=false, TB=false, EPI=BIAS_RES>",
-    "gemm_nn_epi3": "gemm_dl_kernel<TO, TA=false, TB=false, EPI=BIAS_GELU>",
-    "gemm_nn_epi4": "gemm_dl_kernel<TO, TA=false, TB=false, EPI=SWIGLU>",
-    "gemm_nt_epi0": "gemm_dl_kernel<TO, TA=false, TB=true, EPI=NONE, MI16>",
+    "gemm_nn_epi0": "gemm_pp_kernel / gemm_small_kernel<TO, TA=false, TB=false, EPI=NONE>",
+    "gemm_nn_epi1": "gemm_pp_kernel / gemm_small_kernel<TO, TA=false, TB=false, EPI=BIAS>",
+    "gemm_nn_epi2": "gemm_pp_kernel / gemm_small_kernel<TO, TA=false, TB=false, EPI=BIAS_RES>",
+    "gemm_nn_epi3": "gemm_pp_kernel / gemm_small_kernel<TO, TA=false, TB=false, EPI=BIAS_GELU>",
+    "gemm_nn_epi4": "gemm_pp_kernel / gemm_small_kernel<TO, TA=false, TB=false, EPI=SWIGLU>",
+    "gemm_nt_epi0": "gemm_pp_kernel / gemm_small_kernel<TO, TA=false, TB=true, EPI=NONE>",
     "gemm_nt_epi5": "gemm_dl_kernel<TO, TA=false, TB=true, EPI=SWIGLU_BWD>",
-    "gemm_nt_epi6": "gemm_dl_kernel<TO, TA=false, TB=true, EPI=GELU_BWD>",
-    "gemm_tt_epi0": "gemm_dl_kernel<TO, TA=true, TB=true, EPI=NONE, MI16> + splitk_reduce_kernel",
+    "gemm_nt_epi6": "gemm_pp_kernel / gemm_small_kernel<TO, TA=false, TB=true, EPI=GELU_BWD>",
+    "gemm_tt_epi0": "gemm_pp_kernel / gemm_small_kernel<TO, TA=true, TB=true, EPI=NONE> + splitk_reduce_kernel",
     "attn_fwd_full": "attn_fwd_x32<5> (segments >= 512 tokens), attn_fwd_mfma<5, 8, 32, true, 2, 4> (shorter)",
     "attn_bwd_full": "attn_delta_rows_kernel + attn_bwd_prepare_kernel + attn_bwd_dkdv_wide<5> + attn_bwd_dq_wide<5>",
     "attn_fwd_window": "attn_fwd_mfma<5, 2, 64, false, 2, 4>",

@@ -421,6 +421,54 @@ def test_gemm_wgrad_layout(dtype, odt, S, No, Ni):
     assert max_rel_err(out, dy.double().t() @ x.double()[:, :Ni]) < TOL[dtype]
 
 
+@pytest.mark.parametrize("layout", ["nn", "nt", "tt"])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (63, 72, 64), (65, 136, 72), (129, 264, 200), (257, 8, 136), (300, 6912, 136), (1030, 1288, 1280), (4100, 1288, 200), (5000, 3848, 1224)])
+def test_gemm_tile_edges(layout, M, N, K):
+    """Edges of every bf16 tile (64 to 256 rows and columns, K tiles of 64), result rows beyond the matrix left alone."""
+    _announce(f"gemm edges {layout} {M}x{N}x{K}")
+    ops = _ops()
+    ta, tb = layout[0] == "t", layout[1] == "t"
+    up = lambda v: -(-v // 8) * 8  # noqa: E731
+    a = _rand((K, up(M)), torch.bfloat16, 0)[:, :M] if ta else _rand((M, K), torch.bfloat16, 0)
+    b = _rand((K, N), torch.bfloat16, 1) if tb else _rand((N, K), torch.bfloat16, 1)
+    a_dev = torch.empty((K, up(M)) if ta else (M, K), dtype=torch.bfloat16, device=DEV)[:, : a.shape[1]]
+    a_dev.copy_(a)
+    full = torch.full((M + 3, N + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.gemm(a_dev, b.to(DEV), full[:M, :N], trans_a=ta, trans_b=tb)
+    A, B = (a.T if ta else a).double(), (b if tb else b.T).double()
+    want, size = A @ B, A.abs() @ B.abs()
+    # K fp32 additions in some order, then one rounding to bf16
+    assert bool(((full[:M, :N].cpu().double() - want).abs() <= size * (K * 2.0**-24) + want.abs() * 2.0**-8).all())
+    assert bool((full[M:] == 7.0).all()) and bool((full[:, N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("unit,offset", [(16, 0), (16, 4), (4, 0), (2, 2), (1, 1)])
+@pytest.mark.parametrize("n", [1, 5, 96, 97, 200])
+def test_copy_ranges_bit_exact(unit, offset, n):
+    """Every word size that the ranges' addresses and lengths leave, whole and partial pieces, more ranges than one launch takes."""
+    import ctypes
+
+    from mi355_vit import _lib
+
+    _announce(f"copy ranges unit={unit} offset={offset} n={n}")
+
+    class Range(ctypes.Structure):
+        _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p), ("bytes", ctypes.c_int64)]
+
+    lengths = [unit * (0 if i % 7 == 3 else [1, 3, 2047, 2048, 2049, 5000][i % 6]) for i in range(n)]
+    total = offset + sum(lengths)
+    src = torch.randint(0, 256, (total + 16,), dtype=torch.uint8, device=DEV)
+    dst, want = torch.full_like(src, 9), torch.full_like(src, 9)
+    ranges, at, to = (Range * n)(), offset, total  # taken in order, laid down in reverse
+    for i, length in enumerate(lengths):
+        to -= length
+        ranges[i] = Range(src.data_ptr() + at, dst.data_ptr() + to, length)
+        want[to : to + length] = src[at : at + length]
+        at += length
+    _lib.check(_lib.load().mvit_copy_ranges(ctypes.addressof(ranges), n, torch.cuda.current_stream().cuda_stream), "mvit_copy_ranges")
+    assert torch.equal(dst, want)
+
+
 @pytest.mark.parametrize("odt", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("split_k", [1, 3])
 @pytest.mark.parametrize("S,No,Ni", [(1, 8, 8), (63, 130, 72), (1000, 1280, 1280), (515, 3840, 256), (2052, 1280, 3420), (4100, 264, 4096), (20011, 3840, 1280)])
