@@ -1,22 +1,23 @@
 // fp32 GEMM (the parity path) on v_mfma_f32_16x16x4_f32:  C[M,N] = epi( sum_k A[m,k] * B[n,k] ).
 //
 // What bounds it is the fp32 matrix rate (157 TFLOP/s, a sixteenth of bf16's) once enough compute units have work: a
-// 64 x 64 tile per work-group of four waves keeps the matrix pipes of its unit busy (a K tile of 32 is 1,024 cycles of MFMA
-// and 16 KiB of operands), and 512 rows of the tower already give 160 to 1,700 of them.
+// 64 x 64 tile per work-group of four waves (a K tile of 32 is 1,024 cycles of MFMA and 16 KiB of operands), or a 32 x 64 tile
+// where there are few of those (half_rows below).
 // K tiles of 32 floats (128-byte rows) in a ring of four LDS stages filled by direct global -> LDS loads, two work-groups
 // per compute unit.  MFMA (s, j) of a K tile contracts k = 16 s + 4 g + j over the lane groups g = 0..3, so one 16-byte read
 // of a [row][k] operand feeds four of them; a [k][row] operand is read as two neighbouring rows (8 bytes) per k, and the two
 // row blocks of a wave are its even and its odd rows.
 // The products are computed transposed (B's fragment first), so a lane ends with eight consecutive columns of a row and
-// stores them from registers.  One tile shape for every size: a row's result does not depend on its batch.
+// stores them from registers.  Both tiles add in the same order: a row's result does not depend on its batch.
 #include "gemm_direct.h"
 
 namespace {
 
-template <int WGM_, int WGN_>
+template <int BM_, int WGM_, int WGN_>
 struct F32Cfg {
-  static constexpr int BM = 64, BN = 64, BK = 32, NST = 4, NTHREADS = 256, WGM = WGM_, WGN = WGN_, WM = BM / WGM, WN = BN / WGN;
-  static constexpr int OPERAND = 64 * 128, STAGE = 2 * OPERAND, LDS = NST * STAGE;
+  static constexpr int BM = BM_, BN = 64, BK = 32, NST = 4, NTHREADS = 256, WGM = WGM_, WGN = WGN_, WM = BM / WGM, WN = BN / WGN;
+  static constexpr int A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128, LDS = NST * STAGE;
+  static constexpr int PER_A = BM / 32, PER_B = 2, PER = PER_A + PER_B;  // 1 KiB loads per wave and K tile
 };
 
 // slot of chunk c (16 bytes) of row `major` ([row][k]: eight chunks) or k-row `major` ([k][row]: sixteen chunks)
@@ -26,12 +27,12 @@ __device__ __forceinline__ int f32_swizzle(int major) {
   return IS_A ? (major >> 1) & 7 : ((major >> 1) & 1) | (((major >> 3) & 3) << 1);
 }
 
-template <bool TA, bool TB, int EPI>
+template <bool TA, bool TB, int EPI, int BM>
 __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmParams p) {
   constexpr bool DUAL = (EPI == MVIT_EPI_SWIGLU);
-  using S = F32Cfg<DUAL ? 4 : 2, DUAL ? 1 : 2>;
+  using S = F32Cfg<BM, DUAL ? 4 : 2, DUAL ? 1 : 2>;
   constexpr int BK = S::BK, NST = S::NST, NA = S::WM / 16, NB = S::WN / 16, NG = DUAL ? 1 : NB / 2, NCOLS = DUAL ? 32 : 64;
-  static_assert(!(TA || TB) || (NA == 2 && NB == 2), "[k][row] operands are read as pairs of rows");
+  static_assert((!TA || NA == 2) && (!TB || NB == 2), "[k][row] operands are read as pairs of rows");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
 
   const unsigned tiles = (unsigned)(p.tiles_m * p.tiles_n), total = tiles * (unsigned)p.split_k, per_xcd = (total + 7) / 8;
@@ -52,51 +53,58 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmParams p) {
   typedef __attribute__((address_space(3))) unsigned char lds_byte;
   const unsigned lds_base = (unsigned)(__UINTPTR_TYPE__)(lds_byte*)smem_raw;
 
-  // ---- loader: two 1 KiB loads per wave, operand and K tile
-  const char *pa[2], *pb[2];
-  int ka[2], kb[2];  // first k of the lane's chunk inside a K tile
+  // ---- loader
+  const char *pa[S::PER_A], *pb[S::PER_B];
+  int ka[S::PER_A], kb[S::PER_B];  // first k of the lane's chunk inside a K tile
   const int64_t step_a = TA ? 4ll * BK * p.lda : 4 * BK, step_b = TB ? 4ll * BK * p.ldb : 4 * BK;
   const int m_left = (int)(p.M - m0 < S::BM ? p.M - m0 : S::BM), n_left = (int)(p.N - n0 < NCOLS ? p.N - n0 : NCOLS);
+  auto place = [&](auto TR, auto IS_A, int q, const void* X, int64_t ld, int64_t row0, int left, int row_of_tile, const char*& ptr, int& k) {
+    const float* x = static_cast<const float*>(X);
+    if (!decltype(TR)::value) {
+      const int c = (l & 7) ^ f32_swizzle<false, decltype(IS_A)::value>(q * 8 + (l >> 3));
+      const int r = row_of_tile < left ? row_of_tile : left - 1;  // rows past the edge repeat the last row: their results are not stored
+      k = c * 4;
+      ptr = reinterpret_cast<const char*>(x + (row0 + r) * ld + k_begin + k);
+    } else {
+      k = q * 4 + (l >> 4);
+      const int c = (l & 15) ^ f32_swizzle<true, decltype(IS_A)::value>(k);
+      ptr = reinterpret_cast<const char*>(x + (k_begin + k) * ld + row0 + (c * 4 < left ? c * 4 : 0));
+    }
+  };
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int q = wv * 2 + j;
-    auto place = [&](auto TR, auto IS_A, const void* X, int64_t ld, int64_t row0, int left, int row_of_tile, const char*& ptr, int& k) {
-      const float* x = static_cast<const float*>(X);
-      if (!decltype(TR)::value) {
-        const int c = (l & 7) ^ f32_swizzle<false, decltype(IS_A)::value>(q * 8 + (l >> 3));
-        const int r = row_of_tile < left ? row_of_tile : left - 1;  // rows past the edge repeat the last row: their results are not stored
-        k = c * 4;
-        ptr = reinterpret_cast<const char*>(x + (row0 + r) * ld + k_begin + k);
-      } else {
-        k = q * 4 + (l >> 4);
-        const int c = (l & 15) ^ f32_swizzle<true, decltype(IS_A)::value>(k);
-        ptr = reinterpret_cast<const char*>(x + (k_begin + k) * ld + row0 + (c * 4 < left ? c * 4 : 0));
-      }
-    };
-    const int row = q * 8 + (l >> 3);
-    place(std::bool_constant<TA>{}, std::true_type{}, p.A, p.lda, m0, m_left, row, pa[j], ka[j]);
+  for (int j = 0; j < S::PER_A; ++j) {
+    const int q = wv * S::PER_A + j;
+    place(std::bool_constant<TA>{}, std::true_type{}, q, p.A, p.lda, m0, m_left, q * 8 + (l >> 3), pa[j], ka[j]);
+  }
+#pragma unroll
+  for (int j = 0; j < S::PER_B; ++j) {
+    const int q = wv * S::PER_B + j, row = q * 8 + (l >> 3);
     // SWIGLU: tile rows 0-31 are gate rows, 32-63 up rows
-    place(std::bool_constant<TB>{}, std::false_type{}, DUAL && q >= 4 ? p.B2 : p.B, p.ldb, n0, n_left, DUAL ? row & 31 : row, pb[j], kb[j]);
+    place(std::bool_constant<TB>{}, std::false_type{}, q, DUAL && q >= 4 ? p.B2 : p.B, p.ldb, n0, n_left, DUAL ? row & 31 : row, pb[j], kb[j]);
   }
   auto issue = [&](int t, unsigned stage_off) {
-    const unsigned da = lds_base + stage_off + wv * 2048, db = da + S::OPERAND;
-    const bool partial = k_tail != 0 && t == n_kt - 1;  // chunks past the end of K are zeros
+    const unsigned da = lds_base + stage_off + wv * (S::PER_A * 1024), db = lds_base + stage_off + S::A_BYTES + wv * (S::PER_B * 1024);
+    if (k_tail != 0 && t == n_kt - 1) {  // the partial K tile: chunks past the end of K are zeros
+      auto load = [&](unsigned at, const char* ptr, int k) {
+        pp_load_at_below(at, ptr, k, k_tail);
+        if (k >= k_tail) *reinterpret_cast<u32x4*>(smem_raw + (at - lds_base) + l * 16) = u32x4{0u, 0u, 0u, 0u};
+      };
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      if (partial) {
-        pp_load_at_below(da + j * 1024, pa[j], ka[j], k_tail);
-        pp_load_at_below(db + j * 1024, pb[j], kb[j], k_tail);
-        unsigned char* at = smem_raw + (da - lds_base) + j * 1024 + l * 16;
-        if (ka[j] >= k_tail) *reinterpret_cast<u32x4*>(at) = u32x4{0u, 0u, 0u, 0u};
-        if (kb[j] >= k_tail) *reinterpret_cast<u32x4*>(at + S::OPERAND) = u32x4{0u, 0u, 0u, 0u};
-      } else {
+      for (int j = 0; j < S::PER_A; ++j) load(da + j * 1024, pa[j], ka[j]);
+#pragma unroll
+      for (int j = 0; j < S::PER_B; ++j) load(db + j * 1024, pb[j], kb[j]);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      return;
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {  // A and B by turns
+      if (j < S::PER_A) {
         pp_load_at(da + j * 1024, pa[j]);
-        pp_load_at(db + j * 1024, pb[j]);
+        pa[j] += step_a;
       }
-      pa[j] += step_a;
+      pp_load_at(db + j * 1024, pb[j]);
       pb[j] += step_b;
     }
-    if (partial) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   };
 #pragma unroll
   for (int t = 0; t < NST - 1; ++t)
@@ -114,11 +122,11 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmParams p) {
   }
   if constexpr (!TB) {
     const int row = wn * S::WN + 8 * (i16 >> 2) + (i16 & 3), f = f32_swizzle<false, false>(row);
-    rb[0] = S::OPERAND + row * 128 + ((g4 ^ f) << 4);
-    rb[1] = S::OPERAND + row * 128 + (((4 + g4) ^ f) << 4);
+    rb[0] = S::A_BYTES + row * 128 + ((g4 ^ f) << 4);
+    rb[1] = S::A_BYTES + row * 128 + (((4 + g4) ^ f) << 4);
   } else {
     const int r = wn * S::WN + 2 * i16;
-    rb[0] = rb[1] = S::OPERAND + 4 * g4 * 256 + (((r >> 2) ^ f32_swizzle<true, false>(4 * g4)) << 4) + (r & 3) * 4;
+    rb[0] = rb[1] = S::A_BYTES + 4 * g4 * 256 + (((r >> 2) ^ f32_swizzle<true, false>(4 * g4)) << 4) + (r & 3) * 4;
   }
 
   f32x4 acc[NA][NB];
@@ -129,8 +137,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmParams p) {
   unsigned st = 0, st_in = (NST - 1) * S::STAGE;  // stage consumed, stage filled
   for (int t = 0; t < n_kt; ++t) {
     const int newer = n_kt - 1 - t;  // K tiles that may still be in flight
-    if (newer >= 2) pp_wait_vm<8>();
-    else if (newer == 1) pp_wait_vm<4>();
+    if (newer >= 2) pp_wait_vm<2 * S::PER>();
+    else if (newer == 1) pp_wait_vm<S::PER>();
     else pp_wait_vm<0>();
     pp_barrier();  // every wave's share of K tile t is in LDS; K tile t - 1 has been consumed
     if (t + NST - 1 < n_kt) issue(t + NST - 1, st_in);
@@ -213,16 +221,36 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmParams p) {
     }
 }
 
-template <bool TA, bool TB, int EPI>
-int launch_f32(GemmParams p, hipStream_t stream) {
+// 32-row tiles where they shorten the launch: while 64-row tiles leave a quarter of the compute units without one, and after that
+// where halving saves part of the last round (us, 64 / 32 rows, input gradients: K = 1280 30 / 21 at 256 rows, 49 / 43 at 1,024,
+// 50 / 58 at 1,536, 76 / 68 at 2,048; K = 6912 145 / 99 at 256 rows, 145 / 140 at 512).  Nearly a tile per unit stays whole: halves
+// are no faster alone (256 rows x 3840: 32 / 31), and beside a second stream's products a step of 256 rows takes 3.19 ms with
+// them and 2.97 without.
+inline bool half_rows(const GemmParams& p) {
+  constexpr int64_t units = 256;
+  const int64_t tn = (p.N + 63) / 64 * p.split_k, tiles = (p.M + 63) / 64 * tn;
+  const int64_t rounds = (tiles + units - 1) / units, half_rounds = ((p.M + 31) / 32 * tn + units - 1) / units;
+  return tiles <= units * 3 / 4 || (rounds > 1 && rounds <= 3 && half_rounds < 2 * rounds);
+}
+
+template <bool TA, bool TB, int EPI, int BM>
+int launch_f32_tiles(GemmParams p, hipStream_t stream) {
   constexpr int NCOLS = EPI == MVIT_EPI_SWIGLU ? 32 : 64;
-  const int64_t tm = (p.M + 63) / 64, tn = (p.N + NCOLS - 1) / NCOLS;
+  const int64_t tm = (p.M + BM - 1) / BM, tn = (p.N + NCOLS - 1) / NCOLS;
   MVIT_REQUIRE(tm * tn * p.split_k < (1ll << 30), "gemm: too many tiles");
   p.tiles_m = (int)tm; p.tiles_n = (int)tn;
   p.panel_w = tn <= 6 ? (int)tn : 4;
-  hipLaunchKernelGGL((gemm_f32_kernel<TA, TB, EPI>), (p.tiles_m * p.tiles_n * p.split_k + 7) / 8 * 8, 256, (F32Cfg<2, 2>::LDS), stream, p);
+  hipLaunchKernelGGL((gemm_f32_kernel<TA, TB, EPI, BM>), (p.tiles_m * p.tiles_n * p.split_k + 7) / 8 * 8, 256, (F32Cfg<BM, 2, 2>::LDS), stream, p);
   MVIT_CHECK_LAUNCH("gemm");
   return MVIT_OK;
+}
+
+template <bool TA, bool TB, int EPI>
+int launch_f32(const GemmParams& p, hipStream_t stream) {
+  if constexpr (!TA && EPI != MVIT_EPI_SWIGLU) {
+    if (half_rows(p)) return launch_f32_tiles<TA, TB, EPI, 32>(p, stream);
+  }
+  return launch_f32_tiles<TA, TB, EPI, 64>(p, stream);
 }
 
 }  // namespace

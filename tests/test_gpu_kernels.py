@@ -442,6 +442,20 @@ def test_gemm_tile_edges(layout, M, N, K):
     assert bool((full[M:] == 7.0).all()) and bool((full[:, N:] == 7.0).all())
 
 
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("N,K", [(1280, 1280), (200, 72), (64, 36)])
+def test_gemm_f32_rows_do_not_depend_on_their_batch(trans_b, N, K):
+    """Few rows take 32-row tiles, many 64-row ones: the same bits, also at the edges of either."""
+    _announce(f"gemm f32 rows N={N} K={K} trans_b={trans_b}")
+    ops = _ops()
+    a, b = _rand((40000 if N < 1280 else 8192, K), torch.float32, 0).to(DEV), _rand((K, N) if trans_b else (N, K), torch.float32, 1).to(DEV)
+    everything = ops.gemm(a, b, torch.empty(a.shape[0], N, device=DEV), trans_b=trans_b)
+    for rows in (1, 31, 32, 33, 64, 65, 100, 513, 1030, 2049):
+        part = torch.full((rows + 1, N), 7.0, device=DEV)
+        ops.gemm(a[:rows], b, part[:rows], trans_b=trans_b)
+        assert torch.equal(part[:rows], everything[:rows]) and bool((part[rows] == 7.0).all()), rows
+
+
 @pytest.mark.parametrize("unit,offset", [(16, 0), (16, 4), (4, 0), (2, 2), (1, 1)])
 @pytest.mark.parametrize("n", [1, 5, 96, 97, 200])
 def test_copy_ranges_bit_exact(unit, offset, n):
