@@ -233,21 +233,24 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
     __builtin_amdgcn_s_setprio(0);
   };
   bool do_rs = false;  // this output tile also sums A's rows
-  // row block wn of the group's four in each A half: the ones stand in rows 0-7 of the first operand for half 0 and in rows
-  // 8-15 for half 1, so that lanes 0-31 end up with the sums of half 0 and lanes 32-63 with those of half 1 (row l % 16)
-  [[maybe_unused]] f32x4 rs;
+  // row block wn of the group's four in each A half, one accumulator per half: every lane's element 0 is the sum of row l % 16.
+  // The first operand is ones throughout, so a row's sum reads that row alone (zeros standing for "the other half's rows" would
+  // carry its infinities and NaNs over: 0 x Inf)
+  [[maybe_unused]] f32x4 rs[2];
   auto row_sums = [&](auto H) {
     if constexpr (ROW_SUMS) {
       if (do_rs) {
-        int lane = l;
-        asm volatile("" : "+v"(lane));  // made where it is used rather than held in registers
-        const unsigned o = ((lane >> 3) & 1) == decltype(H)::value ? 0x3f803f80u : 0u;
+        unsigned o = 0x3f803f80u;
+        asm volatile("" : "+v"(o));  // made where it is used rather than held in registers
         const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{o, o, o, o});
 #pragma unroll
         for (int a = 0; a < 4; ++a)
           if (wn == a) {
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) rs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, fa[a][ks], rs, 0, 0, 0);
+            for (int ks = 0; ks < 2; ++ks) {
+              f32x4& c = rs[decltype(H)::value];
+              c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, fa[a][ks], c, 0, 0, 0);
+            }
           }
       }
     }
@@ -304,7 +307,7 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
     st = 0;
     if constexpr (ROW_SUMS) {
       do_rs = p.row_sums != nullptr && n0 == 0;
-      rs = f32x4{0.f, 0.f, 0.f, 0.f};
+      rs[0] = rs[1] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     pp_wait_vm<(8 + TRAILING < 63 ? 8 + TRAILING : 63)>();
     pp_barrier();
@@ -354,8 +357,9 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
       if (do_rs) {
         const int64_t m = m_lane + (g4 >> 1) * 128 + wn * 16;
         if ((g4 & 1) == 0 && m < p.M) {  // stores that the next tile's waits do not count only make them wait for more
-          if (to_ws) p.row_ws[(int64_t)slice * p.M + m] = rs[0];
-          else static_cast<TO*>(p.row_sums)[m] = from_f32<TO>(rs[0]);
+          const float sum = g4 >> 1 ? rs[1][0] : rs[0][0];
+          if (to_ws) p.row_ws[(int64_t)slice * p.M + m] = sum;
+          else static_cast<TO*>(p.row_sums)[m] = from_f32<TO>(sum);
         }
       }
     }

@@ -505,6 +505,35 @@ def test_gemm_wgrad_row_sums(odt, split_k, S, No, Ni):
     assert bool(((sums.cpu().double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("full_tiles", [False, True])
+@pytest.mark.parametrize("S,No,split_k", [(200, 130, 1), (1000, 386, 1), (1000, 386, 3), (20011, 3834, 3)])
+def test_gemm_wgrad_row_sums_read_their_own_row_only(S, No, split_k, full_tiles, monkeypatch):
+    """Infinities and NaNs of one channel, and whatever stands in the columns that pad a row to 16 bytes, reach no other channel's
+    sum and no other row of the product, in the 256-row tiles as in the small ones."""
+    _announce(f"gemm row sums, poisoned S={S} No={No} split_k={split_k} full_tiles={full_tiles}")
+    ops = _ops()
+    if full_tiles:
+        monkeypatch.setenv("MVIT_GEMM_NO_HALF_TILES", "1")
+    Ni = 264
+    dy = _rand((S, -(-No // 8) * 8), torch.bfloat16, 0).to(DEV)
+    act = _rand((S, Ni), torch.bfloat16, 1).to(DEV)
+
+    def run():
+        out, sums = torch.full((No, Ni), 7.0, device=DEV), torch.full((No,), 7.0, device=DEV)
+        ops.gemm(dy[:, :No], act, out, trans_a=True, trans_b=True, split_k=split_k, row_sums=sums)
+        return out, sums
+
+    dy[:, No:] = 0
+    out, sums = run()
+    dy[:, No:] = float("nan")
+    dy[3, 1], dy[S - 1, No - 1], dy[S // 2, No // 2] = float("inf"), float("nan"), float("-inf")
+    out_p, sums_p = run()
+    keep = torch.ones(No, dtype=torch.bool, device=DEV)
+    keep[[1, No // 2, No - 1]] = False
+    assert torch.equal(sums_p[keep], sums[keep]) and torch.equal(out_p[keep], out[keep])
+    assert sums_p[1] == float("inf") and sums_p[No // 2] == float("-inf") and bool(sums_p[No - 1].isnan())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_gemm_gelu_and_swiglu_epilogues(dtype):
     ops = _ops()
