@@ -29,7 +29,8 @@ def _int64_row(t: torch.Tensor) -> torch.Tensor:
 
 
 def _ranks(input_ids: torch.Tensor, labels: Optional[torch.Tensor], image_token_id: int):
-    """(rank of every token, pinned counts, event after which the host may read them)."""
+    """(rank of every token, pinned counts, event after which the host may read them).  The kernel writes the counts, and the
+    pinned allocator does not know of it: the caller holds them until the event has passed, on every way out."""
     ids = _int64_row(input_ids)
     lab = None
     if labels is not None:
@@ -39,11 +40,11 @@ def _ranks(input_ids: torch.Tensor, labels: Optional[torch.Tensor], image_token_
     n = ids.numel()
     rank = torch.empty(n, dtype=torch.int32, device=ids.device)
     counts = torch.empty(2, dtype=torch.int64, pin_memory=True)  # the kernel writes them where the host reads them
+    ready, stream = torch.cuda.Event(), torch.cuda.current_stream(ids.device)  # nothing between the launch and the record may fail
     rc = _lib.load().mvit_image_token_ranks(ids.data_ptr(), None if lab is None else lab.data_ptr(), n, image_token_id, -100,
                                             rank.data_ptr(), None, counts.data_ptr(), _stream(ids))
     _lib.check(rc, "mvit_image_token_ranks")
-    ready = torch.cuda.Event()
-    ready.record(torch.cuda.current_stream(ids.device))
+    ready.record(stream)
     return rank, counts, ready
 
 
@@ -101,8 +102,10 @@ def merge_vision_embeddings(inputs_embeds: torch.Tensor, input_ids: torch.Tensor
     ranks, counts, ready = _ranks(input_ids, labels, image_token_id)
     # the merge is queued before the host waits for the counts: it stays inside its arrays whatever they are, and its result
     # is dropped when one of the checks below refuses the call
-    merged = _MergeRowsFn.apply(inputs_embeds, vision_embeddings, ranks)
-    ready.synchronize()  # the one host wait (the reference has three)
+    try:
+        merged = _MergeRowsFn.apply(inputs_embeds, vision_embeddings, ranks)
+    finally:  # also when the merge cannot be allocated: the counts must not go back to the allocator while the kernel may write them
+        ready.synchronize()  # the one host wait (the reference has three)
     n_image, n_bad = counts.tolist()
     if n_image == 0:
         raise RuntimeError(

@@ -73,6 +73,35 @@ def test_guards_raise_like_the_reference():
     assert out[0, :, 0].tolist() == [0.0, 1.0, 0.0, 1.0]
 
 
+def test_a_merge_that_fails_still_waits_for_the_counts(monkeypatch):
+    """The ranking kernel writes the counts in pinned host memory: they are not given back before it has run."""
+    from mi355_vit import handoff
+
+    taken = []
+    ranks = handoff._ranks
+
+    def spy(*args):
+        out = ranks(*args)
+        taken.append(out[2])
+        return out
+
+    class Fails:
+        @staticmethod
+        def apply(*args):
+            torch.cuda._sleep(1 << 20)  # work behind the ranking kernel: the wait is for the counts, not for the stream
+            raise torch.OutOfMemoryError("no room for the merged rows")
+
+    monkeypatch.setattr(handoff, "_ranks", spy)
+    monkeypatch.setattr(handoff, "_MergeRowsFn", Fails)
+    ids = torch.randint(0, 1000, (1, 200000), device=DEV)
+    emb = torch.zeros(1, ids.shape[1], 8, device=DEV)
+    torch.cuda.synchronize()
+    torch.cuda._sleep(1 << 26)  # some 30 ms in front of the ranking kernel
+    with pytest.raises(torch.OutOfMemoryError):
+        handoff.merge_vision_embeddings(emb, ids, torch.zeros(2, 8, device=DEV))
+    assert len(taken) == 1 and taken[0].query()
+
+
 def test_tower_output_feeds_the_handoff():
     """End of the path: the tower's [M, O] output goes into the placeholders and its gradient comes back unchanged
     in shape and order (the vision actor's backward_step accepts the 2-D gradient)."""
