@@ -229,7 +229,7 @@ def gather_rows(src: torch.Tensor, index: torch.Tensor, rows_per_index: int = 1)
 def segment_copies(copies: Sequence[Tuple[torch.Tensor, torch.Tensor, Sequence[Tuple[int, int, int]]]]) -> None:
     """Copy rows: for every (src, dst, segments) and every (src_row, dst_row, n_rows) of its segments, all in one launch.
     The host validates bounds; the kernel moves bytes."""
-    ranges, at = [], None
+    ranges, device = [], None
     for src, dst, segments in copies:
         if src.dim() != 2 or dst.dim() != 2 or not (src.is_contiguous() and dst.is_contiguous()):
             raise ValueError("segment_copy: src and dst must be contiguous 2-D")
@@ -237,16 +237,23 @@ def segment_copies(copies: Sequence[Tuple[torch.Tensor, torch.Tensor, Sequence[T
             raise ValueError("segment_copy: column count / dtype mismatch")
         n_src, n_dst, row = src.shape[0], dst.shape[0], src.shape[1] * src.element_size()
         p_src, p_dst = src.data_ptr(), dst.data_ptr()
+        before = len(ranges)
         for a, b, n in segments:
             if n <= 0:
                 continue
             if a < 0 or b < 0 or a + n > n_src or b + n > n_dst:
                 raise ValueError(f"segment_copy: segment ({a},{b},{n}) out of bounds for {n_src} -> {n_dst} rows")
             ranges += (p_src + a * row, p_dst + b * row, n * row)
-        at = src
+        if len(ranges) > before:  # a kernel will read src and write dst: both on the GPU that the launch goes to
+            for t in (src, dst):
+                if not t.is_cuda:
+                    raise RuntimeError("mi355_vit kernels need tensors on the GPU; there is no CPU path")
+                device = device or t.device
+                if t.device != device:
+                    raise ValueError(f"segment_copy: tensors on {device} and {t.device} in one call")
     if ranges:
         flat = (C.c_uint64 * len(ranges))(*ranges)
-        _lib.check(_lib.load().mvit_copy_ranges(C.addressof(flat), len(ranges) // 3, _stream(at)), "mvit_copy_ranges")
+        _lib.check(_lib.load().mvit_copy_ranges(C.addressof(flat), len(ranges) // 3, _current_raw_stream(device.index)), "mvit_copy_ranges")
 
 
 def segment_copy(src: torch.Tensor, dst: torch.Tensor, segments: Sequence[Tuple[int, int, int]]) -> torch.Tensor:

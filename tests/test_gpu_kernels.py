@@ -483,6 +483,24 @@ def test_copy_ranges_bit_exact(unit, offset, n):
     assert torch.equal(dst, want)
 
 
+@pytest.mark.parametrize("cpu", ["first source", "first destination", "last source", "last destination"])
+def test_segment_copies_refuse_host_memory_anywhere_in_the_list(cpu):
+    """Addresses go straight to a kernel: every tensor of the list is on the GPU, not the last source alone."""
+    _announce(f"segment copies: {cpu} on the CPU")
+    ops = _ops()
+    copies = [[torch.ones(4, 8, device=DEV), torch.zeros(4, 8, device=DEV), [(0, 1, 2)]] for _ in range(3)]
+    at = copies[0 if "first" in cpu else 2]
+    which = 0 if "source" in cpu else 1
+    at[which] = at[which].cpu()
+    with pytest.raises(RuntimeError, match="no CPU path"):
+        ops.segment_copies(copies)
+    torch.cuda.synchronize()
+    assert all(int(c[1].sum()) == 0 for c in copies)  # refused before any launch
+    at[2] = []  # no range of this pair: nothing of it is read or written
+    ops.segment_copies(copies)
+    assert [int(c[1].sum()) for c in copies if c is not at] == [16, 16]
+
+
 @pytest.mark.parametrize("odt", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("split_k", [1, 3])
 @pytest.mark.parametrize("S,No,Ni", [(1, 8, 8), (63, 130, 72), (1000, 1280, 1280), (515, 3840, 256), (2052, 1280, 3420), (4100, 264, 4096), (20011, 3840, 1280)])
