@@ -239,6 +239,7 @@ def segment_copies(copies: Sequence[Tuple[torch.Tensor, torch.Tensor, Sequence[T
         p_src, p_dst = src.data_ptr(), dst.data_ptr()
         before = len(ranges)
         for a, b, n in segments:
+            a, b, n = int(a), int(b), int(n)  # of a narrow integer type the products below would wrap
             if n <= 0:
                 continue
             if a < 0 or b < 0 or a + n > n_src or b + n > n_dst:

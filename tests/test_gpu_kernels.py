@@ -501,6 +501,17 @@ def test_segment_copies_refuse_host_memory_anywhere_in_the_list(cpu):
     assert [int(c[1].sum()) for c in copies if c is not at] == [16, 16]
 
 
+def test_segments_of_a_narrow_integer_type_beyond_two_gib():
+    """Row numbers may come from an int32 array; their byte offsets do not fit one."""
+    _announce("segments as int32 at an offset of 2 GiB")
+    ops = _ops()
+    row = 1 << 30
+    src, dst = torch.empty(3, row, dtype=torch.uint8, device=DEV), torch.zeros(1, row, dtype=torch.uint8, device=DEV)
+    src[2] = 5
+    ops.segment_copies([(src, dst, np.array([[2, 0, 1]], dtype=np.int32))])
+    assert bool((dst == 5).all())
+
+
 @pytest.mark.parametrize("odt", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("split_k", [1, 3])
 @pytest.mark.parametrize("S,No,Ni", [(1, 8, 8), (63, 130, 72), (1000, 1280, 1280), (515, 3840, 256), (2052, 1280, 3420), (4100, 264, 4096), (20011, 3840, 1280)])
