@@ -750,16 +750,21 @@ int mvit_copy_ranges(const mvit_copy_range* ranges, int n_ranges, mvit_stream_t 
     return MVIT_OK;
   };
   for (int i = 0; i < n_ranges; ++i) {
-    if (ranges[i].bytes == 0) continue;
-    const int64_t words = ranges[i].bytes / word, need = (words + COPY_PIECE - 1) / COPY_PIECE;
-    MVIT_REQUIRE(need < (1ll << 31), "copy_ranges: range %d too long", i);
-    if (a.n == COPY_MAX_RANGES || pieces + need >= (1ll << 31))
-      if (int rc = flush()) return rc;
-    a.first_piece[a.n] = (int)pieces;
-    a.src[a.n] = ranges[i].src;
-    a.dst[a.n] = ranges[i].dst;
-    a.words[a.n++] = words;
-    pieces += need;
+    const char* src = static_cast<const char*>(ranges[i].src);
+    char* dst = static_cast<char*>(ranges[i].dst);
+    for (int64_t left = ranges[i].bytes / word; left > 0;) {  // a range longer than a launch is cut
+      if (a.n == COPY_MAX_RANGES || pieces == MVIT_MAX_GROUPS_256)
+        if (int rc = flush()) return rc;
+      const int64_t room = (MVIT_MAX_GROUPS_256 - pieces) * COPY_PIECE, words = left < room ? left : room;
+      a.first_piece[a.n] = (int)pieces;
+      a.src[a.n] = src;
+      a.dst[a.n] = dst;
+      a.words[a.n++] = words;
+      pieces += (words + COPY_PIECE - 1) / COPY_PIECE;
+      src += words * word;
+      dst += words * word;
+      left -= words;
+    }
   }
   return flush();
 }

@@ -20,6 +20,9 @@ typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
 
 #define MVIT_WAVE 64
 
+// Work-groups of 256 threads that one launch can have: the runtime takes fewer than 2^32 threads per grid dimension.
+constexpr int64_t MVIT_MAX_GROUPS_256 = (1ll << 24) - 1;
+
 // Records a formatted message for mvit_last_error() and returns `code`.
 int mvit_set_error(int code, const char* fmt, ...);
 

@@ -366,9 +366,15 @@ int mvit_resample_u8_batch(const mvit_resample_job* list, int n_jobs, mvit_strea
                  "resample_u8: axis too long");
   }
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  // work-groups for `outer` rows of the outermost axis
+  auto groups = [](int kind, const mvit_resample_job& j, int64_t outer) {
+    return kind == 5 ? outer * j.out_len * ((j.inner / 4 + 255) / 256) : (j.out_len + 63) / 64 * ((outer + 4 * RESAMPLE_ROWS - 1) / (4 * RESAMPLE_ROWS));
+  };
   // jobs of one kind (wide words; 1 .. 4 bytes) share launches; 0: everything else, a launch each
-  auto kind_of = [](const mvit_resample_job& j) {
-    if (j.inner % 4 == 0 && j.inner > RESAMPLE_MAX_CHANNELS && reinterpret_cast<uintptr_t>(j.src) % 4 == 0 && reinterpret_cast<uintptr_t>(j.dst) % 4 == 0) return 5;
+  auto kind_of = [&](const mvit_resample_job& j) {
+    if (j.inner % 4 == 0 && j.inner > RESAMPLE_MAX_CHANNELS && reinterpret_cast<uintptr_t>(j.src) % 4 == 0 && reinterpret_cast<uintptr_t>(j.dst) % 4 == 0 &&
+        groups(5, j, 1) <= MVIT_MAX_GROUPS_256)
+      return 5;
     return j.inner <= RESAMPLE_MAX_CHANNELS ? (int)j.inner : 0;
   };
   for (int kind = 0; kind <= 5; ++kind) {
@@ -400,14 +406,23 @@ int mvit_resample_u8_batch(const mvit_resample_job* list, int n_jobs, mvit_strea
         MVIT_CHECK_LAUNCH("resample_u8");
         continue;
       }
-      const int64_t need = kind == 5 ? j.outer * j.out_len * ((j.inner / 4 + 255) / 256)
-                                     : (j.out_len + 63) / 64 * ((j.outer + 4 * RESAMPLE_ROWS - 1) / (4 * RESAMPLE_ROWS));
-      MVIT_REQUIRE(need < (1ll << 31), "resample_u8: too many rows for one launch");
-      if (jobs.n == RESAMPLE_MAX_JOBS || blocks + need >= (1ll << 31))
-        if (int rc = flush()) return rc;
-      jobs.first_block[jobs.n] = (int)blocks;
-      jobs.job[jobs.n++] = j;
-      blocks += need;
+      // the grid of a launch is limited: what does not fit goes to the next one, a job of more work-groups in pieces of whole rows
+      const int64_t unit = kind == 5 ? 1 : 4 * RESAMPLE_ROWS;  // rows that a work-group shares
+      for (int64_t o = 0; o < j.outer;) {
+        const int64_t fit = (MVIT_MAX_GROUPS_256 - blocks) / groups(kind, j, 1) * unit;
+        if (jobs.n == RESAMPLE_MAX_JOBS || fit == 0) {
+          if (int rc = flush()) return rc;
+          continue;
+        }
+        mvit_resample_job& piece = jobs.job[jobs.n];
+        piece = j;
+        piece.src = j.src + o * j.in_len * j.inner;
+        piece.dst = j.dst + o * j.out_len * j.inner;
+        piece.outer = j.outer - o < fit ? j.outer - o : fit;
+        jobs.first_block[jobs.n++] = (int)blocks;
+        blocks += groups(kind, j, piece.outer);
+        o += piece.outer;
+      }
     }
     if (int rc = flush()) return rc;
   }

@@ -512,6 +512,26 @@ def test_segments_of_a_narrow_integer_type_beyond_two_gib():
     assert bool((dst == 5).all())
 
 
+def test_copy_ranges_of_more_pieces_than_a_launch_takes():
+    """A launch takes fewer than 2^24 work-groups of 256 threads: at single bytes 32 GiB.  Longer ranges are cut."""
+    import ctypes
+
+    from mi355_vit import _lib
+
+    _announce("copy ranges, 33 GiB at odd addresses")
+    n = 33 << 30
+    src = torch.empty(n + 1, dtype=torch.uint8, device=DEV)
+    block = torch.randint(0, 256, (1 << 30,), dtype=torch.uint8, device=DEV)
+    for i in range(33):
+        src[1 + (i << 30) : 1 + ((i + 1) << 30)] = block ^ (7 * i)
+    dst = torch.zeros(n + 2, dtype=torch.uint8, device=DEV)
+    ranges = (ctypes.c_uint64 * 6)(src.data_ptr() + 1, dst.data_ptr() + 1, 5000, src.data_ptr() + 5001, dst.data_ptr() + 5001, n - 5000)
+    _lib.check(_lib.load().mvit_copy_ranges(ctypes.addressof(ranges), 2, torch.cuda.current_stream().cuda_stream), "mvit_copy_ranges")
+    for i in range(33):
+        assert torch.equal(dst[1 + (i << 30) : 1 + ((i + 1) << 30)], block ^ (7 * i)), i
+    assert int(dst[0]) == 0 and int(dst[n + 1]) == 0
+
+
 @pytest.mark.parametrize("odt", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("split_k", [1, 3])
 @pytest.mark.parametrize("S,No,Ni", [(1, 8, 8), (63, 130, 72), (1000, 1280, 1280), (515, 3840, 256), (2052, 1280, 3420), (4100, 264, 4096), (20011, 3840, 1280)])

@@ -441,3 +441,18 @@ def test_resize_rejects_what_it_cannot_do():
         resize_frames(x.cpu(), 56, 56)
     same = resize_frames(x, 28, 28)
     assert same.data_ptr() != x.data_ptr() and torch.equal(same, x)
+
+
+@pytest.mark.parametrize("outer,inner", [((1 << 29) + 100, 1), ((1 << 24) + 5, 8)])
+def test_resample_of_more_work_groups_than_a_launch_takes(outer, inner):
+    """A launch takes fewer than 2^24 work-groups of 256 threads; longer passes go in several.  One tap of weight one: a copy."""
+    from mi355_vit import _lib
+
+    _announce(f"resample outer={outer} inner={inner}")
+    src = torch.randint(0, 256, (outer * inner,), dtype=torch.uint8, device=DEV)
+    dst = torch.zeros_like(src)
+    bounds, kk = torch.tensor([0, 1], dtype=torch.int32, device=DEV), torch.tensor([1 << 22], dtype=torch.int32, device=DEV)
+    rc = _lib.load().mvit_resample_u8(src.data_ptr(), dst.data_ptr(), outer, 1, 1, inner, bounds.data_ptr(), kk.data_ptr(), 1,
+                                      torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "mvit_resample_u8")
+    assert torch.equal(src, dst)
