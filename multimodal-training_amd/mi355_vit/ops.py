@@ -399,10 +399,13 @@ def swiglu_bwd_sums_columns(rows: int, cols: int, k: int) -> bool:
     return bool(_lib.load().mvit_gemm_swiglu_bwd_sums_columns(rows, cols, k))
 
 
+MAX_DIRECT_PITCH = 1 << 22  # elements; wider rows go to the register-staged product, which makes no row sums
+
+
 def weight_grad(dy: torch.Tensor, act: torch.Tensor, out: torch.Tensor, bias_dtype: Optional[torch.dtype], n: Optional[int] = None) -> Optional[torch.Tensor]:
     """Gradients of a Linear layer's weight (``out`` = dy^T act) and, with ``bias_dtype``, bias (returned: the column sums of
-    dy).  In bf16 the product sums the operand it reads anyway."""
-    fused = dy.dtype == torch.bfloat16 and bias_dtype == out.dtype
+    dy).  In bf16 the product sums the operand it reads anyway (not so with a row pitch beyond 32-bit lane offsets)."""
+    fused = dy.dtype == torch.bfloat16 and bias_dtype == out.dtype and max(dy.stride(0), act.stride(0)) <= MAX_DIRECT_PITCH
     bias = None
     if bias_dtype is not None:
         bias = torch.empty(dy.shape[1], dtype=bias_dtype, device=dy.device) if fused else colsum(dy, bias_dtype)

@@ -830,6 +830,24 @@ def test_gemm_bf16_with_a_row_pitch_beyond_32_bit_lane_offsets():
     assert max_rel_err(out, ref) < TOL[torch.bfloat16] and max_rel_err(dense, ref) < TOL[torch.bfloat16]
 
 
+@pytest.mark.parametrize("wide", ["gradient", "activation"])
+def test_weight_grad_with_a_row_pitch_beyond_32_bit_lane_offsets(wide):
+    """The product of such rows makes no row sums: the bias gradient comes from a pass of its own."""
+    ops = _ops()
+    _announce(f"weight and bias gradient, huge row pitch of the {wide}")
+    S, No, Ni, pitch = 40, 264, 72, (1 << 22) + 8
+    dy, act = _rand((S, No), torch.bfloat16, 31), _rand((S, Ni), torch.bfloat16, 32)
+    big = torch.zeros(S * pitch, dtype=torch.bfloat16, device=DEV)
+    view = big.as_strided((S, No if wide == "gradient" else Ni), (pitch, 1))
+    view.copy_(dy if wide == "gradient" else act)
+    dw = torch.empty(No, Ni, dtype=torch.bfloat16, device=DEV)
+    db = ops.weight_grad(view if wide == "gradient" else dy.to(DEV), view if wide == "activation" else act.to(DEV), dw, torch.bfloat16)
+    assert max_rel_err(dw, dy.double().t() @ act.double()) < TOL[torch.bfloat16]
+    want, size = dy.double().sum(0), dy.double().abs().sum(0)
+    # S - 1 fp32 additions in some order, then one rounding to bf16
+    assert bool(((db.cpu().double() - want).abs() <= size * (S * 2.0**-24) + want.abs() * 2.0**-8).all())
+
+
 def test_empty_inputs_are_no_ops():
     """Zero rows, zero segments, zero tokens: every kernel wrapper returns (an empty result, or its output untouched)
     without a launch error - the shapes an empty rank-local pack or an image-free batch produce."""
