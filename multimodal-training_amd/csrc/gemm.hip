@@ -1111,9 +1111,10 @@ int launch_var(int var, const GemmParams& p, hipStream_t s) {
   {
     // direct-to-LDS main loop: v_mfma_f32_16x16x32_bf16 for the plain GEMMs with an operand behind the transposing
     // LDS read (weight gradients +6 %, input gradients +1 % on real data), v_mfma_f32_32x32x16_bf16 for the forward
-    // GEMMs (both operands row-major: 3-5 % faster that way) and for the fused backward epilogues
+    // GEMMs (both operands row-major: 3-5 % faster that way).  SwiGLU backward takes the form of the smaller tiles that
+    // serve few rows (gemm_small.hip): a row's gradient has the same bits whatever batch it lies in
     constexpr int NS = 4;
-    if (var == 3) return (TB && EPI == MVIT_EPI_NONE) ? launch_dl<TO, TA, TB, EPI, NS, 8, true>(p, s) : launch_dl<TO, TA, TB, EPI, NS, 8>(p, s);
+    if (var == 3) return (TB && (EPI == MVIT_EPI_NONE || EPI == MVIT_EPI_SWIGLU_BWD)) ? launch_dl<TO, TA, TB, EPI, NS, 8, true>(p, s) : launch_dl<TO, TA, TB, EPI, NS, 8>(p, s);
   }
   return launch<T, TO, TA, TB, EPI, 1>(p, s);  // register-staged main loop: operands whose row pitch exceeds 32-bit lane offsets
 }

@@ -456,6 +456,30 @@ def test_gemm_f32_rows_do_not_depend_on_their_batch(trans_b, N, K):
         assert torch.equal(part[:rows], everything[:rows]) and bool((part[rows] == 7.0).all()), rows
 
 
+@pytest.mark.parametrize("N,K", [(3456, 1280), (200, 72)])
+def test_swiglu_backward_rows_do_not_depend_on_their_batch(N, K):
+    """Few rows take 64-row tiles, many 256-row ones: the same bits, also at the edges of either and with column sums asked for."""
+    _announce(f"gemm swiglu backward rows N={N} K={K}")
+    ops = _ops()
+    from mi355_vit import _lib as E
+
+    M = 12000
+    dy, w = _rand((M, K), torch.bfloat16, 0).to(DEV), _rand((K, N), torch.bfloat16, 1, K**-0.5).to(DEV)
+    gu = _rand((M, 2 * N), torch.bfloat16, 2).to(DEV)
+
+    def run(rows, sums):
+        out = torch.full((rows + 1, 2 * N), 7.0, dtype=torch.bfloat16, device=DEV)
+        part = torch.empty(-(-rows // 256), 2 * N, device=DEV) if sums else None
+        ops.gemm(dy[:rows], w, out[:rows], trans_b=True, epilogue=E.EPI_SWIGLU_BWD, residual=gu[:rows], aux_off=N, colsum_partial=part)
+        assert bool((out[rows] == 7.0).all())
+        return out[:rows]
+
+    everything = run(M, True)
+    for rows in (1, 63, 64, 65, 100, 257, 1030, 2900, 3000, 4096, 5000, 7000, 9500, M):
+        for sums in (False, True):
+            assert torch.equal(run(rows, sums), everything[:rows]), (rows, sums)
+
+
 @pytest.mark.parametrize("unit,offset", [(16, 0), (16, 4), (4, 0), (2, 2), (1, 1)])
 @pytest.mark.parametrize("n", [1, 5, 96, 97, 200])
 def test_copy_ranges_bit_exact(unit, offset, n):

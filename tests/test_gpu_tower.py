@@ -406,6 +406,37 @@ def test_windowed_block_on_each_sequence_parallel_share_equals_the_unsharded_blo
     assert sum(o.shape[0] for o in outs) == S and min(o.shape[0] for o in outs) > 0
 
 
+def test_windowed_block_of_4096_rows_equals_its_four_shares():
+    """The same at 4,096 rows, where the whole block and its shares run on tiles of different sizes."""
+    from mi355_vit import ops
+    from mi355_vit.config import Qwen2_5_VLVisionConfig
+    from mi355_vit.modeling import Qwen2_5_VLVisionBlock
+
+    print("[case] windowed block, 4096 rows and four shares", flush=True)
+    torch.manual_seed(8)
+    cfg = Qwen2_5_VLVisionConfig(depth=1, hidden_size=1280, intermediate_size=3420, num_heads=16, out_hidden_size=256, fullatt_block_indexes=[])
+    blk = Qwen2_5_VLVisionBlock(cfg, 0).to(torch.bfloat16).to(DEV)
+    S, n = 4096, 1024
+    _, cu = ops.window_index(torch.tensor([[1, 64, 64]]), 2, 112, 14)
+    assert cu.tolist() == list(range(0, S + 1, 64))
+    g = torch.Generator().manual_seed(8)
+    x, gy = (torch.randn(S, 1280, generator=g).to(torch.bfloat16).to(DEV) for _ in range(2))
+    ang = torch.randn(S, 40, generator=g)
+    emb = torch.cat((ang, ang), dim=-1)
+    cos, sin = emb.cos().to(DEV), emb.sin().to(DEV)
+
+    def run(a, b):
+        xr = x[a:b].clone().requires_grad_(True)
+        y = blk(xr, cu_seqlens=cu[: (b - a) // 64 + 1].to(DEV), position_embeddings=(cos[a:b], sin[a:b]))
+        y.backward(gy[a:b])
+        return y.detach(), xr.grad
+
+    y_full, dx_full = run(0, S)
+    for a in range(0, S, n):
+        y, dx = run(a, a + n)
+        assert torch.equal(y, y_full[a : a + n]) and torch.equal(dx, dx_full[a : a + n]), a
+
+
 def test_a_step_recorded_in_a_hip_graph_replays_bit_identically():
     """The library's launches allocate nothing, wait for nothing and use no stream but the caller's (the eager backward's
     second stream joins through events), so a whole forward and a whole backward can be recorded in HIP graphs.  Three
