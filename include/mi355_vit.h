@@ -37,7 +37,7 @@ enum { MVIT_OK = 0, MVIT_ERR_ARG = -1, MVIT_ERR_LAUNCH = -2, MVIT_ERR_UNSUPPORTE
  * 200: mvit_attn_bwd takes the size of its workspace (delta_elems) and checks that outputs and inputs are disjoint;
  *      mvit_adam_tensor rows are 96 bytes (shadow copy fields).  A caller built against an older header must be
  *      rebuilt: compare mvit_version() with the value the header was written for. */
-#define MVIT_VERSION 201
+#define MVIT_VERSION 202
 int mvit_version(void);
 const char* mvit_last_error(void);
 
@@ -174,8 +174,9 @@ typedef struct mvit_gemm_args {
   int64_t ldaux;
   int64_t aux_off; /* column offset of the second half in aux (SWIGLU) / R and C (SWIGLU_BWD) */
   void* workspace; /* split_k > 1: fp32 scratch of split_k * M * N floats.  MVIT_EPI_SWIGLU_BWD (optional): receives
-                      fp32 column sums of C per 256-row tile, [ceil(M/256)][ldc] (columns [0,N) and
-                      [aux_off, aux_off+N) are written); add the rows with mvit_reduce_partials for the bias gradient */
+                      fp32 column sums of C, of its values before they are rounded, per `colsum_rows` rows:
+                      [ceil(M/colsum_rows)][ldc] (columns [0,N) and [aux_off, aux_off+N) are written); add the rows
+                      with mvit_reduce_partials for the bias gradient */
   int64_t workspace_bytes;
   int split_k;   /* <= 1: one work-group per tile walks all of K.  > 1 (EPI_NONE, EPI_BIAS, EPI_BIAS_RES): K is cut in
                     split_k slices whose fp32 partial tiles go to `workspace`; a second kernel sums them in a fixed
@@ -185,6 +186,8 @@ typedef struct mvit_gemm_args {
   void* row_sums; /* optional, bf16 operands with trans_a = trans_b = 1 and EPI_NONE only: receives sum_k A[m,k], [M], in
                      out_dtype.  For a weight gradient dW = dY^T X this is the bias gradient.  With split_k > 1 the
                      workspace holds split_k * M more floats */
+  int colsum_rows; /* MVIT_EPI_SWIGLU_BWD with a workspace: rows of C per row of column sums, 256 (also 0) or 64; the rows
+                      of the tile that makes them, see mvit_gemm_swiglu_bwd_colsum_rows.  C does not depend on it */
 } mvit_gemm_args;
 
 /* C[M,N] = epilogue(sum_k A[m,k] * B[n,k]).  Operands must be 16-byte aligned with lda/ldb multiples of
@@ -195,9 +198,8 @@ int mvit_gemm(const mvit_gemm_args* args, mvit_stream_t stream);
 
 /* Host-only: the split_k to ask for when C[out_rows, out_cols] is a weight gradient contracted over k tokens (bf16). */
 int mvit_gemm_wgrad_split_k(int64_t out_rows, int64_t out_cols, int64_t k);
-/* Host-only: 1 when a bf16 MVIT_EPI_SWIGLU_BWD product of this shape is fastest on the kernel that can hand back column sums
- * of C (of its fp32 values), 0 when it is faster without a workspace (the weight gradient's row_sums then take the sums). */
-int mvit_gemm_swiglu_bwd_sums_columns(int64_t M, int64_t N, int64_t K);
+/* Host-only: the colsum_rows with which a bf16 MVIT_EPI_SWIGLU_BWD product of this shape is fastest. */
+int mvit_gemm_swiglu_bwd_colsum_rows(int64_t M, int64_t N, int64_t K);
 
 /* ---------------------------------------------------------------- varlen attention */
 

@@ -45,6 +45,7 @@ mvit_gemm_args gemm_args(int dtype, int out_dtype) {
 // Layout of the backward's workspace; with base == nullptr only the size is computed.
 struct BwdWorkspace {
   float *colsum, *swiglu_cols, *rms, *delta, *splitk;
+  int colsum_rows, n_swiglu_cols;  // rows of dgu per row of swiglu_cols, and how many
   int64_t delta_elems, splitk_bytes, total;
 };
 BwdWorkspace plan_bwd_workspace(const mvit_block_args* a, void* base) {
@@ -52,7 +53,9 @@ BwdWorkspace plan_bwd_workspace(const mvit_block_args* a, void* base) {
   Bump b{static_cast<char*>(base), 0, 0};
   BwdWorkspace w;
   w.colsum = static_cast<float*>(b.take(a->dtype == MVIT_BF16 ? 0 : 64 * (3 * C > 2 * Ipad ? 3 * C : 2 * Ipad) * 4));
-  w.swiglu_cols = static_cast<float*>(b.take((S + 255) / 256 * 2 * Ipad * 4));
+  w.colsum_rows = mvit_gemm_swiglu_bwd_colsum_rows(S, Ipad, C);
+  w.n_swiglu_cols = (int)((S + w.colsum_rows - 1) / w.colsum_rows);
+  w.swiglu_cols = static_cast<float*>(b.take((int64_t)w.n_swiglu_cols * 2 * Ipad * 4));
   w.rms = static_cast<float*>(b.take((int64_t)RMS_PARTIALS * C * 4));
   w.delta_elems = mvit_attn_bwd_delta_elems(a->max_seqlen, S, a->nheads, a->head_dim, a->dtype);
   w.delta = static_cast<float*>(b.take(w.delta_elems * 4));
@@ -194,23 +197,23 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
     if (!st && two) return MVIT_ERR_LAUNCH;
     STEP(weight_grad(a->dx2, C, C, a->h, Ipad, I, a->g_wdown, a->g_bdown, a->split_k_down, st));
   }
-  // dgu = (dx2 . Wdown) through the SwiGLU derivative.  With many rows the per-tile column sums of dgu come back with it, from
-  // its fp32 values; with few the product runs on smaller tiles and the weight gradient sums the operand it reads
-  const bool fused_cols = dt == MVIT_BF16 && mvit_gemm_swiglu_bwd_sums_columns(S, Ipad, C);
+  // dgu = (dx2 . Wdown) through the SwiGLU derivative.  In bf16 the per-tile column sums of dgu come back with it, from its fp32
+  // values: the gate / up bias gradient
+  const bool fused_cols = dt == MVIT_BF16;
   {
     mvit_gemm_args g = gemm_args(dt, dt);
     g.trans_b = 1; g.epilogue = MVIT_EPI_SWIGLU_BWD;
     g.M = S; g.N = Ipad; g.K = C;
     g.A = a->dx2; g.lda = C; g.B = a->wdown; g.ldb = Ipad; g.C = a->dgu; g.ldc = 2 * Ipad; g.R = a->gu; g.ldr = 2 * Ipad; g.aux_off = Ipad;
     if (fused_cols) {
-      g.workspace = w.swiglu_cols; g.workspace_bytes = (S + 255) / 256 * 2 * Ipad * 4;
+      g.workspace = w.swiglu_cols; g.workspace_bytes = (int64_t)w.n_swiglu_cols * 2 * Ipad * 4; g.colsum_rows = w.colsum_rows;
     }
     STEP(mvit_gemm(&g, stream));
   }
   {
     mvit_stream_t st = fork(1);
     if (!st && two) return MVIT_ERR_LAUNCH;
-    if (fused_cols) STEP(mvit_reduce_partials(w.swiglu_cols, (int)((S + 255) / 256), 2 * Ipad, a->g_bgu, gdt, st));
+    if (fused_cols) STEP(mvit_reduce_partials(w.swiglu_cols, w.n_swiglu_cols, 2 * Ipad, a->g_bgu, gdt, st));
     STEP(weight_grad(a->dgu, 2 * Ipad, 2 * Ipad, a->n2, C, C, a->g_wgu, fused_cols ? nullptr : a->g_bgu, a->split_k_gate_up, st));
   }
   {  // dn2 = dgu . Wgu

@@ -1050,10 +1050,10 @@ int launch(const GemmParams& p, hipStream_t stream) {
   return MVIT_OK;
 }
 
-// Column sums of C per 256 rows, columns [0, N) and [aux_off, aux_off + N): what the bf16 SwiGLU-backward epilogue hands back
-// from its tiles, for the fp32 product whose tiles are smaller.
-__global__ __launch_bounds__(256) void tile_colsum_kernel(const float* __restrict__ C, int64_t ldc, int64_t M, int64_t N, int64_t aux_off, float* __restrict__ out) {
-  const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x, m0 = (int64_t)blockIdx.y * 256, m1 = m0 + 256 < M ? m0 + 256 : M;
+// Column sums of C per `rows` rows, columns [0, N) and [aux_off, aux_off + N): what the bf16 SwiGLU-backward epilogue hands back
+// from its tiles, for the fp32 product.
+__global__ __launch_bounds__(256) void tile_colsum_kernel(const float* __restrict__ C, int64_t ldc, int64_t M, int64_t N, int64_t aux_off, int rows, float* __restrict__ out) {
+  const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x, m0 = (int64_t)blockIdx.y * rows, m1 = m0 + rows < M ? m0 + rows : M;
   if (n >= N) return;
   const int64_t col = n + blockIdx.z * aux_off;
   float s = 0.f;
@@ -1195,7 +1195,8 @@ struct TileChoice {
   int bm, bn;
   double us;
 };
-TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk, int64_t k_last, int64_t slices, int n_cu) {
+// `full_rows`: whether the 256-row SwiGLU-backward kernel (bm = 0) may be chosen
+TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk, int64_t k_last, int64_t slices, int n_cu, bool full_rows = true) {
   const bool tt = kind == TT_NONE || kind == TT_NONE_F32;
   const double steps = (double)((k_chunk + 63) / 64);
   const int64_t n_mul = kind == NN_SWIGLU ? 2 : 1;
@@ -1209,19 +1210,22 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
   };
   const bool swiglu = kind == NN_SWIGLU;
   if (pp_takes(kind, k_chunk, k_last)) consider(256, 256, tt ? 1.2 : 1.15, 0., swiglu ? 11. : 7.);
-  if (kind == NT_SWIGLU_BWD) {  // two inputs and two outputs per element lengthen its epilogue
+  if (kind == NT_SWIGLU_BWD) {  // two inputs, two outputs and the column sums lengthen its epilogue
     consider(64, 64, 0.30, 0.43, 2.);
-    consider(64, 128, 0.46, 0.57, 2.);
+    consider(64, 128, 0.47, 0.70, 2.);
   } else {
     if (!swiglu) consider(64, 64, 0.23, 0.36, 2.);
     consider(64, 128, 0.37, 0.52, 2.);
     consider(128, 128, 0.60, 0.72, swiglu ? 6. : 2.5);
   }
-  // SwiGLU backward of many rows: the 256-row kernel, which also sums the columns of its result
-  if (kind == NT_SWIGLU_BWD) {
-    const double tiles = (double)(((M + 255) / 256) * ((N + 255) / 256)), us = 4. + ceil(tiles / n_cu) * (steps * 1.6 + 16.);
-    if (us < best.us + (double)M * (double)N * 4. / 4e6) best = TileChoice{0, 0, us};
-  }
+  // SwiGLU backward: the 256-row kernel as soon as its tiles give half of the units work.  Its launch shares the GPU with the
+  // down projection's weight gradient on the second stream, which fills the units it leaves idle, while two small tiles per
+  // unit compete with it for the L2s.  us per block of the tower, forward and backward, 64 x 64 / 64 x 128 / 256-row:
+  // recorded in a graph at 256 rows 291 / 296 / 334, 1,024: 402 / 403 / 428, 2,048: 581 / 578 / 598, 2,688: 689 / 683 / 697,
+  // 3,136: 755 / 741 / 751; issued one by one at 2,304 rows 603 / 591 / 588, 2,688: 676 / 670 / 650, 4,864: 1,004 / 990 / 970,
+  // 10,400: 1,748 / 1,713 / 1,662, 14,336: 2,457 / 2,415 / 2,359 (the launch alone would be faster on small tiles wherever the
+  // 256-row tiles end in a bad round: 4,864 rows 91 / 76 / 105, 10,240: 182 / 142 / 164)
+  if (kind == NT_SWIGLU_BWD && full_rows && 2 * ((M + 255) / 256) * ((N + 255) / 256) >= n_cu) best = TileChoice{0, 0, 0.};
   return best;
 }
 
@@ -1346,13 +1350,15 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
   p.panel_w = tn <= 6 ? (int)tn : 4;
   p.split_k = 1; p.k_chunk = a->K; p.workspace = nullptr; p.reduce_epi = MVIT_EPI_NONE;
   p.colsum = nullptr;
+  const int colsum_rows = a->colsum_rows == 64 ? 64 : 256;
   p.row_sums = a->row_sums; p.row_ws = nullptr;
   if (a->row_sums)
     MVIT_REQUIRE(a->dtype == MVIT_BF16 && a->trans_a && a->trans_b && epi == MVIT_EPI_NONE && var == 3,
                  "gemm: row sums come with a plain bf16 product of two transposed operands");
   if (epi == MVIT_EPI_SWIGLU_BWD && a->workspace) {
-    MVIT_REQUIRE(mvit_aligned16(a->workspace) && a->workspace_bytes >= (int64_t)sizeof(float) * tm * a->ldc,
-                 "gemm: SWIGLU_BWD column sums need a workspace of %lld bytes", (long long)(sizeof(float) * tm * a->ldc));
+    MVIT_REQUIRE(a->colsum_rows == 0 || a->colsum_rows == 256 || a->colsum_rows == 64, "gemm: colsum_rows %d is not 256 or 64", a->colsum_rows);
+    const int64_t need = (int64_t)sizeof(float) * ((a->M + colsum_rows - 1) / colsum_rows) * a->ldc;
+    MVIT_REQUIRE(mvit_aligned16(a->workspace) && a->workspace_bytes >= need, "gemm: SWIGLU_BWD column sums need a workspace of %lld bytes", (long long)need);
     p.colsum = static_cast<float*>(a->workspace);
   }
   if (a->split_k > 1) {
@@ -1381,7 +1387,8 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
     const int n_cu = device_cu_count(dev);
     TileChoice c = choose_tile(kind, p.M, p.N, p.k_chunk, p.K - (p.split_k - 1) * p.k_chunk, p.split_k, n_cu);
     if (getenv("MVIT_GEMM_NO_HALF_TILES") != nullptr && c.bm != 256 && pp_takes(kind, p.k_chunk, p.K - (p.split_k - 1) * p.k_chunk)) c = TileChoice{256, 256, 0.};
-    if (kind == NT_SWIGLU_BWD && p.colsum != nullptr) c.bm = 0;  // per-256-row column sums: the 256-row kernel makes them
+    // the column sums are per tile row: their granularity names the kernel (64 rows: 64 x 64 or 64 x 128 tiles, below)
+    if (kind == NT_SWIGLU_BWD && p.colsum != nullptr) c = colsum_rows == 64 ? choose_tile(kind, p.M, p.N, p.k_chunk, p.K, 1, n_cu, false) : TileChoice{0, 0, 0.};
     if (c.bm != 0) {
       p.tiles_m = (int)((p.M + c.bm - 1) / c.bm);
       const int n_cols = kind == NN_SWIGLU ? c.bn / 2 : c.bn;
@@ -1399,6 +1406,7 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
     }
   }
   if (a->dtype == MVIT_BF16) {
+    MVIT_REQUIRE(p.colsum == nullptr || colsum_rows == 256, "gemm: column sums per 64 rows need bf16 results and row pitches of at most 2^22 elements");
     if (a->out_dtype == MVIT_BF16) return dispatch_trans<bf16_t, bf16_t>(a->trans_a, a->trans_b, epi, var, p, s);
     return dispatch_trans<bf16_t, float>(a->trans_a, a->trans_b, epi, var, p, s);
   }
@@ -1410,7 +1418,8 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
     MVIT_CHECK_LAUNCH("gemm split-k reduce");
   }
   if (p.colsum != nullptr) {
-    hipLaunchKernelGGL(tile_colsum_kernel, dim3((unsigned)((p.N + 255) / 256), (unsigned)tm, 2), 256, 0, s, static_cast<const float*>(p.C), p.ldc, p.M, p.N, p.aux_off, p.colsum);
+    hipLaunchKernelGGL(tile_colsum_kernel, dim3((unsigned)((p.N + 255) / 256), (unsigned)((p.M + colsum_rows - 1) / colsum_rows), 2), 256, 0, s,
+                       static_cast<const float*>(p.C), p.ldc, p.M, p.N, p.aux_off, colsum_rows, p.colsum);
     MVIT_CHECK_LAUNCH("gemm column sums");
   }
   return MVIT_OK;
@@ -1435,6 +1444,6 @@ extern "C" int mvit_gemm_wgrad_split_k(int64_t out_rows, int64_t out_cols, int64
   return best;
 }
 
-extern "C" int mvit_gemm_swiglu_bwd_sums_columns(int64_t M, int64_t N, int64_t K) {
-  return choose_tile(NT_SWIGLU_BWD, M, N, K, K, 1, 256).bm == 0 ? 1 : 0;
+extern "C" int mvit_gemm_swiglu_bwd_colsum_rows(int64_t M, int64_t N, int64_t K) {
+  return choose_tile(NT_SWIGLU_BWD, M, N, K, K, 1, 256).bm == 0 ? 256 : 64;
 }

@@ -27,7 +27,7 @@ struct GemmParams {
   float* workspace;   // [split_k][M][N] fp32 partial sums when split_k > 1
   int vec_ok;         // every epilogue pointer / stride allows 16-byte accesses
   int half_vec_ok;    // the output allows 8-byte stores of bf16 (a row pitch that is a multiple of 4 elements only)
-  float* colsum;      // SWIGLU_BWD: per-tile-row column sums of the output, [tiles_m][ldc] (null: not wanted)
+  float* colsum;      // SWIGLU_BWD: column sums of the output before rounding, one row per tile row, [tiles_m][ldc] (null: not wanted)
   void* row_sums;     // TT_NONE(_F32), optional: [M] sums of op(A) over k, in the type of C (a bias gradient beside its weight gradient)
   float* row_ws;      // split_k > 1: their partial sums, [split_k][M]
   int panel_w;        // tiles are walked in panels of this many tile columns (M fastest across a panel's rows)

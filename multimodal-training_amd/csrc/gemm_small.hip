@@ -243,8 +243,14 @@ __global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(cons
   }
 
   // ---- epilogue
+  constexpr bool CAN_CS = EPI == MVIT_EPI_SWIGLU_BWD;
+  const bool do_cs = CAN_CS && p.colsum != nullptr;
+  float cs[CAN_CS ? NG : 1][16];
+#pragma unroll
+  for (int g = 0; g < (CAN_CS ? NG : 1); ++g)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) cs[g][e] = 0.f;
   float* ws = to_ws ? p.workspace + (int64_t)slice * p.M * p.N : nullptr;
-  float no_cs[16];
   if constexpr (ROW_SUMS) {
 #pragma unroll
     for (int i = 0; i < NRS; ++i) {
@@ -274,7 +280,7 @@ __global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(cons
       if (HAS_BIAS) unpack8<T>(bias_g[g], hb);
       if (HAS_BIAS && DUAL) unpack8<T>(bias_u, hb2);
       if (to_ws) store8_cached(ws + m * p.N + n, v);
-      else emit8_impl<T, TO, EPI, true, HAS_IN>(p, m, n, v, u, HAS_IN ? pre[it] : nullptr, no_cs, false, HAS_BIAS ? hb : nullptr, HAS_BIAS && DUAL ? hb2 : nullptr);
+      else emit8_impl<T, TO, EPI, true, HAS_IN>(p, m, n, v, u, HAS_IN ? pre[it] : nullptr, cs[CAN_CS ? g : 0], do_cs, HAS_BIAS ? hb : nullptr, HAS_BIAS && DUAL ? hb2 : nullptr);
     } else {
       if (m >= p.M || n >= p.N) continue;
       if (to_ws) {
@@ -283,7 +289,31 @@ __global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(cons
         else
           for (int e = 0; e < 8 && n + e < p.N; ++e) w[e] = v[e];
       } else {
-        emit8<T, TO, EPI>(p, m, n, v, u, vec, no_cs, false);
+        emit8<T, TO, EPI>(p, m, n, v, u, vec, cs[CAN_CS ? g : 0], do_cs);
+      }
+    }
+  }
+  if constexpr (CAN_CS) {
+    // a lane's sums over its rows meet those of the 16 lanes and S::WGM waves that share its columns: parked in LDS (rows four
+    // floats apart in their banks), added in a fixed order
+    if (do_cs) {
+      constexpr int ROWS = S::WGM * 16, PITCH = 2 * NCOLS + 4;
+      static_assert(ROWS * PITCH * 4 <= S::LDS, "the sums fit the operand stages");
+      float* red = reinterpret_cast<float*>(smem_raw);
+      __syncthreads();  // the last K tile has been consumed
+#pragma unroll
+      for (int g = 0; g < NG; ++g)
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+          *reinterpret_cast<f32x4*>(red + (wm * 16 + i16) * PITCH + (h >> 1) * NCOLS + (int)(n_lane[g] - n0) + (h & 1) * 4) =
+              f32x4{cs[g][4 * h], cs[g][4 * h + 1], cs[g][4 * h + 2], cs[g][4 * h + 3]};
+      __syncthreads();
+      for (int c = threadIdx.x; c < 2 * NCOLS; c += S::NTHREADS) {
+        const int half = c / NCOLS, col = c % NCOLS;
+        float t = 0.f;
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) t += red[r * PITCH + c];
+        if (n0 + col < p.N) p.colsum[(int64_t)tm * p.ldc + (half ? p.aux_off : 0) + n0 + col] = t;
       }
     }
   }

@@ -305,9 +305,9 @@ def _block_backward(dx2: torch.Tensor, x: torch.Tensor, saved: tuple, W: BlockWe
     g_wd = torch.empty(C, I, dtype=gdt["mlp.down_proj.weight"], device=dev)
     g_bd = off_chain(lambda: ops.weight_grad(dx2, h, g_wd, gdt["mlp.down_proj.bias"], n=I))
     dgu = torch.empty(S, 2 * Ipad, dtype=x.dtype, device=dev)
-    # with many rows the epilogue also hands back per-tile column sums of dgu in fp32: the gate / up bias gradient
-    fused = x.dtype == torch.bfloat16 and ops.swiglu_bwd_sums_columns(S, Ipad, C)
-    part = torch.empty(-(-S // 256), 2 * Ipad, dtype=torch.float32, device=dev) if fused else None
+    # the bf16 epilogue also hands back per-tile column sums of dgu, of its fp32 values: the gate / up bias gradient
+    fused = x.dtype == torch.bfloat16
+    part = torch.empty(-(-S // ops.swiglu_bwd_colsum_rows(S, Ipad, C)), 2 * Ipad, dtype=torch.float32, device=dev) if fused else None
     ops.gemm(dx2, W.wdown, dgu, trans_b=True, epilogue=E.EPI_SWIGLU_BWD, residual=gu, aux_off=Ipad, colsum_partial=part)
     g_wgu = torch.empty(2 * Ipad, C, dtype=gdt["mlp.gate_proj.weight"], device=dev)
     b_gu = gdt["mlp.gate_proj.bias"]

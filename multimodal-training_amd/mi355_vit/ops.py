@@ -319,7 +319,8 @@ def gemm(
 
     Shapes: a [M,K] (or [K,M]); b [N,K] (or [K,N]); all 2-D with unit column stride (row strides free).
     ``n`` narrows the logical N (columns of B / out) below b's extent.
-    ``colsum_partial`` (EPI_SWIGLU_BWD only): fp32 [ceil(M/256), out.stride(0)] receiving per-tile column sums of out.
+    ``colsum_partial`` (EPI_SWIGLU_BWD only): fp32 [ceil(M/256) or ceil(M/64), out.stride(0)] receiving the column sums of that
+    many rows of out each (see ``swiglu_bwd_colsum_rows``), before the rounding to out's dtype.
     ``row_sums`` (bf16, both operands transposed, plain epilogue): [M] of out's dtype, receives the sums of op(A) over k.
     """
     for t, nm in ((a, "a"), (b, "b"), (out, "out")):
@@ -376,8 +377,10 @@ def gemm(
         if epilogue != _lib.EPI_SWIGLU_BWD:
             raise ValueError("gemm: colsum_partial is an output of the SwiGLU-backward epilogue only")
         cp = colsum_partial
-        if cp.dtype != torch.float32 or not cp.is_contiguous() or cp.shape != (-(-M // 256), out.stride(0)) or cp.device != a.device:
-            raise ValueError(f"gemm: colsum_partial must be contiguous fp32 [{-(-M // 256)}, {out.stride(0)}]")
+        by_64 = cp.shape[0] != -(-M // 256)  # up to 64 rows there is one row of sums either way: either kernel will do
+        if cp.dtype != torch.float32 or not cp.is_contiguous() or cp.shape != (-(-M // (64 if by_64 else 256)), out.stride(0)) or cp.device != a.device:
+            raise ValueError(f"gemm: colsum_partial must be contiguous fp32 [{-(-M // 256)} or {-(-M // 64)}, {out.stride(0)}]")
+        args.colsum_rows = 64 if by_64 or M <= 64 else 256
         args.workspace, args.workspace_bytes = cp.data_ptr(), cp.numel() * 4
     st = _stream(a)
     tag = f"gemm_{'t' if trans_a else 'n'}{'t' if trans_b else 'n'}_epi{epilogue}"
@@ -394,9 +397,9 @@ def wgrad_split_k(out_rows: int, out_cols: int, k: int) -> int:
 
 
 @functools.lru_cache(maxsize=None)
-def swiglu_bwd_sums_columns(rows: int, cols: int, k: int) -> bool:
-    """Whether the bf16 SwiGLU-backward product of this shape hands back the column sums of its result (many rows)."""
-    return bool(_lib.load().mvit_gemm_swiglu_bwd_sums_columns(rows, cols, k))
+def swiglu_bwd_colsum_rows(rows: int, cols: int, k: int) -> int:
+    """Rows per row of column sums (256 or 64) with which the bf16 SwiGLU-backward product of this shape is fastest."""
+    return _lib.load().mvit_gemm_swiglu_bwd_colsum_rows(rows, cols, k)
 
 
 MAX_DIRECT_PITCH = 1 << 22  # elements; wider rows go to the register-staged product, which makes no row sums

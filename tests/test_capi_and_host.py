@@ -338,3 +338,24 @@ def test_block_entry_points_refuse_malformed_arguments_before_any_launch():
     a.S = 0  # an empty block is accepted and does nothing
     a.side_stream = None
     assert lib.mvit_block_fwd(ctypes.byref(a), None) == 0 and lib.mvit_block_bwd(ctypes.byref(a), None) == 0
+
+
+def test_column_sums_of_the_swiglu_backward_are_refused_where_no_kernel_makes_them():
+    """colsum_rows is 256 (also 0) or 64, its workspace is checked, and 64 needs the bf16 tiles; nothing is launched."""
+    import ctypes
+
+    from mi355_vit import _lib
+
+    lib, fake = _lib.load(), 0x10000000
+    a = _lib.GemmArgs(dtype=_lib.BF16, out_dtype=_lib.BF16, trans_b=1, epilogue=_lib.EPI_SWIGLU_BWD, M=300, N=64, K=64, A=fake, lda=64, B=fake,
+                      ldb=64, C=fake, ldc=128, R=fake, ldr=128, aux_off=64, workspace=fake, workspace_bytes=5 * 128 * 4, colsum_rows=128)
+    call = lambda: lib.mvit_gemm(ctypes.byref(a), None)  # noqa: E731
+    assert call() == -1 and b"colsum_rows 128" in lib.mvit_last_error()
+    a.colsum_rows, a.workspace_bytes = 64, 5 * 128 * 4 - 1
+    assert call() == -1 and b"workspace of 2560 bytes" in lib.mvit_last_error()
+    a.colsum_rows, a.workspace_bytes = 0, 2 * 128 * 4 - 1
+    assert call() == -1 and b"workspace of 1024 bytes" in lib.mvit_last_error()
+    a.colsum_rows, a.workspace_bytes, a.out_dtype = 64, 5 * 128 * 4, _lib.F32
+    assert call() == -1 and b"need bf16 results" in lib.mvit_last_error()
+    for rows in (1, 64, 256, 2048, 8192, 65536):
+        assert lib.mvit_gemm_swiglu_bwd_colsum_rows(rows, 3456, 1280) in (64, 256)

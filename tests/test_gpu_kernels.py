@@ -480,6 +480,31 @@ def test_swiglu_backward_rows_do_not_depend_on_their_batch(N, K):
             assert torch.equal(run(rows, sums), everything[:rows]), (rows, sums)
 
 
+@pytest.mark.parametrize("per", [64, 256])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (64, 64, 72), (65, 72, 72), (257, 136, 64), (1030, 3456, 72), (5000, 200, 72)])
+def test_swiglu_backward_column_sums_are_of_unrounded_values(M, N, K, per):
+    """Per 64 or 256 rows, from either kernel, whole and partial tiles: sums of the fp32 results, not of their bf16 copies."""
+    _announce(f"gemm swiglu backward column sums {M}x{N}x{K} per {per}")
+    ops = _ops()
+    from mi355_vit import _lib as E
+
+    dy, w = _rand((M, K), torch.bfloat16, 0).to(DEV), _rand((K, N), torch.bfloat16, 1, K**-0.5).to(DEV)
+    gu = _rand((M, 2 * N + 16), torch.bfloat16, 2).to(DEV)[:, : 2 * N + 8]
+    out = torch.full((M, 2 * N + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    part = torch.full((-(-M // per), 2 * N + 8), 7.0, device=DEV)
+    ops.gemm(dy, w, out, trans_b=True, epilogue=E.EPI_SWIGLU_BWD, residual=gu, aux_off=N + 8, colsum_partial=part)
+    dh, g, u = dy.double() @ w.double(), gu[:, :N].double(), gu[:, N + 8 :].double()
+    s = torch.sigmoid(g)
+    mag = dy.double().abs() @ w.double().abs()
+    for at, fac in ((0, u * s * (1 + g * (1 - s))), (N + 8, g * s)):
+        exact, size = (torch.nn.functional.pad(v, (0, 0, 0, -M % per)).view(-1, per, N).sum(1) for v in (dh * fac, mag * fac.abs()))
+        # K fp32 additions per value, a few roundings of the derivative (its terms are at most about twice its size here; 2^-20
+        # covers them and the hardware exponential and reciprocal), `per` additions
+        err = (part[:, at : at + N].double() - exact).abs()
+        assert bool((err <= size * ((K + per) * 2.0**-24) + 2.0**-20 * size.clamp(min=1e-3 * size.max())).all()), float((err / size).max())
+    assert bool((part[:, N : N + 8] == 7.0).all()) and bool((out[:, N : N + 8] == 7.0).all())
+
+
 @pytest.mark.parametrize("unit,offset", [(16, 0), (16, 4), (4, 0), (2, 2), (1, 1)])
 @pytest.mark.parametrize("n", [1, 5, 96, 97, 200])
 def test_copy_ranges_bit_exact(unit, offset, n):

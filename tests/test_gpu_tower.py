@@ -437,6 +437,38 @@ def test_windowed_block_of_4096_rows_equals_its_four_shares():
         assert torch.equal(y, y_full[a : a + n]) and torch.equal(dx, dx_full[a : a + n]), a
 
 
+@pytest.mark.parametrize("one_call", [True, False])
+@pytest.mark.parametrize("S", [320, 4096, 5120])
+def test_gate_and_up_bias_gradients_are_sums_of_fp32_values(S, one_call, monkeypatch):
+    """The SwiGLU backward's results are summed before they are rounded to bf16, at any number of rows."""
+    from mi355_vit import functional as MF
+    from mi355_vit.config import Qwen2_5_VLVisionConfig
+    from mi355_vit.modeling import Qwen2_5_VLVisionBlock
+
+    print(f"[case] gate/up bias gradients, {S} rows, one call {one_call}", flush=True)
+    monkeypatch.setattr(MF, "BLOCK_CALLS", one_call)
+    torch.manual_seed(9)
+    cfg = Qwen2_5_VLVisionConfig(depth=1, hidden_size=1280, intermediate_size=3420, num_heads=16, out_hidden_size=256, fullatt_block_indexes=[])
+    blk = Qwen2_5_VLVisionBlock(cfg, 0).to(DEV)  # fp32 parameters: their gradients are not rounded
+    g = torch.Generator().manual_seed(9)
+    x, gy = (torch.randn(S, 1280, generator=g).to(torch.bfloat16).to(DEV) for _ in range(2))
+    emb = torch.randn(S, 40, generator=g).repeat(1, 2)
+    cu = torch.arange(0, S + 1, 64, dtype=torch.int32, device=DEV)
+    kept = []
+    backward = MF._block_backward
+    monkeypatch.setattr(MF, "_block_backward", lambda dx2, x, saved, W, *rest: (kept.append((saved[8], W)), backward(dx2, x, saved, W, *rest))[1])
+    xr = x.clone().requires_grad_(True)
+    blk(xr, cu_seqlens=cu, position_embeddings=(emb.cos().to(DEV), emb.sin().to(DEV))).backward(gy)
+    (gu, W), = kept
+    gate, up = gu[:, : W.I].double(), gu[:, W.Ipad : W.Ipad + W.I].double()
+    dh, s = gy.double() @ W.wdown.double()[:, : W.I], torch.sigmoid(gate)
+    for param, exact in ((blk.mlp.gate_proj.bias, (dh * up * s * (1 + gate * (1 - s))).sum(0)), (blk.mlp.up_proj.bias, (dh * gate * s).sum(0))):
+        err = float((param.grad.double() - exact).norm() / exact.norm())
+        # fp32 sums of 1,280 products, each value then with a relative error near sqrt(1280) * 2^-24 = 2e-6 (and as much again
+        # from the hardware exponential and reciprocal); summed after a rounding to bf16 it would be near 2^-9 / sqrt(3) = 1e-3
+        assert param.grad.dtype == torch.float32 and err < 2e-5, err
+
+
 def test_a_step_recorded_in_a_hip_graph_replays_bit_identically():
     """The library's launches allocate nothing, wait for nothing and use no stream but the caller's (the eager backward's
     second stream joins through events), so a whole forward and a whole backward can be recorded in HIP graphs.  Three
