@@ -10,6 +10,7 @@
 // with an IEEE division), so fp32 results can be compared bit for bit with a numpy restatement.
 #include "mvit_common.h"
 #include <string.h>
+#include <type_traits>
 
 namespace {
 
@@ -139,7 +140,7 @@ __device__ __forceinline__ TapWindow tap_window(const int32_t* __restrict__ boun
 // coordinate a window of `bounds[2*x + 1]` input coordinates starting at `bounds[2*x]`, 22-bit fixed-point weights
 // kk[x * ksize + i], an accumulator that starts at one half, an arithmetic shift and a clamp to 0..255.
 // inner is the contiguous dimension: pixels times channels for the vertical pass, 3 channels for the horizontal one.  The
-// kernels for those two follow; this one, a thread per output byte, takes everything else.
+// kernels for those two follow; resample_pass_kernel takes everything else.
 constexpr int RESAMPLE_PRECISION_BITS = 22;
 __device__ __forceinline__ unsigned clip8(int v) {
   v >>= RESAMPLE_PRECISION_BITS;
@@ -148,18 +149,44 @@ __device__ __forceinline__ unsigned clip8(int v) {
   asm("" : "+v"(v));
   return (unsigned)(v < 0 ? 0 : (v > 255 ? 255 : v));
 }
+// A thread makes four consecutive output bytes: of one output coordinate where inner is a multiple of four and the arrays are
+// made of aligned words (WORDS), else of the flattened [out_len * inner] row, each byte with its own window.
+template <bool WORDS>
 __global__ __launch_bounds__(256) void resample_pass_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, int64_t outer,
                                                             int64_t in_len, int64_t out_len, int64_t inner,
                                                             const int32_t* __restrict__ bounds, const int32_t* __restrict__ kk, int ksize) {
-  const int64_t row_out = out_len * inner, row_in = in_len * inner;
-  const int64_t total = outer * row_out;
+  const int64_t row_out = out_len * inner, row_in = in_len * inner, quads = (row_out + 3) / 4, total = outer * quads;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-    const int64_t o = i / row_out, e = i % row_out, x = e / inner, c = e % inner;
-    const TapWindow tw = tap_window(bounds, x, ksize, in_len);
-    const int32_t* k = kk + x * ksize;
-    int a = 1 << (RESAMPLE_PRECISION_BITS - 1);
-    for (int t = 0; t < tw.n; ++t) a += (int)src[o * row_in + (int64_t)(tw.xmin + t) * inner + c] * k[t];
-    dst[i] = (uint8_t)clip8(a);
+    const int64_t o = i / quads, first = i % quads * 4;
+    const uint8_t* s = src + o * row_in;
+    uint8_t* d = dst + o * row_out + first;
+    int64_t x = first / inner, c = first % inner;
+    if constexpr (WORDS) {
+      const TapWindow tw = tap_window(bounds, x, ksize, in_len);
+      const int32_t* k = kk + x * ksize;
+      int a[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[e] = 1 << (RESAMPLE_PRECISION_BITS - 1);
+      for (int t = 0; t < tw.n; ++t) {
+        const unsigned w = *reinterpret_cast<const unsigned*>(s + (int64_t)(tw.xmin + t) * inner + c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[e] += (int)((w >> (8 * e)) & 0xffu) * k[t];
+      }
+      *reinterpret_cast<unsigned*>(d) = clip8(a[0]) | (clip8(a[1]) << 8) | (clip8(a[2]) << 16) | (clip8(a[3]) << 24);
+    } else {
+      const int n_bytes = row_out - first < 4 ? (int)(row_out - first) : 4;
+      for (int e = 0; e < n_bytes; ++e) {
+        const TapWindow tw = tap_window(bounds, x, ksize, in_len);
+        const int32_t* k = kk + x * ksize;
+        int a = 1 << (RESAMPLE_PRECISION_BITS - 1);
+        for (int t = 0; t < tw.n; ++t) a += (int)s[(int64_t)(tw.xmin + t) * inner + c] * k[t];
+        d[e] = (uint8_t)clip8(a);
+        if (++c == inner) {
+          c = 0;
+          ++x;
+        }
+      }
+    }
   }
 }
 
@@ -267,46 +294,60 @@ __global__ __launch_bounds__(256) void resample_narrow_kernel(const ResampleJobs
   }
 }
 
-// The pass for a long contiguous dimension of whole words (the vertical pass): the window and its weights are the same for a
-// whole output row, so they are read once per work-group, and a thread makes four consecutive bytes.
+// The pass for a long contiguous dimension of whole words (the vertical pass).  A wave makes 1 KiB of one output row: the window
+// and its weights are the same for all of it (scalar loads), a lane makes 16 bytes from one 16-byte load per tap.  The four waves
+// of a work-group make the same KiB of four consecutive rows, whose windows overlap and meet in the L1.  Bound by the byte
+// extractions and multiply-adds (two instructions per byte and tap).  4,480 x 4,480 to 3,584 x 3,584 takes 137 us with the
+// horizontal pass; one word per lane, a row per work-group and the weights read by each took 180, four bytes per lane of the
+// flattened array 145.  A wave costs as much with few lanes as with 64: 480 rows to 168, 12 taps, 64 times, us of
+// resample_pass_kernel<true> / this one: 336 bytes 11.5 by the first, 420: 16.3 / 13.4, 512: 17.7 / 13.4, 1,024: 32.7 / 16.0, 3,024: 87 / 40
+constexpr int RESAMPLE_STRIP = 1024, RESAMPLE_WIDE_FROM = 400;
 template <bool FAST>
-__device__ __forceinline__ unsigned resample_wide_word(const uint8_t* p, int64_t inner, int n, const int32_t* __restrict__ k) {
-  int a[4];
+__device__ __forceinline__ void resample_wide_bytes(const uint8_t* p, int64_t inner, int n, const int32_t* __restrict__ k, unsigned (&out)[4]) {
+  typedef __attribute__((address_space(1))) const uint8_t* global_bytes;
+  int a[16];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) a[e] = 1 << (RESAMPLE_PRECISION_BITS - 1);
+  for (int e = 0; e < 16; ++e) a[e] = 1 << (RESAMPLE_PRECISION_BITS - 1);
+  auto taps = [&](auto COUNT, int t) {
+    constexpr int N = decltype(COUNT)::value;
+    unsigned w[N][4];
+#pragma unroll
+    for (int i = 0; i < N; ++i) __builtin_memcpy(w[i], (global_bytes)(uintptr_t)(p + (int64_t)(t + i) * inner), 16);
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) a[e] = tap<FAST>(a[e], (w[i][e >> 2] >> (8 * (e & 3))) & 0xffu, k[t + i]);
+  };
   int t = 0;
-  for (; t + 4 <= n; t += 4) {
-    unsigned w[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) w[i] = *reinterpret_cast<const unsigned*>(p + (int64_t)(t + i) * inner);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) a[e] = tap<FAST>(a[e], (w[i] >> (8 * e)) & 0xffu, k[t + i]);
+  for (; t + 4 <= n; t += 4) taps(std::integral_constant<int, 4>{}, t);
+  if (n & 2) {
+    taps(std::integral_constant<int, 2>{}, t);
+    t += 2;
   }
-  for (; t < n; ++t) {
-    const unsigned w = *reinterpret_cast<const unsigned*>(p + (int64_t)t * inner);
+  if (n & 1) taps(std::integral_constant<int, 1>{}, t);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) a[e] = tap<FAST>(a[e], (w >> (8 * e)) & 0xffu, k[t]);
-  }
-  return clip8(a[0]) | (clip8(a[1]) << 8) | (clip8(a[2]) << 16) | (clip8(a[3]) << 24);
+  for (int e = 0; e < 4; ++e) out[e] = clip8(a[4 * e]) | (clip8(a[4 * e + 1]) << 8) | (clip8(a[4 * e + 2]) << 16) | (clip8(a[4 * e + 3]) << 24);
 }
 __global__ __launch_bounds__(256) void resample_wide_kernel(const ResampleJobs jobs) {
   const int j = resample_job_of(jobs, blockIdx.x);
   const mvit_resample_job& jb = jobs.job[j];
-  const int block = blockIdx.x - jobs.first_block[j];
-  const int64_t words = jb.inner / 4;
-  const int wblocks = (int)((words + 255) / 256);
-  const int64_t row = block / wblocks, o = row / jb.out_len, x = row % jb.out_len;
+  const unsigned block = blockIdx.x - jobs.first_block[j];
+  const unsigned strips = (unsigned)((jb.inner + RESAMPLE_STRIP - 1) / RESAMPLE_STRIP), groups = (unsigned)((jb.out_len + 3) / 4);
+  const unsigned line = block / strips, o = line / groups;
+  const int x = (int)(line % groups) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (x >= jb.out_len) return;
   const TapWindow tw = tap_window(jb.bounds, x, jb.ksize, jb.in_len);
-  const int32_t* k = jb.kk + x * jb.ksize;
+  const int32_t* __restrict__ k = jb.kk + (int64_t)x * jb.ksize;
   bool narrow = true;
   for (int t = 0; t < tw.n; ++t) narrow = narrow && fits24(k[t]);
-  const int64_t w = (int64_t)(block % wblocks) * 256 + threadIdx.x;
-  if (w >= words) return;
-  const uint8_t* p = jb.src + (o * jb.in_len + tw.xmin) * jb.inner + 4 * w;
-  const unsigned v = narrow ? resample_wide_word<true>(p, jb.inner, tw.n, k) : resample_wide_word<false>(p, jb.inner, tw.n, k);
-  *reinterpret_cast<unsigned*>(jb.dst + row * jb.inner + 4 * w) = v;
+  int64_t at = (int64_t)(block % strips) * RESAMPLE_STRIP + (threadIdx.x & 63) * 16;
+  if (at >= jb.inner) return;
+  if (at > jb.inner - 16) at = jb.inner - 16;  // the last lane of a row ends with it and repeats bytes of its neighbour
+  const uint8_t* p = jb.src + ((int64_t)o * jb.in_len + tw.xmin) * jb.inner + at;
+  unsigned v[4];
+  if (narrow) resample_wide_bytes<true>(p, jb.inner, tw.n, k, v);
+  else resample_wide_bytes<false>(p, jb.inner, tw.n, k, v);
+  __builtin_memcpy(jb.dst + ((int64_t)o * jb.out_len + x) * jb.inner + at, v, 16);
 }
 
 extern "C" {
@@ -368,14 +409,14 @@ int mvit_resample_u8_batch(const mvit_resample_job* list, int n_jobs, mvit_strea
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   // work-groups for `outer` rows of the outermost axis
   auto groups = [](int kind, const mvit_resample_job& j, int64_t outer) {
-    return kind == 5 ? outer * j.out_len * ((j.inner / 4 + 255) / 256) : (j.out_len + 63) / 64 * ((outer + 4 * RESAMPLE_ROWS - 1) / (4 * RESAMPLE_ROWS));
+    return kind == 5 ? outer * ((j.out_len + 3) / 4) * ((j.inner + RESAMPLE_STRIP - 1) / RESAMPLE_STRIP) : (j.out_len + 63) / 64 * ((outer + 4 * RESAMPLE_ROWS - 1) / (4 * RESAMPLE_ROWS));
   };
-  // jobs of one kind (wide words; 1 .. 4 bytes) share launches; 0: everything else, a launch each
+  // jobs of one kind (wide words; 1 .. 4 bytes) share launches; 0: everything else, a launch each.  On short rows most lanes
+  // of the wide kernel would have nothing to do
+  auto words = [](const mvit_resample_job& j) { return j.inner % 4 == 0 && reinterpret_cast<uintptr_t>(j.src) % 4 == 0 && reinterpret_cast<uintptr_t>(j.dst) % 4 == 0; };
   auto kind_of = [&](const mvit_resample_job& j) {
-    if (j.inner % 4 == 0 && j.inner > RESAMPLE_MAX_CHANNELS && reinterpret_cast<uintptr_t>(j.src) % 4 == 0 && reinterpret_cast<uintptr_t>(j.dst) % 4 == 0 &&
-        groups(5, j, 1) <= MVIT_MAX_GROUPS_256)
-      return 5;
-    return j.inner <= RESAMPLE_MAX_CHANNELS ? (int)j.inner : 0;
+    if (j.inner <= RESAMPLE_MAX_CHANNELS) return (int)j.inner;
+    return words(j) && j.inner >= RESAMPLE_WIDE_FROM && groups(5, j, 1) <= MVIT_MAX_GROUPS_256 ? 5 : 0;
   };
   for (int kind = 0; kind <= 5; ++kind) {
     ResampleJobs jobs;
@@ -400,9 +441,10 @@ int mvit_resample_u8_batch(const mvit_resample_job* list, int n_jobs, mvit_strea
       const mvit_resample_job& j = list[i];
       if (j.outer == 0 || kind_of(j) != kind) continue;
       if (kind == 0) {
-        const int64_t total = j.outer * j.out_len * j.inner;
-        hipLaunchKernelGGL(resample_pass_kernel, dim3((unsigned)((total + 255) / 256 < 65535 * 16 ? (total + 255) / 256 : 65535 * 16)), 256, 0, s,
-                           j.src, j.dst, j.outer, j.in_len, j.out_len, j.inner, j.bounds, j.kk, j.ksize);
+        const int64_t total = j.outer * ((j.out_len * j.inner + 3) / 4), want = (total + 255) / 256;
+        const dim3 grid((unsigned)(want < 65535 * 16 ? want : 65535 * 16));
+        if (words(j)) hipLaunchKernelGGL((resample_pass_kernel<true>), grid, 256, 0, s, j.src, j.dst, j.outer, j.in_len, j.out_len, j.inner, j.bounds, j.kk, j.ksize);
+        else hipLaunchKernelGGL((resample_pass_kernel<false>), grid, 256, 0, s, j.src, j.dst, j.outer, j.in_len, j.out_len, j.inner, j.bounds, j.kk, j.ksize);
         MVIT_CHECK_LAUNCH("resample_u8");
         continue;
       }

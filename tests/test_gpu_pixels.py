@@ -443,6 +443,40 @@ def test_resize_rejects_what_it_cannot_do():
     assert same.data_ptr() != x.data_ptr() and torch.equal(same, x)
 
 
+@pytest.mark.parametrize("offset", [0, 2])
+@pytest.mark.parametrize("inner", [1, 4, 5, 8, 396, 400, 404, 510, 1020, 1024, 1028, 2060, 3087])
+def test_resample_over_every_inner_length(inner, offset):
+    """Channels, words, whole and partial strips, rows that are no whole words, arrays off the word boundary; windows of one to
+    nine taps, of which some have weights of more than 24 bits; bytes beyond the result left alone."""
+    from mi355_vit import _lib
+
+    _announce(f"resample inner={inner} offset={offset}")
+    rng = np.random.default_rng(inner)
+    outer, in_len, out_len, ksize = 3, 20, 13, 9
+    src = rng.integers(0, 256, (outer, in_len, inner), dtype=np.uint8)
+    bounds, kk = np.zeros((out_len, 2), dtype=np.int32), np.zeros((out_len, ksize), dtype=np.int32)
+    ref = np.empty((outer, out_len, inner), dtype=np.uint8)
+    for x in range(out_len):
+        n = x % ksize + 1
+        bounds[x] = (min(x, in_len - n), n)
+        kk[x, :n] = rng.integers(-(1 << 20), 1 << 21, n)
+        if n > 1 and x % 2:
+            kk[x, :2] = ((1 << 23) + 5, -(1 << 23))
+            kk[x, 2:n] //= 1024  # 2^21 + 255 * (2^23 + 5) + 7 * 255 * 2^11 < 2^31: the 32-bit sums do not wrap
+        lo = bounds[x, 0]
+        acc = (1 << 21) + (src[:, lo : lo + n, :].astype(np.int64) * kk[x, :n, None]).sum(axis=1)
+        ref[:, x, :] = np.clip(acc >> 22, 0, 255)
+    d_src, d_dst = (torch.full((a.size + 32,), 9, dtype=torch.uint8, device=DEV) for a in (src, ref))
+    d_src[offset : offset + src.size] = torch.from_numpy(src.reshape(-1)).to(DEV)
+    d_b, d_k = torch.from_numpy(bounds).to(DEV), torch.from_numpy(kk).to(DEV)
+    rc = _lib.load().mvit_resample_u8(d_src.data_ptr() + offset, d_dst.data_ptr() + offset, outer, in_len, out_len, inner, d_b.data_ptr(), d_k.data_ptr(),
+                                      ksize, torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "mvit_resample_u8")
+    got = d_dst.cpu().numpy()
+    assert np.array_equal(got[offset : offset + ref.size].reshape(ref.shape), ref)
+    assert (got[:offset] == 9).all() and (got[offset + ref.size :] == 9).all()
+
+
 @pytest.mark.parametrize("outer,inner", [((1 << 29) + 100, 1), ((1 << 24) + 5, 8)])
 def test_resample_of_more_work_groups_than_a_launch_takes(outer, inner):
     """A launch takes fewer than 2^24 work-groups of 256 threads; longer passes go in several.  One tap of weight one: a copy."""
