@@ -532,6 +532,24 @@ def test_copy_ranges_bit_exact(unit, offset, n):
     assert torch.equal(dst, want)
 
 
+@pytest.mark.parametrize("row_bytes", [2, 6, 20, 32, 2560, 5120 * 16])
+def test_segment_copy_entry_point_with_its_list_on_the_device(row_bytes):
+    """mvit_segment_copy, for callers whose list is in device memory; words of 2, 4 and 16 bytes, bit-exact."""
+    from mi355_vit import _lib
+
+    _announce(f"segment copy, rows of {row_bytes} bytes")
+    g = torch.Generator().manual_seed(row_bytes)
+    src = torch.randint(0, 256, (300, row_bytes), dtype=torch.uint8, generator=g)
+    segs = [(0, 260, 40), (40, 200, 0), (290, 0, 10), (41, 11, 189)]
+    want = torch.full((310, row_bytes), 9, dtype=torch.uint8)
+    for a, b, n in segs:
+        want[b : b + n] = src[a : a + n]
+    d_src, dst, desc = src.to(DEV), torch.full_like(want, 9).to(DEV), torch.tensor(segs, dtype=torch.int64, device=DEV)
+    _lib.check(_lib.load().mvit_segment_copy(d_src.data_ptr(), dst.data_ptr(), desc.data_ptr(), len(segs), 189, row_bytes,
+                                             torch.cuda.current_stream().cuda_stream), "mvit_segment_copy")
+    assert torch.equal(dst.cpu(), want)
+
+
 @pytest.mark.parametrize("cpu", ["first source", "first destination", "last source", "last destination"])
 def test_segment_copies_refuse_host_memory_anywhere_in_the_list(cpu):
     """Addresses go straight to a kernel: every tensor of the list is on the GPU, not the last source alone."""

@@ -44,6 +44,16 @@ def test_patchify_bit_exact_against_oracle_ragged_images_and_videos(seed):
     assert np.array_equal(got.numpy().view(np.uint32), ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("n", [64, 65, 150])
+def test_patchify_image_tables_that_travel_with_the_launch_and_longer_ones(n):
+    """Tables of up to 64 images are a kernel argument, longer ones are copied to the device."""
+    _announce(f"patchify {n} images")
+    images = _batch(7, [(1 + (i % 5 == 4), 28 * (1 + i % 3), 28 * (1 + i % 2)) for i in range(n)])
+    got, grid = _run(images)
+    ref, ref_grid = po.patchify_batch(images)
+    assert grid.tolist() == ref_grid.tolist() and np.array_equal(got.numpy().view(np.uint32), ref.view(np.uint32))
+
+
 def test_patchify_bf16_is_the_rounded_fp32_result():
     _announce("patchify bf16")
     images = _batch(2, RAGGED[:5])
@@ -477,7 +487,7 @@ def test_resample_over_every_inner_length(inner, offset):
     assert (got[:offset] == 9).all() and (got[offset + ref.size :] == 9).all()
 
 
-@pytest.mark.parametrize("outer,inner", [((1 << 29) + 100, 1), ((1 << 24) + 5, 8)])
+@pytest.mark.parametrize("outer,inner", [((1 << 29) + 100, 1), ((1 << 24) + 5, 8), ((1 << 24) + 5, 400)])
 def test_resample_of_more_work_groups_than_a_launch_takes(outer, inner):
     """A launch takes fewer than 2^24 work-groups of 256 threads; longer passes go in several.  One tap of weight one: a copy."""
     from mi355_vit import _lib
