@@ -756,13 +756,6 @@ struct DlFrag {
   }
 };
 
-// Whether gemm_dl_kernel starts the next tile's loads before the epilogue of the current one: the weight-gradient
-// GEMMs (A transposed) with a plain or bias epilogue.  Measured on the full tower: those kernels get 2-3 % faster and
-// the step follows; the forward and input-gradient GEMMs also get 1-3 % faster alone, but the step with the
-// weight gradients running beside them on a second stream gets slower, so they keep starting a tile after the
-// epilogue.  The fused epilogues have no registers to spare for the next tile's addresses.
-constexpr bool dl_prefetches(int epi, bool ta) { return (epi == MVIT_EPI_NONE || epi == MVIT_EPI_BIAS) && ta; }
-
 // Wait until at most n K tiles' loads (PER per lane each) are still in flight.
 template <int PER>
 __device__ __forceinline__ void wait_tiles(int n) {
@@ -775,7 +768,7 @@ __device__ __forceinline__ void wait_tiles(int n) {
 // PIX: the A operand is made from decoded frames (DlPixelOperand)
 template <typename TO, bool TA, bool TB, int EPI, int NSTAGE, int NW, bool MI16 = false, bool PIX = false>
 __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_dl_kernel(const GemmParams p) {
-  static_assert(!PIX || (!TA && !MI16 && !dl_prefetches(EPI, TA)), "frames as the A operand: [row][k] layout, 32x32x16 fragments, no early loads");
+  static_assert(!PIX || (!TA && !MI16), "frames as the A operand: [row][k] layout, 32x32x16 fragments");
   using T = bf16_t;
   using D = DL<NW>;
   constexpr int BM = D::BM, BN = D::BN, WM = D::WM, WN = D::WN, TILE = D::TILE_BYTES, SLICE = D::CPT * 1024;
@@ -797,12 +790,6 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_dl_kernel(const GemmPara
 
   // Persistent work-groups: the grid has at most one work-group per CU; work-group (xcd, slot) walks that XCD's
   // tile range with stride slots-per-XCD, the order a one-tile-per-work-group grid would be dispatched in.
-  // Where dl_prefetches() says so, the first two K tiles of a work-group's next output tile are requested before the
-  // epilogue of the current one, so they travel while the results are parked and stored: the epilogue then stages
-  // through the later B stages and the LDS behind them, which those loads do not touch.
-  constexpr bool PREFETCH = dl_prefetches(EPI, TA);
-  constexpr int EARLY = PREFETCH ? (NSTAGE - 1 < 2 ? NSTAGE - 1 : 2) : NSTAGE - 1;  // K tiles requested by start_tile
-  constexpr int STAGING_OFF = PREFETCH ? (NSTAGE + EARLY) * TILE : 0;
   typename std::conditional<PIX, DlPixelOperand<NW>, DlOperand<TA, false, NW, MI16>>::type la;
   DlOperand<TB, DUAL, NW, MI16> lb;
   int T_ = 0, k_tail = 0;  // of the tile whose operands are being loaded
@@ -852,17 +839,11 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_dl_kernel(const GemmPara
     T_ = (klen + DL_BK - 1) / DL_BK;
     k_tail = klen % DL_BK;
 #pragma unroll
-    for (int t = 0; t < EARLY; ++t) issue(t, t);
+    for (int t = 0; t < NSTAGE - 1; ++t) issue(t, t);
     return true;
   };
   int idx = blockIdx.x >> 3;
-  [[maybe_unused]] bool have = PREFETCH ? start_tile(idx) : true;
-  while (true) {
-  if constexpr (PREFETCH) {
-    if (!have) break;
-  } else {
-    if (!start_tile(idx)) break;
-  }
+  while (start_tile(idx)) {
   const int slice = next_slice;
   const int64_t m0 = next_m0, n0 = next_n0;
 
@@ -876,8 +857,6 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_dl_kernel(const GemmPara
 
   EpiPre<T, EPI, BM, BN, WM, D::NTHREADS> ep;
   ep.init(p, m0, n0);
-#pragma unroll
-  for (int t = EARLY; t < NSTAGE - 1; ++t) issue(t, t);  // the stages the previous tile's epilogue was using
 
   [[maybe_unused]] bf16x8 fa[2][MT], fb[2][NT];
   for (int t0 = 0; t0 < T_; t0 += NSTAGE) {
@@ -949,10 +928,9 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_dl_kernel(const GemmPara
       }
     }
   }
-  __syncthreads();  // operands fully consumed before the next tile's first loads (or the epilogue) overwrite them
+  __syncthreads();  // operands fully consumed before the epilogue overwrites them
   idx += gridDim.x >> 3;
-  if constexpr (PREFETCH) have = start_tile(idx);
-  run_epilogue<T, TO, EPI, BM, BN, WM, WN, D::NTHREADS, MI16>(p, acc, smem_raw + STAGING_OFF, m0, n0, wm, wn, slice, ep);
+  run_epilogue<T, TO, EPI, BM, BN, WM, WN, D::NTHREADS, MI16>(p, acc, smem_raw, m0, n0, wm, wn, slice, ep);
   __syncthreads();  // the staging area is free again before operands land in it
   }
 }
@@ -1078,9 +1056,7 @@ int launch_dl(const GemmParams& p, hipStream_t stream) {
   using D = DL<NW>;
   constexpr size_t operands = 2 * (size_t)NSTAGE * D::TILE_BYTES;
   constexpr size_t staging = (size_t)(D::BM / D::WM) * 32 * D::BN * sizeof(float);
-  // with prefetching the staging area starts behind the B stages that the next tile's first two K tiles arrive in
-  constexpr size_t staging_end = dl_prefetches(EPI, TA) ? (NSTAGE + (NSTAGE - 1 < 2 ? NSTAGE - 1 : 2)) * D::TILE_BYTES + staging : staging;
-  constexpr size_t lds = staging_end > operands ? staging_end : operands;
+  constexpr size_t lds = staging > operands ? staging : operands;
   static_assert(lds <= 160 * 1024, "operand stages plus the epilogue staging area exceed the LDS of a CU");
   auto kern = gemm_dl_kernel<TO, TA, TB, EPI, NSTAGE, NW, MI16, PIX>;
   static bool attr_set_on[MVIT_MAX_DEVICES] = {};  // once per kernel and device
@@ -1108,13 +1084,17 @@ int launch_dl(const GemmParams& p, hipStream_t stream) {
 
 template <typename T, typename TO, bool TA, bool TB, int EPI>
 int launch_var(int var, const GemmParams& p, hipStream_t s) {
-  {
+  // always served by the tiles that choose_tile() picks from, unless a row pitch exceeds 32-bit lane offsets
+  constexpr bool TILED = sizeof(TO) == 2 ? (EPI == MVIT_EPI_NONE || EPI == MVIT_EPI_GELU_BWD) : (TA && TB && EPI == MVIT_EPI_NONE);
+  if constexpr (!TILED) {
     // direct-to-LDS main loop: v_mfma_f32_16x16x32_bf16 for the plain GEMMs with an operand behind the transposing
-    // LDS read (weight gradients +6 %, input gradients +1 % on real data), v_mfma_f32_32x32x16_bf16 for the forward
-    // GEMMs (both operands row-major: 3-5 % faster that way).  SwiGLU backward takes the form of the smaller tiles that
-    // serve few rows (gemm_small.hip): a row's gradient has the same bits whatever batch it lies in
-    constexpr int NS = 4;
-    if (var == 3) return (TB && (EPI == MVIT_EPI_NONE || EPI == MVIT_EPI_SWIGLU_BWD)) ? launch_dl<TO, TA, TB, EPI, NS, 8, true>(p, s) : launch_dl<TO, TA, TB, EPI, NS, 8>(p, s);
+    // LDS read (input gradients +1 % on real data), v_mfma_f32_32x32x16_bf16 for the forward GEMMs (both operands
+    // row-major: 3-5 % faster that way).  SwiGLU backward takes the form of the smaller tiles that serve few rows
+    // (gemm_small.hip): a row's gradient has the same bits whatever batch it lies in
+    constexpr bool MI16 = TB && (EPI == MVIT_EPI_NONE || EPI == MVIT_EPI_SWIGLU_BWD);
+    if (var == 3) return launch_dl<TO, TA, TB, EPI, 4, 8, MI16>(p, s);
+  } else if (var == 3) {
+    return mvit_set_error(MVIT_ERR_UNSUPPORTED, "gemm: epilogue %d of trans_a=%d trans_b=%d is served by tiles", EPI, (int)TA, (int)TB);
   }
   return launch<T, TO, TA, TB, EPI, 1>(p, s);  // register-staged main loop: operands whose row pitch exceeds 32-bit lane offsets
 }
