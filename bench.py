@@ -79,9 +79,11 @@ def seg_sq_sum(cu: torch.Tensor) -> float:
 
 def summarise_trace(records, cfg_kw, dtype):
     """Per-tag totals: launches, milliseconds, algorithmic FLOPs or bytes."""
+    from mi355_vit.functional import padded_inner
+
     I = cfg_kw["intermediate_size"]
-    ipad = (I + 7) // 8 * 8
-    unpad = {ipad: I, 2 * ipad: 2 * I}
+    ipad = padded_inner(I)
+    unpad = {ipad: I, 2 * ipad: 2 * I}  # the padding of the MLP's hidden width is no work
     out = {}
     for tag, info, e0, e1 in records:
         ms = e0.elapsed_time(e1)
@@ -96,7 +98,13 @@ def summarise_trace(records, cfg_kw, dtype):
         ent["ms_counted"] += ms
         if tag.startswith("gemm"):
             halves = 2.0 if tag.endswith("epi4") else 1.0  # SWIGLU: N counts one of the two weight matrices
-            ent["flops"] += halves * 2.0 * info["M"] * unpad.get(info["N"], info["N"]) * unpad.get(info["K"], info["K"])
+            # M counts tokens, or features in a weight gradient, whose K counts tokens
+            m, n, k = info["M"], unpad.get(info["N"], info["N"]), info["K"]
+            if tag.startswith("gemm_tt"):
+                m = unpad.get(m, m)
+            else:
+                k = unpad.get(k, k)
+            ent["flops"] += halves * 2.0 * m * n * k
         elif tag.startswith("attn_fwd"):
             ent["flops"] += 4.0 * seg_sq_sum(info["cu"].cpu()) * info["head_dim"] * info["nheads"]
         elif tag.startswith("attn_bwd"):

@@ -359,3 +359,23 @@ def test_column_sums_of_the_swiglu_backward_are_refused_where_no_kernel_makes_th
     assert call() == -1 and b"need bf16 results" in lib.mvit_last_error()
     for rows in (1, 64, 256, 2048, 8192, 65536):
         assert lib.mvit_gemm_swiglu_bwd_colsum_rows(rows, 3456, 1280) in (64, 256)
+
+
+def test_benchmark_counts_no_padding_as_work():
+    import sys
+
+    sys.path.insert(0, str(ROOT))
+    import bench
+    from mi355_vit.functional import padded_inner
+
+    class Event:
+        def elapsed_time(self, other):
+            return 1.0
+
+    ipad = padded_inner(3420)
+    assert ipad != 3420
+    records = [("gemm_tt_epi0", {"M": 2 * ipad, "N": 1280, "K": ipad}, Event(), Event()),  # a gate/up weight gradient over as many tokens
+               ("gemm_nn_epi2", {"M": ipad, "N": 1280, "K": ipad}, Event(), Event()),      # a down projection of as many tokens
+               ("gemm_nn_epi4", {"M": 100, "N": ipad, "K": 1280}, Event(), Event())]
+    flops = {tag: ent["flops"] for tag, ent in bench.summarise_trace(records, {"intermediate_size": 3420}, None).items()}
+    assert flops == {"gemm_tt_epi0": 2.0 * 6840 * 1280 * ipad, "gemm_nn_epi2": 2.0 * ipad * 1280 * 3420, "gemm_nn_epi4": 4.0 * 100 * 3420 * 1280}
