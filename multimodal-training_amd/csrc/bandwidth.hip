@@ -374,7 +374,8 @@ static inline hipStream_t S_(mvit_stream_t s) { return reinterpret_cast<hipStrea
 // replaced by the vision rows, the k-th placeholder taking vision row k (masked_scatter with a row mask).
 // One work-group ranks the placeholders: each of its 16 waves counts a contiguous slice 64 tokens at a time (ballots), the
 // counts are scanned, and the slice is walked again, from the cache, to write ranks and positions.  The row merge is then a
-// pure byte copy.  Bound by the latency of two walks (7,405 tokens: 16.6 us with a slice per thread, 5 us so).
+// pure byte copy.  Bound by the latency of two walks (7,405 tokens: 17.1 us with a slice per thread, so 6.6 with the ids in the
+// cache and 12.8 in place, where they are cold and the counts go to host memory).
 __global__ __launch_bounds__(1024) void image_token_ranks_kernel(const int64_t* __restrict__ ids, const int64_t* __restrict__ labels,
                                                                  int64_t n, int64_t image_id, int64_t ignore_label,
                                                                  int32_t* __restrict__ rank, int64_t* __restrict__ positions,
