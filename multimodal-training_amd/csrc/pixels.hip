@@ -301,7 +301,7 @@ __global__ __launch_bounds__(256) void resample_narrow_kernel(const ResampleJobs
 // horizontal pass; one word per lane, a row per work-group and the weights read by each took 180, four bytes per lane of the
 // flattened array 145.  A wave costs as much with few lanes as with 64: 480 rows to 168, 12 taps, 64 times, us of
 // resample_pass_kernel<true> / this one: 336 bytes 11.5 by the first, 420: 16.3 / 13.4, 512: 17.7 / 13.4, 1,024: 32.7 / 16.0, 3,024: 87 / 40
-constexpr int RESAMPLE_STRIP = 1024, RESAMPLE_WIDE_FROM = 400;
+constexpr int RESAMPLE_STRIP = 1024, RESAMPLE_WIDE_FROM = 400, RESAMPLE_FEW_ROWS = 4096;
 template <bool FAST>
 __device__ __forceinline__ void resample_wide_bytes(const uint8_t* p, int64_t inner, int n, const int32_t* __restrict__ k, unsigned (&out)[4]) {
   typedef __attribute__((address_space(1))) const uint8_t* global_bytes;
@@ -411,12 +411,13 @@ int mvit_resample_u8_batch(const mvit_resample_job* list, int n_jobs, mvit_strea
   auto groups = [](int kind, const mvit_resample_job& j, int64_t outer) {
     return kind == 5 ? outer * ((j.out_len + 3) / 4) * ((j.inner + RESAMPLE_STRIP - 1) / RESAMPLE_STRIP) : (j.out_len + 63) / 64 * ((outer + 4 * RESAMPLE_ROWS - 1) / (4 * RESAMPLE_ROWS));
   };
-  // jobs of one kind (wide words; 1 .. 4 bytes) share launches; 0: everything else, a launch each.  On short rows most lanes
-  // of the wide kernel would have nothing to do
+  // jobs of one kind (wide words; 1 .. 4 bytes) share launches; 0: everything else, a launch each.  Of short rows the
+  // wide kernel only takes so few (about 5 us) that a launch of their own would cost as much
   auto words = [](const mvit_resample_job& j) { return j.inner % 4 == 0 && reinterpret_cast<uintptr_t>(j.src) % 4 == 0 && reinterpret_cast<uintptr_t>(j.dst) % 4 == 0; };
   auto kind_of = [&](const mvit_resample_job& j) {
     if (j.inner <= RESAMPLE_MAX_CHANNELS) return (int)j.inner;
-    return words(j) && j.inner >= RESAMPLE_WIDE_FROM && groups(5, j, 1) <= MVIT_MAX_GROUPS_256 ? 5 : 0;
+    const bool wide = j.inner >= RESAMPLE_WIDE_FROM || (j.inner >= 16 && j.outer * j.out_len <= RESAMPLE_FEW_ROWS);
+    return words(j) && wide && groups(5, j, 1) <= MVIT_MAX_GROUPS_256 ? 5 : 0;
   };
   for (int kind = 0; kind <= 5; ++kind) {
     ResampleJobs jobs;

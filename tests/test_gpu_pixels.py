@@ -453,16 +453,17 @@ def test_resize_rejects_what_it_cannot_do():
     assert same.data_ptr() != x.data_ptr() and torch.equal(same, x)
 
 
+@pytest.mark.parametrize("outer", [3, 320])
 @pytest.mark.parametrize("offset", [0, 2])
-@pytest.mark.parametrize("inner", [1, 4, 5, 8, 396, 400, 404, 510, 1020, 1024, 1028, 2060, 3087])
-def test_resample_over_every_inner_length(inner, offset):
-    """Channels, words, whole and partial strips, rows that are no whole words, arrays off the word boundary; windows of one to
+@pytest.mark.parametrize("inner", [1, 4, 5, 8, 12, 16, 20, 396, 400, 404, 510, 1020, 1024, 1028, 2060, 3087])
+def test_resample_over_every_inner_length(inner, offset, outer):
+    """Channels, words, few and many short rows, whole and partial strips, rows that are no whole words, arrays off the word boundary; windows of one to
     nine taps, of which some have weights of more than 24 bits; bytes beyond the result left alone."""
     from mi355_vit import _lib
 
-    _announce(f"resample inner={inner} offset={offset}")
+    _announce(f"resample inner={inner} offset={offset} outer={outer}")
     rng = np.random.default_rng(inner)
-    outer, in_len, out_len, ksize = 3, 20, 13, 9
+    in_len, out_len, ksize = 20, 13, 9
     src = rng.integers(0, 256, (outer, in_len, inner), dtype=np.uint8)
     bounds, kk = np.zeros((out_len, 2), dtype=np.int32), np.zeros((out_len, ksize), dtype=np.int32)
     ref = np.empty((outer, out_len, inner), dtype=np.uint8)
