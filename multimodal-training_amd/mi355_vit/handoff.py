@@ -40,11 +40,15 @@ def _ranks(input_ids: torch.Tensor, labels: Optional[torch.Tensor], image_token_
     n = ids.numel()
     rank = torch.empty(n, dtype=torch.int32, device=ids.device)
     counts = torch.empty(2, dtype=torch.int64, pin_memory=True)  # the kernel writes them where the host reads them
-    ready, stream = torch.cuda.Event(), torch.cuda.current_stream(ids.device)  # nothing between the launch and the record may fail
     rc = _lib.load().mvit_image_token_ranks(ids.data_ptr(), None if lab is None else lab.data_ptr(), n, image_token_id, -100,
                                             rank.data_ptr(), None, counts.data_ptr(), _stream(ids))
     _lib.check(rc, "mvit_image_token_ranks")
-    ready.record(stream)
+    try:
+        ready = torch.cuda.Event()
+        ready.record(torch.cuda.current_stream(ids.device))
+    except BaseException:
+        torch.cuda.synchronize(ids.device)
+        raise
     return rank, counts, ready
 
 
