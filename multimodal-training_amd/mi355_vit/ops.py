@@ -231,30 +231,35 @@ def segment_copies(copies: Sequence[Tuple[torch.Tensor, torch.Tensor, Sequence[T
     The host validates bounds; the kernel moves bytes."""
     ranges, device = [], None
     for src, dst, segments in copies:
-        if src.dim() != 2 or dst.dim() != 2 or not (src.is_contiguous() and dst.is_contiguous()):
+        shape, to = src.shape, dst.shape
+        if len(shape) != 2 or len(to) != 2 or not (src.is_contiguous() and dst.is_contiguous()):
             raise ValueError("segment_copy: src and dst must be contiguous 2-D")
-        if src.shape[1] != dst.shape[1] or src.dtype != dst.dtype:
+        (n_src, cols), (n_dst, cols_dst) = shape, to
+        if cols != cols_dst or src.dtype != dst.dtype:
             raise ValueError("segment_copy: column count / dtype mismatch")
-        n_src, n_dst, row = src.shape[0], dst.shape[0], src.shape[1] * src.element_size()
+        row = cols * src.element_size()
         p_src, p_dst = src.data_ptr(), dst.data_ptr()
         before = len(ranges)
         for a, b, n in segments:
-            a, b, n = int(a), int(b), int(n)  # of a narrow integer type the products below would wrap
+            a_end, b_end = a + n, b + n
+            if a_end.__class__ is not int or b_end.__class__ is not int:  # of a narrow integer type the products below would wrap
+                a, b, n = int(a), int(b), int(n)
+                a_end, b_end = a + n, b + n
             if n <= 0:
                 continue
-            if a < 0 or b < 0 or a + n > n_src or b + n > n_dst:
+            if a < 0 or b < 0 or a_end > n_src or b_end > n_dst:
                 raise ValueError(f"segment_copy: segment ({a},{b},{n}) out of bounds for {n_src} -> {n_dst} rows")
             ranges += (p_src + a * row, p_dst + b * row, n * row)
         if len(ranges) > before:  # a kernel will read src and write dst: both on the GPU that the launch goes to
-            for t in (src, dst):
-                if not t.is_cuda:
-                    raise RuntimeError("mi355_vit kernels need tensors on the GPU; there is no CPU path")
-                device = device or t.device
-                if t.device != device:
-                    raise ValueError(f"segment_copy: tensors on {device} and {t.device} in one call")
+            on_src, on_dst = src.get_device(), dst.get_device()
+            if on_src < 0 or on_dst < 0:
+                raise RuntimeError("mi355_vit kernels need tensors on the GPU; there is no CPU path")
+            device = on_src if device is None else device
+            if on_src != device or on_dst != device:
+                raise ValueError(f"segment_copy: tensors on devices {device}, {on_src} and {on_dst} in one call")
     if ranges:
         flat = (C.c_uint64 * len(ranges))(*ranges)
-        _lib.check(_lib.load().mvit_copy_ranges(C.addressof(flat), len(ranges) // 3, _current_raw_stream(device.index)), "mvit_copy_ranges")
+        _lib.check(_lib.load().mvit_copy_ranges(C.addressof(flat), len(ranges) // 3, _current_raw_stream(device)), "mvit_copy_ranges")
 
 
 def segment_copy(src: torch.Tensor, dst: torch.Tensor, segments: Sequence[Tuple[int, int, int]]) -> torch.Tensor:
