@@ -4,7 +4,7 @@
 //   bf16, the products of the vision tower: gemm_pp_kernel (gemm_pingpong.hip) and, where its 256x256 tiles are too few,
 //      gemm_small_kernel (gemm_small.hip); choose_tile() below picks.
 //   bf16, the rest (SwiGLU backward of many rows, patch embedding from frames, fp32 outputs, accumulation): 256x256 tile, 8
-//      waves of 128x64 (4x2 MFMA 32x32x16 tiles each), BK = 32, four LDS stages filled by direct global -> LDS loads (see
+//      waves of 128x64 (4x2 blocks of 32x32 each), BK = 32, four LDS stages filled by direct global -> LDS loads (see
 //      gemm_dl_kernel).
 //   bf16 operands whose row pitch exceeds 2^22 elements (the direct loads use 32-bit lane offsets): 256x256 tile, 8 waves,
 //      BK = 64, global -> registers -> LDS, double-buffered LDS, one barrier per K step (gemm_kernel).
@@ -1164,7 +1164,7 @@ bool pp_takes(GemmTiledKind kind, int64_t k_chunk, int64_t k_last) {  // at leas
 
 // Modelled times (us) of the tiles on one MI355X, fitted to every tile's time at 256 ... 16,384 rows of the tower's products: a
 // step of 64 along K takes 1.15 us in a 256 x 256 tile (one work-group per compute unit; 1.2 with both operands behind the
-// transposing LDS read), and in the smaller ones `one` us while every unit has at most one work-group and `two` us once it has
+// transposing LDS read; 2,435 cycles, so more when the clock falls under a long load, which lengthens every tile's steps alike), and in the smaller ones `one` us while every unit has at most one work-group and `two` us once it has
 // two.  A fuller last round, a shorter step and more units at work all lower the estimate; the epilogue of a 256 x 256 tile is
 // the longest.  The line between the tiles follows from these numbers and not from any shape: e.g. input gradients of 1280
 // columns, K = 3840, are fastest on 64 x 64 up to 1,500 rows, on 64 x 128 to 3,100, on 128 x 128 to 6,500 and on 256 x 256 at
