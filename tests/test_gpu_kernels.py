@@ -480,17 +480,18 @@ def test_swiglu_backward_rows_do_not_depend_on_their_batch(N, K):
             assert torch.equal(run(rows, sums), everything[:rows]), (rows, sums)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("per", [64, 256])
 @pytest.mark.parametrize("M,N,K", [(1, 8, 8), (64, 64, 72), (65, 72, 72), (257, 136, 64), (1030, 3456, 72), (5000, 200, 72)])
-def test_swiglu_backward_column_sums_are_of_unrounded_values(M, N, K, per):
+def test_swiglu_backward_column_sums_are_of_unrounded_values(M, N, K, per, dtype):
     """Per 64 or 256 rows, from either kernel, whole and partial tiles: sums of the fp32 results, not of their bf16 copies."""
-    _announce(f"gemm swiglu backward column sums {M}x{N}x{K} per {per}")
+    _announce(f"gemm swiglu backward column sums {M}x{N}x{K} per {per} {dtype}")
     ops = _ops()
     from mi355_vit import _lib as E
 
-    dy, w = _rand((M, K), torch.bfloat16, 0).to(DEV), _rand((K, N), torch.bfloat16, 1, K**-0.5).to(DEV)
-    gu = _rand((M, 2 * N + 16), torch.bfloat16, 2).to(DEV)[:, : 2 * N + 8]
-    out = torch.full((M, 2 * N + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    dy, w = _rand((M, K), dtype, 0).to(DEV), _rand((K, N), dtype, 1, K**-0.5).to(DEV)
+    gu = _rand((M, 2 * N + 16), dtype, 2).to(DEV)[:, : 2 * N + 8]
+    out = torch.full((M, 2 * N + 8), 7.0, dtype=dtype, device=DEV)
     part = torch.full((-(-M // per), 2 * N + 8), 7.0, device=DEV)
     ops.gemm(dy, w, out, trans_b=True, epilogue=E.EPI_SWIGLU_BWD, residual=gu, aux_off=N + 8, colsum_partial=part)
     dh, g, u = dy.double() @ w.double(), gu[:, :N].double(), gu[:, N + 8 :].double()
