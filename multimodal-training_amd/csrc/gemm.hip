@@ -1166,11 +1166,16 @@ bool pp_takes(GemmTiledKind kind, int64_t k_chunk, int64_t k_last) {  // at leas
 // step of 64 along K takes 1.15 us in a 256 x 256 tile (one work-group per compute unit; 1.2 with both operands behind the
 // transposing LDS read; 2,435 cycles, so more when the clock falls under a long load, which lengthens every tile's steps alike), and in the smaller ones `one` us while every unit has at most one work-group and `two` us once it has
 // two.  A fuller last round, a shorter step and more units at work all lower the estimate; the epilogue of a 256 x 256 tile is
-// the longest.  The line between the tiles follows from these numbers and not from any shape: e.g. input gradients of 1280
-// columns, K = 3840, are fastest on 64 x 64 up to 1,500 rows, on 64 x 128 to 3,100, on 128 x 128 to 6,500 and on 256 x 256 at
-// 8,192 (us at 256 / 1,024 / 2,048 / 4,096 / 8,192 rows: 19 / 26 / 35 / 47 / 80, with 256 x 256 tiles alone 69 / 69 / 69 / 70 / 80);
-// weight gradients of 3840 x 1280 over 4,096 rows take 49 us in one slice on 128 x 128 and 57 in three on 256 x 256, over 8,192
-// rows 93 and 87.
+// the longest.  The line between the tiles follows from these numbers and not from any shape: e.g. weight gradients of
+// 3840 x 1280 over 4,096 rows take 49 us in one slice on 128 x 128 and 57 in three on 256 x 256, over 8,192 rows 93 and 87.
+//
+// What a launch costs is its time alone only where nothing runs beside it.  In the backward the input gradients and the weight
+// gradients run on two streams, and the units that one launch's last round leaves idle work for the other: there the estimate is
+// a mean of the time alone (weight `alone`) and of the units' time divided by the number of units, which favours the tile that
+// wastes least over the one that ends its rounds best.  us per 32-block step, tiles by time alone -> by this mean: 14,336 rows
+// 69.6 -> 67.5 ms, 16,384 (checkpointed, optimizer included) 102.9 -> 98.5, 9,600 50.2 -> 49.2 (weight gradients 1.0 of it), 4,096
+// and 20,000 unchanged; weights of 0.25 ... 0.6 (input gradients) and 0.3 ... 0.7 (weight gradients) lie within 1 % of each other.
+constexpr double PP_STEP_US = 1.15, PP_TILE_US = 7., PP_SWIGLU_TILE_US = 11.;
 struct TileChoice {
   int bm, bn;
   double us;
@@ -1180,16 +1185,19 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
   const bool tt = kind == TT_NONE || kind == TT_NONE_F32;
   const double steps = (double)((k_chunk + 63) / 64);
   const int64_t n_mul = kind == NN_SWIGLU ? 2 : 1;
+  const double alone = tt ? 0.5 : (kind == NT_NONE || kind == NT_GELU_BWD ? 0.3 : 1.);
   TileChoice best{0, 0, 1e30};
   auto consider = [&](int bm, int bn, double one, double two, double per_tile) {
     const int64_t items = ((M + bm - 1) / bm) * ((N * n_mul + bn - 1) / bn) * slices;
     const int64_t slots = two > 0. ? 2 * (int64_t)n_cu : n_cu, full = items / slots, rest = items % slots;
-    double us = 4. + full * (steps * (two > 0. ? two : one) + per_tile);
+    const double round = steps * (two > 0. ? two : one) + per_tile;
+    double us = full * round;
     if (rest > 0) us += steps * (two > 0. && rest > n_cu ? two : one) + per_tile;
+    us = 4. + alone * us + (1. - alone) * round * (double)items / (double)slots;
     if (us < best.us) best = TileChoice{bm, bn, us};
   };
   const bool swiglu = kind == NN_SWIGLU;
-  if (pp_takes(kind, k_chunk, k_last)) consider(256, 256, tt ? 1.2 : 1.15, 0., swiglu ? 11. : 7.);
+  if (pp_takes(kind, k_chunk, k_last)) consider(256, 256, tt ? 1.2 : PP_STEP_US, 0., swiglu ? PP_SWIGLU_TILE_US : PP_TILE_US);
   if (kind == NT_SWIGLU_BWD) {  // two inputs, two outputs and the column sums lengthen its epilogue
     consider(64, 64, 0.30, 0.43, 2.);
     consider(64, 128, 0.47, 0.70, 2.);
@@ -1207,6 +1215,19 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
   // 256-row tiles end in a bad round: 4,864 rows 91 / 76 / 105, 10,240: 182 / 142 / 164)
   if (kind == NT_SWIGLU_BWD && full_rows && 2 * ((M + 255) / 256) * ((N + 255) / 256) >= n_cu) best = TileChoice{0, 0, 0.};
   return best;
+}
+
+// Rows of a forward product that fill whole rounds of 256 x 256 tiles, when the rest is better taken by a second launch of the
+// tiles that suit it (0: one launch for all).  14,336 rows are 56 x 5 tiles of 1280 columns, 1.09 rounds of 256 units: a second
+// round for 24 tiles, or 2.2 rounds of 128 x 128 tiles at two thirds of the rate.  255 tiles in one round and 1,280 rows on small
+// tiles are faster than either (forward products of the tower, time alone of the step: 14,336 rows 71.6 -> 69.6 ms, 9,600 51.7 ->
+// 50.2, 4,360 without gradients 8.92 -> 8.61).  In the backward the second stream fills the last round, see choose_tile.
+int64_t rows_in_full_rounds(GemmTiledKind kind, int64_t M, int64_t N, int64_t K, int n_cu) {
+  if (!(kind == NN_NONE || kind == NN_BIAS || kind == NN_BIAS_RES || kind == NN_BIAS_GELU || kind == NN_SWIGLU) || !pp_takes(kind, K, K)) return 0;
+  const int64_t tn = (N * (kind == NN_SWIGLU ? 2 : 1) + 255) / 256, rounds = (M + 255) / 256 * tn / n_cu, rows = rounds * n_cu / tn * 256;
+  if (rows == 0 || rows >= M) return 0;
+  const double head = 4. + (double)rounds * ((double)((K + 63) / 64) * PP_STEP_US + (kind == NN_SWIGLU ? PP_SWIGLU_TILE_US : PP_TILE_US));
+  return head + choose_tile(kind, M - rows, N, K, K, 1, n_cu).us + 1. < choose_tile(kind, M, N, K, K, 1, n_cu).us ? rows : 0;
 }
 
 // packed[n][line * 48 + b] = w[n][channel * 392 + frame * 196 + y * 14 + x] for b = x * 3 + channel < 42, else 0
@@ -1366,16 +1387,32 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
     if (dev < 0) return MVIT_ERR_LAUNCH;
     const int n_cu = device_cu_count(dev);
     TileChoice c = choose_tile(kind, p.M, p.N, p.k_chunk, p.K - (p.split_k - 1) * p.k_chunk, p.split_k, n_cu);
-    if (getenv("MVIT_GEMM_NO_HALF_TILES") != nullptr && c.bm != 256 && pp_takes(kind, p.k_chunk, p.K - (p.split_k - 1) * p.k_chunk)) c = TileChoice{256, 256, 0.};
+    const bool all_256 = getenv("MVIT_GEMM_NO_HALF_TILES") != nullptr;
+    if (all_256 && c.bm != 256 && pp_takes(kind, p.k_chunk, p.K - (p.split_k - 1) * p.k_chunk)) c = TileChoice{256, 256, 0.};
     // the column sums are per tile row: their granularity names the kernel (64 rows: 64 x 64 or 64 x 128 tiles, below)
     if (kind == NT_SWIGLU_BWD && p.colsum != nullptr) c = colsum_rows == 64 ? choose_tile(kind, p.M, p.N, p.k_chunk, p.K, 1, n_cu, false) : TileChoice{0, 0, 0.};
     if (c.bm != 0) {
-      p.tiles_m = (int)((p.M + c.bm - 1) / c.bm);
-      const int n_cols = kind == NN_SWIGLU ? c.bn / 2 : c.bn;
-      p.tiles_n = (int)((p.N + n_cols - 1) / n_cols);
-      MVIT_REQUIRE((int64_t)p.tiles_m * p.tiles_n * p.split_k < (1ll << 30), "gemm: too many tiles");
-      p.panel_w = p.tiles_n <= 6 ? p.tiles_n : 4;
-      const int rc = c.bm == 256 ? mvit_gemm_pp(kind, p, n_cu, s) : mvit_gemm_small(kind, c.bm, c.bn, p, s);
+      auto run = [&](GemmParams q, const TileChoice& t) -> int {
+        q.tiles_m = (int)((q.M + t.bm - 1) / t.bm);
+        const int n_cols = kind == NN_SWIGLU ? t.bn / 2 : t.bn;
+        q.tiles_n = (int)((q.N + n_cols - 1) / n_cols);
+        MVIT_REQUIRE((int64_t)q.tiles_m * q.tiles_n * q.split_k < (1ll << 30), "gemm: too many tiles");
+        q.panel_w = q.tiles_n <= 6 ? q.tiles_n : 4;
+        return t.bm == 256 ? mvit_gemm_pp(kind, q, n_cu, s) : mvit_gemm_small(kind, t.bm, t.bn, q, s);
+      };
+      const int64_t head = all_256 || p.split_k > 1 ? 0 : rows_in_full_rounds(kind, p.M, p.N, p.K, n_cu);
+      if (head > 0) {  // a row's result does not depend on the tile that computes it
+        GemmParams q = p;
+        q.M = head;
+        if (int rc = run(q, TileChoice{256, 256, 0.})) return rc;
+        q.M = p.M - head;
+        q.A = static_cast<const bf16_t*>(p.A) + head * p.lda;
+        q.C = static_cast<bf16_t*>(p.C) + head * p.ldc;
+        if (p.R) q.R = static_cast<const bf16_t*>(p.R) + head * p.ldr;
+        if (p.aux) q.aux = static_cast<bf16_t*>(p.aux) + head * p.ldaux;
+        return run(q, choose_tile(kind, q.M, q.N, q.K, q.K, 1, n_cu));
+      }
+      const int rc = run(p, c);
       if (rc != MVIT_OK) return rc;
       if (p.split_k > 1) {
         if (kind == TT_NONE_F32) launch_splitk_reduce<bf16_t, float>(p, s);

@@ -408,6 +408,39 @@ def test_gemm_half_height_tiles_give_the_same_bits_as_full_tiles(M, K, monkeypat
     assert max_rel_err(dgrad_half, a.cpu().double() @ w.cpu().double()) < TOL[dtype]
 
 
+@pytest.mark.parametrize("epi", ["none", "bias", "bias_res", "gelu", "swiglu", "swiglu without aux"])
+@pytest.mark.parametrize("M,N", [(4353, 3840), (4607, 3840), (13057, 1280), (14336, 1280)])
+def test_gemm_rows_in_full_rounds_and_the_rest_give_the_same_bits_as_one_launch(M, N, epi, monkeypatch):
+    """Forward products whose 256 x 256 tiles end in a nearly empty round go in two launches, the rows of the full rounds and
+    the rest (one row, part of a tile, several tiles): every output has the bits of one launch, and nothing else is written."""
+    _announce(f"gemm rows in full rounds M={M} N={N} {epi}")
+    ops = _ops()
+    from mi355_vit import _lib as E
+
+    K, dtype = 1280, torch.bfloat16
+    if epi.startswith("swiglu"):
+        N //= 2
+    a, b, b2 = (_rand(s, dtype, i, sc).to(DEV) for i, (s, sc) in enumerate((((M, K), 1.0), ((N, K), K**-0.5), ((N, K), K**-0.5))))
+    bias, bias2, res = _rand((N,), dtype, 3).to(DEV), _rand((N,), dtype, 4).to(DEV), _rand((M, N), dtype, 5).to(DEV)
+    kw = {"none": {}, "bias": dict(epilogue=E.EPI_BIAS, bias=bias), "bias_res": dict(epilogue=E.EPI_BIAS_RES, bias=bias, residual=res),
+          "gelu": dict(epilogue=E.EPI_BIAS_GELU, bias=bias)}.get(epi, dict(epilogue=E.EPI_SWIGLU, b2=b2, bias=bias, bias2=bias2))
+
+    def run():
+        out, aux = torch.full((M + 8, N), 7.0, dtype=dtype, device=DEV), torch.full((M + 8, 2 * N), 7.0, dtype=dtype, device=DEV)
+        more = dict(aux=aux[:M, :N]) if epi == "gelu" else dict(aux=aux[:M], aux_off=N) if epi == "swiglu" else {}
+        ops.gemm(a, b, out[:M], **kw, **more)
+        return out, aux
+
+    split = run()
+    monkeypatch.setenv("MVIT_GEMM_NO_HALF_TILES", "1")
+    whole = run()
+    assert all(torch.equal(x, y) for x, y in zip(split, whole))
+    assert bool((split[0][M:] == 7.0).all()) and bool((split[1][M:] == 7.0).all())
+    if epi in ("none", "bias"):
+        want = a.cpu().double() @ b.cpu().double().T + (bias.cpu().double() if epi == "bias" else 0.0)
+        assert max_rel_err(split[0][:M], want) < TOL[dtype]
+
+
 @pytest.mark.parametrize("dtype,odt", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32)])
 @pytest.mark.parametrize("S,No,Ni", [(1000, 1280, 1280), (515, 3840, 256), (70, 6848, 1280), (2052, 1280, 3420)])
 def test_gemm_wgrad_layout(dtype, odt, S, No, Ni):
