@@ -15,9 +15,10 @@
 // passed a barrier behind those reads.  Before the barrier of phase P each wave waits until its own loads of n <= P + 2
 // have landed: at most four half tiles (eight loads) may still be in flight, fewer at the end of K.
 //
-// The products are computed transposed (B's fragment is the MFMA's first operand) with B's columns dealt so that a lane
-// ends up with eight consecutive columns of one row: results leave the registers as 16-byte vectors with no LDS staging and
-// no barrier, and the next tile's first loads run under them.  K order and MFMA form are the same for every tile shape of
+// The products are computed transposed (B's fragment is the MFMA's first operand) so that a lane ends up with eight consecutive
+// columns of one row: by the way a row-major B's columns are dealt to the fragments, or, where the fragments come through the
+// transposing read, by a lane exchange in the epilogue (tr_columns): results leave the registers as 16-byte vectors with no LDS
+// staging and no barrier, and the next tile's first loads run under them.  K order and MFMA form are the same for every tile shape of
 // this file, so a result does not depend on the shape that computed it.
 //
 // LDS layouts (a direct load writes 1 KiB of contiguous LDS per instruction; the lanes choose which 16 bytes they fetch):
@@ -69,13 +70,16 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
 
   // ---- fragment addresses (stage 0, half 0)
   const int i16 = l & 15, g4 = l >> 4;
+  // a transposing read takes 16 consecutive columns (32 bytes) of four k-rows per 16 lanes; this swizzle spreads the sixteen k-rows
+  // of a wave's instruction over all 256 bytes of the banks
+  auto tr_swizzle = [](int k) { return ((k & 3) << 1) | (((k >> 3) & 1) << 3); };
   unsigned ra[TA ? 4 : 2], rb[2];
   if constexpr (!TA) {
     const int row = wm * 64 + i16;
     ra[0] = row * 128 + ((g4 ^ ((i16 >> 1) & 7)) << 4);
     ra[1] = row * 128 + (((4 + g4) ^ ((i16 >> 1) & 7)) << 4);
   } else {
-    const int k = 8 * g4 + (i16 >> 2), sw = ((k & 3) << 1) | (((k >> 3) & 1) << 3);
+    const int k = 8 * g4 + (i16 >> 2), sw = tr_swizzle(k);
 #pragma unroll
     for (int a = 0; a < 4; ++a) ra[a] = k * 256 + (((wm * 8 + a * 2 + ((i16 & 3) >> 1)) ^ sw) << 4) + (i16 & 1) * 8;
   }
@@ -84,9 +88,9 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
     rb[0] = 2 * HALF + row * 128 + ((g4 ^ f) << 4);
     rb[1] = 2 * HALF + row * 128 + (((4 + g4) ^ f) << 4);
   } else {
-    const int k = 8 * g4 + (i16 >> 2);
-    rb[0] = 2 * HALF + k * 256 + (((wn * 4 + (i16 & 3)) ^ ((k & 3) << 2)) << 4);
-    rb[1] = rb[0] + 8;
+    const int k = 8 * g4 + (i16 >> 2), sw = tr_swizzle(k);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) rb[b] = 2 * HALF + k * 256 + (((wn * 4 + b * 2 + ((i16 & 3) >> 1)) ^ sw) << 4) + (i16 & 1) * 8;
   }
   unsigned st = 0;  // byte offset of the stage being consumed
   auto read_a = [&](bf16x8 (&f)[4][2], int half) {
@@ -151,7 +155,7 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
           va[h][j] = (unsigned)((r * p.lda + c * 8) * 2);
         } else {
           const int k = q * 4 + (l >> 4);
-          int r = h * 128 + (((l & 15) ^ (((k & 3) << 1) | (((k >> 3) & 1) << 3))) << 3);
+          int r = h * 128 + (((l & 15) ^ tr_swizzle(k)) << 3);
           if (r >= m_left) r = 0;
           va[h][j] = (unsigned)((k * p.lda + r) * 2);
         }
@@ -162,7 +166,7 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
           vb[h][j] = (unsigned)((r * p.ldb + c * 8) * 2);
         } else {
           const int k = q * 4 + (l >> 4);
-          int r = h * 128 + (((l & 15) ^ ((k & 3) << 2)) << 3);
+          int r = h * 128 + (((l & 15) ^ tr_swizzle(k)) << 3);
           if (r >= n_left) r = 0;
           vb[h][j] = (unsigned)((k * p.ldb + r) * 2);
         }
@@ -330,7 +334,7 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
     const int64_t m_lane = m0 + wm * 64 + i16;
     int64_t n_lane[2];
 #pragma unroll
-    for (int g = 0; g < 2; ++g) n_lane[g] = n0 + (DUAL ? wn * 32 : (TB ? g * 128 + wn * 32 : wn * 64 + g * 32)) + 8 * g4;
+    for (int g = 0; g < 2; ++g) n_lane[g] = TB ? n0 + g * 128 + wn * 32 + tr_first_column(g4) : n0 + (DUAL ? wn * 32 : wn * 64 + g * 32) + 8 * g4;
     float hb[2][8];
     if constexpr (HAS_BIAS) {
       const unsigned char* bl = smem_raw + PpCfg::BIAS_OFF + bias_now * 2048 + wv * 256;
@@ -347,6 +351,7 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
       for (int e = 0; e < 4; ++e) {
         v[e] = acc[a][2 * g][e];
         v[4 + e] = acc[a][2 * g + 1][e];
+        if (TB) tr_columns(v[e], v[4 + e]);
         if (DUAL) {
           u[e] = acc[a][2][e];
           u[4 + e] = acc[a][3][e];

@@ -28,8 +28,8 @@ struct SmallCfg {
 template <bool TR, bool IS_A, int ROWS>
 __device__ __forceinline__ int small_swizzle(int major) {
   if (!TR) return IS_A ? (major >> 1) & 7 : ((major >> 1) & 1) | (((major >> 3) & 3) << 1);
-  if (ROWS == 64) return IS_A ? (((major >> 1) & 1) << 1) | (((major >> 3) & 1) << 2) : ((major >> 1) & 1) << 2;
-  return IS_A ? ((major & 3) << 1) | (((major >> 3) & 1) << 3) : (major & 3) << 2;
+  if (ROWS == 64) return (((major >> 1) & 1) << 1) | (((major >> 3) & 1) << 2);
+  return ((major & 3) << 1) | (((major >> 3) & 1) << 3);
 }
 
 template <typename TO, bool TA, bool TB, int EPI, typename S>
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(cons
   } else {
     const int k = 8 * g4 + (i16 >> 2), sw = small_swizzle<TB, false, BN>(k);
 #pragma unroll
-    for (int b = 0; b < 2 * NGB; ++b) rb[b] = S::A_BYTES + k * (BN * 2) + ((((wn * S::WN + (b >> 1) * 32) / 8 + (i16 & 3)) ^ sw) << 4) + (b & 1) * 8;
+    for (int b = 0; b < 2 * NGB; ++b) rb[b] = S::A_BYTES + k * (BN * 2) + ((((wn * S::WN + b * 16) / 8 + ((i16 & 3) >> 1)) ^ sw) << 4) + (i16 & 1) * 8;
   }
 
   // ---- epilogue inputs of this lane: row l % 16 of each row block, columns 8 * (l / 16) .. of each 32-column group
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(cons
   const bool interior = vec && m0 + BM <= p.M && n0 + NCOLS <= p.N;
   int64_t n_lane[NG];
 #pragma unroll
-  for (int g = 0; g < NG; ++g) n_lane[g] = n0 + (DUAL ? wn * 32 : wn * S::WN + g * 32) + 8 * g4;
+  for (int g = 0; g < NG; ++g) n_lane[g] = n0 + (DUAL ? wn * 32 : wn * S::WN + g * 32) + (TB ? tr_first_column(g4) : 8 * g4);
   auto row_of = [&](int it) { return m0 + wm * S::WM + (it / NG) * 16 + i16; };
   constexpr int NLOAD = EPI == MVIT_EPI_SWIGLU_BWD ? 2 : 1;
   [[maybe_unused]] bf16x8 pre[HAS_IN ? ITEMS : 1][NLOAD];
@@ -270,6 +270,7 @@ __global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(cons
     for (int e = 0; e < 4; ++e) {
       v[e] = acc[a][2 * g][e];
       v[4 + e] = acc[a][2 * g + 1][e];
+      if (TB) tr_columns(v[e], v[4 + e]);
       if (DUAL) {
         u[e] = acc[a][NB - 2][e];
         u[4 + e] = acc[a][NB - 1][e];
