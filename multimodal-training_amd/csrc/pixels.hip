@@ -40,6 +40,7 @@ __device__ __forceinline__ void store4(bf16_t* dst, const float (&v)[4]) {
   *reinterpret_cast<bf16x4*>(dst) = bf16x4{from_f32<bf16_t>(v[0]), from_f32<bf16_t>(v[1]), from_f32<bf16_t>(v[2]), from_f32<bf16_t>(v[3])};
 }
 
+constexpr int PATCHIFY_GROUPS = 2048;  // eight per compute unit, as many as its waves allow
 constexpr int SQ = 2 * PATCH;          // a merge block is a square of 28 x 28 pixels
 constexpr int SQ_LINE = SQ * 3;        // 84 bytes (21 dwords) per line of the square
 constexpr int SQ_DWORDS = SQ * SQ_LINE / 4;  // 588
@@ -50,7 +51,7 @@ struct TableArg {
   mvit_image im[TABLE_ARG_IMAGES + 1];
 };
 template <typename TO>
-__device__ __forceinline__ void patchify_block(const mvit_image* images, int n_images, TO* __restrict__ out, int64_t total_rows, const Norm& nm) {
+__device__ __forceinline__ void patchify_blocks(const mvit_image* images, int n_images, TO* __restrict__ out, int64_t total_rows, const Norm& nm) {
 #pragma clang fp contract(off)
   // a byte has 256 values: the work-group computes the result for each of them and each channel once (exact
   // arithmetic, three divisions per thread) and every element of its rows is then a byte read and a table lookup
@@ -61,63 +62,67 @@ __device__ __forceinline__ void patchify_block(const mvit_image* images, int n_i
     const float x = (float)((double)(int)threadIdx.x * nm.rescale);
     lut[c][threadIdx.x] = (x - nm.mean[c]) / nm.std[c];
   }
-  // everything up to the barrier is the same for the whole work-group: its four rows are one merge block
-  const int64_t row0 = (int64_t)blockIdx.x * 4;
-  const mvit_image im = images[find_image(images, n_images, row0)];
-  const int gh = im.height / PATCH, gw = im.width / PATCH;
-  const int per_t = gh * gw;
-  const int64_t local = (row0 - im.first_row) & ~(int64_t)3;
-  bool ok = row0 < total_rows && im.frames > 0 && gh > 0 && gw > 0 && !((gh | gw) & 1);  // malformed entry: nothing is read
-  const int t = ok ? (int)(local / per_t) : 0, rem = ok ? (int)(local % per_t) : 0;
-  ok = ok && t * TPS < im.frames;  // first_row entries that promise more rows than the frames give
-  // rem = ((block row * (gw / 2) + block column) * 2 + row in block) * 2 + column in block
-  const int blk = rem >> 2, hb = ok ? blk / (gw >> 1) : 0, wb = ok ? blk % (gw >> 1) : 0;
-  const int64_t line = (int64_t)im.width * 3, frame_bytes = line * im.height;
-  const int f0 = t * TPS, f1 = f0 + 1 < im.frames ? f0 + 1 : im.frames - 1;  // the last frame fills an odd count up
-  if (ok) {
-    const int nf = f1 != f0 ? 2 : 1;
-    const uint8_t* corner = im.pixels + (int64_t)hb * SQ * line + wb * SQ_LINE;  // of the square in frame 0
-    // width is a multiple of 28, so lines are a multiple of 84 bytes: with a 4-byte aligned frame buffer every
-    // line of the square is 21 aligned dwords
-    if ((reinterpret_cast<uintptr_t>(im.pixels) & 3u) == 0) {
-      for (int i = threadIdx.x; i < nf * SQ_DWORDS; i += 256) {
-        const int fi = i / SQ_DWORDS, j = i % SQ_DWORDS, y = j / (SQ_LINE / 4), xw = j % (SQ_LINE / 4);
-        square[fi][j] = *reinterpret_cast<const uint32_t*>(corner + (fi ? f1 : f0) * frame_bytes + y * line + xw * 4);
-      }
-    } else {
-      uint8_t* sq8 = reinterpret_cast<uint8_t*>(&square[0][0]);
-      for (int i = threadIdx.x; i < nf * SQ_DWORDS * 4; i += 256) {
-        const int fi = i / (SQ_DWORDS * 4), j = i % (SQ_DWORDS * 4), y = j / SQ_LINE, xb = j % SQ_LINE;
-        sq8[i] = corner[(fi ? f1 : f0) * frame_bytes + y * line + xb];
+  // merge blocks blockIdx.x, blockIdx.x + gridDim.x, ...: the table above is made once for all of them
+  for (int64_t row0 = (int64_t)blockIdx.x * 4; row0 < total_rows; row0 += (int64_t)gridDim.x * 4) {
+    __syncthreads();  // the table is complete; the previous block's pixels have been read
+    // everything up to the barrier is the same for the whole work-group: its four rows are one merge block
+    const mvit_image im = images[find_image(images, n_images, row0)];
+    const int gh = im.height / PATCH, gw = im.width / PATCH;
+    const int per_t = gh * gw;
+    const int64_t local = (row0 - im.first_row) & ~(int64_t)3;
+    bool ok = row0 < total_rows && im.frames > 0 && gh > 0 && gw > 0 && !((gh | gw) & 1);  // malformed entry: nothing is read
+    const int t = ok ? (int)(local / per_t) : 0, rem = ok ? (int)(local % per_t) : 0;
+    ok = ok && t * TPS < im.frames;  // first_row entries that promise more rows than the frames give
+    // rem = ((block row * (gw / 2) + block column) * 2 + row in block) * 2 + column in block
+    const int blk = rem >> 2, hb = ok ? blk / (gw >> 1) : 0, wb = ok ? blk % (gw >> 1) : 0;
+    const int64_t line = (int64_t)im.width * 3, frame_bytes = line * im.height;
+    const int f0 = t * TPS, f1 = f0 + 1 < im.frames ? f0 + 1 : im.frames - 1;  // the last frame fills an odd count up
+    if (ok) {
+      const int nf = f1 != f0 ? 2 : 1;
+      const uint8_t* corner = im.pixels + (int64_t)hb * SQ * line + wb * SQ_LINE;  // of the square in frame 0
+      // width is a multiple of 28, so lines are a multiple of 84 bytes: with a 4-byte aligned frame buffer every
+      // line of the square is 21 aligned dwords
+      if ((reinterpret_cast<uintptr_t>(im.pixels) & 3u) == 0) {
+        for (int i = threadIdx.x; i < nf * SQ_DWORDS; i += 256) {
+          const int fi = i / SQ_DWORDS, j = i % SQ_DWORDS, y = j / (SQ_LINE / 4), xw = j % (SQ_LINE / 4);
+          square[fi][j] = *reinterpret_cast<const uint32_t*>(corner + (fi ? f1 : f0) * frame_bytes + y * line + xw * 4);
+        }
+      } else {
+        uint8_t* sq8 = reinterpret_cast<uint8_t*>(&square[0][0]);
+        for (int i = threadIdx.x; i < nf * SQ_DWORDS * 4; i += 256) {
+          const int fi = i / (SQ_DWORDS * 4), j = i % (SQ_DWORDS * 4), y = j / SQ_LINE, xb = j % SQ_LINE;
+          sq8[i] = corner[(fi ? f1 : f0) * frame_bytes + y * line + xb];
+        }
       }
     }
-  }
-  __syncthreads();
-  if (!ok) return;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const uint8_t* p0 = reinterpret_cast<const uint8_t*>(&square[0][0]) + (wave >> 1) * PATCH * SQ_LINE + (wave & 1) * PATCH * 3;
-  const uint8_t* p1 = f1 != f0 ? p0 + SQ_DWORDS * 4 : p0;
-  TO* dst = out + (row0 + wave) * ROW;
-  for (int g = lane; g < 3 * QUADS; g += 64) {
-    const int c = g / QUADS, q = g % QUADS;
-    float v0[4], v1[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int p = 4 * q + e, off = (p / PATCH) * SQ_LINE + (p % PATCH) * 3 + c;
-      v0[e] = lut[c][p0[off]];
-      v1[e] = lut[c][p1[off]];
+    __syncthreads();
+    if (!ok) continue;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint8_t* p0 = reinterpret_cast<const uint8_t*>(&square[0][0]) + (wave >> 1) * PATCH * SQ_LINE + (wave & 1) * PATCH * 3;
+    TO* dst = out + (row0 + wave) * ROW;
+    const bool two = f1 != f0;  // a still image's one frame fills both halves: looked up once (vector issue bounds these loops)
+    for (int g = lane; g < 3 * QUADS; g += 64) {
+      const int c = g / QUADS, q = g % QUADS, y = 4 * q / PATCH, x = 4 * q - y * PATCH;
+      const uint8_t* at = p0 + y * SQ_LINE + x * 3 + c;
+      float v[4];
+      auto look_up = [&](const uint8_t* p) {
+  #pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = lut[c][p[3 * e + (x + e >= PATCH ? SQ_LINE - PATCH * 3 : 0)]];
+      };
+      look_up(at);
+      store4(dst + (c * TPS + 0) * PLANE + 4 * q, v);
+      if (two) look_up(at + SQ_DWORDS * 4);
+      store4(dst + (c * TPS + 1) * PLANE + 4 * q, v);
     }
-    store4(dst + (c * TPS + 0) * PLANE + 4 * q, v0);
-    store4(dst + (c * TPS + 1) * PLANE + 4 * q, v1);
   }
 }
 template <typename TO>
 __global__ __launch_bounds__(256) void patchify_kernel(const mvit_image* __restrict__ images, int n_images, TO* __restrict__ out, int64_t total_rows, Norm nm) {
-  patchify_block<TO>(images, n_images, out, total_rows, nm);
+  patchify_blocks<TO>(images, n_images, out, total_rows, nm);
 }
 template <typename TO>
 __global__ __launch_bounds__(256) void patchify_arg_kernel(const TableArg images, int n_images, TO* __restrict__ out, int64_t total_rows, Norm nm) {
-  patchify_block<TO>(images.im, n_images, out, total_rows, nm);
+  patchify_blocks<TO>(images.im, n_images, out, total_rows, nm);
 }
 
 }  // namespace
@@ -193,7 +198,7 @@ __global__ __launch_bounds__(256) void resample_pass_kernel(const uint8_t* __res
 // ---- several passes in one launch
 constexpr int RESAMPLE_MAX_JOBS = 32;
 struct ResampleJobs {
-  int n;
+  int n, rows_per_wave;  // the latter of resample_narrow_lds_kernel
   int first_block[RESAMPLE_MAX_JOBS];
   mvit_resample_job job[RESAMPLE_MAX_JOBS];
 };
@@ -294,6 +299,197 @@ __global__ __launch_bounds__(256) void resample_narrow_kernel(const ResampleJobs
   }
 }
 
+// The same pass where a wave's 64 windows span at most NARROW_SPAN bytes of a row (three channels shrunk up to fivefold) and have
+// at most NARROW_TAPS taps.  Those bytes (the windows overlap) come in one coalesced 16-byte load per lane and row, through a
+// piece of LDS of the wave's own, so there is no barrier; a thread then reads its window as aligned words and shifts it into
+// place.  Windows loaded from memory, 16 unaligned bytes per lane, keep the address units busy (75 % of the time, one access per
+// lane).  Four taps of a channel are one 8-bit dot product per digit: a weight is three signed digits of 8 bits, a pixel is taken
+// less 128 (one exclusive or on the way into LDS), and 128 times the sum of the weights is added back.  Whole numbers modulo 2^32
+// throughout, so the sums are those of plain multiply-adds.  us by the kernel above / this one: four photographs of 1,080 x 1,920 ...
+// 2,448 x 3,264 to 0.8 million pixels each 42.6 / 28.1, 4,480 x 4,480 to 3,584 x 3,584 124 / 57, 480 x 640 to 0.2 million 11.0 / 8.7;
+// what bounds it now is vector issue (a row of 64 outputs: 63 instructions at 8 taps, 99 at 16, and 18 to store it).
+constexpr int NARROW_SPAN = 1024, NARROW_TAPS = 24, NARROW_BATCH = 2, NARROW_SLACK = NARROW_TAPS * RESAMPLE_MAX_CHANNELS + 16;  // a window's padding reads past its row
+__device__ __forceinline__ bool fits_digits(int k) { return k <= 0x7f7f7f && k >= -0x808080; }
+// bytes first, first + step, first + 2 step, first + 3 step of the consecutive words w
+template <int STEP, int N>
+__device__ __forceinline__ unsigned gather_bytes(const unsigned (&w)[N], int first) {
+  if constexpr (STEP == 1) {
+    return w[first / 4];
+  } else {
+    auto pair = [&](int i, int j) {  // bytes i and j in the lower half
+      const int lo = i / 4, hi = j / 4;
+      return __builtin_amdgcn_perm(w[hi], w[lo], 0x0c0c0000u | (unsigned)((j % 4 + 4) << 8) | (unsigned)(i % 4));
+    };
+    if (first / 4 + 1 >= (first + 2 * STEP) / 4 && STEP < 4) {  // the first three lie in two neighbouring words
+      const int lo = first / 4, hi = (first + 3 * STEP) / 4, mid = (first + 2 * STEP) / 4;
+      auto sel = [&](int b) { return (unsigned)(b / 4 == lo ? b % 4 : b % 4 + 4); };
+      const unsigned three = __builtin_amdgcn_perm(w[mid], w[lo], sel(first) | sel(first + STEP) << 8 | sel(first + 2 * STEP) << 16 | 0x0c000000u);
+      return __builtin_amdgcn_perm(w[hi], three, 0x00020100u | (unsigned)((first + 3 * STEP) % 4 + 4) << 24);
+    }
+    if ((first + STEP) / 4 + 1 >= (first + 3 * STEP) / 4 && STEP < 4) {  // the last three do
+      const int lo = (first + STEP) / 4, hi = (first + 3 * STEP) / 4;
+      auto sel = [&](int b) { return (unsigned)(b / 4 == lo ? b % 4 : b % 4 + 4); };
+      const unsigned three = __builtin_amdgcn_perm(w[hi], w[lo], sel(first + STEP) << 8 | sel(first + 2 * STEP) << 16 | sel(first + 3 * STEP) << 24 | 0x0cu);
+      return __builtin_amdgcn_perm(w[first / 4], three, 0x03020100u | (unsigned)(first % 4 + 4));
+    }
+    return __builtin_amdgcn_perm(pair(first + 2 * STEP, first + 3 * STEP), pair(first, first + STEP), 0x05040100u);
+  }
+}
+// Output coordinate `x` of every staged row from GROUPS groups of four taps; at: byte offset of the window from the row's first
+// staged byte; digit: the groups' digits of the lane's weights, 64 lanes apart, and behind them the sums of the weights
+template <int INNER, int GROUPS, typename Emit>
+__device__ __forceinline__ void resample_narrow_digits(const unsigned char* lds, int at, uintptr_t start, int64_t row_in, int rows,
+                                                       const unsigned (*dig)[4][64], int lane, Emit emit) {
+  unsigned digit[GROUPS][3], total = 0;
+#pragma unroll
+  for (int g = 0; g < GROUPS; ++g) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) digit[g][d] = dig[g][d][lane];
+    total += dig[g][3][lane];
+  }
+  total = total * 128 + (1u << (RESAMPLE_PRECISION_BITS - 1));
+#pragma unroll 2
+  for (int r = 0; r < rows; ++r) {
+    const int b = r * NARROW_SPAN + at + (int)((start + r * row_in) & 15);
+    const unsigned* q = reinterpret_cast<const unsigned*>(lds + (b & ~3));
+    unsigned raw[GROUPS * INNER + 1], w[GROUPS * INNER];
+#pragma unroll
+    for (int i = 0; i <= GROUPS * INNER; ++i) raw[i] = q[i];
+#pragma unroll
+    for (int i = 0; i < GROUPS * INNER; ++i) w[i] = __builtin_amdgcn_alignbyte(raw[i + 1], raw[i], b);
+    unsigned out[INNER];
+#pragma unroll
+    for (int c = 0; c < INNER; ++c) {
+      int sum[3] = {(int)total, 0, 0};
+#pragma unroll
+      for (int g = 0; g < GROUPS; ++g) {
+        const unsigned four = gather_bytes<INNER>(w, g * 4 * INNER + c);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) sum[d] = __builtin_amdgcn_sdot4((int)four, (int)digit[g][d], sum[d], false);
+      }
+      out[c] = clip8((int)((unsigned)sum[0] + ((unsigned)sum[1] << 8) + ((unsigned)sum[2] << 16)));
+    }
+    emit(r, out);
+  }
+}
+template <int INNER>
+__global__ __launch_bounds__(256, 5) void resample_narrow_lds_kernel(const ResampleJobs jobs) {
+  const int j = resample_job_of(jobs, blockIdx.x);
+  const mvit_resample_job& jb = jobs.job[j];
+  const int block = blockIdx.x - jobs.first_block[j], lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int in_len = (int)jb.in_len, out_len = (int)jb.out_len, ksize = jb.ksize;
+  const int xblocks = (out_len + 63) / 64, xb = block % xblocks;
+  const bool mine = xb * 64 + lane < out_len;
+  const int x = mine ? xb * 64 + lane : out_len - 1;
+  const int64_t row_in = (int64_t)in_len * INNER, row_out = (int64_t)out_len * INNER;
+  const int64_t o0 = ((int64_t)(block / xblocks) * 4 + wave) * jobs.rows_per_wave;
+  const int rows = o0 >= jb.outer ? 0 : (jb.outer - o0 < jobs.rows_per_wave ? (int)(jb.outer - o0) : jobs.rows_per_wave);
+  const int32_t* __restrict__ kk = jb.kk + (int64_t)x * ksize;
+  const TapWindow tw = tap_window(jb.bounds, x, ksize, in_len);
+  // the bytes of a row from the first output's window to the last one's; windows out of that order go tap by tap
+  const int first = __builtin_amdgcn_readlane(tw.xmin, 0), last = __builtin_amdgcn_readlane(tw.xmin + tw.n, 63);
+  const int span = (last - first) * INNER;
+  bool fits = tw.xmin >= first && tw.xmin + tw.n <= last && tw.n <= NARROW_TAPS && span + 15 <= NARROW_SPAN;
+
+  __shared__ __attribute__((aligned(16))) unsigned char staged[4][NARROW_BATCH * NARROW_SPAN + NARROW_SLACK];
+  __shared__ unsigned dig[NARROW_TAPS / 4][4][64];
+  unsigned char* lds = staged[wave];
+  const uintptr_t start = reinterpret_cast<uintptr_t>(jb.src) + o0 * row_in + (int64_t)first * INNER;
+  // aligned chunks; one that sticks out of the array is filled byte by byte
+  const uintptr_t lo = reinterpret_cast<uintptr_t>(jb.src), hi = lo + jb.outer * row_in;
+  u32x4 v[NARROW_BATCH];
+  auto request = [&](int batch) {
+#pragma unroll
+    for (int r = 0; r < NARROW_BATCH; ++r) {
+      v[r] = u32x4{0u, 0u, 0u, 0u};
+      if (batch + r >= rows) continue;
+      const uintptr_t from = start + (batch + r) * row_in, chunk = (from & ~(uintptr_t)15) + 16 * lane;
+      typedef __attribute__((address_space(1))) const u32x4* global_words;
+      if (chunk >= lo && chunk + 16 <= hi && chunk < from + span) v[r] = *(global_words)chunk;
+    }
+  };
+  const bool in_lds = __all(fits);
+  if (in_lds) request(0);
+  // wave g makes the digits of tap group g (and g + 4) of the 64 outputs, for all four waves
+  for (int g = wave; g < NARROW_TAPS / 4; g += 4) {
+    unsigned d3[3] = {0u, 0u, 0u}, total = 0;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      int k = 4 * g + t < tw.n ? kk[4 * g + t] : 0;  // taps past the window have weight 0
+      fits = fits && fits_digits(k);
+      total += (unsigned)k;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        d3[d] |= (unsigned)(k & 0xff) << (8 * t);
+        k = (k + 128) >> 8;  // less the signed digit, by 256
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) dig[g][d][lane] = d3[d];
+    dig[g][3][lane] = total;
+  }
+  const bool digits = __syncthreads_and(fits) != 0;
+
+  // four pixels of three channels leave as three words, each made by one lane from its own and its neighbour's bytes
+  const bool words = INNER == 3 && out_len % 4 == 0 && (reinterpret_cast<uintptr_t>(jb.dst) & 3u) == 0;
+  auto emit = [&](uint8_t* d, const unsigned (&b)[INNER]) {  // d: output row
+    if (words) {
+      const unsigned p = b[0] | (b[INNER > 1 ? 1 : 0] << 8) | (b[INNER > 2 ? 2 : 0] << 16);
+      const unsigned next = __builtin_amdgcn_mov_dpp((int)p, 0xf9, 0xf, 0xf, false);  // of the next lane of the four
+      const int q = lane & 3;
+      if (mine && q < 3) *reinterpret_cast<unsigned*>(d + (x - q) * 3 + 4 * q) = (p >> (8 * q)) | (next << (24 - 8 * q));
+    } else if (mine) {
+#pragma unroll
+      for (int c = 0; c < INNER; ++c) d[(int64_t)x * INNER + c] = (uint8_t)b[c];
+    }
+  };
+  uint8_t* out_row = jb.dst + o0 * row_out;
+  if (!digits) {  // windows or weights that no resampling table has
+    for (int r = 0; r < rows; ++r) {
+      unsigned out[INNER];
+#pragma unroll 1
+      for (int c = 0; c < INNER; ++c) {
+        const uint8_t* p = jb.src + (o0 + r) * row_in + (int64_t)tw.xmin * INNER + c;
+        unsigned a = 1u << (RESAMPLE_PRECISION_BITS - 1);
+        for (int t = 0; t < tw.n; ++t) a += (unsigned)p[t * INNER] * (unsigned)kk[t];
+        out[c] = clip8((int)a);
+      }
+      emit(out_row + r * row_out, out);
+    }
+    return;
+  }
+  const int at = (tw.xmin - first) * INNER, groups = __any(tw.n > 16) ? 6 : __any(tw.n > 12) ? 4 : __any(tw.n > 8) ? 3 : __any(tw.n > 4) ? 2 : 1;
+  for (int batch = 0; batch < rows; batch += NARROW_BATCH) {
+    const int n = rows - batch < NARROW_BATCH ? rows - batch : NARROW_BATCH;
+    const uintptr_t row0 = start + batch * row_in;
+#pragma unroll
+    for (int r = 0; r < NARROW_BATCH; ++r) *reinterpret_cast<u32x4*>(lds + r * NARROW_SPAN + 16 * lane) = v[r] ^ 0x80808080u;  // pixels less 128
+    if ((row0 & ~(uintptr_t)15) < lo || ((row0 + (n - 1) * row_in) & ~(uintptr_t)15) + 1024 > hi) {
+#pragma unroll 1
+      for (int i = 0; i < n * 16; ++i) {
+        const uintptr_t from = row0 + (i / 16) * row_in, chunk = (from & ~(uintptr_t)15) + 16 * lane, byte = chunk + i % 16;
+        if ((chunk < lo || chunk + 16 > hi) && byte >= lo && byte < hi && byte < from + span)
+          lds[(i / 16) * NARROW_SPAN + 16 * lane + i % 16] = *reinterpret_cast<const uint8_t*>(byte) ^ 0x80u;
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    request(batch + NARROW_BATCH);  // past the wave's rows: nothing
+    uint8_t* d0 = out_row + batch * row_out;
+    auto put = [&](int r, const unsigned (&b)[INNER]) { emit(d0 + r * row_out, b); };
+    switch (groups) {
+      case 1: resample_narrow_digits<INNER, 1>(lds, at, row0, row_in, n, dig, lane, put); break;
+      case 2: resample_narrow_digits<INNER, 2>(lds, at, row0, row_in, n, dig, lane, put); break;
+      case 3: resample_narrow_digits<INNER, 3>(lds, at, row0, row_in, n, dig, lane, put); break;
+      case 4: resample_narrow_digits<INNER, 4>(lds, at, row0, row_in, n, dig, lane, put); break;
+      default: resample_narrow_digits<INNER, NARROW_TAPS / 4>(lds, at, row0, row_in, n, dig, lane, put); break;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
 // The pass for a long contiguous dimension of whole words (the vertical pass).  A wave makes 1 KiB of one output row: the window
 // and its weights are the same for all of it (scalar loads), a lane makes 16 bytes from one 16-byte load per tap.  The four waves
 // of a work-group make the same KiB of four consecutive rows, whose windows overlap and meet in the L1.  Bound by the byte
@@ -363,7 +559,7 @@ int mvit_patchify(const mvit_image* images, int n_images, int64_t total_rows, vo
   MVIT_REQUIRE(out != nullptr && mvit_aligned16(out), "patchify: output must be a 16-byte aligned device pointer");
   Norm nm{rescale, {mean_r, mean_g, mean_b}, {std_r, std_g, std_b}};
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const unsigned grid = (unsigned)(total_rows / 4);
+  const unsigned grid = (unsigned)(total_rows / 4 < PATCHIFY_GROUPS ? total_rows / 4 : PATCHIFY_GROUPS);
   if (dtype == MVIT_BF16)
     hipLaunchKernelGGL((patchify_kernel<bf16_t>), dim3(grid), 256, 0, s, images, n_images, static_cast<bf16_t*>(out), total_rows, nm);
   else
@@ -387,7 +583,7 @@ int mvit_patchify_host_table(const mvit_image* images, int n_images, int64_t tot
   memcpy(table.im, images, sizeof(mvit_image) * ((size_t)n_images + 1));
   Norm nm{rescale, {mean_r, mean_g, mean_b}, {std_r, std_g, std_b}};
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const unsigned grid = (unsigned)(total_rows / 4);
+  const unsigned grid = (unsigned)(total_rows / 4 < PATCHIFY_GROUPS ? total_rows / 4 : PATCHIFY_GROUPS);
   if (dtype == MVIT_BF16)
     hipLaunchKernelGGL((patchify_arg_kernel<bf16_t>), dim3(grid), 256, 0, s, table, n_images, static_cast<bf16_t*>(out), total_rows, nm);
   else
@@ -407,30 +603,51 @@ int mvit_resample_u8_batch(const mvit_resample_job* list, int n_jobs, mvit_strea
                  "resample_u8: axis too long");
   }
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  // Rows per wave of the short-row kernel: as many as keep 1,024 work-groups (four per compute unit) busy, up to 16, because the
+  // weights' digits are made once per work-group.  us with 4 / 8 / 16 rows: 480 x 640 to 448 x 588-like sizes 11.5 / 13.2 / 16.6,
+  // 2,448 x 3,264 and three smaller to 0.8 million pixels each 31.8 / 30.3 / 30.1, 4,480 x 4,480 to 3,584 x 3,584 69.5 / 59.6 / 56.2
+  int rows_per_wave = 4;
+  auto shared_rows = [&](int kind) -> int64_t { return kind == 5 ? 1 : kind > 5 ? 4 * rows_per_wave : 4 * RESAMPLE_ROWS; };  // of a work-group
   // work-groups for `outer` rows of the outermost axis
-  auto groups = [](int kind, const mvit_resample_job& j, int64_t outer) {
-    return kind == 5 ? outer * ((j.out_len + 3) / 4) * ((j.inner + RESAMPLE_STRIP - 1) / RESAMPLE_STRIP) : (j.out_len + 63) / 64 * ((outer + 4 * RESAMPLE_ROWS - 1) / (4 * RESAMPLE_ROWS));
+  auto groups = [&](int kind, const mvit_resample_job& j, int64_t outer) {
+    if (kind == 5) return outer * ((j.out_len + 3) / 4) * ((j.inner + RESAMPLE_STRIP - 1) / RESAMPLE_STRIP);
+    return (j.out_len + 63) / 64 * ((outer + shared_rows(kind) - 1) / shared_rows(kind));
   };
-  // jobs of one kind (wide words; 1 .. 4 bytes) share launches; 0: everything else, a launch each.  Of short rows the
+  // jobs of one kind (wide words; 1 .. 4 bytes, with or without LDS) share launches; 0: everything else, a launch each.  Of short rows the
   // wide kernel only takes so few (about 5 us) that a launch of their own would cost as much
   auto words = [](const mvit_resample_job& j) { return j.inner % 4 == 0 && reinterpret_cast<uintptr_t>(j.src) % 4 == 0 && reinterpret_cast<uintptr_t>(j.dst) % 4 == 0; };
+  // short rows through LDS (6 .. 9) where the windows of 64 outputs fit, as bounds of any resampling between these lengths do
+  auto through_lds = [](const mvit_resample_job& j) {
+    return j.ksize <= NARROW_TAPS && ((63 * j.in_len + j.out_len - 1) / j.out_len + j.ksize + 1) * j.inner + 15 <= NARROW_SPAN;
+  };
   auto kind_of = [&](const mvit_resample_job& j) {
-    if (j.inner <= RESAMPLE_MAX_CHANNELS) return (int)j.inner;
+    if (j.inner <= RESAMPLE_MAX_CHANNELS) return (int)j.inner + (through_lds(j) ? 5 : 0);
     const bool wide = j.inner >= RESAMPLE_WIDE_FROM || (j.inner >= 16 && j.outer * j.out_len <= RESAMPLE_FEW_ROWS);
     return words(j) && wide && groups(5, j, 1) <= MVIT_MAX_GROUPS_256 ? 5 : 0;
   };
-  for (int kind = 0; kind <= 5; ++kind) {
+  for (int kind = 0; kind <= 9; ++kind) {
+    if (kind > 5) {
+      int64_t waves = 0;
+      for (int i = 0; i < n_jobs; ++i)
+        if (kind_of(list[i]) == kind) waves += (list[i].out_len + 63) / 64 * list[i].outer;
+      rows_per_wave = waves >= 4 * 1024 * 16 ? 16 : waves >= 4 * 1024 * 8 ? 8 : 4;
+    }
     ResampleJobs jobs;
     memset(&jobs, 0, sizeof(jobs));
     int64_t blocks = 0;
     auto flush = [&]() -> int {
       if (jobs.n == 0) return MVIT_OK;
+      jobs.rows_per_wave = rows_per_wave;
       const dim3 grid((unsigned)blocks);
       switch (kind) {
         case 1: hipLaunchKernelGGL((resample_narrow_kernel<1>), grid, 256, 0, s, jobs); break;
         case 2: hipLaunchKernelGGL((resample_narrow_kernel<2>), grid, 256, 0, s, jobs); break;
         case 3: hipLaunchKernelGGL((resample_narrow_kernel<3>), grid, 256, 0, s, jobs); break;
         case 4: hipLaunchKernelGGL((resample_narrow_kernel<4>), grid, 256, 0, s, jobs); break;
+        case 6: hipLaunchKernelGGL((resample_narrow_lds_kernel<1>), grid, 256, 0, s, jobs); break;
+        case 7: hipLaunchKernelGGL((resample_narrow_lds_kernel<2>), grid, 256, 0, s, jobs); break;
+        case 8: hipLaunchKernelGGL((resample_narrow_lds_kernel<3>), grid, 256, 0, s, jobs); break;
+        case 9: hipLaunchKernelGGL((resample_narrow_lds_kernel<4>), grid, 256, 0, s, jobs); break;
         default: hipLaunchKernelGGL(resample_wide_kernel, grid, 256, 0, s, jobs); break;
       }
       MVIT_CHECK_LAUNCH("resample_u8");
@@ -450,7 +667,7 @@ int mvit_resample_u8_batch(const mvit_resample_job* list, int n_jobs, mvit_strea
         continue;
       }
       // the grid of a launch is limited: what does not fit goes to the next one, a job of more work-groups in pieces of whole rows
-      const int64_t unit = kind == 5 ? 1 : 4 * RESAMPLE_ROWS;  // rows that a work-group shares
+      const int64_t unit = shared_rows(kind);
       for (int64_t o = 0; o < j.outer;) {
         const int64_t fit = (MVIT_MAX_GROUPS_256 - blocks) / groups(kind, j, 1) * unit;
         if (jobs.n == RESAMPLE_MAX_JOBS || fit == 0) {

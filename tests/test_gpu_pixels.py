@@ -488,6 +488,42 @@ def test_resample_over_every_inner_length(inner, offset, outer):
     assert (got[:offset] == 9).all() and (got[offset + ref.size :] == 9).all()
 
 
+@pytest.mark.parametrize("inner", [1, 2, 3, 4])
+@pytest.mark.parametrize("ksize,shrink", [(1, 1.0), (4, 0.4), (5, 1.0), (9, 2.0), (13, 3.0), (17, 4.0), (24, 4.6), (24, 5.2), (25, 4.0)])
+@pytest.mark.parametrize("outer,offset", [(1, 0), (7, 1), (33, 3), (1100, 2)])
+def test_resample_short_rows_through_lds_and_past_its_limits(inner, ksize, shrink, outer, offset):
+    """Windows of one to `ksize` taps over rows of one to four bytes per pixel: tap counts on both sides of every group of four, spans below
+    and above what a wave stages, one row and many, arrays at any address, weights at the ends of three 8-bit digits and one past
+    them; sums modulo 2^32.  Bytes around the result are left alone."""
+    from mi355_vit import _lib
+
+    _announce(f"resample short rows inner={inner} ksize={ksize} shrink={shrink} outer={outer} offset={offset}")
+    rng = np.random.default_rng(ksize * 10 + inner)
+    out_len = 131
+    in_len = max(ksize, int(out_len * shrink))
+    src = rng.integers(0, 256, (outer, in_len, inner), dtype=np.uint8)
+    bounds, kk = np.zeros((out_len, 2), dtype=np.int32), np.zeros((out_len, ksize), dtype=np.int32)
+    ref = np.empty((outer, out_len, inner), dtype=np.uint8)
+    for x in range(out_len):
+        n = ksize - (x % 3 if ksize > 3 else 0)
+        bounds[x] = (min(int(x * in_len / out_len), in_len - n), n)
+        kk[x, :n] = rng.integers(-(1 << 19), 1 << 20, n)
+        if x % 7 == 0:
+            kk[x, :1] = rng.choice([0x7F7F7F, -0x808080, 0x7F7F7F + (1 if x == 70 else 0)])
+        lo = bounds[x, 0]
+        acc = (1 << 21) + (src[:, lo : lo + n, :].astype(np.int64) * kk[x, :n, None]).sum(axis=1)
+        ref[:, x, :] = np.clip(acc.astype(np.int32) >> 22, 0, 255)
+    d_src, d_dst = (torch.full((a.size + 32,), 9, dtype=torch.uint8, device=DEV) for a in (src, ref))
+    d_src[offset : offset + src.size] = torch.from_numpy(src.reshape(-1)).to(DEV)
+    d_b, d_k = torch.from_numpy(bounds).to(DEV), torch.from_numpy(kk).to(DEV)
+    rc = _lib.load().mvit_resample_u8(d_src.data_ptr() + offset, d_dst.data_ptr() + offset, outer, in_len, out_len, inner, d_b.data_ptr(), d_k.data_ptr(),
+                                      ksize, torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "mvit_resample_u8")
+    got = d_dst.cpu().numpy()
+    assert np.array_equal(got[offset : offset + ref.size].reshape(ref.shape), ref)
+    assert (got[:offset] == 9).all() and (got[offset + ref.size :] == 9).all()
+
+
 @pytest.mark.parametrize("outer,inner", [((1 << 29) + 100, 1), ((1 << 24) + 5, 8), ((1 << 24) + 5, 400)])
 def test_resample_of_more_work_groups_than_a_launch_takes(outer, inner):
     """A launch takes fewer than 2^24 work-groups of 256 threads; longer passes go in several.  One tap of weight one: a copy."""
