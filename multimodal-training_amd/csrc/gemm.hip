@@ -1172,9 +1172,10 @@ bool pp_takes(GemmTiledKind kind, int64_t k_chunk, int64_t k_last) {  // at leas
 // What a launch costs is its time alone only where nothing runs beside it.  In the backward the input gradients and the weight
 // gradients run on two streams, and the units that one launch's last round leaves idle work for the other: there the estimate is
 // a mean of the time alone (weight `alone`) and of the units' time divided by the number of units, which favours the tile that
-// wastes least over the one that ends its rounds best.  us per 32-block step, tiles by time alone -> by this mean: 14,336 rows
-// 69.6 -> 67.5 ms, 16,384 (checkpointed, optimizer included) 102.9 -> 98.5, 9,600 50.2 -> 49.2 (weight gradients 1.0 of it), 4,096
-// and 20,000 unchanged; weights of 0.25 ... 0.6 (input gradients) and 0.3 ... 0.7 (weight gradients) lie within 1 % of each other.
+// wastes least over the one that ends its rounds best.  That holds where there is work for idle units, i.e. not for input
+// gradients of so few rows that 256 x 256 tiles would give less than half of the units work.  ms per 32-block step, tiles by time
+// alone -> by this mean: 14,336 rows 69.0 -> 66.7, 16,384 (checkpointed, optimizer included) 102.6 -> 100.4, 9,600 50.0 -> 49.0 (that
+// one by the weight gradients' tiles), 4,096, 6,084 and 20,000 unchanged; with the mean at few rows too 1,760 rows 15.6 -> 16.2.
 constexpr double PP_STEP_US = 1.15, PP_TILE_US = 7., PP_SWIGLU_TILE_US = 11.;
 struct TileChoice {
   int bm, bn;
@@ -1185,7 +1186,8 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
   const bool tt = kind == TT_NONE || kind == TT_NONE_F32;
   const double steps = (double)((k_chunk + 63) / 64);
   const int64_t n_mul = kind == NN_SWIGLU ? 2 : 1;
-  const double alone = tt ? 0.5 : (kind == NT_NONE || kind == NT_GELU_BWD ? 0.3 : 1.);
+  const bool fills = 2 * ((M + 255) / 256) * ((N + 255) / 256) >= n_cu;
+  const double alone = tt ? 0.5 : ((kind == NT_NONE || kind == NT_GELU_BWD) && fills ? 0.3 : 1.);
   TileChoice best{0, 0, 1e30};
   auto consider = [&](int bm, int bn, double one, double two, double per_tile) {
     const int64_t items = ((M + bm - 1) / bm) * ((N * n_mul + bn - 1) / bn) * slices;
