@@ -154,11 +154,10 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __res
 // The same sum for cols % 4 == 0: a block owns 16 columns (4 lanes x float4) and 64 row groups, so that a tall
 // partial array (1024 rows from the RMSNorm backward) is walked by many short, independent load chains.
 template <typename T>
-__global__ __launch_bounds__(256) void reduce_partials_vec_kernel(const float* __restrict__ partial, int n_partial,
-                                                                  int64_t cols, T* __restrict__ out) {
+__device__ __forceinline__ void reduce_partials_16(const float* __restrict__ partial, int n_partial, int64_t cols, T* __restrict__ out, int64_t c0) {
   __shared__ float red[64][17];
   const int cx = threadIdx.x & 3, ry = threadIdx.x >> 2;
-  const int64_t c = (int64_t)blockIdx.x * 16 + cx * 4;
+  const int64_t c = c0 + cx * 4;
   f32x4 s = {0.f, 0.f, 0.f, 0.f};
   if (c < cols) {
 #pragma unroll 4
@@ -167,12 +166,29 @@ __global__ __launch_bounds__(256) void reduce_partials_vec_kernel(const float* _
 #pragma unroll
   for (int e = 0; e < 4; ++e) red[ry][cx * 4 + e] = s[e];
   __syncthreads();
-  if (threadIdx.x < 16 && (int64_t)blockIdx.x * 16 + threadIdx.x < cols) {
+  if (threadIdx.x < 16 && c0 + threadIdx.x < cols) {
     float t = 0.f;
 #pragma unroll
     for (int k = 0; k < 64; ++k) t += red[k][threadIdx.x];
-    out[(int64_t)blockIdx.x * 16 + threadIdx.x] = from_f32<T>(t);
+    out[c0 + threadIdx.x] = from_f32<T>(t);
   }
+}
+template <typename T>
+__global__ __launch_bounds__(256) void reduce_partials_vec_kernel(const float* __restrict__ partial, int n_partial, int64_t cols, T* __restrict__ out) {
+  reduce_partials_16(partial, n_partial, cols, out, (int64_t)blockIdx.x * 16);
+}
+// several such sums in one launch
+constexpr int PARTIALS_GROUP_MAX = 4;
+struct PartialsGroup {
+  int n, first_block[PARTIALS_GROUP_MAX];
+  mvit_partials p[PARTIALS_GROUP_MAX];
+};
+template <typename T>
+__global__ __launch_bounds__(256) void reduce_partials_group_kernel(const PartialsGroup g) {
+  int i = 0;
+  while (i + 1 < g.n && (int)blockIdx.x >= g.first_block[i + 1]) ++i;
+  const mvit_partials& p = g.p[i];
+  reduce_partials_16(p.partial, p.n_partial, p.cols, static_cast<T*>(p.out), (int64_t)(blockIdx.x - g.first_block[i]) * 16);
 }
 
 // Column sums with 16-byte loads: a block owns 128 columns (16 lanes x 8/4 elements) and 16 row phases.
@@ -456,6 +472,28 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(const W* __restrict__ e
 }
 
 static inline int clamp_grid(int64_t v, int64_t hi) { return (int)(v < 1 ? 1 : (v > hi ? hi : v)); }
+
+int mvit_reduce_partials_group(const mvit_partials* list, int n, int out_dtype, hipStream_t stream) {
+  bool together = n >= 2 && n <= PARTIALS_GROUP_MAX && (out_dtype == MVIT_BF16 || out_dtype == MVIT_F32);
+  for (int i = 0; i < n; ++i) together = together && list[i].partial && list[i].out && list[i].n_partial > 0 && list[i].cols > 0 && list[i].cols % 4 == 0 && mvit_aligned16(list[i].partial);
+  if (!together) {
+    for (int i = 0; i < n; ++i)
+      if (int rc = mvit_reduce_partials(list[i].partial, list[i].n_partial, list[i].cols, list[i].out, out_dtype, stream)) return rc;
+    return MVIT_OK;
+  }
+  PartialsGroup g = {};
+  g.n = n;
+  int blocks = 0;
+  for (int i = 0; i < n; ++i) {
+    g.p[i] = list[i];
+    g.first_block[i] = blocks;
+    blocks += (int)((list[i].cols + 15) / 16);
+  }
+  if (out_dtype == MVIT_BF16) hipLaunchKernelGGL((reduce_partials_group_kernel<bf16_t>), blocks, 256, 0, stream, g);
+  else hipLaunchKernelGGL((reduce_partials_group_kernel<float>), blocks, 256, 0, stream, g);
+  MVIT_CHECK_LAUNCH("reduce_partials");
+  return MVIT_OK;
+}
 
 extern "C" {
 

@@ -11,7 +11,15 @@
 
 namespace {
 
-constexpr int RMS_PARTIALS = 1024;  // work-groups (= partial rows) of the RMSNorm backward
+// work-groups (= partial rows) of the RMSNorm backward: four rows at a time each, up to 1,024 of them
+inline int rms_partials(int64_t rows) { return (int)(rows < 1 ? 1 : (rows + 3) / 4 < 1024 ? (rows + 3) / 4 : 1024); }
+
+// Up to how many rows the weight gradients go in one launch behind the input-gradient chain, and the column sums in another,
+// instead of starting on the second stream as soon as their inputs are complete: seven launches and ten event calls fewer per
+// block.  A host that issues slower than the GPU computes gains them, and so few rows leave the GPU little to overlap.  ms per
+// 32-block step, second stream / one launch: 64 rows 12.7 / 9.3, 256 12.9 / 9.7, 1,024 13.2 / 11.6, where the GPU is the slower side
+// 1,296 13.21 / 13.35, 1,600 14.6 / 14.9.
+constexpr int64_t GROUP_MAX_ROWS = 1280;
 
 struct Bump {  // hands out 256-byte aligned pieces of the caller's workspace
   char* base;
@@ -44,7 +52,7 @@ mvit_gemm_args gemm_args(int dtype, int out_dtype) {
 
 // Layout of the backward's workspace; with base == nullptr only the size is computed.
 struct BwdWorkspace {
-  float *colsum, *swiglu_cols, *rms, *delta, *splitk;
+  float *colsum, *swiglu_cols, *rms2, *rms1, *delta, *splitk;
   int colsum_rows, n_swiglu_cols;  // rows of dgu per row of swiglu_cols, and how many
   int64_t delta_elems, splitk_bytes, total;
 };
@@ -56,7 +64,8 @@ BwdWorkspace plan_bwd_workspace(const mvit_block_args* a, void* base) {
   w.colsum_rows = mvit_gemm_swiglu_bwd_colsum_rows(S, Ipad, C);
   w.n_swiglu_cols = (int)((S + w.colsum_rows - 1) / w.colsum_rows);
   w.swiglu_cols = static_cast<float*>(b.take((int64_t)w.n_swiglu_cols * 2 * Ipad * 4));
-  w.rms = static_cast<float*>(b.take((int64_t)RMS_PARTIALS * C * 4));
+  w.rms2 = static_cast<float*>(b.take((int64_t)rms_partials(S) * C * 4));
+  w.rms1 = static_cast<float*>(b.take((int64_t)rms_partials(S) * C * 4));
   w.delta_elems = mvit_attn_bwd_delta_elems(a->max_seqlen, S, a->nheads, a->head_dim, a->dtype);
   w.delta = static_cast<float*>(b.take(w.delta_elems * 4));
   const int64_t sk[4] = {a->split_k_down * C * I, a->split_k_gate_up * 2 * Ipad * C, a->split_k_proj * C * C, a->split_k_qkv * 3 * C * C};
@@ -150,8 +159,10 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
                "block_bwd: null parameter-gradient buffer");
   MVIT_REQUIRE(a->grad_dtype == MVIT_BF16 || a->grad_dtype == MVIT_F32, "block_bwd: grad_dtype %d", a->grad_dtype);
   MVIT_REQUIRE(a->split_k_down >= 1 && a->split_k_gate_up >= 1 && a->split_k_proj >= 1 && a->split_k_qkv >= 1, "block_bwd: split_k counts must be >= 1");
-  const bool two = a->side_stream != nullptr;
-  if (two) MVIT_REQUIRE(a->events[0] && a->events[1] && a->events[2] && a->events[3] && a->events[4], "block_bwd: a second stream needs five events");
+  const bool grouped = a->dtype == MVIT_BF16 && a->grad_dtype == MVIT_BF16 && a->S <= GROUP_MAX_ROWS && a->split_k_down == 1 && a->split_k_gate_up == 1 &&
+                       a->split_k_proj == 1 && a->split_k_qkv == 1;
+  const bool two = a->side_stream != nullptr && !grouped;
+  if (a->side_stream != nullptr) MVIT_REQUIRE(a->events[0] && a->events[1] && a->events[2] && a->events[3] && a->events[4], "block_bwd: a second stream needs five events");
   if (a->S == 0) return MVIT_OK;
   const BwdWorkspace w = plan_bwd_workspace(a, a->workspace);
   MVIT_REQUIRE(a->workspace && mvit_aligned16(a->workspace) && a->workspace_bytes >= w.total, "block_bwd: the workspace holds %lld bytes, %lld are needed",
@@ -178,6 +189,8 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
     return mvit_reduce_partials(w.colsum, np, cols, out, gdt, st);
   };
   // dW[M, N] = dY^T . X over the S rows and db[M], the column sums of dY: bf16 products sum them from the operand they read
+  mvit_gemm_args later[4];
+  int n_later = 0;
   auto weight_grad = [&](const void* dy, int64_t ldy, int64_t M, const void* x, int64_t ldx, int64_t N, void* out, void* bias, int split_k, mvit_stream_t st) -> int {
     if (bias && dt != MVIT_BF16) STEP(bias_grad(dy, ldy, M, bias, st));
     mvit_gemm_args g = gemm_args(dt, gdt);
@@ -188,6 +201,10 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
       g.split_k = split_k; g.workspace = w.splitk; g.workspace_bytes = (int64_t)split_k * M * (N + 1) * 4;
     }
     if (dt == MVIT_BF16) g.row_sums = bias;
+    if (grouped) {
+      later[n_later++] = g;
+      return MVIT_OK;
+    }
     return mvit_gemm(&g, st);
   };
 
@@ -213,7 +230,7 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   {
     mvit_stream_t st = fork(1);
     if (!st && two) return MVIT_ERR_LAUNCH;
-    if (fused_cols) STEP(mvit_reduce_partials(w.swiglu_cols, w.n_swiglu_cols, 2 * Ipad, a->g_bgu, gdt, st));
+    if (fused_cols && !grouped) STEP(mvit_reduce_partials(w.swiglu_cols, w.n_swiglu_cols, 2 * Ipad, a->g_bgu, gdt, st));
     STEP(weight_grad(a->dgu, 2 * Ipad, 2 * Ipad, a->n2, C, C, a->g_wgu, fused_cols ? nullptr : a->g_bgu, a->split_k_gate_up, st));
   }
   {  // dn2 = dgu . Wgu
@@ -223,8 +240,8 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
     g.A = a->dgu; g.lda = 2 * Ipad; g.B = a->wgu; g.ldb = C; g.C = a->dn; g.ldc = C;
     STEP(mvit_gemm(&g, stream));
   }
-  STEP(mvit_rmsnorm_bwd(a->dn, a->x1, a->norm2, a->rstd2, a->dx2, a->dx1, w.rms, RMS_PARTIALS, S, C, dt, stream));
-  STEP(mvit_reduce_partials(w.rms, RMS_PARTIALS, C, a->g_norm2, gdt, stream));
+  const int n_rms = rms_partials(S);
+  STEP(mvit_rmsnorm_bwd(a->dn, a->x1, a->norm2, a->rstd2, a->dx2, a->dx1, w.rms2, n_rms, S, C, dt, stream));
 
   // ---- attention: x1 = x + proj(attn(rope(qkv(norm1(x)))))
   {
@@ -255,8 +272,10 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
     g.A = a->dqkv; g.lda = 3 * C; g.B = a->wqkv; g.ldb = C; g.C = a->dn; g.ldc = C;
     STEP(mvit_gemm(&g, stream));
   }
-  STEP(mvit_rmsnorm_bwd(a->dn, a->x, a->norm1, a->rstd1, a->dx1, a->dx, w.rms, RMS_PARTIALS, S, C, dt, stream));
-  STEP(mvit_reduce_partials(w.rms, RMS_PARTIALS, C, a->g_norm1, gdt, stream));
+  STEP(mvit_rmsnorm_bwd(a->dn, a->x, a->norm1, a->rstd1, a->dx1, a->dx, w.rms1, n_rms, S, C, dt, stream));
+  if (grouped) STEP(mvit_gemm_wgrad_group(later, n_later, main_s));
+  const mvit_partials sums[3] = {{w.rms2, n_rms, C, a->g_norm2}, {w.rms1, n_rms, C, a->g_norm1}, {w.swiglu_cols, w.n_swiglu_cols, 2 * Ipad, a->g_bgu}};
+  STEP(mvit_reduce_partials_group(sums, grouped ? 3 : 2, gdt, main_s));
   if (two) {  // the gradients are complete on the main stream when the call's work is
     hipEvent_t ev = reinterpret_cast<hipEvent_t>(a->events[4]);
     if (hipEventRecord(ev, side_s) != hipSuccess || hipStreamWaitEvent(main_s, ev, 0) != hipSuccess)

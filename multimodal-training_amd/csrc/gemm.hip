@@ -1444,6 +1444,60 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
   return MVIT_OK;
 }
 
+// Weight gradients of a few rows in one launch of small tiles, instead of a launch each (plain bf16 products of two transposed
+// operands; anything else is done one by one).  A row's result does not depend on the tile, so the results are the same.
+int mvit_gemm_wgrad_group(const mvit_gemm_args* list, int n, hipStream_t s) {
+  bool together = n >= 2 && n <= GEMM_GROUP_MAX;
+  for (int i = 0; i < n; ++i) {
+    const mvit_gemm_args& a = list[i];
+    together = together && a.dtype == MVIT_BF16 && a.out_dtype == MVIT_BF16 && a.trans_a && a.trans_b && a.epilogue == MVIT_EPI_NONE && a.split_k <= 1 &&
+               a.M > 0 && a.N > 0 && a.K > 0 && a.A && a.B && a.C && mvit_aligned16(a.A) && mvit_aligned16(a.B) && a.lda % 8 == 0 && a.ldb % 8 == 0 &&
+               a.lda >= (a.M + 7) / 8 * 8 && a.ldb >= (a.N + 7) / 8 * 8 && a.ldc >= a.N && a.lda <= (1ll << 22) && a.ldb <= (1ll << 22);
+  }
+  if (!together) {
+    for (int i = 0; i < n; ++i)
+      if (int rc = mvit_gemm(&list[i], s)) return rc;
+    return MVIT_OK;
+  }
+  const int dev = mvit_current_device("gemm");
+  if (dev < 0) return MVIT_ERR_LAUNCH;
+  const int n_cu = device_cu_count(dev);
+  // one tile shape for all of them: the model of choose_tile over the sum of their tiles
+  struct { int bm, bn; double one, two, per_tile; } const shapes[] = {{64, 64, 0.23, 0.36, 2.}, {64, 128, 0.37, 0.52, 2.}, {128, 128, 0.60, 0.72, 2.5}};
+  int bm = 128, bn = 128;
+  double best = 1e30;
+  for (const auto& t : shapes) {
+    int64_t items = 0, k = 0;
+    for (int i = 0; i < n; ++i) {
+      items += ((list[i].M + t.bm - 1) / t.bm) * ((list[i].N + t.bn - 1) / t.bn);
+      k = list[i].K > k ? list[i].K : k;
+    }
+    MVIT_REQUIRE(items < (1ll << 30), "gemm: too many tiles");
+    const double steps = (double)((k + 63) / 64);
+    const int64_t rest = items % (2 * n_cu);
+    double us = (double)(items / (2 * n_cu)) * (steps * t.two + t.per_tile);
+    if (rest > 0) us += steps * (rest > n_cu ? t.two : t.one) + t.per_tile;
+    if (us < best) best = us, bm = t.bm, bn = t.bn;
+  }
+  GemmGroup g;
+  memset(&g, 0, sizeof(g));
+  g.n = n;
+  for (int i = 0; i < n; ++i) {
+    const mvit_gemm_args& a = list[i];
+    GemmParams& p = g.p[i];
+    p.M = a.M; p.N = a.N; p.K = a.K;
+    p.A = a.A; p.lda = a.lda; p.B = a.B; p.ldb = a.ldb; p.C = a.C; p.ldc = a.ldc;
+    p.row_sums = a.row_sums;
+    p.vec_ok = vec16(a.C, a.ldc, 2);
+    p.half_vec_ok = a.ldc % 4 == 0 && reinterpret_cast<uintptr_t>(a.C) % 8 == 0;
+    p.split_k = 1; p.k_chunk = a.K; p.reduce_epi = MVIT_EPI_NONE;
+    p.tiles_m = (int)((a.M + bm - 1) / bm);
+    p.tiles_n = (int)((a.N + bn - 1) / bn);
+    p.panel_w = p.tiles_n <= 6 ? p.tiles_n : 4;
+  }
+  return mvit_gemm_small_group(bm, bn, g, s);
+}
+
 extern "C" int mvit_gemm_wgrad_split_k(int64_t out_rows, int64_t out_cols, int64_t k) {
   // Slices along the contraction for a product with few output tiles and a long contraction (a weight gradient, contracted
   // over the tokens): the count with the lowest modelled time.  Every slice costs an fp32 partial tile written and read back

@@ -44,6 +44,14 @@ enum GemmTiledKind { TILED_NONE = -1, NN_NONE, NN_BIAS, NN_BIAS_RES, NN_BIAS_GEL
 int mvit_gemm_pp(GemmTiledKind kind, const GemmParams& p, int n_cu, hipStream_t stream);                  // gemm_pingpong.hip
 int mvit_gemm_small(GemmTiledKind kind, int bm, int bn, const GemmParams& p, hipStream_t stream);         // gemm_small.hip
 
+constexpr int GEMM_GROUP_MAX = 4;
+struct GemmGroup {
+  int n;
+  unsigned first_block[GEMM_GROUP_MAX];
+  GemmParams p[GEMM_GROUP_MAX];
+};
+int mvit_gemm_small_group(int bm, int bn, GemmGroup& group, hipStream_t stream);                                // gemm_small.hip
+
 int mvit_gemm_f32(int ta, int tb, int epi, const GemmParams& p, hipStream_t stream);                        // gemm_f32.hip
 
 namespace {

@@ -33,7 +33,7 @@ __device__ __forceinline__ int small_swizzle(int major) {
 }
 
 template <typename TO, bool TA, bool TB, int EPI, typename S>
-__global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(const GemmParams p) {  // two work-groups fit a compute unit
+__device__ __forceinline__ void gemm_small_tile(const GemmParams& p, const unsigned block) {
   using T = bf16_t;
   constexpr int BM = S::BM, BN = S::BN, BK = S::BK, NST = S::NST;
   constexpr bool DUAL = (EPI == MVIT_EPI_SWIGLU);
@@ -45,8 +45,8 @@ __global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(cons
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
 
   const unsigned tiles = (unsigned)(p.tiles_m * p.tiles_n), total = tiles * (unsigned)p.split_k, per_xcd = (total + 7) / 8;
-  const unsigned work = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if ((blockIdx.x >> 3) >= per_xcd || work >= total) return;
+  const unsigned work = (block & 7) * per_xcd + (block >> 3);
+  if ((block >> 3) >= per_xcd || work >= total) return;
   const unsigned slice = p.split_k > 1 ? work / tiles : 0;
   int tm, tn;
   tile_coords(p, (int)(work - slice * tiles), tm, tn);
@@ -320,18 +320,24 @@ __global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(cons
   }
 }
 
-}  // namespace
-
-namespace {
+template <typename TO, bool TA, bool TB, int EPI, typename S>
+__global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(const GemmParams p) {  // two work-groups fit a compute unit
+  gemm_small_tile<TO, TA, TB, EPI, S>(p, blockIdx.x);
+}
+// several independent products: each takes a range of work-groups, a multiple of eight so that it stays dealt to the XCDs
+template <typename TO, bool TA, bool TB, int EPI, typename S>
+__global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_group_kernel(const GemmGroup g) {
+  int i = 0;
+  while (i + 1 < g.n && blockIdx.x >= g.first_block[i + 1]) ++i;
+  gemm_small_tile<TO, TA, TB, EPI, S>(g.p[i], blockIdx.x - g.first_block[i]);
+}
 
 using Small64 = SmallCfg<64, 64, 2, 2, 4>;      // 64 KiB of LDS
 using Small64x128 = SmallCfg<64, 128, 2, 2, 3>;  // 72 KiB
 using Small128 = SmallCfg<128, 128, 2, 2, 2>;    // 64 KiB
 
-template <typename TO, bool TA, bool TB, int EPI, typename S>
-int launch_small(const GemmParams& p, hipStream_t stream) {
-  auto kern = gemm_small_kernel<TO, TA, TB, EPI, S>;
-  static bool attr_set_on[MVIT_MAX_DEVICES] = {};
+template <typename S, typename P>
+int launch_grid(void (*kern)(P), const P& p, unsigned grid, bool (&attr_set_on)[MVIT_MAX_DEVICES], hipStream_t stream) {
   const int dev = mvit_current_device("gemm");
   if (dev < 0) return MVIT_ERR_LAUNCH;
   if (!attr_set_on[dev] && S::LDS > 64 * 1024) {  // dynamic LDS above 64 KiB is opted into once per kernel and device
@@ -339,9 +345,26 @@ int launch_small(const GemmParams& p, hipStream_t stream) {
     if (e != hipSuccess) return mvit_set_error(MVIT_ERR_LAUNCH, "gemm: hipFuncSetAttribute(%d B LDS): %s", S::LDS, hipGetErrorString(e));
     attr_set_on[dev] = true;
   }
-  hipLaunchKernelGGL(kern, (p.tiles_m * p.tiles_n * p.split_k + 7) / 8 * 8, S::NTHREADS, S::LDS, stream, p);
+  hipLaunchKernelGGL(kern, grid, S::NTHREADS, S::LDS, stream, p);
   MVIT_CHECK_LAUNCH("gemm");
   return MVIT_OK;
+}
+inline unsigned grid_of(const GemmParams& p) { return (unsigned)((p.tiles_m * p.tiles_n * p.split_k + 7) / 8 * 8); }
+
+template <typename TO, bool TA, bool TB, int EPI, typename S>
+int launch_small(const GemmParams& p, hipStream_t stream) {
+  static bool attr_set_on[MVIT_MAX_DEVICES] = {};
+  return launch_grid<S>(gemm_small_kernel<TO, TA, TB, EPI, S>, p, grid_of(p), attr_set_on, stream);
+}
+template <typename S>
+int launch_group(GemmGroup& g, hipStream_t stream) {
+  static bool attr_set_on[MVIT_MAX_DEVICES] = {};
+  unsigned blocks = 0;
+  for (int i = 0; i < g.n; ++i) {
+    g.first_block[i] = blocks;
+    blocks += grid_of(g.p[i]);
+  }
+  return launch_grid<S>(gemm_small_group_kernel<bf16_t, true, true, MVIT_EPI_NONE, S>, g, blocks, attr_set_on, stream);
 }
 
 template <typename S>
@@ -372,4 +395,10 @@ int mvit_gemm_small(GemmTiledKind kind, int bm, int bn, const GemmParams& p, hip
   if (bm == 128) return dispatch_small<Small128>(kind, p, stream);
   if (bn == 128) return dispatch_small<Small64x128>(kind, p, stream);
   return dispatch_small<Small64>(kind, p, stream);
+}
+// weight gradients (both operands transposed, bf16 results), tiles_m / tiles_n set for bm x bn
+int mvit_gemm_small_group(int bm, int bn, GemmGroup& g, hipStream_t stream) {
+  if (bm == 128) return launch_group<Small128>(g, stream);
+  if (bn == 128) return launch_group<Small64x128>(g, stream);
+  return launch_group<Small64>(g, stream);
 }

@@ -41,6 +41,16 @@ int mvit_set_error(int code, const char* fmt, ...);
 
 static inline bool mvit_aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// Launches that several steps of a block share (block.cpp).
+int mvit_gemm_wgrad_group(const mvit_gemm_args* list, int n, hipStream_t stream);  // gemm.hip
+struct mvit_partials {  // out[c] = the sum of n_partial rows of `cols` floats, in the order of mvit_reduce_partials
+  const float* partial;
+  int n_partial;
+  int64_t cols;
+  void* out;
+};
+int mvit_reduce_partials_group(const mvit_partials* list, int n, int out_dtype, hipStream_t stream);  // bandwidth.hip
+
 // Per-device host state (function attributes set, compute-unit counts, symbol addresses) is kept in arrays of this
 // many slots indexed by the current device's ordinal.
 #define MVIT_MAX_DEVICES 64

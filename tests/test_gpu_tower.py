@@ -188,6 +188,29 @@ def test_one_call_per_block_equals_the_call_by_call_sequence(dtype, checkpoint):
             assert torch.equal(grads[k], ref_grads[k]), (key, k)
 
 
+@pytest.mark.parametrize("hidden,inner", [(512, 1200), (64, 72)])
+@pytest.mark.parametrize("grid", [[[1, 2, 2]], [[1, 6, 10]], [[1, 16, 16], [1, 2, 6]], [[1, 32, 40]], [[1, 32, 40], [1, 2, 2]]])
+def test_weight_gradients_of_few_rows_in_one_launch_equal_a_launch_each(grid, hidden, inner):
+    """Up to 1,280 rows the backward of a block sends its weight gradients in one launch and its column sums in another (4, 60, 268 and
+    1,280 rows; 1,284 go as longer ones do): output and gradients have the bits of the call-by-call sequence."""
+    from mi355_vit import functional
+
+    kw = dict(depth=2, hidden_size=hidden, intermediate_size=inner, num_heads=hidden // 32, out_hidden_size=256, window_size=56, fullatt_block_indexes=[1])
+    g = torch.Generator().manual_seed(13)
+    grid = torch.tensor(grid)
+    S = int(grid.prod(1).sum())
+    pixels, gout = torch.randn(S, 1176, generator=g), torch.randn(S // 4, 256, generator=g)
+    res, old = [], functional.BLOCK_CALLS
+    try:
+        for functional.BLOCK_CALLS in (True, False):
+            res.append(_run_gpu(_build(kw, 8, torch.bfloat16), pixels, grid, gout))
+    finally:
+        functional.BLOCK_CALLS = old
+    assert torch.equal(res[0][0], res[1][0]) and torch.isfinite(res[0][0]).all()
+    for k in res[1][1]:
+        assert torch.equal(res[0][1][k], res[1][1][k]), k
+
+
 def test_reference_smoke_shape():
     """The reference's own smoke case (tests/test_ragged_sp_smoke.py:27-98): output [192, 256]."""
     kw = dict(hidden_size=256, num_heads=8, depth=2, patch_size=14, in_channels=3, out_hidden_size=256, spatial_merge_size=2,
