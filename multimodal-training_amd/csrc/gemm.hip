@@ -379,7 +379,7 @@ __device__ __forceinline__ void run_epilogue(const GemmParams& p, f32x16 (&acc)[
               u[4 + e] = u1[e];
             }
           }
-          if (to_ws) store8_cached(ws + m * p.N + n, v);
+          if (to_ws) store8(ws + m * p.N + n, v);
           else if constexpr (EP::HAS_IN) {
             // the same item of pass a + NBUF is requested before this item's stores are issued: a wave's memory
             // instructions complete in order, so the wait for a load also waits for every store issued before it
@@ -443,7 +443,7 @@ __device__ __forceinline__ void run_epilogue(const GemmParams& p, f32x16 (&acc)[
       }
       if (to_ws) {
         float* w = ws + m * p.N + n;
-        if (ws_vec && n + 8 <= p.N) store8_cached(w, v);
+        if (ws_vec && n + 8 <= p.N) store8(w, v);
         else
           for (int e = 0; e < 8 && n + e < p.N; ++e) w[e] = v[e];
       } else {

@@ -101,22 +101,19 @@ __device__ __forceinline__ void unpack8(const T __attribute__((ext_vector_type(8
 #pragma unroll
   for (int e = 0; e < 8; ++e) v[e] = (float)x[e];
 }
-// Epilogue outputs and per-element epilogue inputs are touched once per launch: they are stored / loaded with the
-// non-temporal hint, so that they do not push the operand panels of the tiles in flight out of the XCD's L2 (a round of
-// 32 output tiles is as large as that L2; with plain stores the main loop after an epilogue ran 18 % slower).
+// Epilogue outputs are stored plainly: the two stores that make a 128-byte line meet in the L2, and the next kernels find what fits
+// the memory-side cache there.  With the non-temporal hint a launch alone is the faster one where its output does not fit (us plain /
+// hinted, 3840 columns with bias of 65,536 rows, 503 MB, 561 / 506, of 14,336 rows 124 / 128; SwiGLU of 25,524 rows 390 / 399), but
+// steps are not, whichever outputs take it (65,536 rows: 639 ms either way), and shorter ones lose: ms per step hinted -> plain
+// 4,360 rows without gradients 8.56 -> 8.17, 4,096 with checkpointing 30.1 -> 29.4, 14,336 65.9 -> 64.9, 25,524 112.4 -> 111.4.
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void store8(bf16_t* p, const float* v) {
   bf16x8 x;
 #pragma unroll
   for (int e = 0; e < 8; ++e) x[e] = (bf16_t)v[e];
-  __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, x), reinterpret_cast<u32x4_t*>(p));
+  *reinterpret_cast<u32x4_t*>(p) = __builtin_bit_cast(u32x4_t, x);
 }
 __device__ __forceinline__ void store8(float* p, const float* v) {
-  __builtin_nontemporal_store(f32x4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f32x4*>(p));
-  __builtin_nontemporal_store(f32x4{v[4], v[5], v[6], v[7]}, reinterpret_cast<f32x4*>(p + 4));
-}
-// split-K partial tiles are read back by the reduction kernel right away: they stay cacheable
-__device__ __forceinline__ void store8_cached(float* p, const float* v) {
   *reinterpret_cast<f32x4*>(p) = f32x4{v[0], v[1], v[2], v[3]};
   *reinterpret_cast<f32x4*>(p + 4) = f32x4{v[4], v[5], v[6], v[7]};
 }

@@ -212,7 +212,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmParams p) {
       }
       if (to_ws) {
         float* w = ws + m * p.N + n;
-        if (vec && n + 8 <= p.N) store8_cached(w, v);
+        if (vec && n + 8 <= p.N) store8(w, v);
         else
           for (int e = 0; e < 8 && n + e < p.N; ++e) w[e] = v[e];
       } else {

@@ -391,7 +391,7 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
         for (int it = 0; it < ITEMS; ++it) {
           float v[8], u[8];
           values(it, v, u);
-          if (to_ws) store8_cached(ws + row_of(it) * p.N + n_lane[it % NG], v);
+          if (to_ws) store8(ws + row_of(it) * p.N + n_lane[it % NG], v);
           else emit8_impl<T, TO, EPI, true, false>(p, row_of(it), n_lane[it % NG], v, u, nullptr, no_cs, false, HAS_BIAS ? hb[it % NG] : nullptr, HAS_BIAS && DUAL ? hb[1] : nullptr);
         }
       }
@@ -405,7 +405,7 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
         if (m >= p.M || n >= p.N) continue;
         if (to_ws) {
           float* w = ws + m * p.N + n;
-          if (vec && n + 8 <= p.N) store8_cached(w, v);
+          if (vec && n + 8 <= p.N) store8(w, v);
           else
             for (int e = 0; e < 8 && n + e < p.N; ++e) w[e] = v[e];
         } else if (vec && n + 8 <= p.N) {

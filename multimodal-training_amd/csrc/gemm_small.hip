@@ -280,13 +280,13 @@ __device__ __forceinline__ void gemm_small_tile(const GemmParams& p, const unsig
       float hb[8], hb2[8];
       if (HAS_BIAS) unpack8<T>(bias_g[g], hb);
       if (HAS_BIAS && DUAL) unpack8<T>(bias_u, hb2);
-      if (to_ws) store8_cached(ws + m * p.N + n, v);
+      if (to_ws) store8(ws + m * p.N + n, v);
       else emit8_impl<T, TO, EPI, true, HAS_IN>(p, m, n, v, u, HAS_IN ? pre[it] : nullptr, cs[CAN_CS ? g : 0], do_cs, HAS_BIAS ? hb : nullptr, HAS_BIAS && DUAL ? hb2 : nullptr);
     } else {
       if (m >= p.M || n >= p.N) continue;
       if (to_ws) {
         float* w = ws + m * p.N + n;
-        if (vec && n + 8 <= p.N) store8_cached(w, v);
+        if (vec && n + 8 <= p.N) store8(w, v);
         else
           for (int e = 0; e < 8 && n + e < p.N; ++e) w[e] = v[e];
       } else {
