@@ -1159,7 +1159,7 @@ GemmTiledKind tiled_kind(int dtype, int out_dtype, int ta, int tb, int epi, cons
 }
 
 bool pp_takes(GemmTiledKind kind, int64_t k_chunk, int64_t k_last) {  // at least three K tiles of 64 in every slice
-  return kind != NT_SWIGLU_BWD && k_chunk > 128 && k_last > 128;
+  return k_chunk > 128 && k_last > 128;
 }
 
 // Modelled times (us) of the tiles on one MI355X, fitted to every tile's time at 256 ... 16,384 rows of the tower's products: a
@@ -1181,7 +1181,11 @@ struct TileChoice {
   int bm, bn;
   double us;
 };
-// `full_rows`: whether the 256-row SwiGLU-backward kernel (bm = 0) may be chosen
+// The 256-row SwiGLU-backward kernel: gemm_pp_kernel, or gemm_dl_kernel (bm = 0) for a contraction of fewer than three K tiles
+TileChoice full_rows_tile(GemmTiledKind kind, int64_t k_chunk, int64_t k_last) {
+  return pp_takes(kind, k_chunk, k_last) ? TileChoice{256, 256, 0.} : TileChoice{0, 0, 0.};
+}
+// `full_rows`: whether that kernel may be chosen
 TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk, int64_t k_last, int64_t slices, int n_cu, bool full_rows = true) {
   const bool tt = kind == TT_NONE || kind == TT_NONE_F32;
   const double steps = (double)((k_chunk + 63) / 64);
@@ -1199,23 +1203,22 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
     if (us < best.us) best = TileChoice{bm, bn, us};
   };
   const bool swiglu = kind == NN_SWIGLU;
-  if (pp_takes(kind, k_chunk, k_last)) consider(256, 256, tt ? 1.2 : PP_STEP_US, 0., swiglu ? PP_SWIGLU_TILE_US : PP_TILE_US);
+  if (pp_takes(kind, k_chunk, k_last) && kind != NT_SWIGLU_BWD) consider(256, 256, tt ? 1.2 : PP_STEP_US, 0., swiglu ? PP_SWIGLU_TILE_US : PP_TILE_US);
   if (kind == NT_SWIGLU_BWD) {  // two inputs, two outputs and the column sums lengthen its epilogue
     consider(64, 64, 0.30, 0.43, 2.);
     consider(64, 128, 0.47, 0.70, 2.);
+    consider(128, 128, 0.55, 0.90, 5.);
   } else {
     if (!swiglu) consider(64, 64, 0.23, 0.36, 2.);
     consider(64, 128, 0.37, 0.52, 2.);
     consider(128, 128, 0.60, 0.72, swiglu ? 6. : 2.5);
   }
-  // SwiGLU backward: the 256-row kernel as soon as its tiles give half of the units work.  Its launch shares the GPU with the
-  // down projection's weight gradient on the second stream, which fills the units it leaves idle, while two small tiles per
-  // unit compete with it for the L2s.  us per block of the tower, forward and backward, 64 x 64 / 64 x 128 / 256-row:
-  // recorded in a graph at 256 rows 291 / 296 / 334, 1,024: 402 / 403 / 428, 2,048: 581 / 578 / 598, 2,688: 689 / 683 / 697,
-  // 3,136: 755 / 741 / 751; issued one by one at 2,304 rows 603 / 591 / 588, 2,688: 676 / 670 / 650, 4,864: 1,004 / 990 / 970,
-  // 10,400: 1,748 / 1,713 / 1,662, 14,336: 2,457 / 2,415 / 2,359 (the launch alone would be faster on small tiles wherever the
-  // 256-row tiles end in a bad round: 4,864 rows 91 / 76 / 105, 10,240: 182 / 142 / 164)
-  if (kind == NT_SWIGLU_BWD && full_rows && 2 * ((M + 255) / 256) * ((N + 255) / 256) >= n_cu) best = TileChoice{0, 0, 0.};
+  // SwiGLU backward: the 256-row kernel as soon as its tiles give nearly half of the units work.  Its launch shares the GPU with
+  // the down projection's weight gradient on the second stream, which fills the units it leaves idle, while two small tiles per
+  // unit compete with it for the L2s.  ms per 32-block step, 64 x 64 / 64 x 128 / 128 x 128 / 256 x 256: 576 rows 9.56 / 9.53 / 9.87 / 10.48,
+  // 1,600 14.8 / 14.6 / 14.4 / 14.8, 2,048 16.4 / 16.2 / 15.8 / 16.2, 2,304 18.0 / 17.8 / 18.0 / 17.5, 3,136 21.9 / 21.7 / 22.0 / 21.8,
+  // 4,900 31.8 / 31.4 / 31.0 / 30.6, 6,084 37.2 / 36.7 / 36.2 / 35.8 (alone 128 x 128 is ahead up to 20,000 rows, 165 us against 185 at 14,336)
+  if (kind == NT_SWIGLU_BWD && full_rows && 32 * ((M + 255) / 256) * ((N + 255) / 256) >= 15 * n_cu) best = full_rows_tile(kind, k_chunk, k_last);
   return best;
 }
 
@@ -1392,7 +1395,7 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
     const bool all_256 = getenv("MVIT_GEMM_NO_HALF_TILES") != nullptr;
     if (all_256 && c.bm != 256 && pp_takes(kind, p.k_chunk, p.K - (p.split_k - 1) * p.k_chunk)) c = TileChoice{256, 256, 0.};
     // the column sums are per tile row: their granularity names the kernel (64 rows: 64 x 64 or 64 x 128 tiles, below)
-    if (kind == NT_SWIGLU_BWD && p.colsum != nullptr) c = colsum_rows == 64 ? choose_tile(kind, p.M, p.N, p.k_chunk, p.K, 1, n_cu, false) : TileChoice{0, 0, 0.};
+    if (kind == NT_SWIGLU_BWD && p.colsum != nullptr) c = colsum_rows == 64 ? choose_tile(kind, p.M, p.N, p.k_chunk, p.K, 1, n_cu, false) : full_rows_tile(kind, p.K, p.K);
     if (c.bm != 0) {
       auto run = [&](GemmParams q, const TileChoice& t) -> int {
         q.tiles_m = (int)((q.M + t.bm - 1) / t.bm);
@@ -1518,5 +1521,6 @@ extern "C" int mvit_gemm_wgrad_split_k(int64_t out_rows, int64_t out_cols, int64
 }
 
 extern "C" int mvit_gemm_swiglu_bwd_colsum_rows(int64_t M, int64_t N, int64_t K) {
-  return choose_tile(NT_SWIGLU_BWD, M, N, K, K, 1, 256).bm == 0 ? 256 : 64;
+  const int bm = choose_tile(NT_SWIGLU_BWD, M, N, K, K, 1, 256).bm;
+  return bm == 0 || bm == 256 ? 256 : 64;
 }

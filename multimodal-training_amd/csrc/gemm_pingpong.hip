@@ -21,6 +21,10 @@
 // staging and no barrier, and the next tile's first loads run under them.  K order and MFMA form are the same for every tile shape of
 // this file, so a result does not depend on the shape that computed it.
 //
+// SwiGLU backward (two inputs and two outputs per element, column sums): us at 4,096 / 14,336 / 65,536 rows of 3456 columns 50 / 187 / 798,
+// with K tiles of 32 and results staged in LDS 64 / 221 / 778; per 32-block step 14,336 rows 64.9 -> 64.5 ms, 16,384 96.2 -> 95.2, 25,524
+// 111.4 -> 110.9.  What bounds it is the epilogue's memory traffic (stores left out: 652 us at 65,536 rows).
+//
 // LDS layouts (a direct load writes 1 KiB of contiguous LDS per instruction; the lanes choose which 16 bytes they fetch):
 //   [row][k] operands: 128-byte rows of 8 chunks, chunk c of row r in slot c ^ f(r); f makes the 16 rows of a fragment read
 //   fall on 16 different 16-byte slots of 256 bytes;
@@ -42,7 +46,8 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
   using T = bf16_t;
   constexpr int BM = PpCfg::BM, BK = PpCfg::BK, HALF = PpCfg::HALF, STAGE = PpCfg::STAGE;
   constexpr bool DUAL = (EPI == MVIT_EPI_SWIGLU);
-  constexpr bool HAS_IN = EPI == MVIT_EPI_BIAS_RES || EPI == MVIT_EPI_GELU_BWD;
+  constexpr bool SW_BWD = EPI == MVIT_EPI_SWIGLU_BWD;
+  constexpr bool HAS_IN = EPI == MVIT_EPI_BIAS_RES || EPI == MVIT_EPI_GELU_BWD || SW_BWD;
   constexpr bool HAS_BIAS = EPI == MVIT_EPI_BIAS || EPI == MVIT_EPI_BIAS_RES || EPI == MVIT_EPI_BIAS_GELU || EPI == MVIT_EPI_SWIGLU;
   constexpr int NCOLS = DUAL ? 128 : 256;
   // sums of A's rows over k (the bias gradient of a weight-gradient product) from the fragments that are in registers anyway:
@@ -54,8 +59,8 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
   // stores of an interior tile's epilogue that are issued after the next tile's first loads (memory instructions of a wave
   // complete in order, so a wait for those loads may leave this many more in flight)
   constexpr int STORES = DUAL ? 8 : (EPI == MVIT_EPI_BIAS_GELU ? 32 : (sizeof(TO) == 4 ? 32 : 16));
-  constexpr int DEPTH = 8;  // items whose input is fetched ahead
-  constexpr int TRAILING = HAS_IN ? DEPTH : STORES;
+  constexpr int NIN = SW_BWD ? 2 : 1, DEPTH = SW_BWD ? 4 : 8;  // inputs of an item; items whose inputs are fetched ahead
+  constexpr int TRAILING = HAS_IN ? DEPTH * NIN : STORES;  // an item stores as many vectors as it has inputs
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
 
   const int l = threadIdx.x & 63;
@@ -341,12 +346,36 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
 #pragma unroll
       for (int g = 0; g < 2; ++g) load8(reinterpret_cast<const bf16_t*>(bl + g * 64 + g4 * 16), hb[g]);
     }
-    float no_cs[16];
+    float no_cs[16];  // SW_BWD: column sums over the lane's rows, of the eight columns' gate and up halves
+    const bool do_cs = SW_BWD && p.colsum != nullptr;
+    float* cs_lds = reinterpret_cast<float*>(smem_raw + PpCfg::BIAS_OFF);
+    // column half g is through: its sums over the 16 lanes of a row block, in a fixed order, parked for the other row group
+    auto park_sums = [&](int g) {
+      if constexpr (SW_BWD) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          float t = no_cs[e];
+          t += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, t), 0x128, 0xf, 0xf, false));  // row_ror:8, 4, 2, 1
+          t += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, t), 0x124, 0xf, 0xf, false));
+          t += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, t), 0x122, 0xf, 0xf, false));
+          t += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, t), 0x121, 0xf, 0xf, false));
+          if (i16 == 0) cs_lds[wv * 128 + g * 64 + (e >> 3) * 32 + tr_first_column(g4) + (e & 7)] = t;
+          no_cs[e] = 0.f;
+        }
+      }
+    };
+    if constexpr (SW_BWD) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) no_cs[e] = 0.f;
+    }
     float* ws = to_ws ? p.workspace + (int64_t)slice * p.M * p.N : nullptr;
     constexpr int NG = DUAL ? 1 : 2, ITEMS = 8 * NG;
-    auto row_of = [&](int it) { return m_lane + (it / NG >> 2) * 128 + (it / NG & 3) * 16; };
+    // item -> row block and column half: by rows, or all rows of a half first where their sums are wanted
+    auto block_of = [](int it) { return SW_BWD ? it & 7 : it / NG; };
+    auto half_of = [](int it) { return SW_BWD ? it >> 3 : it % NG; };
+    auto row_of = [&](int it) { return m_lane + (block_of(it) >> 2) * 128 + (block_of(it) & 3) * 16; };
     auto values = [&](int it, float (&v)[8], float (&u)[8]) {
-      const int a = it / NG, g = it % NG;
+      const int a = block_of(it), g = half_of(it);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         v[e] = acc[a][2 * g][e];
@@ -372,18 +401,25 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
       if constexpr (HAS_IN) {
         // the input was written a few launches ago and is often still in the memory-side cache: a plain load finds it there
         // (25,524 x 1280 x 1280 with residual: 98 us with non-temporal loads, 83 us with plain ones)
-        bf16x8 pre[DEPTH];
-        auto fetch = [&](int it) { return *reinterpret_cast<const bf16x8*>(static_cast<const T*>(p.R) + row_of(it) * p.ldr + n_lane[it % NG]); };
+        bf16x8 pre[DEPTH][NIN];
+        auto fetch = [&](int it, bf16x8 (&to)[NIN]) {
+          const T* r = static_cast<const T*>(p.R) + row_of(it) * p.ldr + n_lane[half_of(it)];
+          to[0] = *reinterpret_cast<const bf16x8*>(r);
+          if constexpr (SW_BWD) to[1] = *reinterpret_cast<const bf16x8*>(r + p.aux_off);
+        };
 #pragma unroll
-        for (int it = 0; it < DEPTH; ++it) pre[it] = fetch(it);
+        for (int it = 0; it < DEPTH; ++it) fetch(it, pre[it]);
 #pragma unroll
         for (int it = 0; it < ITEMS; ++it) {
           float v[8], u[8];
           values(it, v, u);
-          const bf16x8 now = pre[it % DEPTH];
-          if (it + DEPTH < ITEMS) pre[it % DEPTH] = fetch(it + DEPTH);
+          bf16x8 now[NIN];
+#pragma unroll
+          for (int i = 0; i < NIN; ++i) now[i] = pre[it % DEPTH][i];
+          if (it + DEPTH < ITEMS) fetch(it + DEPTH, pre[it % DEPTH]);
           if (it == ITEMS - DEPTH && have) issue_first();  // behind the last of this tile's input loads
-          emit8_impl<T, TO, EPI, true, true>(p, row_of(it), n_lane[it % NG], v, u, &now, no_cs, false, HAS_BIAS ? hb[it % NG] : nullptr, nullptr);
+          emit8_impl<T, TO, EPI, true, true>(p, row_of(it), n_lane[half_of(it)], v, u, now, no_cs, do_cs, HAS_BIAS ? hb[half_of(it)] : nullptr, nullptr);
+          if (do_cs && (it & 7) == 7) park_sums(it >> 3);
           __builtin_amdgcn_sched_barrier(0);
         }
       } else {
@@ -391,8 +427,8 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
         for (int it = 0; it < ITEMS; ++it) {
           float v[8], u[8];
           values(it, v, u);
-          if (to_ws) store8(ws + row_of(it) * p.N + n_lane[it % NG], v);
-          else emit8_impl<T, TO, EPI, true, false>(p, row_of(it), n_lane[it % NG], v, u, nullptr, no_cs, false, HAS_BIAS ? hb[it % NG] : nullptr, HAS_BIAS && DUAL ? hb[1] : nullptr);
+          if (to_ws) store8(ws + row_of(it) * p.N + n_lane[half_of(it)], v);
+          else emit8_impl<T, TO, EPI, true, false>(p, row_of(it), n_lane[half_of(it)], v, u, nullptr, no_cs, false, HAS_BIAS ? hb[half_of(it)] : nullptr, HAS_BIAS && DUAL ? hb[1] : nullptr);
         }
       }
     } else {
@@ -401,7 +437,8 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
       for (int it = 0; it < ITEMS; ++it) {
         float v[8], u[8];
         values(it, v, u);
-        const int64_t m = row_of(it), n = n_lane[it % NG];
+        const int64_t m = row_of(it), n = n_lane[half_of(it)];
+        if (do_cs && (it & 7) == 0 && it > 0) park_sums((it >> 3) - 1);
         if (m >= p.M || n >= p.N) continue;
         if (to_ws) {
           float* w = ws + m * p.N + n;
@@ -409,12 +446,29 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
           else
             for (int e = 0; e < 8 && n + e < p.N; ++e) w[e] = v[e];
         } else if (vec && n + 8 <= p.N) {
-          emit8_impl<T, TO, EPI, true>(p, m, n, v, u, nullptr, no_cs, false, HAS_BIAS ? hb[it % NG] : nullptr, HAS_BIAS && DUAL ? hb[1] : nullptr);
+          emit8_impl<T, TO, EPI, true>(p, m, n, v, u, nullptr, no_cs, do_cs, HAS_BIAS ? hb[half_of(it)] : nullptr, HAS_BIAS && DUAL ? hb[1] : nullptr);
         } else {
-          emit8<T, TO, EPI>(p, m, n, v, u, false, no_cs, false);
+          emit8<T, TO, EPI>(p, m, n, v, u, false, no_cs, do_cs);
         }
       }
+      if (do_cs) park_sums(NG - 1);
       pp_wait_vm<0>();  // the count of this path's memory instructions is not known to the waits of the next tile
+    }
+    if constexpr (SW_BWD) {
+      if (do_cs) {
+        // group 1 is one barrier behind: when it is through this one, group 0 has arrived at its next and parked its sums long ago
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        pp_barrier();
+        if (wm == 1) {
+          const int g = lane >> 5, col = lane & 31;
+#pragma unroll
+          for (int half = 0; half < 2; ++half) {
+            const int at = wn * 128 + g * 64 + half * 32 + col;
+            const int64_t n = n0 + g * 128 + wn * 32 + col;
+            if (n < p.N) p.colsum[m0 / BM * p.ldc + (half ? p.aux_off : 0) + n] = cs_lds[at] + cs_lds[4 * 128 + at];
+          }
+        }
+      }
     }
     if (!have) break;
   }
@@ -446,6 +500,7 @@ int mvit_gemm_pp(GemmTiledKind kind, const GemmParams& p, int n_cu, hipStream_t 
     case NN_SWIGLU: return go(gemm_pp_kernel<bf16_t, false, false, MVIT_EPI_SWIGLU>, set[4]);
     case NT_NONE: return go(gemm_pp_kernel<bf16_t, false, true, MVIT_EPI_NONE>, set[5]);
     case NT_GELU_BWD: return go(gemm_pp_kernel<bf16_t, false, true, MVIT_EPI_GELU_BWD>, set[6]);
+    case NT_SWIGLU_BWD: return go(gemm_pp_kernel<bf16_t, false, true, MVIT_EPI_SWIGLU_BWD>, set[9]);
     case TT_NONE: return go(gemm_pp_kernel<bf16_t, true, true, MVIT_EPI_NONE>, set[7]);
     case TT_NONE_F32: return go(gemm_pp_kernel<float, true, true, MVIT_EPI_NONE>, set[8]);
     default: return mvit_set_error(MVIT_ERR_UNSUPPORTED, "gemm: product kind %d has no 256 x 256 ping-pong kernel", (int)kind);

@@ -9,6 +9,7 @@
 // step moves 16 KiB into LDS, the 256 x 256 tile's 64 KiB) and put more compute units to work.
 // Fragment layouts, K order, MFMA form and epilogue arithmetic are those of gemm_pp_kernel (gemm_pingpong.hip), so the results
 // are the same bits whichever of the two computed them.
+// SwiGLU backward, 128 x 128 (224 registers: two inputs per element beside the accumulators) / 64 x 128 alone, us at 2,048 rows: 27 / 34.
 // A work-group computes one tile, so bias, residual and saved activations are fetched into registers before the main loop.
 #include "gemm_direct.h"
 
@@ -298,8 +299,9 @@ __device__ __forceinline__ void gemm_small_tile(const GemmParams& p, const unsig
     // a lane's sums over its rows meet those of the 16 lanes and S::WGM waves that share its columns: parked in LDS (rows four
     // floats apart in their banks), added in a fixed order
     if (do_cs) {
-      constexpr int ROWS = S::WGM * 16, PITCH = 2 * NCOLS + 4;
-      static_assert(ROWS * PITCH * 4 <= S::LDS, "the sums fit the operand stages");
+      // tiles of 128 rows give two rows of sums: their two halves are the waves of wm = 0 and 1
+      constexpr int HALVES = BM / 64, ROWS = S::WGM * 16 / HALVES, PITCH = 2 * NCOLS + 4;
+      static_assert(S::WGM % HALVES == 0 && HALVES * ROWS * PITCH * 4 <= S::LDS, "64 rows per row of sums, which fit the operand stages");
       float* red = reinterpret_cast<float*>(smem_raw);
       __syncthreads();  // the last K tile has been consumed
 #pragma unroll
@@ -309,12 +311,12 @@ __device__ __forceinline__ void gemm_small_tile(const GemmParams& p, const unsig
           *reinterpret_cast<f32x4*>(red + (wm * 16 + i16) * PITCH + (h >> 1) * NCOLS + (int)(n_lane[g] - n0) + (h & 1) * 4) =
               f32x4{cs[g][4 * h], cs[g][4 * h + 1], cs[g][4 * h + 2], cs[g][4 * h + 3]};
       __syncthreads();
-      for (int c = threadIdx.x; c < 2 * NCOLS; c += S::NTHREADS) {
-        const int half = c / NCOLS, col = c % NCOLS;
+      for (int c = threadIdx.x; c < HALVES * 2 * NCOLS; c += S::NTHREADS) {
+        const int part = c / (2 * NCOLS), cc = c % (2 * NCOLS), half = cc / NCOLS, col = cc % NCOLS;
         float t = 0.f;
 #pragma unroll
-        for (int r = 0; r < ROWS; ++r) t += red[r * PITCH + c];
-        if (n0 + col < p.N) p.colsum[(int64_t)tm * p.ldc + (half ? p.aux_off : 0) + n0 + col] = t;
+        for (int r = 0; r < ROWS; ++r) t += red[(part * ROWS + r) * PITCH + cc];
+        if (n0 + col < p.N && m0 + part * 64 < p.M) p.colsum[((int64_t)tm * HALVES + part) * p.ldc + (half ? p.aux_off : 0) + n0 + col] = t;
       }
     }
   }
@@ -379,9 +381,7 @@ int dispatch_small(GemmTiledKind kind, const GemmParams& p, hipStream_t s) {
       break;
     case NT_NONE: return launch_small<bf16_t, false, true, MVIT_EPI_NONE, S>(p, s);
     case NT_GELU_BWD: return launch_small<bf16_t, false, true, MVIT_EPI_GELU_BWD, S>(p, s);
-    case NT_SWIGLU_BWD:  // 128 x 128 with two inputs per element would not leave registers for two work-groups per unit
-      if constexpr (S::BM == 64) return launch_small<bf16_t, false, true, MVIT_EPI_SWIGLU_BWD, S>(p, s);
-      break;
+    case NT_SWIGLU_BWD: return launch_small<bf16_t, false, true, MVIT_EPI_SWIGLU_BWD, S>(p, s);
     case TT_NONE: return launch_small<bf16_t, true, true, MVIT_EPI_NONE, S>(p, s);
     case TT_NONE_F32: return launch_small<float, true, true, MVIT_EPI_NONE, S>(p, s);
     default: break;

@@ -539,6 +539,14 @@ def test_swiglu_backward_column_sums_are_of_unrounded_values(M, N, K, per, dtype
     assert bool((part[:, N : N + 8] == 7.0).all()) and bool((out[:, N : N + 8] == 7.0).all())
 
 
+@pytest.mark.parametrize("M,N,K,per", [(1, 72, 136, 256), (255, 264, 192, 256), (257, 136, 192, 256), (513, 520, 136, 256), (2600, 3456, 192, 256),
+                                       (1920, 3456, 192, 64), (1985, 3456, 136, 64), (2047, 3400, 192, 64)])
+def test_swiglu_backward_column_sums_of_longer_contractions(M, N, K, per):
+    """From three K tiles on: 256 x 256 tiles (a tile, parts of one, several per work-group) and 128 x 128 ones (both halves of the
+    last tile, only its first 64 rows and one, a partial half)."""
+    test_swiglu_backward_column_sums_are_of_unrounded_values(M, N, K, per, torch.bfloat16)
+
+
 @pytest.mark.parametrize("unit,offset", [(16, 0), (16, 4), (4, 0), (2, 2), (1, 1)])
 @pytest.mark.parametrize("n", [1, 5, 96, 97, 200])
 def test_copy_ranges_bit_exact(unit, offset, n):
