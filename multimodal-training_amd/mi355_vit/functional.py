@@ -11,6 +11,7 @@ Reference spans (python/models/qwen2_5_vl/modeling_qwen2_5_vl.py):
 from __future__ import annotations
 
 import ctypes
+import math
 import os
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Tuple
@@ -59,6 +60,22 @@ class BlockWeights:
     I: int
     Ipad: int
     alias: bool = False  # norm1 / norm2 / wproj / bproj / bdown are the parameters themselves (same dtype), not copies
+    args: Optional["_lib.BlockArgs"] = None  # the block call's arguments that depend on the weights alone, see block_args
+
+    def block_args(self) -> Optional["_lib.BlockArgs"]:
+        """The weight operands as the C calls take them, filled once per pack and copied per call; None: not laid out for them."""
+        if self.args is None:
+            w = (self.norm1, self.norm2, self.wqkv, self.bqkv, self.wproj, self.bproj, self.wgu, self.bgu, self.wdown, self.bdown)
+            dtype = self.wqkv.dtype
+            if dtype not in ops._DT or not all(t.is_contiguous() and t.dtype == dtype for t in w):
+                return None
+            a = self.args = _lib.BlockArgs()
+            a.dtype, a.C, a.I, a.Ipad = ops._DT[dtype], self.C, self.I, self.Ipad
+            a.norm1, a.norm2, a.wqkv, a.bqkv, a.wproj, a.bproj, a.wgu, a.bgu, a.wdown, a.bdown = (t.data_ptr() for t in w)
+        return self.args
+
+    def __getstate__(self):  # addresses are not copied or saved with the operands
+        return dict(self.__dict__, args=None)
 
 
 # order of the parameter tensors handed to VisionBlockFn
@@ -115,6 +132,7 @@ def pack_block_weights(params: List[torch.Tensor], dtype: torch.dtype, into: Opt
         fill(w, into.wgu[j * Ipad : j * Ipad + I])
         fill(b, into.bgu[:, j * Ipad : j * Ipad + I])
     fill(wd, into.wdown[:, :I])
+    into.args = None
     return into
 
 
@@ -130,82 +148,144 @@ class AttnGeometry:
     sin: torch.Tensor
     order: Optional[torch.Tensor] = None  # device int32 permutation of the segments, longest first (ops.segment_order)
 
+    def block_call_ok(self, x: torch.Tensor) -> bool:
+        """What the call-by-call wrappers check launch by launch of the geometry, once for the block."""
+        S, hd = x.shape[0], self.head_dim
+        return (self.cu.dtype == torch.int32 and self.cu.is_contiguous() and self.cu.device == x.device
+                and all(t.dtype == torch.float32 and tuple(t.shape) == (S, hd) and t.is_contiguous() for t in (self.cos, self.sin))
+                and (self.order is None or (self.order.dtype == torch.int32 and self.order.is_contiguous() and self.order.numel() == self.cu.numel() - 1)))
+
 
 # One C call per block and direction (mvit_block_fwd / mvit_block_bwd) instead of one per kernel: the same launches with
 # the same operands, issued from inside the library.  MVIT_BLOCK_CALLS=0 keeps the call-by-call sequence below, which is
 # also what runs while launches are being timed one by one (ops.set_trace) and for parameters of mixed gradient dtypes.
 BLOCK_CALLS = os.environ.get("MVIT_BLOCK_CALLS", "1") != "0"
 _join_events: dict = {}
+_GRAD_DTYPES = (torch.bfloat16, torch.float32)  # one dtype for all of a block's gradients, as the C call writes them
 
 
 def _block_args(x: torch.Tensor, W: BlockWeights, geo: AttnGeometry, eps: float) -> "_lib.BlockArgs":
-    a = _lib.BlockArgs()
-    a.dtype = ops.dt(x)
-    a.S, a.C, a.I, a.Ipad, a.nheads, a.head_dim = x.shape[0], W.C, W.I, W.Ipad, geo.nheads, geo.head_dim
+    a = _lib.BlockArgs.from_buffer_copy(W.block_args())
+    a.S, a.nheads, a.head_dim = x.shape[0], geo.nheads, geo.head_dim
     a.eps, a.q_lead_scale, a.attn_scale = eps, geo.head_dim**-0.5 * LOG2E, 1.0 / LOG2E
-    a.n_seg, a.max_seqlen = geo.cu.numel() - 1, geo.max_seqlen
-    a.norm1, a.norm2, a.wqkv, a.bqkv, a.wproj = W.norm1.data_ptr(), W.norm2.data_ptr(), W.wqkv.data_ptr(), W.bqkv.data_ptr(), W.wproj.data_ptr()
-    a.bproj, a.wgu, a.bgu, a.wdown, a.bdown = W.bproj.data_ptr(), W.wgu.data_ptr(), W.bgu.data_ptr(), W.wdown.data_ptr(), W.bdown.data_ptr()
+    a.n_seg, a.max_seqlen = geo.cu.shape[0] - 1, geo.max_seqlen
     a.cu, a.cos, a.sin = geo.cu.data_ptr(), geo.cos.data_ptr(), geo.sin.data_ptr()
-    a.seg_order = None if geo.order is None else geo.order.data_ptr()
+    if geo.order is not None:
+        a.seg_order = geo.order.data_ptr()
     a.x = x.data_ptr()
     return a
 
 
 def _block_geometry_ok(x: torch.Tensor, W: BlockWeights, geo: AttnGeometry) -> bool:
     """What the call-by-call wrappers check launch by launch, once for the block: operand layouts the C sequence assumes."""
-    S, hd = x.shape[0], geo.head_dim
-    return (x.is_cuda and x.is_contiguous() and x.shape[1] == W.C and geo.nheads * hd == W.C
-            and geo.cu.dtype == torch.int32 and geo.cu.is_contiguous() and geo.cu.device == x.device
-            and all(t.dtype == torch.float32 and tuple(t.shape) == (S, hd) and t.is_contiguous() for t in (geo.cos, geo.sin))
-            and (geo.order is None or (geo.order.dtype == torch.int32 and geo.order.is_contiguous() and geo.order.numel() == geo.cu.numel() - 1))
-            and all(t.is_contiguous() and t.dtype == x.dtype for t in (W.norm1, W.norm2, W.wqkv, W.bqkv, W.wproj, W.bproj, W.wgu, W.bgu, W.wdown, W.bdown)))
+    return (W.block_args() is not None and x.is_cuda and x.is_contiguous() and x.shape[1] == W.C and geo.nheads * geo.head_dim == W.C
+            and x.dtype == W.wqkv.dtype and geo.block_call_ok(x))
+
+
+class _Buffers:
+    """Pieces of one allocation, each at a 256-byte address: a block's saved activations, or the scratch of its backward.  At few
+    rows an allocation per tensor costs the host more than the kernels cost the GPU."""
+
+    __slots__ = ("buf", "at", "shapes", "dtypes")
+
+    def __init__(self, device, shapes, dtypes):
+        self.shapes, self.dtypes, self.at, end = shapes, dtypes, [], 0
+        for shape, dtype in zip(shapes, dtypes):
+            self.at.append(end)
+            n = dtype.itemsize
+            for d in shape:
+                n *= d
+            end += (n + 255) // 256 * 256
+        self.buf = torch.empty(end, dtype=torch.uint8, device=device)
+
+    def ptr(self, i: int) -> int:
+        return self.buf.data_ptr() + self.at[i]
+
+    def tensor(self, i: int) -> torch.Tensor:
+        shape, dtype = self.shapes[i], self.dtypes[i]
+        return self.buf[self.at[i] : self.at[i] + math.prod(shape) * dtype.itemsize].view(dtype).view(shape)
+
+
+class _Saved:
+    """What a one-call forward keeps for the backward, in the order (rstd1, n1, qkv, o, lse, x1, rstd2, n2, gu, h): addresses for the
+    C call, tensors for whoever asks for one by position or for all of them."""
+
+    __slots__ = ("buffers", "index", "attn")
+
+    def __init__(self, buffers, index, attn):
+        self.buffers, self.index, self.attn = buffers, index, attn  # index: position -> piece (None: not kept); attn: (o, lse) when they are tensors of their own
+
+    def ptr(self, i: int):
+        if self.attn is not None and i in (3, 4):
+            return self.attn[i - 3].data_ptr()
+        piece = self.index[i]
+        return None if piece is None else self.buffers.ptr(piece)
+
+    def __getitem__(self, i: int) -> Optional[torch.Tensor]:
+        if self.attn is not None and i in (3, 4):
+            return self.attn[i - 3]
+        piece = self.index[i]
+        return None if piece is None else self.buffers.tensor(piece)
+
+    def __iter__(self):
+        return (self[i] for i in range(10))
 
 
 def _block_forward_one_call(x, W, geo, eps, attn_out, for_backward, output):
     S, C = x.shape
-    dev, T = x.device, x.dtype
-    f32 = torch.float32
-    n1, x1, n2 = torch.empty_like(x), torch.empty_like(x), torch.empty_like(x)
-    rstd1, rstd2 = torch.empty(S, dtype=f32, device=dev), torch.empty(S, dtype=f32, device=dev)
-    qkv = torch.empty(S, 3 * C, dtype=T, device=dev)
-    if attn_out is None:
-        o, lse = torch.empty_like(x), torch.empty(geo.nheads, S, dtype=f32, device=dev)
+    T, f32, Ipad = x.dtype, torch.float32, W.Ipad
+    if attn_out is None and geo.max_seqlen > KEEP_ATTENTION_ABOVE:  # may outlive the rest
+        attn_out, skip = (torch.empty_like(x), torch.empty(geo.nheads, S, dtype=f32, device=x.device)), 0
     else:
-        o, lse = attn_out
-    gu = torch.empty(S, 2 * W.Ipad, dtype=T, device=dev) if for_backward else None
-    h = torch.empty(S, W.Ipad, dtype=T, device=dev)
+        skip = int(attn_out is not None)
+    shapes, dtypes = [(S,), (S, C), (S, 3 * C), (S, C), (S,), (S, C), (S, Ipad)], [f32, T, T, T, f32, T, T]
+    index = [0, 1, 2, None, None, 3, 4, 5, None, 6]
+    if for_backward:
+        index[8] = len(shapes)
+        shapes.append((S, 2 * Ipad))
+        dtypes.append(T)
+    if attn_out is None:
+        index[3], index[4] = len(shapes), len(shapes) + 1
+        shapes += [(S, C), (geo.nheads, S)]
+        dtypes += [T, f32]
+    saved = _Saved(_Buffers(x.device, shapes, dtypes), index, attn_out)
     x2 = torch.empty_like(x) if output else None
     a = _block_args(x, W, geo, eps)
-    a.skip_attention = int(attn_out is not None)
-    a.n1, a.qkv, a.o, a.x1, a.n2, a.h = n1.data_ptr(), qkv.data_ptr(), o.data_ptr(), x1.data_ptr(), n2.data_ptr(), h.data_ptr()
-    a.rstd1, a.rstd2, a.lse = rstd1.data_ptr(), rstd2.data_ptr(), lse.data_ptr()
-    a.gu, a.x2 = ops._p(gu), ops._p(x2)
+    a.skip_attention = skip
+    p = saved.ptr
+    a.rstd1, a.n1, a.qkv, a.o, a.lse, a.x1, a.rstd2, a.n2, a.gu, a.h = p(0), p(1), p(2), p(3), p(4), p(5), p(6), p(7), p(8), p(9)
+    if output:
+        a.x2 = x2.data_ptr()
     _lib.check(_lib.load().mvit_block_fwd(ctypes.byref(a), ops._stream(x)), "mvit_block_fwd")
-    return x2, (rstd1, n1, qkv, o, lse, x1, rstd2, n2, gu, h)
+    return x2, saved
 
 
-def _block_backward_one_call(dx2, x, saved, W, geo, gdt):
-    rstd1, n1, qkv, o, lse, x1, rstd2, n2, gu, h = saved
+def _block_backward_one_call(dx2, x, saved, W, geo, G):
     S, Cc = x.shape
     I, Ipad = W.I, W.Ipad
     dev, T = x.device, x.dtype
-    G = gdt["norm1.weight"]
-    e = lambda *shape, dtype=T: torch.empty(*shape, dtype=dtype, device=dev)  # noqa: E731
-    dx, dn, dx1 = torch.empty_like(x), torch.empty_like(x), torch.empty_like(x)
-    dgu, dqkv = e(S, 2 * Ipad), e(S, 3 * Cc)
-    g_n1, g_n2, g_bp, g_bd = e(Cc, dtype=G), e(Cc, dtype=G), e(Cc, dtype=G), e(Cc, dtype=G)
-    g_wqkv, g_bqkv = e(3 * Cc, Cc, dtype=G), e(3 * Cc, dtype=G)
-    g_wp, g_wgu, g_bgu, g_wd = e(Cc, Cc, dtype=G), e(2 * Ipad, Cc, dtype=G), e(2 * Ipad, dtype=G), e(Cc, I, dtype=G)
     a = _block_args(x, W, geo, 0.0)
     a.grad_dtype = ops._DT[G]
-    a.n1, a.qkv, a.o, a.x1, a.n2, a.gu, a.h = n1.data_ptr(), qkv.data_ptr(), o.data_ptr(), x1.data_ptr(), n2.data_ptr(), gu.data_ptr(), h.data_ptr()
-    a.rstd1, a.rstd2, a.lse = rstd1.data_ptr(), rstd2.data_ptr(), lse.data_ptr()
-    a.dx2, a.dx, a.dgu, a.dn, a.dx1, a.dqkv = dx2.data_ptr(), dx.data_ptr(), dgu.data_ptr(), dn.data_ptr(), dx1.data_ptr(), dqkv.data_ptr()
-    a.g_norm1, a.g_norm2, a.g_wqkv, a.g_bqkv, a.g_wproj = g_n1.data_ptr(), g_n2.data_ptr(), g_wqkv.data_ptr(), g_bqkv.data_ptr(), g_wp.data_ptr()
-    a.g_bproj, a.g_wgu, a.g_bgu, a.g_wdown, a.g_bdown = g_bp.data_ptr(), g_wgu.data_ptr(), g_bgu.data_ptr(), g_wd.data_ptr(), g_bd.data_ptr()
+    if type(saved) is _Saved:
+        p = saved.ptr
+        a.rstd1, a.n1, a.qkv, a.o, a.lse, a.x1, a.rstd2, a.n2, a.gu, a.h = p(0), p(1), p(2), p(3), p(4), p(5), p(6), p(7), p(8), p(9)
+    else:
+        a.rstd1, a.n1, a.qkv, a.o, a.lse, a.x1, a.rstd2, a.n2, a.gu, a.h = (t.data_ptr() for t in saved)
     sk = ops.wgrad_split_k
     a.split_k_down, a.split_k_gate_up, a.split_k_proj, a.split_k_qkv = sk(Cc, I, S), sk(2 * Ipad, Cc, S), sk(Cc, Cc, S), sk(3 * Cc, Cc, S)
+    lib = _lib.load()
+    nbytes = lib.mvit_block_bwd_workspace_bytes(ctypes.byref(a))
+    scratch = _Buffers(dev, ((S, 2 * Ipad), (S, 3 * Cc), (S, Cc), (S, Cc), (nbytes,)), (T, T, T, T, torch.uint8))
+    a.dgu, a.dqkv, a.dn, a.dx1, a.workspace = scratch.ptr(0), scratch.ptr(1), scratch.ptr(2), scratch.ptr(3), scratch.ptr(4)
+    a.workspace_bytes = nbytes
+    dx = torch.empty_like(x)
+    a.dx2, a.dx = dx2.data_ptr(), dx.data_ptr()
+    e = torch.empty
+    g_n1, g_n2, g_bp, g_bd = e(Cc, dtype=G, device=dev), e(Cc, dtype=G, device=dev), e(Cc, dtype=G, device=dev), e(Cc, dtype=G, device=dev)
+    g_wqkv, g_bqkv = e(3, Cc, Cc, dtype=G, device=dev), e(3, Cc, dtype=G, device=dev)
+    g_wp, g_wgu, g_bgu, g_wd = e(Cc, Cc, dtype=G, device=dev), e(2, Ipad, Cc, dtype=G, device=dev), e(2, Ipad, dtype=G, device=dev), e(Cc, I, dtype=G, device=dev)
+    a.g_norm1, a.g_norm2, a.g_wqkv, a.g_bqkv, a.g_wproj = g_n1.data_ptr(), g_n2.data_ptr(), g_wqkv.data_ptr(), g_bqkv.data_ptr(), g_wp.data_ptr()
+    a.g_bproj, a.g_wgu, a.g_bgu, a.g_wdown, a.g_bdown = g_bp.data_ptr(), g_wgu.data_ptr(), g_bgu.data_ptr(), g_wd.data_ptr(), g_bd.data_ptr()
     side = ops.side_stream(dev)
     if side is not None:
         key = dev.index if dev.index is not None else torch.cuda.current_device()
@@ -216,21 +296,13 @@ def _block_backward_one_call(dx2, x, saved, W, geo, gdt):
                 ev.record()  # an event object gets its handle with its first record
             _join_events[key] = evs
         a.side_stream = side.cuda_stream
-        for i, ev in enumerate(evs):
-            a.events[i] = ev.cuda_event
-    lib = _lib.load()
-    nbytes = lib.mvit_block_bwd_workspace_bytes(ctypes.byref(a))
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-    a.workspace, a.workspace_bytes = ws.data_ptr(), nbytes
+        a.events[:] = [ev.cuda_event for ev in evs]
     _lib.check(lib.mvit_block_bwd(ctypes.byref(a), ops._stream(x)), "mvit_block_bwd")
-    grads = (
-        g_n1, g_n2,
-        g_wqkv[:Cc], g_bqkv[:Cc], g_wqkv[Cc : 2 * Cc], g_bqkv[Cc : 2 * Cc], g_wqkv[2 * Cc :], g_bqkv[2 * Cc :],
-        g_wp, g_bp,
-        g_wgu[:I], g_bgu[:I], g_wgu[Ipad : Ipad + I], g_bgu[Ipad : Ipad + I],
-        g_wd, g_bd,
-    )
-    return dx, grads
+    wq, wk, wv = g_wqkv.unbind(0)
+    bq, bk, bv = g_bqkv.unbind(0)
+    wg, wu = g_wgu[:, :I].unbind(0)
+    bg, bu = g_bgu[:, :I].unbind(0)
+    return dx, (g_n1, g_n2, wq, bq, wk, bk, wv, bv, g_wp, g_bp, wg, bg, wu, bu, g_wd, g_bd)
 
 
 def _block_forward(x: torch.Tensor, W: BlockWeights, geo: AttnGeometry, eps: float,
@@ -275,17 +347,18 @@ def _block_forward(x: torch.Tensor, W: BlockWeights, geo: AttnGeometry, eps: flo
     return x2, (rstd1, n1, qkv, o, lse, x1, rstd2, n2, gu, h)
 
 
-def _block_backward(dx2: torch.Tensor, x: torch.Tensor, saved: tuple, W: BlockWeights, geo: AttnGeometry, gdt: Dict[str, torch.dtype]):
-    """Returns (dx, grads in BLOCK_PARAM_ORDER).  gdt maps parameter name -> gradient dtype."""
+def _block_backward(dx2: torch.Tensor, x: torch.Tensor, saved: tuple, W: BlockWeights, geo: AttnGeometry, gdt):
+    """Returns (dx, grads in BLOCK_PARAM_ORDER).  gdt: the gradients' dtype, or a map parameter name -> gradient dtype."""
+    dx2 = dx2.contiguous()
+    if BLOCK_CALLS and ops._trace is None and gdt in _GRAD_DTYPES and dx2.dtype == x.dtype and _block_geometry_ok(x, W, geo):
+        return _block_backward_one_call(dx2, x, saved, W, geo, gdt)
+    if not isinstance(gdt, dict):
+        gdt = dict.fromkeys(BLOCK_PARAM_ORDER, gdt)
     rstd1, n1, qkv, o, lse, x1, rstd2, n2, gu, h = saved
     S, C = x.shape
     H, hd = geo.nheads, geo.head_dim
     I, Ipad = W.I, W.Ipad
     dev = x.device
-    dx2 = dx2.contiguous()
-    if (BLOCK_CALLS and ops._trace is None and len(set(gdt.values())) == 1 and gdt["norm1.weight"] in ops._DT and dx2.dtype == x.dtype
-            and _block_geometry_ok(x, W, geo)):
-        return _block_backward_one_call(dx2, x, saved, W, geo, gdt)
     main = torch.cuda.current_stream(dev)
     side = ops.side_stream(dev)
 
@@ -363,7 +436,8 @@ class VisionBlockFn(torch.autograd.Function):
         if not differentiated:
             return x2
         ctx.holder, ctx.geo, ctx.eps, ctx.checkpoint = holder, geo, eps, checkpoint
-        ctx.gdt = {name: p.dtype for name, p in zip(BLOCK_PARAM_ORDER, params)}
+        G = params[0].dtype
+        ctx.gdt = G if all([p.dtype is G for p in params]) else {name: p.dtype for name, p in zip(BLOCK_PARAM_ORDER, params)}
         ctx.x = x
         ctx.saved = None if checkpoint else saved
         ctx.attn_out = (saved[3], saved[4]) if checkpoint and geo.max_seqlen > KEEP_ATTENTION_ABOVE else None

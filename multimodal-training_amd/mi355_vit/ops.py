@@ -35,7 +35,9 @@ def side_stream(device: torch.device) -> Optional["torch.cuda.Stream"]:
     units of the input-gradient chain; None while launches are being timed one by one."""
     if not OVERLAP_WGRAD or _trace is not None:
         return None
-    key = torch.device(device).index if torch.device(device).index is not None else torch.cuda.current_device()
+    key = torch.device(device).index
+    if key is None:
+        key = torch.cuda.current_device()
     st = _side_streams.get(key)
     if st is None:
         st = _side_streams[key] = torch.cuda.Stream(device=key)

@@ -379,3 +379,23 @@ def test_benchmark_counts_no_padding_as_work():
                ("gemm_nn_epi4", {"M": 100, "N": ipad, "K": 1280}, Event(), Event())]
     flops = {tag: ent["flops"] for tag, ent in bench.summarise_trace(records, {"intermediate_size": 3420}, None).items()}
     assert flops == {"gemm_tt_epi0": 2.0 * 6840 * 1280 * ipad, "gemm_nn_epi2": 2.0 * ipad * 1280 * 3420, "gemm_nn_epi4": 4.0 * 100 * 3420 * 1280}
+
+
+def test_packed_weights_can_be_copied_and_pickled_after_their_addresses_were_laid_out():
+    """A block's packed operands keep the argument struct of the C calls; copies and pickles lay out their own."""
+    import copy
+    import pickle
+
+    import torch
+
+    from mi355_vit.functional import BlockWeights
+
+    C, I = 16, 24
+    z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16)  # noqa: E731
+    W = BlockWeights(z(1, C), z(1, C), z(3 * C, C), z(1, 3 * C), z(C, C), z(1, C), z(2 * I, C), z(1, 2 * I), z(C, I), z(1, C), C, I, I)
+    assert W.block_args().wqkv == W.wqkv.data_ptr() and W.block_args() is W.block_args()
+    for other in (copy.deepcopy(W), pickle.loads(pickle.dumps(W))):
+        assert other.args is None and other.block_args().wqkv == other.wqkv.data_ptr() != W.wqkv.data_ptr()
+    W.wproj = W.wproj.t()[:, :8]
+    W.args = None
+    assert W.block_args() is None  # not laid out for the C calls: the call-by-call path checks and takes it
