@@ -316,11 +316,14 @@ __global__ __launch_bounds__(64 * NWAVES, MINW) void attn_fwd_mfma(const AttnPar
 #pragma unroll
   for (int j = 0; j < 8; ++j) ones[j] = (bf16_t)1.f;
 
-  TileStager<ND, BNK, G::PK, PIPE ? NT : BNK * G::CH> sk;  // (degenerate when not pipelined)
-  TileStager<ND, BNK, G::PV, PIPE ? NT : BNK * G::CH> sv;
-  if (PIPE) {
+  constexpr bool STAGED = PIPE || QB == 1;  // through registers, all of a tile's loads in flight at once
+  TileStager<ND, BNK, G::PK, STAGED ? NT : BNK * G::CH> sk;  // (degenerate when not)
+  TileStager<ND, BNK, G::PV, STAGED ? NT : BNK * G::CH> sv;
+  if (STAGED) {
     sk.init(p.k_stride);
     sv.init(p.v_stride);
+  }
+  if (PIPE) {
     sk.load(K, min(BNK, L));
     sv.load(V, min(BNK, L));
     sk.store(lds_k[0]);
@@ -339,9 +342,17 @@ __global__ __launch_bounds__(64 * NWAVES, MINW) void attn_fwd_mfma(const AttnPar
         sv.load(V + (int64_t)(k0 + BNK) * p.v_stride, nv);
       }
     } else {
-      if (k0 > 0) __syncthreads();
-      stage_tile<ND, G::PK, NT>(lds_k[0], K + (int64_t)k0 * p.k_stride, p.k_stride, BNK, valid);
-      stage_tile<ND, G::PV, NT>(lds_v[0], V + (int64_t)k0 * p.v_stride, p.v_stride, BNK, valid);
+      if constexpr (STAGED) {
+        sk.load(K + (int64_t)k0 * p.k_stride, valid);
+        sv.load(V + (int64_t)k0 * p.v_stride, valid);
+        if (k0 > 0) __syncthreads();
+        sk.store(lds_k[0]);
+        sv.store(lds_v[0]);
+      } else {
+        if (k0 > 0) __syncthreads();
+        stage_tile<ND, G::PK, NT>(lds_k[0], K + (int64_t)k0 * p.k_stride, p.k_stride, BNK, valid);
+        stage_tile<ND, G::PV, NT>(lds_v[0], V + (int64_t)k0 * p.v_stride, p.v_stride, BNK, valid);
+      }
       __syncthreads();
     }
     const bf16_t* tk = lds_k[PIPE ? buf : 0];
@@ -1969,10 +1980,13 @@ int launch_fwd_mfma(const AttnParams& p, int n_seg, int max_seqlen, hipStream_t 
   const int nw = pick_waves(max_seqlen);
   dim3 grid((unsigned)((max_seqlen + 64 * nw - 1) / (64 * nw)), (unsigned)n_seg, (unsigned)p.nheads);
   if (nw == 1 && ND <= 5) {
-    // windows: two waves x 32 queries share the staged K / V tiles (more waves per CU hide the load latency)
+    // windows: four waves x 16 queries share the staged K / V tiles.  Bound by memory (671 MB at 65,536 rows x 16 heads) and by the
+    // chain load -> products -> store, i.e. by how many waves a compute unit holds: 96 registers, five per SIMD.  Two waves of 32
+    // queries (128 registers, a tile staged load by load) / this, us: 16,384 rows 39.5 / 37.2, 25,524 in windows of 4 ... 64 61.7 / 52.3,
+    // 65,536 177 / 154
     AttnParams pw = p;
     if (grid.x == 1 && ((int64_t)n_seg * p.nheads) % 8 == 0) pw.seg_major = 2;  // heads of a segment together on one XCD
-    if constexpr (ND <= 5) hipLaunchKernelGGL((attn_fwd_mfma<ND, 2, 64, false, 2, 4>), grid, 128, 0, s, pw);
+    if constexpr (ND <= 5) hipLaunchKernelGGL((attn_fwd_mfma<ND, 4, 64, false, 1, 5>), grid, 256, 0, s, pw);
   } else if (nw == 1) hipLaunchKernelGGL((attn_fwd_mfma<ND, 1, 64, false>), grid, 64, 0, s, p);
   else if (nw == 2) hipLaunchKernelGGL((attn_fwd_mfma<ND, 2, 64, false>), grid, 128, 0, s, p);
   else if constexpr (ND <= 5) {
