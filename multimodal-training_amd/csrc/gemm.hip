@@ -1165,7 +1165,10 @@ bool pp_takes(GemmTiledKind kind, int64_t k_chunk, int64_t k_last) {  // at leas
 // Modelled times (us) of the tiles on one MI355X, fitted to every tile's time at 256 ... 16,384 rows of the tower's products: a
 // step of 64 along K takes 1.15 us in a 256 x 256 tile (one work-group per compute unit; 1.2 with both operands behind the
 // transposing LDS read; 2,435 cycles, so more when the clock falls under a long load, which lengthens every tile's steps alike), and in the smaller ones `one` us while every unit has at most one work-group and `two` us once it has
-// two.  A fuller last round, a shorter step and more units at work all lower the estimate; the epilogue of a 256 x 256 tile is
+// two.  Tiles of one work-group per unit (`lone`) interleave loads, LDS reads and MFMAs, so their steps are shorter than those of a
+// single work-group of the kind that shares its unit: 128 x 128 is taken up to 256 tiles and 192 x 128 from there to 256 tiles again
+// (input gradient of 6912 x 1280, us, shared / 128 lone / 192 lone: 2,048 rows 70 / 48 / 61, 3,136 73 / 55 / 65, 4,096 78 / 95 / 68,
+// 6,084 91 / 104 / 127; ms per step before -> with them: 3,136 rows 21.0 -> 19.9, 4,096 checkpointed 29.2 -> 28.0).  A fuller last round, a shorter step and more units at work all lower the estimate; the epilogue of a 256 x 256 tile is
 // the longest.  The line between the tiles follows from these numbers and not from any shape: e.g. weight gradients of
 // 3840 x 1280 over 4,096 rows take 49 us in one slice on 128 x 128 and 57 in three on 256 x 256, over 8,192 rows 93 and 87.
 //
@@ -1180,6 +1183,7 @@ constexpr double PP_STEP_US = 1.15, PP_TILE_US = 7., PP_SWIGLU_TILE_US = 11.;
 struct TileChoice {
   int bm, bn;
   double us;
+  bool lone = false;  // the tile's kernel of one work-group per compute unit
 };
 // The 256-row SwiGLU-backward kernel: gemm_pp_kernel, or gemm_dl_kernel (bm = 0) for a contraction of fewer than three K tiles
 TileChoice full_rows_tile(GemmTiledKind kind, int64_t k_chunk, int64_t k_last) {
@@ -1193,14 +1197,14 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
   const bool fills = 2 * ((M + 255) / 256) * ((N + 255) / 256) >= n_cu;
   const double alone = tt ? 0.5 : ((kind == NT_NONE || kind == NT_GELU_BWD) && fills ? 0.3 : 1.);
   TileChoice best{0, 0, 1e30};
-  auto consider = [&](int bm, int bn, double one, double two, double per_tile) {
+  auto consider = [&](int bm, int bn, double one, double two, double per_tile, bool lone = false) {
     const int64_t items = ((M + bm - 1) / bm) * ((N * n_mul + bn - 1) / bn) * slices;
     const int64_t slots = two > 0. ? 2 * (int64_t)n_cu : n_cu, full = items / slots, rest = items % slots;
     const double round = steps * (two > 0. ? two : one) + per_tile;
     double us = full * round;
     if (rest > 0) us += steps * (two > 0. && rest > n_cu ? two : one) + per_tile;
     us = 4. + alone * us + (1. - alone) * round * (double)items / (double)slots;
-    if (us < best.us) best = TileChoice{bm, bn, us};
+    if (us < best.us) best = TileChoice{bm, bn, us, lone};
   };
   const bool swiglu = kind == NN_SWIGLU;
   if (pp_takes(kind, k_chunk, k_last) && kind != NT_SWIGLU_BWD) consider(256, 256, tt ? 1.2 : PP_STEP_US, 0., swiglu ? PP_SWIGLU_TILE_US : PP_TILE_US);
@@ -1209,9 +1213,14 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
     consider(64, 128, 0.47, 0.70, 2.);
     consider(128, 128, 0.55, 0.90, 5.);
   } else {
-    if (!swiglu) consider(64, 64, 0.23, 0.36, 2.);
+    if (!swiglu) consider(64, 64, tt ? 0.23 : 0.19, 0.36, 2.);
     consider(64, 128, 0.37, 0.52, 2.);
     consider(128, 128, 0.60, 0.72, swiglu ? 6. : 2.5);
+    if (!swiglu && !tt) {
+      consider(64, 64, 0.18, 0., 2., true);
+      consider(128, 128, 0.44, 0., 3., true);
+      consider(192, 128, 0.60, 0., 4., true);
+    }
   }
   // SwiGLU backward: the 256-row kernel as soon as its tiles give nearly half of the units work.  Its launch shares the GPU with
   // the down projection's weight gradient on the second stream, which fills the units it leaves idle, while two small tiles per
@@ -1403,7 +1412,7 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
         q.tiles_n = (int)((q.N + n_cols - 1) / n_cols);
         MVIT_REQUIRE((int64_t)q.tiles_m * q.tiles_n * q.split_k < (1ll << 30), "gemm: too many tiles");
         q.panel_w = q.tiles_n <= 6 ? q.tiles_n : 4;
-        return t.bm == 256 ? mvit_gemm_pp(kind, q, n_cu, s) : mvit_gemm_small(kind, t.bm, t.bn, q, s);
+        return t.bm == 256 ? mvit_gemm_pp(kind, q, n_cu, s) : mvit_gemm_small(kind, t.bm, t.bn, t.lone, q, s);
       };
       const int64_t head = all_256 || p.split_k > 1 ? 0 : rows_in_full_rounds(kind, p.M, p.N, p.K, n_cu);
       if (head > 0) {  // a row's result does not depend on the tile that computes it

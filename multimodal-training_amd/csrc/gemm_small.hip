@@ -1,7 +1,17 @@
 // bf16 GEMM for products with too few 256 x 256 tiles to fill the chip: one work-group per BM x BN tile, NW waves of
 // WM x WN, K tiles of 64 in a ring of NST LDS stages filled by direct global -> LDS loads up to NST - 1 K tiles ahead.
-// Two work-groups share a compute unit: one multiplies while the other waits for LDS or memory (reading the next K tile's
-// fragments ahead inside one work-group, and deeper rings with one work-group per unit, measured no better).
+// Rings of four stages and more: a wave reads the next half K tile's fragments from LDS, and requests its share of the K tile
+// NST - 1 ahead, between the MFMAs of the present half.  Requesting the whole share at once stalls the wave's MFMAs until the
+// address unit has taken it (16 clocks per KiB: half of the step).  us, one step after the other -> interleaved, operands in the
+// cache: 256 rows, K = 3456 on 64 x 64 17.6 -> 13.7, K = 6912 (input gradient) 30.2 -> 25.2; 2,048 rows on 128 x 128, one work-group
+// per unit, 39.4 -> 28, 70 -> 52; MFMAs alone would take 21 and 33.  Moving the reads to the half's beginning, or a fifth stage
+// there, gives nothing.  Loads requested later need more stages: weights from memory, 256 rows, K = 6912, rings of 4 / 6 / 10 stages
+// 35.6 / 34.1 / 35.4 (34.8 with all loads at the beginning of the step and 4), hence Lone64; 64 x 128 with three stages is slower
+// interleaved (SwiGLU of 256 rows 14.7 -> 18.0).
+// Two or three stages (so that two work-groups share a compute unit): one work-group multiplies while the other waits.  The same
+// loop serves the weight gradients (A behind the transposing read) with every ring: interleaved they are no faster (1280 x 1280
+// over 6,084 rows 44.9 / 44.4 us; ms per step 4,096 rows 29.0 / 29.2, 4,900 30.2 / 30.0, 6,084 35.4 / 35.6).  Their tiles that sum A's rows
+// have a loop of their own: a branch in the loop made the others wait too (3840 x 1280 over 6,084 rows 80.7 -> 71.5, over 4,096 58.6 -> 52.7).
 // A wave's tile is as square as its registers allow, because LDS reads are the next limit: 128 x 128 split in eight waves of
 // 32 x 64 read 96 KiB per K tile, in four of 64 x 64 64 KiB (4,096 rows, two transposed-layout operands, K = 6848: 84 -> 77 us;
 // K contiguous in both, K = 3424: 55 -> 52; weight gradient of 3840 x 1280 over 2,048 rows: 32 -> 27).
@@ -13,6 +23,8 @@
 // A work-group computes one tile, so bias, residual and saved activations are fetched into registers before the main loop.
 #include "gemm_direct.h"
 
+#include <type_traits>
+
 namespace {
 
 template <int BM_, int BN_, int WGM_, int WGN_, int NST_>
@@ -21,14 +33,23 @@ struct SmallCfg {
   static constexpr int NW = WGM * WGN, NTHREADS = 64 * NW, WM = BM / WGM, WN = BN / WGN;
   static constexpr int A_BYTES = BM * BK * 2, STAGE = (BM + BN) * BK * 2, LDS = NST * STAGE;
   static constexpr int PER_A = BM / 8 / NW, PER_B = BN / 8 / NW, PER = PER_A + PER_B;  // 1 KiB loads per wave and K tile
-  static_assert(NST >= 2 && NST <= 4 && (BM == 64 || BM == 128) && (BN == 64 || BN == 128), "ring depths and swizzles built");
+  static_assert(NST >= 2 && (NST - 2) * PER < 64 && (BM == 64 || BM == 128 || BM == 192) && (BN == 64 || BN == 128), "ring depths and swizzles built");
   static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0 && WM % 16 == 0 && WN % 32 == 0, "whole load instructions and MFMA blocks per wave");
 };
+
+template <int PER, int MOST>
+__device__ __forceinline__ void wait_tiles(int in_flight) {
+  if constexpr (MOST > 0) {
+    if (in_flight < MOST) return wait_tiles<PER, MOST - 1>(in_flight);
+  }
+  pp_wait_vm<MOST * PER>();
+}
 
 // chunk (16 bytes) swizzle of a staged operand: [row][k] tiles by row, [k][row] tiles of ROWS rows by k
 template <bool TR, bool IS_A, int ROWS>
 __device__ __forceinline__ int small_swizzle(int major) {
   if (!TR) return IS_A ? (major >> 1) & 7 : ((major >> 1) & 1) | (((major >> 3) & 3) << 1);
+  static_assert(!TR || ROWS == 64 || ROWS == 128, "rows of a [k][row] tile");
   if (ROWS == 64) return (((major >> 1) & 1) << 1) | (((major >> 3) & 1) << 2);
   return ((major & 3) << 1) | (((major >> 3) & 1) << 3);
 }
@@ -180,10 +201,11 @@ __device__ __forceinline__ void gemm_small_tile(const GemmParams& p, const unsig
     }
   }
 
+  constexpr bool INTERLEAVED = NST >= 4 && !TA;
   // sums of A's rows over k, see gemm_pingpong.hip: wave wn of a row group takes NRS row blocks, two MFMAs more each per K tile
   constexpr bool ROW_SUMS = TA && TB && EPI == MVIT_EPI_NONE;
   constexpr int NRS = NA / S::WGN;  // row blocks that a wave sums
-  static_assert(!ROW_SUMS || NA % S::WGN == 0, "the waves of a row group share its row blocks");
+  static_assert(!ROW_SUMS || (NA % S::WGN == 0 && !INTERLEAVED), "the waves of a row group share its row blocks");
   const bool do_rs = ROW_SUMS && p.row_sums != nullptr && tn == 0;
   [[maybe_unused]] f32x4 rs[ROW_SUMS ? NRS : 1];
 #pragma unroll
@@ -196,51 +218,113 @@ __device__ __forceinline__ void gemm_small_tile(const GemmParams& p, const unsig
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
   unsigned st = 0, st_in = (NST - 1) * S::STAGE;  // stage consumed, stage filled
-  for (int t = 0; t < n_kt; ++t) {
-    // K tile t has landed once only tiles requested after it are in flight
-    const int newer = n_kt - 1 - t;
-    if (newer >= NST - 2) pp_wait_vm<(NST - 2) * S::PER>();
-    else if (NST > 3 && newer == 1) pp_wait_vm<S::PER>();
-    else pp_wait_vm<0>();
-    pp_barrier();  // every wave's share of K tile t is in LDS; K tile t - 1 has been consumed
-    if (t + NST - 1 < n_kt) issue(t + NST - 1, st_in);
-    const unsigned char* at = smem_raw + st;
-    bf16x8 fa[NA][2], fb[NB][2];
+  bf16x8 fa[2][NA], fb[2][NB];                    // fragments of the two halves of a K tile
+  auto read_a = [&](const unsigned char* at, int ks, int a) {
+    if constexpr (!TA) fa[ks][a] = *reinterpret_cast<const bf16x8*>(at + ra[ks] + a * 2048);
+    else fa[ks][a] = pp_read_tr(at + ra[a] + ks * 32 * (BM * 2), 4 * (BM * 2));
+  };
+  auto read_b = [&](const unsigned char* at, int ks, int b) {
+    if constexpr (!TB) fb[ks][b] = *reinterpret_cast<const bf16x8*>(at + rb[ks] + (b >> 1) * 4096 + (b & 1) * 512);
+    else fb[ks][b] = pp_read_tr(at + rb[b] + ks * 32 * (BN * 2), 4 * (BN * 2));
+  };
+  auto multiply_row = [&](int ks, int a) {
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        if constexpr (!TB) fb[b][ks] = *reinterpret_cast<const bf16x8*>(at + rb[ks] + (b >> 1) * 4096 + (b & 1) * 512);
-        else fb[b][ks] = pp_read_tr(at + rb[b] + ks * 32 * (BN * 2), 4 * (BN * 2));
-      }
+    for (int b = 0; b < NB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[ks][b], fa[ks][a], acc[a][b], 0, 0, 0);
+  };
+  auto landed = [&](int newer) {  // this wave's share of a K tile has landed once only the `newer` tiles requested after it are in flight
+    wait_tiles<S::PER, NST - 2>(newer);
+  };
+  auto next_stage = [&](unsigned& stage) { stage = stage + S::STAGE == S::LDS ? 0 : stage + S::STAGE; };
+  if constexpr (INTERLEAVED) {
+    constexpr int FIRST = S::PER / 2;  // loads requested in the first half
+    // half `ks` of a K tile: its MFMAs row by row, between them the reads of the half after it (at `next`) and loads into stage_off.
+    // The compiler keeps to this order.
+    auto half = [&](auto half_ks, auto with_loads, const unsigned char* next, unsigned stage_off) {
+      constexpr int ks = decltype(half_ks)::value, LOADS = !decltype(with_loads)::value ? 0 : ks ? S::PER - FIRST : FIRST, READS = NA + NB;
 #pragma unroll
       for (int a = 0; a < NA; ++a) {
-        if constexpr (!TA) fa[a][ks] = *reinterpret_cast<const bf16x8*>(at + ra[ks] + a * 2048);
-        else fa[a][ks] = pp_read_tr(at + ra[a] + ks * 32 * (BM * 2), 4 * (BM * 2));
+#pragma unroll
+        for (int i = a * LOADS / NA; i < (a + 1) * LOADS / NA; ++i) {
+          const int j = ks * FIRST + i;
+          if (j < S::PER_A) pp_load(lds_base + stage_off + (wv * S::PER_A + j) * 1024, va[j], ba);
+          else pp_load(lds_base + stage_off + S::A_BYTES + (wv * S::PER_B + j - S::PER_A) * 1024, vb[j - S::PER_A], bb);
+        }
+#pragma unroll
+        for (int r = a * READS / NA; r < (a + 1) * READS / NA; ++r) {
+          if (r < NB) read_b(next, 1 - ks, r);
+          else read_a(next, 1 - ks, r - NB);
+        }
+        multiply_row(ks, a);
+        __builtin_amdgcn_sched_barrier(0);
       }
+    };
+    constexpr std::integral_constant<int, 0> first{};
+    constexpr std::integral_constant<int, 1> second{};
+    landed(n_kt - 1);
+    pp_barrier();
+#pragma unroll
+    for (int b = 0; b < NB; ++b) read_b(smem_raw, 0, b);
+#pragma unroll
+    for (int a = 0; a < NA; ++a) read_a(smem_raw, 0, a);
+    // The barrier between the halves of K tile t: every wave's share of tile t + 1 has landed, and every wave has read all of tile t,
+    // whose stage tile t + NST overwrites from the next step on.  The last step's reads past the end stay in the ring and are not used.
+    int t = 0;
+    for (const int whole = n_kt - (NST - 1) - (k_tail != 0 ? 1 : 0); t < whole; ++t) {  // tile t + NST - 1 exists and is a whole one
+      half(first, std::true_type{}, smem_raw + st, st_in);
+      next_stage(st);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      pp_wait_vm<(NST - 3) * S::PER + FIRST>();
+      pp_barrier();
+      half(second, std::true_type{}, smem_raw + st, st_in);
+      next_stage(st_in);
+      ba += step_a;
+      bb += step_b;
     }
-    __builtin_amdgcn_sched_barrier(0);
+    for (; t < n_kt; ++t) {
+      if (t + NST - 1 < n_kt) issue(t + NST - 1, st_in);
+      half(first, std::false_type{}, smem_raw + st, 0);
+      next_stage(st);
+      next_stage(st_in);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      landed(n_kt - 2 - t);
+      pp_barrier();
+      half(second, std::false_type{}, smem_raw + st, 0);
+    }
+  } else {
+    auto loop = [&](auto with_row_sums) {
+      for (int t = 0; t < n_kt; ++t) {
+        landed(n_kt - 1 - t);
+        pp_barrier();  // every wave's share of K tile t is in LDS; K tile t - 1 has been consumed
+        if (t + NST - 1 < n_kt) issue(t + NST - 1, st_in);
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
+        for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
-      for (int a = 0; a < NA; ++a)
+          for (int b = 0; b < NB; ++b) read_b(smem_raw + st, ks, b);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[b][ks], fa[a][ks], acc[a][b], 0, 0, 0);
-    if constexpr (ROW_SUMS) {
-      if (do_rs) {
-        const bf16_t one = (bf16_t)1.f;
-        const bf16x8 ones = {one, one, one, one, one, one, one, one};
+          for (int a = 0; a < NA; ++a) read_a(smem_raw + st, ks, a);
+        }
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int a = 0; a < NA; ++a)
-          if (wn == a / NRS) {
+        for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) rs[a % NRS] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, fa[a][ks], rs[a % NRS], 0, 0, 0);
-          }
+          for (int a = 0; a < NA; ++a) multiply_row(ks, a);
+        if constexpr (decltype(with_row_sums)::value) {
+          const bf16_t one = (bf16_t)1.f;
+          const bf16x8 ones = {one, one, one, one, one, one, one, one};
+#pragma unroll
+          for (int a = 0; a < NA; ++a)
+            if (wn == a / NRS) {
+#pragma unroll
+              for (int ks = 0; ks < 2; ++ks) rs[a % NRS] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, fa[ks][a], rs[a % NRS], 0, 0, 0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        next_stage(st);
+        next_stage(st_in);
       }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    st = st + S::STAGE == S::LDS ? 0 : st + S::STAGE;
-    st_in = st_in + S::STAGE == S::LDS ? 0 : st_in + S::STAGE;
+    };
+    if (ROW_SUMS && do_rs) loop(std::bool_constant<ROW_SUMS>{});
+    else loop(std::false_type{});
   }
 
   // ---- epilogue
@@ -334,9 +418,13 @@ __global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_group_kerne
   gemm_small_tile<TO, TA, TB, EPI, S>(g.p[i], blockIdx.x - g.first_block[i]);
 }
 
-using Small64 = SmallCfg<64, 64, 2, 2, 4>;      // 64 KiB of LDS
+using Small64 = SmallCfg<64, 64, 2, 2, 4>;       // 64 KiB of LDS
 using Small64x128 = SmallCfg<64, 128, 2, 2, 3>;  // 72 KiB
 using Small128 = SmallCfg<128, 128, 2, 2, 2>;    // 64 KiB
+// one work-group per compute unit, which has work for one at most
+using Lone64 = SmallCfg<64, 64, 2, 2, 6>;     // 96 KiB
+using Lone128 = SmallCfg<128, 128, 2, 2, 4>;  // 128 KiB
+using Lone192 = SmallCfg<192, 128, 2, 2, 4>;  // 160 KiB
 
 template <typename S, typename P>
 int launch_grid(void (*kern)(P), const P& p, unsigned grid, bool (&attr_set_on)[MVIT_MAX_DEVICES], hipStream_t stream) {
@@ -389,9 +477,25 @@ int dispatch_small(GemmTiledKind kind, const GemmParams& p, hipStream_t s) {
   return mvit_set_error(MVIT_ERR_UNSUPPORTED, "gemm: product kind %d has no %d x %d kernel", (int)kind, S::BM, S::BN);
 }
 
+// the tiles of which one work-group fills a compute unit: products with one operand or none behind the transposing LDS read
+template <typename S>
+int dispatch_lone(GemmTiledKind kind, const GemmParams& p, hipStream_t s) {
+  switch (kind) {
+    case NN_NONE: return launch_small<bf16_t, false, false, MVIT_EPI_NONE, S>(p, s);
+    case NN_BIAS: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS, S>(p, s);
+    case NN_BIAS_RES: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_RES, S>(p, s);
+    case NN_BIAS_GELU: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_GELU, S>(p, s);
+    case NT_NONE: return launch_small<bf16_t, false, true, MVIT_EPI_NONE, S>(p, s);
+    case NT_GELU_BWD: return launch_small<bf16_t, false, true, MVIT_EPI_GELU_BWD, S>(p, s);
+    default: break;
+  }
+  return mvit_set_error(MVIT_ERR_UNSUPPORTED, "gemm: product kind %d has no %d x %d kernel of one work-group per unit", (int)kind, S::BM, S::BN);
+}
+
 }  // namespace
 
-int mvit_gemm_small(GemmTiledKind kind, int bm, int bn, const GemmParams& p, hipStream_t stream) {
+int mvit_gemm_small(GemmTiledKind kind, int bm, int bn, bool lone, const GemmParams& p, hipStream_t stream) {
+  if (lone) return bm == 192 ? dispatch_lone<Lone192>(kind, p, stream) : bm == 128 ? dispatch_lone<Lone128>(kind, p, stream) : dispatch_lone<Lone64>(kind, p, stream);
   if (bm == 128) return dispatch_small<Small128>(kind, p, stream);
   if (bn == 128) return dispatch_small<Small64x128>(kind, p, stream);
   return dispatch_small<Small64>(kind, p, stream);

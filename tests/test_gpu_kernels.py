@@ -441,6 +441,44 @@ def test_gemm_rows_in_full_rounds_and_the_rest_give_the_same_bits_as_one_launch(
         assert max_rel_err(split[0][:M], want) < TOL[dtype]
 
 
+# rows whose tiles are 64 x 64 and 64 x 128, the ring of stages never full, once full, refilled, with and without a partial last K tile ...
+_RING_SHAPES = [(70, 200, k) for k in (8, 64, 72, 128, 136, 192, 200, 256, 264, 320)] + [(1500, 1288, k) for k in (8, 64, 72, 136, 192, 264)]
+# ... and one work-group per unit: 128 x 128 up to 256 tiles, 192 x 128 from there to 256 tiles
+_RING_SHAPES += [(1700, 1280, 1288), (3200, 1280, 840), (3201, 1280, 840), (3277, 1280, 1280), (4800, 1280, 1288), (4801, 1280, 840)]
+
+
+@pytest.mark.parametrize("form", ["nn", "nn bias_res", "nn gelu", "nt", "nt gelu_bwd", "tt"])
+@pytest.mark.parametrize("M,N,K", _RING_SHAPES)
+def test_gemm_of_few_rows_over_the_edges_of_its_ring_and_tiles(M, N, K, form, monkeypatch):
+    _announce(f"gemm ring {form} {M}x{N}x{K}")
+    ops = _ops()
+    from mi355_vit import _lib as E
+
+    dtype = torch.bfloat16
+    ta, tb = form == "tt", form[:2] != "nn"
+    a = _rand((K, (M + 7) // 8 * 8) if ta else (M, K), dtype, 1, K**-0.5).to(DEV)[:, :M if ta else K]
+    b = _rand((K, N) if tb else (N, K), dtype, 2).to(DEV)
+    bias, res = _rand((N,), dtype, 3).to(DEV), _rand((M, N), dtype, 4).to(DEV)
+    kw = {"nn bias_res": dict(epilogue=E.EPI_BIAS_RES, bias=bias, residual=res), "nn gelu": dict(epilogue=E.EPI_BIAS_GELU, bias=bias, aux=torch.empty_like(res)),
+          "nt gelu_bwd": dict(epilogue=E.EPI_GELU_BWD, residual=res)}.get(form, {})
+
+    def run():
+        out = torch.full((M + 8, N), 7.0, dtype=dtype, device=DEV)
+        ops.gemm(a, b, out[:M], trans_a=ta, trans_b=tb, **kw)
+        return out
+
+    got = run()
+    assert bool((got[M:] == 7.0).all())
+    x = (a.T if ta else a).double() @ (b if tb else b.T).double()
+    r = res.double()
+    want = {"nn bias_res": lambda: x + bias.double() + r, "nn gelu": lambda: torch.nn.functional.gelu(x + bias.double()),
+            "nt gelu_bwd": lambda: x * (0.5 * (1 + torch.erf(r * 0.5**0.5)) + r * torch.exp(-r * r / 2) / (2 * torch.pi) ** 0.5)}.get(form, lambda: x)()
+    assert max_rel_err(got[:M], want.cpu()) < TOL[dtype]
+    if K > 128:  # every tile gives the same bits
+        monkeypatch.setenv("MVIT_GEMM_NO_HALF_TILES", "1")
+        assert torch.equal(got, run())
+
+
 @pytest.mark.parametrize("dtype,odt", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32)])
 @pytest.mark.parametrize("S,No,Ni", [(1000, 1280, 1280), (515, 3840, 256), (70, 6848, 1280), (2052, 1280, 3420)])
 def test_gemm_wgrad_layout(dtype, odt, S, No, Ni):
