@@ -242,30 +242,30 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
     __builtin_amdgcn_s_setprio(0);
   };
   bool do_rs = false;  // this output tile also sums A's rows
+  // (a loop of their own for these tiles: the branch inside the K loop cost the other tiles up to 2 %, 6912 x 1280 over 14,336 rows 260 -> 256 us,
+  // and a step of 9,600 rows 49.2 -> 48.6 ms, of 25,524 114.3 -> 113.7)
   // row block wn of the group's four in each A half, one accumulator per half: every lane's element 0 is the sum of row l % 16.
   // The first operand is ones throughout, so a row's sum reads that row alone (zeros standing for "the other half's rows" would
   // carry its infinities and NaNs over: 0 x Inf)
   [[maybe_unused]] f32x4 rs[2];
-  auto row_sums = [&](auto H) {
-    if constexpr (ROW_SUMS) {
-      if (do_rs) {
-        unsigned o = 0x3f803f80u;
-        asm volatile("" : "+v"(o));  // made where it is used rather than held in registers
-        const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{o, o, o, o});
+  auto row_sums = [&](auto H, auto RS) {
+    if constexpr (decltype(RS)::value) {
+      unsigned o = 0x3f803f80u;
+      asm volatile("" : "+v"(o));  // made where it is used rather than held in registers
+      const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{o, o, o, o});
 #pragma unroll
-        for (int a = 0; a < 4; ++a)
-          if (wn == a) {
+      for (int a = 0; a < 4; ++a)
+        if (wn == a) {
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-              f32x4& c = rs[decltype(H)::value];
-              c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, fa[a][ks], c, 0, 0, 0);
-            }
+          for (int ks = 0; ks < 2; ++ks) {
+            f32x4& c = rs[decltype(H)::value];
+            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, fa[a][ks], c, 0, 0, 0);
           }
-      }
+        }
     }
   };
   // K tile t.  MODE 0: steady, 1: first of the output tile, 2: last but one, 3: last
-  auto ktile = [&](auto MODE_, int t) {
+  auto ktile = [&](auto MODE_, int t, auto RS) {
     constexpr int MODE = decltype(MODE_)::value;
     constexpr int W = MODE == 1 ? (8 + TRAILING < 63 ? 8 + TRAILING : 63) : 8;
     using F = std::integral_constant<bool, MODE == 1>;
@@ -285,7 +285,7 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
     pp_wait_vm<MODE == 3 ? 0 : W>();
     pp_barrier();
     mfma(X0{}, X1{}, fb[1], F{});
-    row_sums(X0{});
+    row_sums(X0{}, RS);
     pp_barrier();
     // phase 2
     read_a(fa, 1);
@@ -299,7 +299,7 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
     if constexpr (MODE != 3) pp_wait_vm<MODE == 2 ? 4 : W>();
     pp_barrier();
     mfma(X1{}, X0{}, fb[0], F{});
-    row_sums(X1{});
+    row_sums(X1{}, RS);
     pp_barrier();
     st = other;
   };
@@ -321,10 +321,14 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
     pp_wait_vm<(8 + TRAILING < 63 ? 8 + TRAILING : 63)>();
     pp_barrier();
     pp_barrier();
-    ktile(X1{}, 0);
-    for (int t = 1; t < n_kt - 2; ++t) ktile(X0{}, t);
-    ktile(X2{}, n_kt - 2);
-    ktile(X3{}, n_kt - 1);
+    auto ktiles = [&](auto RS) {
+      ktile(X1{}, 0, RS);
+      for (int t = 1; t < n_kt - 2; ++t) ktile(X0{}, t, RS);
+      ktile(X2{}, n_kt - 2, RS);
+      ktile(X3{}, n_kt - 1, RS);
+    };
+    if (ROW_SUMS && do_rs) ktiles(std::integral_constant<bool, ROW_SUMS>{});
+    else ktiles(std::false_type{});
     idx += gridDim.x >> 3;
     const bool have = start_tile(idx);
     if (have && !HAS_IN) issue_first();
