@@ -7,9 +7,14 @@
 // per compute unit.  MFMA (s, j) of a K tile contracts k = 16 s + 4 g + j over the lane groups g = 0..3, so one 16-byte read
 // of a [row][k] operand feeds four of them; a [k][row] operand is read as two neighbouring rows (8 bytes) per k, and the two
 // row blocks of a wave are its even and its odd rows.
+// Loads, the LDS reads of the next half K tile and MFMAs alternate: one after the other, a wave's MFMAs waited for its requests
+// and its reads (us: 512 rows K = 1280 x 3840 48.6 -> 44.6, input gradient K = 6912 137 -> 121, its weight gradient 92 -> 80; 2,048
+// rows 340 -> 293, 337 -> 292, i.e. 123 TFLOP/s; 4-block step of 512 rows 4.00 -> 3.62 ms, of 2,048 11.8 -> 10.3).
 // The products are computed transposed (B's fragment first), so a lane ends with eight consecutive columns of a row and
 // stores them from registers.  Both tiles add in the same order: a row's result does not depend on its batch.
 #include "gemm_direct.h"
+
+#include <type_traits>
 
 namespace {
 
@@ -135,58 +140,89 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmParams p) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
   unsigned st = 0, st_in = (NST - 1) * S::STAGE;  // stage consumed, stage filled
-  for (int t = 0; t < n_kt; ++t) {
-    const int newer = n_kt - 1 - t;  // K tiles that may still be in flight
-    if (newer >= 2) pp_wait_vm<2 * S::PER>();
-    else if (newer == 1) pp_wait_vm<S::PER>();
-    else pp_wait_vm<0>();
-    pp_barrier();  // every wave's share of K tile t is in LDS; K tile t - 1 has been consumed
-    if (t + NST - 1 < n_kt) issue(t + NST - 1, st_in);
-    const unsigned char* at = smem_raw + st;
-    float fa[NA][8], fb[NB][8];  // [block][4 s + j]
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
+  float fa[NA][8], fb[NB][8];                     // [block][4 s + j], s the half of the K tile
+  constexpr int READS_A = TA ? 4 : NA, READS_B = TB ? 4 : NB, READS = READS_A + READS_B;
+  auto read = [&](const unsigned char* at, int s, int r) {  // the r-th read of half s
+    if (r < READS_A) {
       if constexpr (!TA) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(at + ra[s] + r * 2048);
 #pragma unroll
-        for (int a = 0; a < NA; ++a) {
-          const f32x4 v = *reinterpret_cast<const f32x4*>(at + ra[s] + a * 2048);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) fa[a][4 * s + j] = v[j];
-        }
+        for (int j = 0; j < 4; ++j) fa[r < NA ? r : 0][4 * s + j] = v[j];
       } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const f32x2 v = *reinterpret_cast<const f32x2*>(at + ra[0] + (16 * s + j) * 256);
-          fa[0][4 * s + j] = v[0];
-          fa[NA - 1][4 * s + j] = v[1];
-        }
+        const f32x2 v = *reinterpret_cast<const f32x2*>(at + ra[0] + (16 * s + r) * 256);
+        fa[0][4 * s + r] = v[0];
+        fa[NA - 1][4 * s + r] = v[1];
       }
+    } else {
+      r -= READS_A;
       if constexpr (!TB) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(at + rb[s] + (r >> 1) * 4096 + (r & 1) * 512);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-          const f32x4 v = *reinterpret_cast<const f32x4*>(at + rb[s] + (b >> 1) * 4096 + (b & 1) * 512);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) fb[b][4 * s + j] = v[j];
-        }
+        for (int j = 0; j < 4; ++j) fb[r < NB ? r : 0][4 * s + j] = v[j];
       } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const f32x2 v = *reinterpret_cast<const f32x2*>(at + rb[0] + (16 * s + j) * 256);
-          fb[0][4 * s + j] = v[0];
-          fb[NB - 1][4 * s + j] = v[1];
-        }
+        const f32x2 v = *reinterpret_cast<const f32x2*>(at + rb[0] + (16 * s + r) * 256);
+        fb[0][4 * s + r] = v[0];
+        fb[NB - 1][4 * s + r] = v[1];
       }
     }
-    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr int FIRST = S::PER / 2;  // loads requested in the first half
+  auto half = [&](auto half_s, auto with_loads, const unsigned char* next, unsigned stage_off) {
+    constexpr int s = decltype(half_s)::value, LOADS = !decltype(with_loads)::value ? 0 : s ? S::PER - FIRST : FIRST;
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
+    for (int k = 0; k < 4; ++k) {
+#pragma unroll
+      for (int i = k * LOADS / 4; i < (k + 1) * LOADS / 4; ++i) {
+        const int j = s * FIRST + i;
+        if (j < S::PER_A) {
+          pp_load_at(lds_base + stage_off + (wv * S::PER_A + j) * 1024, pa[j]);
+          pa[j] += step_a;
+        } else {
+          pp_load_at(lds_base + stage_off + S::A_BYTES + (wv * S::PER_B + j - S::PER_A) * 1024, pb[j - S::PER_A]);
+          pb[j - S::PER_A] += step_b;
+        }
+      }
+#pragma unroll
+      for (int r = k * READS / 4; r < (k + 1) * READS / 4; ++r) read(next, 1 - s, r);
 #pragma unroll
       for (int a = 0; a < NA; ++a)
 #pragma unroll
-        for (int b = 0; b < NB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[b][k], fa[a][k], acc[a][b], 0, 0, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    st = st + S::STAGE == S::LDS ? 0 : st + S::STAGE;
-    st_in = st_in + S::STAGE == S::LDS ? 0 : st_in + S::STAGE;
+        for (int b = 0; b < NB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[b][4 * s + k], fa[a][4 * s + k], acc[a][b], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto landed = [&](int newer) {  // this wave's share of a K tile has landed once only the `newer` tiles requested after it are in flight
+    if (newer >= 2) pp_wait_vm<2 * S::PER>();
+    else if (newer == 1) pp_wait_vm<S::PER>();
+    else pp_wait_vm<0>();
+  };
+  auto next_stage = [&](unsigned& stage) { stage = stage + S::STAGE == S::LDS ? 0 : stage + S::STAGE; };
+  constexpr std::integral_constant<int, 0> first{};
+  constexpr std::integral_constant<int, 1> second{};
+  landed(n_kt - 1);
+  pp_barrier();
+#pragma unroll
+  for (int r = 0; r < READS; ++r) read(smem_raw, 0, r);
+  // the barrier between the halves of K tile t: every wave's share of tile t + 1 has landed, and every wave has read all of tile t
+  int t = 0;
+  for (const int whole = n_kt - (NST - 1) - (k_tail != 0 ? 1 : 0); t < whole; ++t) {  // tile t + NST - 1 exists and is a whole one
+    half(first, std::true_type{}, smem_raw + st, st_in);
+    next_stage(st);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    pp_wait_vm<(NST - 3) * S::PER + FIRST>();
+    pp_barrier();
+    half(second, std::true_type{}, smem_raw + st, st_in);
+    next_stage(st_in);
+  }
+  for (; t < n_kt; ++t) {
+    if (t + NST - 1 < n_kt) issue(t + NST - 1, st_in);
+    half(first, std::false_type{}, smem_raw + st, 0);
+    next_stage(st);
+    next_stage(st_in);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    landed(n_kt - 2 - t);
+    pp_barrier();
+    half(second, std::false_type{}, smem_raw + st, 0);
   }
 
   // ---- epilogue: the lane holds columns 8 g .. 8 g + 7 of each 32-column group, one row per row block
@@ -222,9 +258,9 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmParams p) {
 }
 
 // 32-row tiles where they shorten the launch: while 64-row tiles leave a quarter of the compute units without one, and after that
-// where halving saves part of the last round (us, 64 / 32 rows, input gradients: K = 1280 30 / 21 at 256 rows, 49 / 43 at 1,024,
-// 50 / 58 at 1,536, 76 / 68 at 2,048; K = 6912 145 / 99 at 256 rows, 145 / 140 at 512).  Nearly a tile per unit stays whole: halves
-// are no faster alone (256 rows x 3840: 32 / 31), and beside a second stream's products a step of 256 rows takes 3.19 ms with
+// where halving saves part of the last round (us, 64 / 32 rows, input gradients: K = 1280 27 / 17 at 256 rows, 45 / 36 at 1,024,
+// 45 / 49 at 1,536, 66 / 58 at 2,048; K = 6912 126 / 77 at 256 rows, 127 / 121 at 512).  Nearly a tile per unit stays whole: halves
+// are hardly faster alone (256 rows x 3840: 28.5 / 27.6), and beside a second stream's products a step of 256 rows took 3.19 ms with
 // them and 2.97 without.
 inline bool half_rows(const GemmParams& p) {
   constexpr int64_t units = 256;

@@ -479,6 +479,25 @@ def test_gemm_of_few_rows_over_the_edges_of_its_ring_and_tiles(M, N, K, form, mo
         assert torch.equal(got, run())
 
 
+@pytest.mark.parametrize("form", ["nn", "nt", "tt"])
+@pytest.mark.parametrize("K", [4, 32, 36, 64, 96, 100, 128, 132, 160, 164, 1284])
+@pytest.mark.parametrize("M,N", [(40, 72), (452, 1280)])
+def test_fp32_gemm_over_the_edges_of_its_ring(M, N, K, form):
+    """K tiles of 32 in a ring of four stages: never full, once full, refilled, with and without a partial last tile."""
+    _announce(f"fp32 gemm ring {form} {M}x{N}x{K}")
+    ops = _ops()
+    ta, tb = form == "tt", form != "nn"
+    a = _rand((K, M) if ta else (M, K), torch.float32, 1, K**-0.5).to(DEV)
+    b = _rand((K, N) if tb else (N, K), torch.float32, 2).to(DEV)
+    out = torch.full((M + 8, N), 7.0, device=DEV)
+    ops.gemm(a, b, out[:M], trans_a=ta, trans_b=tb)
+    assert bool((out[M:] == 7.0).all())
+    want = (a.T if ta else a).double() @ (b if tb else b.T).double()
+    # sums of K products in 32 bits: each of the K additions rounds to 2^-24 of a partial sum that |a| |b| bounds
+    bound = (a.T if ta else a).double().abs() @ (b if tb else b.T).double().abs() * K * 2.0**-24
+    assert bool(((out[:M].double() - want).abs() <= bound + 1e-30).all())
+
+
 @pytest.mark.parametrize("dtype,odt", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32)])
 @pytest.mark.parametrize("S,No,Ni", [(1000, 1280, 1280), (515, 3840, 256), (70, 6848, 1280), (2052, 1280, 3420)])
 def test_gemm_wgrad_layout(dtype, odt, S, No, Ni):
