@@ -53,6 +53,32 @@ def test_merge_and_backward_bit_exact(dtype, B, T, frac, hidden):
     assert torch.equal(out.detach(), ref)
 
 
+@pytest.mark.parametrize("n", [0, 1, 63, 64, 511, 512, 513, 8191, 8192, 8193, 16384, 20001])
+@pytest.mark.parametrize("with_labels", [True, False])
+def test_ranks_over_the_edges_of_waves_and_spans(n, with_labels):
+    """A wave takes 512 tokens, the work-group 8,192 at a time: ranks, positions and both counts are exact around those edges."""
+    from mi355_vit import _lib
+
+    _announce(f"image token ranks n={n} labels={with_labels}")
+    g = torch.Generator().manual_seed(n)
+    ids, labels = torch.randint(0, 3, (n,), generator=g), torch.where(torch.rand(n, generator=g) < 0.7, -100, 5)
+    dev = [ids.to(DEV), labels.to(DEV)]
+    rank = torch.full((n + 8,), -7, dtype=torch.int32, device=DEV)
+    positions = torch.full((n + 8,), -7, dtype=torch.int64, device=DEV)
+    counts = torch.full((2,), -7, dtype=torch.int64, device=DEV)
+    rc = _lib.load().mvit_image_token_ranks(dev[0].data_ptr(), dev[1].data_ptr() if with_labels else None, n, 1, -100, rank.data_ptr(),
+                                            positions.data_ptr(), counts.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    if n == 0 and rc != 0:  # nothing to rank is refused, or counts nothing
+        return
+    assert rc == 0
+    img = ids == 1
+    want = torch.where(img, torch.cumsum(img, 0) - 1, -1)
+    assert torch.equal(rank[:n].cpu().long(), want) and bool((rank[n:] == -7).all())
+    at = img.nonzero().flatten()
+    assert torch.equal(positions[: at.numel()].cpu(), at) and bool((positions[at.numel():] == -7).all())
+    assert counts.tolist() == [at.numel(), int((img & (labels != -100)).sum()) if with_labels else 0]
+
+
 def test_guards_raise_like_the_reference():
     from mi355_vit.handoff import extract_vision_grad, merge_vision_embeddings
 
