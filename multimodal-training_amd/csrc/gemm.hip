@@ -1164,7 +1164,7 @@ bool pp_takes(GemmTiledKind kind, int64_t k_chunk, int64_t k_last) {  // at leas
 
 // Modelled times (us) of the tiles on one MI355X, fitted to every tile's time at 256 ... 16,384 rows of the tower's products: a
 // step of 64 along K takes 1.15 us in a 256 x 256 tile (one work-group per compute unit; 1.2 with both operands behind the
-// transposing LDS read; 2,435 cycles, so more when the clock falls under a long load, which lengthens every tile's steps alike), and in the smaller ones `one` us while every unit has at most one work-group and `two` us once it has
+// transposing LDS read; 2,392 cycles, so more when the clock falls under a long load, which lengthens every tile's steps alike), and in the smaller ones `one` us while every unit has at most one work-group and `two` us once it has
 // two.  Tiles of one work-group per unit (`lone`) interleave loads, LDS reads and MFMAs, so their steps are shorter than those of a
 // single work-group of the kind that shares its unit: 128 x 128 is taken up to 256 tiles and 192 x 128 from there to 256 tiles again
 // (input gradient of 6912 x 1280, us, shared / 128 lone / 192 lone: 2,048 rows 70 / 48 / 61, 3,136 73 / 55 / 65, 4,096 78 / 95 / 68,
