@@ -1,8 +1,8 @@
 // fp32 GEMM (the parity path) on v_mfma_f32_16x16x4_f32:  C[M,N] = epi( sum_k A[m,k] * B[n,k] ).
 //
 // What bounds it is the fp32 matrix rate (157 TFLOP/s, a sixteenth of bf16's) once enough compute units have work: a
-// 64 x 64 tile per work-group of four waves (a K tile of 32 is 1,024 cycles of MFMA and 16 KiB of operands), or a 32 x 64 tile
-// where there are few of those (half_rows below).
+// 64 x 64 tile per work-group of four waves (a K tile of 32 is 1,024 cycles of MFMA and 16 KiB of operands), or a 32 x 64 or 32 x 32
+// tile where there are few of those (half_rows, quarters below).
 // K tiles of 32 floats (128-byte rows) in a ring of four LDS stages filled by direct global -> LDS loads, two work-groups
 // per compute unit.  MFMA (s, j) of a K tile contracts k = 16 s + 4 g + j over the lane groups g = 0..3, so one 16-byte read
 // of a [row][k] operand feeds four of them; a [k][row] operand is read as two neighbouring rows (8 bytes) per k, and the two
@@ -11,33 +11,35 @@
 // and its reads (us: 512 rows K = 1280 x 3840 48.6 -> 44.6, input gradient K = 6912 137 -> 121, its weight gradient 92 -> 80; 2,048
 // rows 340 -> 293, 337 -> 292, i.e. 123 TFLOP/s; 4-block step of 512 rows 4.00 -> 3.62 ms, of 2,048 11.8 -> 10.3).
 // The products are computed transposed (B's fragment first), so a lane ends with eight consecutive columns of a row and
-// stores them from registers.  Both tiles add in the same order: a row's result does not depend on its batch.
+// stores them from registers (a 32 x 32 tile's lanes trade four for that).  All tiles add in the same order: a row's result does not depend on its batch.
 #include "gemm_direct.h"
 
 #include <type_traits>
 
 namespace {
 
-template <int BM_, int WGM_, int WGN_>
+template <int BM_, int BN_, int WGM_, int WGN_>
 struct F32Cfg {
-  static constexpr int BM = BM_, BN = 64, BK = 32, NST = 4, NTHREADS = 256, WGM = WGM_, WGN = WGN_, WM = BM / WGM, WN = BN / WGN;
+  static constexpr int BM = BM_, BN = BN_, BK = 32, NST = 4, NTHREADS = 256, WGM = WGM_, WGN = WGN_, WM = BM / WGM, WN = BN / WGN;
   static constexpr int A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128, LDS = NST * STAGE;
-  static constexpr int PER_A = BM / 32, PER_B = 2, PER = PER_A + PER_B;  // 1 KiB loads per wave and K tile
+  static constexpr int PER_A = BM / 32, PER_B = BN / 32, PER = PER_A + PER_B;  // 1 KiB loads per wave and K tile
 };
 
-// slot of chunk c (16 bytes) of row `major` ([row][k]: eight chunks) or k-row `major` ([k][row]: sixteen chunks)
-template <bool TR, bool IS_A>
+// slot of chunk c (16 bytes) of row `major` ([row][k]: eight chunks) or k-row `major` ([k][row]: CHUNKS of them).  DEALT: rows as a
+// fragment of two column blocks takes them
+template <bool TR, bool DEALT, int CHUNKS>
 __device__ __forceinline__ int f32_swizzle(int major) {
-  if (TR) return ((major >> 2) & 1) << 3;
-  return IS_A ? (major >> 1) & 7 : ((major >> 1) & 1) | (((major >> 3) & 3) << 1);
+  if (TR) return ((major >> 2) & 1) * (CHUNKS / 2);
+  return !DEALT ? (major >> 1) & 7 : ((major >> 1) & 1) | (((major >> 3) & 3) << 1);
 }
 
-template <bool TA, bool TB, int EPI, int BM>
+template <bool TA, bool TB, int EPI, int BM, int BN>
 __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmParams p) {
   constexpr bool DUAL = (EPI == MVIT_EPI_SWIGLU);
-  using S = F32Cfg<BM, DUAL ? 4 : 2, DUAL ? 1 : 2>;
-  constexpr int BK = S::BK, NST = S::NST, NA = S::WM / 16, NB = S::WN / 16, NG = DUAL ? 1 : NB / 2, NCOLS = DUAL ? 32 : 64;
-  static_assert((!TA || NA == 2) && (!TB || NB == 2), "[k][row] operands are read as pairs of rows");
+  using S = F32Cfg<BM, BN, DUAL ? 4 : 2, DUAL ? 1 : 2>;
+  constexpr int BK = S::BK, NST = S::NST, NA = S::WM / 16, NB = S::WN / 16, NG = DUAL || NB == 1 ? 1 : NB / 2, NCOLS = DUAL ? 32 : BN;
+  constexpr bool DEALT = NB > 1;  // B's rows ([row][k]) are dealt to two column blocks
+  static_assert((!TA || NA == 2) && (!TB || NB <= 2), "[k][row] operands are read as pairs of rows, or B's one by one");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
 
   const unsigned tiles = (unsigned)(p.tiles_m * p.tiles_n), total = tiles * (unsigned)p.split_k, per_xcd = (total + 7) / 8;
@@ -63,29 +65,30 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmParams p) {
   int ka[S::PER_A], kb[S::PER_B];  // first k of the lane's chunk inside a K tile
   const int64_t step_a = TA ? 4ll * BK * p.lda : 4 * BK, step_b = TB ? 4ll * BK * p.ldb : 4 * BK;
   const int m_left = (int)(p.M - m0 < S::BM ? p.M - m0 : S::BM), n_left = (int)(p.N - n0 < NCOLS ? p.N - n0 : NCOLS);
-  auto place = [&](auto TR, auto IS_A, int q, const void* X, int64_t ld, int64_t row0, int left, int row_of_tile, const char*& ptr, int& k) {
+  auto place = [&](auto TR, auto DEALT_, auto CHUNKS, int q, const void* X, int64_t ld, int64_t row0, int left, int row_of_tile, const char*& ptr, int& k) {
     const float* x = static_cast<const float*>(X);
     if (!decltype(TR)::value) {
-      const int c = (l & 7) ^ f32_swizzle<false, decltype(IS_A)::value>(q * 8 + (l >> 3));
+      const int c = (l & 7) ^ f32_swizzle<false, decltype(DEALT_)::value, 8>(q * 8 + (l >> 3));
       const int r = row_of_tile < left ? row_of_tile : left - 1;  // rows past the edge repeat the last row: their results are not stored
       k = c * 4;
       ptr = reinterpret_cast<const char*>(x + (row0 + r) * ld + k_begin + k);
     } else {
-      k = q * 4 + (l >> 4);
-      const int c = (l & 15) ^ f32_swizzle<true, decltype(IS_A)::value>(k);
+      constexpr int CH = decltype(CHUNKS)::value;
+      k = q * (64 / CH) + l / CH;
+      const int c = (l % CH) ^ f32_swizzle<true, false, CH>(k);
       ptr = reinterpret_cast<const char*>(x + (k_begin + k) * ld + row0 + (c * 4 < left ? c * 4 : 0));
     }
   };
 #pragma unroll
   for (int j = 0; j < S::PER_A; ++j) {
     const int q = wv * S::PER_A + j;
-    place(std::bool_constant<TA>{}, std::true_type{}, q, p.A, p.lda, m0, m_left, q * 8 + (l >> 3), pa[j], ka[j]);
+    place(std::bool_constant<TA>{}, std::false_type{}, std::integral_constant<int, BM / 4>{}, q, p.A, p.lda, m0, m_left, q * 8 + (l >> 3), pa[j], ka[j]);
   }
 #pragma unroll
   for (int j = 0; j < S::PER_B; ++j) {
     const int q = wv * S::PER_B + j, row = q * 8 + (l >> 3);
     // SWIGLU: tile rows 0-31 are gate rows, 32-63 up rows
-    place(std::bool_constant<TB>{}, std::false_type{}, q, DUAL && q >= 4 ? p.B2 : p.B, p.ldb, n0, n_left, DUAL ? row & 31 : row, pb[j], kb[j]);
+    place(std::bool_constant<TB>{}, std::bool_constant<DEALT>{}, std::integral_constant<int, BN / 4>{}, q, DUAL && q >= 4 ? p.B2 : p.B, p.ldb, n0, n_left, DUAL ? row & 31 : row, pb[j], kb[j]);
   }
   auto issue = [&](int t, unsigned stage_off) {
     const unsigned da = lds_base + stage_off + wv * (S::PER_A * 1024), db = lds_base + stage_off + S::A_BYTES + wv * (S::PER_B * 1024);
@@ -107,8 +110,10 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmParams p) {
         pp_load_at(da + j * 1024, pa[j]);
         pa[j] += step_a;
       }
-      pp_load_at(db + j * 1024, pb[j]);
-      pb[j] += step_b;
+      if (j < S::PER_B) {
+        pp_load_at(db + j * 1024, pb[j]);
+        pb[j] += step_b;
+      }
     }
   };
 #pragma unroll
@@ -118,20 +123,20 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmParams p) {
   // ---- fragment addresses (stage 0)
   unsigned ra[2], rb[2];  // [row][k]: chunk 4 s + g of the lane's row; [k][row]: entry 0, k-row 4 g
   if constexpr (!TA) {
-    const int row = wm * S::WM + i16, f = f32_swizzle<false, true>(row);
+    const int row = wm * S::WM + i16, f = f32_swizzle<false, false, 8>(row);
     ra[0] = row * 128 + ((g4 ^ f) << 4);
     ra[1] = row * 128 + (((4 + g4) ^ f) << 4);
   } else {
     const int r = wm * S::WM + 2 * i16;
-    ra[0] = ra[1] = 4 * g4 * 256 + (((r >> 2) ^ f32_swizzle<true, true>(4 * g4)) << 4) + (r & 3) * 4;
+    ra[0] = ra[1] = 4 * g4 * 256 + (((r >> 2) ^ f32_swizzle<true, false, 16>(4 * g4)) << 4) + (r & 3) * 4;
   }
   if constexpr (!TB) {
-    const int row = wn * S::WN + 8 * (i16 >> 2) + (i16 & 3), f = f32_swizzle<false, false>(row);
+    const int row = wn * S::WN + (DEALT ? 8 * (i16 >> 2) + (i16 & 3) : i16), f = f32_swizzle<false, DEALT, 8>(row);
     rb[0] = S::A_BYTES + row * 128 + ((g4 ^ f) << 4);
     rb[1] = S::A_BYTES + row * 128 + (((4 + g4) ^ f) << 4);
   } else {
-    const int r = wn * S::WN + 2 * i16;
-    rb[0] = rb[1] = S::A_BYTES + 4 * g4 * 256 + (((r >> 2) ^ f32_swizzle<true, false>(4 * g4)) << 4) + (r & 3) * 4;
+    const int r = wn * S::WN + NB * i16;
+    rb[0] = rb[1] = S::A_BYTES + 4 * g4 * (BN * 4) + (((r >> 2) ^ f32_swizzle<true, false, BN / 4>(4 * g4)) << 4) + (r & 3) * 4;
   }
 
   f32x4 acc[NA][NB];
@@ -159,10 +164,12 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmParams p) {
         const f32x4 v = *reinterpret_cast<const f32x4*>(at + rb[s] + (r >> 1) * 4096 + (r & 1) * 512);
 #pragma unroll
         for (int j = 0; j < 4; ++j) fb[r < NB ? r : 0][4 * s + j] = v[j];
-      } else {
-        const f32x2 v = *reinterpret_cast<const f32x2*>(at + rb[0] + (16 * s + r) * 256);
+      } else if constexpr (NB == 2) {
+        const f32x2 v = *reinterpret_cast<const f32x2*>(at + rb[0] + (16 * s + r) * (BN * 4));
         fb[0][4 * s + r] = v[0];
         fb[NB - 1][4 * s + r] = v[1];
+      } else {
+        fb[0][4 * s + r] = *reinterpret_cast<const float*>(at + rb[0] + (16 * s + r) * (BN * 4));
       }
     }
   };
@@ -234,13 +241,21 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmParams p) {
   for (int a = 0; a < NA; ++a)
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
-      const int64_t m = m0 + wm * S::WM + (TA ? 2 * i16 + a : a * 16 + i16), n = n0 + (DUAL ? 0 : wn * S::WN) + g * 32 + 8 * g4;
-      if (m >= p.M || n >= p.N) continue;
+      const int64_t m = m0 + wm * S::WM + (TA ? 2 * i16 + a : a * 16 + i16), n = n0 + (DUAL ? 0 : wn * S::WN) + (NB == 1 ? 4 * g4 : g * 32 + 8 * g4);
       float v[8], u[8];
+      if constexpr (NB == 1) {  // one block: every other group of 16 lanes takes its neighbour's four columns to its own
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
+        for (int r = 0; r < 4; ++r) {
+          v[r] = acc[a][0][r];
+          v[4 + r] = __shfl_xor(v[r], 16);
+        }
+        if (g4 & 1) continue;
+      }
+      if (m >= p.M || n >= p.N) continue;
+#pragma unroll
+      for (int r = 0; r < (NB == 1 ? 0 : 4); ++r) {
         v[TB ? 2 * r : r] = acc[a][2 * g][r];
-        v[TB ? 2 * r + 1 : 4 + r] = acc[a][2 * g + 1][r];
+        v[TB ? 2 * r + 1 : 4 + r] = acc[a][NB == 1 ? 0 : 2 * g + 1][r];
         if (DUAL) {
           u[r] = acc[a][NB - 2][r];
           u[4 + r] = acc[a][NB - 1][r];
@@ -269,14 +284,24 @@ inline bool half_rows(const GemmParams& p) {
   return tiles <= units * 3 / 4 || (rounds > 1 && rounds <= 3 && half_rounds < 2 * rounds);
 }
 
-template <bool TA, bool TB, int EPI, int BM>
+// 32 x 32 tiles (a wave's share is one MFMA block) where every compute unit has at most one, or three where 32 x 64 tiles would be two
+// to a unit: the matrix pipes of a unit with two of those work 1.6 times as long as the average's.  us, 32 x 64 / 32 x 32, input
+// gradients K = 6912 x 1280: 64 and 128 rows (one each) 77 / 55, 256 (two) 77 / 80, 512 (three) 121 / 103, 768 (four; 64 x 64 128) - / 130, 1,024
+// 177 / 238; 4-block step of 512 rows 3.62 / 3.47 ms, of 64 (bound by the host) 2.21 / 2.18.
+inline bool quarters(const GemmParams& p) {
+  constexpr int64_t units = 256;
+  const int64_t per_unit = ((p.M + 31) / 32 * ((p.N + 31) / 32) * p.split_k + units - 1) / units;
+  return per_unit == 1 || per_unit == 3;
+}
+
+template <bool TA, bool TB, int EPI, int BM, int BN = 64>
 int launch_f32_tiles(GemmParams p, hipStream_t stream) {
-  constexpr int NCOLS = EPI == MVIT_EPI_SWIGLU ? 32 : 64;
+  constexpr int NCOLS = EPI == MVIT_EPI_SWIGLU ? 32 : BN;
   const int64_t tm = (p.M + BM - 1) / BM, tn = (p.N + NCOLS - 1) / NCOLS;
   MVIT_REQUIRE(tm * tn * p.split_k < (1ll << 30), "gemm: too many tiles");
   p.tiles_m = (int)tm; p.tiles_n = (int)tn;
   p.panel_w = tn <= 6 ? (int)tn : 4;
-  hipLaunchKernelGGL((gemm_f32_kernel<TA, TB, EPI, BM>), (p.tiles_m * p.tiles_n * p.split_k + 7) / 8 * 8, 256, (F32Cfg<BM, 2, 2>::LDS), stream, p);
+  hipLaunchKernelGGL((gemm_f32_kernel<TA, TB, EPI, BM, BN>), (p.tiles_m * p.tiles_n * p.split_k + 7) / 8 * 8, 256, (F32Cfg<BM, BN, 2, 2>::LDS), stream, p);
   MVIT_CHECK_LAUNCH("gemm");
   return MVIT_OK;
 }
@@ -284,6 +309,7 @@ int launch_f32_tiles(GemmParams p, hipStream_t stream) {
 template <bool TA, bool TB, int EPI>
 int launch_f32(const GemmParams& p, hipStream_t stream) {
   if constexpr (!TA && EPI != MVIT_EPI_SWIGLU) {
+    if (quarters(p)) return launch_f32_tiles<TA, TB, EPI, 32, 32>(p, stream);
     if (half_rows(p)) return launch_f32_tiles<TA, TB, EPI, 32>(p, stream);
   }
   return launch_f32_tiles<TA, TB, EPI, 64>(p, stream);

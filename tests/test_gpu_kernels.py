@@ -481,7 +481,7 @@ def test_gemm_of_few_rows_over_the_edges_of_its_ring_and_tiles(M, N, K, form, mo
 
 @pytest.mark.parametrize("form", ["nn", "nt", "tt"])
 @pytest.mark.parametrize("K", [4, 32, 36, 64, 96, 100, 128, 132, 160, 164, 1284])
-@pytest.mark.parametrize("M,N", [(40, 72), (452, 1280)])
+@pytest.mark.parametrize("M,N", [(40, 72), (452, 1280), (252, 1280), (700, 1280)])  # 32 x 32 (one and three per unit), 32 x 64, 64 x 64 tiles
 def test_fp32_gemm_over_the_edges_of_its_ring(M, N, K, form):
     """K tiles of 32 in a ring of four stages: never full, once full, refilled, with and without a partial last tile."""
     _announce(f"fp32 gemm ring {form} {M}x{N}x{K}")
