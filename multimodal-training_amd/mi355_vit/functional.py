@@ -63,16 +63,19 @@ class BlockWeights:
     args: Optional["_lib.BlockArgs"] = None  # the block call's arguments that depend on the weights alone, see block_args
 
     def block_args(self) -> Optional["_lib.BlockArgs"]:
-        """The weight operands as the C calls take them, filled once per pack and copied per call; None: not laid out for them."""
-        if self.args is None:
+        """The weight operands as the C calls take them, filled once per pack and copied per call; None: not laid out for them.
+        Another thread may run the same model: `args` is set to a struct that is complete, and not written again."""
+        a = self.args
+        if a is None:
             w = (self.norm1, self.norm2, self.wqkv, self.bqkv, self.wproj, self.bproj, self.wgu, self.bgu, self.wdown, self.bdown)
             dtype = self.wqkv.dtype
             if dtype not in ops._DT or not all(t.is_contiguous() and t.dtype == dtype for t in w):
                 return None
-            a = self.args = _lib.BlockArgs()
+            a = _lib.BlockArgs()
             a.dtype, a.C, a.I, a.Ipad = ops._DT[dtype], self.C, self.I, self.Ipad
             a.norm1, a.norm2, a.wqkv, a.bqkv, a.wproj, a.bproj, a.wgu, a.bgu, a.wdown, a.bdown = (t.data_ptr() for t in w)
-        return self.args
+            self.args = a
+        return a
 
     def __getstate__(self):  # addresses are not copied or saved with the operands
         return dict(self.__dict__, args=None)

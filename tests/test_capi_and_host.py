@@ -399,3 +399,37 @@ def test_packed_weights_can_be_copied_and_pickled_after_their_addresses_were_lai
     W.wproj = W.wproj.t()[:, :8]
     W.args = None
     assert W.block_args() is None  # not laid out for the C calls: the call-by-call path checks and takes it
+
+
+def test_packed_weights_laid_out_in_one_thread_are_never_seen_half_filled_by_another(monkeypatch):
+    """Threads that run one model share its packed operands: one that asks for the argument struct while another lays it out gets a whole one."""
+    import threading
+
+    import torch
+
+    from mi355_vit import _lib, functional
+
+    C, I = 16, 24
+    z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16)  # noqa: E731
+    W = functional.BlockWeights(z(1, C), z(1, C), z(3 * C, C), z(1, 3 * C), z(C, C), z(1, C), z(2 * I, C), z(1, 2 * I), z(C, I), z(1, C), C, I, I)
+    weights = ("norm1", "norm2", "wqkv", "bqkv", "wproj", "bproj", "wgu", "bgu", "wdown", "bdown")
+    expected = (_lib.BF16, C, I, I) + tuple(getattr(W, n).data_ptr() for n in weights)
+    seen, interrupted = [], []
+
+    def look():
+        a = W.block_args()
+        seen.append((a.dtype, a.C, a.I, a.Ipad) + tuple(getattr(a, n) for n in weights))
+
+    class Interrupted(_lib.BlockArgs):
+        def __setattr__(self, name, value):
+            super().__setattr__(name, value)
+            if name in weights and name not in interrupted:  # another thread gets its turn here, once per field
+                interrupted.append(name)
+                other = threading.Thread(target=look)
+                other.start()
+                other.join()
+
+    monkeypatch.setattr(_lib, "BlockArgs", Interrupted)
+    look()
+    assert len(seen) == len(weights) + 1 and interrupted == list(weights)
+    assert all(s == expected for s in seen)
