@@ -60,21 +60,29 @@ class BlockWeights:
     I: int
     Ipad: int
     alias: bool = False  # norm1 / norm2 / wproj / bproj / bdown are the parameters themselves (same dtype), not copies
-    args: Optional["_lib.BlockArgs"] = None  # the block call's arguments that depend on the weights alone, see block_args
+    args: Optional[tuple] = None  # (what the struct was filled from, the struct), see block_args
 
     def block_args(self) -> Optional["_lib.BlockArgs"]:
-        """The weight operands as the C calls take them, filled once per pack and copied per call; None: not laid out for them.
-        Another thread may run the same model: `args` is set to a struct that is complete, and not written again."""
-        a = self.args
-        if a is None:
-            w = (self.norm1, self.norm2, self.wqkv, self.bqkv, self.wproj, self.bproj, self.wgu, self.bgu, self.wdown, self.bdown)
-            dtype = self.wqkv.dtype
-            if dtype not in ops._DT or not all(t.is_contiguous() and t.dtype == dtype for t in w):
+        """The weight operands as the C calls take them; None: not laid out for them.  Layouts, types and addresses are looked at on
+        every call (3.2 us), as the call-by-call wrappers do; the struct that is kept saves filling another (1.2 us) and is taken
+        only while the operands are what it was filled from.  Another thread may run the same model: `args` is set to a struct that
+        is complete, and not written again."""
+        w = (self.norm1, self.norm2, self.wqkv, self.bqkv, self.wproj, self.bproj, self.wgu, self.bgu, self.wdown, self.bdown)
+        dtype = self.wqkv.dtype
+        if dtype not in ops._DT:
+            return None
+        source = [dtype, self.C, self.I, self.Ipad]
+        for t in w:
+            if t.dtype is not dtype or not t.is_contiguous():
                 return None
-            a = _lib.BlockArgs()
-            a.dtype, a.C, a.I, a.Ipad = ops._DT[dtype], self.C, self.I, self.Ipad
-            a.norm1, a.norm2, a.wqkv, a.bqkv, a.wproj, a.bproj, a.wgu, a.bgu, a.wdown, a.bdown = (t.data_ptr() for t in w)
-            self.args = a
+            source.append(t.data_ptr())
+        kept = self.args
+        if kept is not None and kept[0] == source:
+            return kept[1]
+        a = _lib.BlockArgs()
+        a.dtype, a.C, a.I, a.Ipad = ops._DT[dtype], self.C, self.I, self.Ipad
+        a.norm1, a.norm2, a.wqkv, a.bqkv, a.wproj, a.bproj, a.wgu, a.bgu, a.wdown, a.bdown = source[4:]
+        self.args = (source, a)
         return a
 
     def __getstate__(self):  # addresses are not copied or saved with the operands
@@ -135,7 +143,6 @@ def pack_block_weights(params: List[torch.Tensor], dtype: torch.dtype, into: Opt
         fill(w, into.wgu[j * Ipad : j * Ipad + I])
         fill(b, into.bgu[:, j * Ipad : j * Ipad + I])
     fill(wd, into.wdown[:, :I])
-    into.args = None
     return into
 
 
@@ -167,8 +174,14 @@ _join_events: dict = {}
 _GRAD_DTYPES = (torch.bfloat16, torch.float32)  # one dtype for all of a block's gradients, as the C call writes them
 
 
-def _block_args(x: torch.Tensor, W: BlockWeights, geo: AttnGeometry, eps: float) -> "_lib.BlockArgs":
-    a = _lib.BlockArgs.from_buffer_copy(W.block_args())
+def _block_args(x: torch.Tensor, W: BlockWeights, geo: AttnGeometry, eps: float) -> Optional["_lib.BlockArgs"]:
+    """The arguments that a block's C calls share, or None where an operand is not laid out as their sequence assumes: what the
+    call-by-call wrappers check launch by launch, once for the block."""
+    weights = W.block_args()
+    if (weights is None or not x.is_cuda or not x.is_contiguous() or x.shape[1] != W.C or geo.nheads * geo.head_dim != W.C
+            or x.dtype != W.wqkv.dtype or not geo.block_call_ok(x)):
+        return None
+    a = _lib.BlockArgs.from_buffer_copy(weights)
     a.S, a.nheads, a.head_dim = x.shape[0], geo.nheads, geo.head_dim
     a.eps, a.q_lead_scale, a.attn_scale = eps, geo.head_dim**-0.5 * LOG2E, 1.0 / LOG2E
     a.n_seg, a.max_seqlen = geo.cu.shape[0] - 1, geo.max_seqlen
@@ -177,12 +190,6 @@ def _block_args(x: torch.Tensor, W: BlockWeights, geo: AttnGeometry, eps: float)
         a.seg_order = geo.order.data_ptr()
     a.x = x.data_ptr()
     return a
-
-
-def _block_geometry_ok(x: torch.Tensor, W: BlockWeights, geo: AttnGeometry) -> bool:
-    """What the call-by-call wrappers check launch by launch, once for the block: operand layouts the C sequence assumes."""
-    return (W.block_args() is not None and x.is_cuda and x.is_contiguous() and x.shape[1] == W.C and geo.nheads * geo.head_dim == W.C
-            and x.dtype == W.wqkv.dtype and geo.block_call_ok(x))
 
 
 class _Buffers:
@@ -234,7 +241,7 @@ class _Saved:
         return (self[i] for i in range(10))
 
 
-def _block_forward_one_call(x, W, geo, eps, attn_out, for_backward, output):
+def _block_forward_one_call(a, x, W, geo, attn_out, for_backward, output):
     S, C = x.shape
     T, f32, Ipad = x.dtype, torch.float32, W.Ipad
     if attn_out is None and geo.max_seqlen > KEEP_ATTENTION_ABOVE:  # may outlive the rest
@@ -253,7 +260,6 @@ def _block_forward_one_call(x, W, geo, eps, attn_out, for_backward, output):
         dtypes += [T, f32]
     saved = _Saved(_Buffers(x.device, shapes, dtypes), index, attn_out)
     x2 = torch.empty_like(x) if output else None
-    a = _block_args(x, W, geo, eps)
     a.skip_attention = skip
     p = saved.ptr
     a.rstd1, a.n1, a.qkv, a.o, a.lse, a.x1, a.rstd2, a.n2, a.gu, a.h = p(0), p(1), p(2), p(3), p(4), p(5), p(6), p(7), p(8), p(9)
@@ -263,11 +269,10 @@ def _block_forward_one_call(x, W, geo, eps, attn_out, for_backward, output):
     return x2, saved
 
 
-def _block_backward_one_call(dx2, x, saved, W, geo, G):
+def _block_backward_one_call(a, dx2, x, saved, W, G):
     S, Cc = x.shape
     I, Ipad = W.I, W.Ipad
     dev, T = x.device, x.dtype
-    a = _block_args(x, W, geo, 0.0)
     a.grad_dtype = ops._DT[G]
     if type(saved) is _Saved:
         p = saved.ptr
@@ -318,8 +323,9 @@ def _block_forward(x: torch.Tensor, W: BlockWeights, geo: AttnGeometry, eps: flo
     pre-activations are not written (the first run of a checkpointed block).  ``output=False``: the block's output is
     not wanted, so the down projection is skipped (the re-run of a checkpointed block: the backward reads `h`, not
     `x2`)."""
-    if BLOCK_CALLS and ops._trace is None and _block_geometry_ok(x, W, geo):
-        return _block_forward_one_call(x, W, geo, eps, attn_out, for_backward, output)
+    a = _block_args(x, W, geo, eps) if BLOCK_CALLS and ops._trace is None else None
+    if a is not None:
+        return _block_forward_one_call(a, x, W, geo, attn_out, for_backward, output)
     S, C = x.shape
     H, hd = geo.nheads, geo.head_dim
     n1, rstd1 = ops.rmsnorm_fwd(x, W.norm1.view(-1), eps)
@@ -353,8 +359,9 @@ def _block_forward(x: torch.Tensor, W: BlockWeights, geo: AttnGeometry, eps: flo
 def _block_backward(dx2: torch.Tensor, x: torch.Tensor, saved: tuple, W: BlockWeights, geo: AttnGeometry, gdt):
     """Returns (dx, grads in BLOCK_PARAM_ORDER).  gdt: the gradients' dtype, or a map parameter name -> gradient dtype."""
     dx2 = dx2.contiguous()
-    if BLOCK_CALLS and ops._trace is None and gdt in _GRAD_DTYPES and dx2.dtype == x.dtype and _block_geometry_ok(x, W, geo):
-        return _block_backward_one_call(dx2, x, saved, W, geo, gdt)
+    a = _block_args(x, W, geo, 0.0) if BLOCK_CALLS and ops._trace is None and gdt in _GRAD_DTYPES and dx2.dtype == x.dtype else None
+    if a is not None:
+        return _block_backward_one_call(a, dx2, x, saved, W, gdt)
     if not isinstance(gdt, dict):
         gdt = dict.fromkeys(BLOCK_PARAM_ORDER, gdt)
     rstd1, n1, qkv, o, lse, x1, rstd2, n2, gu, h = saved

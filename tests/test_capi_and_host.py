@@ -433,3 +433,25 @@ def test_packed_weights_laid_out_in_one_thread_are_never_seen_half_filled_by_ano
     look()
     assert len(seen) == len(weights) + 1 and interrupted == list(weights)
     assert all(s == expected for s in seen)
+
+
+def test_packed_weights_are_looked_at_on_every_call():
+    """An operand that was replaced, moved or given another layout after the argument struct was filled is seen by the next call."""
+    import torch
+
+    from mi355_vit.functional import BlockWeights
+
+    C, I = 16, 24
+    z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16)  # noqa: E731
+    W = BlockWeights(z(1, C), z(1, C), z(3 * C, C), z(1, 3 * C), z(C, C), z(1, C), z(2 * I, C), z(1, 2 * I), z(C, I), z(1, C), C, I, I)
+    first = W.block_args()
+    old, W.wproj = W.wproj, z(C, C)  # another tensor
+    assert W.block_args().wproj == W.wproj.data_ptr() != old.data_ptr() == first.wproj
+    W.wdown.set_(z(C, I))  # the same tensor with another storage
+    assert W.block_args().wdown == W.wdown.data_ptr() != first.wdown
+    W.wproj = z(C, 2 * C)[:, :C]  # rows apart: the call-by-call path checks it and takes or refuses it
+    assert W.block_args() is None
+    W.wproj = torch.zeros(C, C)  # another dtype
+    assert W.block_args() is None
+    W.wproj = old
+    assert W.block_args().wproj == old.data_ptr()
