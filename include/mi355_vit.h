@@ -33,11 +33,13 @@ typedef void* mvit_stream_t; /* hipStream_t */
 enum { MVIT_F32 = 0, MVIT_BF16 = 1 };
 enum { MVIT_OK = 0, MVIT_ERR_ARG = -1, MVIT_ERR_LAUNCH = -2, MVIT_ERR_UNSUPPORTED = -3 };
 
-/* 201: mvit_gemm_args has row_sums at its end.
+/* 203: mvit_gemm_args ends with overlapped; mvit_gemm_wgrad_split_k answers for a product that has the GPU to itself.
+ * 202: mvit_gemm_args ends with colsum_rows.
+ * 201: mvit_gemm_args has row_sums at its end.
  * 200: mvit_attn_bwd takes the size of its workspace (delta_elems) and checks that outputs and inputs are disjoint;
  *      mvit_adam_tensor rows are 96 bytes (shadow copy fields).  A caller built against an older header must be
  *      rebuilt: compare mvit_version() with the value the header was written for. */
-#define MVIT_VERSION 202
+#define MVIT_VERSION 203
 int mvit_version(void);
 const char* mvit_last_error(void);
 
@@ -188,6 +190,9 @@ typedef struct mvit_gemm_args {
                      workspace holds split_k * M more floats */
   int colsum_rows; /* MVIT_EPI_SWIGLU_BWD with a workspace: rows of C per row of column sums, 256 (also 0) or 64; the rows
                       of the tile that makes them, see mvit_gemm_swiglu_bwd_colsum_rows.  C does not depend on it */
+  int overlapped;  /* 0: nothing else runs on the GPU beside this product.  1: work of another stream does, and fills the compute
+                      units that this product leaves idle: the tile that wastes least is preferred to the one that is done first.
+                      Results do not depend on it */
 } mvit_gemm_args;
 
 /* C[M,N] = epilogue(sum_k A[m,k] * B[n,k]).  Operands must be 16-byte aligned with lda/ldb multiples of
@@ -198,6 +203,8 @@ int mvit_gemm(const mvit_gemm_args* args, mvit_stream_t stream);
 
 /* Host-only: the split_k to ask for when C[out_rows, out_cols] is a weight gradient contracted over k tokens (bf16). */
 int mvit_gemm_wgrad_split_k(int64_t out_rows, int64_t out_cols, int64_t k);
+/* Host-only: the same for a product that shares the GPU with another stream's (`overlapped`). */
+int mvit_gemm_wgrad_split_k_overlapped(int64_t out_rows, int64_t out_cols, int64_t k);
 /* Host-only: the colsum_rows with which a bf16 MVIT_EPI_SWIGLU_BWD product of this shape is fastest. */
 int mvit_gemm_swiglu_bwd_colsum_rows(int64_t M, int64_t N, int64_t K);
 

@@ -194,7 +194,7 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   auto weight_grad = [&](const void* dy, int64_t ldy, int64_t M, const void* x, int64_t ldx, int64_t N, void* out, void* bias, int split_k, mvit_stream_t st) -> int {
     if (bias && dt != MVIT_BF16) STEP(bias_grad(dy, ldy, M, bias, st));
     mvit_gemm_args g = gemm_args(dt, gdt);
-    g.trans_a = 1; g.trans_b = 1;
+    g.trans_a = 1; g.trans_b = 1; g.overlapped = two;
     g.M = M; g.N = N; g.K = S;
     g.A = dy; g.lda = ldy; g.B = x; g.ldb = ldx; g.C = out; g.ldc = N;
     if (split_k > 1) {
@@ -219,7 +219,7 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   const bool fused_cols = dt == MVIT_BF16;
   {
     mvit_gemm_args g = gemm_args(dt, dt);
-    g.trans_b = 1; g.epilogue = MVIT_EPI_SWIGLU_BWD;
+    g.trans_b = 1; g.epilogue = MVIT_EPI_SWIGLU_BWD; g.overlapped = two;
     g.M = S; g.N = Ipad; g.K = C;
     g.A = a->dx2; g.lda = C; g.B = a->wdown; g.ldb = Ipad; g.C = a->dgu; g.ldc = 2 * Ipad; g.R = a->gu; g.ldr = 2 * Ipad; g.aux_off = Ipad;
     if (fused_cols) {
@@ -235,7 +235,7 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   }
   {  // dn2 = dgu . Wgu
     mvit_gemm_args g = gemm_args(dt, dt);
-    g.trans_b = 1;
+    g.trans_b = 1; g.overlapped = two;
     g.M = S; g.N = C; g.K = 2 * Ipad;
     g.A = a->dgu; g.lda = 2 * Ipad; g.B = a->wgu; g.ldb = C; g.C = a->dn; g.ldc = C;
     STEP(mvit_gemm(&g, stream));
@@ -251,7 +251,7 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   }
   {  // d_o = dx1 . Wproj  (into the dn buffer, whose contents the norm backward above has consumed)
     mvit_gemm_args g = gemm_args(dt, dt);
-    g.trans_b = 1;
+    g.trans_b = 1; g.overlapped = two;
     g.M = S; g.N = C; g.K = C;
     g.A = a->dx1; g.lda = C; g.B = a->wproj; g.ldb = C; g.C = a->dn; g.ldc = C;
     STEP(mvit_gemm(&g, stream));
@@ -267,7 +267,7 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   }
   {  // dn1 = dqkv . Wqkv
     mvit_gemm_args g = gemm_args(dt, dt);
-    g.trans_b = 1;
+    g.trans_b = 1; g.overlapped = two;
     g.M = S; g.N = C; g.K = 3 * C;
     g.A = a->dqkv; g.lda = 3 * C; g.B = a->wqkv; g.ldb = C; g.C = a->dn; g.ldc = C;
     STEP(mvit_gemm(&g, stream));

@@ -1172,13 +1172,19 @@ bool pp_takes(GemmTiledKind kind, int64_t k_chunk, int64_t k_last) {  // at leas
 // the longest.  The line between the tiles follows from these numbers and not from any shape: e.g. weight gradients of
 // 3840 x 1280 over 4,096 rows take 49 us in one slice on 128 x 128 and 57 in three on 256 x 256, over 8,192 rows 93 and 87.
 //
-// What a launch costs is its time alone only where nothing runs beside it.  In the backward the input gradients and the weight
-// gradients run on two streams, and the units that one launch's last round leaves idle work for the other: there the estimate is
-// a mean of the time alone (weight `alone`) and of the units' time divided by the number of units, which favours the tile that
-// wastes least over the one that ends its rounds best.  That holds where there is work for idle units, i.e. not for input
+// What a launch costs is its time alone only where nothing runs beside it.  In a block's backward the input gradients and the weight
+// gradients run on two streams, and the units that one launch's last round leaves idle work for the other: there (`overlapped`, which
+// the caller says) the estimate is a mean of the time alone (weight `alone`) and of the units' time divided by the number of units,
+// which favours the tile that wastes least over the one that ends its rounds best.  That holds where there is work for idle units, i.e. not for input
 // gradients of so few rows that 256 x 256 tiles would give less than half of the units work.  ms per 32-block step, tiles by time
 // alone -> by this mean: 14,336 rows 69.0 -> 66.7, 16,384 (checkpointed, optimizer included) 102.6 -> 100.4, 9,600 50.0 -> 49.0 (that
 // one by the weight gradients' tiles), 4,096, 6,084 and 20,000 unchanged; with the mean at few rows too 1,760 rows 15.6 -> 16.2.
+// An input gradient that has the GPU to itself takes the tile that is done first.  There the small tiles' steps grow with the length
+// of the launch (clock, and operands that the L2s and the memory-side cache no longer hold): a launch of r rounds takes 5 % longer per round beyond the
+// first on 128 x 128 tiles, 15 % on 64-row ones.  us, input gradients of 1280 columns, the mean above -> this: K = 6912 13,312 rows 268 -> 215,
+// 14,336 267 -> 223, 16,384 282 -> 294 (4 % off the best), 18,432 and 27,648 284 and 432 (328 and 540 without the growth); K = 3840 13,312 rows
+// 155 -> 129, 16,384 160 -> 148; 5120 columns, K = 5120 (the merger) 3,584 rows 202 -> 171.  Over 107 sizes from 1,024 to 65,536 rows the
+// choice is 0.1 % off the fastest tile on average.
 constexpr double PP_STEP_US = 1.15, PP_TILE_US = 7., PP_SWIGLU_TILE_US = 11.;
 struct TileChoice {
   int bm, bn;
@@ -1190,12 +1196,12 @@ TileChoice full_rows_tile(GemmTiledKind kind, int64_t k_chunk, int64_t k_last) {
   return pp_takes(kind, k_chunk, k_last) ? TileChoice{256, 256, 0.} : TileChoice{0, 0, 0.};
 }
 // `full_rows`: whether that kernel may be chosen
-TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk, int64_t k_last, int64_t slices, int n_cu, bool full_rows = true) {
+TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk, int64_t k_last, int64_t slices, int n_cu, bool overlapped, bool full_rows = true) {
   const bool tt = kind == TT_NONE || kind == TT_NONE_F32;
   const double steps = (double)((k_chunk + 63) / 64);
   const int64_t n_mul = kind == NN_SWIGLU ? 2 : 1;
-  const bool fills = 2 * ((M + 255) / 256) * ((N + 255) / 256) >= n_cu;
-  const double alone = tt ? 0.5 : ((kind == NT_NONE || kind == NT_GELU_BWD) && fills ? 0.3 : 1.);
+  const bool input_grad = kind == NT_NONE || kind == NT_GELU_BWD, fills = 2 * ((M + 255) / 256) * ((N + 255) / 256) >= n_cu;
+  const double alone = !overlapped ? 1. : tt ? 0.5 : (input_grad && fills ? 0.3 : 1.);
   TileChoice best{0, 0, 1e30};
   auto consider = [&](int bm, int bn, double one, double two, double per_tile, bool lone = false) {
     const int64_t items = ((M + bm - 1) / bm) * ((N * n_mul + bn - 1) / bn) * slices;
@@ -1203,6 +1209,7 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
     const double round = steps * (two > 0. ? two : one) + per_tile;
     double us = full * round;
     if (rest > 0) us += steps * (two > 0. && rest > n_cu ? two : one) + per_tile;
+    if (input_grad && !overlapped && two > 0. && items > slots) us *= 1. + (bm == 128 ? 0.05 : 0.15) * (double)((items - 1) / slots);
     us = 4. + alone * us + (1. - alone) * round * (double)items / (double)slots;
     if (us < best.us) best = TileChoice{bm, bn, us, lone};
   };
@@ -1241,7 +1248,7 @@ int64_t rows_in_full_rounds(GemmTiledKind kind, int64_t M, int64_t N, int64_t K,
   const int64_t tn = (N * (kind == NN_SWIGLU ? 2 : 1) + 255) / 256, rounds = (M + 255) / 256 * tn / n_cu, rows = rounds * n_cu / tn * 256;
   if (rows == 0 || rows >= M) return 0;
   const double head = 4. + (double)rounds * ((double)((K + 63) / 64) * PP_STEP_US + (kind == NN_SWIGLU ? PP_SWIGLU_TILE_US : PP_TILE_US));
-  return head + choose_tile(kind, M - rows, N, K, K, 1, n_cu).us + 1. < choose_tile(kind, M, N, K, K, 1, n_cu).us ? rows : 0;
+  return head + choose_tile(kind, M - rows, N, K, K, 1, n_cu, false).us + 1. < choose_tile(kind, M, N, K, K, 1, n_cu, false).us ? rows : 0;
 }
 
 // packed[n][line * 48 + b] = w[n][channel * 392 + frame * 196 + y * 14 + x] for b = x * 3 + channel < 42, else 0
@@ -1400,11 +1407,11 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
     const int dev = mvit_current_device("gemm");
     if (dev < 0) return MVIT_ERR_LAUNCH;
     const int n_cu = device_cu_count(dev);
-    TileChoice c = choose_tile(kind, p.M, p.N, p.k_chunk, p.K - (p.split_k - 1) * p.k_chunk, p.split_k, n_cu);
+    TileChoice c = choose_tile(kind, p.M, p.N, p.k_chunk, p.K - (p.split_k - 1) * p.k_chunk, p.split_k, n_cu, a->overlapped != 0);
     const bool all_256 = getenv("MVIT_GEMM_NO_HALF_TILES") != nullptr;
     if (all_256 && c.bm != 256 && pp_takes(kind, p.k_chunk, p.K - (p.split_k - 1) * p.k_chunk)) c = TileChoice{256, 256, 0.};
     // the column sums are per tile row: their granularity names the kernel (64 rows: 64 x 64 or 64 x 128 tiles, below)
-    if (kind == NT_SWIGLU_BWD && p.colsum != nullptr) c = colsum_rows == 64 ? choose_tile(kind, p.M, p.N, p.k_chunk, p.K, 1, n_cu, false) : full_rows_tile(kind, p.K, p.K);
+    if (kind == NT_SWIGLU_BWD && p.colsum != nullptr) c = colsum_rows == 64 ? choose_tile(kind, p.M, p.N, p.k_chunk, p.K, 1, n_cu, a->overlapped != 0, false) : full_rows_tile(kind, p.K, p.K);
     if (c.bm != 0) {
       auto run = [&](GemmParams q, const TileChoice& t) -> int {
         q.tiles_m = (int)((q.M + t.bm - 1) / t.bm);
@@ -1424,7 +1431,7 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
         q.C = static_cast<bf16_t*>(p.C) + head * p.ldc;
         if (p.R) q.R = static_cast<const bf16_t*>(p.R) + head * p.ldr;
         if (p.aux) q.aux = static_cast<bf16_t*>(p.aux) + head * p.ldaux;
-        return run(q, choose_tile(kind, q.M, q.N, q.K, q.K, 1, n_cu));
+        return run(q, choose_tile(kind, q.M, q.N, q.K, q.K, 1, n_cu, false));
       }
       const int rc = run(p, c);
       if (rc != MVIT_OK) return rc;
@@ -1510,16 +1517,16 @@ int mvit_gemm_wgrad_group(const mvit_gemm_args* list, int n, hipStream_t s) {
   return mvit_gemm_small_group(bm, bn, g, s);
 }
 
-extern "C" int mvit_gemm_wgrad_split_k(int64_t out_rows, int64_t out_cols, int64_t k) {
-  // Slices along the contraction for a product with few output tiles and a long contraction (a weight gradient, contracted
-  // over the tokens): the count with the lowest modelled time.  Every slice costs an fp32 partial tile written and read back
-  // (3.5 TB/s) and one more launch sums them.
+// Slices along the contraction for a product with few output tiles and a long contraction (a weight gradient, contracted
+// over the tokens): the count with the lowest modelled time.  Every slice costs an fp32 partial tile written and read back
+// (3.5 TB/s) and one more launch sums them.
+static int wgrad_split_k(int64_t out_rows, int64_t out_cols, int64_t k, bool overlapped) {
   if (out_rows <= 0 || out_cols <= 0 || k <= 0) return 1;
   int best = 1;
   double best_us = 1e30;
   for (int sk = 1; sk <= 16 && (sk == 1 || k / sk >= 512); ++sk) {
     const int64_t chunk = ((k + sk - 1) / sk + 63) / 64 * 64, slices = (k + chunk - 1) / chunk;
-    double us = choose_tile(TT_NONE, out_rows, out_cols, chunk, k - (slices - 1) * chunk, slices, 256).us;
+    double us = choose_tile(TT_NONE, out_rows, out_cols, chunk, k - (slices - 1) * chunk, slices, 256, overlapped).us;
     if (slices > 1) us += 5. + (double)slices * (double)out_rows * (double)out_cols * 4. / 3.5e6;
     if (us < best_us) {
       best_us = us;
@@ -1529,7 +1536,11 @@ extern "C" int mvit_gemm_wgrad_split_k(int64_t out_rows, int64_t out_cols, int64
   return best;
 }
 
+extern "C" int mvit_gemm_wgrad_split_k(int64_t out_rows, int64_t out_cols, int64_t k) { return wgrad_split_k(out_rows, out_cols, k, false); }
+
+extern "C" int mvit_gemm_wgrad_split_k_overlapped(int64_t out_rows, int64_t out_cols, int64_t k) { return wgrad_split_k(out_rows, out_cols, k, true); }
+
 extern "C" int mvit_gemm_swiglu_bwd_colsum_rows(int64_t M, int64_t N, int64_t K) {
-  const int bm = choose_tile(NT_SWIGLU_BWD, M, N, K, K, 1, 256).bm;
+  const int bm = choose_tile(NT_SWIGLU_BWD, M, N, K, K, 1, 256, false).bm;
   return bm == 0 || bm == 256 ? 256 : 64;
 }

@@ -27,7 +27,7 @@ class GemmArgs(C.Structure):
         ("C", _vp), ("ldc", _i64),
         ("R", _vp), ("ldr", _i64),
         ("aux", _vp), ("ldaux", _i64), ("aux_off", _i64),
-        ("workspace", _vp), ("workspace_bytes", _i64), ("split_k", _i32), ("row_sums", _vp), ("colsum_rows", _i32),
+        ("workspace", _vp), ("workspace_bytes", _i64), ("split_k", _i32), ("row_sums", _vp), ("colsum_rows", _i32), ("overlapped", _i32),
     ]
 
 
@@ -91,6 +91,7 @@ PROTOTYPES = {
     "mvit_cast2d": [_vp, _i64, _i32, _vp, _i64, _i32, _i64, _i64, _vp],
     "mvit_gemm": [C.POINTER(GemmArgs), _vp],
     "mvit_gemm_wgrad_split_k": [_i64, _i64, _i64],
+    "mvit_gemm_wgrad_split_k_overlapped": [_i64, _i64, _i64],
     "mvit_gemm_swiglu_bwd_colsum_rows": [_i64, _i64, _i64],
     "mvit_attn_fwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i64, _i32, _i32, _i64, _i64, _i64, _i64, _f32, _i32, _vp],
     "mvit_image_token_ranks": [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp],
@@ -111,7 +112,7 @@ PROTOTYPES = {
     "mvit_attn_bwd": [_vp] * 10 + [_i64, _vp, _vp] + [_i32, _i32, _i64, _i32, _i32] + [_i64] * 8 + [_f32, _i32, _vp],
 }
 EXPORTS = sorted(list(PROTOTYPES) + ["mvit_version", "mvit_last_error", "mvit_attn_bwd_delta_elems", "mvit_block_bwd_workspace_bytes"])
-HEADER_VERSION = 202  # MVIT_VERSION of include/mi355_vit.h these prototypes were written for
+HEADER_VERSION = 203  # MVIT_VERSION of include/mi355_vit.h these prototypes were written for
 
 _lib = None
 

@@ -269,6 +269,12 @@ def _block_forward_one_call(a, x, W, geo, attn_out, for_backward, output):
     return x2, saved
 
 
+def _block_split_k(out_rows: int, out_cols: int, rows: int) -> int:
+    """K slices of a block's weight gradient: those of a product beside the input-gradient chain, also where the second stream is
+    switched off, so that the gradients are the same bits either way."""
+    return ops.wgrad_split_k(out_rows, out_cols, rows, True)
+
+
 def _block_backward_one_call(a, dx2, x, saved, W, G):
     S, Cc = x.shape
     I, Ipad = W.I, W.Ipad
@@ -279,7 +285,7 @@ def _block_backward_one_call(a, dx2, x, saved, W, G):
         a.rstd1, a.n1, a.qkv, a.o, a.lse, a.x1, a.rstd2, a.n2, a.gu, a.h = p(0), p(1), p(2), p(3), p(4), p(5), p(6), p(7), p(8), p(9)
     else:
         a.rstd1, a.n1, a.qkv, a.o, a.lse, a.x1, a.rstd2, a.n2, a.gu, a.h = (t.data_ptr() for t in saved)
-    sk = ops.wgrad_split_k
+    sk = _block_split_k
     a.split_k_down, a.split_k_gate_up, a.split_k_proj, a.split_k_qkv = sk(Cc, I, S), sk(2 * Ipad, Cc, S), sk(Cc, Cc, S), sk(3 * Cc, Cc, S)
     lib = _lib.load()
     nbytes = lib.mvit_block_bwd_workspace_bytes(ctypes.byref(a))
@@ -384,35 +390,40 @@ def _block_backward(dx2: torch.Tensor, x: torch.Tensor, saved: tuple, W: BlockWe
             side.wait_event(ev)
             return fn()
 
+    beside = side is not None
+
+    def weight_grad(dy, act, out, bias_dtype, n=None):
+        return ops.weight_grad(dy, act, out, bias_dtype, n=n, split_k=_block_split_k(out.shape[0], out.shape[1], S), overlapped=beside)
+
     # ---- MLP: x2 = x1 + down(silu(g) * u)
     g_wd = torch.empty(C, I, dtype=gdt["mlp.down_proj.weight"], device=dev)
-    g_bd = off_chain(lambda: ops.weight_grad(dx2, h, g_wd, gdt["mlp.down_proj.bias"], n=I))
+    g_bd = off_chain(lambda: weight_grad(dx2, h, g_wd, gdt["mlp.down_proj.bias"], n=I))
     dgu = torch.empty(S, 2 * Ipad, dtype=x.dtype, device=dev)
     # the bf16 epilogue also hands back per-tile column sums of dgu, of its fp32 values: the gate / up bias gradient
     fused = x.dtype == torch.bfloat16
     part = torch.empty(-(-S // ops.swiglu_bwd_colsum_rows(S, Ipad, C)), 2 * Ipad, dtype=torch.float32, device=dev) if fused else None
-    ops.gemm(dx2, W.wdown, dgu, trans_b=True, epilogue=E.EPI_SWIGLU_BWD, residual=gu, aux_off=Ipad, colsum_partial=part)
+    ops.gemm(dx2, W.wdown, dgu, trans_b=True, epilogue=E.EPI_SWIGLU_BWD, residual=gu, aux_off=Ipad, colsum_partial=part, overlapped=beside)
     g_wgu = torch.empty(2 * Ipad, C, dtype=gdt["mlp.gate_proj.weight"], device=dev)
     b_gu = gdt["mlp.gate_proj.bias"]
-    g_bgu = off_chain(lambda: (ops.reduce_partials(part, b_gu), ops.weight_grad(dgu, n2, g_wgu, None))[0] if fused else ops.weight_grad(dgu, n2, g_wgu, b_gu))
+    g_bgu = off_chain(lambda: (ops.reduce_partials(part, b_gu), weight_grad(dgu, n2, g_wgu, None))[0] if fused else weight_grad(dgu, n2, g_wgu, b_gu))
     dn2 = torch.empty_like(x)
-    ops.gemm(dgu, W.wgu, dn2, trans_b=True)
+    ops.gemm(dgu, W.wgu, dn2, trans_b=True, overlapped=beside)
     dx1, g_n2 = ops.rmsnorm_bwd(dn2, x1, W.norm2.view(-1), rstd2, dx_add=dx2, w_grad_dtype=gdt["norm2.weight"])
 
     # ---- attention: x1 = x + proj(attn(rope(qkv(norm1(x)))))
     g_wp = torch.empty(C, C, dtype=gdt["attn.proj.weight"], device=dev)
-    g_bp = off_chain(lambda: ops.weight_grad(dx1, o, g_wp, gdt["attn.proj.bias"]))
+    g_bp = off_chain(lambda: weight_grad(dx1, o, g_wp, gdt["attn.proj.bias"]))
     d_o = dn2  # reuse the buffer
-    ops.gemm(dx1, W.wproj, d_o, trans_b=True)
+    ops.gemm(dx1, W.wproj, d_o, trans_b=True, overlapped=beside)
     dqkv = torch.empty_like(qkv)
     ops.attn_bwd(qkv[:, :C], qkv[:, C : 2 * C], qkv[:, 2 * C :], o, d_o, lse, geo.cu, geo.max_seqlen, H, hd, 1.0 / LOG2E,
                  dqkv[:, :C], dqkv[:, C : 2 * C], dqkv[:, 2 * C :], seg_order=geo.order)
     # dq arrives as the gradient with respect to the scaled, rotated queries: the same factor on the way back
     ops.rope_(dqkv, geo.cos, geo.sin, 2 * H, hd, backward=True, lead_heads=H, lead_scale=hd**-0.5 * LOG2E)
     g_wqkv = torch.empty(3 * C, C, dtype=gdt["attn.q_proj.weight"], device=dev)
-    g_bqkv = off_chain(lambda: ops.weight_grad(dqkv, n1, g_wqkv, gdt["attn.q_proj.bias"]))
+    g_bqkv = off_chain(lambda: weight_grad(dqkv, n1, g_wqkv, gdt["attn.q_proj.bias"]))
     dn1 = d_o
-    ops.gemm(dqkv, W.wqkv, dn1, trans_b=True)
+    ops.gemm(dqkv, W.wqkv, dn1, trans_b=True, overlapped=beside)
     dx, g_n1 = ops.rmsnorm_bwd(dn1, x, W.norm1.view(-1), rstd1, dx_add=dx1, w_grad_dtype=gdt["norm1.weight"])
     if side is not None:
         main.wait_stream(side)

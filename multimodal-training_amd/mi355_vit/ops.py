@@ -321,6 +321,7 @@ def gemm(
     split_k: int = 1,
     colsum_partial: Optional[torch.Tensor] = None,
     row_sums: Optional[torch.Tensor] = None,
+    overlapped: bool = False,
 ) -> torch.Tensor:
     """out[M, N] = epilogue(A . B^T) with A = a (or a^T if trans_a) and B = b (or b^T if trans_b), see include/mi355_vit.h.
 
@@ -329,6 +330,7 @@ def gemm(
     ``colsum_partial`` (EPI_SWIGLU_BWD only): fp32 [ceil(M/256) or ceil(M/64), out.stride(0)] receiving the column sums of that
     many rows of out each (see ``swiglu_bwd_colsum_rows``), before the rounding to out's dtype.
     ``row_sums`` (bf16, both operands transposed, plain epilogue): [M] of out's dtype, receives the sums of op(A) over k.
+    ``overlapped``: another stream's work runs beside this product and fills the compute units it leaves idle (no effect on results).
     """
     for t, nm in ((a, "a"), (b, "b"), (out, "out")):
         _rowmajor(t, f"gemm {nm}")
@@ -344,7 +346,7 @@ def gemm(
         raise ValueError(f"gemm: out {tuple(out.shape)} too small for M={M}, N={N}")
     args = GemmArgs()
     args.dtype, args.out_dtype = dt(a), dt(out)
-    args.trans_a, args.trans_b, args.epilogue = int(trans_a), int(trans_b), epilogue
+    args.trans_a, args.trans_b, args.epilogue, args.overlapped = int(trans_a), int(trans_b), epilogue, int(overlapped)
     args.M, args.N, args.K = M, N, K
     args.A, args.lda = a.data_ptr(), a.stride(0)
     args.B, args.ldb = b.data_ptr(), b.stride(0)
@@ -396,11 +398,13 @@ def gemm(
 
 
 @functools.lru_cache(maxsize=None)
-def wgrad_split_k(out_rows: int, out_cols: int, k: int) -> int:
+def wgrad_split_k(out_rows: int, out_cols: int, k: int, overlapped: bool = False) -> int:
     """K slices for a GEMM with few output tiles and a long contraction: the weight gradients (contraction over the
     tokens).  The model uses it for those only: on a forward or input-gradient GEMM a slice count chosen from the batch
-    size would make a row's result depend on how many rows share its batch."""
-    return _lib.load().mvit_gemm_wgrad_split_k(out_rows, out_cols, k)
+    size would make a row's result depend on how many rows share its batch.  ``overlapped``: the count for a product that shares the
+    GPU with another stream's."""
+    lib = _lib.load()
+    return (lib.mvit_gemm_wgrad_split_k_overlapped if overlapped else lib.mvit_gemm_wgrad_split_k)(out_rows, out_cols, k)
 
 
 @functools.lru_cache(maxsize=None)
@@ -412,14 +416,18 @@ def swiglu_bwd_colsum_rows(rows: int, cols: int, k: int) -> int:
 MAX_DIRECT_PITCH = 1 << 22  # elements; wider rows go to the register-staged product, which makes no row sums
 
 
-def weight_grad(dy: torch.Tensor, act: torch.Tensor, out: torch.Tensor, bias_dtype: Optional[torch.dtype], n: Optional[int] = None) -> Optional[torch.Tensor]:
+def weight_grad(dy: torch.Tensor, act: torch.Tensor, out: torch.Tensor, bias_dtype: Optional[torch.dtype], n: Optional[int] = None,
+                split_k: Optional[int] = None, overlapped: bool = False) -> Optional[torch.Tensor]:
     """Gradients of a Linear layer's weight (``out`` = dy^T act) and, with ``bias_dtype``, bias (returned: the column sums of
-    dy).  In bf16 the product sums the operand it reads anyway (not so with a row pitch beyond 32-bit lane offsets)."""
+    dy).  In bf16 the product sums the operand it reads anyway (not so with a row pitch beyond 32-bit lane offsets).
+    ``split_k``: K slices, by default those of a product that has the GPU to itself; ``overlapped`` as in ``gemm``."""
     fused = dy.dtype == torch.bfloat16 and bias_dtype == out.dtype and max(dy.stride(0), act.stride(0)) <= MAX_DIRECT_PITCH
     bias = None
     if bias_dtype is not None:
         bias = torch.empty(dy.shape[1], dtype=bias_dtype, device=dy.device) if fused else colsum(dy, bias_dtype)
-    gemm(dy, act, out, trans_a=True, trans_b=True, n=n, split_k=wgrad_split_k(out.shape[0], out.shape[1], dy.shape[0]), row_sums=bias if fused else None)
+    if split_k is None:
+        split_k = wgrad_split_k(out.shape[0], out.shape[1], dy.shape[0])
+    gemm(dy, act, out, trans_a=True, trans_b=True, n=n, split_k=split_k, row_sums=bias if fused else None, overlapped=overlapped)
     return bias
 
 

@@ -408,6 +408,28 @@ def test_gemm_half_height_tiles_give_the_same_bits_as_full_tiles(M, K, monkeypat
     assert max_rel_err(dgrad_half, a.cpu().double() @ w.cpu().double()) < TOL[dtype]
 
 
+@pytest.mark.parametrize("M,N,K", [(1601, 5112, 520), (3585, 2552, 520), (6657, 2552, 1288), (6657, 2552, 2056)])
+def test_gemm_input_gradient_has_the_same_bits_beside_another_stream(M, N, K):
+    """`overlapped` chooses another tile for these input gradients (256 or 192 x 128 rows and columns alone, 128 x 128 or 256 beside
+    another stream's work); no result depends on it, nor a weight gradient's, and nothing is written beyond the last row."""
+    _announce(f"gemm overlapped M={M} N={N} K={K}")
+    ops = _ops()
+    from mi355_vit import _lib as E
+
+    dtype = torch.bfloat16
+    dy, w, x = _rand((M, K), dtype, 1).to(DEV), _rand((K, N), dtype, 2, K**-0.5).to(DEV), _rand((M, N), dtype, 3).to(DEV)
+    got = []
+    for overlapped in (False, True):
+        out, gelu, grad = (torch.full((r + 8, N), 7.0, dtype=dtype, device=DEV) for r in (M, M, K))
+        ops.gemm(dy, w, out[:M], trans_b=True, overlapped=overlapped)
+        ops.gemm(dy, w, gelu[:M], trans_b=True, epilogue=E.EPI_GELU_BWD, residual=x, overlapped=overlapped)
+        bias = ops.weight_grad(dy, x, grad[:K], dtype, split_k=2, overlapped=overlapped)
+        got.append((out, gelu, grad, bias))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+    assert all(bool((t[-8:] == 7.0).all()) for t in got[0][:3])
+    assert max_rel_err(got[0][0][:M], dy.cpu().double() @ w.cpu().double()) < TOL[dtype]
+
+
 @pytest.mark.parametrize("epi", ["none", "bias", "bias_res", "gelu", "swiglu", "swiglu without aux"])
 @pytest.mark.parametrize("M,N", [(4353, 3840), (4607, 3840), (13057, 1280), (14336, 1280)])
 def test_gemm_rows_in_full_rounds_and_the_rest_give_the_same_bits_as_one_launch(M, N, epi, monkeypatch):

@@ -151,6 +151,24 @@ def test_second_stream_overlap_gives_identical_gradients():
         assert torch.equal(res[0][1][k], res[1][1][k]), k
 
 
+def test_products_are_told_whether_a_second_stream_runs_beside_them(monkeypatch):
+    """Backward products of a block are chosen as ones that share the GPU where its second stream runs, and only there: not the
+    forward's, not the merger's and the patch embedding's, and none with the second stream switched off."""
+    from mi355_vit import functional, ops
+
+    kw = dict(depth=2, hidden_size=256, intermediate_size=300, num_heads=8, out_hidden_size=128, fullatt_block_indexes=[1])
+    told, gemm = [], ops.gemm
+    monkeypatch.setattr(ops, "gemm", lambda *a, **k: (told.append(bool(k.get("overlapped"))), gemm(*a, **k))[1])
+    monkeypatch.setattr(functional, "BLOCK_CALLS", False)
+    pixels, gout = torch.randn(256, 1176), torch.randn(64, 128)
+    for overlap in (True, False):
+        monkeypatch.setattr(ops, "OVERLAP_WGRAD", overlap)
+        told.clear()
+        _run_gpu(_build(kw, 3, torch.bfloat16), pixels, torch.tensor([[1, 16, 16]]), gout)
+        merger, patch_embedding, block = 4, 1, 8
+        assert told == [False] * (1 + 2 * 4 + 2 + merger) + [overlap] * (2 * block) + [False] * patch_embedding
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("checkpoint", [False, True])
 def test_one_call_per_block_equals_the_call_by_call_sequence(dtype, checkpoint):
