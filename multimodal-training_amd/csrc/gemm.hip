@@ -1449,7 +1449,9 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
     return dispatch_trans<bf16_t, float>(a->trans_a, a->trans_b, epi, var, p, s);
   }
   MVIT_REQUIRE(a->out_dtype == MVIT_F32, "gemm: fp32 operands need fp32 output");
-  const int rc = mvit_gemm_f32(a->trans_a, a->trans_b, epi, p, s);
+  const int dev = mvit_current_device("gemm");
+  if (dev < 0) return MVIT_ERR_LAUNCH;
+  const int rc = mvit_gemm_f32(a->trans_a, a->trans_b, epi, p, device_cu_count(dev), s);
   if (rc != MVIT_OK) return rc;
   if (p.split_k > 1) {
     launch_splitk_reduce<float, float>(p, s);

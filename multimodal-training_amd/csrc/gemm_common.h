@@ -52,7 +52,7 @@ struct GemmGroup {
 };
 int mvit_gemm_small_group(int bm, int bn, GemmGroup& group, hipStream_t stream);                                // gemm_small.hip
 
-int mvit_gemm_f32(int ta, int tb, int epi, const GemmParams& p, hipStream_t stream);                        // gemm_f32.hip
+int mvit_gemm_f32(int ta, int tb, int epi, const GemmParams& p, int n_cu, hipStream_t stream);              // gemm_f32.hip
 
 namespace {
 

@@ -277,19 +277,21 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const GemmParams p) {
 // 45 / 49 at 1,536, 66 / 58 at 2,048; K = 6912 126 / 77 at 256 rows, 127 / 121 at 512).  Nearly a tile per unit stays whole: halves
 // are hardly faster alone (256 rows x 3840: 28.5 / 27.6), and beside a second stream's products a step of 256 rows took 3.19 ms with
 // them and 2.97 without.
-inline bool half_rows(const GemmParams& p) {
-  constexpr int64_t units = 256;
+inline bool half_rows(const GemmParams& p, int64_t units) {
   const int64_t tn = (p.N + 63) / 64 * p.split_k, tiles = (p.M + 63) / 64 * tn;
   const int64_t rounds = (tiles + units - 1) / units, half_rounds = ((p.M + 31) / 32 * tn + units - 1) / units;
   return tiles <= units * 3 / 4 || (rounds > 1 && rounds <= 3 && half_rounds < 2 * rounds);
 }
 
 // 32 x 32 tiles (a wave's share is one MFMA block) where every compute unit has at most one, or three where 32 x 64 tiles would be two
-// to a unit: the matrix pipes of a unit with two of those work 1.6 times as long as the average's.  us, 32 x 64 / 32 x 32, input
-// gradients K = 6912 x 1280: 64 and 128 rows (one each) 77 / 55, 256 (two) 77 / 80, 512 (three) 121 / 103, 768 (four; 64 x 64 128) - / 130, 1,024
-// 177 / 238; 4-block step of 512 rows 3.62 / 3.47 ms, of 64 (bound by the host) 2.21 / 2.18.
-inline bool quarters(const GemmParams& p) {
-  constexpr int64_t units = 256;
+// to a unit: there the matrix pipes of a unit with two of those work 1.6 times as long as the average's.  At other counts halving saves
+// no part of a round, or each tile's own steps cost more than it saves.  us, input gradients, 32 x 32 / 32 x 64 / 64 x 64 tiles by 32 x 32 tiles
+// per unit, K = 6912: one 56 / 78 / 128 (3840 columns, 32 rows), two 86 / 80 / 129 (1280 columns, 256 rows), three 107 / 125 / 129 (512), four 130 / 126 /
+// 130 (640), five 211 / 179 / 221 (896), seven 252 / 243 / 222 (1280); K = 1280: one 15.2 / 18.9 / 28.3, two 20.7 / 19.5 / 28.5, three 24.9 / 28.0 / 28.5,
+// four 30.0 / 28.2 / 28.9, five 39.9 / 38.0 / 46.2, seven 48.4 / 50.4 / 46.2.  Of 168 products (1280 and 3840 columns, K = 1280, 3840 and 6912, 32 to 1,536
+// rows, forward and input gradient) the tile taken is never more than 6 % behind the best, that at four per unit.  4-block step of 512 rows 3.62 ->
+// 3.47 ms, of 64 (bound by the host) 2.21 -> 2.18.
+inline bool quarters(const GemmParams& p, int64_t units) {
   const int64_t per_unit = ((p.M + 31) / 32 * ((p.N + 31) / 32) * p.split_k + units - 1) / units;
   return per_unit == 1 || per_unit == 3;
 }
@@ -307,41 +309,41 @@ int launch_f32_tiles(GemmParams p, hipStream_t stream) {
 }
 
 template <bool TA, bool TB, int EPI>
-int launch_f32(const GemmParams& p, hipStream_t stream) {
+int launch_f32(const GemmParams& p, int n_cu, hipStream_t stream) {
   if constexpr (!TA && EPI != MVIT_EPI_SWIGLU) {
-    if (quarters(p)) return launch_f32_tiles<TA, TB, EPI, 32, 32>(p, stream);
-    if (half_rows(p)) return launch_f32_tiles<TA, TB, EPI, 32>(p, stream);
+    if (quarters(p, n_cu)) return launch_f32_tiles<TA, TB, EPI, 32, 32>(p, stream);
+    if (half_rows(p, n_cu)) return launch_f32_tiles<TA, TB, EPI, 32>(p, stream);
   }
   return launch_f32_tiles<TA, TB, EPI, 64>(p, stream);
 }
 
 }  // namespace
 
-int mvit_gemm_f32(int ta, int tb, int epi, const GemmParams& p, hipStream_t s) {
+int mvit_gemm_f32(int ta, int tb, int epi, const GemmParams& p, int n_cu, hipStream_t s) {
   if (!ta && !tb) {
     switch (epi) {
-      case MVIT_EPI_NONE: return launch_f32<false, false, MVIT_EPI_NONE>(p, s);
-      case MVIT_EPI_BIAS: return launch_f32<false, false, MVIT_EPI_BIAS>(p, s);
-      case MVIT_EPI_BIAS_RES: return launch_f32<false, false, MVIT_EPI_BIAS_RES>(p, s);
-      case MVIT_EPI_BIAS_GELU: return launch_f32<false, false, MVIT_EPI_BIAS_GELU>(p, s);
-      case MVIT_EPI_SWIGLU: return launch_f32<false, false, MVIT_EPI_SWIGLU>(p, s);
-      case MVIT_EPI_ACCUM: return launch_f32<false, false, MVIT_EPI_ACCUM>(p, s);
+      case MVIT_EPI_NONE: return launch_f32<false, false, MVIT_EPI_NONE>(p, n_cu, s);
+      case MVIT_EPI_BIAS: return launch_f32<false, false, MVIT_EPI_BIAS>(p, n_cu, s);
+      case MVIT_EPI_BIAS_RES: return launch_f32<false, false, MVIT_EPI_BIAS_RES>(p, n_cu, s);
+      case MVIT_EPI_BIAS_GELU: return launch_f32<false, false, MVIT_EPI_BIAS_GELU>(p, n_cu, s);
+      case MVIT_EPI_SWIGLU: return launch_f32<false, false, MVIT_EPI_SWIGLU>(p, n_cu, s);
+      case MVIT_EPI_ACCUM: return launch_f32<false, false, MVIT_EPI_ACCUM>(p, n_cu, s);
       default: break;
     }
   } else if (!ta && tb) {
     switch (epi) {
-      case MVIT_EPI_NONE: return launch_f32<false, true, MVIT_EPI_NONE>(p, s);
-      case MVIT_EPI_BIAS: return launch_f32<false, true, MVIT_EPI_BIAS>(p, s);
-      case MVIT_EPI_SWIGLU_BWD: return launch_f32<false, true, MVIT_EPI_SWIGLU_BWD>(p, s);
-      case MVIT_EPI_GELU_BWD: return launch_f32<false, true, MVIT_EPI_GELU_BWD>(p, s);
-      case MVIT_EPI_ACCUM: return launch_f32<false, true, MVIT_EPI_ACCUM>(p, s);
+      case MVIT_EPI_NONE: return launch_f32<false, true, MVIT_EPI_NONE>(p, n_cu, s);
+      case MVIT_EPI_BIAS: return launch_f32<false, true, MVIT_EPI_BIAS>(p, n_cu, s);
+      case MVIT_EPI_SWIGLU_BWD: return launch_f32<false, true, MVIT_EPI_SWIGLU_BWD>(p, n_cu, s);
+      case MVIT_EPI_GELU_BWD: return launch_f32<false, true, MVIT_EPI_GELU_BWD>(p, n_cu, s);
+      case MVIT_EPI_ACCUM: return launch_f32<false, true, MVIT_EPI_ACCUM>(p, n_cu, s);
       default: break;
     }
   } else if (ta && tb) {
     switch (epi) {
-      case MVIT_EPI_NONE: return launch_f32<true, true, MVIT_EPI_NONE>(p, s);
-      case MVIT_EPI_BIAS: return launch_f32<true, true, MVIT_EPI_BIAS>(p, s);
-      case MVIT_EPI_ACCUM: return launch_f32<true, true, MVIT_EPI_ACCUM>(p, s);
+      case MVIT_EPI_NONE: return launch_f32<true, true, MVIT_EPI_NONE>(p, n_cu, s);
+      case MVIT_EPI_BIAS: return launch_f32<true, true, MVIT_EPI_BIAS>(p, n_cu, s);
+      case MVIT_EPI_ACCUM: return launch_f32<true, true, MVIT_EPI_ACCUM>(p, n_cu, s);
       default: break;
     }
   } else {
