@@ -1229,12 +1229,14 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
       consider(192, 128, 0.60, 0., 4., true);
     }
   }
-  // SwiGLU backward: the 256-row kernel as soon as its tiles give nearly half of the units work.  Its launch shares the GPU with
+  // SwiGLU backward: the 256-row kernel as soon as its tiles give half of the units work.  Its launch shares the GPU with
   // the down projection's weight gradient on the second stream, which fills the units it leaves idle, while two small tiles per
   // unit compete with it for the L2s.  ms per 32-block step, 64 x 64 / 64 x 128 / 128 x 128 / 256 x 256: 576 rows 9.56 / 9.53 / 9.87 / 10.48,
   // 1,600 14.8 / 14.6 / 14.4 / 14.8, 2,048 16.4 / 16.2 / 15.8 / 16.2, 2,304 18.0 / 17.8 / 18.0 / 17.5, 3,136 21.9 / 21.7 / 22.0 / 21.8,
   // 4,900 31.8 / 31.4 / 31.0 / 30.6, 6,084 37.2 / 36.7 / 36.2 / 35.8 (alone 128 x 128 is ahead up to 20,000 rows, 165 us against 185 at 14,336)
-  if (kind == NT_SWIGLU_BWD && full_rows && 32 * ((M + 255) / 256) * ((N + 255) / 256) >= 15 * n_cu) best = full_rows_tile(kind, k_chunk, k_last);
+  // The line stays at one half, although 256 x 256 is ahead at 2,304 rows, just below it: the tile decides how many rows a partial
+  // column sum has, so moving the line changes the rounding of the gate / up bias gradients.
+  if (kind == NT_SWIGLU_BWD && full_rows && 2 * ((M + 255) / 256) * ((N + 255) / 256) >= n_cu) best = full_rows_tile(kind, k_chunk, k_last);
   return best;
 }
 

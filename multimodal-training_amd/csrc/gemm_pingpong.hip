@@ -37,7 +37,8 @@ struct PpCfg {
   static constexpr int BM = 256, BN = 256, BK = 64, NTHREADS = 512;
   static constexpr int HALF = 16384, STAGE = 4 * HALF;      // A0 | A1 | B0 | B1
   static constexpr int BIAS_OFF = 2 * STAGE, BIAS_BYTES = 2 * 8 * 256;  // two tiles' worth, 256 bytes per wave
-  static constexpr int LDS = BIAS_OFF + BIAS_BYTES;
+  static constexpr int SUMS_BYTES = 32768;  // SwiGLU backward, in place of the biases: 16 lanes' column sums of all 256 columns, gate and up
+  static constexpr int lds(int epi) { return BIAS_OFF + (epi == MVIT_EPI_SWIGLU_BWD ? SUMS_BYTES : BIAS_BYTES); }
   static constexpr int MIN_K = 2 * BK + 1;  // at least three K tiles
 };
 
@@ -350,32 +351,47 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
 #pragma unroll
       for (int g = 0; g < 2; ++g) load8(reinterpret_cast<const bf16_t*>(bl + g * 64 + g4 * 16), hb[g]);
     }
-    float no_cs[16];  // SW_BWD: column sums over the lane's rows, of the eight columns' gate and up halves
+    // SW_BWD: column sums over the lane's rows, of the eight columns' gate and up halves.  They are added in the order of gemm_dl_kernel,
+    // so that the sums of 256 rows have the same bits whichever kernel made them: lane l % 16 adds rows 32 a + {0, 16, 128, 144} for
+    // a = 0 .. 3, i.e. group 1 goes on from group 0's sums, and the sums of the sixteen lanes are added one after the other.
+    float no_cs[16];
     const bool do_cs = SW_BWD && p.colsum != nullptr;
-    float* cs_lds = reinterpret_cast<float*>(smem_raw + PpCfg::BIAS_OFF);
-    // column half g is through: its sums over the 16 lanes of a row block, in a fixed order, parked for the other row group
-    auto park_sums = [&](int g) {
+    // Group 1's epilogue lies behind the barrier that group 0 arrives at after its own, so it finds group 0's sums there.  Chunks of
+    // four sums, chunk c of lane i in slot c ^ i: stores of sixteen lanes, and loads of one chunk of each, fall on all banks.
+    float* cs_lds = reinterpret_cast<float*>(smem_raw + PpCfg::BIAS_OFF) + wn * 2048;
+    auto chunk_of = [&](int g, int h) { return reinterpret_cast<f32x4*>(cs_lds + g * 1024 + i16 * 64 + ((g4 * 4 + h) ^ i16) * 4); };
+    auto begin_sums = [&](int g) {
       if constexpr (SW_BWD) {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          float t = no_cs[e];
-          t += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, t), 0x128, 0xf, 0xf, false));  // row_ror:8, 4, 2, 1
-          t += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, t), 0x124, 0xf, 0xf, false));
-          t += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, t), 0x122, 0xf, 0xf, false));
-          t += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, t), 0x121, 0xf, 0xf, false));
-          if (i16 == 0) cs_lds[wv * 128 + g * 64 + (e >> 3) * 32 + tr_first_column(g4) + (e & 7)] = t;
-          no_cs[e] = 0.f;
+        for (int h = 0; h < 4; ++h) {
+          const f32x4 t = do_cs && wm == 1 ? *chunk_of(g, h) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) no_cs[4 * h + e] = t[e];
         }
       }
     };
-    if constexpr (SW_BWD) {
+    auto end_sums = [&](int g) {
+      if constexpr (SW_BWD) {
 #pragma unroll
-      for (int e = 0; e < 16; ++e) no_cs[e] = 0.f;
-    }
+        for (int h = 0; h < 4; ++h) *chunk_of(g, h) = f32x4{no_cs[4 * h], no_cs[4 * h + 1], no_cs[4 * h + 2], no_cs[4 * h + 3]};
+        if (wm == 0) {
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // before this group's next barrier
+        } else {
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          float t = 0.f;
+#pragma unroll
+          for (int k = 0; k < 16; ++k) t += cs_lds[g * 1024 + k * 64 + (((lane >> 2) ^ k) << 2) + (lane & 3)];
+          const int64_t n = n0 + g * 128 + wn * 32 + tr_first_column(g4) + (lane & 7);
+          if (n < p.N) p.colsum[m0 / BM * p.ldc + (lane & 8 ? p.aux_off : 0) + n] = t;
+        }
+      }
+    };
     float* ws = to_ws ? p.workspace + (int64_t)slice * p.M * p.N : nullptr;
     constexpr int NG = DUAL ? 1 : 2, ITEMS = 8 * NG;
-    // item -> row block and column half: by rows, or all rows of a half first where their sums are wanted
-    auto block_of = [](int it) { return SW_BWD ? it & 7 : it / NG; };
+    // item -> row block and column half: by rows, or all rows of a half first, in the order of their sums
+    auto block_of = [](int it) { return SW_BWD ? (it & 1) | ((it & 2) << 1) | ((it & 4) >> 1) : it / NG; };
     auto half_of = [](int it) { return SW_BWD ? it >> 3 : it % NG; };
     auto row_of = [&](int it) { return m_lane + (block_of(it) >> 2) * 128 + (block_of(it) & 3) * 16; };
     auto values = [&](int it, float (&v)[8], float (&u)[8]) {
@@ -415,6 +431,7 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
         for (int it = 0; it < DEPTH; ++it) fetch(it, pre[it]);
 #pragma unroll
         for (int it = 0; it < ITEMS; ++it) {
+          if ((it & 7) == 0) begin_sums(it >> 3);
           float v[8], u[8];
           values(it, v, u);
           bf16x8 now[NIN];
@@ -423,7 +440,7 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
           if (it + DEPTH < ITEMS) fetch(it + DEPTH, pre[it % DEPTH]);
           if (it == ITEMS - DEPTH && have) issue_first();  // behind the last of this tile's input loads
           emit8_impl<T, TO, EPI, true, true>(p, row_of(it), n_lane[half_of(it)], v, u, now, no_cs, do_cs, HAS_BIAS ? hb[half_of(it)] : nullptr, nullptr);
-          if (do_cs && (it & 7) == 7) park_sums(it >> 3);
+          if (do_cs && (it & 7) == 7) end_sums(it >> 3);
           __builtin_amdgcn_sched_barrier(0);
         }
       } else {
@@ -439,10 +456,11 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
       if (have && HAS_IN) issue_first();
 #pragma unroll
       for (int it = 0; it < ITEMS; ++it) {
+        if (do_cs && it == 8) end_sums(0);
+        if ((it & 7) == 0) begin_sums(it >> 3);
         float v[8], u[8];
         values(it, v, u);
         const int64_t m = row_of(it), n = n_lane[half_of(it)];
-        if (do_cs && (it & 7) == 0 && it > 0) park_sums((it >> 3) - 1);
         if (m >= p.M || n >= p.N) continue;
         if (to_ws) {
           float* w = ws + m * p.N + n;
@@ -455,24 +473,8 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
           emit8<T, TO, EPI>(p, m, n, v, u, false, no_cs, do_cs);
         }
       }
-      if (do_cs) park_sums(NG - 1);
+      if (do_cs) end_sums(NG - 1);
       pp_wait_vm<0>();  // the count of this path's memory instructions is not known to the waits of the next tile
-    }
-    if constexpr (SW_BWD) {
-      if (do_cs) {
-        // group 1 is one barrier behind: when it is through this one, group 0 has arrived at its next and parked its sums long ago
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        pp_barrier();
-        if (wm == 1) {
-          const int g = lane >> 5, col = lane & 31;
-#pragma unroll
-          for (int half = 0; half < 2; ++half) {
-            const int at = wn * 128 + g * 64 + half * 32 + col;
-            const int64_t n = n0 + g * 128 + wn * 32 + col;
-            if (n < p.N) p.colsum[m0 / BM * p.ldc + (half ? p.aux_off : 0) + n] = cs_lds[at] + cs_lds[4 * 128 + at];
-          }
-        }
-      }
     }
     if (!have) break;
   }
@@ -482,16 +484,16 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
 }  // namespace
 
 int mvit_gemm_pp(GemmTiledKind kind, const GemmParams& p, int n_cu, hipStream_t stream) {
-  auto go = [&](auto kern, bool (&attr_set_on)[MVIT_MAX_DEVICES]) -> int {
+  auto go = [&](auto kern, bool (&attr_set_on)[MVIT_MAX_DEVICES], int lds = PpCfg::lds(MVIT_EPI_NONE)) -> int {
     const int dev = mvit_current_device("gemm");
     if (dev < 0) return MVIT_ERR_LAUNCH;
     if (!attr_set_on[dev]) {  // dynamic LDS above 64 KiB is opted into once per kernel and device
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, PpCfg::LDS);
-      if (e != hipSuccess) return mvit_set_error(MVIT_ERR_LAUNCH, "gemm: hipFuncSetAttribute(%d B LDS): %s", PpCfg::LDS, hipGetErrorString(e));
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+      if (e != hipSuccess) return mvit_set_error(MVIT_ERR_LAUNCH, "gemm: hipFuncSetAttribute(%d B LDS): %s", lds, hipGetErrorString(e));
       attr_set_on[dev] = true;
     }
     const int want = (p.tiles_m * p.tiles_n * p.split_k + 7) / 8 * 8;
-    hipLaunchKernelGGL(kern, want < n_cu ? want : n_cu, PpCfg::NTHREADS, PpCfg::LDS, stream, p);
+    hipLaunchKernelGGL(kern, want < n_cu ? want : n_cu, PpCfg::NTHREADS, lds, stream, p);
     MVIT_CHECK_LAUNCH("gemm");
     return MVIT_OK;
   };
@@ -504,7 +506,7 @@ int mvit_gemm_pp(GemmTiledKind kind, const GemmParams& p, int n_cu, hipStream_t 
     case NN_SWIGLU: return go(gemm_pp_kernel<bf16_t, false, false, MVIT_EPI_SWIGLU>, set[4]);
     case NT_NONE: return go(gemm_pp_kernel<bf16_t, false, true, MVIT_EPI_NONE>, set[5]);
     case NT_GELU_BWD: return go(gemm_pp_kernel<bf16_t, false, true, MVIT_EPI_GELU_BWD>, set[6]);
-    case NT_SWIGLU_BWD: return go(gemm_pp_kernel<bf16_t, false, true, MVIT_EPI_SWIGLU_BWD>, set[9]);
+    case NT_SWIGLU_BWD: return go(gemm_pp_kernel<bf16_t, false, true, MVIT_EPI_SWIGLU_BWD>, set[9], PpCfg::lds(MVIT_EPI_SWIGLU_BWD));
     case TT_NONE: return go(gemm_pp_kernel<bf16_t, true, true, MVIT_EPI_NONE>, set[7]);
     case TT_NONE_F32: return go(gemm_pp_kernel<float, true, true, MVIT_EPI_NONE>, set[8]);
     default: return mvit_set_error(MVIT_ERR_UNSUPPORTED, "gemm: product kind %d has no 256 x 256 ping-pong kernel", (int)kind);

@@ -335,6 +335,26 @@ __device__ __forceinline__ void gemm_small_tile(const GemmParams& p, const unsig
   for (int g = 0; g < (CAN_CS ? NG : 1); ++g)
 #pragma unroll
     for (int e = 0; e < 16; ++e) cs[g][e] = 0.f;
+  // A lane's sums over two row blocks (32 rows) meet those of the 16 lanes that share its columns, parked in LDS in chunks of four, chunk
+  // c of lane i in slot c ^ i: all banks.  A row of sums is 64 rows: 32 lanes' sums, added one after the other in the order of the
+  // rows, so that it has the same bits whichever tile of this file made it (a tile of 128 rows makes two).
+  constexpr int HALVES = BM / 64, PITCH = 2 * NCOLS;
+  float* red = reinterpret_cast<float*>(smem_raw);
+  auto park_sums = [&](int pair) {
+    if constexpr (CAN_CS) {
+      static_assert(S::WM % 32 == 0 && BM % 64 == 0 && BM / 2 * PITCH * 4 <= S::LDS, "pairs of row blocks, whose sums fit the operand stages");
+#pragma unroll
+      for (int g = 0; g < NG; ++g)
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const int chunk = ((h >> 1) * NCOLS + (int)(n_lane[g] - n0)) / 4 + (h & 1);
+          *reinterpret_cast<f32x4*>(red + (wm * (S::WM / 2) + pair * 16 + i16) * PITCH + (chunk ^ i16) * 4) =
+              f32x4{cs[g][4 * h], cs[g][4 * h + 1], cs[g][4 * h + 2], cs[g][4 * h + 3]};
+          cs[g][4 * h] = cs[g][4 * h + 1] = cs[g][4 * h + 2] = cs[g][4 * h + 3] = 0.f;
+        }
+    }
+  };
+  if (do_cs) __syncthreads();  // the last K tile has been consumed
   float* ws = to_ws ? p.workspace + (int64_t)slice * p.M * p.N : nullptr;
   if constexpr (ROW_SUMS) {
 #pragma unroll
@@ -350,6 +370,7 @@ __device__ __forceinline__ void gemm_small_tile(const GemmParams& p, const unsig
   for (int it = 0; it < ITEMS; ++it) {
     const int a = it / NG, g = it % NG;
     const int64_t m = row_of(it), n = n_lane[g];
+    if (do_cs && g == 0 && a % 2 == 0 && a > 0) park_sums(a / 2 - 1);
     float v[8], u[8];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -380,26 +401,14 @@ __device__ __forceinline__ void gemm_small_tile(const GemmParams& p, const unsig
     }
   }
   if constexpr (CAN_CS) {
-    // a lane's sums over its rows meet those of the 16 lanes and S::WGM waves that share its columns: parked in LDS (rows four
-    // floats apart in their banks), added in a fixed order
     if (do_cs) {
-      // tiles of 128 rows give two rows of sums: their two halves are the waves of wm = 0 and 1
-      constexpr int HALVES = BM / 64, ROWS = S::WGM * 16 / HALVES, PITCH = 2 * NCOLS + 4;
-      static_assert(S::WGM % HALVES == 0 && HALVES * ROWS * PITCH * 4 <= S::LDS, "64 rows per row of sums, which fit the operand stages");
-      float* red = reinterpret_cast<float*>(smem_raw);
-      __syncthreads();  // the last K tile has been consumed
-#pragma unroll
-      for (int g = 0; g < NG; ++g)
-#pragma unroll
-        for (int h = 0; h < 4; ++h)
-          *reinterpret_cast<f32x4*>(red + (wm * 16 + i16) * PITCH + (h >> 1) * NCOLS + (int)(n_lane[g] - n0) + (h & 1) * 4) =
-              f32x4{cs[g][4 * h], cs[g][4 * h + 1], cs[g][4 * h + 2], cs[g][4 * h + 3]};
+      park_sums(NA / 2 - 1);
       __syncthreads();
-      for (int c = threadIdx.x; c < HALVES * 2 * NCOLS; c += S::NTHREADS) {
-        const int part = c / (2 * NCOLS), cc = c % (2 * NCOLS), half = cc / NCOLS, col = cc % NCOLS;
+      for (int c = threadIdx.x; c < HALVES * PITCH; c += S::NTHREADS) {
+        const int part = c / PITCH, cc = c % PITCH, half = cc / NCOLS, col = cc % NCOLS;
         float t = 0.f;
 #pragma unroll
-        for (int r = 0; r < ROWS; ++r) t += red[(part * ROWS + r) * PITCH + cc];
+        for (int r = 0; r < 32; ++r) t += red[(part * 32 + r) * PITCH + (((cc >> 2) ^ (r & 15)) << 2) + (cc & 3)];
         if (n0 + col < p.N && m0 + part * 64 < p.M) p.colsum[((int64_t)tm * HALVES + part) * p.ldc + (half ? p.aux_off : 0) + n0 + col] = t;
       }
     }

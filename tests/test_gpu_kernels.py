@@ -618,6 +618,39 @@ def test_swiglu_backward_column_sums_are_of_unrounded_values(M, N, K, per, dtype
     assert bool((part[:, N : N + 8] == 7.0).all()) and bool((out[:, N : N + 8] == 7.0).all())
 
 
+@pytest.mark.parametrize("per,M,N,K", [(64, 100, 72, 64), (64, 1030, 3456, 1280), (64, 2085, 3456, 1280), (256, 300, 264, 64), (256, 300, 264, 192), (256, 5000, 3456, 200)])
+def test_swiglu_backward_column_sums_have_one_order_of_addition(per, M, N, K):
+    """The gate / up bias gradient does not depend on the tile that made its parts: per 64 rows on tiles of 64 x 64, 64 x 128 and
+    128 x 128, per 256 rows on both kernels of 256 x 256 tiles, whole and partial, the fp32 values are added in one order.  The values
+    here are exact (one product each, a saturated gate), so the sums are those of plain fp32 additions in that order, bit for bit."""
+    _announce(f"gemm swiglu backward column sums, order, {M}x{N}x{K} per {per}")
+    ops = _ops()
+    from mi355_vit import _lib as E
+
+    gen = torch.Generator().manual_seed(M + N)
+    power = lambda *shape: torch.exp2(torch.randint(-3, 4, shape, generator=gen).float())  # noqa: E731
+    dy, w = torch.zeros(M, K), torch.zeros(K, N)
+    dy[:, 0], w[0] = torch.randn(M, generator=gen).bfloat16().float(), power(N)
+    u = power(M, N)
+    gu = torch.cat([torch.full((M, N), 128.0), u], 1)  # sigmoid(128) = 1: silu = 128, its derivative 1
+    out, part = torch.empty(M, 2 * N, dtype=torch.bfloat16, device=DEV), torch.empty(-(-M // per), 2 * N, device=DEV)
+    ops.gemm(dy.bfloat16().to(DEV), w.bfloat16().to(DEV), out, trans_b=True, epilogue=E.EPI_SWIGLU_BWD, residual=gu.bfloat16().to(DEV), aux_off=N, colsum_partial=part)
+    v = dy[:, :1] * w[:1]
+    exact = torch.cat([v * u, v * 128], 1)
+    assert torch.equal(out.cpu().float(), exact)
+    rows = torch.nn.functional.pad(exact, (0, 0, 0, -M % per)).view(-1, per, 2 * N)
+    # lane i of 16 adds rows `first + i`, one after the other; then the lanes' sums are added one after the other
+    firsts = [[0, 16], [32, 48]] if per == 64 else [[32 * a + b for a in range(4) for b in (0, 16, 128, 144)]]
+    total = torch.zeros(rows.shape[0], 2 * N)
+    for group in firsts:
+        lanes = torch.zeros(rows.shape[0], 16, 2 * N)
+        for first in group:
+            lanes += rows[:, first : first + 16]
+        for i in range(16):
+            total += lanes[:, i]
+    assert torch.equal(part.cpu(), total)
+
+
 @pytest.mark.parametrize("M,N,K,per", [(1, 72, 136, 256), (255, 264, 192, 256), (257, 136, 192, 256), (513, 520, 136, 256), (2600, 3456, 192, 256),
                                        (1920, 3456, 192, 64), (1985, 3456, 136, 64), (2047, 3400, 192, 64)])
 def test_swiglu_backward_column_sums_of_longer_contractions(M, N, K, per):
