@@ -257,7 +257,10 @@ int mvit_attn_bwd(const void* q, const void* k, const void* v, const void* o, co
  *            [S,2*Ipad], dn [S,C], dx1 [S,C], dqkv [S,3C] and `workspace` (mvit_block_bwd_workspace_bytes) as scratch.
  *            split_k_*: K slices of the four weight-gradient GEMMs (>= 1).  side_stream (may be null): a second stream
  *            of the caller's on which weight and bias gradients run beside the input-gradient chain; it then needs
- *            five events of the caller's (hipEvent_t), and the call leaves the main stream waiting for the side one. */
+ *            five events of the caller's (hipEvent_t), and the call leaves the main stream waiting for the side one.
+ *            A bf16 block of so little work that the host's launches cost more than the GPU's idle units does not use
+ *            it (mvit_block_bwd_uses_side_stream; the events are asked for all the same): its four weight gradients are
+ *            one launch on the main stream, behind the chain, and its column sums another, with the same results. */
 typedef struct mvit_block_args {
   int dtype, grad_dtype;
   int C, I, Ipad, nheads, head_dim;
@@ -282,6 +285,9 @@ typedef struct mvit_block_args {
 
 int mvit_block_fwd(const mvit_block_args* args, mvit_stream_t stream);
 int64_t mvit_block_bwd_workspace_bytes(const mvit_block_args* args);
+/* Host-only: whether the call runs weight gradients on a given side_stream (1) or in one launch behind the input-gradient
+ * chain (0).  Of the arguments only dtypes, sizes and split_k_* are looked at. */
+int mvit_block_bwd_uses_side_stream(const mvit_block_args* args);
 int mvit_block_bwd(const mvit_block_args* args, mvit_stream_t stream);
 
 /* ---------------------------------------------------------------- vision -> text hand-off */

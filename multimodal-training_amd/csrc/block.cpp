@@ -14,12 +14,20 @@ namespace {
 // work-groups (= partial rows) of the RMSNorm backward: four rows at a time each, up to 1,024 of them
 inline int rms_partials(int64_t rows) { return (int)(rows < 1 ? 1 : (rows + 3) / 4 < 1024 ? (rows + 3) / 4 : 1024); }
 
-// Up to how many rows the weight gradients go in one launch behind the input-gradient chain, and the column sums in another,
-// instead of starting on the second stream as soon as their inputs are complete: seven launches and ten event calls fewer per
-// block.  A host that issues slower than the GPU computes gains them, and so few rows leave the GPU little to overlap.  ms per
-// 32-block step, second stream / one launch: 64 rows 12.7 / 9.3, 256 12.9 / 9.7, 1,024 13.2 / 11.6, where the GPU is the slower side
-// 1,296 13.21 / 13.35, 1,600 14.6 / 14.9.
-constexpr int64_t GROUP_MAX_ROWS = 1280;
+// Whether the weight gradients go in one launch behind the input-gradient chain, and the column sums in another, instead of starting
+// on the second stream as soon as their inputs are complete: seven launches and ten event calls fewer per block.  A host that issues
+// slower than the GPU computes gains them, and so few rows leave the GPU little to overlap; where the GPU is the slower side its idle
+// units are worth more.  So the line is one of work: the products of a block of 1280 columns (MLP 3420) of 1,280 rows, the reading and
+// writing of the weights counted as 100 rows more.  ms per 32-block step of that width, second stream / one launch: 64 rows 12.7 / 9.3,
+// 256 12.9 / 9.7, 1,024 13.2 / 11.6, 1,296 13.21 / 13.35, 1,600 14.6 / 14.9; per 8-block step, 1920 (MLP 5120): 512 rows (in) 3.61 / 3.34,
+// 640 (out) 3.85 / 3.80, 768 3.93 / 4.03, 1,280 4.79 / 5.29; 2560 (6840): 128 (in) 3.70 / 3.63, 256 (out) 3.90 / 4.07, 1,024 6.14 / 6.91; 3840 (10240):
+// 64 (out) 5.04 / 5.08, 512 8.42 / 9.10.  Narrower blocks stop at 1,280 rows too (not measured beyond).
+constexpr int64_t GROUP_MAX_ROWS = 1280, GROUP_WEIGHT_ROWS = 100, GROUP_MAX_WORK = (GROUP_MAX_ROWS + GROUP_WEIGHT_ROWS) * 1280 * (4 * 1280 + 3 * 3420);
+inline bool grouped_wgrads(const mvit_block_args* a) {
+  return a->dtype == MVIT_BF16 && a->grad_dtype == MVIT_BF16 && a->S <= GROUP_MAX_ROWS &&
+         (double)(a->S + GROUP_WEIGHT_ROWS) * a->C * (4. * a->C + 3. * a->I) <= (double)GROUP_MAX_WORK && a->split_k_down == 1 &&
+         a->split_k_gate_up == 1 && a->split_k_proj == 1 && a->split_k_qkv == 1;
+}
 
 struct Bump {  // hands out 256-byte aligned pieces of the caller's workspace
   char* base;
@@ -152,6 +160,8 @@ extern "C" int64_t mvit_block_bwd_workspace_bytes(const mvit_block_args* a) {
   return plan_bwd_workspace(a, nullptr).total;
 }
 
+extern "C" int mvit_block_bwd_uses_side_stream(const mvit_block_args* a) { return a != nullptr && !grouped_wgrads(a); }
+
 extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   if (int rc = check_block("block_bwd", a)) return rc;
   MVIT_REQUIRE(a->gu && a->dx2 && a->dx && a->dgu && a->dn && a->dx1 && a->dqkv, "block_bwd: null gradient buffer");
@@ -159,8 +169,7 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
                "block_bwd: null parameter-gradient buffer");
   MVIT_REQUIRE(a->grad_dtype == MVIT_BF16 || a->grad_dtype == MVIT_F32, "block_bwd: grad_dtype %d", a->grad_dtype);
   MVIT_REQUIRE(a->split_k_down >= 1 && a->split_k_gate_up >= 1 && a->split_k_proj >= 1 && a->split_k_qkv >= 1, "block_bwd: split_k counts must be >= 1");
-  const bool grouped = a->dtype == MVIT_BF16 && a->grad_dtype == MVIT_BF16 && a->S <= GROUP_MAX_ROWS && a->split_k_down == 1 && a->split_k_gate_up == 1 &&
-                       a->split_k_proj == 1 && a->split_k_qkv == 1;
+  const bool grouped = grouped_wgrads(a);
   const bool two = a->side_stream != nullptr && !grouped;
   if (a->side_stream != nullptr) MVIT_REQUIRE(a->events[0] && a->events[1] && a->events[2] && a->events[3] && a->events[4], "block_bwd: a second stream needs five events");
   if (a->S == 0) return MVIT_OK;

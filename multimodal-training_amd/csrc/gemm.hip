@@ -1195,6 +1195,12 @@ struct TileChoice {
 TileChoice full_rows_tile(GemmTiledKind kind, int64_t k_chunk, int64_t k_last) {
   return pp_takes(kind, k_chunk, k_last) ? TileChoice{256, 256, 0.} : TileChoice{0, 0, 0.};
 }
+// The small tiles of weight gradients, two work-groups to a unit
+struct TileTimes {
+  int bm, bn;
+  double one, two, per_tile;
+};
+constexpr TileTimes WGRAD_TILES[] = {{64, 64, 0.23, 0.36, 2.}, {64, 128, 0.37, 0.52, 2.}, {128, 128, 0.60, 0.72, 2.5}};
 // `full_rows`: whether that kernel may be chosen
 TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk, int64_t k_last, int64_t slices, int n_cu, bool overlapped, bool full_rows = true) {
   const bool tt = kind == TT_NONE || kind == TT_NONE_F32;
@@ -1219,11 +1225,13 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
     consider(64, 64, 0.30, 0.43, 2.);
     consider(64, 128, 0.47, 0.70, 2.);
     consider(128, 128, 0.55, 0.90, 5.);
+  } else if (tt) {
+    for (const TileTimes& t : WGRAD_TILES) consider(t.bm, t.bn, t.one, t.two, t.per_tile);
   } else {
-    if (!swiglu) consider(64, 64, tt ? 0.23 : 0.19, 0.36, 2.);
+    if (!swiglu) consider(64, 64, 0.19, 0.36, 2.);
     consider(64, 128, 0.37, 0.52, 2.);
     consider(128, 128, 0.60, 0.72, swiglu ? 6. : 2.5);
-    if (!swiglu && !tt) {
+    if (!swiglu) {
       consider(64, 64, 0.18, 0., 2., true);
       consider(128, 128, 0.44, 0., 3., true);
       consider(192, 128, 0.60, 0., 4., true);
@@ -1486,10 +1494,9 @@ int mvit_gemm_wgrad_group(const mvit_gemm_args* list, int n, hipStream_t s) {
   if (dev < 0) return MVIT_ERR_LAUNCH;
   const int n_cu = device_cu_count(dev);
   // one tile shape for all of them: the model of choose_tile over the sum of their tiles
-  struct { int bm, bn; double one, two, per_tile; } const shapes[] = {{64, 64, 0.23, 0.36, 2.}, {64, 128, 0.37, 0.52, 2.}, {128, 128, 0.60, 0.72, 2.5}};
   int bm = 128, bn = 128;
   double best = 1e30;
-  for (const auto& t : shapes) {
+  for (const TileTimes& t : WGRAD_TILES) {
     int64_t items = 0, k = 0;
     for (int i = 0; i < n; ++i) {
       items += ((list[i].M + t.bm - 1) / t.bm) * ((list[i].N + t.bn - 1) / t.bn);

@@ -109,6 +109,7 @@ PROTOTYPES = {
     "mvit_patch_embed_frames": [_vp, _i32, _i64, _vp, _i64, _vp, _i64, _i32, C.c_double] + [_f32] * 6 + [_vp],
     "mvit_block_fwd": [C.POINTER(BlockArgs), _vp],
     "mvit_block_bwd": [C.POINTER(BlockArgs), _vp],
+    "mvit_block_bwd_uses_side_stream": [C.POINTER(BlockArgs)],
     "mvit_attn_bwd": [_vp] * 10 + [_i64, _vp, _vp] + [_i32, _i32, _i64, _i32, _i32] + [_i64] * 8 + [_f32, _i32, _vp],
 }
 EXPORTS = sorted(list(PROTOTYPES) + ["mvit_version", "mvit_last_error", "mvit_attn_bwd_delta_elems", "mvit_block_bwd_workspace_bytes"])

@@ -166,8 +166,8 @@ class AttnGeometry:
                 and (self.order is None or (self.order.dtype == torch.int32 and self.order.is_contiguous() and self.order.numel() == self.cu.numel() - 1)))
 
 
-# One C call per block and direction (mvit_block_fwd / mvit_block_bwd) instead of one per kernel: the same launches with
-# the same operands, issued from inside the library.  MVIT_BLOCK_CALLS=0 keeps the call-by-call sequence below, which is
+# One C call per block and direction (mvit_block_fwd / mvit_block_bwd) instead of one per kernel: the same steps on the
+# same operands, issued from inside the library, where the weight gradients of a few rows are one launch.  MVIT_BLOCK_CALLS=0 keeps the call-by-call sequence below, which is
 # also what runs while launches are being timed one by one (ops.set_trace) and for parameters of mixed gradient dtypes.
 BLOCK_CALLS = os.environ.get("MVIT_BLOCK_CALLS", "1") != "0"
 _join_events: dict = {}

@@ -466,3 +466,27 @@ def test_weight_gradient_slices_follow_whether_another_stream_runs_beside():
     for (rows, cols, k), (alone, beside) in {(6912, 1280, 25524): (5, 3), (6912, 1280, 65536): (7, 5), (1280, 1280, 6084): (5, 1),
                                              (6912, 1280, 14336): (3, 3), (3840, 1280, 4096): (1, 1)}.items():
         assert (ops.wgrad_split_k(rows, cols, k), ops.wgrad_split_k(rows, cols, k, True)) == (alone, beside), (rows, cols, k)
+
+
+def test_weight_gradients_leave_the_second_stream_where_a_block_has_little_work():
+    """One launch behind the chain up to the work of 1,280 rows of a block of 1280 columns: a wider block keeps its second stream at
+    fewer rows, a narrower one at more than 1,280; fp32 and K slices do at any size."""
+    import ctypes
+
+    from mi355_vit import _lib
+
+    uses = _lib.load().mvit_block_bwd_uses_side_stream
+
+    def side(S, C, I, dtype=_lib.BF16, grad=_lib.BF16, split=1):
+        a = _lib.BlockArgs()
+        a.dtype, a.grad_dtype, a.S, a.C, a.I, a.Ipad = dtype, grad, S, C, I, (I + 63) // 64 * 64
+        a.split_k_down, a.split_k_gate_up, a.split_k_proj, a.split_k_qkv = 1, 1, 1, split
+        return uses(ctypes.byref(a))
+
+    assert uses(None) == 0
+    assert [side(S, 1280, 3420) for S in (1, 256, 1280, 1281, 16384)] == [0, 0, 0, 1, 1]
+    assert [side(S, 1920, 5120) for S in (256, 512, 640, 1024)] == [0, 0, 1, 1]
+    assert [side(S, 2560, 6840) for S in (128, 256, 1000)] == [0, 1, 1]
+    assert [side(S, 3840, 10240) for S in (64, 1000)] == [1, 1]
+    assert [side(S, 64, 72) for S in (1280, 1281)] == [0, 1]
+    assert side(256, 1280, 3420, dtype=_lib.F32, grad=_lib.F32) == side(256, 1280, 3420, grad=_lib.F32) == side(256, 1280, 3420, split=2) == 1
