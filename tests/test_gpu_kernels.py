@@ -463,9 +463,10 @@ def test_gemm_rows_in_full_rounds_and_the_rest_give_the_same_bits_as_one_launch(
         assert max_rel_err(split[0][:M], want) < TOL[dtype]
 
 
-# rows whose tiles are 64 x 64 and 64 x 128, the ring of stages never full, once full, refilled, with and without a partial last K tile ...
-_RING_SHAPES = [(70, 200, k) for k in (8, 64, 72, 128, 136, 192, 200, 256, 264, 320)] + [(1500, 1288, k) for k in (8, 64, 72, 136, 192, 264)]
-# ... and one work-group per unit: 128 x 128 up to 256 tiles, 192 x 128 from there to 256 tiles
+# 64 x 64 tiles, one work-group per unit (a ring of six stages; four for `tt`) and two (four stages): the ring never full, once full,
+# refilled in turn, with and without a partial last K tile ...
+_RING_SHAPES = [(70, 200, k) for k in (8, 64, 72, 128, 136, 192, 200, 256, 264, 320, 384, 392, 456, 840)] + [(1500, 1288, k) for k in (8, 64, 72, 136, 192, 264)]
+# ... and one work-group per unit: 128 x 128 up to 256 tiles, 192 x 128 from there to 256 tiles; 64 x 128 and 128 x 128 beyond them and for `tt`
 _RING_SHAPES += [(1700, 1280, 1288), (3200, 1280, 840), (3201, 1280, 840), (3277, 1280, 1280), (4800, 1280, 1288), (4801, 1280, 840)]
 
 

@@ -206,11 +206,14 @@ def test_one_call_per_block_equals_the_call_by_call_sequence(dtype, checkpoint):
             assert torch.equal(grads[k], ref_grads[k]), (key, k)
 
 
-@pytest.mark.parametrize("hidden,inner", [(512, 1200), (64, 72)])
-@pytest.mark.parametrize("grid", [[[1, 2, 2]], [[1, 6, 10]], [[1, 16, 16], [1, 2, 6]], [[1, 32, 40]], [[1, 32, 40], [1, 2, 2]]])
+_FEW_ROWS = ([[1, 2, 2]], [[1, 6, 10]], [[1, 16, 16], [1, 2, 6]], [[1, 32, 40]], [[1, 32, 40], [1, 2, 2]])
+
+
+@pytest.mark.parametrize("hidden,inner,grid", [(h, i, g) for h, i in ((512, 1200), (64, 72)) for g in _FEW_ROWS] + [(1280, 3420, g) for g in _FEW_ROWS[1:4]])
 def test_weight_gradients_of_few_rows_in_one_launch_equal_a_launch_each(grid, hidden, inner):
     """Up to 1,280 rows the backward of a block sends its weight gradients in one launch and its column sums in another (4, 60, 268 and
-    1,280 rows; 1,284 go as longer ones do): output and gradients have the bits of the call-by-call sequence."""
+    1,280 rows; 1,284 go as longer ones do), on tiles of 64 x 128, 64 x 64 and, at the tower's own width, 128 x 128: output and gradients
+    have the bits of the call-by-call sequence."""
     from mi355_vit import functional
 
     kw = dict(depth=2, hidden_size=hidden, intermediate_size=inner, num_heads=hidden // 32, out_hidden_size=256, window_size=56, fullatt_block_indexes=[1])
