@@ -1982,8 +1982,8 @@ int launch_fwd_mfma(const AttnParams& p, int n_seg, int max_seqlen, hipStream_t 
   if (nw == 1 && ND <= 5) {
     // windows: four waves x 16 queries share the staged K / V tiles.  Bound by memory (671 MB at 65,536 rows x 16 heads) and by the
     // chain load -> products -> store, i.e. by how many waves a compute unit holds: 96 registers, five per SIMD.  Two waves of 32
-    // queries (128 registers, a tile staged load by load) / this, us: 16,384 rows 39.5 / 37.2, 25,524 in windows of 4 ... 64 61.7 / 52.3,
-    // 65,536 177 / 154
+    // queries (128 registers, a tile staged load by load) / this, us, operands from HBM: 16,384 rows 51 / 43, 25,524 in windows of
+    // 4 ... 64 76 / 64, 65,536 179 / 152
     AttnParams pw = p;
     if (grid.x == 1 && ((int64_t)n_seg * p.nheads) % 8 == 0) pw.seg_major = 2;  // heads of a segment together on one XCD
     if constexpr (ND <= 5) hipLaunchKernelGGL((attn_fwd_mfma<ND, 4, 64, false, 1, 5>), grid, 256, 0, s, pw);

@@ -1420,7 +1420,7 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
     TileChoice c = choose_tile(kind, p.M, p.N, p.k_chunk, p.K - (p.split_k - 1) * p.k_chunk, p.split_k, n_cu, a->overlapped != 0);
     const bool all_256 = getenv("MVIT_GEMM_NO_HALF_TILES") != nullptr;
     if (all_256 && c.bm != 256 && pp_takes(kind, p.k_chunk, p.K - (p.split_k - 1) * p.k_chunk)) c = TileChoice{256, 256, 0.};
-    // the column sums are per tile row: their granularity names the kernel (64 rows: 64 x 64 or 64 x 128 tiles, below)
+    // the column sums are per tile row: their granularity names the kernels (64 rows: a tile of 64 x 64, 64 x 128 or 128 x 128)
     if (kind == NT_SWIGLU_BWD && p.colsum != nullptr) c = colsum_rows == 64 ? choose_tile(kind, p.M, p.N, p.k_chunk, p.K, 1, n_cu, a->overlapped != 0, false) : full_rows_tile(kind, p.K, p.K);
     if (c.bm != 0) {
       auto run = [&](GemmParams q, const TileChoice& t) -> int {

@@ -415,8 +415,9 @@ __device__ __forceinline__ void gemm_small_tile(const GemmParams& p, const unsig
   }
 }
 
+// registers for two work-groups per compute unit; LDS holds two of the smaller rings, one of the deeper ones (Lone*)
 template <typename TO, bool TA, bool TB, int EPI, typename S>
-__global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(const GemmParams p) {  // two work-groups fit a compute unit
+__global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(const GemmParams p) {
   gemm_small_tile<TO, TA, TB, EPI, S>(p, blockIdx.x);
 }
 // several independent products: each takes a range of work-groups, a multiple of eight so that it stays dealt to the XCDs
