@@ -1336,7 +1336,7 @@ extern "C" int mvit_patch_embed_frames(const mvit_image* images, int n_images, i
   const int64_t tm = (total_rows + 255) / 256, tn = (n_out + 255) / 256;
   MVIT_REQUIRE(tm * tn < (1ll << 30), "patch_embed_frames: too many tiles");
   p.tiles_m = (int)tm; p.tiles_n = (int)tn;
-  p.panel_w = tn <= 6 ? (int)tn : 4;
+  set_tile_order(p, 256);
   p.split_k = 1; p.k_chunk = PX_K; p.reduce_epi = MVIT_EPI_NONE;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (out_dtype == MVIT_BF16) return launch_dl<bf16_t, false, false, MVIT_EPI_NONE, 4, 8, false, true>(p, s);
@@ -1379,7 +1379,7 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
   const int64_t tm = (a->M + BM - 1) / BM, tn = (a->N + n_per_block - 1) / n_per_block;
   MVIT_REQUIRE(tm * tn < (1ll << 30), "gemm: too many tiles");
   p.tiles_m = (int)tm; p.tiles_n = (int)tn;
-  p.panel_w = tn <= 6 ? (int)tn : 4;
+  set_tile_order(p, BM);
   p.split_k = 1; p.k_chunk = a->K; p.workspace = nullptr; p.reduce_epi = MVIT_EPI_NONE;
   p.colsum = nullptr;
   const int colsum_rows = a->colsum_rows == 64 ? 64 : 256;
@@ -1428,7 +1428,7 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
         const int n_cols = kind == NN_SWIGLU ? t.bn / 2 : t.bn;
         q.tiles_n = (int)((q.N + n_cols - 1) / n_cols);
         MVIT_REQUIRE((int64_t)q.tiles_m * q.tiles_n * q.split_k < (1ll << 30), "gemm: too many tiles");
-        q.panel_w = q.tiles_n <= 6 ? q.tiles_n : 4;
+        set_tile_order(q, t.bm);
         return t.bm == 256 ? mvit_gemm_pp(kind, q, n_cu, s) : mvit_gemm_small(kind, t.bm, t.bn, t.lone, q, s);
       };
       const int64_t head = all_256 || p.split_k > 1 ? 0 : rows_in_full_rounds(kind, p.M, p.N, p.K, n_cu);
@@ -1523,7 +1523,7 @@ int mvit_gemm_wgrad_group(const mvit_gemm_args* list, int n, hipStream_t s) {
     p.split_k = 1; p.k_chunk = a.K; p.reduce_epi = MVIT_EPI_NONE;
     p.tiles_m = (int)((a.M + bm - 1) / bm);
     p.tiles_n = (int)((a.N + bn - 1) / bn);
-    p.panel_w = p.tiles_n <= 6 ? p.tiles_n : 4;
+    set_tile_order(p, bm);
   }
   return mvit_gemm_small_group(bm, bn, g, s);
 }

@@ -30,13 +30,24 @@ struct GemmParams {
   float* colsum;      // SWIGLU_BWD: column sums of the output before rounding, one row per tile row, [tiles_m][ldc] (null: not wanted)
   void* row_sums;     // TT_NONE(_F32), optional: [M] sums of op(A) over k, in the type of C (a bias gradient beside its weight gradient)
   float* row_ws;      // split_k > 1: their partial sums, [split_k][M]
-  int panel_w;        // tiles are walked in panels of this many tile columns (M fastest across a panel's rows)
+  int group_m, panel_w;  // tiles are walked in groups of this many tile rows, and a group in panels of this many tile columns
   // A operand made from decoded frames (gemm_dl_kernel<..., PIX = true>): image table and the affine form of the
   // rescale / normalise step, value = byte * px_a[channel] + px_c[channel]
   const mvit_image* px_images;
   int px_n_images;
   float px_a[3], px_c[3];
 };
+
+// The bf16 products' tile order, for tiles of bm rows (tile_coords): groups of 2,048 rows, 8 x 4 tiles of 256 x 256 per XCD at a time, once
+// A is too large to stay in the memory-side cache (256 MB) beside the output from one panel to the next.  us, whole panels -> groups
+// (K = 1280): 3840 columns with bias 32,768 rows (A is 84 MB) 257 / 247 -> 258 / 247, 36,864 (94 MB) 299 -> 288, 40,960 333 -> 318, 65,536 557 -> 507;
+// SwiGLU 32,768 rows 525 / 511 -> 530 / 528, 36,864 619 -> 587, 40,960 717 -> 628, 65,536 1,143 -> 1,050; SwiGLU backward 394 -> 393, 453 -> 441, 505 -> 489,
+// 788 -> 775.  Groups of 1,024, 4,096 and 8,192 rows at 65,536: 552, 535, 549 and 1,040, 1,074, 1,153; panels of eight columns 544, 1,067.
+constexpr int64_t TILE_GROUP_BYTES = 88ll << 20;
+inline void set_tile_order(GemmParams& p, int bm) {
+  p.panel_w = p.tiles_n <= 6 ? p.tiles_n : 4;
+  p.group_m = p.tiles_n > p.panel_w && p.M * p.K * 2 > TILE_GROUP_BYTES && 2048 / bm < p.tiles_m ? 2048 / bm : p.tiles_m;
+}
 
 // bf16 kernels behind mvit_gemm that live in translation units of their own; gemm.hip chooses (the K slices of a split
 // product are reduced there too).  They cover the products of the vision tower, see mvit_gemm_tiled_kind.
@@ -56,19 +67,26 @@ int mvit_gemm_f32(int ta, int tb, int epi, const GemmParams& p, int n_cu, hipStr
 
 namespace {
 
-// Tile order inside one K slice: panels of panel_w tile columns; within a panel row by row.  Work-groups that run
-// at the same time on one XCD (consecutive tile indices) then cover a compact block of the output, e.g. 8 x 4
-// tiles, so the A and B panels they stream through that XCD's L2 are shared as widely as possible.
+// Tile order inside one K slice: groups of group_m tile rows; within a group panels of panel_w tile columns, row by row.  Work-groups
+// that run at the same time on one XCD (consecutive tile indices) then cover a compact block of the output, e.g. 8 x 4 tiles, so the
+// A and B panels they stream through that XCD's L2 are shared as widely as possible; and a group's rows of A are in the memory-side
+// cache when its next panel reads them, where whole panels of tall products read all of A from HBM once per panel.
 __device__ __forceinline__ void tile_coords(const GemmParams& p, int tile, int& tm, int& tn) {
   const int pw = p.panel_w;
-  const int full_panels = p.tiles_n / pw, per_panel = p.tiles_m * pw;
+  int row0 = 0, rows = p.tiles_m;
+  if (p.group_m < p.tiles_m) {
+    row0 = tile / (p.group_m * p.tiles_n) * p.group_m;
+    rows = p.tiles_m - row0 < p.group_m ? p.tiles_m - row0 : p.group_m;
+    tile -= row0 * p.tiles_n;
+  }
+  const int full_panels = p.tiles_n / pw, per_panel = rows * pw;
   if (tile < full_panels * per_panel) {
     const int r = tile % per_panel;
-    tm = r / pw;
+    tm = row0 + r / pw;
     tn = (tile / per_panel) * pw + r % pw;
   } else {
     const int r = tile - full_panels * per_panel, w = p.tiles_n - full_panels * pw;
-    tm = r / w;
+    tm = row0 + r / w;
     tn = full_panels * pw + r % w;
   }
 }

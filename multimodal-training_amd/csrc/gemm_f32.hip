@@ -302,6 +302,7 @@ int launch_f32_tiles(GemmParams p, hipStream_t stream) {
   const int64_t tm = (p.M + BM - 1) / BM, tn = (p.N + NCOLS - 1) / NCOLS;
   MVIT_REQUIRE(tm * tn * p.split_k < (1ll << 30), "gemm: too many tiles");
   p.tiles_m = (int)tm; p.tiles_n = (int)tn;
+  p.group_m = p.tiles_m;
   p.panel_w = tn <= 6 ? (int)tn : 4;
   hipLaunchKernelGGL((gemm_f32_kernel<TA, TB, EPI, BM, BN>), (p.tiles_m * p.tiles_n * p.split_k + 7) / 8 * 8, 256, (F32Cfg<BM, BN, 2, 2>::LDS), stream, p);
   MVIT_CHECK_LAUNCH("gemm");

@@ -463,6 +463,28 @@ def test_gemm_rows_in_full_rounds_and_the_rest_give_the_same_bits_as_one_launch(
         assert max_rel_err(split[0][:M], want) < TOL[dtype]
 
 
+@pytest.mark.parametrize("form", ["none", "trans_b", "swiglu"])
+@pytest.mark.parametrize("M,N,K", [(5000, 2184, 9280), (36100, 1800, 1280)])
+def test_gemm_of_tall_operands_walks_its_tiles_in_groups_of_rows(M, N, K, form):
+    """An A beyond 88 MiB is walked in groups of 2,048 rows (here a last one of 904 and of 1,284 rows, and a last panel of fewer than
+    four tile columns): every row has the bits it has in shorter products, which are walked in whole panels."""
+    _announce(f"gemm tile groups M={M} N={N} K={K} {form}")
+    ops = _ops()
+    from mi355_vit import _lib as E
+
+    dtype = torch.bfloat16
+    g = torch.Generator(device=DEV).manual_seed(M)
+    a, b, b2 = (torch.randn(s, generator=g, device=DEV).to(dtype) for s in ((M, K), (K, N) if form == "trans_b" else (N, K), (N, K)))
+    bias = torch.randn(N, generator=g, device=DEV).to(dtype)
+    kw = {"none": {}, "trans_b": dict(trans_b=True), "swiglu": dict(epilogue=E.EPI_SWIGLU, b2=b2, bias=bias, bias2=bias)}[form]
+    assert 2 * M * K > 88 << 20 >= 2 * 4000 * K
+    whole, parts = (torch.full((M, N), float("nan"), dtype=dtype, device=DEV) for _ in range(2))
+    ops.gemm(a, b, whole, **kw)
+    for i in range(0, M, 4000):
+        ops.gemm(a[i : i + 4000], b, parts[i : i + 4000], **kw)
+    assert torch.isfinite(whole).all() and torch.equal(whole, parts)
+
+
 # 64 x 64 tiles, one work-group per unit (a ring of six stages; four for `tt`) and two (four stages): the ring never full, once full,
 # refilled in turn, with and without a partial last K tile ...
 _RING_SHAPES = [(70, 200, k) for k in (8, 64, 72, 128, 136, 192, 200, 256, 264, 320, 384, 392, 456, 840)] + [(1500, 1288, k) for k in (8, 64, 72, 136, 192, 264)]
