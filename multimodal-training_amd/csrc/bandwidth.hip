@@ -59,6 +59,63 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const T* __restrict__ 
   }
 }
 
+// The same for rows of at most NCH vectors per lane: a row is read once, all its loads in flight at a time, and stays in registers; the next
+// row's loads are under way before this one's result is stored.  us for 1280 columns in bf16, before (a second pass over the row) / now: 1,024 rows
+// 4.2 / 3.7, 4,096 6.5 / 5.6, 14,336 17.4 / 15.3, 25,524 23.2 / 20.4, 65,536 68 / 59 (5.6 TB/s).
+template <typename T, int NCH>
+__global__ __launch_bounds__(256) void rmsnorm_fwd_row_kernel(const T* __restrict__ x, const T* __restrict__ w, T* __restrict__ y,
+                                                              float* __restrict__ rstd, int64_t rows, int cols, float eps) {
+  constexpr int V = mvit_elem<T>::vec;
+  typedef T vec_t __attribute__((ext_vector_type(V)));
+  const int lane = threadIdx.x & 63;
+  const int64_t nwaves = (int64_t)gridDim.x * 4;
+  int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (r >= rows) return;
+  vec_t v[NCH], g[NCH];
+  auto load = [&](int64_t row, vec_t (&to)[NCH], const T* from) {
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int c = (i * 64 + lane) * V;
+      if (i < NCH - 1 || c < cols) to[i] = *reinterpret_cast<const vec_t*>(from + row * cols + c);
+    }
+  };
+  load(r, v, x);
+  load(0, g, w);
+  while (true) {
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i)
+      if (i < NCH - 1 || (i * 64 + lane) * V < cols) {
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+          const float f = to_f32(v[i][j]);
+          ss += f * f;
+        }
+      }
+    ss = wave_sum(ss);
+    const float rs = rsqrtf(ss / (float)cols + eps);
+    if (lane == 0) rstd[r] = rs;
+    vec_t o[NCH];
+#pragma unroll
+    for (int i = 0; i < NCH; ++i)
+#pragma unroll
+      for (int j = 0; j < V; ++j) {
+        // normalise in fp32, round to the storage type, then scale (two roundings, like the reference)
+        const T n = from_f32<T>(to_f32(v[i][j]) * rs);
+        o[i][j] = from_f32<T>(to_f32(g[i][j]) * to_f32(n));
+      }
+    const int64_t next = r + nwaves;
+    if (next < rows) load(next, v, x);
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int c = (i * 64 + lane) * V;
+      if (i < NCH - 1 || c < cols) *reinterpret_cast<vec_t*>(y + r * cols + c) = o[i];
+    }
+    if (next >= rows) return;
+    r = next;
+  }
+}
+
 // RMSNorm backward.  Same row ownership; each block keeps its weight-gradient partial in LDS (fp32 [cols])
 // and writes it to dw_partial[blockIdx.x, :] at the end, so the result does not depend on atomics order.
 // Algorithmic bytes per row: read dy, x (2*cols*e) [+ dx_add], write dx (cols*e).
@@ -124,6 +181,93 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const T* __restrict__ 
       }
     }
   }
+  __syncthreads();
+  float* out = dw_partial + (size_t)blockIdx.x * cols;
+  for (int c = threadIdx.x; c < cols; c += 256)
+    out[c] = dw_lds[c] + dw_lds[cols + c] + dw_lds[2 * (size_t)cols + c] + dw_lds[3 * (size_t)cols + c];
+}
+
+// The same for rows of at most NCH vectors per lane: a row's operands are read once, all loads in flight at a time, and a lane's part of the
+// weight gradient stays in registers.  Bound by HBM from some thousand rows on; us for 1280 columns with dx_add, before (two passes over the row,
+// the weight gradient in LDS) / now: 1,024 rows 7.0 / 5.4, 4,096 14.4 / 13.6, 14,336 34.3 / 30.5, 25,524 55.1 / 52.3, 65,536 130 / 130; with the next row's
+// loads under way as well 5.7 / 14.2 / 30.3 / 51.4 / 129, in twice the registers.
+template <typename T, int NCH, bool ADD>
+__global__ __launch_bounds__(256) void rmsnorm_bwd_row_kernel(const T* __restrict__ dy, const T* __restrict__ x, const T* __restrict__ w,
+                                                              const float* __restrict__ rstd, const T* dx_add, T* dx,
+                                                              float* __restrict__ dw_partial, int64_t rows, int cols) {
+  constexpr int V = mvit_elem<T>::vec;
+  typedef T vec_t __attribute__((ext_vector_type(V)));
+  extern __shared__ __attribute__((aligned(16))) float dw_lds[];  // [4][cols]
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t nwaves = (int64_t)gridDim.x * 4;
+  const float inv_cols = 1.f / (float)cols;
+  float dw[NCH][V];
+#pragma unroll
+  for (int i = 0; i < NCH; ++i)
+#pragma unroll
+    for (int j = 0; j < V; ++j) dw[i][j] = 0.f;
+  auto mine = [&](int i) { return i < NCH - 1 || (i * 64 + lane) * V < cols; };
+  struct Row {
+    vec_t x[NCH], g[NCH], a[NCH];
+    float rs;
+  };
+  auto load = [&](int64_t r, Row& to) {
+    to.rs = rstd[r];
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int64_t at = r * cols + (i * 64 + lane) * V;
+      if (mine(i)) {
+        to.x[i] = *reinterpret_cast<const vec_t*>(x + at);
+        to.g[i] = *reinterpret_cast<const vec_t*>(dy + at);
+        if (ADD) to.a[i] = *reinterpret_cast<const vec_t*>(dx_add + at);
+      }
+    }
+  };
+  int64_t r = (int64_t)blockIdx.x * 4 + wv;
+  if (r < rows) {
+    Row now;
+    load(r, now);
+    vec_t wt[NCH];
+#pragma unroll
+    for (int i = 0; i < NCH; ++i)
+      if (mine(i)) wt[i] = *reinterpret_cast<const vec_t*>(w + (i * 64 + lane) * V);
+    while (true) {
+      float dot = 0.f;
+#pragma unroll
+      for (int i = 0; i < NCH; ++i)
+        if (mine(i)) {
+#pragma unroll
+          for (int j = 0; j < V; ++j) dot += to_f32(now.g[i][j]) * to_f32(wt[i][j]) * to_f32(now.x[i][j]);
+        }
+      const float rs = now.rs;
+      dot = wave_sum(dot) * rs * inv_cols;  // mean(dy*w*xhat)
+#pragma unroll
+      for (int i = 0; i < NCH; ++i)
+        if (mine(i)) {
+          vec_t o;
+#pragma unroll
+          for (int j = 0; j < V; ++j) {
+            const float xhat = to_f32(now.x[i][j]) * rs;
+            const float g = to_f32(now.g[i][j]);
+            float d = rs * (g * to_f32(wt[i][j]) - xhat * dot);
+            if (ADD) d += to_f32(now.a[i][j]);
+            o[j] = from_f32<T>(d);
+            dw[i][j] += g * xhat;
+          }
+          *reinterpret_cast<vec_t*>(dx + r * cols + (i * 64 + lane) * V) = o;
+        }
+      r += nwaves;
+      if (r >= rows) break;
+      load(r, now);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NCH; ++i)
+    if (mine(i)) {
+#pragma unroll
+      for (int q = 0; q < V; q += 4)
+        *reinterpret_cast<f32x4*>(dw_lds + (size_t)wv * cols + (i * 64 + lane) * V + q) = f32x4{dw[i][q], dw[i][q + 1], dw[i][q + 2], dw[i][q + 3]};
+    }
   __syncthreads();
   float* out = dw_partial + (size_t)blockIdx.x * cols;
   for (int c = threadIdx.x; c < cols; c += 256)
@@ -243,57 +387,86 @@ __global__ __launch_bounds__(256) void colsum_kernel(const T* __restrict__ x, in
 }
 
 // ------------------------------------------------------------------------------------------------
+__device__ __forceinline__ void rope_pair(float a, float b, float c0, float c1, float s0, float s1, int backward, float& oa, float& ob) {
+  if (!backward) {
+    oa = a * c0 - b * s0;
+    ob = b * c1 + a * s1;
+  } else {
+    oa = a * c0 + b * s1;
+    ob = b * c1 - a * s0;
+  }
+}
+
 // Rotary embedding in place.  A thread owns V consecutive elements of the first half of one head and
 // the matching V of the second half.  Algorithmic bytes per (row, head): 2*head_dim*e + table share.
 // The first `lead_heads` heads are multiplied by `lead_scale` before the one rounding to the storage type (the
 // queries of an attention layer take the softmax scale here, so that no later pass rounds them a second time).
-template <typename T, int V>
-__global__ __launch_bounds__(256) void rope_kernel(T* __restrict__ x, const float* __restrict__ cosb,
-                                                   const float* __restrict__ sinb, int64_t rows, int nheads,
-                                                   int head_dim, int64_t row_stride, int backward, int lead_heads,
-                                                   float lead_scale) {
-  typedef T vec_t __attribute__((ext_vector_type(V)));
+template <typename T>
+__global__ __launch_bounds__(256) void rope_kernel(T* __restrict__ x, const float* __restrict__ cosb, const float* __restrict__ sinb, int64_t rows,
+                                                   int nheads, int head_dim, int64_t row_stride, int backward, int lead_heads, float lead_scale) {
   const int half = head_dim / 2;
-  const int chunks = half / V;  // per head
-  const int64_t total = rows * nheads * chunks;
+  const int64_t total = rows * nheads * half;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-    const int ch = (int)(i % chunks);
-    const int64_t rh = i / chunks;
+    const int j = (int)(i % half);
+    const int64_t rh = i / half;
     const int h = (int)(rh % nheads);
     const int64_t r = rh / nheads;
-    T* p = x + r * row_stride + (int64_t)h * head_dim + ch * V;
+    T* p = x + r * row_stride + (int64_t)h * head_dim + j;
+    const float* c = cosb + r * head_dim + j;
+    const float* s = sinb + r * head_dim + j;
+    float oa, ob;
+    rope_pair(to_f32(p[0]), to_f32(p[half]), c[0], c[half], s[0], s[half], backward, oa, ob);
     const float gain = h < lead_heads ? lead_scale : 1.f;
+    p[0] = from_f32<T>(oa * gain);
+    p[half] = from_f32<T>(ob * gain);
+  }
+}
+
+// The same on vectors: a thread takes one chunk of V pairs of every `groups`-th head of a row, whose angles it reads once, with the loads
+// of ROPE_HEADS heads in flight.  Bound by HBM (bytes of x twice, angles once); a thread per chunk of a head, which read its angles for one head
+// each and found its place by 64-bit divisions, took, us at 1,024 / 4,096 / 25,524 / 65,536 rows of 32 heads of 80 (row pitch 3840), 5.0 / 12.2 /
+// 60.6 / 145; this 4.5 / 11.5 / 54.1 / 139, with four heads in flight 4.5 / 11.3 / 53.1 / 140, with eight 4.5 / 12.5 / 56 / 142.
+constexpr int ROPE_HEADS = 2;
+template <typename T>
+__global__ __launch_bounds__(256) void rope_vec_kernel(T* __restrict__ x, const float* __restrict__ cosb, const float* __restrict__ sinb, int64_t rows,
+                                                       int nheads, int head_dim, int64_t row_stride, int backward, int lead_heads, float lead_scale,
+                                                       int chunks, int groups) {
+  constexpr int V = mvit_elem<T>::vec;
+  typedef T vec_t __attribute__((ext_vector_type(V)));
+  const int half = head_dim / 2, per_row = chunks * groups, rows_here = 256 / per_row;
+  const int row = threadIdx.x / per_row, at = threadIdx.x - row * per_row, first = at / chunks, ch = at - first * chunks;
+  if (row >= rows_here) return;
+  for (int64_t r = (int64_t)blockIdx.x * rows_here + row; r < rows; r += (int64_t)gridDim.x * rows_here) {
     const float* c = cosb + r * head_dim + ch * V;
     const float* s = sinb + r * head_dim + ch * V;
-    vec_t lo, hi, olo, ohi;
-    if (V > 1) {
-      lo = *reinterpret_cast<const vec_t*>(p);
-      hi = *reinterpret_cast<const vec_t*>(p + half);
-    } else {
-      lo[0] = p[0];
-      hi[0] = p[half];
-    }
+    float c0[V], c1[V], s0[V], s1[V];
 #pragma unroll
-    for (int j = 0; j < V; ++j) {
-      const float a = to_f32(lo[j]), b = to_f32(hi[j]);
-      const float c0 = c[j], c1 = c[j + half], s0 = s[j], s1 = s[j + half];
-      float oa, ob;
-      if (!backward) {
-        oa = a * c0 - b * s0;
-        ob = b * c1 + a * s1;
-      } else {
-        oa = a * c0 + b * s1;
-        ob = b * c1 - a * s0;
-      }
-      olo[j] = from_f32<T>(oa * gain);
-      ohi[j] = from_f32<T>(ob * gain);
-    }
-    if (V > 1) {
-      *reinterpret_cast<vec_t*>(p) = olo;
-      *reinterpret_cast<vec_t*>(p + half) = ohi;
-    } else {
-      p[0] = olo[0];
-      p[half] = ohi[0];
+    for (int j = 0; j < V; ++j) c0[j] = c[j], c1[j] = c[j + half], s0[j] = s[j], s1[j] = s[j + half];
+    for (int h0 = first; h0 < nheads; h0 += ROPE_HEADS * groups) {
+      T* p = x + r * row_stride + (int64_t)h0 * head_dim + ch * V;
+      const int64_t step = (int64_t)groups * head_dim;
+      vec_t lo[ROPE_HEADS], hi[ROPE_HEADS];
+#pragma unroll
+      for (int k = 0; k < ROPE_HEADS; ++k)
+        if (h0 + k * groups < nheads) {
+          lo[k] = *reinterpret_cast<const vec_t*>(p + k * step);
+          hi[k] = *reinterpret_cast<const vec_t*>(p + k * step + half);
+        }
+#pragma unroll
+      for (int k = 0; k < ROPE_HEADS; ++k)
+        if (h0 + k * groups < nheads) {
+          const float gain = h0 + k * groups < lead_heads ? lead_scale : 1.f;
+          vec_t olo, ohi;
+#pragma unroll
+          for (int j = 0; j < V; ++j) {
+            float oa, ob;
+            rope_pair(to_f32(lo[k][j]), to_f32(hi[k][j]), c0[j], c1[j], s0[j], s1[j], backward, oa, ob);
+            olo[j] = from_f32<T>(oa * gain);
+            ohi[j] = from_f32<T>(ob * gain);
+          }
+          *reinterpret_cast<vec_t*>(p + k * step) = olo;
+          *reinterpret_cast<vec_t*>(p + k * step + half) = ohi;
+        }
     }
   }
 }
@@ -486,6 +659,45 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(const W* __restrict__ e
 
 static inline int clamp_grid(int64_t v, int64_t hi) { return (int)(v < 1 ? 1 : (v > hi ? hi : v)); }
 
+template <typename T>
+static void launch_rope(T* x, const float* cosb, const float* sinb, int64_t rows, int nheads, int head_dim, int64_t row_stride, int backward,
+                        int lead_heads, float lead_scale, hipStream_t stream) {
+  constexpr int V = mvit_elem<T>::vec;
+  const int half = head_dim / 2, chunks = half / V;
+  if (half % V == 0 && chunks <= 256 && row_stride % V == 0 && mvit_aligned16(x)) {
+    const int want = (nheads + ROPE_HEADS - 1) / ROPE_HEADS, groups = want * chunks <= 256 ? want : 256 / chunks, rows_here = 256 / (chunks * groups);
+    const int grid = clamp_grid((rows + rows_here - 1) / rows_here, MVIT_MAX_GROUPS_256);
+    hipLaunchKernelGGL((rope_vec_kernel<T>), grid, 256, 0, stream, x, cosb, sinb, rows, nheads, head_dim, row_stride, backward, lead_heads, lead_scale, chunks, groups);
+  } else {
+    const int grid = clamp_grid((rows * nheads * half + 255) / 256, 65535 * 16);
+    hipLaunchKernelGGL((rope_kernel<T>), grid, 256, 0, stream, x, cosb, sinb, rows, nheads, head_dim, row_stride, backward, lead_heads, lead_scale);
+  }
+}
+
+// A row in registers: the kernel of that many vectors per lane, null where a row is longer
+template <typename T>
+static auto rms_fwd_row(int64_t cols) -> decltype(&rmsnorm_fwd_row_kernel<T, 1>) {
+  switch ((cols + 64 * mvit_elem<T>::vec - 1) / (64 * mvit_elem<T>::vec)) {
+    case 1: return rmsnorm_fwd_row_kernel<T, 1>;
+    case 2: return rmsnorm_fwd_row_kernel<T, 2>;
+    case 3: return rmsnorm_fwd_row_kernel<T, 3>;
+    case 4: return rmsnorm_fwd_row_kernel<T, 4>;
+    case 5: return rmsnorm_fwd_row_kernel<T, 5>;
+    default: return nullptr;
+  }
+}
+template <typename T, bool ADD>
+static auto rms_bwd_row(int64_t cols) -> decltype(&rmsnorm_bwd_row_kernel<T, 1, ADD>) {
+  switch ((cols + 64 * mvit_elem<T>::vec - 1) / (64 * mvit_elem<T>::vec)) {
+    case 1: return rmsnorm_bwd_row_kernel<T, 1, ADD>;
+    case 2: return rmsnorm_bwd_row_kernel<T, 2, ADD>;
+    case 3: return rmsnorm_bwd_row_kernel<T, 3, ADD>;
+    case 4: return rmsnorm_bwd_row_kernel<T, 4, ADD>;
+    case 5: return rmsnorm_bwd_row_kernel<T, 5, ADD>;
+    default: return nullptr;
+  }
+}
+
 int mvit_reduce_partials_group(const mvit_partials* list, int n, int out_dtype, hipStream_t stream) {
   bool together = n >= 2 && n <= PARTIALS_GROUP_MAX && (out_dtype == MVIT_BF16 || out_dtype == MVIT_F32);
   for (int i = 0; i < n; ++i) together = together && list[i].partial && list[i].out && list[i].n_partial > 0 && list[i].cols > 0 && list[i].cols % 4 == 0 && mvit_aligned16(list[i].partial);
@@ -515,22 +727,17 @@ int mvit_rmsnorm_fwd(const void* x, const void* w, void* y, float* rstd, int64_t
   MVIT_REQUIRE(rows >= 0 && cols > 0 && cols < (1 << 24), "rmsnorm_fwd: bad shape %lld x %lld", (long long)rows, (long long)cols);
   if (rows == 0) return MVIT_OK;
   MVIT_REQUIRE(x && w && y && rstd, "rmsnorm_fwd: null pointer");
-  const int grid = clamp_grid((rows + 3) / 4, 8192);
-  if (dtype == MVIT_BF16) {
-    const bool vec = cols % 8 == 0 && mvit_aligned16(x) && mvit_aligned16(y) && mvit_aligned16(w);
-    if (vec)
-      hipLaunchKernelGGL((rmsnorm_fwd_kernel<bf16_t, true>), grid, 256, 0, S_(stream), (const bf16_t*)x, (const bf16_t*)w, (bf16_t*)y, rstd, rows, (int)cols, eps);
-    else
-      hipLaunchKernelGGL((rmsnorm_fwd_kernel<bf16_t, false>), grid, 256, 0, S_(stream), (const bf16_t*)x, (const bf16_t*)w, (bf16_t*)y, rstd, rows, (int)cols, eps);
-  } else if (dtype == MVIT_F32) {
-    const bool vec = cols % 4 == 0 && mvit_aligned16(x) && mvit_aligned16(y) && mvit_aligned16(w);
-    if (vec)
-      hipLaunchKernelGGL((rmsnorm_fwd_kernel<float, true>), grid, 256, 0, S_(stream), (const float*)x, (const float*)w, (float*)y, rstd, rows, (int)cols, eps);
-    else
-      hipLaunchKernelGGL((rmsnorm_fwd_kernel<float, false>), grid, 256, 0, S_(stream), (const float*)x, (const float*)w, (float*)y, rstd, rows, (int)cols, eps);
-  } else {
-    return mvit_set_error(MVIT_ERR_UNSUPPORTED, "rmsnorm_fwd: dtype %d", dtype);
-  }
+  auto go = [&](auto zero) -> void {
+    using T = decltype(zero);
+    const bool vec = cols % mvit_elem<T>::vec == 0 && mvit_aligned16(x) && mvit_aligned16(y) && mvit_aligned16(w);
+    auto kern = rms_fwd_row<T>(cols);
+    if (!vec) kern = rmsnorm_fwd_kernel<T, false>;
+    else if (kern == nullptr) kern = rmsnorm_fwd_kernel<T, true>;
+    hipLaunchKernelGGL(kern, clamp_grid((rows + 3) / 4, 8192), 256, 0, S_(stream), (const T*)x, (const T*)w, (T*)y, rstd, rows, (int)cols, eps);
+  };
+  if (dtype == MVIT_BF16) go(bf16_t{});
+  else if (dtype == MVIT_F32) go(float{});
+  else return mvit_set_error(MVIT_ERR_UNSUPPORTED, "rmsnorm_fwd: dtype %d", dtype);
   MVIT_CHECK_LAUNCH("rmsnorm_fwd");
   return MVIT_OK;
 }
@@ -543,19 +750,17 @@ int mvit_rmsnorm_bwd(const void* dy, const void* x, const void* w, const float* 
   MVIT_REQUIRE(lds <= 160 * 1024, "rmsnorm_bwd: cols %lld needs %zu B of LDS (> 160 KiB)", (long long)cols, lds);
   const int grid = n_partial;  // every block writes its partial row, rows or not
   bool al = mvit_aligned16(dy) && mvit_aligned16(x) && mvit_aligned16(w) && mvit_aligned16(dx) && (!dx_add || mvit_aligned16(dx_add));
-  if (dtype == MVIT_BF16) {
-    if (cols % 8 == 0 && al)
-      hipLaunchKernelGGL((rmsnorm_bwd_kernel<bf16_t, true>), grid, 256, lds, S_(stream), (const bf16_t*)dy, (const bf16_t*)x, (const bf16_t*)w, rstd, (const bf16_t*)dx_add, (bf16_t*)dx, dw_partial, rows, (int)cols);
-    else
-      hipLaunchKernelGGL((rmsnorm_bwd_kernel<bf16_t, false>), grid, 256, lds, S_(stream), (const bf16_t*)dy, (const bf16_t*)x, (const bf16_t*)w, rstd, (const bf16_t*)dx_add, (bf16_t*)dx, dw_partial, rows, (int)cols);
-  } else if (dtype == MVIT_F32) {
-    if (cols % 4 == 0 && al)
-      hipLaunchKernelGGL((rmsnorm_bwd_kernel<float, true>), grid, 256, lds, S_(stream), (const float*)dy, (const float*)x, (const float*)w, rstd, (const float*)dx_add, (float*)dx, dw_partial, rows, (int)cols);
-    else
-      hipLaunchKernelGGL((rmsnorm_bwd_kernel<float, false>), grid, 256, lds, S_(stream), (const float*)dy, (const float*)x, (const float*)w, rstd, (const float*)dx_add, (float*)dx, dw_partial, rows, (int)cols);
-  } else {
-    return mvit_set_error(MVIT_ERR_UNSUPPORTED, "rmsnorm_bwd: dtype %d", dtype);
-  }
+  auto go = [&](auto zero) -> void {
+    using T = decltype(zero);
+    const bool vec = cols % mvit_elem<T>::vec == 0 && al;
+    auto kern = dx_add ? rms_bwd_row<T, true>(cols) : rms_bwd_row<T, false>(cols);
+    if (!vec) kern = rmsnorm_bwd_kernel<T, false>;
+    else if (kern == nullptr) kern = rmsnorm_bwd_kernel<T, true>;
+    hipLaunchKernelGGL(kern, grid, 256, lds, S_(stream), (const T*)dy, (const T*)x, (const T*)w, rstd, (const T*)dx_add, (T*)dx, dw_partial, rows, (int)cols);
+  };
+  if (dtype == MVIT_BF16) go(bf16_t{});
+  else if (dtype == MVIT_F32) go(float{});
+  else return mvit_set_error(MVIT_ERR_UNSUPPORTED, "rmsnorm_bwd: dtype %d", dtype);
   MVIT_CHECK_LAUNCH("rmsnorm_bwd");
   return MVIT_OK;
 }
@@ -615,27 +820,9 @@ int mvit_rope_scaled(void* x, const float* cosb, const float* sinb, int64_t rows
                "rope: bad shape rows=%lld heads=%d head_dim=%d stride=%lld", (long long)rows, nheads, head_dim, (long long)row_stride);
   if (rows == 0) return MVIT_OK;
   MVIT_REQUIRE(x && cosb && sinb, "rope: null pointer");
-  const int half = head_dim / 2;
-  const int64_t work_scalar = rows * nheads * half;
-  if (dtype == MVIT_BF16) {
-    if (half % 8 == 0 && row_stride % 8 == 0 && mvit_aligned16(x)) {
-      const int grid = clamp_grid((work_scalar / 8 + 255) / 256, 65535 * 16);
-      hipLaunchKernelGGL((rope_kernel<bf16_t, 8>), grid, 256, 0, S_(stream), (bf16_t*)x, cosb, sinb, rows, nheads, head_dim, row_stride, backward, lead_heads, lead_scale);
-    } else {
-      const int grid = clamp_grid((work_scalar + 255) / 256, 65535 * 16);
-      hipLaunchKernelGGL((rope_kernel<bf16_t, 1>), grid, 256, 0, S_(stream), (bf16_t*)x, cosb, sinb, rows, nheads, head_dim, row_stride, backward, lead_heads, lead_scale);
-    }
-  } else if (dtype == MVIT_F32) {
-    if (half % 4 == 0 && row_stride % 4 == 0 && mvit_aligned16(x)) {
-      const int grid = clamp_grid((work_scalar / 4 + 255) / 256, 65535 * 16);
-      hipLaunchKernelGGL((rope_kernel<float, 4>), grid, 256, 0, S_(stream), (float*)x, cosb, sinb, rows, nheads, head_dim, row_stride, backward, lead_heads, lead_scale);
-    } else {
-      const int grid = clamp_grid((work_scalar + 255) / 256, 65535 * 16);
-      hipLaunchKernelGGL((rope_kernel<float, 1>), grid, 256, 0, S_(stream), (float*)x, cosb, sinb, rows, nheads, head_dim, row_stride, backward, lead_heads, lead_scale);
-    }
-  } else {
-    return mvit_set_error(MVIT_ERR_UNSUPPORTED, "rope: dtype %d", dtype);
-  }
+  if (dtype == MVIT_BF16) launch_rope((bf16_t*)x, cosb, sinb, rows, nheads, head_dim, row_stride, backward, lead_heads, lead_scale, S_(stream));
+  else if (dtype == MVIT_F32) launch_rope((float*)x, cosb, sinb, rows, nheads, head_dim, row_stride, backward, lead_heads, lead_scale, S_(stream));
+  else return mvit_set_error(MVIT_ERR_UNSUPPORTED, "rope: dtype %d", dtype);
   MVIT_CHECK_LAUNCH("rope");
   return MVIT_OK;
 }

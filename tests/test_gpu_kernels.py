@@ -59,7 +59,50 @@ def test_rmsnorm_fwd_bwd(dtype, rows, cols):
     assert max_rel_err(dx2, xr.grad) < TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("cols", [8, 248, 256, 264, 512, 776, 1032, 1280, 1288, 1536, 2056, 2560, 2568])
+@pytest.mark.parametrize("rows", [1, 3, 4101])
+def test_rmsnorm_rows_of_whole_and_partial_vectors_per_lane(dtype, rows, cols):
+    """A row held in one to five vectors per lane, the last one whole, partial or one lane's, and a row too long for that (a pass per
+    use); one row per wave and more (4,101 rows on the 4,096 waves of the backward)."""
+    _announce(f"rmsnorm vectors per lane {dtype} {rows}x{cols}")
+    ops = _ops()
+    x, dy, add = (_rand((rows, cols), dtype, i) for i in range(3))
+    w = (1.0 + 0.1 * _rand((cols,), torch.float32, 3)).to(dtype)
+    y, rstd = ops.rmsnorm_fwd(x.to(DEV), w.to(DEV), 1e-6)
+    xr, wr = x.float().requires_grad_(True), w.float().requires_grad_(True)
+    yr = vit_oracle.rms_norm(xr, wr, 1e-6)
+    yr.backward(dy.float())
+    assert max_rel_err(y, yr) < TOL[dtype]
+    for with_add in (add, None):
+        dx, dw = ops.rmsnorm_bwd(dy.to(DEV), x.to(DEV), w.to(DEV), rstd, dx_add=None if with_add is None else with_add.to(DEV))
+        assert max_rel_err(dx, xr.grad + (0.0 if with_add is None else with_add.float())) < TOL[dtype]
+        assert max_rel_err(dw, wr.grad) < TOL[dtype]
+
+
 # ------------------------------------------------------------------------------------------ RoPE
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("S,H,d", [(1, 1, 16), (13, 5, 80), (7, 64, 128), (3, 3, 2048), (2, 2, 4112), (5, 700, 16), (2, 3, 8208)])
+def test_rope_chunks_over_heads_and_rows(dtype, S, H, d):
+    """Heads that a work-group takes at once or in turns, odd numbers of them, as many chunks per head as it has threads and more (which
+    go one pair at a time): each pair equals the rotation in float64, rounded once; the columns behind the heads stay."""
+    _announce(f"rope chunks {dtype} S={S} H={H} d={d}")
+    ops = _ops()
+    x, ang = _rand((S, H * d + 16), dtype, 0), _rand((S, d), torch.float32, 1, 3.0)
+    cos, sin, half = ang.cos(), ang.sin(), d // 2
+    c, s = cos.double().unsqueeze(1), sin.double().unsqueeze(1)
+    v = x[:, : H * d].double().reshape(S, H, d)
+    lo, hi, c0, c1, s0, s1 = v[..., :half], v[..., half:], c[..., :half], c[..., half:], s[..., :half], s[..., half:]
+    for backward, want in ((False, torch.cat([lo * c0 - hi * s0, hi * c1 + lo * s1], -1)), (True, torch.cat([lo * c0 + hi * s1, hi * c1 - lo * s0], -1))):
+        got = x.to(DEV)
+        ops.rope_(got, cos.to(DEV), sin.to(DEV), H, d, backward=backward, lead_heads=H // 2, lead_scale=0.25)
+        want = want * torch.where(torch.arange(H) < H // 2, 0.25, 1.0).view(1, H, 1)
+        # two products and a sum in fp32 of values below 6 in size, then one rounding to the type
+        bound = want.abs() * (2.0**-8 if dtype == torch.bfloat16 else 2.0**-24) + 6 * 2.0**-22
+        assert bool(((got[:, : H * d].cpu().double().reshape(S, H, d) - want).abs() <= bound).all())
+        assert torch.equal(got[:, H * d :].cpu(), x[:, H * d :])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("S,H,d", [(300, 16, 80), (64, 8, 32), (17, 4, 6)])
 def test_rope_fwd_bwd(dtype, S, H, d):
