@@ -198,7 +198,7 @@ __global__ __launch_bounds__(256) void resample_pass_kernel(const uint8_t* __res
 // ---- several passes in one launch
 constexpr int RESAMPLE_MAX_JOBS = 32;
 struct ResampleJobs {
-  int n, rows_per_wave;  // the latter of resample_narrow_lds_kernel
+  int n, rows_per_wave;  // the latter of resample_narrow_lds_kernel and resample_matrix_kernel
   int first_block[RESAMPLE_MAX_JOBS];
   mvit_resample_job job[RESAMPLE_MAX_JOBS];
 };
@@ -490,6 +490,276 @@ __global__ __launch_bounds__(256, 5) void resample_narrow_lds_kernel(const Resam
   }
 }
 
+// The same pass on the matrix cores, where a row's windows fit (on_mfma): a wave makes MATRIX_OUT output bytes of some rows, sixteen rows at
+// a time.  Sixteen output bytes of sixteen rows are a product of a 16 x 64 (KB times) matrix of weights, as v_mfma_i32_16x16x64_i8 takes it,
+// with the input bytes as they lie in the rows: a weight stands in the columns of its own channel's bytes, zeros elsewhere.  A weight is
+// three signed digits of 8 bits and a pixel is taken less 128 (one exclusive or on the way into LDS); 128 times the sum of the weights is
+// added back, itself a product with rows of -128.  Whole numbers modulo 2^32 throughout, so the sums are those of plain multiply-adds.
+// A wave keeps the weights of its three tiles in registers for all rows; the rows come as aligned 16-byte loads, LPR lanes to a row, and
+// are shifted on the way into the wave's own piece of LDS so that every row begins at the same alignment: no barrier.
+// Rows of a work-group: as many as make one round of MATRIX_GROUPS, three to a compute unit (150 registers), because a wave's weights take as long
+// to lay out as some fifty rows.  What bounds it: laying out the weights (6 us of 21), vector issue (145 instructions per sixteen rows) and stores
+// of 16 bytes per row (4 us).  us by the kernel above / this one, to 0.8 million pixels: 800 x 1,333 10.5 / 9.2, 1,080 x 1,920 12.9 / 11.8, 1,800 x 2,400 15.6 / 12.8,
+// 2,448 x 3,264 18.4 / 15.3, 2,700 x 3,600 17.9 / 15.6, these and 427 x 640 (below: made larger) together 25.9 / 20.2; 4,480 x 4,480 to 3,584 x 3,584 55 / 43; with 256 / 512 / 1,024
+// work-groups 31.0 / 22.7 / 26.4 and 65.7 / 43.9 / 49.8.  Not taken: larger windows (three times 64 bytes: 3,000 x 4,000 20 / 36) and images made larger, whose
+// four taps are little work for vector instructions (427 x 640 6.6 / 7.5, six of 240 x 320 12.7 / 14.2).
+constexpr int MATRIX_OUT = 48, MATRIX_TILES = MATRIX_OUT / 16, MATRIX_ROWS = 16, MATRIX_BLOCKS = 2, MATRIX_GROUPS = 768;
+// input bytes that sixteen output bytes' windows span at most, in units of 64, as bounds of any resampling between these lengths have them
+__host__ __device__ inline int64_t matrix_blocks(const mvit_resample_job& j) { return (((5 * j.in_len + j.out_len - 1) / j.out_len + 1 + j.ksize) * 3 + 15 + 63) / 64; }
+// v_perm selector that spreads a channel's taps, eight bytes, over word q of sixteen bytes of which its first is byte `skip`
+template <int INNER>
+constexpr unsigned tap_selector(int q, int skip) {
+  unsigned sel = 0;
+  for (int e = 0; e < 4; ++e) {
+    const int n = 4 * q + e - skip;
+    sel |= (unsigned)(n >= 0 && n % INNER == 0 ? (n / INNER) & 7 : 0x0c) << (8 * e);
+  }
+  return sel;
+}
+// Two values shifted right by the weights' fraction and clamped to a byte each, in the lower half; the upper half keeps old bits
+__device__ __forceinline__ unsigned clip8_pair(int a, int b) {
+  unsigned r;
+  asm("v_ashr_pk_u8_i32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "n"(RESAMPLE_PRECISION_BITS));
+  return r;
+}
+__global__ __launch_bounds__(256, 3) void resample_matrix_kernel(const ResampleJobs jobs) {
+  typedef int i32x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(1))) const unsigned char* global_bytes;
+  typedef __attribute__((address_space(1))) const u32x4* global_words;
+  constexpr int INNER = 3, LPR = 16, PXS = MATRIX_OUT / INNER, ROWS_AT_ONCE = 64 / LPR, LOADS = MATRIX_ROWS / ROWS_AT_ONCE;
+  constexpr int PITCH = LPR * 16 + 16;  // 16 bytes in front; sixteen rows fall on 16 different 16-byte slots of 256
+  constexpr int TAPS = (16 + INNER - 1) / INNER, PAD = (TAPS + 3) & ~3;  // taps of one channel in sixteen bytes; zeros around a window's digits
+  constexpr int DIG_DWORDS = (PAD + NARROW_TAPS + PAD) / 4;
+  __shared__ __attribute__((aligned(16))) unsigned char staged_all[4][MATRIX_ROWS * PITCH + 64 * MATRIX_BLOCKS];
+  __shared__ unsigned dig_all[4][3][PXS * DIG_DWORDS + 1];
+  const int j = resample_job_of(jobs, blockIdx.x);
+  const mvit_resample_job& jb = jobs.job[j];
+  const int block = blockIdx.x - jobs.first_block[j], lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  unsigned char* const staged = staged_all[wave];
+  unsigned(*const dig)[PXS * DIG_DWORDS + 1] = dig_all[wave];
+  const int i16 = lane & 15, g4 = lane >> 4;
+  const int in_len = (int)jb.in_len, out_len = (int)jb.out_len, ksize = jb.ksize;
+  const int row_in = in_len * INNER, row_out = out_len * INNER;
+  const int xblocks = (row_out + 4 * MATRIX_OUT - 1) / (4 * MATRIX_OUT), xb = (block % xblocks) * 4 + wave;
+  const int64_t o0 = (int64_t)(block / xblocks) * jobs.rows_per_wave;
+  const int rows = jb.outer - o0 < jobs.rows_per_wave ? (int)(jb.outer - o0) : jobs.rows_per_wave;
+  const int px0 = xb * PXS, px1 = px0 + PXS < out_len ? px0 + PXS : out_len;
+  if (px0 >= out_len) return;
+  auto window = [&](int x) { return tap_window(jb.bounds, x, ksize, in_len); };
+  // the bytes of a row from the first output's window to the last one's; windows out of that order go tap by tap
+  const TapWindow head = window(px0), tail = window(px1 - 1);
+  const int first = head.xmin, span = (tail.xmin + tail.n - first) * INNER;
+  bool fits = span >= 0 && span + 15 <= LPR * 16;
+  const uintptr_t start = reinterpret_cast<uintptr_t>(jb.src) + (uintptr_t)o0 * row_in + (unsigned)(first * INNER), start16 = start & ~(uintptr_t)15;
+  const uintptr_t lo = reinterpret_cast<uintptr_t>(jb.src), hi = lo + jb.outer * row_in;
+  const int below = lo > start16 ? (int)(lo - start16) : 0, end = hi - start16 < 0x7fffffff ? (int)(hi - start16) : 0x7fffffff;  // of the array, from start16
+
+  // A lane's chunk of each of its rows, aligned.  Where a row's chunks may stick out of the array (its first and last rows), those that do are
+  // filled byte by byte.
+  const int chunk = (lane % LPR) * 16, lane_at = (int)(start & 15) + (lane / LPR) * row_in;
+  const bool wanted = chunk < span + 15;
+  auto inside = [&](int step) {  // all chunks of these sixteen rows, the same for the wave
+    const int at = (int)(start & 15) + step * MATRIX_ROWS * row_in;
+    return (at & ~15) >= below && at + (MATRIX_ROWS - 1) * row_in + LPR * 16 <= end && (step + 1) * MATRIX_ROWS <= rows;
+  };
+  u32x4 v[LOADS];
+  auto request = [&](int step) {
+    const int at0 = lane_at + step * MATRIX_ROWS * row_in;
+    if (inside(step)) {
+#pragma unroll
+      for (int q = 0; q < LOADS; ++q)
+        if (wanted) v[q] = *reinterpret_cast<global_words>((global_bytes)start16 + (unsigned)(((at0 + q * ROWS_AT_ONCE * row_in) & ~15) + chunk));
+    } else {
+#pragma unroll
+      for (int q = 0; q < LOADS; ++q) {
+        const int row = step * MATRIX_ROWS + q * ROWS_AT_ONCE + lane / LPR, at = at0 + q * ROWS_AT_ONCE * row_in, from = (at & ~15) + chunk;
+        v[q] = u32x4{0u, 0u, 0u, 0u};
+        if (row < rows && wanted) {
+          if (from >= below && from + 16 <= end) {
+            v[q] = *reinterpret_cast<global_words>((global_bytes)start16 + (unsigned)from);
+          } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll 1
+              for (int e = 0; e < 4; ++e) {
+                const int byte = from + 4 * i + e;
+                if (byte >= below && byte < end) v[q][i] |= (unsigned)((global_bytes)start16)[(unsigned)byte] << (8 * e);
+              }
+          }
+        }
+      }
+    }
+  };
+  unsigned char* const put_at = staged + (lane / LPR) * PITCH + 16 + chunk;
+  auto put = [&](int step) {
+    const int at0 = lane_at + step * MATRIX_ROWS * row_in;
+#pragma unroll
+    for (int q = 0; q < LOADS; ++q) {
+      const unsigned at = (unsigned)(at0 + q * ROWS_AT_ONCE * row_in);
+      unsigned w[5] = {v[q][0], v[q][1], v[q][2], v[q][3], 0u};
+      w[4] = (unsigned)__builtin_amdgcn_update_dpp(0, (int)w[0], 0x101, 0xf, 0xf, true);  // of the next lane of the row's sixteen
+      unsigned* to = reinterpret_cast<unsigned*>(put_at + q * ROWS_AT_ONCE * PITCH - (at & 12));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) to[i] = __builtin_amdgcn_alignbyte(w[i + 1], w[i], at) ^ 0x80808080u;  // pixels less 128
+    }
+  };
+  if (fits) request(0);
+
+  int base[MATRIX_TILES], xmin[MATRIX_TILES];  // first input byte of a tile's product; the lane's window
+  const int k_blocks = matrix_blocks(jb);
+  TapWindow tws[MATRIX_TILES];
+#pragma unroll
+  for (int tl = 0; tl < MATRIX_TILES; ++tl) {
+    const int px = px0 + (tl * 16 + i16) / INNER;
+    tws[tl] = window(px < out_len ? px : out_len - 1);
+  }
+  // ---- signed digits of every output's weights, four taps a word
+  constexpr int DIG_LOOPS = (PXS * DIG_DWORDS + 63) / 64;
+  int k[DIG_LOOPS][4];
+#pragma unroll
+  for (int l = 0; l < DIG_LOOPS; ++l) {
+    const int i = l * 64 + lane, x = px0 + i / DIG_DWORDS, t0 = (i % DIG_DWORDS) * 4 - PAD;
+    const bool weights = x < px1 && t0 >= 0 && t0 < NARROW_TAPS;
+    const TapWindow tw = window(weights ? x : px0);
+    const int32_t* __restrict__ kk = jb.kk + (int64_t)x * ksize;
+    if (weights) fits = fits && tw.n <= NARROW_TAPS;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) k[l][t] = weights && t0 + t < tw.n ? kk[t0 + t] : 0;  // taps past the window have weight 0
+  }
+#pragma unroll
+  for (int l = 0; l < DIG_LOOPS; ++l) {
+    const int i = l * 64 + lane;
+    unsigned d[3] = {0u, 0u, 0u};
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      int rest = k[l][t];
+      fits = fits && fits_digits(rest);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        d[q] |= (unsigned)(rest & 0xff) << (8 * t);
+        rest = (rest + 128) >> 8;  // less the signed digit, by 256
+      }
+    }
+    if (i < PXS * DIG_DWORDS) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) dig[q][i] = d[q];
+    }
+  }
+#pragma unroll
+  for (int tl = 0; tl < MATRIX_TILES; ++tl) {
+    const int tile_first = __builtin_amdgcn_readfirstlane(tws[tl].xmin), last = (tws[tl].xmin + tws[tl].n - first) * INNER;
+    xmin[tl] = tws[tl].xmin;
+    base[tl] = ((tile_first - first) * INNER) & ~15;
+    fits = fits && tws[tl].xmin >= tile_first && tile_first >= first && last <= base[tl] + 64 * k_blocks && last <= span;
+  }
+  if (!__all(fits)) {  // windows or weights that no resampling table has
+    const int px = px1 - px0;
+    for (int i = lane; i < rows * px; i += 64) {
+      const int r = i / px, x = px0 + i % px;
+      const TapWindow tw = window(x);
+      const int32_t* __restrict__ kk = jb.kk + (int64_t)x * ksize;
+#pragma unroll 1
+      for (int c = 0; c < INNER; ++c) {
+        const uint8_t* p = jb.src + (o0 + r) * row_in + (int64_t)tw.xmin * INNER + c;
+        unsigned a = 1u << (RESAMPLE_PRECISION_BITS - 1);
+        for (int t = 0; t < tw.n; ++t) a += (unsigned)p[t * INNER] * (unsigned)kk[t];
+        jb.dst[(o0 + r) * row_out + (int64_t)x * INNER + c] = (uint8_t)clip8((int)a);
+      }
+    }
+    return;
+  }
+  auto in_order = [] {  // LDS operations of a wave are carried out in order; the compiler is to keep to it
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  in_order();
+
+  // ---- the lane's weights: output byte i16 of each tile, input bytes 16 * g4 .. + 15 of each 64
+  i32x4 weight[MATRIX_TILES][MATRIX_BLOCKS][3];
+#pragma unroll
+  for (int tl = 0; tl < MATRIX_TILES; ++tl) {
+    const int ob = tl * 16 + i16, x = ob / INNER, c = ob - x * INNER;
+#pragma unroll
+    for (int kb = 0; kb < MATRIX_BLOCKS; ++kb) {
+      const int p0 = base[tl] + kb * 64 + g4 * 16, px = p0 / INNER, skip = (c + INNER - (p0 - px * INNER)) % INNER;  // the channel's first byte
+      int t0 = px + (p0 - px * INNER > c ? 1 : 0) + first - xmin[tl];  // its tap
+      t0 = max(-PAD, min(t0, NARROW_TAPS)) + PAD;
+      unsigned sel[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        sel[q] = tap_selector<INNER>(q, 0);
+#pragma unroll
+        for (int e = 1; e < INNER; ++e) sel[q] = skip == e ? tap_selector<INNER>(q, e) : sel[q];
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const unsigned* at = &dig[i][x * DIG_DWORDS + (t0 >> 2)];
+        constexpr int N = (TAPS + 3) / 4;
+        unsigned raw[N + 1], taps[N];
+#pragma unroll
+        for (int q = 0; q <= N; ++q) raw[q] = at[q];
+#pragma unroll
+        for (int q = 0; q < N; ++q) taps[q] = __builtin_amdgcn_alignbyte(raw[q + 1], raw[q], (unsigned)t0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) weight[tl][kb][i][q] = (int)__builtin_amdgcn_perm(taps[1], taps[0], sel[q]);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // one product's digits at a time: registers
+    }
+  }
+  // a tile's sixteen output bytes of sixteen rows
+  auto product = [&](int tl, const i32x4 (&b)[MATRIX_BLOCKS]) {
+    i32x4 sum[3] = {};
+#pragma unroll
+    for (int kb = 0; kb < MATRIX_BLOCKS; ++kb)
+      if (kb < k_blocks) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) sum[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(weight[tl][kb][i], b[kb], sum[i], 0, 0, 0);
+      }
+    i32x4 all;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) all[e] = (int)((unsigned)sum[0][e] + ((unsigned)sum[1][e] << 8) + ((unsigned)sum[2][e] << 16));
+    return all;
+  };
+  i32x4 offset[MATRIX_TILES];  // 128 times the sum of the weights, and one half
+  {
+    i32x4 b[MATRIX_BLOCKS];
+#pragma unroll
+    for (int kb = 0; kb < MATRIX_BLOCKS; ++kb) b[kb] = i32x4{(int)0x80808080u, (int)0x80808080u, (int)0x80808080u, (int)0x80808080u};
+#pragma unroll
+    for (int tl = 0; tl < MATRIX_TILES; ++tl) offset[tl] = (1 << (RESAMPLE_PRECISION_BITS - 1)) - product(tl, b);
+  }
+  const bool words = row_out % 4 == 0 && (reinterpret_cast<uintptr_t>(jb.dst) & 3u) == 0;
+  const int steps = (rows + MATRIX_ROWS - 1) / MATRIX_ROWS, byte0 = 4 * g4, bytes = (px1 - px0) * INNER;
+  // a lane ends up with four consecutive bytes of row i16
+  uint8_t* d = jb.dst + o0 * row_out + (int64_t)px0 * INNER + ((int64_t)i16 * row_out + byte0);
+  for (int s = 0; s < steps; ++s, d += (int64_t)MATRIX_ROWS * row_out) {
+    put(s);
+    request(s + 1);
+    in_order();
+    const bool mine = s * MATRIX_ROWS + i16 < rows;
+    const unsigned char* at = staged + i16 * PITCH + 16 + 16 * g4;
+#pragma unroll
+    for (int tl = 0; tl < MATRIX_TILES; ++tl) {
+      i32x4 b[MATRIX_BLOCKS];
+#pragma unroll
+      for (int kb = 0; kb < MATRIX_BLOCKS; ++kb)
+        if (kb < k_blocks) b[kb] = *reinterpret_cast<const i32x4*>(at + base[tl] + kb * 64);
+      const i32x4 sum = offset[tl] + product(tl, b);
+      if (mine && byte0 + tl * 16 < bytes) {
+        if (words) {
+          *reinterpret_cast<unsigned*>(d + tl * 16) = __builtin_amdgcn_perm(clip8_pair(sum[2], sum[3]), clip8_pair(sum[0], sum[1]), 0x05040100u);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (byte0 + tl * 16 + e < bytes) d[tl * 16 + e] = (uint8_t)clip8(sum[e]);
+        }
+      }
+    }
+    in_order();
+  }
+}
+
 // The pass for a long contiguous dimension of whole words (the vertical pass).  A wave makes 1 KiB of one output row: the window
 // and its weights are the same for all of it (scalar loads), a lane makes 16 bytes from one 16-byte load per tap.  The four waves
 // of a work-group make the same KiB of four consecutive rows, whose windows overlap and meet in the L1.  Bound by the byte
@@ -607,11 +877,11 @@ int mvit_resample_u8_batch(const mvit_resample_job* list, int n_jobs, mvit_strea
   // weights' digits are made once per work-group.  us with 4 / 8 / 16 rows: 480 x 640 to 448 x 588-like sizes 11.5 / 13.2 / 16.6,
   // 2,448 x 3,264 and three smaller to 0.8 million pixels each 31.8 / 30.3 / 30.1, 4,480 x 4,480 to 3,584 x 3,584 69.5 / 59.6 / 56.2
   int rows_per_wave = 4;
-  auto shared_rows = [&](int kind) -> int64_t { return kind == 5 ? 1 : kind > 5 ? 4 * rows_per_wave : 4 * RESAMPLE_ROWS; };  // of a work-group
+  auto shared_rows = [&](int kind) -> int64_t { return kind == 5 ? 1 : kind == 10 ? rows_per_wave : kind > 5 ? 4 * rows_per_wave : 4 * RESAMPLE_ROWS; };  // of a work-group
   // work-groups for `outer` rows of the outermost axis
   auto groups = [&](int kind, const mvit_resample_job& j, int64_t outer) {
     if (kind == 5) return outer * ((j.out_len + 3) / 4) * ((j.inner + RESAMPLE_STRIP - 1) / RESAMPLE_STRIP);
-    return (j.out_len + 63) / 64 * ((outer + shared_rows(kind) - 1) / shared_rows(kind));
+    return (kind == 10 ? (j.out_len * 3 + 4 * MATRIX_OUT - 1) / (4 * MATRIX_OUT) : (j.out_len + 63) / 64) * ((outer + shared_rows(kind) - 1) / shared_rows(kind));
   };
   // jobs of one kind (wide words; 1 .. 4 bytes, with or without LDS) share launches; 0: everything else, a launch each.  Of short rows the
   // wide kernel only takes so few (about 5 us) that a launch of their own would cost as much
@@ -620,17 +890,33 @@ int mvit_resample_u8_batch(const mvit_resample_job* list, int n_jobs, mvit_strea
   auto through_lds = [](const mvit_resample_job& j) {
     return j.ksize <= NARROW_TAPS && ((63 * j.in_len + j.out_len - 1) / j.out_len + j.ksize + 1) * j.inner + 15 <= NARROW_SPAN;
   };
+  // three channels on the matrix cores (10), up to the windows that its registers hold the weights of, about 3.8-fold; rows made longer only go
+  // along with others, because a launch of their own would cost more than the vector instructions save
+  auto fits_matrix = [](const mvit_resample_job& j) {
+    return j.inner == 3 && j.ksize <= NARROW_TAPS && matrix_blocks(j) <= MATRIX_BLOCKS && j.in_len < (1 << 18) && j.out_len < (1 << 28) &&
+           (((MATRIX_OUT / 3 - 1) * j.in_len + j.out_len - 1) / j.out_len + 1 + j.ksize) * 3 + 15 <= 256;
+  };
+  bool matrix = false;
+  for (int i = 0; i < n_jobs; ++i) matrix = matrix || (list[i].outer > 0 && list[i].out_len <= list[i].in_len && fits_matrix(list[i]));
   auto kind_of = [&](const mvit_resample_job& j) {
+    if (matrix && fits_matrix(j)) return 10;
     if (j.inner <= RESAMPLE_MAX_CHANNELS) return (int)j.inner + (through_lds(j) ? 5 : 0);
     const bool wide = j.inner >= RESAMPLE_WIDE_FROM || (j.inner >= 16 && j.outer * j.out_len <= RESAMPLE_FEW_ROWS);
     return words(j) && wide && groups(5, j, 1) <= MVIT_MAX_GROUPS_256 ? 5 : 0;
   };
-  for (int kind = 0; kind <= 9; ++kind) {
+  for (int kind = 0; kind <= 10; ++kind) {
     if (kind > 5) {
       int64_t waves = 0;
       for (int i = 0; i < n_jobs; ++i)
         if (kind_of(list[i]) == kind) waves += (list[i].out_len + 63) / 64 * list[i].outer;
       rows_per_wave = waves >= 4 * 1024 * 16 ? 16 : waves >= 4 * 1024 * 8 ? 8 : 4;
+    }
+    if (kind == 10) {
+      int64_t steps = 0;
+      for (int i = 0; i < n_jobs; ++i)
+        if (kind_of(list[i]) == kind) steps += (list[i].out_len * 3 + 4 * MATRIX_OUT - 1) / (4 * MATRIX_OUT) * ((list[i].outer + MATRIX_ROWS - 1) / MATRIX_ROWS);
+      const int64_t each = (steps + MATRIX_GROUPS - 1) / MATRIX_GROUPS;
+      rows_per_wave = MATRIX_ROWS * (int)(each < 1 ? 1 : each > 64 ? 64 : each);
     }
     ResampleJobs jobs;
     memset(&jobs, 0, sizeof(jobs));
@@ -648,6 +934,7 @@ int mvit_resample_u8_batch(const mvit_resample_job* list, int n_jobs, mvit_strea
         case 7: hipLaunchKernelGGL((resample_narrow_lds_kernel<2>), grid, 256, 0, s, jobs); break;
         case 8: hipLaunchKernelGGL((resample_narrow_lds_kernel<3>), grid, 256, 0, s, jobs); break;
         case 9: hipLaunchKernelGGL((resample_narrow_lds_kernel<4>), grid, 256, 0, s, jobs); break;
+        case 10: hipLaunchKernelGGL(resample_matrix_kernel, grid, 256, 0, s, jobs); break;
         default: hipLaunchKernelGGL(resample_wide_kernel, grid, 256, 0, s, jobs); break;
       }
       MVIT_CHECK_LAUNCH("resample_u8");
