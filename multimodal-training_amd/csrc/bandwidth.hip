@@ -499,7 +499,13 @@ __global__ __launch_bounds__(256) void segment_copy_kernel(const W* __restrict__
 
 // Copies of contiguous byte ranges, the list being a kernel argument: nothing has to reach the device in front of the launch.
 // A work-group moves one 32 KiB piece; every thread has eight independent 16-byte loads in flight.  HBM-bound.
+// A launch's loads and stores carry the non-temporal hint by what it moves in all (COPY_NT_LOADS, COPY_NT_STORES): a source that
+// is read once only pushes the destination out of the 256 MB memory-side cache, and a destination that fills most of it is gone
+// before its reader comes.  Split over ranks and put together again, us plain / with the hint: 320 MiB 248 / 210 (four ranks),
+// 240 MiB 178 / 149 (two ranks).  Smaller launches find their source in that cache: 39 MiB 33.4 / 36.6 with hinted loads, 40 MiB
+// a rank 51.6 / 56; stores with the hint at 120 MiB a rank 160 instead of 149.
 constexpr int COPY_MAX_RANGES = 96, COPY_STEPS = 8, COPY_PIECE = 256 * COPY_STEPS;  // words per piece
+constexpr int64_t COPY_NT_LOADS = 64ll << 20, COPY_NT_STORES = 160ll << 20;         // bytes of a launch
 struct CopyRanges {
   int n;
   int first_piece[COPY_MAX_RANGES];
@@ -507,7 +513,7 @@ struct CopyRanges {
   void* dst[COPY_MAX_RANGES];
   int64_t words[COPY_MAX_RANGES];
 };
-template <typename W>
+template <typename W, bool NT_LOADS, bool NT_STORES>
 __global__ __launch_bounds__(256) void copy_ranges_kernel(const CopyRanges a) {
   int lo = 0, hi = a.n;  // invariant: first_piece[lo] <= blockIdx.x < first_piece[hi]
   while (hi - lo > 1) {
@@ -518,16 +524,21 @@ __global__ __launch_bounds__(256) void copy_ranges_kernel(const CopyRanges a) {
   const int64_t begin = (int64_t)(blockIdx.x - a.first_piece[lo]) * COPY_PIECE + threadIdx.x, words = a.words[lo];
   const W* s = static_cast<const W*>(a.src[lo]) + begin;
   W* d = static_cast<W*>(a.dst[lo]) + begin;
+  auto load = [&](int i) { return NT_LOADS ? __builtin_nontemporal_load(s + i * 256) : s[i * 256]; };
+  auto store = [&](int i, W v) {
+    if (NT_STORES) __builtin_nontemporal_store(v, d + i * 256);
+    else d[i * 256] = v;
+  };
   if (begin - (int64_t)threadIdx.x + COPY_PIECE <= words) {
     W v[COPY_STEPS];
 #pragma unroll
-    for (int i = 0; i < COPY_STEPS; ++i) v[i] = s[i * 256];
+    for (int i = 0; i < COPY_STEPS; ++i) v[i] = load(i);
 #pragma unroll
-    for (int i = 0; i < COPY_STEPS; ++i) d[i * 256] = v[i];
+    for (int i = 0; i < COPY_STEPS; ++i) store(i, v[i]);
   } else {
 #pragma unroll
     for (int i = 0; i < COPY_STEPS; ++i)
-      if (begin + i * 256 < words) d[i * 256] = s[i * 256];
+      if (begin + i * 256 < words) store(i, load(i));
   }
 }
 
@@ -974,18 +985,20 @@ int mvit_copy_ranges(const mvit_copy_range* ranges, int n_ranges, mvit_stream_t 
   }
   const int64_t word = bits % 16 == 0 ? 16 : (bits % 4 == 0 ? 4 : (bits % 2 == 0 ? 2 : 1));  // the widest that suits every range
   CopyRanges a;
-  int64_t pieces = 0;
+  int64_t pieces = 0, bytes = 0;
   a.n = 0;
   auto flush = [&]() -> int {
     if (a.n == 0) return MVIT_OK;
     const dim3 grid((unsigned)pieces);
-    if (word == 16) hipLaunchKernelGGL((copy_ranges_kernel<u32x4>), grid, 256, 0, S_(stream), a);
-    else if (word == 4) hipLaunchKernelGGL((copy_ranges_kernel<uint32_t>), grid, 256, 0, S_(stream), a);
-    else if (word == 2) hipLaunchKernelGGL((copy_ranges_kernel<uint16_t>), grid, 256, 0, S_(stream), a);
-    else hipLaunchKernelGGL((copy_ranges_kernel<uint8_t>), grid, 256, 0, S_(stream), a);
+    if (word == 16 && bytes >= COPY_NT_STORES) hipLaunchKernelGGL((copy_ranges_kernel<u32x4, true, true>), grid, 256, 0, S_(stream), a);
+    else if (word == 16 && bytes >= COPY_NT_LOADS) hipLaunchKernelGGL((copy_ranges_kernel<u32x4, true, false>), grid, 256, 0, S_(stream), a);
+    else if (word == 16) hipLaunchKernelGGL((copy_ranges_kernel<u32x4, false, false>), grid, 256, 0, S_(stream), a);
+    else if (word == 4) hipLaunchKernelGGL((copy_ranges_kernel<uint32_t, false, false>), grid, 256, 0, S_(stream), a);
+    else if (word == 2) hipLaunchKernelGGL((copy_ranges_kernel<uint16_t, false, false>), grid, 256, 0, S_(stream), a);
+    else hipLaunchKernelGGL((copy_ranges_kernel<uint8_t, false, false>), grid, 256, 0, S_(stream), a);
     MVIT_CHECK_LAUNCH("copy_ranges");
     a.n = 0;
-    pieces = 0;
+    pieces = bytes = 0;
     return MVIT_OK;
   };
   for (int i = 0; i < n_ranges; ++i) {
@@ -1000,6 +1013,7 @@ int mvit_copy_ranges(const mvit_copy_range* ranges, int n_ranges, mvit_stream_t 
       a.dst[a.n] = dst;
       a.words[a.n++] = words;
       pieces += (words + COPY_PIECE - 1) / COPY_PIECE;
+      bytes += words * word;
       src += words * word;
       dst += words * word;
       left -= words;

@@ -752,6 +752,28 @@ def test_copy_ranges_bit_exact(unit, offset, n):
     assert torch.equal(dst, want)
 
 
+@pytest.mark.parametrize("total", [(64 << 20) - 16, 64 << 20, (160 << 20) - 16, 160 << 20, (160 << 20) + 16])
+def test_copy_ranges_at_the_sizes_where_loads_and_stores_change_their_hint(total):
+    """Launches that move this many bytes in all, in ranges of whole and partial pieces; around them nothing is written."""
+    import ctypes
+
+    from mi355_vit import _lib
+
+    _announce(f"copy ranges of {total} bytes in all")
+    src = torch.randint(-(2**31), 2**31 - 1, (total // 4,), dtype=torch.int32, device=DEV)
+    dst = torch.full((total // 4 + 8,), 9, dtype=torch.int32, device=DEV)
+    cuts = [0, 16, 16 + 32768, 16 + 2 * 32768 - 16, total // 2 // 16 * 16 + 16, total]
+    ranges, to = [], total + 16  # taken in order, laid down in reverse, 16 bytes free on both sides
+    want = dst.clone()
+    for a, b in zip(cuts, cuts[1:]):
+        to -= b - a
+        ranges += [src.data_ptr() + a, dst.data_ptr() + to, b - a]
+        want[to // 4 : (to + b - a) // 4] = src[a // 4 : b // 4]
+    arg = (ctypes.c_uint64 * len(ranges))(*ranges)
+    _lib.check(_lib.load().mvit_copy_ranges(ctypes.addressof(arg), len(ranges) // 3, torch.cuda.current_stream().cuda_stream), "mvit_copy_ranges")
+    assert torch.equal(dst, want)
+
+
 @pytest.mark.parametrize("row_bytes", [2, 6, 20, 32, 2560, 5120 * 16])
 def test_segment_copy_entry_point_with_its_list_on_the_device(row_bytes):
     """mvit_segment_copy, for callers whose list is in device memory; words of 2, 4 and 16 bytes, bit-exact."""
