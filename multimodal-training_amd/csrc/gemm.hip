@@ -1166,7 +1166,10 @@ bool pp_takes(GemmTiledKind kind, int64_t k_chunk, int64_t k_last) {  // at leas
 // step of 64 along K takes 1.15 us in a 256 x 256 tile (one work-group per compute unit; 1.2 with both operands behind the
 // transposing LDS read; 2,392 cycles, so more when the clock falls under a long load, which lengthens every tile's steps alike), and in the smaller ones `one` us while every unit has at most one work-group and `two` us once it has
 // two.  Tiles of one work-group per unit (`lone`) interleave loads, LDS reads and MFMAs, so their steps are shorter than those of a
-// single work-group of the kind that shares its unit: 128 x 128 is taken up to 256 tiles and 192 x 128 from there to 256 tiles again
+// single work-group of the kind that shares its unit: 32 x 64 is taken up to 256 tiles, then 64 x 64 up to 256, two of them to a unit up to 448, 64 x 128
+// from there to 256, 128 x 128 and 192 x 128 in the same way (1280 columns, weights from HBM, us at K = 6912, 3840, 3456, 1280, 64 x 64 / 32 x 64: 256 rows
+// 34.8, 21.9, 18.7, 9.5 / 28.6, 18.0, 14.5, 8.3, 512 rows 34.4, 21.5, 18.6, 9.5 / 36.9, 22.1, 17.8, 9.4; 64 x 64 / 64 x 128: 1,024 rows 43.4, 25.8, 23.4, 11.6 /
+// 44.4, 27.7, 25.4, 13.1, 1,400 rows 46.2, 27.4, 24.8, 12.6 / 44.6, 27.8, 26.6, 14.5, 1,600 rows 55.9, 33.7, 28.5, 13.9 / 45.0, 27.9, 25.6, 13.2)
 // (input gradient of 6912 x 1280, us, shared / 128 lone / 192 lone: 2,048 rows 70 / 48 / 61, 3,136 73 / 55 / 65, 4,096 78 / 95 / 68,
 // 6,084 91 / 104 / 127; ms per step before -> with them: 3,136 rows 21.0 -> 19.9, 4,096 checkpointed 29.2 -> 28.0).  A fuller last round, a shorter step and more units at work all lower the estimate; the epilogue of a 256 x 256 tile is
 // the longest.  The line between the tiles follows from these numbers and not from any shape: e.g. weight gradients of
@@ -1214,6 +1217,7 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
     const int64_t slots = two > 0. ? 2 * (int64_t)n_cu : n_cu, full = items / slots, rest = items % slots;
     const double round = steps * (two > 0. ? two : one) + per_tile;
     double us = full * round;
+    if (bm * bn == 64 * 64 && full == 0 && 4 * rest > 7 * n_cu) two *= 1.15;  // nearly all units with two
     if (rest > 0) us += steps * (two > 0. && rest > n_cu ? two : one) + per_tile;
     if (input_grad && !overlapped && two > 0. && items > slots) us *= 1. + (bm == 128 ? 0.05 : 0.15) * (double)((items - 1) / slots);
     us = 4. + alone * us + (1. - alone) * round * (double)items / (double)slots;
@@ -1222,6 +1226,7 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
   const bool swiglu = kind == NN_SWIGLU;
   if (pp_takes(kind, k_chunk, k_last) && kind != NT_SWIGLU_BWD) consider(256, 256, tt ? 1.2 : PP_STEP_US, 0., swiglu ? PP_SWIGLU_TILE_US : PP_TILE_US);
   if (kind == NT_SWIGLU_BWD) {  // two inputs, two outputs and the column sums lengthen its epilogue
+    consider(64, 64, 0.28, 0., 2., true);
     consider(64, 64, 0.30, 0.43, 2.);
     consider(64, 128, 0.47, 0.70, 2.);
     consider(128, 128, 0.55, 0.90, 5.);
@@ -1231,9 +1236,11 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
     if (!swiglu) consider(64, 64, 0.19, 0.36, 2.);
     consider(64, 128, 0.37, 0.52, 2.);
     consider(128, 128, 0.60, 0.72, swiglu ? 6. : 2.5);
+    consider(128, 128, swiglu ? 0.45 : 0.44, 0., swiglu ? 2.5 : 3., true);
     if (!swiglu) {
+      consider(32, 64, 0.15, 0., 1.2, true);
       consider(64, 64, 0.18, 0., 2., true);
-      consider(128, 128, 0.44, 0., 3., true);
+      consider(64, 128, 0.365, 0., 2., true);
       consider(192, 128, 0.60, 0., 4., true);
     }
   }

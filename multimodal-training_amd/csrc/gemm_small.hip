@@ -1,22 +1,29 @@
 // bf16 GEMM for products with too few 256 x 256 tiles to fill the chip: one work-group per BM x BN tile, NW waves of
 // WM x WN, K tiles of 64 in a ring of NST LDS stages filled by direct global -> LDS loads up to NST - 1 K tiles ahead.
-// Rings of four stages and more: a wave reads the next half K tile's fragments from LDS, and requests its share of the K tile
-// NST - 1 ahead, between the MFMAs of the present half.  Requesting the whole share at once stalls the wave's MFMAs until the
-// address unit has taken it (16 clocks per KiB: half of the step).  us, one step after the other -> interleaved, operands in the
-// cache: 256 rows, K = 3456 on 64 x 64 17.6 -> 13.7, K = 6912 (input gradient) 30.2 -> 25.2; 2,048 rows on 128 x 128, one work-group
-// per unit, 39.4 -> 28, 70 -> 52; MFMAs alone would take 21 and 33.  Moving the reads to the half's beginning, or a fifth stage
-// there, gives nothing.  Loads requested later need more stages: weights from memory, 256 rows, K = 6912, rings of 4 / 6 / 10 stages
-// 35.6 / 34.1 / 35.4 (34.8 with all loads at the beginning of the step and 4), hence Lone64; 64 x 128 with three stages is slower
-// interleaved (SwiGLU of 256 rows 14.7 -> 18.0).
-// Two or three stages (so that two work-groups share a compute unit): one work-group multiplies while the other waits.  The same
+// A wave reads the next fragments from LDS, and requests its share of a K tile further on, between the MFMAs of the present ones.
+// Requesting the whole share at once stalls the wave's MFMAs until the address unit has taken it (16 clocks per KiB: half of the step).
+// What bounds a step is the unit's way from L2 into LDS and out of it again: some 64 bytes per clock in, 200 out, one after the other, i.e.
+// 0.18 us for a 64 x 64 tile's K tile of 64 whether one work-group has the unit or two share it, 0.27 for 64 x 128, 0.13 for 32 x 64.  So the
+// tile that puts each unit to work once wins, and the fewer bytes per product the better.  Weights that come from HBM make a step 1.2 to 1.6 times
+// as long, again by its bytes and whatever the ring's depth (a unit's requests in flight).  1280 columns, operands in the caches, us, 64 x 64 (two to
+// a unit beyond 256 tiles) / 64 x 128 (one), K = 6912, 3840, 3456 and 1280: 1,024 rows 42.3, 25.0, 21.9, 11.2 / 34.8, 20.1, 18.0, 10.4; 1,600 rows
+// 52.4, 27.5, 23.3, 12.0 / 41.7, 21.0, 19.0, 10.8; 64 x 64 / 32 x 64, 256 rows 24.6, 15.6, 13.5, 7.7 / 20.6, 12.9, 10.5, 6.5.  From HBM: choose_tile.
+// Two forms of the loop:
+// * `WHOLE`: the fragments of a whole K tile are read one K tile ahead, so a step has one barrier and one LDS latency, and the stage that a
+//   step has read is free for the K tile a whole ring ahead: the tiles of 64 rows and fewer that have a unit to themselves.  As many stages as cover
+//   the latency of L2 and no more, because the first K tile waits for the ring's first requests (64 x 64, us at K = 6912 / 1280: 4 stages 24.1 / 7.3,
+//   6 24.6 / 7.8, 9 25.4 / 8.8; by halves and 6 stages 24.6 / 7.7).
+// * by halves of a K tile: 128 x 128 and 192 x 128, whose halves have MFMAs enough to cover the LDS latency (whole K tiles: 192 x 128 66 -> 76 us at
+//   4,096 rows and K = 6912; 128 x 128 with residual 13.3 -> 14.4 at K = 1280), and 64 x 64 where two share a unit (weights from HBM, 1,024 rows, input
+//   gradients, whole K tiles / halves 46.6, 27.6, 11.7 / 43.4, 25.8, 11.3).  One step after the other -> by halves, 2,048 rows on 128 x 128 39.4 -> 28,
+//   70 -> 52; MFMAs alone would take 21 and 33.  SwiGLU of 257 to 512 rows on 128 x 128, two work-groups of two stages / one of four: 18.3 / 14.5.
+// Two stages of 128 x 128 and three of 64 x 128 (so that two work-groups share a compute unit): one multiplies while the other waits.  The same
 // loop serves the weight gradients (A behind the transposing read) with every ring: interleaved they are no faster (1280 x 1280
 // over 6,084 rows 44.9 / 44.4 us; ms per step 4,096 rows 29.0 / 29.2, 4,900 30.2 / 30.0, 6,084 35.4 / 35.6).  Their tiles that sum A's rows
 // have a loop of their own: a branch in the loop made the others wait too (3840 x 1280 over 6,084 rows 80.7 -> 71.5, over 4,096 58.6 -> 52.7).
 // A wave's tile is as square as its registers allow, because LDS reads are the next limit: 128 x 128 split in eight waves of
 // 32 x 64 read 96 KiB per K tile, in four of 64 x 64 64 KiB (4,096 rows, two transposed-layout operands, K = 6848: 84 -> 77 us;
 // K contiguous in both, K = 3424: 55 -> 52; weight gradient of 3840 x 1280 over 2,048 rows: 32 -> 27).
-// What bounds it is the chain of K steps of one tile, not the matrix pipe: small tiles make the step short (a 64 x 64 tile's
-// step moves 16 KiB into LDS, the 256 x 256 tile's 64 KiB) and put more compute units to work.
 // Fragment layouts, K order, MFMA form and epilogue arithmetic are those of gemm_pp_kernel (gemm_pingpong.hip), so the results
 // are the same bits whichever of the two computed them.
 // SwiGLU backward, 128 x 128 (224 registers: two inputs per element beside the accumulators) / 64 x 128 alone, us at 2,048 rows: 27 / 34.
@@ -27,13 +34,14 @@
 
 namespace {
 
-template <int BM_, int BN_, int WGM_, int WGN_, int NST_>
+template <int BM_, int BN_, int WGM_, int WGN_, int NST_, bool WHOLE_ = false>
 struct SmallCfg {
+  static constexpr bool WHOLE = WHOLE_;  // form of the main loop, see above
   static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, NST = NST_, BK = 64;
   static constexpr int NW = WGM * WGN, NTHREADS = 64 * NW, WM = BM / WGM, WN = BN / WGN;
   static constexpr int A_BYTES = BM * BK * 2, STAGE = (BM + BN) * BK * 2, LDS = NST * STAGE;
   static constexpr int PER_A = BM / 8 / NW, PER_B = BN / 8 / NW, PER = PER_A + PER_B;  // 1 KiB loads per wave and K tile
-  static_assert(NST >= 2 && (NST - 2) * PER < 64 && (BM == 64 || BM == 128 || BM == 192) && (BN == 64 || BN == 128), "ring depths and swizzles built");
+  static_assert(NST >= 2 && (NST - 1) * PER < 64 && (BM == 32 || BM == 64 || BM == 128 || BM == 192) && (BN == 64 || BN == 128), "ring depths and swizzles built");
   static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0 && WM % 16 == 0 && WN % 32 == 0, "whole load instructions and MFMA blocks per wave");
 };
 
@@ -201,7 +209,7 @@ __device__ __forceinline__ void gemm_small_tile(const GemmParams& p, const unsig
     }
   }
 
-  constexpr bool INTERLEAVED = NST >= 4 && !TA;
+  constexpr bool INTERLEAVED = (NST >= 4 || S::WHOLE) && !TA;
   // sums of A's rows over k, see gemm_pingpong.hip: wave wn of a row group takes NRS row blocks, two MFMAs more each per K tile
   constexpr bool ROW_SUMS = TA && TB && EPI == MVIT_EPI_NONE;
   constexpr int NRS = NA / S::WGN;  // row blocks that a wave sums
@@ -235,7 +243,81 @@ __device__ __forceinline__ void gemm_small_tile(const GemmParams& p, const unsig
     wait_tiles<S::PER, NST - 2>(newer);
   };
   auto next_stage = [&](unsigned& stage) { stage = stage + S::STAGE == S::LDS ? 0 : stage + S::STAGE; };
-  if constexpr (INTERLEAVED) {
+  if constexpr (INTERLEAVED && S::WHOLE) {
+    // The K tile of parity `par` in registers: its MFMAs row by row, between them the reads of the K tile after it (at `next`) and the loads
+    // of the one NST ahead into the stage that this tile was read from.  The compiler keeps to this order.
+    bf16x8 ga[2][2][NA], gb[2][2][NB];  // fragments: parity of the K tile, half, block
+    auto read_next = [&](const unsigned char* at, int par, int r) {
+      const int ks = r / (NA + NB), i = r % (NA + NB);
+      if (i < NB) {
+        if constexpr (!TB) gb[par][ks][i] = *reinterpret_cast<const bf16x8*>(at + rb[ks] + (i >> 1) * 4096 + (i & 1) * 512);
+        else gb[par][ks][i] = pp_read_tr(at + rb[i] + ks * 32 * (BN * 2), 4 * (BN * 2));
+      } else {
+        if constexpr (!TA) ga[par][ks][i - NB] = *reinterpret_cast<const bf16x8*>(at + ra[ks] + (i - NB) * 2048);
+        else ga[par][ks][i - NB] = pp_read_tr(at + ra[i - NB] + ks * 32 * (BM * 2), 4 * (BM * 2));
+      }
+    };
+    auto step = [&](auto parity, auto with_loads, const unsigned char* next, unsigned stage_off) {
+      constexpr int par = decltype(parity)::value, LOADS = decltype(with_loads)::value ? S::PER : 0, READS = 2 * (NA + NB), ROWS = 2 * NA;
+#pragma unroll
+      for (int a = 0; a < ROWS; ++a) {
+#pragma unroll
+        for (int r = a * READS / ROWS; r < (a + 1) * READS / ROWS; ++r) read_next(next, 1 - par, r);
+#pragma unroll
+        for (int j = a * LOADS / ROWS; j < (a + 1) * LOADS / ROWS; ++j) {
+          if (j < S::PER_A) pp_load(lds_base + stage_off + (wv * S::PER_A + j) * 1024, va[j], ba);
+          else pp_load(lds_base + stage_off + S::A_BYTES + (wv * S::PER_B + j - S::PER_A) * 1024, vb[j - S::PER_A], bb);
+        }
+        const int ks = a / NA, i = a % NA;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[i][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gb[par][ks][b], ga[par][ks][i], acc[i][b], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    auto landed_after = [&](int newer) { wait_tiles<S::PER, NST - 2>(newer < 0 ? 0 : newer); };
+    if (NST - 1 < n_kt) issue(NST - 1, st_in);  // the last stage is free as well
+    wait_tiles<S::PER, NST - 1>(n_kt - 1);
+    pp_barrier();
+#pragma unroll
+    for (int r = 0; r < 2 * (NA + NB); ++r) read_next(smem_raw, 0, r);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    landed_after(n_kt - 2);
+    pp_barrier();
+    // At the top of step t every wave has the fragments of K tile t, so its stage is free, and tile t + 1 has landed.  The last step's reads
+    // past the end stay in the ring and are not used.
+    int t = 0;
+    auto advance = [&](auto parity) {  // tile t + NST exists and is a whole one
+      const unsigned here = st;
+      next_stage(st);
+      step(parity, std::true_type{}, smem_raw + st, here);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      pp_wait_vm<(NST - 2) * S::PER>();
+      pp_barrier();
+      ba += step_a;
+      bb += step_b;
+      ++t;
+    };
+    auto finish = [&](auto parity) {
+      const unsigned here = st;
+      next_stage(st);
+      if (t + NST < n_kt) issue(t + NST, here);
+      step(parity, std::false_type{}, smem_raw + st, 0);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      landed_after(n_kt - 3 - t);
+      pp_barrier();
+      ++t;
+    };
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    for (const int whole = n_kt - NST - (k_tail != 0 ? 1 : 0); t + 1 < whole;) {
+      advance(even);
+      advance(odd);
+    }
+    while (t < n_kt) {
+      finish(even);
+      if (t < n_kt) finish(odd);
+    }
+  } else if constexpr (INTERLEAVED) {
     constexpr int FIRST = S::PER / 2;  // loads requested in the first half
     // half `ks` of a K tile: its MFMAs row by row, between them the reads of the half after it (at `next`) and loads into stage_off.
     // The compiler keeps to this order.
@@ -432,9 +514,11 @@ using Small64 = SmallCfg<64, 64, 2, 2, 4>;       // 64 KiB of LDS
 using Small64x128 = SmallCfg<64, 128, 2, 2, 3>;  // 72 KiB
 using Small128 = SmallCfg<128, 128, 2, 2, 2>;    // 64 KiB
 // one work-group per compute unit, which has work for one at most
-using Lone64 = SmallCfg<64, 64, 2, 2, 6>;     // 96 KiB
-using Lone128 = SmallCfg<128, 128, 2, 2, 4>;  // 128 KiB
-using Lone192 = SmallCfg<192, 128, 2, 2, 4>;  // 160 KiB
+using Lone32x64 = SmallCfg<32, 64, 2, 2, 5, true>;    // 60 KiB
+using Lone64 = SmallCfg<64, 64, 2, 2, 4, true>;       // 64 KiB
+using Lone64x128 = SmallCfg<64, 128, 2, 2, 4, true>;  // 96 KiB
+using Lone128 = SmallCfg<128, 128, 2, 2, 4>;          // 128 KiB
+using Lone192 = SmallCfg<192, 128, 2, 2, 4>;          // 160 KiB
 
 template <typename S, typename P>
 int launch_grid(void (*kern)(P), const P& p, unsigned grid, bool (&attr_set_on)[MVIT_MAX_DEVICES], hipStream_t stream) {
@@ -497,6 +581,12 @@ int dispatch_lone(GemmTiledKind kind, const GemmParams& p, hipStream_t s) {
     case NN_BIAS_GELU: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_GELU, S>(p, s);
     case NT_NONE: return launch_small<bf16_t, false, true, MVIT_EPI_NONE, S>(p, s);
     case NT_GELU_BWD: return launch_small<bf16_t, false, true, MVIT_EPI_GELU_BWD, S>(p, s);
+    case NN_SWIGLU:
+      if constexpr (S::BM == 128) return launch_small<bf16_t, false, false, MVIT_EPI_SWIGLU, S>(p, s);
+      break;
+    case NT_SWIGLU_BWD:
+      if constexpr (S::BM == 64 && S::BN == 64) return launch_small<bf16_t, false, true, MVIT_EPI_SWIGLU_BWD, S>(p, s);
+      break;
     default: break;
   }
   return mvit_set_error(MVIT_ERR_UNSUPPORTED, "gemm: product kind %d has no %d x %d kernel of one work-group per unit", (int)kind, S::BM, S::BN);
@@ -505,7 +595,12 @@ int dispatch_lone(GemmTiledKind kind, const GemmParams& p, hipStream_t s) {
 }  // namespace
 
 int mvit_gemm_small(GemmTiledKind kind, int bm, int bn, bool lone, const GemmParams& p, hipStream_t stream) {
-  if (lone) return bm == 192 ? dispatch_lone<Lone192>(kind, p, stream) : bm == 128 ? dispatch_lone<Lone128>(kind, p, stream) : dispatch_lone<Lone64>(kind, p, stream);
+  if (lone) {
+    if (bm == 192) return dispatch_lone<Lone192>(kind, p, stream);
+    if (bm == 128) return dispatch_lone<Lone128>(kind, p, stream);
+    if (bm == 32) return dispatch_lone<Lone32x64>(kind, p, stream);
+    return bn == 128 ? dispatch_lone<Lone64x128>(kind, p, stream) : dispatch_lone<Lone64>(kind, p, stream);
+  }
   if (bm == 128) return dispatch_small<Small128>(kind, p, stream);
   if (bn == 128) return dispatch_small<Small64x128>(kind, p, stream);
   return dispatch_small<Small64>(kind, p, stream);

@@ -528,9 +528,12 @@ def test_gemm_of_tall_operands_walks_its_tiles_in_groups_of_rows(M, N, K, form):
     assert torch.isfinite(whole).all() and torch.equal(whole, parts)
 
 
-# 64 x 64 tiles, one work-group per unit (a ring of six stages; four for `tt`) and two (four stages): the ring never full, once full,
-# refilled in turn, with and without a partial last K tile ...
+# 32 x 64 tiles (a ring of five stages; 64 x 64 and four for `tt`) and 64 x 64 ones, two work-groups per unit (four stages): the ring never
+# full, once full, refilled in turn, with and without a partial last K tile ...
 _RING_SHAPES = [(70, 200, k) for k in (8, 64, 72, 128, 136, 192, 200, 256, 264, 320, 384, 392, 456, 840)] + [(1500, 1288, k) for k in (8, 64, 72, 136, 192, 264)]
+# ... the same for 64 x 64, one work-group per unit, and 64 x 128 (four stages each), with the last row count of a tile and the first of the next ...
+_RING_SHAPES += [(m, 1280, k) for m in (385, 1601) for k in (8, 64, 72, 128, 136, 192, 200, 256, 264, 320, 328, 384, 392)]
+_RING_SHAPES += [(m, 1280, 840) for m in (31, 32, 33, 384, 768, 769, 1600, 1638, 1665)]
 # ... and one work-group per unit: 128 x 128 up to 256 tiles, 192 x 128 from there to 256 tiles; 64 x 128 and 128 x 128 beyond them and for `tt`
 _RING_SHAPES += [(1700, 1280, 1288), (3200, 1280, 840), (3201, 1280, 840), (3277, 1280, 1280), (4800, 1280, 1288), (4801, 1280, 840)]
 
@@ -565,6 +568,33 @@ def test_gemm_of_few_rows_over_the_edges_of_its_ring_and_tiles(M, N, K, form, mo
     if K > 128:  # every tile gives the same bits
         monkeypatch.setenv("MVIT_GEMM_NO_HALF_TILES", "1")
         assert torch.equal(got, run())
+
+
+@pytest.mark.parametrize("K", [8, 64, 72, 128, 136, 192, 200, 256, 264, 320, 392, 1280])
+@pytest.mark.parametrize("M,N", [(1, 32), (63, 136), (256, 3456), (257, 3456), (300, 3424), (512, 3456), (513, 3456), (1100, 3456)])
+def test_gemm_swiglu_of_few_rows_over_the_edges_of_its_ring_and_tiles(M, N, K, monkeypatch):
+    """64 x 128 tiles in a ring of three stages up to 256 of them, 128 x 128 ones in a ring of four from there on, and the tiles beyond those."""
+    _announce(f"gemm swiglu ring {M}x{N}x{K}")
+    ops = _ops()
+    from mi355_vit import _lib as E
+
+    dtype = torch.bfloat16
+    a, w = _rand((M, K), dtype, 1).to(DEV), _rand((2 * N, K), dtype, 2, K**-0.5).to(DEV)
+    bias = _rand((2 * N,), dtype, 3).to(DEV)
+
+    def run():
+        h, gu = torch.full((M + 8, N), 7.0, dtype=dtype, device=DEV), torch.full((M + 8, 2 * N), 7.0, dtype=dtype, device=DEV)
+        ops.gemm(a, w[:N], h[:M], epilogue=E.EPI_SWIGLU, b2=w[N:], bias=bias[:N], bias2=bias[N:], aux=gu[:M], aux_off=N)
+        return h, gu
+
+    got = run()
+    assert bool((got[0][M:] == 7.0).all()) and bool((got[1][M:] == 7.0).all())
+    x = a.double() @ w.double().T + bias.double()
+    assert max_rel_err(got[1][:M], x.cpu()) < TOL[dtype]
+    assert max_rel_err(got[0][:M], (torch.nn.functional.silu(x[:, :N]) * x[:, N:]).cpu()) < TOL[dtype]
+    if K > 128:  # every tile gives the same bits
+        monkeypatch.setenv("MVIT_GEMM_NO_HALF_TILES", "1")
+        assert all(torch.equal(p, q) for p, q in zip(got, run()))
 
 
 @pytest.mark.parametrize("form", ["nn", "nt", "tt"])
