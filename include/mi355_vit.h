@@ -302,6 +302,10 @@ int mvit_image_token_ranks(const int64_t* input_ids, const int64_t* labels, int6
                            int64_t ignore_label, int32_t* rank, int64_t* positions, int64_t* counts,
                            mvit_stream_t stream);
 
+/* Host-only: waits until none of n values that a kernel writes to pinned host memory is negative, for timeout_us microseconds at
+ * most.  0: all are there; 1: not yet.  The caller sets them to -1 before the launch. */
+int mvit_wait_host_values(const int64_t* values, int n, int64_t timeout_us);
+
 /* merged[t, :] = rank[t] >= 0 ? vision[rank[t], :] : embeds[t, :] over rows of row_bytes bytes (bit-exact copy);
  * with vision == NULL the selected rows are zero-filled instead.  A rank >= n_vision keeps the embeds row.
  * Forward: inputs_embeds.masked_scatter(image_mask, vision_embeds_flat), python/ray/text.py:913.  Backward: the

@@ -3,6 +3,8 @@
 // accesses are 16-byte vectors along the contiguous dimension whenever shapes allow it.
 #include "mvit_common.h"
 
+#include <chrono>
+
 // ------------------------------------------------------------------------------------------------
 // RMSNorm forward.  One wave per row, 4 rows per 256-thread block; grid-stride over rows.
 // Algorithmic bytes per row: read cols*e, write cols*e (+ the weight once, + 4 B rstd).
@@ -925,6 +927,16 @@ int mvit_image_token_ranks(const int64_t* input_ids, const int64_t* labels, int6
   hipLaunchKernelGGL(image_token_ranks_kernel, dim3(1), 1024, 0, S_(stream), input_ids, labels, n_tokens, image_token_id, ignore_label,
                      rank, positions, counts);
   MVIT_CHECK_LAUNCH("image_token_ranks");
+  return MVIT_OK;
+}
+
+int mvit_wait_host_values(const int64_t* values, int n, int64_t timeout_us) {
+  MVIT_REQUIRE(values != nullptr && n > 0 && timeout_us >= 0, "wait_host_values: null pointer or bad count");
+  const auto end = std::chrono::steady_clock::now() + std::chrono::microseconds(timeout_us);
+  for (int i = 0; i < n;) {
+    if (__atomic_load_n(values + i, __ATOMIC_ACQUIRE) >= 0) ++i;
+    else if (std::chrono::steady_clock::now() >= end) return 1;
+  }
   return MVIT_OK;
 }
 

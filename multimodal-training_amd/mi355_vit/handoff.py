@@ -13,6 +13,7 @@ read-backs and ``masked_scatter``; the backward is one pass over the gradient.
 
 from __future__ import annotations
 
+import time
 from typing import Optional
 
 import torch
@@ -28,9 +29,32 @@ def _int64_row(t: torch.Tensor) -> torch.Tensor:
     return t if t.dtype == torch.int64 and t.is_contiguous() else t.to(torch.int64).contiguous()
 
 
+class _Arrival:
+    """Counts that a kernel writes to pinned host memory, -1 until then.  They are seen there as soon as they arrive, some 10 us before an
+    event behind the kernel would tell the host."""
+
+    __slots__ = ("counts", "device")
+
+    def __init__(self, counts: torch.Tensor, device: torch.device):
+        self.counts, self.device = counts, device
+
+    def _after(self, microseconds: int) -> bool:
+        return _lib.load().mvit_wait_host_values(self.counts.data_ptr(), self.counts.numel(), microseconds) == 0
+
+    def query(self) -> bool:
+        return self._after(0)
+
+    def synchronize(self) -> None:
+        if self._after(2000):  # without the interpreter's lock
+            return
+        stream = torch.cuda.current_stream(self.device)
+        while not self.query() and not stream.query():  # a stream that has failed raises here
+            time.sleep(1e-4)
+
+
 def _ranks(input_ids: torch.Tensor, labels: Optional[torch.Tensor], image_token_id: int):
-    """(rank of every token, pinned counts, event after which the host may read them).  The kernel writes the counts, and the
-    pinned allocator does not know of it: the caller holds them until the event has passed, on every way out."""
+    """(rank of every token, pinned counts, their arrival).  The pinned allocator does not know of the kernel that writes the
+    counts: the caller holds them until they have arrived, on every way out."""
     ids = _int64_row(input_ids)
     lab = None
     if labels is not None:
@@ -39,17 +63,11 @@ def _ranks(input_ids: torch.Tensor, labels: Optional[torch.Tensor], image_token_
         lab = _int64_row(labels)
     n = ids.numel()
     rank = torch.empty(n, dtype=torch.int32, device=ids.device)
-    counts = torch.empty(2, dtype=torch.int64, pin_memory=True)  # the kernel writes them where the host reads them
+    counts = torch.empty(2, dtype=torch.int64, pin_memory=True).fill_(-1)  # the kernel writes them where the host reads them
     rc = _lib.load().mvit_image_token_ranks(ids.data_ptr(), None if lab is None else lab.data_ptr(), n, image_token_id, -100,
                                             rank.data_ptr(), None, counts.data_ptr(), _stream(ids))
     _lib.check(rc, "mvit_image_token_ranks")
-    try:
-        ready = torch.cuda.Event()
-        ready.record(torch.cuda.current_stream(ids.device))
-    except BaseException:
-        torch.cuda.synchronize(ids.device)
-        raise
-    return rank, counts, ready
+    return rank, counts, _Arrival(counts, ids.device)
 
 
 class _MergeRowsFn(torch.autograd.Function):

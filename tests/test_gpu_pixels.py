@@ -93,6 +93,23 @@ def test_patchify_frames_at_an_odd_address():
     assert np.array_equal(got.cpu().numpy().view(np.uint32), ref.view(np.uint32))
 
 
+def test_patchify_of_more_merge_blocks_than_work_groups():
+    """Beyond 16,384 rows a work-group makes several merge blocks and requests the next one's pixels meanwhile: from a still image to a
+    video of an odd frame count and on to frames at an odd address."""
+    from mi355_vit.pixels import patchify
+
+    _announce("patchify 25,600 rows, mixed")
+    images = _batch(8, [(1, 1120, 1120), (5, 896, 896), (1, 1120, 1120), (1, 28, 28)])
+    frames = [torch.from_numpy(im).to(DEV) for im in images]
+    odd = torch.zeros(images[2].size + 1, dtype=torch.uint8, device=DEV)
+    odd[1:].copy_(frames[2].reshape(-1))
+    frames[2] = odd[1:].view(images[2].shape)
+    ref, _ = po.patchify_batch(images)
+    got, _ = patchify(frames)
+    assert ref.shape[0] > 16384 and np.array_equal(got.cpu().numpy().view(np.uint32), ref.view(np.uint32))
+    assert torch.equal(patchify(frames, dtype=torch.bfloat16)[0].cpu(), torch.from_numpy(ref).to(torch.bfloat16))
+
+
 def test_patchify_full_benchmark_batch():
     """The 8 ragged images of the benchmark workload (25,524 rows): bit-exact, and a still image fills both halves."""
     _announce("patchify cfg2 batch")
