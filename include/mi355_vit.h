@@ -458,6 +458,20 @@ int mvit_resample_u8_batch(const mvit_resample_job* jobs, int n_jobs, mvit_strea
 int mvit_resample_u8(const uint8_t* src, uint8_t* dst, int64_t outer, int64_t in_len, int64_t out_len, int64_t inner,
                      const int32_t* bounds, const int32_t* kk, int ksize, mvit_stream_t stream);
 
+/* The vertical pass and mvit_patchify in one launch, for still images of which the horizontal pass has been made: image i has src_height
+ * lines of `width` pixels at src and becomes height x width (multiples of 28), its rows from first_row on; bounds and kk are the
+ * vertical pass's tables on the device, both null where src_height == height.  The table (n_images + 1 entries, the last one's
+ * first_row the total) is in host memory, at most 64 images; MVIT_ERR_UNSUPPORTED for more, and for images shrunk so far that 28 lines
+ * need more than 128 or a window more than 32 of src (the caller then makes the passes one by one). */
+typedef struct mvit_resized_image {
+  const uint8_t* src;
+  const int32_t *bounds, *kk;
+  int32_t src_height, height, width, ksize;
+  int64_t first_row;
+} mvit_resized_image;
+int mvit_resize_patchify(const mvit_resized_image* images, int n_images, int64_t total_rows, void* out, double rescale, float mean_r,
+                         float mean_g, float mean_b, float std_r, float std_g, float std_b, int dtype, mvit_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -44,6 +44,44 @@ constexpr int SQ = 2 * PATCH;          // a merge block is a square of 28 x 28 p
 constexpr int SQ_LINE = SQ * 3;        // 84 bytes (21 dwords) per line of the square
 constexpr int SQ_DWORDS = SQ * SQ_LINE / 4;  // 588
 
+// The result for every byte value and channel, by the work-group (exact arithmetic, three divisions per thread)
+template <typename TO>
+__device__ __forceinline__ void make_lut(TO (&lut)[3][256], const Norm& nm) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const float x = (float)((double)(int)threadIdx.x * nm.rescale);
+    lut[c][threadIdx.x] = from_f32<TO>((x - nm.mean[c]) / nm.std[c]);
+  }
+}
+// A wave makes one patch of the square, a lane four consecutive values of each plane: two pairs of pixels, six bytes each at even
+// addresses, the second pair on the line below where the first ends one.
+struct PatchLane {
+  int q, pair0, pair1;
+};
+__device__ __forceinline__ PatchLane patch_lane() {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int q = lane < QUADS ? lane : 0, y = 4 * q / PATCH, x = 4 * q - y * PATCH;
+  const int origin = (wave >> 1) * PATCH * SQ_LINE + (wave & 1) * PATCH * 3, pair0 = origin + y * SQ_LINE + x * 3;
+  return {q, pair0, x + 2 < PATCH ? pair0 + 6 : origin + (y + 1) * SQ_LINE};
+}
+template <typename TO>
+__device__ __forceinline__ void look_up(const uint32_t* square, const TO (&lut)[3][256], const PatchLane& pl, TO (&v)[3][4]) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int at = h ? pl.pair1 : pl.pair0;
+    const uint32_t *w = &square[at >> 2], w0 = w[0], w1 = w[1], lo = __builtin_amdgcn_alignbyte(w1, w0, at & 2), hi = w1 >> (8 * (at & 2));
+    const uint32_t b[6] = {lo & 0xff, (lo >> 8) & 0xff, (lo >> 16) & 0xff, lo >> 24, hi & 0xff, (hi >> 8) & 0xff};
+#pragma unroll
+    for (int e = 0; e < 6; ++e) v[e % 3][2 * h + e / 3] = lut[e % 3][b[e]];
+  }
+}
+template <typename TO>
+__device__ __forceinline__ void store_patch(TO* row, int frame, const PatchLane& pl, const TO (&v)[3][4]) {
+#pragma unroll
+  for (int c = 0; c < 3; ++c) *reinterpret_cast<quad_t<TO>*>(row + (c * TPS + frame) * PLANE + 4 * pl.q) = quad_t<TO>{v[c][0], v[c][1], v[c][2], v[c][3]};
+}
+
 // The image table travels as a kernel argument when it is short (no copy to the device in front of the launch).
 constexpr int TABLE_ARG_IMAGES = 64;
 struct TableArg {
@@ -51,9 +89,8 @@ struct TableArg {
 };
 template <typename TO>
 __device__ __forceinline__ void patchify_blocks(const mvit_image* images, int n_images, TO* __restrict__ out, int64_t total_rows, const Norm& nm) {
-#pragma clang fp contract(off)
-  // a byte has 256 values: the work-group computes the result for each of them and each channel once (exact
-  // arithmetic, three divisions per thread) and every element of its rows is then a byte read and a table lookup
+  // a byte has 256 values: the work-group computes the result for each of them and each channel once, and every element of its rows
+  // is then a byte and a table lookup
   __shared__ TO lut[3][256];
   __shared__ __attribute__((aligned(16))) uint32_t square[TPS][SQ_DWORDS];  // the block's pixels, one copy per frame of the pair
   constexpr int LOADS = (TPS * SQ_DWORDS + 255) / 256;                       // dwords of the square per thread
@@ -111,17 +148,9 @@ __device__ __forceinline__ void patchify_blocks(const mvit_image* images, int n_
   if (row0 >= total_rows) return;
   Block now = locate(row0);
   request(now);
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    const float x = (float)((double)(int)threadIdx.x * nm.rescale);
-    lut[c][threadIdx.x] = from_f32<TO>((x - nm.mean[c]) / nm.std[c]);
-  }
-  // A lane makes four consecutive values of each plane: two pairs of pixels, six bytes each at even addresses, the second pair on the
-  // line below where the first ends one.
+  make_lut<TO>(lut, nm);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int q = lane < QUADS ? lane : 0, y = 4 * q / PATCH, x = 4 * q - y * PATCH;
-  const int origin = (wave >> 1) * PATCH * SQ_LINE + (wave & 1) * PATCH * 3;
-  const int pair0 = origin + y * SQ_LINE + x * 3, pair1 = x + 2 < PATCH ? pair0 + 6 : origin + (y + 1) * SQ_LINE;
+  const PatchLane pl = patch_lane();
   while (true) {
     __syncthreads();  // the previous block's pixels have been read
     if (now.corner != nullptr) put(now);
@@ -133,26 +162,12 @@ __device__ __forceinline__ void patchify_blocks(const mvit_image* images, int n_
       request(then);
     }
     if (now.corner != nullptr && lane < QUADS) {
-      TO* dst = out + (row0 + wave) * ROW + 4 * q;
+      TO* dst = out + (row0 + wave) * ROW;
       TO v[3][4];
-      auto look_up = [&](int frame) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int at = h ? pair1 : pair0;
-          const uint32_t *w = &square[frame][at >> 2], w0 = w[0], w1 = w[1], lo = __builtin_amdgcn_alignbyte(w1, w0, at & 2), hi = w1 >> (8 * (at & 2));
-          const uint32_t b[6] = {lo & 0xff, (lo >> 8) & 0xff, (lo >> 16) & 0xff, lo >> 24, hi & 0xff, (hi >> 8) & 0xff};
-#pragma unroll
-          for (int e = 0; e < 6; ++e) v[e % 3][2 * h + e / 3] = lut[e % 3][b[e]];
-        }
-      };
-      auto store = [&](int frame) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) *reinterpret_cast<quad_t<TO>*>(dst + (c * TPS + frame) * PLANE) = quad_t<TO>{v[c][0], v[c][1], v[c][2], v[c][3]};
-      };
-      look_up(0);
-      store(0);
-      if (now.two) look_up(1);
-      store(1);
+      look_up<TO>(&square[0][0], lut, pl, v);
+      store_patch<TO>(dst, 0, pl, v);
+      if (now.two) look_up<TO>(&square[1][0], lut, pl, v);
+      store_patch<TO>(dst, 1, pl, v);
     }
     if (next >= total_rows) return;
     row0 = next;
@@ -859,6 +874,93 @@ __global__ __launch_bounds__(256) void resample_wide_kernel(const ResampleJobs j
   __builtin_memcpy(jb.dst + ((int64_t)o * jb.out_len + x) * jb.inner + at, v, 16);
 }
 
+// The vertical pass and patchify in one: a work-group resamples the 28 x 28 square of its merge block into LDS, so the resized image is
+// never written and one launch goes.  The rows that the square's windows span are staged as dwords, the weights beside them; a lane
+// makes twelve bytes of a line (seven lanes a line, 196 of 256).  Rows or taps beyond what LDS is laid out for are the caller's to pass
+// separately; windows that no resampling table has are read tap by tap.  The arithmetic is resample_wide_kernel's.
+// Bound by vector issue (two instructions per byte and tap) beside patchify's writes, with eight work-groups to a unit to cover the loads.  us of the
+// whole input side in bf16, vertical pass and patchify one after the other / this: to 0.8 million pixels 427 x 640 19.8 / 15.4, 1,080 x 1,920 26.7 / 23.0,
+// 2,448 x 3,264 30.3 / 29.6, these and 800 x 1,333 together 47.2 / 44.5, eight of 240 x 320 58.5 / 45.5; 4,480 x 4,480 to 3,584 x 3,584 130 / 99
+// (104 with six work-groups to a unit).
+constexpr int FUSED_ROWS = 128, FUSED_TAPS = 32, FUSED_GROUPS = 2048;
+struct ResizedTable {
+  mvit_resized_image im[TABLE_ARG_IMAGES + 1];
+};
+template <typename TO>
+__global__ __launch_bounds__(256, 8) void resize_patchify_kernel(const ResizedTable images, int n_images, TO* __restrict__ out, int64_t total_rows, Norm nm) {
+  __shared__ TO lut[3][256];
+  __shared__ __attribute__((aligned(16))) uint32_t square[SQ_DWORDS], staged[FUSED_ROWS * SQ_DWORDS / SQ];
+  __shared__ int32_t weights[SQ * FUSED_TAPS];
+  constexpr int LINE = SQ_LINE / 4, BYTES = 12, LANES = SQ_LINE / BYTES;  // dwords, bytes of a lane, lanes of a line
+  make_lut<TO>(lut, nm);
+  const PatchLane pl = patch_lane();
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int64_t row0 = (int64_t)blockIdx.x * 4; row0 < total_rows; row0 += (int64_t)gridDim.x * 4) {
+    int lo = 0, hi = n_images;  // invariant: im[lo].first_row <= row0 < im[hi].first_row
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (images.im[mid].first_row <= row0) lo = mid;
+      else hi = mid;
+    }
+    const mvit_resized_image& im = images.im[lo];
+    const int gw = im.width / PATCH, blocks_across = gw >> 1;
+    const int blk = (int)((row0 - im.first_row) >> 2), hb = blk / blocks_across, wb = blk % blocks_across;
+    const int64_t line = (int64_t)im.width * 3;
+    const uint8_t* corner = im.src + wb * SQ_LINE;
+    const int y0 = hb * SQ, ksize = im.ksize;
+    auto dword = [](const uint8_t* p) {
+      uint32_t w;
+      __builtin_memcpy(&w, p, 4);
+      return w;
+    };
+    __syncthreads();  // the previous square has been read
+    if (im.bounds == nullptr) {  // as high as it has to be
+      for (int i = threadIdx.x; i < SQ_DWORDS; i += 256) square[i] = dword(corner + (y0 + i / LINE) * line + i % LINE * 4);
+    } else {
+      const TapWindow head = tap_window(im.bounds, y0, ksize, im.src_height), tail = tap_window(im.bounds, y0 + SQ - 1, ksize, im.src_height);
+      const int first = head.xmin, rows = max(0, min(tail.xmin + tail.n - first, FUSED_ROWS));
+      for (int i = threadIdx.x; i < rows * LINE; i += 256) staged[i] = dword(corner + (first + i / LINE) * line + i % LINE * 4);
+      for (int i = threadIdx.x; i < SQ * ksize; i += 256) weights[i] = im.kk[(int64_t)y0 * ksize + i];
+      __syncthreads();
+      if ((int)threadIdx.x < SQ * LANES) {
+        const int y = threadIdx.x / LANES, c = threadIdx.x % LANES;
+        const TapWindow tw = tap_window(im.bounds, y0 + y, ksize, im.src_height);
+        const int32_t* k = weights + y * ksize;
+        const int from = tw.xmin - first;
+        bool usual = from >= 0 && from + tw.n <= rows;
+        for (int t = 0; t < tw.n; ++t) usual = usual && fits24(k[t]);
+        int a[BYTES];
+#pragma unroll
+        for (int e = 0; e < BYTES; ++e) a[e] = 1 << (RESAMPLE_PRECISION_BITS - 1);
+        if (usual) {
+          const uint32_t* w = staged + from * LINE + c * 3;
+#pragma unroll 1
+          for (int t = 0; t < tw.n; ++t)
+#pragma unroll
+            for (int e = 0; e < BYTES; ++e) a[e] = tap<true>(a[e], (w[t * LINE + (e >> 2)] >> (8 * (e & 3))) & 0xffu, k[t]);
+        } else {
+          const uint8_t* p = corner + tw.xmin * line + c * BYTES;
+#pragma unroll 1
+          for (int t = 0; t < tw.n; ++t)
+#pragma unroll
+            for (int e = 0; e < BYTES; ++e) a[e] = tap<false>(a[e], p[t * line + e], k[t]);
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          square[y * LINE + c * 3 + i] = clip8(a[4 * i]) | (clip8(a[4 * i + 1]) << 8) | (clip8(a[4 * i + 2]) << 16) | (clip8(a[4 * i + 3]) << 24);
+      }
+    }
+    __syncthreads();  // the square and the table are complete
+    if (lane < QUADS) {
+      TO* dst = out + (row0 + wave) * ROW;
+      TO v[3][4];
+      look_up<TO>(square, lut, pl, v);
+      store_patch<TO>(dst, 0, pl, v);
+      store_patch<TO>(dst, 1, pl, v);
+    }
+  }
+}
+
 extern "C" {
 
 int mvit_patchify(const mvit_image* images, int n_images, int64_t total_rows, void* out, double rescale, float mean_r,
@@ -878,6 +980,39 @@ int mvit_patchify(const mvit_image* images, int n_images, int64_t total_rows, vo
   else
     hipLaunchKernelGGL((patchify_kernel<float>), dim3(grid), 256, 0, s, images, n_images, static_cast<float*>(out), total_rows, nm);
   MVIT_CHECK_LAUNCH("patchify");
+  return MVIT_OK;
+}
+
+int mvit_resize_patchify(const mvit_resized_image* images, int n_images, int64_t total_rows, void* out, double rescale, float mean_r,
+                         float mean_g, float mean_b, float std_r, float std_g, float std_b, int dtype, mvit_stream_t stream) {
+  MVIT_REQUIRE(images != nullptr && n_images > 0, "resize_patchify: empty image table");
+  if (n_images > TABLE_ARG_IMAGES) return mvit_set_error(MVIT_ERR_UNSUPPORTED, "resize_patchify: %d images; the table holds at most %d", n_images, TABLE_ARG_IMAGES);
+  MVIT_REQUIRE(dtype == MVIT_BF16 || dtype == MVIT_F32, "resize_patchify: dtype %d", dtype);
+  MVIT_REQUIRE(std_r != 0.f && std_g != 0.f && std_b != 0.f, "resize_patchify: zero std");
+  int64_t rows = 0;
+  for (int i = 0; i < n_images; ++i) {
+    const mvit_resized_image& im = images[i];
+    MVIT_REQUIRE(im.src && im.height > 0 && im.width > 0 && im.height % SQ == 0 && im.width % SQ == 0 && im.src_height > 0 && im.first_row == rows,
+                 "resize_patchify: image %d, %d x %d from %d lines, first row %lld", i, im.height, im.width, im.src_height, (long long)im.first_row);
+    MVIT_REQUIRE((im.bounds == nullptr) == (im.kk == nullptr) && (im.bounds ? im.ksize > 0 : im.src_height == im.height), "resize_patchify: image %d: tables", i);
+    rows += (int64_t)(im.height / PATCH) * (im.width / PATCH);
+    // lines that the windows of 28 output lines span at most, as any resampling between these heights has them
+    if (im.bounds && (im.ksize > FUSED_TAPS || ((int64_t)SQ * im.src_height + im.height - 1) / im.height + 1 + im.ksize > FUSED_ROWS))
+      return mvit_set_error(MVIT_ERR_UNSUPPORTED, "resize_patchify: image %d: %d lines from %d are passes of their own", i, im.height, im.src_height);
+  }
+  MVIT_REQUIRE(images[n_images].first_row == rows && total_rows == rows && rows / 4 <= 0x7fffffffLL, "resize_patchify: total_rows %lld", (long long)total_rows);
+  MVIT_REQUIRE(out != nullptr && mvit_aligned16(out), "resize_patchify: output must be a 16-byte aligned device pointer");
+  ResizedTable table;
+  memset(&table, 0, sizeof(table));
+  memcpy(table.im, images, sizeof(mvit_resized_image) * ((size_t)n_images + 1));
+  Norm nm{rescale, {mean_r, mean_g, mean_b}, {std_r, std_g, std_b}};
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const unsigned grid = (unsigned)(rows / 4 < FUSED_GROUPS ? rows / 4 : FUSED_GROUPS);
+  if (dtype == MVIT_BF16)
+    hipLaunchKernelGGL((resize_patchify_kernel<bf16_t>), dim3(grid), 256, 0, s, table, n_images, static_cast<bf16_t*>(out), rows, nm);
+  else
+    hipLaunchKernelGGL((resize_patchify_kernel<float>), dim3(grid), 256, 0, s, table, n_images, static_cast<float*>(out), rows, nm);
+  MVIT_CHECK_LAUNCH("resize_patchify");
   return MVIT_OK;
 }
 

@@ -104,6 +104,7 @@ PROTOTYPES = {
     "mvit_grad_sumsq_static": [_vp, _i32, _i64, _vp, _i32, _vp],
     "mvit_patchify": [_vp, _i32, _i64, _vp, C.c_double] + [_f32] * 6 + [_i32, _vp],
     "mvit_patchify_host_table": [_vp, _i32, _i64, _vp, C.c_double] + [_f32] * 6 + [_i32, _vp],
+    "mvit_resize_patchify": [_vp, _i32, _i64, _vp, C.c_double] + [_f32] * 6 + [_i32, _vp],
     "mvit_resample_u8_batch": [_vp, _i32, _vp],
     "mvit_resample_u8": [_vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _i32, _vp],
     "mvit_patch_embed_pack_weight": [_vp, _i32, _i64, _i64, _vp, _vp],

@@ -98,16 +98,18 @@ def _dtype_code(dtype: torch.dtype) -> int:
     raise TypeError(f"unsupported dtype {dtype} (float32 and bfloat16 only)")
 
 
-def _patchify_table(table: bytes, n: int, total: int, out: torch.Tensor, code: int, image_mean, image_std, rescale_factor) -> None:
+def _norm(image_mean, image_std, rescale_factor) -> tuple:
+    return (float(rescale_factor), *(float(np.float32(v)) for v in image_mean), *(float(np.float32(v)) for v in image_std))
+
+
+def _patchify_table(table: bytes, n: int, total: int, out: torch.Tensor, code: int, norm: tuple) -> None:
     """The launch, on the current device."""
-    mean = [float(np.float32(m)) for m in image_mean]
-    std = [float(np.float32(s)) for s in image_std]
     lib, stream = _lib.load(), _stream(out)
     if n <= _HOST_TABLE_IMAGES:
-        rc = lib.mvit_patchify_host_table(table, n, total, out.data_ptr(), float(rescale_factor), *mean, *std, code, stream)
+        rc = lib.mvit_patchify_host_table(table, n, total, out.data_ptr(), *norm, code, stream)
     else:
         dev_table = _on_device(table, out.device)
-        rc = lib.mvit_patchify(dev_table.data_ptr(), n, total, out.data_ptr(), float(rescale_factor), *mean, *std, code, stream)
+        rc = lib.mvit_patchify(dev_table.data_ptr(), n, total, out.data_ptr(), *norm, code, stream)
     _lib.check(rc, "mvit_patchify")
 
 
@@ -127,7 +129,7 @@ def patchify(frames: Sequence[torch.Tensor], dtype: torch.dtype = torch.float32,
     elif out.shape != (total, _lib.PIXEL_ROW) or out.dtype != dtype or out.device != device or not out.is_contiguous():
         raise RuntimeError(f"patchify: out must be a contiguous {dtype} [{total}, {_lib.PIXEL_ROW}] tensor on {device}")
     with torch.cuda.device(device):
-        _patchify_table(table, n, total, out, code, image_mean, image_std, rescale_factor)
+        _patchify_table(table, n, total, out, code, _norm(image_mean, image_std, rescale_factor))
     return out, grid
 
 
@@ -264,6 +266,7 @@ def _check_resizable(frames: torch.Tensor) -> None:
         raise RuntimeError("resize_frames: frames must be contiguous")
 
 
+_RESIZED_FORMAT = "3Q4iq"  # mvit_resized_image: src, bounds, kk, src_height, height, width, ksize, first_row
 _JOB_FORMAT = "8q2i"  # mvit_resample_job: src, dst, bounds, kk, outer, in_len, out_len, inner, ksize, reserved
 
 
@@ -313,8 +316,8 @@ def preprocess(images: Sequence[torch.Tensor], dtype: torch.dtype = torch.float3
     """Decoded still images (uint8 GPU tensors ``[1, height, width, 3]`` of any size) -> (``pixel_values``,
     ``image_grid_thw``): the image processor's smart_resize + resize + rescale + normalise + patchify, on the GPU.
 
-    The horizontal passes of all images are one launch, the vertical ones another, and the images in between share one allocation:
-    the host would take longer than the GPU with a tensor for each (four photographs 69 us of host time, now 41)."""
+    The horizontal passes of all images are one launch, the vertical ones and patchify another, and the images in between share one
+    allocation: the host would take longer than the GPU with a tensor for each (four photographs 69 us of host time, now 40)."""
     images, plans = list(images), []  # per image: height, width, resized height and width
     for i, f in enumerate(images):
         if f.dim() != 4 or f.shape[0] != 1 or f.shape[3] != 3:
@@ -327,31 +330,51 @@ def preprocess(images: Sequence[torch.Tensor], dtype: torch.dtype = torch.float3
     if not images:
         raise ValueError("patchify: no images")
     code, device = _dtype_code(dtype), images[0].device
-    index, ch, size = device.index or 0, 3, 0
-    places = []  # of an image after each pass that changes it
-    for h, w, oh, ow in plans:
-        a = size
+    index, ch, size, places = device.index or 0, 3, 0, []
+    for h, w, oh, ow in plans:  # places of the images as wide as they have to be
+        places.append(size)
         size += -(-h * ow * ch // 256) * 256 if w != ow else 0
-        places.append((a, size))
-        size += -(-oh * ow * ch // 256) * 256 if h != oh else 0
     between = torch.empty(size, dtype=torch.uint8, device=device)  # lives until the last launch is queued
-    base, across, down, held, rows, grid, total = between.data_ptr(), [], [], [], [], [], 0
-    for f, (h, w, oh, ow), (a, d) in zip(images, plans, places):
+    base, across, held, rows, grid, total = between.data_ptr(), [], [], [], [], 0
+    for f, (h, w, oh, ow), place in zip(images, plans, places):
         at = f.data_ptr()
         if w != ow:
-            across.append(_across_job(at, base + a, 1, h, w, ow, ch, resample, index, held))
-            at = base + a
+            across.append(_across_job(at, base + place, 1, h, w, ow, ch, resample, index, held))
+            at = base + place
+        bounds, kk, ksize = 0, 0, 0
         if h != oh:
-            down.append(_down_job(at, base + d, 1, h, oh, ow, ch, resample, index, held))
-            at = base + d
-        rows.append((at, 1, oh, ow, 0, total))
+            job = _down_job(at, 0, 1, h, oh, ow, ch, resample, index, held)
+            bounds, kk, ksize = job[2], job[3], job[8]
+        rows.append((at, bounds, kk, h, oh, ow, ksize, total))
         grid.append((1, oh // PATCH_SIZE, ow // PATCH_SIZE))
         total += (oh // PATCH_SIZE) * (ow // PATCH_SIZE)
-    rows.append((0, 0, 0, 0, 0, total))
+    rows.append((0, 0, 0, 0, 0, 0, 0, total))
     out = torch.empty((total, _lib.PIXEL_ROW), dtype=dtype, device=device)
+    norm = _norm(OPENAI_CLIP_MEAN, OPENAI_CLIP_STD, 1.0 / 255.0)
     with torch.cuda.device(device):
         stream = _stream(out)
         _resample_passes(across, stream)
-        _resample_passes(down, stream)
-        _patchify_table(_packed(_IMAGE_FORMAT, rows), len(images), total, out, code, OPENAI_CLIP_MEAN, OPENAI_CLIP_STD, 1.0 / 255.0)
+        try:
+            _lib.check(_lib.load().mvit_resize_patchify(_packed(_RESIZED_FORMAT, rows), len(images), total, out.data_ptr(), *norm, code, stream),
+                       "mvit_resize_patchify")
+        except _lib.Unsupported:  # many images, or one made a quarter as high and less
+            _resize_down_and_patchify(rows, out, code, norm, stream, device)
     return out, torch.tensor(grid, dtype=torch.int64)
+
+
+def _resize_down_and_patchify(rows: list, out: torch.Tensor, code: int, norm: tuple, stream: int, device: torch.device) -> None:
+    """The vertical passes in one launch and patchify in another, for the table of ``mvit_resize_patchify``."""
+    ch, size, places = 3, 0, []
+    for _, bounds, _, _, oh, ow, _, _ in rows[:-1]:
+        places.append(size)
+        size += -(-oh * ow * ch // 256) * 256 if bounds else 0
+    resized = torch.empty(size, dtype=torch.uint8, device=device)
+    down, images = [], []
+    for (at, bounds, kk, h, oh, ow, ksize, first), place in zip(rows, places):
+        if bounds:
+            down.append((at, resized.data_ptr() + place, bounds, kk, 1, h, oh, ow * ch, ksize, 0))
+            at = resized.data_ptr() + place
+        images.append((at, 1, oh, ow, 0, first))
+    images.append((0, 0, 0, 0, 0, rows[-1][-1]))
+    _resample_passes(down, stream)
+    _patchify_table(_packed(_IMAGE_FORMAT, images), len(images) - 1, rows[-1][-1], out, code, norm)

@@ -554,3 +554,66 @@ def test_resample_of_more_work_groups_than_a_launch_takes(outer, inner):
                                       torch.cuda.current_stream().cuda_stream)
     _lib.check(rc, "mvit_resample_u8")
     assert torch.equal(src, dst)
+
+
+def _resized_then_patchified(images, sizes, dtype):
+    from mi355_vit import pixels as P
+
+    return P.patchify([P.resize_frames(im, oh, ow) for im, (oh, ow) in zip(images, sizes)], dtype=dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("pixels,sizes", [
+    (28 * 28 * 64, [(200, 333), (224, 224), (900, 140), (61, 61), (224, 500), (500, 224)]),  # smaller, unchanged, taller, larger, one axis alone
+    (28 * 28 * 16, [(430, 430), (436, 436), (441, 439), (500, 470)]),                        # shrunk 3.8 to 4.2-fold: on both sides of the line
+    (28 * 28 * 4, [(333, 57), (30, 31)] * 33),                                                # more images than a table holds
+    (28 * 28 * 6000, [(1500, 2801), (2200, 2200)]),                                           # more merge blocks than work-groups
+])
+def test_preprocess_resamples_vertically_inside_patchify(pixels, sizes, dtype):
+    """The vertical pass inside patchify gives the bits of the passes one by one, whatever the ratio, also where it is not taken."""
+    from mi355_vit import pixels as P
+
+    _announce(f"preprocess {len(sizes)} images to {pixels} pixels {dtype}")
+    rng = np.random.default_rng(len(sizes))
+    images = [torch.from_numpy(rng.integers(0, 256, size=(1, h, w, 3), dtype=np.uint8)).to(DEV) for h, w in sizes]
+    images[0] = torch.where(images[0] > 127, 255, 0).to(torch.uint8)  # overshoots at every edge are clamped
+    odd = torch.zeros(images[1].numel() + 3, dtype=torch.uint8, device=DEV)
+    images[1] = odd[3:].copy_(images[1].reshape(-1)).view(images[1].shape)  # at an odd address
+    got, grid = P.preprocess(images, dtype=dtype, min_pixels=pixels, max_pixels=pixels)
+    targets = [P.smart_resize(h, w, min_pixels=pixels, max_pixels=pixels) for h, w in sizes]
+    want, want_grid = _resized_then_patchified(images, targets, dtype)
+    assert grid.tolist() == want_grid.tolist() and got.dtype == dtype
+    assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+
+
+@pytest.mark.parametrize("kind", ["windows out of order", "weights of more than 24 bits"])
+def test_resize_patchify_with_tables_that_no_resampling_has(kind):
+    """Tables within the entry point's contract that the staging is not laid out for: the same bytes as the vertical pass alone."""
+    import struct
+
+    from mi355_vit import _lib
+    from mi355_vit import pixels as P
+
+    _announce(f"resize + patchify, {kind}")
+    rng = np.random.default_rng(3)
+    h, oh, ow, ksize = 301, 84, 56, 9
+    src = torch.from_numpy(rng.integers(0, 256, size=(1, h, ow, 3), dtype=np.uint8)).to(DEV)
+    starts = rng.integers(0, h - ksize, size=oh) if "order" in kind else np.linspace(0, h - ksize, oh).astype(np.int64)
+    bounds = torch.from_numpy(np.stack([starts, rng.integers(0, ksize + 1, size=oh)], 1).astype(np.int32)).to(DEV)
+    weights = rng.integers(-(1 << 21), 1 << 22, size=(oh, ksize))
+    if "bits" in kind:
+        weights[::5] *= 16
+    kk = torch.from_numpy(weights.astype(np.int32)).to(DEV)
+    resized = torch.empty(1, oh, ow, 3, dtype=torch.uint8, device=DEV)
+    stream = torch.cuda.current_stream().cuda_stream
+    P._resample_passes([(src.data_ptr(), resized.data_ptr(), bounds.data_ptr(), kk.data_ptr(), 1, h, oh, ow * 3, ksize, 0)], stream)
+    want, _ = P.patchify([resized])
+    out = torch.full_like(want, float("nan"))
+    total = out.shape[0]
+    table = struct.pack("<3Q4iq3Q4iq", src.data_ptr(), bounds.data_ptr(), kk.data_ptr(), h, oh, ow, ksize, 0, 0, 0, 0, 0, 0, 0, 0, total)
+    rc = _lib.load().mvit_resize_patchify(table, 1, total, out.data_ptr(), *P._norm(P.OPENAI_CLIP_MEAN, P.OPENAI_CLIP_STD, 1 / 255), _lib.F32, stream)
+    _lib.check(rc, "mvit_resize_patchify")
+    assert torch.equal(out, want)
+    with pytest.raises(RuntimeError, match="first row"):
+        _lib.check(_lib.load().mvit_resize_patchify(struct.pack("<3Q4iq3Q4iq", src.data_ptr(), 0, 0, oh, oh, ow, 0, 4, 0, 0, 0, 0, 0, 0, 0, total), 1, total,
+                                                    out.data_ptr(), *P._norm(P.OPENAI_CLIP_MEAN, P.OPENAI_CLIP_STD, 1 / 255), _lib.F32, stream), "mvit_resize_patchify")
