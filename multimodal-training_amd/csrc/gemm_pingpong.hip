@@ -310,6 +310,7 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
   issue_first();
   pp_wait_vm<0>();
   if (wm == 1) pp_barrier();  // group 1 runs one barrier behind
+  pp_barrier();
   while (true) {
     const int64_t m0 = next_m0, n0 = next_n0;
     const int slice = next_slice, bias_now = bias_buf;
@@ -320,8 +321,7 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
       rs[0] = rs[1] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     pp_wait_vm<(8 + TRAILING < 63 ? 8 + TRAILING : 63)>();
-    pp_barrier();
-    pp_barrier();
+    pp_barrier();  // group 1's loads have landed as well: it waited for them before the barrier that meets this one
     auto ktiles = [&](auto RS) {
       ktile(X1{}, 0, RS);
       for (int t = 1; t < n_kt - 2; ++t) ktile(X0{}, t, RS);
@@ -333,6 +333,11 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
     idx += gridDim.x >> 3;
     const bool have = start_tile(idx);
     if (have && !HAS_IN) issue_first();
+    // Group 0 meets the end of group 1's MFMAs here, not behind its own epilogue, so that both groups' epilogues run side by side (SwiGLU
+    // backward: after its first half, whose sums group 1 goes on from).  One behind the other -> now, us at 25,524 rows: SwiGLU 399 -> 397, its
+    // backward 337 -> 333, 1280 x 1280 with residual 80.0 -> 77.4, input gradients within 1 %; the clock takes back most of what the units gain.
+    // Steps 0.3 to 0.5 % shorter: 4,096 rows checkpointed, 14,336, 25,524 and 65,536 (paired passes, +- 0.1 %).
+    if (!SW_BWD && wm == 0) pp_barrier();
 
     // ---- epilogue: row block a of 16, half g: lane owns row l % 16 and the eight columns 8 * (l / 16) ..
     const bool to_ws = (EPI == MVIT_EPI_NONE) && p.split_k > 1;
@@ -356,8 +361,8 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
     // a = 0 .. 3, i.e. group 1 goes on from group 0's sums, and the sums of the sixteen lanes are added one after the other.
     float no_cs[16];
     const bool do_cs = SW_BWD && p.colsum != nullptr;
-    // Group 1's epilogue lies behind the barrier that group 0 arrives at after its own, so it finds group 0's sums there.  Chunks of
-    // four sums, chunk c of lane i in slot c ^ i: stores of sixteen lanes, and loads of one chunk of each, fall on all banks.
+    // A half of group 1's epilogue lies behind a barrier that group 0 arrives at after the same half of its own, so it finds group 0's sums
+    // there.  Chunks of four sums, chunk c of lane i in slot c ^ i: stores of sixteen lanes, and loads of one chunk of each, fall on all banks.
     float* cs_lds = reinterpret_cast<float*>(smem_raw + PpCfg::BIAS_OFF) + wn * 2048;
     auto chunk_of = [&](int g, int h) { return reinterpret_cast<f32x4*>(cs_lds + g * 1024 + i16 * 64 + ((g4 * 4 + h) ^ i16) * 4); };
     auto begin_sums = [&](int g) {
@@ -442,6 +447,7 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
           emit8_impl<T, TO, EPI, true, true>(p, row_of(it), n_lane[half_of(it)], v, u, now, no_cs, do_cs, HAS_BIAS ? hb[half_of(it)] : nullptr, nullptr);
           if (do_cs && (it & 7) == 7) end_sums(it >> 3);
           __builtin_amdgcn_sched_barrier(0);
+          if (SW_BWD && it == 7) pp_barrier();
         }
       } else {
 #pragma unroll
@@ -457,6 +463,7 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
 #pragma unroll
       for (int it = 0; it < ITEMS; ++it) {
         if (do_cs && it == 8) end_sums(0);
+        if (SW_BWD && it == 8) pp_barrier();
         if ((it & 7) == 0) begin_sums(it >> 3);
         float v[8], u[8];
         values(it, v, u);
@@ -476,9 +483,13 @@ __global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmP
       if (do_cs) end_sums(NG - 1);
       pp_wait_vm<0>();  // the count of this path's memory instructions is not known to the waits of the next tile
     }
+    if (SW_BWD && wm == 0) pp_barrier();
     if (!have) break;
+    if (wm == 1) {  // its share of the next tile's first half tiles, for group 0
+      pp_wait_vm<(8 + TRAILING < 63 ? 8 + TRAILING : 63)>();
+      pp_barrier();
+    }
   }
-  if (wm == 0) pp_barrier();
 }
 
 }  // namespace
