@@ -193,7 +193,11 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const T* __restrict__ 
 // weight gradient stays in registers.  Bound by HBM from some thousand rows on; us for 1280 columns with dx_add, before (two passes over the row,
 // the weight gradient in LDS) / now: 1,024 rows 7.0 / 5.4, 4,096 14.4 / 13.6, 14,336 34.3 / 30.5, 25,524 55.1 / 52.3, 65,536 130 / 130; with the next row's
 // loads under way as well 5.7 / 14.2 / 30.3 / 51.4 / 129, in twice the registers.
-template <typename T, int NCH, bool ADD>
+// ONCE: the two operands that nothing reads after this pass, dy and x, go past the caches where each is ONCE_BYTES and more, and leave them to what the
+// next launches read.  ms per step with / without, paired passes: 14,336 rows -0.29 (0.44 %), 25,524 -0.11, 16,384 checkpointed -0.2; at 4,096 rows, where they are
+// in the caches, +0.05.
+constexpr int64_t ONCE_BYTES = 24ll << 20;
+template <typename T, int NCH, bool ADD, bool ONCE>
 __global__ __launch_bounds__(256) void rmsnorm_bwd_row_kernel(const T* __restrict__ dy, const T* __restrict__ x, const T* __restrict__ w,
                                                               const float* __restrict__ rstd, const T* dx_add, T* dx,
                                                               float* __restrict__ dw_partial, int64_t rows, int cols) {
@@ -219,8 +223,8 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_row_kernel(const T* __restric
     for (int i = 0; i < NCH; ++i) {
       const int64_t at = r * cols + (i * 64 + lane) * V;
       if (mine(i)) {
-        to.x[i] = *reinterpret_cast<const vec_t*>(x + at);
-        to.g[i] = *reinterpret_cast<const vec_t*>(dy + at);
+        to.x[i] = ONCE ? load_once(reinterpret_cast<const vec_t*>(x + at)) : *reinterpret_cast<const vec_t*>(x + at);
+        to.g[i] = ONCE ? load_once(reinterpret_cast<const vec_t*>(dy + at)) : *reinterpret_cast<const vec_t*>(dy + at);
         if (ADD) to.a[i] = *reinterpret_cast<const vec_t*>(dx_add + at);
       }
     }
@@ -699,14 +703,14 @@ static auto rms_fwd_row(int64_t cols) -> decltype(&rmsnorm_fwd_row_kernel<T, 1>)
     default: return nullptr;
   }
 }
-template <typename T, bool ADD>
-static auto rms_bwd_row(int64_t cols) -> decltype(&rmsnorm_bwd_row_kernel<T, 1, ADD>) {
+template <typename T, bool ADD, bool ONCE>
+static auto rms_bwd_row(int64_t cols) -> decltype(&rmsnorm_bwd_row_kernel<T, 1, ADD, ONCE>) {
   switch ((cols + 64 * mvit_elem<T>::vec - 1) / (64 * mvit_elem<T>::vec)) {
-    case 1: return rmsnorm_bwd_row_kernel<T, 1, ADD>;
-    case 2: return rmsnorm_bwd_row_kernel<T, 2, ADD>;
-    case 3: return rmsnorm_bwd_row_kernel<T, 3, ADD>;
-    case 4: return rmsnorm_bwd_row_kernel<T, 4, ADD>;
-    case 5: return rmsnorm_bwd_row_kernel<T, 5, ADD>;
+    case 1: return rmsnorm_bwd_row_kernel<T, 1, ADD, ONCE>;
+    case 2: return rmsnorm_bwd_row_kernel<T, 2, ADD, ONCE>;
+    case 3: return rmsnorm_bwd_row_kernel<T, 3, ADD, ONCE>;
+    case 4: return rmsnorm_bwd_row_kernel<T, 4, ADD, ONCE>;
+    case 5: return rmsnorm_bwd_row_kernel<T, 5, ADD, ONCE>;
     default: return nullptr;
   }
 }
@@ -766,7 +770,8 @@ int mvit_rmsnorm_bwd(const void* dy, const void* x, const void* w, const float* 
   auto go = [&](auto zero) -> void {
     using T = decltype(zero);
     const bool vec = cols % mvit_elem<T>::vec == 0 && al;
-    auto kern = dx_add ? rms_bwd_row<T, true>(cols) : rms_bwd_row<T, false>(cols);
+    const bool once = rows * cols * (int64_t)sizeof(T) >= ONCE_BYTES;
+    auto kern = !dx_add ? rms_bwd_row<T, false, false>(cols) : once ? rms_bwd_row<T, true, true>(cols) : rms_bwd_row<T, true, false>(cols);
     if (!vec) kern = rmsnorm_bwd_kernel<T, false>;
     else if (kern == nullptr) kern = rmsnorm_bwd_kernel<T, true>;
     hipLaunchKernelGGL(kern, grid, 256, lds, S_(stream), (const T*)dy, (const T*)x, (const T*)w, rstd, (const T*)dx_add, (T*)dx, dw_partial, rows, (int)cols);

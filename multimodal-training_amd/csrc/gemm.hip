@@ -937,7 +937,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemm_dl_kernel(const GemmPara
 
 // C[m, n] = epilogue(sum over slices of the fp32 partial tiles) (fixed order, so the result is reproducible); the
 // epilogue is none, + bias[n] or + bias[n] + R[m, n], in the order of the one-pass kernels' epilogue.
-// VEC: four consecutive columns per thread (N, the pitches and the pointers allow vector accesses).
+// VEC: four consecutive columns per thread (N, the pitches and the pointers allow vector accesses).  The partial tiles are not read again.
 template <typename T, typename TO, bool VEC>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ ws, int split_k, int64_t M, int64_t N,
                                                             TO* __restrict__ C, int64_t ldc, int epi, const T* __restrict__ bias,
@@ -955,7 +955,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < quads; i += (int64_t)gridDim.x * 256) {
       f32x4 s = {0.f, 0.f, 0.f, 0.f};  // the same sum, from the same zero, as the scalar form
       for (int k = 0; k < split_k; ++k) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(ws + (int64_t)k * total + 4 * i);
+        const f32x4 v = load_once(reinterpret_cast<const f32x4*>(ws + (int64_t)k * total + 4 * i));
         s = f32x4{s[0] + v[0], s[1] + v[1], s[2] + v[2], s[3] + v[3]};
       }
       const int64_t m = i / nq, n = (i % nq) * 4;

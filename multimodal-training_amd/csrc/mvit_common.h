@@ -89,6 +89,12 @@ __device__ __forceinline__ bf16_t from_f32<bf16_t>(float v) {
   return (bf16_t)v;  // round-to-nearest-even
 }
 
+// A vector that is not read again before it has left the caches anyway: it does not push out what is
+template <typename V>
+__device__ __forceinline__ V load_once(const V* p) {
+  return __builtin_nontemporal_load(p);
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

@@ -1,5 +1,6 @@
 // Multi-tensor Adam step and gradient sum of squares for gfx950: one launch over every parameter tensor
-// instead of several launches (and one host read-back) per tensor.  Both kernels are HBM-bound streams.
+// instead of several launches (and one host read-back) per tensor.  Both kernels are HBM-bound streams, of gigabytes that are not
+// read again before the next step: non-temporal loads, and stores of the moments.
 //
 // Work is cut into chunks of CHUNK elements that never straddle two tensors; chunk c belongs to the tensor t
 // with tensors[t].first_chunk <= c < tensors[t + 1].first_chunk (binary search by the block, the table has one
@@ -126,8 +127,8 @@ __global__ __launch_bounds__(NT) void adam_multi_kernel(const mvit_adam_tensor* 
   if (mis == 0) {  // 16-byte vectors over the aligned body
     const int nvec = n / V;
     for (int i = threadIdx.x; i < nvec; i += NT) {
-      vec_t p = reinterpret_cast<vec_t*>(P)[i], g = reinterpret_cast<const vec_t*>(G)[i];
-      vec_t m = reinterpret_cast<vec_t*>(M)[i], v = reinterpret_cast<vec_t*>(Vv)[i];
+      vec_t p = load_once(reinterpret_cast<vec_t*>(P) + i), g = load_once(reinterpret_cast<const vec_t*>(G) + i);
+      vec_t m = load_once(reinterpret_cast<vec_t*>(M) + i), v = load_once(reinterpret_cast<vec_t*>(Vv) + i);
       float pnew[V];
 #pragma unroll
       for (int j = 0; j < V; ++j) {
@@ -140,8 +141,8 @@ __global__ __launch_bounds__(NT) void adam_multi_kernel(const mvit_adam_tensor* 
         v[j] = from_f32<T>(vf);
       }
       reinterpret_cast<vec_t*>(P)[i] = p;
-      reinterpret_cast<vec_t*>(M)[i] = m;
-      reinterpret_cast<vec_t*>(Vv)[i] = v;
+      __builtin_nontemporal_store(m, reinterpret_cast<vec_t*>(M) + i);
+      __builtin_nontemporal_store(v, reinterpret_cast<vec_t*>(Vv) + i);
       if (wg) reinterpret_cast<vec_t*>(G)[i] = g;
       if (t.shadow) {
         if (sh_bf16) shadow_store<bf16_t>(t.shadow, base + (int64_t)i * V, V, sh_cols, sh_ld, pnew);  // fp32 parameters: element-wise
@@ -183,7 +184,7 @@ __global__ __launch_bounds__(NT) void sumsq_multi_kernel(const mvit_adam_tensor*
   if ((reinterpret_cast<uintptr_t>(G) & 15u) == 0) {
     const int nvec = n / V;
     for (int i = threadIdx.x; i < nvec; i += NT) {
-      const vec_t g = reinterpret_cast<const vec_t*>(G)[i];
+      const vec_t g = load_once(reinterpret_cast<const vec_t*>(G) + i);
 #pragma unroll
       for (int j = 0; j < V; ++j) {
         const float x = to_f32(g[j]);

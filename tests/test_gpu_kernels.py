@@ -80,6 +80,24 @@ def test_rmsnorm_rows_of_whole_and_partial_vectors_per_lane(dtype, rows, cols):
         assert max_rel_err(dw, wr.grad) < TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype,cols", [(torch.bfloat16, 1280), (torch.bfloat16, 264), (torch.bfloat16, 2560), (torch.float32, 1288), (torch.float32, 8)])
+def test_rmsnorm_backward_operands_beyond_the_size_that_goes_past_the_caches(dtype, cols):
+    """One row more, and the two operands that are not read again are loaded past the caches: the same bits, row by row and in the
+    weight gradient, which both sides sum in rows of the same work-groups."""
+    _announce(f"rmsnorm backward at 24 MiB {dtype} {cols} columns")
+    ops = _ops()
+    g = torch.Generator(device=DEV).manual_seed(cols)
+    rows = -(-(24 << 20) // (cols * dtype.itemsize))
+    x, dy, add = (torch.randn(rows, cols, generator=g, device=DEV).to(dtype) for _ in range(3))
+    w = (1.0 + 0.1 * torch.randn(cols, generator=g, device=DEV)).to(dtype)
+    _, rstd = ops.rmsnorm_fwd(x, w, 1e-6)
+    dy[-1] = 0  # adds nothing to the weight gradient
+    dx, dw = ops.rmsnorm_bwd(dy, x, w, rstd, dx_add=add)
+    below_dx, below_dw = ops.rmsnorm_bwd(dy[:-1], x[:-1], w, rstd[:-1], dx_add=add[:-1])
+    assert torch.equal(dx[:-1], below_dx) and torch.equal(dw, below_dw)
+    assert torch.equal(dx[-1], add[-1])
+
+
 # ------------------------------------------------------------------------------------------ RoPE
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("S,H,d", [(1, 1, 16), (13, 5, 80), (7, 64, 128), (3, 3, 2048), (2, 2, 4112), (5, 700, 16), (2, 3, 8208)])
