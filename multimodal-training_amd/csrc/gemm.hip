@@ -1236,11 +1236,11 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
     if (!swiglu) consider(64, 64, 0.19, 0.36, 2.);
     consider(64, 128, 0.37, 0.52, 2.);
     consider(128, 128, 0.60, 0.72, swiglu ? 6. : 2.5);
-    consider(128, 128, swiglu ? 0.45 : 0.44, 0., swiglu ? 2.5 : 3., true);
+    consider(128, 128, swiglu ? 0.45 : 0.40, 0., swiglu ? 2.5 : 3., true);
     if (!swiglu) {
-      consider(32, 64, 0.15, 0., 1.2, true);
-      consider(64, 64, 0.18, 0., 2., true);
-      consider(64, 128, 0.365, 0., 2., true);
+      consider(32, 64, 0.13, 0., 1.2, true);
+      consider(64, 64, 0.155, 0., 1.5, true);
+      consider(64, 128, 0.30, 0., 2., true);
       consider(192, 128, 0.60, 0., 4., true);
     }
   }
@@ -1436,7 +1436,7 @@ extern "C" int mvit_gemm(const mvit_gemm_args* a, mvit_stream_t stream) {
         q.tiles_n = (int)((q.N + n_cols - 1) / n_cols);
         MVIT_REQUIRE((int64_t)q.tiles_m * q.tiles_n * q.split_k < (1ll << 30), "gemm: too many tiles");
         set_tile_order(q, t.bm);
-        return t.bm == 256 ? mvit_gemm_pp(kind, q, n_cu, s) : mvit_gemm_small(kind, t.bm, t.bn, t.lone, q, s);
+        return t.bm == 256 ? mvit_gemm_pp(kind, q, n_cu, s) : mvit_gemm_small(kind, t.bm, t.bn, t.lone, q, a->overlapped ? 0 : n_cu, s);
       };
       const int64_t head = all_256 || p.split_k > 1 ? 0 : rows_in_full_rounds(kind, p.M, p.N, p.K, n_cu);
       if (head > 0) {  // a row's result does not depend on the tile that computes it

@@ -53,7 +53,7 @@ inline void set_tile_order(GemmParams& p, int bm) {
 // product are reduced there too).  They cover the products of the vision tower, see mvit_gemm_tiled_kind.
 enum GemmTiledKind { TILED_NONE = -1, NN_NONE, NN_BIAS, NN_BIAS_RES, NN_BIAS_GELU, NN_SWIGLU, NT_NONE, NT_GELU_BWD, NT_SWIGLU_BWD, TT_NONE, TT_NONE_F32 };
 int mvit_gemm_pp(GemmTiledKind kind, const GemmParams& p, int n_cu, hipStream_t stream);                  // gemm_pingpong.hip
-int mvit_gemm_small(GemmTiledKind kind, int bm, int bn, bool lone, const GemmParams& p, hipStream_t stream);  // gemm_small.hip
+int mvit_gemm_small(GemmTiledKind kind, int bm, int bn, bool lone, const GemmParams& p, int own_units, hipStream_t stream);  // gemm_small.hip; own_units: compute units that no other stream's work fills
 
 constexpr int GEMM_GROUP_MAX = 4;
 struct GemmGroup {

@@ -497,9 +497,53 @@ __device__ __forceinline__ void gemm_small_tile(const GemmParams& p, const unsig
   }
 }
 
+// A wave beside the others that reads two bytes of every 64 of B's part of its tile column, as fast as memory gives them: of the K tiles,
+// tile row tm takes every tiles_m-th, so that together they run ahead of the main loops, which then find B in the memory-side cache.
+// For launches that have units to themselves: there a unit's requests in flight bound the main loop, the more the further away its
+// operands are.  us without / with, weights from HBM, 1280 columns, K = 6912, 3840, 3456 and 1280: 32 x 64, 256 rows 28.5, 18.0, 14.5, 8.1 / 24.8,
+// 15.2, 12.0, 7.8; 64 x 64, 704 rows 34.2, 21.5, 18.6, 9.5 / 29.0, 17.4, 14.8, 8.6; 64 x 128, 1,600 rows 44.8, 27.9, 25.6, 12.2 / 37.8, 22.9, 20.8, 10.9;
+// 128 x 128, 2,048 rows 59.1, 36.6, 34.7, 15.6 / 51.3, 30.8, 27.2, 14.4, 3,136 rows 56.8, 34.3, 33.3, 15.2 / 57.7, 33.8, 32.0, 14.8.  Not on 192 x 128
+// (4,096 rows 67.8, 40.2, 38.0, 17.5 / 70.7, 41.2, 38.8, 18.0) nor where two work-groups share a unit (1,024 rows on 64 x 64 43.3 / 46.1), nor for fewer than
+// four tile rows, whose waves would have too much to read (encoding 64 patches 2.32 / 2.67 ms; 128 rows 28.9, 18.5, 14.6, 8.2 / 28.3, 16.9, 13.4, 8.1),
+// nor beside a second stream (ms per step without / with in the backward: 1,600 rows 14.14 / 13.81, 1,936 15.32 / 15.54, 2,600 18.83 / 18.91; checkpointed
+// 1,600 16.55 / 16.65, 1,936 18.38 / 18.56).
+template <bool TB, bool DUAL, typename S>
+__device__ __forceinline__ void touch_b(const GemmParams& p, const unsigned block) {
+  const unsigned tiles = (unsigned)(p.tiles_m * p.tiles_n), per_xcd = (tiles + 7) / 8, work = (block & 7) * per_xcd + (block >> 3);
+  if ((block >> 3) >= per_xcd || work >= tiles) return;
+  int tm, tn;
+  tile_coords(p, (int)work, tm, tn);
+  constexpr int COLS = DUAL ? S::BN / 2 : S::BN;  // of one matrix
+  constexpr int STEP = 32, PER = S::BN * S::BK / STEP / 64, AT_ONCE = 16 / PER;  // elements; loads of a lane and K tile; K tiles at once
+  const int64_t n0 = (int64_t)tn * COLS;
+  const int lane = threadIdx.x & 63, n_kt = (int)((p.K + S::BK - 1) / S::BK), n_last = (int)(p.N - n0 < COLS ? p.N - n0 : COLS) - 1;
+  unsigned seen = 0;
+  for (int t0 = tm; t0 < n_kt; t0 += p.tiles_m * AT_ONCE) {
+    unsigned v[AT_ONCE][PER];
+#pragma unroll
+    for (int a = 0; a < AT_ONCE; ++a)
+#pragma unroll
+      for (int j = 0; j < PER; ++j) {
+        const int t = t0 + a * p.tiles_m, i = j * 64 + lane;  // past the end: the last K tile, column or k again
+        const int64_t k = (int64_t)(t < n_kt ? t : n_kt - 1) * S::BK + (TB ? i / (S::BN / STEP) : i % (S::BK / STEP) * STEP), k_in = k < p.K ? k : p.K - 1;
+        const int all = TB ? i % (S::BN / STEP) * STEP : i / (S::BK / STEP), n = all % COLS, n_in = n < n_last ? n : n_last;
+        const bf16_t* B = static_cast<const bf16_t*>(DUAL && all >= COLS ? p.B2 : p.B) + (TB ? n0 : n0 * p.ldb);
+        v[a][j] = *reinterpret_cast<const unsigned short*>(B + (TB ? k_in * p.ldb + n_in : n_in * p.ldb + k_in));
+      }
+#pragma unroll
+    for (int a = 0; a < AT_ONCE; ++a)
+#pragma unroll
+      for (int j = 0; j < PER; ++j) seen ^= v[a][j];
+  }
+  asm volatile("" : : "v"(seen));
+}
+
 // registers for two work-groups per compute unit; LDS holds two of the smaller rings, one of the deeper ones (Lone*)
 template <typename TO, bool TA, bool TB, int EPI, typename S>
-__global__ __launch_bounds__(S::NTHREADS, S::NW / 2) void gemm_small_kernel(const GemmParams p) {
+__global__ __launch_bounds__(S::NTHREADS + (TA ? 0 : 64), S::NW / 2) void gemm_small_kernel(const GemmParams p) {
+  if constexpr (!TA) {
+    if (threadIdx.x >= S::NTHREADS) return touch_b<TB, EPI == MVIT_EPI_SWIGLU, S>(p, blockIdx.x);
+  }
   gemm_small_tile<TO, TA, TB, EPI, S>(p, blockIdx.x);
 }
 // several independent products: each takes a range of work-groups, a multiple of eight so that it stays dealt to the XCDs
@@ -521,7 +565,7 @@ using Lone128 = SmallCfg<128, 128, 2, 2, 4>;          // 128 KiB
 using Lone192 = SmallCfg<192, 128, 2, 2, 4>;          // 160 KiB
 
 template <typename S, typename P>
-int launch_grid(void (*kern)(P), const P& p, unsigned grid, bool (&attr_set_on)[MVIT_MAX_DEVICES], hipStream_t stream) {
+int launch_grid(void (*kern)(P), const P& p, unsigned grid, bool (&attr_set_on)[MVIT_MAX_DEVICES], hipStream_t stream, bool extra_wave = false) {
   const int dev = mvit_current_device("gemm");
   if (dev < 0) return MVIT_ERR_LAUNCH;
   if (!attr_set_on[dev] && S::LDS > 64 * 1024) {  // dynamic LDS above 64 KiB is opted into once per kernel and device
@@ -529,16 +573,16 @@ int launch_grid(void (*kern)(P), const P& p, unsigned grid, bool (&attr_set_on)[
     if (e != hipSuccess) return mvit_set_error(MVIT_ERR_LAUNCH, "gemm: hipFuncSetAttribute(%d B LDS): %s", S::LDS, hipGetErrorString(e));
     attr_set_on[dev] = true;
   }
-  hipLaunchKernelGGL(kern, grid, S::NTHREADS, S::LDS, stream, p);
+  hipLaunchKernelGGL(kern, grid, S::NTHREADS + (extra_wave ? 64 : 0), S::LDS, stream, p);
   MVIT_CHECK_LAUNCH("gemm");
   return MVIT_OK;
 }
 inline unsigned grid_of(const GemmParams& p) { return (unsigned)((p.tiles_m * p.tiles_n * p.split_k + 7) / 8 * 8); }
 
 template <typename TO, bool TA, bool TB, int EPI, typename S>
-int launch_small(const GemmParams& p, hipStream_t stream) {
+int launch_small(const GemmParams& p, bool alone, hipStream_t stream) {
   static bool attr_set_on[MVIT_MAX_DEVICES] = {};
-  return launch_grid<S>(gemm_small_kernel<TO, TA, TB, EPI, S>, p, grid_of(p), attr_set_on, stream);
+  return launch_grid<S>(gemm_small_kernel<TO, TA, TB, EPI, S>, p, grid_of(p), attr_set_on, stream, !TA && S::BM < 192 && p.split_k == 1 && alone);
 }
 template <typename S>
 int launch_group(GemmGroup& g, hipStream_t stream) {
@@ -552,20 +596,20 @@ int launch_group(GemmGroup& g, hipStream_t stream) {
 }
 
 template <typename S>
-int dispatch_small(GemmTiledKind kind, const GemmParams& p, hipStream_t s) {
+int dispatch_small(GemmTiledKind kind, const GemmParams& p, bool alone, hipStream_t s) {
   switch (kind) {
-    case NN_NONE: return launch_small<bf16_t, false, false, MVIT_EPI_NONE, S>(p, s);
-    case NN_BIAS: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS, S>(p, s);
-    case NN_BIAS_RES: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_RES, S>(p, s);
-    case NN_BIAS_GELU: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_GELU, S>(p, s);
+    case NN_NONE: return launch_small<bf16_t, false, false, MVIT_EPI_NONE, S>(p, alone, s);
+    case NN_BIAS: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS, S>(p, alone, s);
+    case NN_BIAS_RES: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_RES, S>(p, alone, s);
+    case NN_BIAS_GELU: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_GELU, S>(p, alone, s);
     case NN_SWIGLU:
-      if constexpr (S::WN == 64) return launch_small<bf16_t, false, false, MVIT_EPI_SWIGLU, S>(p, s);
+      if constexpr (S::WN == 64) return launch_small<bf16_t, false, false, MVIT_EPI_SWIGLU, S>(p, alone, s);
       break;
-    case NT_NONE: return launch_small<bf16_t, false, true, MVIT_EPI_NONE, S>(p, s);
-    case NT_GELU_BWD: return launch_small<bf16_t, false, true, MVIT_EPI_GELU_BWD, S>(p, s);
-    case NT_SWIGLU_BWD: return launch_small<bf16_t, false, true, MVIT_EPI_SWIGLU_BWD, S>(p, s);
-    case TT_NONE: return launch_small<bf16_t, true, true, MVIT_EPI_NONE, S>(p, s);
-    case TT_NONE_F32: return launch_small<float, true, true, MVIT_EPI_NONE, S>(p, s);
+    case NT_NONE: return launch_small<bf16_t, false, true, MVIT_EPI_NONE, S>(p, alone, s);
+    case NT_GELU_BWD: return launch_small<bf16_t, false, true, MVIT_EPI_GELU_BWD, S>(p, alone, s);
+    case NT_SWIGLU_BWD: return launch_small<bf16_t, false, true, MVIT_EPI_SWIGLU_BWD, S>(p, alone, s);
+    case TT_NONE: return launch_small<bf16_t, true, true, MVIT_EPI_NONE, S>(p, alone, s);
+    case TT_NONE_F32: return launch_small<float, true, true, MVIT_EPI_NONE, S>(p, alone, s);
     default: break;
   }
   return mvit_set_error(MVIT_ERR_UNSUPPORTED, "gemm: product kind %d has no %d x %d kernel", (int)kind, S::BM, S::BN);
@@ -573,19 +617,19 @@ int dispatch_small(GemmTiledKind kind, const GemmParams& p, hipStream_t s) {
 
 // the tiles of which one work-group fills a compute unit: products with one operand or none behind the transposing LDS read
 template <typename S>
-int dispatch_lone(GemmTiledKind kind, const GemmParams& p, hipStream_t s) {
+int dispatch_lone(GemmTiledKind kind, const GemmParams& p, bool alone, hipStream_t s) {
   switch (kind) {
-    case NN_NONE: return launch_small<bf16_t, false, false, MVIT_EPI_NONE, S>(p, s);
-    case NN_BIAS: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS, S>(p, s);
-    case NN_BIAS_RES: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_RES, S>(p, s);
-    case NN_BIAS_GELU: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_GELU, S>(p, s);
-    case NT_NONE: return launch_small<bf16_t, false, true, MVIT_EPI_NONE, S>(p, s);
-    case NT_GELU_BWD: return launch_small<bf16_t, false, true, MVIT_EPI_GELU_BWD, S>(p, s);
+    case NN_NONE: return launch_small<bf16_t, false, false, MVIT_EPI_NONE, S>(p, alone, s);
+    case NN_BIAS: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS, S>(p, alone, s);
+    case NN_BIAS_RES: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_RES, S>(p, alone, s);
+    case NN_BIAS_GELU: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_GELU, S>(p, alone, s);
+    case NT_NONE: return launch_small<bf16_t, false, true, MVIT_EPI_NONE, S>(p, alone, s);
+    case NT_GELU_BWD: return launch_small<bf16_t, false, true, MVIT_EPI_GELU_BWD, S>(p, alone, s);
     case NN_SWIGLU:
-      if constexpr (S::BM == 128) return launch_small<bf16_t, false, false, MVIT_EPI_SWIGLU, S>(p, s);
+      if constexpr (S::BM == 128) return launch_small<bf16_t, false, false, MVIT_EPI_SWIGLU, S>(p, alone, s);
       break;
     case NT_SWIGLU_BWD:
-      if constexpr (S::BM == 64 && S::BN == 64) return launch_small<bf16_t, false, true, MVIT_EPI_SWIGLU_BWD, S>(p, s);
+      if constexpr (S::BM == 64 && S::BN == 64) return launch_small<bf16_t, false, true, MVIT_EPI_SWIGLU_BWD, S>(p, alone, s);
       break;
     default: break;
   }
@@ -594,16 +638,17 @@ int dispatch_lone(GemmTiledKind kind, const GemmParams& p, hipStream_t s) {
 
 }  // namespace
 
-int mvit_gemm_small(GemmTiledKind kind, int bm, int bn, bool lone, const GemmParams& p, hipStream_t stream) {
+int mvit_gemm_small(GemmTiledKind kind, int bm, int bn, bool lone, const GemmParams& p, int own_units, hipStream_t stream) {
+  const bool alone = p.tiles_m * p.tiles_n <= own_units && p.tiles_m >= 4;  // a work-group has its unit to itself, and few K tiles to read ahead, see touch_b
   if (lone) {
-    if (bm == 192) return dispatch_lone<Lone192>(kind, p, stream);
-    if (bm == 128) return dispatch_lone<Lone128>(kind, p, stream);
-    if (bm == 32) return dispatch_lone<Lone32x64>(kind, p, stream);
-    return bn == 128 ? dispatch_lone<Lone64x128>(kind, p, stream) : dispatch_lone<Lone64>(kind, p, stream);
+    if (bm == 192) return dispatch_lone<Lone192>(kind, p, alone, stream);
+    if (bm == 128) return dispatch_lone<Lone128>(kind, p, alone, stream);
+    if (bm == 32) return dispatch_lone<Lone32x64>(kind, p, alone, stream);
+    return bn == 128 ? dispatch_lone<Lone64x128>(kind, p, alone, stream) : dispatch_lone<Lone64>(kind, p, alone, stream);
   }
-  if (bm == 128) return dispatch_small<Small128>(kind, p, stream);
-  if (bn == 128) return dispatch_small<Small64x128>(kind, p, stream);
-  return dispatch_small<Small64>(kind, p, stream);
+  if (bm == 128) return dispatch_small<Small128>(kind, p, alone, stream);
+  if (bn == 128) return dispatch_small<Small64x128>(kind, p, alone, stream);
+  return dispatch_small<Small64>(kind, p, alone, stream);
 }
 // weight gradients (both operands transposed, bf16 results), tiles_m / tiles_n set for bm x bn
 int mvit_gemm_small_group(int bm, int bn, GemmGroup& g, hipStream_t stream) {
