@@ -505,18 +505,20 @@ __device__ __forceinline__ void gemm_small_tile(const GemmParams& p, const unsig
 // 128 x 128, 2,048 rows 59.1, 36.6, 34.7, 15.6 / 51.3, 30.8, 27.2, 14.4, 3,136 rows 56.8, 34.3, 33.3, 15.2 / 57.7, 33.8, 32.0, 14.8.  Not on 192 x 128
 // (4,096 rows 67.8, 40.2, 38.0, 17.5 / 70.7, 41.2, 38.8, 18.0) nor where two work-groups share a unit (1,024 rows on 64 x 64 43.3 / 46.1), nor for fewer than
 // four tile rows, whose waves would have too much to read (encoding 64 patches 2.32 / 2.67 ms; 128 rows 28.9, 18.5, 14.6, 8.2 / 28.3, 16.9, 13.4, 8.1),
-// nor beside a second stream (ms per step without / with in the backward: 1,600 rows 14.14 / 13.81, 1,936 15.32 / 15.54, 2,600 18.83 / 18.91; checkpointed
+// nor on SwiGLU, which loses more than it gains (K = 1280, two of 3456 columns: 64 x 128, 200 rows 13.6 / 15.8, 256 14.7 / 15.8; 128 x 128, 448 rows
+// 18.5 / 19.1, 512 18.7 / 18.0), nor beside a second stream (ms per step without / with in the backward: 1,600 rows 14.14 / 13.81, 1,936 15.32 / 15.54, 2,600 18.83 / 18.91; checkpointed
 // 1,600 16.55 / 16.65, 1,936 18.38 / 18.56).
-template <bool TB, bool DUAL, typename S>
+template <bool TA, int EPI, typename S>
+constexpr bool TOUCHES = !TA && S::BM < 192 && EPI != MVIT_EPI_SWIGLU;
+template <bool TB, typename S>
 __device__ __forceinline__ void touch_b(const GemmParams& p, const unsigned block) {
   const unsigned tiles = (unsigned)(p.tiles_m * p.tiles_n), per_xcd = (tiles + 7) / 8, work = (block & 7) * per_xcd + (block >> 3);
   if ((block >> 3) >= per_xcd || work >= tiles) return;
   int tm, tn;
   tile_coords(p, (int)work, tm, tn);
-  constexpr int COLS = DUAL ? S::BN / 2 : S::BN;  // of one matrix
   constexpr int STEP = 32, PER = S::BN * S::BK / STEP / 64, AT_ONCE = 16 / PER;  // elements; loads of a lane and K tile; K tiles at once
-  const int64_t n0 = (int64_t)tn * COLS;
-  const int lane = threadIdx.x & 63, n_kt = (int)((p.K + S::BK - 1) / S::BK), n_last = (int)(p.N - n0 < COLS ? p.N - n0 : COLS) - 1;
+  const int64_t n0 = (int64_t)tn * S::BN;
+  const int lane = threadIdx.x & 63, n_kt = (int)((p.K + S::BK - 1) / S::BK), n_last = (int)(p.N - n0 < S::BN ? p.N - n0 : S::BN) - 1;
   unsigned seen = 0;
   for (int t0 = tm; t0 < n_kt; t0 += p.tiles_m * AT_ONCE) {
     unsigned v[AT_ONCE][PER];
@@ -526,8 +528,8 @@ __device__ __forceinline__ void touch_b(const GemmParams& p, const unsigned bloc
       for (int j = 0; j < PER; ++j) {
         const int t = t0 + a * p.tiles_m, i = j * 64 + lane;  // past the end: the last K tile, column or k again
         const int64_t k = (int64_t)(t < n_kt ? t : n_kt - 1) * S::BK + (TB ? i / (S::BN / STEP) : i % (S::BK / STEP) * STEP), k_in = k < p.K ? k : p.K - 1;
-        const int all = TB ? i % (S::BN / STEP) * STEP : i / (S::BK / STEP), n = all % COLS, n_in = n < n_last ? n : n_last;
-        const bf16_t* B = static_cast<const bf16_t*>(DUAL && all >= COLS ? p.B2 : p.B) + (TB ? n0 : n0 * p.ldb);
+        const int n = TB ? i % (S::BN / STEP) * STEP : i / (S::BK / STEP), n_in = n < n_last ? n : n_last;
+        const bf16_t* B = static_cast<const bf16_t*>(p.B) + (TB ? n0 : n0 * p.ldb);
         v[a][j] = *reinterpret_cast<const unsigned short*>(B + (TB ? k_in * p.ldb + n_in : n_in * p.ldb + k_in));
       }
 #pragma unroll
@@ -540,9 +542,9 @@ __device__ __forceinline__ void touch_b(const GemmParams& p, const unsigned bloc
 
 // registers for two work-groups per compute unit; LDS holds two of the smaller rings, one of the deeper ones (Lone*)
 template <typename TO, bool TA, bool TB, int EPI, typename S>
-__global__ __launch_bounds__(S::NTHREADS + (TA ? 0 : 64), S::NW / 2) void gemm_small_kernel(const GemmParams p) {
-  if constexpr (!TA) {
-    if (threadIdx.x >= S::NTHREADS) return touch_b<TB, EPI == MVIT_EPI_SWIGLU, S>(p, blockIdx.x);
+__global__ __launch_bounds__(S::NTHREADS + (TOUCHES<TA, EPI, S> ? 64 : 0), S::NW / 2) void gemm_small_kernel(const GemmParams p) {
+  if constexpr (TOUCHES<TA, EPI, S>) {
+    if (threadIdx.x >= S::NTHREADS) return touch_b<TB, S>(p, blockIdx.x);
   }
   gemm_small_tile<TO, TA, TB, EPI, S>(p, blockIdx.x);
 }
@@ -582,7 +584,7 @@ inline unsigned grid_of(const GemmParams& p) { return (unsigned)((p.tiles_m * p.
 template <typename TO, bool TA, bool TB, int EPI, typename S>
 int launch_small(const GemmParams& p, bool alone, hipStream_t stream) {
   static bool attr_set_on[MVIT_MAX_DEVICES] = {};
-  return launch_grid<S>(gemm_small_kernel<TO, TA, TB, EPI, S>, p, grid_of(p), attr_set_on, stream, !TA && S::BM < 192 && p.split_k == 1 && alone);
+  return launch_grid<S>(gemm_small_kernel<TO, TA, TB, EPI, S>, p, grid_of(p), attr_set_on, stream, TOUCHES<TA, EPI, S> && p.split_k == 1 && alone);
 }
 template <typename S>
 int launch_group(GemmGroup& g, hipStream_t stream) {
