@@ -305,6 +305,9 @@ int mvit_image_token_ranks(const int64_t* input_ids, const int64_t* labels, int6
 /* Host-only: waits until none of n values that a kernel writes to pinned host memory is negative, for timeout_us microseconds at
  * most.  0: all are there; 1: not yet.  The caller sets them to -1 before the launch. */
 int mvit_wait_host_values(const int64_t* values, int n, int64_t timeout_us);
+/* The same without a time limit, for a kernel on `stream`: returns when the values are there (0), or when the stream has failed or has
+ * nothing left that could write them (MVIT_ERR_LAUNCH).  A stream that is being captured fails. */
+int mvit_await_host_values(const int64_t* values, int n, mvit_stream_t stream);
 
 /* merged[t, :] = rank[t] >= 0 ? vision[rank[t], :] : embeds[t, :] over rows of row_bytes bytes (bit-exact copy);
  * with vision == NULL the selected rows are zero-filled instead.  A rank >= n_vision keeps the embeds row.

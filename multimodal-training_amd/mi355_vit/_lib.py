@@ -96,6 +96,7 @@ PROTOTYPES = {
     "mvit_attn_fwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i64, _i32, _i32, _i64, _i64, _i64, _i64, _f32, _i32, _vp],
     "mvit_image_token_ranks": [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp],
     "mvit_wait_host_values": [_vp, _i32, _i64],
+    "mvit_await_host_values": [_vp, _i32, _vp],
     "mvit_split_rows": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp],
     "mvit_copy_ranges": [_vp, _i32, _vp],
     "mvit_merge_rows": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp],

@@ -13,7 +13,6 @@ read-backs and ``masked_scatter``; the backward is one pass over the gradient.
 
 from __future__ import annotations
 
-import time
 from typing import Optional
 
 import torch
@@ -30,26 +29,28 @@ def _int64_row(t: torch.Tensor) -> torch.Tensor:
 
 
 class _Arrival:
-    """Counts that a kernel writes to pinned host memory, -1 until then.  They are seen there as soon as they arrive, some 10 us before an
-    event behind the kernel would tell the host."""
+    """Counts that a kernel on `stream` writes to pinned host memory, -1 until then.  They are seen there as soon as they arrive, some 10 us
+    before an event behind the kernel would tell the host."""
 
-    __slots__ = ("counts", "device")
+    __slots__ = ("counts", "stream")
 
-    def __init__(self, counts: torch.Tensor, device: torch.device):
-        self.counts, self.device = counts, device
-
-    def _after(self, microseconds: int) -> bool:
-        return _lib.load().mvit_wait_host_values(self.counts.data_ptr(), self.counts.numel(), microseconds) == 0
+    def __init__(self, counts: torch.Tensor, stream: int):
+        self.counts, self.stream = counts, stream
 
     def query(self) -> bool:
-        return self._after(0)
+        return _lib.load().mvit_wait_host_values(self.counts.data_ptr(), self.counts.numel(), 0) == 0
+
+    def _wait(self) -> None:
+        # one call, which no signal handler ends early
+        _lib.check(_lib.load().mvit_await_host_values(self.counts.data_ptr(), self.counts.numel(), self.stream), "mvit_await_host_values")
 
     def synchronize(self) -> None:
-        if self._after(2000):  # without the interpreter's lock
-            return
-        stream = torch.cuda.current_stream(self.device)
-        while not self.query() and not stream.query():  # a stream that has failed raises here
-            time.sleep(1e-4)
+        """Returns or raises when the counts are there or the stream has nothing left that could write them."""
+        try:
+            self._wait()
+        except BaseException:  # of a signal handler that ran before the call, too
+            self._wait()
+            raise
 
 
 def _ranks(input_ids: torch.Tensor, labels: Optional[torch.Tensor], image_token_id: int):
@@ -61,13 +62,17 @@ def _ranks(input_ids: torch.Tensor, labels: Optional[torch.Tensor], image_token_
         if labels.numel() != ids.numel():
             raise ValueError("labels and input_ids differ in size")
         lab = _int64_row(labels)
-    n = ids.numel()
+    n, stream = ids.numel(), _stream(ids)
     rank = torch.empty(n, dtype=torch.int32, device=ids.device)
     counts = torch.empty(2, dtype=torch.int64, pin_memory=True).fill_(-1)  # the kernel writes them where the host reads them
-    rc = _lib.load().mvit_image_token_ranks(ids.data_ptr(), None if lab is None else lab.data_ptr(), n, image_token_id, -100,
-                                            rank.data_ptr(), None, counts.data_ptr(), _stream(ids))
-    _lib.check(rc, "mvit_image_token_ranks")
-    return rank, counts, _Arrival(counts, ids.device)
+    try:
+        rc = _lib.load().mvit_image_token_ranks(ids.data_ptr(), None if lab is None else lab.data_ptr(), n, image_token_id, -100,
+                                                rank.data_ptr(), None, counts.data_ptr(), stream)
+        _lib.check(rc, "mvit_image_token_ranks")
+        return rank, counts, _Arrival(counts, stream)
+    except BaseException:
+        torch.cuda.synchronize(ids.device)
+        raise
 
 
 class _MergeRowsFn(torch.autograd.Function):

@@ -128,6 +128,30 @@ def test_a_merge_that_fails_still_waits_for_the_counts(monkeypatch):
     assert len(taken) == 1 and taken[0].query()
 
 
+def test_the_wait_behind_queued_work_is_one_call(monkeypatch):
+    """The counts arrive long after the merge has been queued: the host waits for them without sleeping in between, and they are right."""
+    import time
+
+    from mi355_vit.handoff import merge_vision_embeddings
+
+    _announce("hand-off behind queued work")
+
+    def sleeps(seconds):
+        raise AssertionError("the host slept while it waited")
+
+    monkeypatch.setattr(time, "sleep", sleeps)
+    ids = torch.full((1, 40), 11, device=DEV)
+    ids[0, 3:8] = IMG
+    emb, vis = torch.randn(1, 40, 64, device=DEV), torch.randn(5, 64, device=DEV)
+    merge_vision_embeddings(emb, ids, vis)
+    torch.cuda._sleep(1 << 25)  # some 15 ms in front of the ranking kernel
+    got = merge_vision_embeddings(emb, ids, vis)
+    assert torch.equal(got[0, 3:8], vis) and torch.equal(got[0, 8:], emb[0, 8:])
+    torch.cuda._sleep(1 << 25)
+    with pytest.raises(RuntimeError, match="4 vision embeddings but 5 <image> tokens"):
+        merge_vision_embeddings(emb, ids, vis[:4])
+
+
 def test_tower_output_feeds_the_handoff():
     """End of the path: the tower's [M, O] output goes into the placeholders and its gradient comes back unchanged
     in shape and order (the vision actor's backward_step accepts the 2-D gradient)."""
