@@ -201,6 +201,10 @@ typedef struct mvit_gemm_args {
  * (merger), with the element-wise ops of :204, :256, :784, :791 fused as epilogues. */
 int mvit_gemm(const mvit_gemm_args* args, mvit_stream_t stream);
 
+/* Host-only: the tile with which a bf16 product of this form and shape is computed on n_cu compute units, biases given, operands
+ * aligned, neither K slices nor column sums: tile[0] x tile[1] (rows x columns; 0: no tile fits, a kernel of 256 rows), tile[2]
+ * work-groups to a unit, tile[3] whether a wave of each reads B ahead of the main loop. */
+int mvit_gemm_tile(int trans_a, int trans_b, int epilogue, int64_t M, int64_t N, int64_t K, int overlapped, int n_cu, int32_t* tile);
 /* Host-only: the split_k to ask for when C[out_rows, out_cols] is a weight gradient contracted over k tokens (bf16). */
 int mvit_gemm_wgrad_split_k(int64_t out_rows, int64_t out_cols, int64_t k);
 /* Host-only: the same for a product that shares the GPU with another stream's (`overlapped`). */

@@ -1166,10 +1166,13 @@ bool pp_takes(GemmTiledKind kind, int64_t k_chunk, int64_t k_last) {  // at leas
 // step of 64 along K takes 1.15 us in a 256 x 256 tile (one work-group per compute unit; 1.2 with both operands behind the
 // transposing LDS read; 2,392 cycles, so more when the clock falls under a long load, which lengthens every tile's steps alike), and in the smaller ones `one` us while every unit has at most one work-group and `two` us once it has
 // two.  Tiles of one work-group per unit (`lone`) interleave loads, LDS reads and MFMAs, so their steps are shorter than those of a
-// single work-group of the kind that shares its unit: 32 x 64 is taken up to 256 tiles, then 64 x 64 up to 256, two of them to a unit up to 448, 64 x 128
-// from there to 256, 128 x 128 and 192 x 128 in the same way (1280 columns, weights from HBM, us at K = 6912, 3840, 3456, 1280, 64 x 64 / 32 x 64: 256 rows
-// 34.8, 21.9, 18.7, 9.5 / 28.6, 18.0, 14.5, 8.3, 512 rows 34.4, 21.5, 18.6, 9.5 / 36.9, 22.1, 17.8, 9.4; 64 x 64 / 64 x 128: 1,024 rows 43.4, 25.8, 23.4, 11.6 /
-// 44.4, 27.7, 25.4, 13.1, 1,400 rows 46.2, 27.4, 24.8, 12.6 / 44.6, 27.8, 26.6, 14.5, 1,600 rows 55.9, 33.7, 28.5, 13.9 / 45.0, 27.9, 25.6, 13.2)
+// single work-group of the kind that shares its unit, and shorter again (`one_ahead`) where a wave reads B ahead of the main loops (gemm_reads_ahead).
+// For 1280 columns that gives 32 x 64 up to 384 rows, 64 x 64 up to 768, 64 x 128 up to 1,600, 128 x 128 up to 3,200 and 192 x 128 from 3,265 to 4,800, one work-group
+// per unit each.  us, input gradients of 1280 columns, weights from HBM, K = 6912, 3840, 3456, 1280: 384 rows, 32 x 64 / 64 x 64 25.0, 15.1, 13.9, 7.7 / 31.0, 19.1, 17.4, 8.9; 512,
+// 32 x 64 in two rounds / 64 x 64 37.1, 21.9, 20.0, 9.7 / 29.1, 17.6, 15.9, 8.7; 784, 32 x 64 in two rounds / 64 x 128 44.4, 26.0, 23.4, 10.9 / 36.5, 23.1, 20.4, 10.6; 1,024, two 64 x 64
+// to a unit / 64 x 128 43.7, 26.0, 23.6, 11.0 / 37.2, 22.5, 20.6, 10.8; 1,600 57.0, 33.3, 30.2, 13.5 / 38.6, 24.0, 22.1, 11.1.  Beside another stream nothing is read ahead (1,024 rows on
+// 64 x 128 45.6, 27.2, 24.7, 11.7), but the same tiles are taken: two 64 x 64 to a unit compete with the other stream for the L2s.  ms per step, 8 blocks of 2560 columns,
+// two 64 x 64 / 64 x 128: 440 rows 4.99 - 5.07 / 4.86 - 5.01, 576 5.42 - 5.49 / 5.12 - 5.27.
 // (input gradient of 6912 x 1280, us, shared / 128 lone / 192 lone: 2,048 rows 70 / 48 / 61, 3,136 73 / 55 / 65, 4,096 78 / 95 / 68,
 // 6,084 91 / 104 / 127; ms per step before -> with them: 3,136 rows 21.0 -> 19.9, 4,096 checkpointed 29.2 -> 28.0).  A fuller last round, a shorter step and more units at work all lower the estimate; the epilogue of a 256 x 256 tile is
 // the longest.  The line between the tiles follows from these numbers and not from any shape: e.g. weight gradients of
@@ -1212,8 +1215,9 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
   const bool input_grad = kind == NT_NONE || kind == NT_GELU_BWD, fills = 2 * ((M + 255) / 256) * ((N + 255) / 256) >= n_cu;
   const double alone = !overlapped ? 1. : tt ? 0.5 : (input_grad && fills ? 0.3 : 1.);
   TileChoice best{0, 0, 1e30};
-  auto consider = [&](int bm, int bn, double one, double two, double per_tile, bool lone = false) {
-    const int64_t items = ((M + bm - 1) / bm) * ((N * n_mul + bn - 1) / bn) * slices;
+  auto consider = [&](int bm, int bn, double one, double two, double per_tile, bool lone = false, double one_ahead = 0.) {
+    const int64_t tiles_m = (M + bm - 1) / bm, items = tiles_m * ((N * n_mul + bn - 1) / bn) * slices;
+    if (one_ahead > 0. && gemm_reads_ahead(kind, bm, tiles_m, items, slices, n_cu)) one = one_ahead;
     const int64_t slots = two > 0. ? 2 * (int64_t)n_cu : n_cu, full = items / slots, rest = items % slots;
     const double round = steps * (two > 0. ? two : one) + per_tile;
     double us = full * round;
@@ -1236,11 +1240,11 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
     if (!swiglu) consider(64, 64, 0.19, 0.36, 2.);
     consider(64, 128, 0.37, 0.52, 2.);
     consider(128, 128, 0.60, 0.72, swiglu ? 6. : 2.5);
-    consider(128, 128, swiglu ? 0.45 : 0.40, 0., swiglu ? 2.5 : 3., true);
+    consider(128, 128, swiglu ? 0.45 : 0.44, 0., swiglu ? 2.5 : 3., true, 0.40);
     if (!swiglu) {
-      consider(32, 64, 0.13, 0., 1.2, true);
-      consider(64, 64, 0.155, 0., 1.5, true);
-      consider(64, 128, 0.30, 0., 2., true);
+      consider(32, 64, 0.15, 0., 1.2, true, 0.13);
+      consider(64, 64, 0.18, 0., 2., true, 0.155);
+      consider(64, 128, 0.365, 0., 2., true, 0.30);
       consider(192, 128, 0.60, 0., 4., true);
     }
   }
@@ -1552,6 +1556,21 @@ static int wgrad_split_k(int64_t out_rows, int64_t out_cols, int64_t k, bool ove
     }
   }
   return best;
+}
+
+extern "C" int mvit_gemm_tile(int trans_a, int trans_b, int epilogue, int64_t M, int64_t N, int64_t K, int overlapped, int n_cu, int32_t* tile) {
+  MVIT_REQUIRE(tile && M > 0 && N > 0 && K > 0 && n_cu > 0, "gemm_tile: null pointer or bad shape");
+  GemmParams p{};
+  p.N = N;
+  p.bias = p.bias2 = &p;  // as a product with biases has them
+  const GemmTiledKind kind = tiled_kind(MVIT_BF16, MVIT_BF16, trans_a, trans_b, epilogue, p);
+  if (kind == TILED_NONE) return mvit_set_error(MVIT_ERR_UNSUPPORTED, "gemm_tile: trans_a=%d trans_b=%d epilogue %d of %lld columns has no choice of tiles", trans_a, trans_b, epilogue, (long long)N);
+  const TileChoice c = choose_tile(kind, M, N, K, K, 1, n_cu, overlapped != 0);
+  tile[0] = c.bm; tile[1] = c.bn;
+  tile[2] = c.bm == 0 || c.bm == 256 || c.lone ? 1 : 2;
+  const int64_t tiles_m = c.bm ? (M + c.bm - 1) / c.bm : 0;
+  tile[3] = c.bm != 0 && c.bm != 256 && gemm_reads_ahead(kind, c.bm, tiles_m, tiles_m * ((N + c.bn - 1) / c.bn), 1, overlapped ? 0 : n_cu);
+  return MVIT_OK;
 }
 
 extern "C" int mvit_gemm_wgrad_split_k(int64_t out_rows, int64_t out_cols, int64_t k) { return wgrad_split_k(out_rows, out_cols, k, false); }

@@ -582,9 +582,9 @@ int launch_grid(void (*kern)(P), const P& p, unsigned grid, bool (&attr_set_on)[
 inline unsigned grid_of(const GemmParams& p) { return (unsigned)((p.tiles_m * p.tiles_n * p.split_k + 7) / 8 * 8); }
 
 template <typename TO, bool TA, bool TB, int EPI, typename S>
-int launch_small(const GemmParams& p, bool alone, hipStream_t stream) {
+int launch_small(const GemmParams& p, bool ahead, hipStream_t stream) {
   static bool attr_set_on[MVIT_MAX_DEVICES] = {};
-  return launch_grid<S>(gemm_small_kernel<TO, TA, TB, EPI, S>, p, grid_of(p), attr_set_on, stream, TOUCHES<TA, EPI, S> && p.split_k == 1 && alone);
+  return launch_grid<S>(gemm_small_kernel<TO, TA, TB, EPI, S>, p, grid_of(p), attr_set_on, stream, TOUCHES<TA, EPI, S> && ahead);
 }
 template <typename S>
 int launch_group(GemmGroup& g, hipStream_t stream) {
@@ -598,20 +598,20 @@ int launch_group(GemmGroup& g, hipStream_t stream) {
 }
 
 template <typename S>
-int dispatch_small(GemmTiledKind kind, const GemmParams& p, bool alone, hipStream_t s) {
+int dispatch_small(GemmTiledKind kind, const GemmParams& p, bool ahead, hipStream_t s) {
   switch (kind) {
-    case NN_NONE: return launch_small<bf16_t, false, false, MVIT_EPI_NONE, S>(p, alone, s);
-    case NN_BIAS: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS, S>(p, alone, s);
-    case NN_BIAS_RES: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_RES, S>(p, alone, s);
-    case NN_BIAS_GELU: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_GELU, S>(p, alone, s);
+    case NN_NONE: return launch_small<bf16_t, false, false, MVIT_EPI_NONE, S>(p, ahead, s);
+    case NN_BIAS: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS, S>(p, ahead, s);
+    case NN_BIAS_RES: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_RES, S>(p, ahead, s);
+    case NN_BIAS_GELU: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_GELU, S>(p, ahead, s);
     case NN_SWIGLU:
-      if constexpr (S::WN == 64) return launch_small<bf16_t, false, false, MVIT_EPI_SWIGLU, S>(p, alone, s);
+      if constexpr (S::WN == 64) return launch_small<bf16_t, false, false, MVIT_EPI_SWIGLU, S>(p, ahead, s);
       break;
-    case NT_NONE: return launch_small<bf16_t, false, true, MVIT_EPI_NONE, S>(p, alone, s);
-    case NT_GELU_BWD: return launch_small<bf16_t, false, true, MVIT_EPI_GELU_BWD, S>(p, alone, s);
-    case NT_SWIGLU_BWD: return launch_small<bf16_t, false, true, MVIT_EPI_SWIGLU_BWD, S>(p, alone, s);
-    case TT_NONE: return launch_small<bf16_t, true, true, MVIT_EPI_NONE, S>(p, alone, s);
-    case TT_NONE_F32: return launch_small<float, true, true, MVIT_EPI_NONE, S>(p, alone, s);
+    case NT_NONE: return launch_small<bf16_t, false, true, MVIT_EPI_NONE, S>(p, ahead, s);
+    case NT_GELU_BWD: return launch_small<bf16_t, false, true, MVIT_EPI_GELU_BWD, S>(p, ahead, s);
+    case NT_SWIGLU_BWD: return launch_small<bf16_t, false, true, MVIT_EPI_SWIGLU_BWD, S>(p, ahead, s);
+    case TT_NONE: return launch_small<bf16_t, true, true, MVIT_EPI_NONE, S>(p, ahead, s);
+    case TT_NONE_F32: return launch_small<float, true, true, MVIT_EPI_NONE, S>(p, ahead, s);
     default: break;
   }
   return mvit_set_error(MVIT_ERR_UNSUPPORTED, "gemm: product kind %d has no %d x %d kernel", (int)kind, S::BM, S::BN);
@@ -619,19 +619,19 @@ int dispatch_small(GemmTiledKind kind, const GemmParams& p, bool alone, hipStrea
 
 // the tiles of which one work-group fills a compute unit: products with one operand or none behind the transposing LDS read
 template <typename S>
-int dispatch_lone(GemmTiledKind kind, const GemmParams& p, bool alone, hipStream_t s) {
+int dispatch_lone(GemmTiledKind kind, const GemmParams& p, bool ahead, hipStream_t s) {
   switch (kind) {
-    case NN_NONE: return launch_small<bf16_t, false, false, MVIT_EPI_NONE, S>(p, alone, s);
-    case NN_BIAS: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS, S>(p, alone, s);
-    case NN_BIAS_RES: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_RES, S>(p, alone, s);
-    case NN_BIAS_GELU: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_GELU, S>(p, alone, s);
-    case NT_NONE: return launch_small<bf16_t, false, true, MVIT_EPI_NONE, S>(p, alone, s);
-    case NT_GELU_BWD: return launch_small<bf16_t, false, true, MVIT_EPI_GELU_BWD, S>(p, alone, s);
+    case NN_NONE: return launch_small<bf16_t, false, false, MVIT_EPI_NONE, S>(p, ahead, s);
+    case NN_BIAS: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS, S>(p, ahead, s);
+    case NN_BIAS_RES: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_RES, S>(p, ahead, s);
+    case NN_BIAS_GELU: return launch_small<bf16_t, false, false, MVIT_EPI_BIAS_GELU, S>(p, ahead, s);
+    case NT_NONE: return launch_small<bf16_t, false, true, MVIT_EPI_NONE, S>(p, ahead, s);
+    case NT_GELU_BWD: return launch_small<bf16_t, false, true, MVIT_EPI_GELU_BWD, S>(p, ahead, s);
     case NN_SWIGLU:
-      if constexpr (S::BM == 128) return launch_small<bf16_t, false, false, MVIT_EPI_SWIGLU, S>(p, alone, s);
+      if constexpr (S::BM == 128) return launch_small<bf16_t, false, false, MVIT_EPI_SWIGLU, S>(p, ahead, s);
       break;
     case NT_SWIGLU_BWD:
-      if constexpr (S::BM == 64 && S::BN == 64) return launch_small<bf16_t, false, true, MVIT_EPI_SWIGLU_BWD, S>(p, alone, s);
+      if constexpr (S::BM == 64 && S::BN == 64) return launch_small<bf16_t, false, true, MVIT_EPI_SWIGLU_BWD, S>(p, ahead, s);
       break;
     default: break;
   }
@@ -641,16 +641,16 @@ int dispatch_lone(GemmTiledKind kind, const GemmParams& p, bool alone, hipStream
 }  // namespace
 
 int mvit_gemm_small(GemmTiledKind kind, int bm, int bn, bool lone, const GemmParams& p, int own_units, hipStream_t stream) {
-  const bool alone = p.tiles_m * p.tiles_n <= own_units && p.tiles_m >= 4;  // a work-group has its unit to itself, and few K tiles to read ahead, see touch_b
+  const bool ahead = gemm_reads_ahead(kind, bm, p.tiles_m, (int64_t)p.tiles_m * p.tiles_n, p.split_k, own_units);
   if (lone) {
-    if (bm == 192) return dispatch_lone<Lone192>(kind, p, alone, stream);
-    if (bm == 128) return dispatch_lone<Lone128>(kind, p, alone, stream);
-    if (bm == 32) return dispatch_lone<Lone32x64>(kind, p, alone, stream);
-    return bn == 128 ? dispatch_lone<Lone64x128>(kind, p, alone, stream) : dispatch_lone<Lone64>(kind, p, alone, stream);
+    if (bm == 192) return dispatch_lone<Lone192>(kind, p, ahead, stream);
+    if (bm == 128) return dispatch_lone<Lone128>(kind, p, ahead, stream);
+    if (bm == 32) return dispatch_lone<Lone32x64>(kind, p, ahead, stream);
+    return bn == 128 ? dispatch_lone<Lone64x128>(kind, p, ahead, stream) : dispatch_lone<Lone64>(kind, p, ahead, stream);
   }
-  if (bm == 128) return dispatch_small<Small128>(kind, p, alone, stream);
-  if (bn == 128) return dispatch_small<Small64x128>(kind, p, alone, stream);
-  return dispatch_small<Small64>(kind, p, alone, stream);
+  if (bm == 128) return dispatch_small<Small128>(kind, p, ahead, stream);
+  if (bn == 128) return dispatch_small<Small64x128>(kind, p, ahead, stream);
+  return dispatch_small<Small64>(kind, p, ahead, stream);
 }
 // weight gradients (both operands transposed, bf16 results), tiles_m / tiles_n set for bm x bn
 int mvit_gemm_small_group(int bm, int bn, GemmGroup& g, hipStream_t stream) {

@@ -90,6 +90,7 @@ PROTOTYPES = {
     "mvit_pad_pack": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, C.c_uint32, _vp],
     "mvit_cast2d": [_vp, _i64, _i32, _vp, _i64, _i32, _i64, _i64, _vp],
     "mvit_gemm": [C.POINTER(GemmArgs), _vp],
+    "mvit_gemm_tile": [_i32, _i32, _i32, _i64, _i64, _i64, _i32, _i32, _vp],
     "mvit_gemm_wgrad_split_k": [_i64, _i64, _i64],
     "mvit_gemm_wgrad_split_k_overlapped": [_i64, _i64, _i64],
     "mvit_gemm_swiglu_bwd_colsum_rows": [_i64, _i64, _i64],

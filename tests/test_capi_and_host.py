@@ -490,3 +490,25 @@ def test_weight_gradients_leave_the_second_stream_where_a_block_has_little_work(
     assert [side(S, 3840, 10240) for S in (64, 1000)] == [1, 1]
     assert [side(S, 64, 72) for S in (1280, 1281)] == [0, 1]
     assert side(256, 1280, 3420, dtype=_lib.F32, grad=_lib.F32) == side(256, 1280, 3420, grad=_lib.F32) == side(256, 1280, 3420, split=2) == 1
+
+
+def _tile(rows, cols, k, trans_b=1, epilogue=0, overlapped=0):
+    import ctypes
+
+    from mi355_vit import _lib
+
+    tile = (ctypes.c_int32 * 4)()
+    _lib.check(_lib.load().mvit_gemm_tile(0, trans_b, epilogue, rows, cols, k, overlapped, 256, tile), "mvit_gemm_tile")
+    return tuple(tile)
+
+
+@pytest.mark.parametrize("trans_b,epilogue", [(1, 0), (0, 2)])  # an input gradient; bias + residual
+@pytest.mark.parametrize("k", [1280, 3456, 3840, 6912])
+def test_the_tiles_of_few_rows_are_those_measured_fastest(k, trans_b, epilogue):
+    """The wave shortens the steps of the tiles that have a unit to themselves; a second round, which has no such wave, is not taken for it."""
+    alone = lambda rows: _tile(rows, 1280, k, trans_b, epilogue)
+    assert [alone(r)[:3] for r in (96, 384, 385, 768)] == [(32, 64, 1), (32, 64, 1), (64, 64, 1), (64, 64, 1)]
+    assert [alone(r) for r in (769, 800, 801, 1024, 1424, 1600)] == [(64, 128, 1, 1)] * 6
+    assert alone(1601) == (128, 128, 1, 1) and alone(96)[3] == 0 and alone(97)[3] == 1
+    for rows in range(1, 1601, 13):  # beside another stream the same tiles, without the wave
+        assert _tile(rows, 1280, k, trans_b, epilogue, overlapped=1) == alone(rows)[:3] + (0,)
