@@ -1221,7 +1221,8 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
     const int64_t slots = two > 0. ? 2 * (int64_t)n_cu : n_cu, full = items / slots, rest = items % slots;
     const double round = steps * (two > 0. ? two : one) + per_tile;
     double us = full * round;
-    if (bm * bn == 64 * 64 && full == 0 && 4 * rest > 7 * n_cu) two *= 1.15;  // nearly all units with two
+    // nearly all units with two (SwiGLU backward, 64 x 64 / 64 x 128: 528 rows 16.2 / 16.4 us, 576 16.9 / 16.5); not weight gradients: 512 x 640 over 8,192 rows so in 12 slices of 64 x 128 24.3, without 6 of 64 x 64 20.3
+    if (!tt && bm * bn == 64 * 64 && full == 0 && 4 * rest > 7 * n_cu) two *= 1.15;
     if (rest > 0) us += steps * (two > 0. && rest > n_cu ? two : one) + per_tile;
     if (input_grad && !overlapped && two > 0. && items > slots) us *= 1. + (bm == 128 ? 0.05 : 0.15) * (double)((items - 1) / slots);
     us = 4. + alone * us + (1. - alone) * round * (double)items / (double)slots;

@@ -512,3 +512,11 @@ def test_the_tiles_of_few_rows_are_those_measured_fastest(k, trans_b, epilogue):
     assert alone(1601) == (128, 128, 1, 1) and alone(96)[3] == 0 and alone(97)[3] == 1
     for rows in range(1, 1601, 13):  # beside another stream the same tiles, without the wave
         assert _tile(rows, 1280, k, trans_b, epilogue, overlapped=1) == alone(rows)[:3] + (0,)
+
+
+@pytest.mark.parametrize("out_rows,out_cols,k,slices", [(256, 1280, 8192, 6), (128, 2560, 8192, 6), (512, 640, 8192, 6), (640, 640, 3072, 5)])
+def test_weight_gradients_of_nearly_two_small_tiles_per_unit_keep_their_slices(out_rows, out_cols, k, slices):
+    """The slice count is the order of the sums over the rows: what was measured on forward products and input gradients leaves it alone."""
+    from mi355_vit import _lib
+
+    assert _lib.load().mvit_gemm_wgrad_split_k(out_rows, out_cols, k) == slices
