@@ -56,7 +56,7 @@ int mvit_gemm_pp(GemmTiledKind kind, const GemmParams& p, int n_cu, hipStream_t 
 // Whether a launch of tiles of bm rows has a wave read B ahead of the main loops (touch_b, gemm_small.hip): a work-group has one of `own_units`
 // compute units, which no other stream's work fills, to itself, and there are tile rows enough to share the reading.
 inline bool gemm_reads_ahead(GemmTiledKind kind, int bm, int64_t tiles_m, int64_t tiles, int64_t slices, int64_t own_units) {
-  return kind != NN_SWIGLU && kind != TT_NONE && kind != TT_NONE_F32 && bm < 192 && slices == 1 && tiles_m >= 4 && tiles <= own_units;
+  return kind != NN_SWIGLU && kind != NT_SWIGLU_BWD && kind != TT_NONE && kind != TT_NONE_F32 && bm < 192 && slices == 1 && tiles_m >= 4 && tiles <= own_units;
 }
 int mvit_gemm_small(GemmTiledKind kind, int bm, int bn, bool lone, const GemmParams& p, int own_units, hipStream_t stream);  // gemm_small.hip; own_units: compute units that no other stream's work fills
 

@@ -506,7 +506,8 @@ __device__ __forceinline__ void gemm_small_tile(const GemmParams& p, const unsig
 // (4,096 rows 67.8, 40.2, 38.0, 17.5 / 70.7, 41.2, 38.8, 18.0) nor where two work-groups share a unit (1,024 rows on 64 x 64 43.3 / 46.1), nor for fewer than
 // four tile rows, whose waves would have too much to read (encoding 64 patches 2.32 / 2.67 ms; 128 rows 28.9, 18.5, 14.6, 8.2 / 28.3, 16.9, 13.4, 8.1),
 // nor on SwiGLU, which loses more than it gains (K = 1280, two of 3456 columns: 64 x 128, 200 rows 13.6 / 15.8, 256 14.7 / 15.8; 128 x 128, 448 rows
-// 18.5 / 19.1, 512 18.7 / 18.0), nor beside a second stream (ms per step without / with in the backward: 1,600 rows 14.14 / 13.81, 1,936 15.32 / 15.54, 2,600 18.83 / 18.91; checkpointed
+// 18.5 / 19.1, 512 18.7 / 18.0), nor on SwiGLU backward (K = 1280, 3456 columns: 64 x 64, 200 rows 9.7 / 10.5, 224 10.5 / 10.6, 256 11.0 / 10.8, with the weights in the caches
+// 9.1 / 10.2, - , 9.2 / 10.4; 64 x 128, 513 rows 14.8 / 16.3, 576 15.4 / 16.5; its kernel keeps the branch to the wave, without which it takes 10.1, 10.8, 11.4 / 15.1, 15.8), nor beside a second stream (ms per step without / with in the backward: 1,600 rows 14.14 / 13.81, 1,936 15.32 / 15.54, 2,600 18.83 / 18.91; checkpointed
 // 1,600 16.55 / 16.65, 1,936 18.38 / 18.56).
 template <bool TA, int EPI, typename S>
 constexpr bool TOUCHES = !TA && S::BM < 192 && EPI != MVIT_EPI_SWIGLU;

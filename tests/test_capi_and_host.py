@@ -520,3 +520,8 @@ def test_weight_gradients_of_nearly_two_small_tiles_per_unit_keep_their_slices(o
     from mi355_vit import _lib
 
     assert _lib.load().mvit_gemm_wgrad_split_k(out_rows, out_cols, k) == slices
+
+
+@pytest.mark.parametrize("rows", [193, 200, 256, 320, 513, 576, 640, 1024])
+def test_swiglu_backward_has_no_wave_that_reads_b_ahead(rows):
+    assert _tile(rows, 3456, 1280, 1, 5)[3] == 0
