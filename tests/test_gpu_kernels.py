@@ -549,8 +549,9 @@ def test_gemm_of_tall_operands_walks_its_tiles_in_groups_of_rows(M, N, K, form):
 # 32 x 64 tiles (a ring of five stages; 64 x 64 and four for `tt`) and 64 x 64 ones, two work-groups per unit (four stages): the ring never
 # full, once full, refilled in turn, with and without a partial last K tile ...
 _RING_SHAPES = [(70, 200, k) for k in (8, 64, 72, 128, 136, 192, 200, 256, 264, 320, 384, 392, 456, 840)] + [(1500, 1288, k) for k in (8, 64, 72, 136, 192, 264)]
-# ... the same for 64 x 64, one work-group per unit, and 64 x 128 (four stages each), with the last row count of a tile and the first of the next ...
-_RING_SHAPES += [(m, 1280, k) for m in (385, 1601) for k in (8, 64, 72, 128, 136, 192, 200, 256, 264, 320, 328, 384, 392)]
+# ... the same for 64 x 64 and 64 x 128, one work-group per unit (four stages each), and 64 x 128, two to a unit (three; from K = 840 on, 128 x 128), with the last
+# row count of a tile and the first of the next ...
+_RING_SHAPES += [(m, 1280, k) for m in (385, 1600, 1601) for k in (8, 64, 72, 128, 136, 192, 200, 256, 264, 320, 328, 384, 392)]
 _RING_SHAPES += [(m, 1280, 840) for m in (31, 32, 33, 384, 768, 769, 1600, 1638, 1665)]
 # ... and one work-group per unit: 128 x 128 up to 256 tiles, 192 x 128 from there to 256 tiles; 64 x 128 and 128 x 128 beyond them and for `tt`
 _RING_SHAPES += [(1700, 1280, 1288), (3200, 1280, 840), (3201, 1280, 840), (3277, 1280, 1280), (4800, 1280, 1288), (4801, 1280, 840)]

@@ -541,6 +541,14 @@ def test_resample_short_rows_through_lds_and_past_its_limits(inner, ksize, shrin
     assert (got[:offset] == 9).all() and (got[offset + ref.size :] == 9).all()
 
 
+@pytest.mark.parametrize("ksize,shrink", [(1, 1.0), (9, 2.0), (13, 3.0)])
+@pytest.mark.parametrize("outer,offset", [(8217, 1), (8217, 3), (16384, 2)])
+def test_resample_of_three_channels_with_several_steps_of_rows_to_a_wave(ksize, shrink, outer, offset):
+    """More rows than one round of work-groups takes sixteen of: each wave goes on to further rows, at odd addresses, with a partial last step
+    and rows that are no whole words (393 bytes); bytes around the result are left alone."""
+    test_resample_short_rows_through_lds_and_past_its_limits(3, ksize, shrink, outer, offset)
+
+
 @pytest.mark.parametrize("outer,inner", [((1 << 29) + 100, 1), ((1 << 24) + 5, 8), ((1 << 24) + 5, 400)])
 def test_resample_of_more_work_groups_than_a_launch_takes(outer, inner):
     """A launch takes fewer than 2^24 work-groups of 256 threads; longer passes go in several.  One tap of weight one: a copy."""
