@@ -507,9 +507,9 @@ __global__ __launch_bounds__(256) void segment_copy_kernel(const W* __restrict__
 // A work-group moves one 32 KiB piece; every thread has eight independent 16-byte loads in flight.  HBM-bound.
 // A launch's loads and stores carry the non-temporal hint by what it moves in all (COPY_NT_LOADS, COPY_NT_STORES): a source that
 // is read once only pushes the destination out of the 256 MB memory-side cache, and a destination that fills most of it is gone
-// before its reader comes.  Split over ranks and put together again, us plain / with the hint: 320 MiB 248 / 210 (four ranks),
-// 240 MiB 178 / 149 (two ranks).  Smaller launches find their source in that cache: 39 MiB 33.4 / 36.6 with hinted loads, 40 MiB
-// a rank 51.6 / 56; stores with the hint at 120 MiB a rank 160 instead of 149.
+// before its reader comes.  us of a copy and a copy of the result, 16 ranges, plain / hinted loads / both hints: 64 MiB 48.6 / 46.6 / -, 72 57.2 / 51.4 / -,
+// 96 75.1 / 69.3 / 70.3, 128 107 / 87.8 / 90.5, 144 115 / 102 / 100, 160 121 / 113 / 110, 192 144 / 133 / 131, 256 190 / 170 / 172, 320 239 / 227 / 213.  Below 64 MiB hinted loads gain or lose
+// with the pattern, so there they are plain: these pairs 48 MiB 42.1 / 37.5, split over ranks and put together again 39 MiB 33.4 / 36.6, 40 MiB a rank 51.6 / 56.
 constexpr int COPY_MAX_RANGES = 96, COPY_STEPS = 8, COPY_PIECE = 256 * COPY_STEPS;  // words per piece
 constexpr int64_t COPY_NT_LOADS = 64ll << 20, COPY_NT_STORES = 160ll << 20;         // bytes of a launch
 struct CopyRanges {

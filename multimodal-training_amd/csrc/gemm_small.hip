@@ -498,17 +498,21 @@ __device__ __forceinline__ void gemm_small_tile(const GemmParams& p, const unsig
 }
 
 // A wave beside the others that reads two bytes of every 64 of B's part of its tile column, as fast as memory gives them: of the K tiles,
-// tile row tm takes every tiles_m-th, so that together they run ahead of the main loops, which then find B in the memory-side cache.
+// tile row tm takes every tiles_m-th, so that together they bring all of it into the memory-side cache, where the main loops find it.  It passes no
+// barrier, and the first barrier of the main loop waits until it has ended: the reading lies in front of the loops (beside the first loads of
+// their rings), which is why it has to be short.
 // For launches that have units to themselves: there a unit's requests in flight bound the main loop, the more the further away its
-// operands are.  us without / with, weights from HBM, 1280 columns, K = 6912, 3840, 3456 and 1280: 32 x 64, 256 rows 28.5, 18.0, 14.5, 8.1 / 24.8,
-// 15.2, 12.0, 7.8; 64 x 64, 704 rows 34.2, 21.5, 18.6, 9.5 / 29.0, 17.4, 14.8, 8.6; 64 x 128, 1,600 rows 44.8, 27.9, 25.6, 12.2 / 37.8, 22.9, 20.8, 10.9;
-// 128 x 128, 2,048 rows 59.1, 36.6, 34.7, 15.6 / 51.3, 30.8, 27.2, 14.4, 3,136 rows 56.8, 34.3, 33.3, 15.2 / 57.7, 33.8, 32.0, 14.8.  Not on 192 x 128
+// operands are.  us without / with, weights from HBM, input gradients of 1280 columns, K = 6912, 3840, 3456 and 1280: 32 x 64, 256 rows 29.6, 17.8, 16.4, 8.0 / 25.0,
+// 14.9, 13.9, 7.9; 64 x 64, 768 rows 35.7, 21.2, 19.5, 9.3 / 29.5, 17.7, 16.2, 8.6; 64 x 128, 1,600 rows 45.8, 27.3, 25.0, 11.8 / 38.6, 24.0, 22.1, 11.1;
+// 128 x 128, 2,048 rows 60.4, 35.7, 32.6, 15.2 / 51.4, 30.9, 28.5, 14.5, 3,136 rows 58.4, 34.7, 31.2, 15.6 / 58.5, 34.8, 32.0, 15.9.  Where the weights are in the
+// memory-side cache already (towers of some six blocks and fewer; a launch does not know) the reading is for nothing: K = 3456 / 1280 32 x 64 11.9, 6.6 / 13.2, 7.4, 64 x 64 14.4,
+// 7.5 / 16.1, 8.4, 64 x 128 20.2, 10.0 / 22.4, 10.7.  Not on 192 x 128
 // (4,096 rows 67.8, 40.2, 38.0, 17.5 / 70.7, 41.2, 38.8, 18.0) nor where two work-groups share a unit (1,024 rows on 64 x 64 43.3 / 46.1), nor for fewer than
-// four tile rows, whose waves would have too much to read (encoding 64 patches 2.32 / 2.67 ms; 128 rows 28.9, 18.5, 14.6, 8.2 / 28.3, 16.9, 13.4, 8.1),
+// four tile rows, whose waves would have too much to read (encoding 64 patches 2.32 / 2.67 ms; 128 rows, four of 32 x 64, 30.5, 18.4, 16.9, 8.2 / 28.3, 16.9, 15.8, 8.2),
 // nor on SwiGLU, which loses more than it gains (K = 1280, two of 3456 columns: 64 x 128, 200 rows 13.6 / 15.8, 256 14.7 / 15.8; 128 x 128, 448 rows
 // 18.5 / 19.1, 512 18.7 / 18.0), nor on SwiGLU backward (K = 1280, 3456 columns: 64 x 64, 200 rows 9.7 / 10.5, 224 10.5 / 10.6, 256 11.0 / 10.8, with the weights in the caches
-// 9.1 / 10.2, - , 9.2 / 10.4; 64 x 128, 513 rows 14.8 / 16.3, 576 15.4 / 16.5; its kernel keeps the branch to the wave, without which it takes 10.1, 10.8, 11.4 / 15.1, 15.8), nor beside a second stream (ms per step without / with in the backward: 1,600 rows 14.14 / 13.81, 1,936 15.32 / 15.54, 2,600 18.83 / 18.91; checkpointed
-// 1,600 16.55 / 16.65, 1,936 18.38 / 18.56).
+// 200 rows 9.1 / 10.2, 256 9.2 / 10.4; 64 x 128, 513 rows 14.8 / 16.3, 576 15.4 / 16.5; its kernel keeps the branch to the wave, without which it takes 10.1, 10.8, 11.4 / 15.1, 15.8), nor
+// beside a second stream (ms per step without / with in the backward: 1,600 rows 14.14 / 13.81, 1,936 15.32 / 15.54, 2,600 18.83 / 18.91; checkpointed 1,600 16.55 / 16.65, 1,936 18.38 / 18.56).
 template <bool TA, int EPI, typename S>
 constexpr bool TOUCHES = !TA && S::BM < 192 && EPI != MVIT_EPI_SWIGLU;
 template <bool TB, typename S>

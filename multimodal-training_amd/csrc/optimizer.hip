@@ -1,6 +1,10 @@
 // Multi-tensor Adam step and gradient sum of squares for gfx950: one launch over every parameter tensor
-// instead of several launches (and one host read-back) per tensor.  Both kernels are HBM-bound streams, of gigabytes that are not
-// read again before the next step: non-temporal loads, and stores of the moments.
+// instead of several launches (and one host read-back) per tensor.  Both kernels are HBM-bound streams, of gigabytes for the full tower, so
+// their loads and the stores of the moments carry the non-temporal hint.  Adam reads the gradients again behind the norm, and a small tower's state
+// fits the memory-side cache (256 MB), but the hints cost nothing there that matters.  us of norm + step from the host, bf16 gradients of 32 / 64 / 128 / 192 / 256 /
+// 512 MB: just written, plain 223 - 232 / 268 - 273 / 370 - 378 / 484 - 487 / 597 - 602 / 1,092 - 1,100, plain in the norm only 222 - 224 / 264 - 269 / 360 - 365 / 453 - 459 / 566 - 571 / 1,061 - 1,071,
+// hints throughout 215 - 223 / 265 - 271 / 365 - 375 / 458 - 469 / 556 - 566 / 1,004 - 1,011; left over from the step before, plain 191 / 241 / 369 / 492 / 612 / 1,076, hints throughout
+// 196 / 239 / 329 / 441 / 575 / 1,021.
 //
 // Work is cut into chunks of CHUNK elements that never straddle two tensors; chunk c belongs to the tensor t
 // with tensors[t].first_chunk <= c < tensors[t + 1].first_chunk (binary search by the block, the table has one
