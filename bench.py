@@ -121,7 +121,7 @@ def summarise_trace(records, cfg_kw, dtype):
 
 
 def measured_traffic_bytes(workload: str, tag: str):
-    """HBM bytes per launch of a kernel group, as measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE (two runs,
+    """Bytes per launch of a kernel group between the L2s and the memory side, as measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE (two runs,
     each scaled by what the same counter reads for a 1 GiB device copy).  The figures live with the counter summaries
     they come from: a line ``traffic_bytes_per_launch <workload> <trace tag> <bytes>`` in a text file under profiles/.
     None when no summary holds such a line."""
