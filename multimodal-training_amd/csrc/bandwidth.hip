@@ -952,11 +952,11 @@ int mvit_await_host_values(const int64_t* values, int n, mvit_stream_t stream) {
   for (;;) {
     if (const int rc = mvit_wait_host_values(values, n, 100 * 1000); rc != 1) return rc;
     const hipError_t e = hipStreamQuery(S_(stream));
+    (void)hipGetLastError();  // reported here, not by the next launch
     if (e != hipErrorNotReady) {
       if (mvit_wait_host_values(values, n, 0) == MVIT_OK) return MVIT_OK;
       return mvit_set_error(MVIT_ERR_LAUNCH, "await_host_values: %s", e == hipSuccess ? "the stream has ended without them" : hipGetErrorString(e));
     }
-    (void)hipGetLastError();  // not an error of the next launch
   }
 }
 
