@@ -206,6 +206,43 @@ def test_one_call_per_block_equals_the_call_by_call_sequence(dtype, checkpoint):
             assert torch.equal(grads[k], ref_grads[k]), (key, k)
 
 
+@pytest.mark.parametrize("checkpoint", [False, True])
+def test_weight_gradients_of_many_rows_are_the_same_bits_however_they_are_sent(checkpoint):
+    """From 12,000 rows of the tower's width on the weight gradients of a block are one launch that deals them out evenly: from one call per block
+    and call by call, on the second stream and in line, on two passes (buffers are recycled); and the gradients are those of the same rows in
+    launches of their own within the roundings of bf16."""
+    from mi355_vit import functional, ops
+
+    kw = dict(depth=1, hidden_size=1280, intermediate_size=3420, num_heads=16, out_hidden_size=256, fullatt_block_indexes=[])
+    grid = torch.tensor([[1, 110, 110]])
+    g = torch.Generator().manual_seed(13)
+    pixels, gout = torch.randn(12100, 1176, generator=g), torch.randn(12100 // 4, 256, generator=g)
+    assert ops.block_wgrads_together(torch.bfloat16, torch.bfloat16, 12100, 1280, 3420, 3456)
+    res = {}
+    old = functional.BLOCK_CALLS, ops.OVERLAP_WGRAD, ops.block_wgrads_together
+    try:
+        for one_call, overlap, together in ((True, True, True), (True, False, True), (False, True, True), (False, False, True), (False, False, False)):
+            functional.BLOCK_CALLS, ops.OVERLAP_WGRAD = one_call, overlap
+            ops.block_wgrads_together = old[2] if together else lambda *_: False
+            model = _build(kw, 7, torch.bfloat16)
+            if checkpoint:
+                model.gradient_checkpointing_enable()
+            _run_gpu(model, pixels, grid, gout)
+            for p_ in model.parameters():
+                p_.grad = None
+            res[(one_call, overlap, together)] = _run_gpu(model, pixels, grid, gout)
+    finally:
+        functional.BLOCK_CALLS, ops.OVERLAP_WGRAD, ops.block_wgrads_together = old
+    ref_out, ref_grads = res[(True, True, True)]
+    for key, (out, grads) in res.items():
+        assert torch.equal(out, ref_out), key
+        for k in ref_grads:
+            if key[2]:
+                assert torch.equal(grads[k], ref_grads[k]), (key, k)
+            else:  # both are sums in fp32, rounded to bf16 once: a unit in the last place where they fall to different sides
+                assert (grads[k].double() - ref_grads[k].double()).norm() <= 2.0**-8 * ref_grads[k].double().norm(), k
+
+
 _FEW_ROWS = ([[1, 2, 2]], [[1, 6, 10]], [[1, 16, 16], [1, 2, 6]], [[1, 32, 40]], [[1, 32, 40], [1, 2, 2]])
 
 
