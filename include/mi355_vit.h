@@ -261,7 +261,8 @@ int mvit_attn_bwd(const void* q, const void* k, const void* v, const void* o, co
  *            q_lead_scale = head_dim^-1/2 * log2 e applied to the queries in the rotary pass, attn_scale = 1 / log2 e
  *   forward  x [S,C] in; written: n1 [S,C], rstd1 [S], qkv [S,3C], o [S,C] and lse [nheads,S] (read instead when
  *            skip_attention != 0: the re-run of a checkpointed block that kept them), x1 [S,C], n2 [S,C], rstd2 [S],
- *            gu [S,2*Ipad] (null: not saved, for a forward that will not be differentiated), h [S,Ipad],
+ *            gu [S,2*Ipad] (null: not saved, for a forward that will not be differentiated; q and k in qkv are then scratch,
+ *            rotated or not), h [S,Ipad],
  *            x2 [S,C] (null: the down projection is skipped, for a re-run whose output nobody reads)
  *   backward reads x and everything the forward wrote (gu required) plus dx2 [S,C]; writes dx [S,C], the parameter
  *            gradients in `grad_dtype` laid out like the weights (g_wdown [C, I] without padding), and uses dgu

@@ -461,6 +461,191 @@ __global__ __launch_bounds__(64 * NWAVES, MINW) void attn_fwd_mfma(const AttnPar
 }
 
 // ================================================================================================
+// Windows (at most 64 tokens), forward, with the rotary embedding of q and k inside: the pass of its own reads and writes both once more.
+// A thread owns eight columns of the first half of a head and the matching eight of the second in one row, so ND waves rotate and four of
+// them compute.  Rounded where the separate passes round (rotation to bf16, then the attention of attn_fwd_mfma): the same bits.
+// Bound by the chain load -> rotation -> products -> store, i.e. by the work-groups that a unit holds, where q, k and v come from the memory-side
+// cache, and by memory beyond (1,006 MB at 65,536 rows x 16 heads where the rotated values are kept for a backward, else 671).  So two forms:
+// * one head to a work-group, 72 registers and 32 KiB, five of them to a unit;
+// * LOOP: `heads` heads of a window one after the other, the tables' part of a thread in registers for all of them, the next head's q, k and v
+//   travelling while the four waves multiply: 136 registers, two work-groups to a unit.
+// us, rotation in a pass of its own (rope_vec_kernel, attn_fwd_mfma) / one head, kept, not kept / LOOP, two heads, kept, four, not kept.  Operands from HBM:
+// 4,096 rows 23.8 / 19.8, 15.3 / 21.3, 14.6; 14,336 66.5 / 65.8, 44.4 / 60.6, 43.7; 25,524 116 / 115, 75.5 / 108, 75.3; 65,536 301 / 293, 192 / 259, 175.  In the caches:
+// 1,024 rows 7.8, 7.3 / 7.4, 9.8; 2,304 9.8, 7.7 / 12.5, 10.3; 4,360 15.8, 12.7 / 20.0, 19.9; 14,336 40.5, 31.4 / 47.0, 37.1.
+// Measured and not kept: half of the table registers (the tables' halves are alike as a rule, but the caller need not give such) 262 and 169 at
+// 65,536; three work-groups of LOOP by spilling 286 and 199.
+struct WindowRope {
+  const float *cos, *sin;
+  float q_gain;
+  int heads, keep, n_seg, parts;
+};
+template <int ND, bool LOOP>
+__global__ __launch_bounds__(64 * ND, LOOP ? 3 : 5) void attn_fwd_window_rope(const AttnParams p, const WindowRope w) {
+  using G = Geo<ND>;
+  static_assert(G::TAIL16 && ND >= 4, "four computing waves; the stabiliser in the spare slots");
+  constexpr int HD = G::HD, NT = 64 * ND, KT = 4, KK = 2, HALF = HD / 2;
+  __shared__ __attribute__((aligned(16))) bf16_t lds_q[64 * G::PK], lds_k[64 * G::PK], lds_v[64 * G::PV];
+
+  // work items are dealt so that all heads of a window meet on one XCD (seg_and_head)
+  int seg = blockIdx.x / w.parts, part = blockIdx.x % w.parts;
+  const unsigned items = (unsigned)w.n_seg * (unsigned)w.parts;
+  if (items % 8 == 0) {
+    const unsigned item = (blockIdx.x & 7) * (items >> 3) + (blockIdx.x >> 3);
+    seg = item / w.parts;
+    part = item % w.parts;
+  }
+  if (p.order) {
+    const int listed = p.order[seg];
+    if ((unsigned)listed < (unsigned)w.n_seg) seg = listed;  // an entry outside the list never becomes an address
+  }
+  const int s0 = p.cu[seg], L = min(p.cu[seg + 1] - s0, 64);
+  if (L <= 0) return;
+  const int t = threadIdx.x, l = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), g = l >> 4, r = l & 15;
+  const int row = t / ND, ch = t % ND;  // this thread's pair of chunks of q and k
+  const int vrow = t / G::CH, vch = t % G::CH;  // and its chunks of v: rows vrow and vrow + 32
+  const bool valid = row < L;
+  // one row pitch for q, k and v; 32-bit byte offsets of the lane from uniform addresses
+  const int64_t first = (int64_t)s0 * p.q_stride + (int64_t)part * w.heads * HD;
+  char* const Q = static_cast<char*>(const_cast<void*>(p.q)) + 2 * first;
+  char* const K = static_cast<char*>(const_cast<void*>(p.k)) + 2 * first;
+  const char* const V = static_cast<const char*>(p.v) + 2 * first;
+  const unsigned at_qk = (unsigned)((row * p.q_stride + ch * 8) * 2), at_v = (unsigned)((vrow * p.q_stride + vch * 8) * 2);
+  auto vec = [](char* base, unsigned at) -> bf16x8& { return *reinterpret_cast<bf16x8*>(base + at); };
+  bf16x8 q0, q1, k0, k1, v0, v1;
+  const bf16x8 zero = {};
+  auto load = [&](int j) {
+    q0 = q1 = k0 = k1 = v0 = v1 = zero;
+    if (valid) {
+      q0 = vec(Q + j * 2 * HD, at_qk);
+      q1 = vec(Q + j * 2 * HD + 2 * HALF, at_qk);
+      k0 = vec(K + j * 2 * HD, at_qk);
+      k1 = vec(K + j * 2 * HD + 2 * HALF, at_qk);
+    }
+    if (vrow < L) v0 = vec(const_cast<char*>(V) + j * 2 * HD, at_v);
+    if (vrow + 32 < L) v1 = vec(const_cast<char*>(V) + 64 * p.q_stride + j * 2 * HD, at_v);
+  };
+  load(0);
+  float c0[8], c1[8], sn0[8], sn1[8];
+  {
+    const int64_t at = (int64_t)(s0 + (valid ? row : 0)) * HD + ch * 8;
+    auto fetch = [&](const float* table, float (&to)[8]) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(table + at), b = *reinterpret_cast<const f32x4*>(table + at + 4);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) to[j] = a[j], to[4 + j] = b[j];
+    };
+    fetch(w.cos, c0);
+    fetch(w.cos + HALF, c1);
+    fetch(w.sin, sn0);
+    fetch(w.sin + HALF, sn1);
+  }
+  auto rotate = [&](bf16x8& a, bf16x8& b, float gain) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float oa, ob;
+      rope_pair((float)a[j], (float)b[j], c0[j], c1[j], sn0[j], sn1[j], 0, oa, ob);
+      a[j] = (bf16_t)(oa * gain);
+      b[j] = (bf16_t)(ob * gain);
+    }
+  };
+  const float c = p.scale * LOG2E;
+  bf16x8 ones;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) ones[j] = (bf16_t)1.f;
+  const bf16_t one_x = (bf16_t)(g == 0 ? 1.f : 0.f);
+  const int q_first = wv * 16, qi = q_first + r;
+
+  for (int j = 0; j < (LOOP ? w.heads : 1); ++j) {
+    rotate(q0, q1, w.q_gain);
+    rotate(k0, k1, 1.f);
+    if (j > 0) __syncthreads();  // the previous head's tiles have been used
+    *reinterpret_cast<bf16x8*>(lds_q + row * G::PK + ch * 8) = q0;
+    *reinterpret_cast<bf16x8*>(lds_q + row * G::PK + HALF + ch * 8) = q1;
+    *reinterpret_cast<bf16x8*>(lds_k + row * G::PK + ch * 8) = k0;
+    *reinterpret_cast<bf16x8*>(lds_k + row * G::PK + HALF + ch * 8) = k1;
+    *reinterpret_cast<bf16x8*>(lds_v + vrow * G::PV + vch * 8) = v0;
+    *reinterpret_cast<bf16x8*>(lds_v + (vrow + 32) * G::PV + vch * 8) = v1;
+    if (w.keep && valid) {
+      vec(Q + j * 2 * HD, at_qk) = q0;
+      vec(Q + j * 2 * HD + 2 * HALF, at_qk) = q1;
+      vec(K + j * 2 * HD, at_qk) = k0;
+      vec(K + j * 2 * HD + 2 * HALF, at_qk) = k1;
+    }
+    if (LOOP && j + 1 < w.heads) load(j + 1);
+    __syncthreads();
+    if (wv >= 4 || q_first >= L) {
+      if (!LOOP) return;
+      continue;
+    }  // for the whole wave; it meets the others at the barriers
+
+    RowFrag<ND> qf;
+    load_rowfrag_lds<ND, G::PK>(qf, lds_q, qi, g);
+    scale_rowfrag<ND>(qf, c);
+    f32x4 s[KT];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) {
+      RowFrag<ND> kf;
+      load_rowfrag_lds<ND, G::PK>(kf, lds_k, kt * 16 + r, g);
+      s[kt] = dot_frag_plus<ND>(kf, qf, one_x, (bf16_t)0.f);
+    }
+    if (L < 64) {
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (kt * 16 + 4 * g + i >= L) s[kt][i] = -INFINITY;
+    }
+    float mx = fmaxf(s[0][0], s[0][1]);
+    mx = max3(mx, s[0][2], s[0][3]);
+#pragma unroll
+    for (int kt = 1; kt < KT; ++kt) {
+      mx = max3(mx, s[kt][0], s[kt][1]);
+      mx = max3(mx, s[kt][2], s[kt][3]);
+    }
+    const float m = (float)(bf16_t)quad_max(mx);
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[kt][i] = __builtin_amdgcn_exp2f(s[kt][i] - m);
+    bf16x8 pb[KK];
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) pb[kk] = pack8(s[2 * kk], s[2 * kk + 1]);
+    f32x4 o[ND], sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) {
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt) {
+        const bf16_t* a0 = lds_v + ((2 * kk) * 16 + 4 * g + (r >> 2)) * G::PV + 16 * dt + 4 * (r & 3);
+        o[dt] = mfma32(tr_pair(a0, a0 + 16 * G::PV), pb[kk], o[dt]);
+      }
+      sum = mfma32(ones, pb[kk], sum);
+    }
+    // the wave's own rows of the q tile, which no other wave reads, turn the results into whole chunks of rows
+    const float inv = 1.f / sum[0];
+    bf16_t* turn = lds_q + q_first * G::PK;
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt) {
+      bf16x4 ov;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) ov[i] = (bf16_t)(o[dt][i] * inv);
+      *reinterpret_cast<bf16x4*>(turn + r * G::PK + 16 * dt + 4 * g) = ov;
+    }
+    const int h = part * w.heads + j;
+    if (g == 0 && qi < L) p.lse[(int64_t)h * p.total + s0 + qi] = (m + __builtin_amdgcn_logf(sum[0])) * LN2;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    bf16_t* O = static_cast<bf16_t*>(p.out) + (int64_t)(s0 + q_first) * p.o_stride + (int64_t)h * HD;
+#pragma unroll
+    for (int i = 0; i < (16 * G::CH + 63) / 64; ++i) {
+      const int at = l + 64 * i, rr = at / G::CH, cc = at % G::CH;
+      if (rr < 16 && q_first + rr < L) *reinterpret_cast<bf16x8*>(O + (int64_t)rr * p.o_stride + cc * 8) = *reinterpret_cast<const bf16x8*>(turn + rr * G::PK + cc * 8);
+    }
+  }
+}
+
+// ================================================================================================
 // Long segments, "wide" kernels: a wave owns 64 rows (two 32-row blocks), four waves per work-group, one
 // work-group per CU (up to 512 registers per lane).  Products whose contraction runs over head_dim use
 // v_mfma_f32_32x32x16_bf16, so head_dim = 16 * ND is contracted exactly (80 = 5 x 16, no padding); products whose
@@ -2089,6 +2274,29 @@ bool strided_rows_overlap(const void* a, int64_t pa, const void* b, int64_t pb, 
 }
 
 }  // namespace
+
+bool mvit_window_rope_takes(const mvit_window_rope& w, int head_dim, int max_seqlen, int dtype) {
+  return dtype == MVIT_BF16 && head_dim == 80 && max_seqlen > 0 && max_seqlen <= 64 && w.n_seg > 0 && w.nheads > 0 && (int64_t)w.n_seg * w.nheads < (1ll << 31) && w.S > 0 &&
+         mvit_aligned16(w.qkv) && mvit_aligned16(w.o) && mvit_aligned16(w.cos) && mvit_aligned16(w.sin);
+}
+int mvit_attn_fwd_window_rope(const mvit_window_rope& w, hipStream_t stream) {
+  const int64_t C = (int64_t)w.nheads * 80;
+  AttnParams p = {};
+  bf16_t* qkv = static_cast<bf16_t*>(w.qkv);
+  p.q = qkv; p.k = qkv + C; p.v = qkv + 2 * C; p.out = w.o; p.lse = w.lse; p.cu = w.cu; p.order = w.order; p.total = w.S; p.nheads = w.nheads;
+  p.q_stride = p.k_stride = p.v_stride = 3 * C; p.o_stride = C; p.scale = w.attn_scale;
+  WindowRope r{w.cos, w.sin, w.q_gain, 1, w.keep ? 1 : 0, w.n_seg, w.nheads};
+  // LOOP once q, k and v are more than stays in the memory-side cache (256 MB) between the product that writes them and this
+  const bool loop = w.S * 3 * C * 2 > (160ll << 20);
+  const int most = !loop ? 1 : w.keep ? 2 : 4;
+  while (2 * r.heads <= most && w.nheads % (2 * r.heads) == 0) r.heads *= 2;
+  r.parts = w.nheads / r.heads;
+  const unsigned items = (unsigned)w.n_seg * (unsigned)r.parts;
+  if (r.heads > 1) hipLaunchKernelGGL((attn_fwd_window_rope<5, true>), items, 320, 0, stream, p, r);
+  else hipLaunchKernelGGL((attn_fwd_window_rope<5, false>), items, 320, 0, stream, p, r);
+  MVIT_CHECK_LAUNCH("attn_fwd_window_rope");
+  return MVIT_OK;
+}
 
 extern "C" {
 

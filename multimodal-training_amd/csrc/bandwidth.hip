@@ -393,16 +393,6 @@ __global__ __launch_bounds__(256) void colsum_kernel(const T* __restrict__ x, in
 }
 
 // ------------------------------------------------------------------------------------------------
-__device__ __forceinline__ void rope_pair(float a, float b, float c0, float c1, float s0, float s1, int backward, float& oa, float& ob) {
-  if (!backward) {
-    oa = a * c0 - b * s0;
-    ob = b * c1 + a * s1;
-  } else {
-    oa = a * c0 + b * s1;
-    ob = b * c1 - a * s0;
-  }
-}
-
 // Rotary embedding in place.  A thread owns V consecutive elements of the first half of one head and
 // the matching V of the second half.  Algorithmic bytes per (row, head): 2*head_dim*e + table share.
 // The first `lead_heads` heads are multiplied by `lead_scale` before the one rounding to the storage type (the

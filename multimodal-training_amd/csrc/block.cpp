@@ -153,9 +153,12 @@ extern "C" int mvit_block_fwd(const mvit_block_args* a, mvit_stream_t stream) {
     g.A = a->n1; g.lda = C; g.B = a->wqkv; g.ldb = C; g.bias = a->bqkv; g.C = a->qkv; g.ldc = 3 * C;
     STEP(mvit_gemm(&g, stream));
   }
-  // rotary embedding of q and k in place; the queries also take the softmax scale in base-2 units
-  STEP(mvit_rope_scaled(a->qkv, a->cos, a->sin, S, 2 * H, hd, 3 * C, 0, H, a->q_lead_scale, dt, stream));
-  if (!a->skip_attention)
+  // rotary embedding of q and k in place; the queries also take the softmax scale in base-2 units.  Windows: inside their attention
+  const mvit_window_rope rotated{a->qkv, a->o, a->lse, a->cu, a->seg_order, a->cos, a->sin, a->n_seg, H, S, a->q_lead_scale, a->attn_scale, a->gu != nullptr};
+  const bool inside = !a->skip_attention && mvit_window_rope_takes(rotated, hd, a->max_seqlen, dt);
+  if (inside) STEP(mvit_attn_fwd_window_rope(rotated, reinterpret_cast<hipStream_t>(stream)));
+  else STEP(mvit_rope_scaled(a->qkv, a->cos, a->sin, S, 2 * H, hd, 3 * C, 0, H, a->q_lead_scale, dt, stream));
+  if (!a->skip_attention && !inside)
     STEP(mvit_attn_fwd(a->qkv, at(a->qkv, C, dt), at(a->qkv, 2 * C, dt), a->o, a->lse, a->cu, a->seg_order, a->n_seg, a->max_seqlen, S, H, hd,
                        3 * C, 3 * C, 3 * C, C, a->attn_scale, dt, stream));
   {  // x1 = x + o . Wproj^T + b

@@ -42,6 +42,20 @@ int mvit_set_error(int code, const char* fmt, ...);
 static inline bool mvit_aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Launches that several steps of a block share (block.cpp).
+// Attention over windows of at most 64 tokens with the rotary embedding of q and k inside (bf16, head_dim 80; qkv [S, 3 * nheads * 80]).  The rotated
+// q and k replace the others in qkv where `keep` is set.  `mvit_window_rope_takes`: whether a block's tensors suit it.
+struct mvit_window_rope {
+  void *qkv, *o;
+  float* lse;
+  const int32_t *cu, *order;
+  const float *cos, *sin;
+  int n_seg, nheads;
+  int64_t S;
+  float q_gain, attn_scale;
+  bool keep;
+};
+bool mvit_window_rope_takes(const mvit_window_rope& w, int head_dim, int max_seqlen, int dtype);  // attention.hip
+int mvit_attn_fwd_window_rope(const mvit_window_rope& w, hipStream_t stream);                     // attention.hip
 int mvit_gemm_wgrad_group(const mvit_gemm_args* list, int n, hipStream_t stream);  // gemm.hip
 struct mvit_partials {  // out[c] = the sum of n_partial rows of `cols` floats, in the order of mvit_reduce_partials
   const float* partial;
@@ -87,6 +101,17 @@ __device__ __forceinline__ float from_f32<float>(float v) {
 template <>
 __device__ __forceinline__ bf16_t from_f32<bf16_t>(float v) {
   return (bf16_t)v;  // round-to-nearest-even
+}
+
+// One pair of a rotary embedding, with the roundings spelled out: the passes of their own and the attention that rotates give the same bits
+__device__ __forceinline__ void rope_pair(float a, float b, float c0, float c1, float s0, float s1, int backward, float& oa, float& ob) {
+  if (!backward) {
+    oa = __builtin_fmaf(a, c0, -(b * s0));
+    ob = __builtin_fmaf(b, c1, a * s1);
+  } else {
+    oa = __builtin_fmaf(a, c0, b * s1);
+    ob = __builtin_fmaf(b, c1, -(a * s0));
+  }
 }
 
 // A vector that is not read again before it has left the caches anyway: it does not push out what is

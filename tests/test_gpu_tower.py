@@ -206,6 +206,41 @@ def test_one_call_per_block_equals_the_call_by_call_sequence(dtype, checkpoint):
             assert torch.equal(grads[k], ref_grads[k]), (key, k)
 
 
+@pytest.mark.parametrize("heads,rows,ragged,tables_alike", [(1, 1, False, True), (1, 64, False, False), (2, 77, True, True), (3, 500, True, False), (16, 256, False, True),
+                                                            (16, 4033, True, False), (16, 22000, False, True), (16, 22001, True, False), (6, 60000, True, True), (5, 70000, False, False)])
+def test_windows_with_the_rotation_inside_give_the_bits_of_two_passes(heads, rows, ragged, tables_alike):
+    """A windowed block behind one call rotates q and k inside its attention: output, attention output and log-sum-exp, and what a backward reads of
+    q, k and v, are those of the call-by-call sequence with its pass of its own; one, two and four heads to a work-group, windows of 1 to 64
+    tokens, rotary tables whose halves differ, with gradients to come and without."""
+    from mi355_vit import functional as F
+
+    C, I, g = 80 * heads, 128, torch.Generator().manual_seed(rows + heads)
+    lengths = []
+    left = rows
+    while left > 0:
+        lengths.append(min(left, int(torch.randint(1, 65, (1,), generator=g)) if ragged else 64))
+        left -= lengths[-1]
+    cu = torch.tensor([0] + lengths).cumsum(0).to(torch.int32).to(DEV)
+    angle = torch.randn(rows, 40, generator=g)
+    angle = torch.cat([angle, angle if tables_alike else angle + 1], 1).to(DEV)
+    geo = F.AttnGeometry(cu, max(lengths), heads, 80, angle.cos().contiguous(), angle.sin().contiguous())
+    r = lambda *shape: (torch.randn(*shape, generator=g) * 0.05).to(torch.bfloat16).to(DEV)  # noqa: E731
+    Ipad = F.padded_inner(I)
+    W = F.BlockWeights(r(1, C) + 1, r(1, C) + 1, r(3 * C, C), r(1, 3 * C), r(C, C), r(1, C), r(2 * Ipad, C), r(1, 2 * Ipad), r(C, Ipad), r(1, C), C, I, Ipad)
+    x, old = torch.randn(rows, C, generator=g).to(torch.bfloat16).to(DEV), F.BLOCK_CALLS
+    try:
+        for for_backward in (True, False):
+            F.BLOCK_CALLS = True
+            y, saved = F._block_forward(x, W, geo, 1e-6, for_backward=for_backward)
+            F.BLOCK_CALLS = False
+            want, want_saved = F._block_forward(x, W, geo, 1e-6, for_backward=for_backward)
+            assert torch.isfinite(want).all() and torch.equal(y, want)
+            for i in (2, 3, 4) if for_backward else (3, 4):
+                assert torch.equal(saved[i], want_saved[i]), (for_backward, i)
+    finally:
+        F.BLOCK_CALLS = old
+
+
 @pytest.mark.parametrize("checkpoint", [False, True])
 def test_weight_gradients_of_many_rows_are_the_same_bits_however_they_are_sent(checkpoint):
     """From 12,000 rows of the tower's width on the weight gradients of a block are one launch that deals them out evenly: from one call per block
