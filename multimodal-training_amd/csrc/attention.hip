@@ -1965,8 +1965,11 @@ __global__ __launch_bounds__(64 * NWAVES) void attn_bwd_dq_mfma(const AttnParams
 // Results are turned in LDS and leave as 16-byte chunks, a row's 160 bytes together: as 8-byte pieces of 32 bytes a row, straight from the accumulators,
 // they took twice the write requests.  us before / now, operands from HBM: 4,096 rows x 16 heads 27.8 / 25.0, 14,336 80 / 68, 25,524 128 / 108, 65,536 307 / 259
 // (4.5 TB/s).
-template <int ND, int NW, int MINW = 1>  // NW waves share the staged tiles; wave w owns query / key blocks [w*4/NW, (w+1)*4/NW)
-__global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const AttnParams p) {
+// ROPE: dQ and dK are turned back by the rotary embedding's angles on their way out (with the roundings of the pass of its own, which read and wrote both
+// once more); dQ waits in LDS for the tables, which are fetched once for both and travel while dK and dV are rounded.  ms per step, pass of its own /
+// inside: 1,024 rows 12.0 / 11.6, 4,096 checkpointed 27.9 / 27.6, 14,336 62.2 / 61.0, 25,524 104.9 / 104.3, 36,864 239.6 / 238.3.
+template <int ND, int NW, int MINW = 1, bool ROPE = false>  // NW waves share the staged tiles; wave w owns query / key blocks [w*4/NW, (w+1)*4/NW)
+__global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const AttnParams p, const WindowRope rope) {
   using G = Geo<ND>;
   constexpr int HD = G::HD, R = 64, PK = G::PK, NB = 4 / NW;  // NB 16-row blocks per wave
   __shared__ __attribute__((aligned(16))) bf16_t lds_q[R * PK];
@@ -1985,10 +1988,13 @@ __global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const Attn
   const float c = p.scale * LOG2E;
   static_assert(NB == 1, "a wave's sixteen rows of the k and v tiles are its own behind pass A");
   // results leave as whole chunks of rows: turned in the wave's own rows of a tile that no other wave reads any more
-  auto leave = [&](bf16_t* tile, const bf16x4 (&v)[ND], bf16_t* dst, int64_t stride) {
-    bf16_t* turn = tile + wv * 16 * PK;
+  auto turn_in = [&](bf16_t* tile, const bf16x4 (&v)[ND]) {
 #pragma unroll
-    for (int d = 0; d < ND; ++d) *reinterpret_cast<bf16x4*>(turn + r * PK + 16 * d + 4 * g) = v[d];
+    for (int d = 0; d < ND; ++d) *reinterpret_cast<bf16x4*>(tile + (wv * 16 + r) * PK + 16 * d + 4 * g) = v[d];
+  };
+  auto leave = [&](bf16_t* tile, const bf16x4 (&v)[ND], bf16_t* dst, int64_t stride) {
+    const bf16_t* turn = tile + wv * 16 * PK;
+    turn_in(tile, v);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -2105,7 +2111,8 @@ __global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const Attn
         dv[kb][d] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
     }
-    if (wv * 16 < L) leave(lds_v, dq_out, DQ, p.dq_stride);
+    if (!ROPE && wv * 16 < L) leave(lds_v, dq_out, DQ, p.dq_stride);
+    if (ROPE) turn_in(lds_v, dq_out);  // stays there until the tables are fetched, once for both
 #pragma unroll 1
     for (int qs = 0; qs < L; qs += 32) {
       const bf16_t* tq = lds_q + qs * PK;
@@ -2151,6 +2158,23 @@ __global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const Attn
     }
     bf16_t* DK = static_cast<bf16_t*>(p.dk) + (int64_t)s0 * p.dk_stride + (int64_t)h * HD;
     bf16_t* DV = static_cast<bf16_t*>(p.dv) + (int64_t)s0 * p.dv_stride + (int64_t)h * HD;
+    // ROPE: a lane takes eight columns of the first half of a head and the matching eight of the second; sixteen rows are 16 * ND such pairs
+    constexpr int HALF = HD / 2, PAIRS = ROPE ? (16 * ND + 63) / 64 : 0;
+    float c0[8], c1[8], sn0[8], sn1[8];
+    auto fetch = [&](int i) {
+      const int at = l + 64 * i, rr = at / ND, row = wv * 16 + rr;
+      const int64_t angle = (int64_t)(s0 + (rr < 16 && row < L ? row : 0)) * HD + at % ND * 8;
+      auto eight = [&](const float* table, float (&to)[8]) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(table + angle), y = *reinterpret_cast<const f32x4*>(table + angle + 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) to[j] = x[j], to[4 + j] = y[j];
+      };
+      eight(rope.cos, c0);
+      eight(rope.cos + HALF, c1);
+      eight(rope.sin, sn0);
+      eight(rope.sin + HALF, sn1);
+    };
+    if (ROPE) fetch(0);
     bf16x4 a[ND], b[ND];
 #pragma unroll
     for (int d = 0; d < ND; ++d)
@@ -2159,7 +2183,34 @@ __global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const Attn
         a[d][i] = (bf16_t)(dk[0][d][i] * LN2);  // dS^T (Q scale log2e) / log2e
         b[d][i] = (bf16_t)dv[0][d][i];
       }
-    leave(lds_k, a, DK, p.dk_stride);
+    if constexpr (!ROPE) {
+      leave(lds_k, a, DK, p.dk_stride);
+    } else {
+      turn_in(lds_k, a);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for (int i = 0; i < PAIRS; ++i) {
+        const int at = l + 64 * i, rr = at / ND, cc = at % ND, row = wv * 16 + rr;
+        if (i > 0) fetch(i);
+        if (rr >= 16 || row >= L) continue;
+        auto back = [&](const bf16_t* tile, bf16_t* dst, int64_t stride, float gain) {
+          bf16x8 lo = *reinterpret_cast<const bf16x8*>(tile + row * PK + cc * 8), hi = *reinterpret_cast<const bf16x8*>(tile + row * PK + HALF + cc * 8);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            float oa, ob;
+            rope_pair((float)lo[j], (float)hi[j], c0[j], c1[j], sn0[j], sn1[j], 1, oa, ob);
+            lo[j] = (bf16_t)(oa * gain);
+            hi[j] = (bf16_t)(ob * gain);
+          }
+          *reinterpret_cast<bf16x8*>(dst + (int64_t)row * stride + cc * 8) = lo;
+          *reinterpret_cast<bf16x8*>(dst + (int64_t)row * stride + HALF + cc * 8) = hi;
+        };
+        back(lds_v, DQ, p.dq_stride, rope.q_gain);
+        back(lds_k, DK, p.dk_stride, 1.f);
+      }
+    }
     leave(lds_v, b, DV, p.dv_stride);
   }
 }
@@ -2213,7 +2264,7 @@ int launch_bwd_mfma(const AttnParams& p, int n_seg, int max_seqlen, hipStream_t 
       // four waves x 16 rows: ~160 registers, three work-groups (12 waves) per CU to cover the load -> MFMA -> store latency
       AttnParams pw = p;
       if (((int64_t)n_seg * p.nheads) % 8 == 0) pw.seg_major = 2;  // heads of a segment together on one XCD
-      hipLaunchKernelGGL((attn_bwd_window_mfma<ND, 4, 2>), grid, 256, 0, s, pw);  // computes delta itself
+      hipLaunchKernelGGL((attn_bwd_window_mfma<ND, 4, 2>), grid, 256, 0, s, pw, WindowRope{});  // computes delta itself
     } else {
       hipLaunchKernelGGL((attn_bwd_dkdv_mfma<ND, 1, 4>), grid, 64, 0, s, p);
       hipLaunchKernelGGL((attn_bwd_dq_mfma<ND, 1, 4>), grid, 64, 0, s, p);
@@ -2284,7 +2335,7 @@ bool strided_rows_overlap(const void* a, int64_t pa, const void* b, int64_t pb, 
 }  // namespace
 
 bool mvit_window_rope_takes(const mvit_window_rope& w, int head_dim, int max_seqlen, int dtype) {
-  return dtype == MVIT_BF16 && head_dim == 80 && max_seqlen > 0 && max_seqlen <= 64 && w.n_seg > 0 && w.nheads > 0 && (int64_t)w.n_seg * w.nheads < (1ll << 31) && w.S > 0 &&
+  return dtype == MVIT_BF16 && head_dim == 80 && max_seqlen > 0 && max_seqlen <= 64 && w.n_seg > 0 && w.n_seg <= 65535 && w.nheads > 0 && w.nheads <= 65535 && w.S > 0 &&
          mvit_aligned16(w.qkv) && mvit_aligned16(w.o) && mvit_aligned16(w.cos) && mvit_aligned16(w.sin);
 }
 int mvit_attn_fwd_window_rope(const mvit_window_rope& w, hipStream_t stream) {
@@ -2303,6 +2354,20 @@ int mvit_attn_fwd_window_rope(const mvit_window_rope& w, hipStream_t stream) {
   if (r.heads > 1) hipLaunchKernelGGL((attn_fwd_window_rope<5, true>), items, 320, 0, stream, p, r);
   else hipLaunchKernelGGL((attn_fwd_window_rope<5, false>), items, 320, 0, stream, p, r);
   MVIT_CHECK_LAUNCH("attn_fwd_window_rope");
+  return MVIT_OK;
+}
+
+int mvit_attn_bwd_window_rope(const mvit_window_rope& w, const void* d_o, void* dqkv, float* delta, hipStream_t stream) {
+  const int64_t C = (int64_t)w.nheads * 80;
+  AttnParams p = {};
+  const bf16_t* qkv = static_cast<const bf16_t*>(w.qkv);
+  bf16_t* d = static_cast<bf16_t*>(dqkv);
+  p.q = qkv; p.k = qkv + C; p.v = qkv + 2 * C; p.d_o = d_o; p.lse = w.lse; p.delta = delta; p.dq = d; p.dk = d + C; p.dv = d + 2 * C;
+  p.cu = w.cu; p.order = w.order; p.total = w.S; p.nheads = w.nheads;
+  p.q_stride = p.k_stride = p.v_stride = p.dq_stride = p.dk_stride = p.dv_stride = 3 * C; p.o_stride = p.do_stride = C; p.scale = w.attn_scale;
+  if (((int64_t)w.n_seg * w.nheads) % 8 == 0) p.seg_major = 2;  // heads of a segment together on one XCD
+  hipLaunchKernelGGL((attn_bwd_window_mfma<5, 4, 2, true>), dim3(1, (unsigned)w.n_seg, (unsigned)w.nheads), 256, 0, stream, p, WindowRope{w.cos, w.sin, w.q_gain, 1, 0, w.n_seg, w.nheads});
+  MVIT_CHECK_LAUNCH("attn_bwd_window_rope");
   return MVIT_OK;
 }
 

@@ -217,6 +217,16 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   const int dt = a->dtype, gdt = a->grad_dtype;
   const int64_t S = a->S, C = a->C, I = a->I, Ipad = a->Ipad;
   const int H = a->nheads, hd = a->head_dim;
+  // windows: the inverse rotation of dq and dk is in their attention's backward
+  const mvit_window_rope rotated{a->qkv, a->o, a->lse, a->cu, a->seg_order, a->cos, a->sin, a->n_seg, H, S, a->q_lead_scale, a->attn_scale, true};
+  const bool inside = mvit_window_rope_takes(rotated, hd, a->max_seqlen, dt) && mvit_aligned16(a->dqkv) && mvit_aligned16(a->dn);
+  if (inside) {  // as mvit_attn_bwd asks of its outputs
+    const struct { const void* ptr; int64_t cols; const char* name; } ins[] = {{a->qkv, 3 * C, "qkv"}, {a->o, C, "o"}, {a->dn, C, "d_o"}};
+    for (const auto& r : ins) {
+      const char *out = static_cast<const char*>(a->dqkv), *in = static_cast<const char*>(r.ptr);
+      MVIT_REQUIRE(out + S * 3 * C * 2 <= in || in + S * r.cols * 2 <= out, "block_bwd: dqkv overlaps %s (outputs are written before all inputs have been read)", r.name);
+    }
+  }
   hipStream_t main_s = reinterpret_cast<hipStream_t>(stream), side_s = reinterpret_cast<hipStream_t>(a->side_stream);
 
   // Weight and bias gradients feed nothing else in the block: with a second stream they start there once their inputs
@@ -303,10 +313,11 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
     g.A = a->dx1; g.lda = C; g.B = a->wproj; g.ldb = C; g.C = a->dn; g.ldc = C;
     STEP(mvit_gemm(&g, stream));
   }
-  STEP(mvit_attn_bwd(a->qkv, at(a->qkv, C, dt), at(a->qkv, 2 * C, dt), a->o, a->dn, a->lse, a->dqkv, at(a->dqkv, C, dt), at(a->dqkv, 2 * C, dt),
+  if (inside) STEP(mvit_attn_bwd_window_rope(rotated, a->dn, a->dqkv, w.delta, main_s));
+  else STEP(mvit_attn_bwd(a->qkv, at(a->qkv, C, dt), at(a->qkv, 2 * C, dt), a->o, a->dn, a->lse, a->dqkv, at(a->dqkv, C, dt), at(a->dqkv, 2 * C, dt),
                      w.delta, w.delta_elems, a->cu, a->seg_order, a->n_seg, a->max_seqlen, S, H, hd, 3 * C, 3 * C, 3 * C, C, C, 3 * C, 3 * C, 3 * C,
                      a->attn_scale, dt, stream));
-  STEP(mvit_rope_scaled(a->dqkv, a->cos, a->sin, S, 2 * H, hd, 3 * C, 1, H, a->q_lead_scale, dt, stream));
+  if (!inside) STEP(mvit_rope_scaled(a->dqkv, a->cos, a->sin, S, 2 * H, hd, 3 * C, 1, H, a->q_lead_scale, dt, stream));
   {
     mvit_stream_t st = fork(3);
     if (!st && two) return MVIT_ERR_LAUNCH;

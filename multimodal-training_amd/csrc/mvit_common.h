@@ -56,6 +56,8 @@ struct mvit_window_rope {
 };
 bool mvit_window_rope_takes(const mvit_window_rope& w, int head_dim, int max_seqlen, int dtype);  // attention.hip
 int mvit_attn_fwd_window_rope(const mvit_window_rope& w, hipStream_t stream);                     // attention.hip
+// its backward: d_o [S, nheads * 80] -> dqkv [S, 3 * nheads * 80], from the rotated q and k; delta [nheads, S]
+int mvit_attn_bwd_window_rope(const mvit_window_rope& w, const void* d_o, void* dqkv, float* delta, hipStream_t stream);
 int mvit_gemm_wgrad_group(const mvit_gemm_args* list, int n, hipStream_t stream);  // gemm.hip
 struct mvit_partials {  // out[c] = the sum of n_partial rows of `cols` floats, in the order of mvit_reduce_partials
   const float* partial;

@@ -539,6 +539,25 @@ def test_weight_gradients_are_dealt_out_evenly_where_a_block_has_much_work():
         setattr(args[1], field, old)
 
 
+def test_windowed_backward_behind_one_call_refuses_gradients_that_share_memory():
+    """Windows of head_dim 80, whose dq and dk are turned back on their way out, refuse what mvit_attn_bwd refuses; nothing is launched."""
+    import ctypes
+
+    from mi355_vit import _lib
+
+    lib, fake, a = _lib.load(), 0x10000000, _lib.BlockArgs()
+    for name, kind in a._fields_:
+        if kind is ctypes.c_void_p:
+            setattr(a, name, fake)
+    a.dtype = a.grad_dtype = _lib.BF16
+    a.S, a.C, a.I, a.Ipad, a.nheads, a.head_dim, a.n_seg, a.max_seqlen, a.side_stream = 128, 320, 300, 304, 4, 80, 2, 64, None
+    a.split_k_down = a.split_k_gate_up = a.split_k_proj = a.split_k_qkv = 1
+    a.qkv, a.workspace_bytes = fake + (1 << 24), lib.mvit_block_bwd_workspace_bytes(ctypes.byref(a))
+    for shared, dqkv in (("qkv", a.qkv + 16), ("qkv", a.qkv - 16), ("o", fake)):
+        a.dqkv = dqkv
+        assert lib.mvit_block_bwd(ctypes.byref(a), None) == -1 and b"dqkv overlaps " + shared.encode() in lib.mvit_last_error()
+
+
 def _tile(rows, cols, k, trans_b=1, epilogue=0, overlapped=0):
     import ctypes
 

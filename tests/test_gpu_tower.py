@@ -209,8 +209,8 @@ def test_one_call_per_block_equals_the_call_by_call_sequence(dtype, checkpoint):
 @pytest.mark.parametrize("heads,rows,ragged,tables_alike", [(1, 1, False, True), (1, 64, False, False), (2, 77, True, True), (3, 500, True, False), (16, 256, False, True),
                                                             (16, 4033, True, False), (16, 22000, False, True), (16, 22001, True, False), (6, 60000, True, True), (5, 70000, False, False)])
 def test_windows_with_the_rotation_inside_give_the_bits_of_two_passes(heads, rows, ragged, tables_alike):
-    """A windowed block behind one call rotates q and k inside its attention: output, attention output and log-sum-exp, and what a backward reads of
-    q, k and v, are those of the call-by-call sequence with its pass of its own; one, two and four heads to a work-group, windows of 1 to 64
+    """A windowed block behind one call rotates q and k inside its attention, both ways: output, attention output and log-sum-exp, what a backward
+    reads of q, k and v, and its gradients are those of the call-by-call sequence with its pass of its own; one, two and four heads to a work-group, windows of 1 to 64
     tokens, rotary tables whose halves differ, with gradients to come and without."""
     from mi355_vit import functional as F
 
@@ -237,6 +237,12 @@ def test_windows_with_the_rotation_inside_give_the_bits_of_two_passes(heads, row
             assert torch.isfinite(want).all() and torch.equal(y, want)
             for i in (2, 3, 4) if for_backward else (3, 4):
                 assert torch.equal(saved[i], want_saved[i]), (for_backward, i)
+            if for_backward:  # the backward turns dq and dk back inside
+                kept, dy = tuple(want_saved), torch.randn(rows, C, generator=g).to(torch.bfloat16).to(DEV)
+                dx, grads = F._block_backward(dy, x, kept, W, geo, torch.bfloat16)  # call by call
+                F.BLOCK_CALLS = True
+                dx1, grads1 = F._block_backward(dy, x, kept, W, geo, torch.bfloat16)
+                assert torch.isfinite(dx).all() and torch.equal(dx1, dx) and all(torch.equal(a, b) for a, b in zip(grads1, grads))
     finally:
         F.BLOCK_CALLS = old
 
