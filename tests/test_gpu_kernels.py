@@ -491,6 +491,29 @@ def test_gemm_input_gradient_has_the_same_bits_beside_another_stream(M, N, K):
     assert max_rel_err(got[0][0][:M], dy.cpu().double() @ w.cpu().double()) < TOL[dtype]
 
 
+@pytest.mark.parametrize("gelu", [False, True])
+@pytest.mark.parametrize("M,N", [(4353, 3840), (13057, 1280), (14336, 1280)])
+def test_gemm_input_gradient_in_full_rounds_and_the_rest_has_the_bits_of_one_launch(M, N, gelu, monkeypatch):
+    """Input gradients that have the GPU to themselves go in two launches as well; the saved activations of the second are those of its rows."""
+    _announce(f"gemm input gradient, rows in full rounds M={M} N={N} gelu={gelu}")
+    ops = _ops()
+    from mi355_vit import _lib as E
+
+    K, dtype = 520, torch.bfloat16
+    dy, w, x = _rand((M, K), dtype, 1).to(DEV), _rand((K, N), dtype, 2, K**-0.5).to(DEV), _rand((M, N), dtype, 3).to(DEV)
+
+    def run():
+        out = torch.full((M + 8, N), 7.0, dtype=dtype, device=DEV)
+        ops.gemm(dy, w, out[:M], trans_b=True, **(dict(epilogue=E.EPI_GELU_BWD, residual=x) if gelu else {}))
+        return out
+
+    got = run()
+    monkeypatch.setenv("MVIT_GEMM_NO_HALF_TILES", "1")  # one launch of 256 x 256 tiles
+    assert torch.equal(got, run()) and bool((got[-8:] == 7.0).all())
+    if not gelu:
+        assert max_rel_err(got[:M], dy.cpu().double() @ w.cpu().double()) < TOL[dtype]
+
+
 @pytest.mark.parametrize("epi", ["none", "bias", "bias_res", "gelu", "swiglu", "swiglu without aux"])
 @pytest.mark.parametrize("M,N", [(4353, 3840), (4607, 3840), (13057, 1280), (14336, 1280)])
 def test_gemm_rows_in_full_rounds_and_the_rest_give_the_same_bits_as_one_launch(M, N, epi, monkeypatch):
