@@ -252,7 +252,8 @@ int mvit_attn_bwd(const void* q, const void* k, const void* v, const void* o, co
 /* Operands of one block (Qwen2_5_VLVisionBlock.forward, modeling:776-792, with _forward_standard :385-472 and the MLP
  * :203-204) for mvit_block_fwd / mvit_block_bwd: the fixed launch sequence of the block behind one call each way, for
  * hosts whose per-call cost would otherwise exceed the kernels' run time at small batches.  Every step is one of the
- * entry points above on these operands, so the results are those of the same sequence issued call by call.
+ * entry points above on these operands, or one kernel that gives the bits of two of them (windows of head_dim 80: rotation and
+ * attention), so the results are those of the same sequence issued call by call.
  * All tensors are contiguous, of `dtype` unless a float* says otherwise; all pointers are device pointers.
  *   weights  norm1, norm2 [C]; wqkv [3C, C], bqkv [3C] (q | k | v stacked); wproj [C, C], bproj [C];
  *            wgu [2*Ipad, C], bgu [2*Ipad] (gate rows [0, I), up rows [Ipad, Ipad+I), padding rows zero);

@@ -1,8 +1,8 @@
 // One transformer block of the vision tower behind a single C call each way: the fixed launch sequence of the block's
 // forward and of its backward (Qwen2_5_VLVisionBlock.forward, modeling_qwen2_5_vl.py:776-792, with _forward_standard
 // :385-472 and the MLP :203-204, and their autograd), issued from here instead of one host-language call per kernel.
-// Nothing is computed here: every step is one of the library's own entry points with the operands the caller laid out,
-// so the results are those of the same sequence issued call by call.  No allocation, no synchronisation; the only
+// Nothing is computed here: every step is one of the library's own entry points with the operands the caller laid out (or, for windows,
+// one kernel in the place of rotation and attention that rounds where they do), so the results are those of the same sequence issued call by call.  No allocation, no synchronisation; the only
 // streams and events used are the caller's.
 #include <math.h>
 #include <string.h>
