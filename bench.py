@@ -99,13 +99,12 @@ def summarise_trace(records, cfg_kw, dtype):
         if tag.startswith("gemm"):
             halves = 2.0 if tag.endswith("epi4") else 1.0  # SWIGLU: N counts one of the two weight matrices
             # M counts tokens, or features in a weight gradient, whose K counts tokens
-            for m, n in info.get("products") or [(info["M"], info["N"])]:
-                n, k = unpad.get(n, n), info["K"]
-                if tag.startswith("gemm_tt"):
-                    m = unpad.get(m, m)
-                else:
-                    k = unpad.get(k, k)
-                ent["flops"] += halves * 2.0 * m * n * k
+            m, n, k = info["M"], unpad.get(info["N"], info["N"]), info["K"]
+            if tag.startswith("gemm_tt"):
+                m = unpad.get(m, m)
+            else:
+                k = unpad.get(k, k)
+            ent["flops"] += halves * 2.0 * m * n * k
         elif tag.startswith("attn_fwd"):
             ent["flops"] += 4.0 * seg_sq_sum(info["cu"].cpu()) * info["head_dim"] * info["nheads"]
         elif tag.startswith("attn_bwd"):
@@ -146,7 +145,6 @@ KERNEL_NAMES = {
     "gemm_nt_epi0": "gemm_pp_kernel / gemm_small_kernel<TO, TA=false, TB=true, EPI=NONE>",
     "gemm_nt_epi5": "gemm_dl_kernel<TO, TA=false, TB=true, EPI=SWIGLU_BWD>",
     "gemm_nt_epi6": "gemm_pp_kernel / gemm_small_kernel<TO, TA=false, TB=true, EPI=GELU_BWD>",
-    "gemm_tt_together": "gemm_pp_wgrads_kernel + wgrads_reduce_kernel",
     "gemm_tt_epi0": "gemm_pp_kernel / gemm_small_kernel<TO, TA=true, TB=true, EPI=NONE> + splitk_reduce_kernel",
     "attn_fwd_full": "attn_fwd_x32<5> (segments >= 512 tokens), attn_fwd_mfma<5, 8, 32, true, 2, 4> (shorter)",
     "attn_bwd_full": "attn_delta_rows_kernel + attn_bwd_prepare_kernel + attn_bwd_dkdv_wide<5> + attn_bwd_dq_wide<5>",

@@ -33,14 +33,14 @@ typedef void* mvit_stream_t; /* hipStream_t */
 enum { MVIT_F32 = 0, MVIT_BF16 = 1 };
 enum { MVIT_OK = 0, MVIT_ERR_ARG = -1, MVIT_ERR_LAUNCH = -2, MVIT_ERR_UNSUPPORTED = -3 };
 
-/* 204: mvit_gemm_wgrads; the backward of blocks of much work uses it.
+/* 205: without 204's mvit_gemm_wgrads, whose sums were further from the exact ones than those of slices.
  * 203: mvit_gemm_args ends with overlapped; mvit_gemm_wgrad_split_k answers for a product that has the GPU to itself.
  * 202: mvit_gemm_args ends with colsum_rows.
  * 201: mvit_gemm_args has row_sums at its end.
  * 200: mvit_attn_bwd takes the size of its workspace (delta_elems) and checks that outputs and inputs are disjoint;
  *      mvit_adam_tensor rows are 96 bytes (shadow copy fields).  A caller built against an older header must be
  *      rebuilt: compare mvit_version() with the value the header was written for. */
-#define MVIT_VERSION 204
+#define MVIT_VERSION 205
 int mvit_version(void);
 const char* mvit_last_error(void);
 
@@ -210,12 +210,6 @@ int mvit_gemm_tile(int trans_a, int trans_b, int epilogue, int64_t M, int64_t N,
 int mvit_gemm_wgrad_split_k(int64_t out_rows, int64_t out_cols, int64_t k);
 /* Host-only: the same for a product that shares the GPU with another stream's (`overlapped`). */
 int mvit_gemm_wgrad_split_k_overlapped(int64_t out_rows, int64_t out_cols, int64_t k);
-/* One to four weight gradients over the same K > 128 (plain bf16 products of two transposed operands, with or without row_sums) in one
- * launch that deals their tiles out evenly: whole rounds of the compute units in one piece, the tiles left over in slices of K, whose fp32
- * sums a second launch adds in a fixed order.  split_k, workspace and overlapped of the products are not looked at.  The 16-byte aligned
- * workspace of mvit_gemm_wgrads_workspace_bytes (host-only; 0: none, or not such products) may be null where that is 0. */
-int mvit_gemm_wgrads(const mvit_gemm_args* list, int n, void* workspace, int64_t workspace_bytes, mvit_stream_t stream);
-int64_t mvit_gemm_wgrads_workspace_bytes(const mvit_gemm_args* list, int n);
 /* Host-only: the colsum_rows with which a bf16 MVIT_EPI_SWIGLU_BWD product of this shape is fastest. */
 int mvit_gemm_swiglu_bwd_colsum_rows(int64_t M, int64_t N, int64_t K);
 
@@ -273,9 +267,7 @@ int mvit_attn_bwd(const void* q, const void* k, const void* v, const void* o, co
  *            five events of the caller's (hipEvent_t), and the call leaves the main stream waiting for the side one.
  *            A bf16 block of so little work that the host's launches cost more than the GPU's idle units does not use
  *            it (mvit_block_bwd_uses_side_stream; the events are asked for all the same): its four weight gradients are
- *            one launch on the main stream, behind the chain, and its column sums another, with the same results.
- *            A bf16 block of much work with bf16 gradients (mvit_block_bwd_wgrads_together) sends its weight gradients through
- *            mvit_gemm_wgrads when the last operand is complete, on side_stream where there is one; split_k_* are not used then. */
+ *            one launch on the main stream, behind the chain, and its column sums another, with the same results. */
 typedef struct mvit_block_args {
   int dtype, grad_dtype;
   int C, I, Ipad, nheads, head_dim;
@@ -303,8 +295,6 @@ int64_t mvit_block_bwd_workspace_bytes(const mvit_block_args* args);
 /* Host-only: whether the call runs weight gradients on a given side_stream (1) or in one launch behind the input-gradient
  * chain (0).  Of the arguments only dtypes, sizes and split_k_* are looked at. */
 int mvit_block_bwd_uses_side_stream(const mvit_block_args* args);
-/* Host-only: whether the call's weight gradients go through mvit_gemm_wgrads (1).  Only dtypes and sizes are looked at. */
-int mvit_block_bwd_wgrads_together(const mvit_block_args* args);
 int mvit_block_bwd(const mvit_block_args* args, mvit_stream_t stream);
 
 /* ---------------------------------------------------------------- vision -> text hand-off */

@@ -29,31 +29,6 @@ inline bool grouped_wgrads(const mvit_block_args* a) {
          a->split_k_gate_up == 1 && a->split_k_proj == 1 && a->split_k_qkv == 1;
 }
 
-// The products of a block's four weight gradients, as far as the plan of their even shares depends on them
-inline void wgrad_shapes(const mvit_block_args* a, mvit_gemm_args (&list)[4]) {
-  const int64_t shape[4][2] = {{a->C, a->I}, {2 * (int64_t)a->Ipad, a->C}, {a->C, a->C}, {3 * (int64_t)a->C, a->C}};
-  memset(list, 0, sizeof(list));
-  for (int i = 0; i < 4; ++i) {
-    list[i].dtype = list[i].out_dtype = MVIT_BF16;
-    list[i].trans_a = list[i].trans_b = 1;
-    list[i].M = shape[i][0]; list[i].N = shape[i][1]; list[i].K = a->S;
-  }
-}
-// Whether the four weight gradients are dealt out evenly in one launch (mvit_gemm_wgrads), which starts beside the last input gradient, instead
-// of starting one by one on the second stream as soon as their operands are complete.  One by one they fill 82 to 98 % of the units and
-// leave fp32 slices to be summed (25,524 rows, us alone: 957 in four launches and four reductions, 813 together), but what they leave idle is filled
-// by the input gradients beside them, and the other way round; behind the chain, input gradients have the units to themselves and
-// take tiles that end in whole rounds (choose_tile, rows_in_full_rounds).  So it pays from some work on: ms per step one by one / together, blocks of 1280
-// columns (MLP 3420), 16 of them, 2,304 rows 8.14 / 8.34, 4,900 14.4 / 15.0, 6,400 17.2 / 17.2, 8,464 22.7 / 22.5, 10,000 25.7 / 26.0, 12,100 29.4 / 29.1; 32 of
-// them, 14,336 rows 65.9 / 64.3, 25,524 112.3 / 110.0, 36,864 257 / 254; six blocks of 2560 (6840): 3,136 rows 11.3 / 11.0, 6,400 20.5 / 20.1; twelve of 640
-// (1712): 10,000 rows 9.2 / 9.8, 25,600 24.2 / 24.2.  Fewer than 2,048 rows were not measured at widths whose work is beyond the line.
-constexpr int64_t TOGETHER_ROWS = 12000, TOGETHER_MIN_ROWS = 2048;
-inline bool wgrads_together(const mvit_block_args* a) {
-  const int64_t longest = 2 * (int64_t)a->Ipad > 3 * (int64_t)a->C ? 2 * (int64_t)a->Ipad : 3 * (int64_t)a->C;
-  return a->dtype == MVIT_BF16 && a->grad_dtype == MVIT_BF16 && a->S >= TOGETHER_MIN_ROWS && a->C % 8 == 0 && longest <= (1ll << 22) &&
-         (double)a->S * a->C * (4. * a->C + 3. * a->I) >= (double)TOGETHER_ROWS * 1280 * (4 * 1280 + 3 * 3420);
-}
-
 struct Bump {  // hands out 256-byte aligned pieces of the caller's workspace
   char* base;
   int64_t used, size;
@@ -107,11 +82,6 @@ BwdWorkspace plan_bwd_workspace(const mvit_block_args* a, void* base) {
   for (int i = 0; i < 4; ++i) {
     const int64_t n = sk[i] + rows[i];
     w.splitk_bytes = n * 4 > w.splitk_bytes ? n * 4 : w.splitk_bytes;
-  }
-  if (wgrads_together(a)) {
-    mvit_gemm_args list[4];
-    wgrad_shapes(a, list);
-    w.splitk_bytes = mvit_gemm_wgrads_workspace_bytes(list, 4);
   }
   w.splitk = static_cast<float*>(b.take(w.splitk_bytes));
   w.total = b.used;
@@ -195,8 +165,6 @@ extern "C" int64_t mvit_block_bwd_workspace_bytes(const mvit_block_args* a) {
 
 extern "C" int mvit_block_bwd_uses_side_stream(const mvit_block_args* a) { return a != nullptr && !grouped_wgrads(a); }
 
-extern "C" int mvit_block_bwd_wgrads_together(const mvit_block_args* a) { return a != nullptr && a->C > 0 && a->I > 0 && wgrads_together(a); }
-
 extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   if (int rc = check_block("block_bwd", a)) return rc;
   MVIT_REQUIRE(a->gu && a->dx2 && a->dx && a->dgu && a->dn && a->dx1 && a->dqkv, "block_bwd: null gradient buffer");
@@ -204,11 +172,8 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
                "block_bwd: null parameter-gradient buffer");
   MVIT_REQUIRE(a->grad_dtype == MVIT_BF16 || a->grad_dtype == MVIT_F32, "block_bwd: grad_dtype %d", a->grad_dtype);
   MVIT_REQUIRE(a->split_k_down >= 1 && a->split_k_gate_up >= 1 && a->split_k_proj >= 1 && a->split_k_qkv >= 1, "block_bwd: split_k counts must be >= 1");
-  const bool together = wgrads_together(a), grouped = !together && grouped_wgrads(a);
+  const bool grouped = grouped_wgrads(a);
   const bool two = a->side_stream != nullptr && !grouped;
-  // whether weight gradients run beside the input gradients; the one launch beside the last of them does not count (14,336 rows: told of it,
-  // that product takes a tile that makes a step of 64.5 ms 65.5)
-  const bool beside = two && !together;
   if (a->side_stream != nullptr) MVIT_REQUIRE(a->events[0] && a->events[1] && a->events[2] && a->events[3] && a->events[4], "block_bwd: a second stream needs five events");
   if (a->S == 0) return MVIT_OK;
   const BwdWorkspace w = plan_bwd_workspace(a, a->workspace);
@@ -232,7 +197,7 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   // Weight and bias gradients feed nothing else in the block: with a second stream they start there once their inputs
   // are complete on the main stream (event n) and are joined at the end; without one they run in line.
   auto fork = [&](int n) -> mvit_stream_t {
-    if (!two || (together && n < 3)) return stream;
+    if (!two) return stream;
     hipEvent_t ev = reinterpret_cast<hipEvent_t>(a->events[n]);
     if (hipEventRecord(ev, main_s) != hipSuccess || hipStreamWaitEvent(side_s, ev, 0) != hipSuccess) {
       mvit_set_error(MVIT_ERR_LAUNCH, "block_bwd: event %d: %s", n, hipGetErrorString(hipGetLastError()));
@@ -251,14 +216,14 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   auto weight_grad = [&](const void* dy, int64_t ldy, int64_t M, const void* x, int64_t ldx, int64_t N, void* out, void* bias, int split_k, mvit_stream_t st) -> int {
     if (bias && dt != MVIT_BF16) STEP(bias_grad(dy, ldy, M, bias, st));
     mvit_gemm_args g = gemm_args(dt, gdt);
-    g.trans_a = 1; g.trans_b = 1; g.overlapped = beside;
+    g.trans_a = 1; g.trans_b = 1; g.overlapped = two;
     g.M = M; g.N = N; g.K = S;
     g.A = dy; g.lda = ldy; g.B = x; g.ldb = ldx; g.C = out; g.ldc = N;
-    if (split_k > 1 && !together) {
+    if (split_k > 1) {
       g.split_k = split_k; g.workspace = w.splitk; g.workspace_bytes = (int64_t)split_k * M * (N + 1) * 4;
     }
     if (dt == MVIT_BF16) g.row_sums = bias;
-    if (grouped || together) {
+    if (grouped) {
       later[n_later++] = g;
       return MVIT_OK;
     }
@@ -268,7 +233,7 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   // ---- MLP: x2 = x1 + down(silu(g) * u)
   {
     mvit_stream_t st = fork(0);
-    if (!st && beside) return MVIT_ERR_LAUNCH;
+    if (!st && two) return MVIT_ERR_LAUNCH;
     STEP(weight_grad(a->dx2, C, C, a->h, Ipad, I, a->g_wdown, a->g_bdown, a->split_k_down, st));
   }
   // dgu = (dx2 . Wdown) through the SwiGLU derivative.  In bf16 the per-tile column sums of dgu come back with it, from its fp32
@@ -276,7 +241,7 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   const bool fused_cols = dt == MVIT_BF16;
   {
     mvit_gemm_args g = gemm_args(dt, dt);
-    g.trans_b = 1; g.epilogue = MVIT_EPI_SWIGLU_BWD; g.overlapped = beside;
+    g.trans_b = 1; g.epilogue = MVIT_EPI_SWIGLU_BWD; g.overlapped = two;
     g.M = S; g.N = Ipad; g.K = C;
     g.A = a->dx2; g.lda = C; g.B = a->wdown; g.ldb = Ipad; g.C = a->dgu; g.ldc = 2 * Ipad; g.R = a->gu; g.ldr = 2 * Ipad; g.aux_off = Ipad;
     if (fused_cols) {
@@ -286,13 +251,13 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   }
   {
     mvit_stream_t st = fork(1);
-    if (!st && beside) return MVIT_ERR_LAUNCH;
-    if (fused_cols && !grouped && !together) STEP(mvit_reduce_partials(w.swiglu_cols, w.n_swiglu_cols, 2 * Ipad, a->g_bgu, gdt, st));
+    if (!st && two) return MVIT_ERR_LAUNCH;
+    if (fused_cols && !grouped) STEP(mvit_reduce_partials(w.swiglu_cols, w.n_swiglu_cols, 2 * Ipad, a->g_bgu, gdt, st));
     STEP(weight_grad(a->dgu, 2 * Ipad, 2 * Ipad, a->n2, C, C, a->g_wgu, fused_cols ? nullptr : a->g_bgu, a->split_k_gate_up, st));
   }
   {  // dn2 = dgu . Wgu
     mvit_gemm_args g = gemm_args(dt, dt);
-    g.trans_b = 1; g.overlapped = beside;
+    g.trans_b = 1; g.overlapped = two;
     g.M = S; g.N = C; g.K = 2 * Ipad;
     g.A = a->dgu; g.lda = 2 * Ipad; g.B = a->wgu; g.ldb = C; g.C = a->dn; g.ldc = C;
     STEP(mvit_gemm(&g, stream));
@@ -303,12 +268,12 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   // ---- attention: x1 = x + proj(attn(rope(qkv(norm1(x)))))
   {
     mvit_stream_t st = fork(2);
-    if (!st && beside) return MVIT_ERR_LAUNCH;
+    if (!st && two) return MVIT_ERR_LAUNCH;
     STEP(weight_grad(a->dx1, C, C, a->o, C, C, a->g_wproj, a->g_bproj, a->split_k_proj, st));
   }
   {  // d_o = dx1 . Wproj  (into the dn buffer, whose contents the norm backward above has consumed)
     mvit_gemm_args g = gemm_args(dt, dt);
-    g.trans_b = 1; g.overlapped = beside;
+    g.trans_b = 1; g.overlapped = two;
     g.M = S; g.N = C; g.K = C;
     g.A = a->dx1; g.lda = C; g.B = a->wproj; g.ldb = C; g.C = a->dn; g.ldc = C;
     STEP(mvit_gemm(&g, stream));
@@ -322,11 +287,10 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
     mvit_stream_t st = fork(3);
     if (!st && two) return MVIT_ERR_LAUNCH;
     STEP(weight_grad(a->dqkv, 3 * C, 3 * C, a->n1, C, C, a->g_wqkv, a->g_bqkv, a->split_k_qkv, st));
-    if (together) STEP(mvit_gemm_wgrads(later, n_later, w.splitk, w.splitk_bytes, st));
   }
   {  // dn1 = dqkv . Wqkv
     mvit_gemm_args g = gemm_args(dt, dt);
-    g.trans_b = 1; g.overlapped = beside;
+    g.trans_b = 1; g.overlapped = two;
     g.M = S; g.N = C; g.K = 3 * C;
     g.A = a->dqkv; g.lda = 3 * C; g.B = a->wqkv; g.ldb = C; g.C = a->dn; g.ldc = C;
     STEP(mvit_gemm(&g, stream));
@@ -334,7 +298,7 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   STEP(mvit_rmsnorm_bwd(a->dn, a->x, a->norm1, a->rstd1, a->dx1, a->dx, w.rms1, n_rms, S, C, dt, stream));
   if (grouped) STEP(mvit_gemm_wgrad_group(later, n_later, main_s));
   const mvit_partials sums[3] = {{w.rms2, n_rms, C, a->g_norm2}, {w.rms1, n_rms, C, a->g_norm1}, {w.swiglu_cols, w.n_swiglu_cols, 2 * Ipad, a->g_bgu}};
-  STEP(mvit_reduce_partials_group(sums, grouped || together ? 3 : 2, gdt, main_s));
+  STEP(mvit_reduce_partials_group(sums, grouped ? 3 : 2, gdt, main_s));
   if (two) {  // the gradients are complete on the main stream when the call's work is
     hipEvent_t ev = reinterpret_cast<hipEvent_t>(a->events[4]);
     if (hipEventRecord(ev, side_s) != hipSuccess || hipStreamWaitEvent(main_s, ev, 0) != hipSuccess)

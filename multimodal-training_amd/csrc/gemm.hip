@@ -1260,12 +1260,12 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
   return best;
 }
 
-// Rows of a forward product that fill whole rounds of 256 x 256 tiles, when the rest is better taken by a second launch of the
+// Rows of a forward product, or of an input gradient that has the units to itself, that fill whole rounds of 256 x 256 tiles, when the rest is better taken by a second launch of the
 // tiles that suit it (0: one launch for all).  14,336 rows are 56 x 5 tiles of 1280 columns, 1.09 rounds of 256 units: a second
-// round for 24 tiles, or 2.2 rounds of 128 x 128 tiles at two thirds of the rate.  Input gradients that have the units to themselves likewise
-// (14,336 rows, K = 6912, 3840 and 1280, us together, 192 x 128 tiles in one launch / head and rest 411 / 377; 16,384 on 128 x 128 549 / 446).  255 tiles in one round and 1,280 rows on small
+// round for 24 tiles, or 2.2 rounds of 128 x 128 tiles at two thirds of the rate.  255 tiles in one round and 1,280 rows on small
 // tiles are faster than either (forward products of the tower, time alone of the step: 14,336 rows 71.6 -> 69.6 ms, 9,600 51.7 ->
-// 50.2, 4,360 without gradients 8.92 -> 8.61).  In the backward the second stream fills the last round, see choose_tile.
+// 50.2, 4,360 without gradients 8.92 -> 8.61).  Input gradients, us in one launch / head and rest: 14,336 x 1280, K = 6912 219 / 194, K = 3840
+// 130 / 114; 3,584 x 5120, K = 3584, GELU backward 168 / 144; 4,096 x 5120 190 / 170; the model errs at 6,381 x 5120, K = 3584, 166 / 170.  In the backward the second stream fills the last round, see choose_tile.
 int64_t rows_in_full_rounds(GemmTiledKind kind, int64_t M, int64_t N, int64_t K, int n_cu, bool overlapped) {
   if (!(kind == NN_NONE || kind == NN_BIAS || kind == NN_BIAS_RES || kind == NN_BIAS_GELU || kind == NN_SWIGLU || ((kind == NT_NONE || kind == NT_GELU_BWD) && !overlapped)) || !pp_takes(kind, K, K)) return 0;
   const int64_t tn = (N * (kind == NN_SWIGLU ? 2 : 1) + 255) / 256, rounds = (M + 255) / 256 * tn / n_cu, rows = rounds * n_cu / tn * 256;
@@ -1539,87 +1539,6 @@ int mvit_gemm_wgrad_group(const mvit_gemm_args* list, int n, hipStream_t s) {
     set_tile_order(p, bm);
   }
   return mvit_gemm_small_group(bm, bn, g, s);
-}
-
-// Several weight gradients of one contraction dealt out evenly: the 256 x 256 tiles of all of them in one launch, whole rounds of the
-// units in one piece each and the tiles left over in so many slices of K that their pieces fill the units as well.  us: modelled time (1.3 us
-// a K tile of 64 and 8 to 10 a tile, as measured with cool units; under a long load both grow alike).  The tower's block has 305 tiles: one
-// round of 256 and 49 in five slices, 479 K tiles per unit of the 475 that the work is at 25,524 rows.
-struct BalancedPlan {
-  int64_t whole, slices, chunk;
-  double us;
-};
-static BalancedPlan plan_balanced(int64_t tiles, int64_t k, int n_cu) {
-  const int64_t steps = (k + 63) / 64, rounds = tiles / n_cu, cut = tiles - rounds * n_cu;
-  BalancedPlan best{rounds * n_cu, 1, k, 1e30};
-  for (int64_t s = 1; s == 1 || (s <= 64 && cut > 0 && s * cut <= 4 * (int64_t)n_cu); ++s) {
-    const int64_t chunk = (steps + s - 1) / s, slices = (steps + chunk - 1) / chunk, pieces = cut * slices;
-    if (slices != s || (s > 1 && (chunk < 4 || k - (slices - 1) * chunk * 64 <= 128))) continue;
-    double us = 4. + (double)rounds * (1.3 * (double)steps + 8.) + (double)((pieces + n_cu - 1) / n_cu) * (1.3 * (double)chunk + 10.);
-    if (s > 1) us += 5. + (double)pieces * 262144. / 5e6;  // the pieces are read again, 5 TB/s, by one more launch
-    if (us < best.us) best.slices = s, best.chunk = s > 1 ? chunk * 64 : k, best.us = us;
-  }
-  if (best.slices == 1) best.whole = tiles;
-  return best;
-}
-constexpr int BALANCED_CU = 256;  // the plan is the same on every device, so that sums are
-static int64_t balanced_tiles(const mvit_gemm_args* list, int n) {
-  int64_t tiles = 0;
-  for (int i = 0; i < n; ++i) tiles += ((list[i].M + 255) / 256) * ((list[i].N + 255) / 256);
-  return tiles;
-}
-static int64_t balanced_bytes(const BalancedPlan& b, int64_t tiles) { return (tiles - b.whole) * b.slices * (65536 + 256) * 4; }
-static bool balanced_list(const mvit_gemm_args* list, int n) {
-  bool ok = list != nullptr && n >= 1 && n <= GEMM_GROUP_MAX;
-  for (int i = 0; ok && i < n; ++i) {
-    const mvit_gemm_args& a = list[i];
-    ok = a.dtype == MVIT_BF16 && a.out_dtype == MVIT_BF16 && a.trans_a && a.trans_b && a.epilogue == MVIT_EPI_NONE && a.M > 0 && a.N > 0 && a.K > 128 &&
-         a.K == list[0].K && a.M < (1ll << 22) && a.N < (1ll << 22);
-  }
-  return ok && balanced_tiles(list, n) < (1ll << 24);
-}
-
-extern "C" int64_t mvit_gemm_wgrads_workspace_bytes(const mvit_gemm_args* list, int n) {
-  if (!balanced_list(list, n)) return 0;
-  const int64_t tiles = balanced_tiles(list, n);
-  return balanced_bytes(plan_balanced(tiles, list[0].K, BALANCED_CU), tiles);
-}
-
-extern "C" int mvit_gemm_wgrads(const mvit_gemm_args* list, int n, void* workspace, int64_t workspace_bytes, mvit_stream_t stream) {
-  MVIT_REQUIRE(list && n >= 1 && n <= GEMM_GROUP_MAX, "gemm_wgrads: one to %d products, got %d", GEMM_GROUP_MAX, n);
-  MVIT_REQUIRE(balanced_list(list, n), "gemm_wgrads: plain bf16 products of two transposed operands over the same K > 128");
-  GemmBalanced g;
-  memset(&g, 0, sizeof(g));
-  g.n = n;
-  const int64_t tiles = balanced_tiles(list, n);
-  const BalancedPlan plan = plan_balanced(tiles, list[0].K, BALANCED_CU);
-  const int64_t need = balanced_bytes(plan, tiles);
-  if (need > 0) MVIT_REQUIRE(workspace && mvit_aligned16(workspace) && workspace_bytes >= need, "gemm_wgrads: a 16-byte aligned workspace of %lld bytes is needed", (long long)need);
-  g.tiles = (int)tiles; g.whole = (int)plan.whole; g.slices = (int)plan.slices;
-  g.workspace = static_cast<float*>(workspace);
-  g.row_ws = g.workspace + (tiles - plan.whole) * plan.slices * 65536;
-  int first = 0;
-  for (int i = 0; i < n; ++i) {
-    const mvit_gemm_args& a = list[i];
-    MVIT_REQUIRE(a.A && a.B && a.C && mvit_aligned16(a.A) && mvit_aligned16(a.B) && a.lda % 8 == 0 && a.ldb % 8 == 0 && a.lda >= (a.M + 7) / 8 * 8 &&
-                     a.ldb >= (a.N + 7) / 8 * 8 && a.ldc >= a.N && a.lda <= (1ll << 22) && a.ldb <= (1ll << 22),
-                 "gemm_wgrads: product %d: null or unaligned operand, or a row pitch that it does not take", i);
-    GemmParams& p = g.p[i];
-    p.M = a.M; p.N = a.N; p.K = a.K;
-    p.A = a.A; p.lda = a.lda; p.B = a.B; p.ldb = a.ldb; p.C = a.C; p.ldc = a.ldc;
-    p.row_sums = a.row_sums;
-    p.vec_ok = vec16(a.C, a.ldc, 2);
-    p.half_vec_ok = a.ldc % 4 == 0 && reinterpret_cast<uintptr_t>(a.C) % 8 == 0;
-    p.split_k = 1; p.k_chunk = plan.chunk; p.reduce_epi = MVIT_EPI_NONE;
-    p.tiles_m = (int)((a.M + 255) / 256);
-    p.tiles_n = (int)((a.N + 255) / 256);
-    set_tile_order(p, 256);
-    g.first_tile[i] = first;
-    first += p.tiles_m * p.tiles_n;
-  }
-  const int dev = mvit_current_device("gemm");
-  if (dev < 0) return MVIT_ERR_LAUNCH;
-  return mvit_gemm_pp_wgrads(g, device_cu_count(dev), reinterpret_cast<hipStream_t>(stream));
 }
 
 // Slices along the contraction for a product with few output tiles and a long contraction (a weight gradient, contracted

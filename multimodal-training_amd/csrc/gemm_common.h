@@ -68,18 +68,6 @@ struct GemmGroup {
 };
 int mvit_gemm_small_group(int bm, int bn, GemmGroup& group, hipStream_t stream);                                // gemm_small.hip
 
-// Weight gradients of one contraction whose 256 x 256 tiles are dealt out evenly: the first `whole` of them, whole rounds of the compute units, are
-// computed in one piece, the others in `slices` pieces of k_chunk (in each p) that leave fp32 partial tiles.
-struct GemmBalanced {
-  int n;
-  int first_tile[GEMM_GROUP_MAX];
-  int tiles, whole, slices;
-  float* workspace;  // [slices][tiles - whole][256][256]
-  float* row_ws;     // [slices][tiles - whole][256]: partial row sums
-  GemmParams p[GEMM_GROUP_MAX];
-};
-int mvit_gemm_pp_wgrads(const GemmBalanced& g, int n_cu, hipStream_t stream);                                   // gemm_pingpong.hip
-
 int mvit_gemm_f32(int ta, int tb, int epi, const GemmParams& p, int n_cu, hipStream_t stream);              // gemm_f32.hip
 
 namespace {

@@ -14,12 +14,6 @@ __device__ __forceinline__ void pp_barrier() {
   asm volatile("s_barrier" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
 }
-// The lane's number, made where it is used rather than held in a register across a main loop
-__device__ __forceinline__ int pp_lane() {
-  int l;
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(l));
-  return l;
-}
 __device__ __forceinline__ void pp_load(unsigned lds_addr, unsigned voff, const char* base) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds_addr), "v"(voff), "s"(base) : "memory");
 }

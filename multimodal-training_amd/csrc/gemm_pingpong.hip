@@ -42,16 +42,9 @@ struct PpCfg {
   static constexpr int MIN_K = 2 * BK + 1;  // at least three K tiles
 };
 
-// Work: GemmParams, one product, or GemmBalanced, several weight gradients whose work is dealt out evenly
-template <typename TO, bool TA, bool TB, int EPI, typename Work>
-__device__ __forceinline__ void gemm_pp_tiles(const Work& w) {
+template <typename TO, bool TA, bool TB, int EPI>
+__global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmParams p) {
   using T = bf16_t;
-  constexpr bool GROUP = std::is_same_v<Work, GemmBalanced>;
-  static_assert(!GROUP || (TA && TB && EPI == MVIT_EPI_NONE), "only weight gradients are dealt out evenly");
-  auto product = [&](int i) -> const GemmParams& {
-    if constexpr (GROUP) return w.p[i];
-    else return w;
-  };
   constexpr int BM = PpCfg::BM, BK = PpCfg::BK, HALF = PpCfg::HALF, STAGE = PpCfg::STAGE;
   constexpr bool DUAL = (EPI == MVIT_EPI_SWIGLU);
   constexpr bool SW_BWD = EPI == MVIT_EPI_SWIGLU_BWD;
@@ -74,16 +67,9 @@ __device__ __forceinline__ void gemm_pp_tiles(const Work& w) {
   const int l = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wv >> 2, wn = wv & 3;
-  unsigned tiles, total, per_xcd;
-  if constexpr (GROUP) {
-    tiles = (unsigned)(w.tiles - w.whole);        // those that are cut
-    total = tiles * (unsigned)w.slices;           // and their pieces
-    per_xcd = (unsigned)(w.whole + 7) / 8;        // of the whole ones
-  } else {
-    tiles = (unsigned)(w.tiles_m * w.tiles_n);
-    total = tiles * (unsigned)w.split_k;
-    per_xcd = (total + 7) / 8;
-  }
+  const unsigned tiles = (unsigned)(p.tiles_m * p.tiles_n);
+  const unsigned total = tiles * (unsigned)p.split_k;
+  const unsigned per_xcd = (total + 7) / 8;
   typedef __attribute__((address_space(3))) unsigned char lds_byte;
   const unsigned lds_base = (unsigned)(__UINTPTR_TYPE__)(lds_byte*)smem_raw;
   const unsigned lds0 = lds_base + wv * 2048;  // this wave's share of a half tile
@@ -135,58 +121,24 @@ __device__ __forceinline__ void gemm_pp_tiles(const Work& w) {
   };
 
   // ---- loader: two 16-byte chunks per lane and half tile
-  // byte offsets of the lane's chunks from the half's base; the two k-rows of a [k][row] operand are four apart and swizzled alike, so
-  // that the second chunk lies the same way behind the first in every lane
-  constexpr int VA = TA ? 1 : 2, VB = TB ? 1 : 2;
-  unsigned va[2][VA], vb[2][VB];
+  unsigned va[2][2], vb[2][2];    // byte offsets of the lane's chunks from the half's base
   const char *ba[2], *bb[2];      // wave-uniform, advanced by one K tile per request
-  int step_a = 2 * BK, step_b = 2 * BK;  // pitches are at most 1 << 22 elements
-  if constexpr (!GROUP) {
-    if (TA) step_a = 2 * BK * (int)w.lda;
-    if (TB) step_b = 2 * BK * (int)w.ldb;
-  }
+  const int64_t step_a = TA ? 2ll * BK * p.lda : 2 * BK, step_b = TB ? 2ll * BK * p.ldb : 2 * BK;
   int T_ = 0, n_kt = 0, k_tail = 0;
-  int next_slice = 0, next_product = 0;  // GROUP: slice = the piece's index, -1 for a tile that is not cut
+  int next_slice = 0;
   int64_t next_m0 = 0, next_n0 = 0;
   int bias_buf = 0;
   auto start_tile = [&](unsigned idx) -> bool {
-    const int l = pp_lane();
-    unsigned slice = 0;
-    int tile, split;
-    if constexpr (GROUP) {
-      if (idx < per_xcd) {
-        tile = (int)((blockIdx.x & 7) * per_xcd + idx);
-        if (tile >= w.whole) return false;  // then none is cut
-        split = 1;
-        next_slice = -1;
-      } else {  // pieces of one slice lie together: the work-groups of an XCD then read the same rows of A and B
-        const unsigned per = (total + 7) / 8, piece = (blockIdx.x & 7) * per + (idx - per_xcd);
-        if (idx - per_xcd >= per || piece >= total) return false;
-        slice = piece / tiles;
-        tile = (int)(w.whole + (piece - slice * tiles));
-        split = w.slices;
-        next_slice = (int)piece;
-      }
-      next_product = 0;
-      while (next_product + 1 < w.n && tile >= w.first_tile[next_product + 1]) ++next_product;
-      tile -= w.first_tile[next_product];
-    } else {
-      const unsigned work = (blockIdx.x & 7) * per_xcd + idx;
-      if (idx >= per_xcd || work >= total) return false;
-      slice = w.split_k > 1 ? work / tiles : 0;
-      tile = (int)(work - slice * tiles);
-      split = w.split_k;
-      next_slice = (int)slice;
-    }
-    const GemmParams& p = product(next_product);
-    if constexpr (GROUP) {
-      step_a = 2 * BK * (int)p.lda;
-      step_b = 2 * BK * (int)p.ldb;
-    }
+    int l = threadIdx.x & 63;
+    asm volatile("" : "+v"(l));  // recomputed per tile rather than held in registers across the main loop
+    const unsigned work = (blockIdx.x & 7) * per_xcd + idx;
+    if (idx >= per_xcd || work >= total) return false;
+    const unsigned slice = p.split_k > 1 ? work / tiles : 0;
     int tm, tn;
-    tile_coords(p, tile, tm, tn);
+    tile_coords(p, (int)(work - slice * tiles), tm, tn);
+    next_slice = (int)slice;
     const int64_t k_begin = (int64_t)slice * p.k_chunk;
-    const int64_t k_end = split > 1 ? (k_begin + p.k_chunk < p.K ? k_begin + p.k_chunk : p.K) : p.K;
+    const int64_t k_end = p.split_k > 1 ? (k_begin + p.k_chunk < p.K ? k_begin + p.k_chunk : p.K) : p.K;
     next_m0 = (int64_t)tm * BM;
     next_n0 = (int64_t)tn * NCOLS;
     const int klen = (int)(k_end - k_begin);
@@ -211,7 +163,7 @@ __device__ __forceinline__ void gemm_pp_tiles(const Work& w) {
           const int k = q * 4 + (l >> 4);
           int r = h * 128 + (((l & 15) ^ tr_swizzle(k)) << 3);
           if (r >= m_left) r = 0;
-          if (j == 0) va[h][0] = (unsigned)((k * p.lda + r) * 2);
+          va[h][j] = (unsigned)((k * p.lda + r) * 2);
         }
         if constexpr (!TB) {
           const int row = q * 8 + (l >> 3), c = (l & 7) ^ (((row >> 1) & 1) | (((row >> 3) & 3) << 1));
@@ -222,7 +174,7 @@ __device__ __forceinline__ void gemm_pp_tiles(const Work& w) {
           const int k = q * 4 + (l >> 4);
           int r = h * 128 + (((l & 15) ^ tr_swizzle(k)) << 3);
           if (r >= n_left) r = 0;
-          if (j == 0) vb[h][0] = (unsigned)((k * p.ldb + r) * 2);
+          vb[h][j] = (unsigned)((k * p.ldb + r) * 2);
         }
       }
     }
@@ -233,25 +185,22 @@ __device__ __forceinline__ void gemm_pp_tiles(const Work& w) {
     constexpr int x = decltype(X)::value, h = x >> 1;
     constexpr bool is_a = (x & 1) != 0, tr = is_a ? TA : TB;
     const char*& base = is_a ? ba[h] : bb[h];
-    const unsigned* const v = is_a ? va[h] : vb[h];
-    constexpr int second = tr ? 0 : 1;
-    const int behind = tr ? (is_a ? step_a : step_b) / 16 : 0;  // four k-rows
+    const unsigned(&v)[2] = is_a ? va[h] : vb[h];
     const unsigned dst = lds0 + stage_off + (is_a ? 0 : 2 * HALF) + h * HALF;
     if (tail) {  // the last, partial K tile: chunks past the end of K are zeros
-      const int lane = pp_lane();
-      unsigned zero = 0u;
-      asm volatile("" : "+v"(zero));  // not to be held in registers for this rare path
+      int lane = l;
+      asm volatile("" : "+v"(lane));  // not to be computed ahead of this rare path
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const int q = wv * 2 + j, row = q * 8 + (lane >> 3);
         const int k = tr ? q * 4 + (lane >> 4) : 8 * ((lane & 7) ^ (is_a ? (row >> 1) & 7 : ((row >> 1) & 1) | (((row >> 3) & 3) << 1)));
-        pp_load_below(dst + j * 1024, v[j * second], base + j * behind, k, k_tail);
-        if (k >= k_tail) *reinterpret_cast<u32x4*>(smem_raw + (dst - lds_base) + j * 1024 + lane * 16) = u32x4{zero, zero, zero, zero};
+        pp_load_below(dst + j * 1024, v[j], base, k, k_tail);
+        if (k >= k_tail) *reinterpret_cast<u32x4*>(smem_raw + (dst - lds_base) + j * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     } else {
       pp_load(dst, v[0], base);
-      pp_load(dst + 1024, v[second], base + behind);
+      pp_load(dst + 1024, v[1], base);
     }
     base += is_a ? step_a : step_b;
   };
@@ -261,9 +210,7 @@ __device__ __forceinline__ void gemm_pp_tiles(const Work& w) {
   using X3 = std::integral_constant<int, 3>;
   auto issue_first = [&]() {
     if constexpr (HAS_BIAS) {  // this wave's 2 x 32 bias values as dwords: lanes 0-15 half 0, lanes 16-31 half 1
-      const int l = pp_lane();
       const int h = (l >> 4) & 1;
-      const GemmParams& p = product(0);
       int64_t n = next_n0 + (DUAL ? wn * 32 : (TB ? h * 128 + wn * 32 : wn * 64 + h * 32)) + 2 * (l & 15);
       if (n > p.N - 2) n = p.N - 2;
       const T* src = static_cast<const T*>(DUAL && h ? p.bias2 : p.bias);
@@ -367,7 +314,6 @@ __device__ __forceinline__ void gemm_pp_tiles(const Work& w) {
   while (true) {
     const int64_t m0 = next_m0, n0 = next_n0;
     const int slice = next_slice, bias_now = bias_buf;
-    const GemmParams& p = product(next_product);
     n_kt = T_;
     st = 0;
     if constexpr (ROW_SUMS) {
@@ -394,10 +340,11 @@ __device__ __forceinline__ void gemm_pp_tiles(const Work& w) {
     if (!SW_BWD && wm == 0) pp_barrier();
 
     // ---- epilogue: row block a of 16, half g: lane owns row l % 16 and the eight columns 8 * (l / 16) ..
-    const bool to_ws = GROUP ? slice >= 0 : (EPI == MVIT_EPI_NONE) && p.split_k > 1;
+    const bool to_ws = (EPI == MVIT_EPI_NONE) && p.split_k > 1;
     const bool vec = to_ws ? (p.N % 4 == 0) : p.vec_ok != 0;
-    const bool interior = GROUP && to_ws ? true : vec && m0 + BM <= p.M && n0 + NCOLS <= p.N;  // a piece is a whole tile of the workspace
-    const int lane = pp_lane();
+    const bool interior = vec && m0 + BM <= p.M && n0 + NCOLS <= p.N;
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
     const int i16 = lane & 15, g4 = lane >> 4;
     const int64_t m_lane = m0 + wm * 64 + i16;
     int64_t n_lane[2];
@@ -446,13 +393,7 @@ __device__ __forceinline__ void gemm_pp_tiles(const Work& w) {
         }
       }
     };
-    float* ws = nullptr;
-    if constexpr (GROUP) {
-      if (to_ws) ws = w.workspace + (int64_t)slice * (BM * NCOLS) - (m0 * NCOLS + n0);
-    } else if (to_ws) {
-      ws = p.workspace + (int64_t)slice * p.M * p.N;
-    }
-    const int64_t ws_pitch = GROUP ? NCOLS : p.N;
+    float* ws = to_ws ? p.workspace + (int64_t)slice * p.M * p.N : nullptr;
     constexpr int NG = DUAL ? 1 : 2, ITEMS = 8 * NG;
     // item -> row block and column half: by rows, or all rows of a half first, in the order of their sums
     auto block_of = [](int it) { return SW_BWD ? (it & 1) | ((it & 2) << 1) | ((it & 4) >> 1) : it / NG; };
@@ -476,8 +417,7 @@ __device__ __forceinline__ void gemm_pp_tiles(const Work& w) {
         const int64_t m = m_lane + (g4 >> 1) * 128 + wn * 16;
         if ((g4 & 1) == 0 && m < p.M) {  // stores that the next tile's waits do not count only make them wait for more
           const float sum = g4 >> 1 ? rs[1][0] : rs[0][0];
-          if (GROUP && to_ws) w.row_ws[(int64_t)slice * BM + (m - m0)] = sum;
-          else if (to_ws) p.row_ws[(int64_t)slice * p.M + m] = sum;
+          if (to_ws) p.row_ws[(int64_t)slice * p.M + m] = sum;
           else static_cast<TO*>(p.row_sums)[m] = from_f32<TO>(sum);
         }
       }
@@ -514,7 +454,7 @@ __device__ __forceinline__ void gemm_pp_tiles(const Work& w) {
         for (int it = 0; it < ITEMS; ++it) {
           float v[8], u[8];
           values(it, v, u);
-          if (to_ws) store8(ws + row_of(it) * ws_pitch + n_lane[half_of(it)], v);
+          if (to_ws) store8(ws + row_of(it) * p.N + n_lane[half_of(it)], v);
           else emit8_impl<T, TO, EPI, true, false>(p, row_of(it), n_lane[half_of(it)], v, u, nullptr, no_cs, false, HAS_BIAS ? hb[half_of(it)] : nullptr, HAS_BIAS && DUAL ? hb[1] : nullptr);
         }
       }
@@ -529,11 +469,11 @@ __device__ __forceinline__ void gemm_pp_tiles(const Work& w) {
         values(it, v, u);
         const int64_t m = row_of(it), n = n_lane[half_of(it)];
         if (m >= p.M || n >= p.N) continue;
-        if (!GROUP && to_ws) {
-          float* to = ws + m * p.N + n;
-          if (vec && n + 8 <= p.N) store8(to, v);
+        if (to_ws) {
+          float* w = ws + m * p.N + n;
+          if (vec && n + 8 <= p.N) store8(w, v);
           else
-            for (int e = 0; e < 8 && n + e < p.N; ++e) to[e] = v[e];
+            for (int e = 0; e < 8 && n + e < p.N; ++e) w[e] = v[e];
         } else if (vec && n + 8 <= p.N) {
           emit8_impl<T, TO, EPI, true>(p, m, n, v, u, nullptr, no_cs, do_cs, HAS_BIAS ? hb[half_of(it)] : nullptr, HAS_BIAS && DUAL ? hb[1] : nullptr);
         } else {
@@ -552,75 +492,21 @@ __device__ __forceinline__ void gemm_pp_tiles(const Work& w) {
   }
 }
 
-template <typename TO, bool TA, bool TB, int EPI>
-__global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_kernel(const GemmParams p) {
-  gemm_pp_tiles<TO, TA, TB, EPI>(p);
-}
-__global__ __launch_bounds__(PpCfg::NTHREADS, 2) void gemm_pp_wgrads_kernel(const GemmBalanced g) {
-  gemm_pp_tiles<bf16_t, true, true, MVIT_EPI_NONE>(g);
-}
-
-// The pieces of the tiles that were cut, added slice after slice.  Eight rows of a tile to a work-group.
-__global__ __launch_bounds__(256) void wgrads_reduce_kernel(const GemmBalanced g) {
-  const int cut = g.tiles - g.whole, r = blockIdx.x >> 5, part = blockIdx.x & 31;
-  int tile = g.whole + r, i = 0;
-  while (i + 1 < g.n && tile >= g.first_tile[i + 1]) ++i;
-  const GemmParams& p = g.p[i];
-  int tm, tn;
-  tile_coords(p, tile - g.first_tile[i], tm, tn);
-  const int row = part * 8 + (threadIdx.x >> 5), col = (threadIdx.x & 31) * 8;
-  const int64_t m = (int64_t)tm * 256 + row, n = (int64_t)tn * 256 + col;
-  if (part == 0 && tn == 0 && p.row_sums != nullptr && (int64_t)tm * 256 + threadIdx.x < p.M) {
-    float s = 0.f;
-    for (int k = 0; k < g.slices; ++k) s += g.row_ws[((int64_t)k * cut + r) * 256 + threadIdx.x];
-    static_cast<bf16_t*>(p.row_sums)[(int64_t)tm * 256 + threadIdx.x] = from_f32<bf16_t>(s);
-  }
-  if (m >= p.M || n >= p.N) return;
-  float v[8] = {};
-  const float* at = g.workspace + (int64_t)r * 65536 + row * 256 + col;
-#pragma unroll 4
-  for (int k = 0; k < g.slices; ++k, at += (int64_t)cut * 65536) {
-    const f32x4 a = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(at)), b = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(at) + 1);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      v[e] += a[e];
-      v[4 + e] += b[e];
-    }
-  }
-  float no_cs[16];
-  emit8<bf16_t, bf16_t, MVIT_EPI_NONE>(p, m, n, v, nullptr, p.vec_ok != 0, no_cs, false);
-}
-
-template <typename P>
-int launch_pp(void (*kern)(P), const P& p, int grid, bool (&attr_set_on)[MVIT_MAX_DEVICES], int lds, hipStream_t stream) {
-  const int dev = mvit_current_device("gemm");
-  if (dev < 0) return MVIT_ERR_LAUNCH;
-  if (!attr_set_on[dev]) {  // dynamic LDS above 64 KiB is opted into once per kernel and device
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    if (e != hipSuccess) return mvit_set_error(MVIT_ERR_LAUNCH, "gemm: hipFuncSetAttribute(%d B LDS): %s", lds, hipGetErrorString(e));
-    attr_set_on[dev] = true;
-  }
-  hipLaunchKernelGGL(kern, grid, PpCfg::NTHREADS, lds, stream, p);
-  MVIT_CHECK_LAUNCH("gemm");
-  return MVIT_OK;
-}
-
 }  // namespace
 
-int mvit_gemm_pp_wgrads(const GemmBalanced& g, int n_cu, hipStream_t stream) {
-  static bool set[MVIT_MAX_DEVICES] = {};
-  const int cut = g.tiles - g.whole, items = cut > 0 && g.whole > 0 ? n_cu : g.whole + cut * g.slices, want = (items + 7) / 8 * 8;
-  if (int rc = launch_pp(gemm_pp_wgrads_kernel, g, want < n_cu ? want : n_cu, set, PpCfg::lds(MVIT_EPI_NONE), stream)) return rc;
-  if (cut == 0) return MVIT_OK;
-  hipLaunchKernelGGL(wgrads_reduce_kernel, cut * 32, 256, 0, stream, g);
-  MVIT_CHECK_LAUNCH("gemm");
-  return MVIT_OK;
-}
-
 int mvit_gemm_pp(GemmTiledKind kind, const GemmParams& p, int n_cu, hipStream_t stream) {
-  const int want = (p.tiles_m * p.tiles_n * p.split_k + 7) / 8 * 8;
-  auto go = [&](void (*kern)(GemmParams), bool (&attr_set_on)[MVIT_MAX_DEVICES], int lds = PpCfg::lds(MVIT_EPI_NONE)) -> int {
-    return launch_pp(kern, p, want < n_cu ? want : n_cu, attr_set_on, lds, stream);
+  auto go = [&](auto kern, bool (&attr_set_on)[MVIT_MAX_DEVICES], int lds = PpCfg::lds(MVIT_EPI_NONE)) -> int {
+    const int dev = mvit_current_device("gemm");
+    if (dev < 0) return MVIT_ERR_LAUNCH;
+    if (!attr_set_on[dev]) {  // dynamic LDS above 64 KiB is opted into once per kernel and device
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+      if (e != hipSuccess) return mvit_set_error(MVIT_ERR_LAUNCH, "gemm: hipFuncSetAttribute(%d B LDS): %s", lds, hipGetErrorString(e));
+      attr_set_on[dev] = true;
+    }
+    const int want = (p.tiles_m * p.tiles_n * p.split_k + 7) / 8 * 8;
+    hipLaunchKernelGGL(kern, want < n_cu ? want : n_cu, PpCfg::NTHREADS, lds, stream, p);
+    MVIT_CHECK_LAUNCH("gemm");
+    return MVIT_OK;
   };
   static bool set[10][MVIT_MAX_DEVICES] = {};
   switch (kind) {

@@ -93,7 +93,6 @@ PROTOTYPES = {
     "mvit_gemm_tile": [_i32, _i32, _i32, _i64, _i64, _i64, _i32, _i32, _vp],
     "mvit_gemm_wgrad_split_k": [_i64, _i64, _i64],
     "mvit_gemm_wgrad_split_k_overlapped": [_i64, _i64, _i64],
-    "mvit_gemm_wgrads": [C.POINTER(GemmArgs), _i32, _vp, _i64, _vp],
     "mvit_gemm_swiglu_bwd_colsum_rows": [_i64, _i64, _i64],
     "mvit_attn_fwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i64, _i32, _i32, _i64, _i64, _i64, _i64, _f32, _i32, _vp],
     "mvit_image_token_ranks": [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp],
@@ -115,11 +114,10 @@ PROTOTYPES = {
     "mvit_block_fwd": [C.POINTER(BlockArgs), _vp],
     "mvit_block_bwd": [C.POINTER(BlockArgs), _vp],
     "mvit_block_bwd_uses_side_stream": [C.POINTER(BlockArgs)],
-    "mvit_block_bwd_wgrads_together": [C.POINTER(BlockArgs)],
     "mvit_attn_bwd": [_vp] * 10 + [_i64, _vp, _vp] + [_i32, _i32, _i64, _i32, _i32] + [_i64] * 8 + [_f32, _i32, _vp],
 }
-EXPORTS = sorted(list(PROTOTYPES) + ["mvit_version", "mvit_last_error", "mvit_attn_bwd_delta_elems", "mvit_block_bwd_workspace_bytes", "mvit_gemm_wgrads_workspace_bytes"])
-HEADER_VERSION = 204  # MVIT_VERSION of include/mi355_vit.h these prototypes were written for
+EXPORTS = sorted(list(PROTOTYPES) + ["mvit_version", "mvit_last_error", "mvit_attn_bwd_delta_elems", "mvit_block_bwd_workspace_bytes"])
+HEADER_VERSION = 205  # MVIT_VERSION of include/mi355_vit.h these prototypes were written for
 
 _lib = None
 
@@ -146,8 +144,6 @@ def load() -> C.CDLL:
         lib.mvit_attn_bwd_delta_elems.restype = _i64
         lib.mvit_block_bwd_workspace_bytes.argtypes = [C.POINTER(BlockArgs)]
         lib.mvit_block_bwd_workspace_bytes.restype = _i64
-        lib.mvit_gemm_wgrads_workspace_bytes.argtypes = [C.POINTER(GemmArgs), _i32]
-        lib.mvit_gemm_wgrads_workspace_bytes.restype = _i64
         if lib.mvit_version() != HEADER_VERSION:
             raise RuntimeError(f"{LIB_PATH} reports interface version {lib.mvit_version()}, these bindings are written for {HEADER_VERSION}: rebuild the library")
         _lib = lib

@@ -378,16 +378,11 @@ def _block_backward(dx2: torch.Tensor, x: torch.Tensor, saved: tuple, W: BlockWe
     main = torch.cuda.current_stream(dev)
     side = ops.side_stream(dev)
 
-    # the weight gradients of many rows are one launch, beside the last input gradient (as the C call sends them)
-    grad_dtype = next(iter(gdt.values())) if len(set(gdt.values())) == 1 else None
-    together = ops.block_wgrads_together(x.dtype, grad_dtype, S, C, I, Ipad)
-    beside = side is not None and not together
-
     def off_chain(fn):
         # work that feeds nothing else in this block (weight and bias gradients) runs on the second stream, after
         # the point its inputs are complete on the main stream, and is joined before the gradients are handed back;
         # one event and one stream switch per point serve the bias and the weight gradient that start there
-        if not beside:
+        if side is None:
             return fn()
         ev = torch.cuda.Event()
         ev.record(main)
@@ -395,13 +390,9 @@ def _block_backward(dx2: torch.Tensor, x: torch.Tensor, saved: tuple, W: BlockWe
             side.wait_event(ev)
             return fn()
 
-    later = []
+    beside = side is not None
 
     def weight_grad(dy, act, out, bias_dtype, n=None):
-        if together:
-            bias = None if bias_dtype is None else torch.empty(dy.shape[1], dtype=bias_dtype, device=dev)
-            later.append((dy, act, out, out.shape[1], bias))
-            return bias
         return ops.weight_grad(dy, act, out, bias_dtype, n=n, split_k=_block_split_k(out.shape[0], out.shape[1], S), overlapped=beside)
 
     # ---- MLP: x2 = x1 + down(silu(g) * u)
@@ -431,14 +422,6 @@ def _block_backward(dx2: torch.Tensor, x: torch.Tensor, saved: tuple, W: BlockWe
     ops.rope_(dqkv, geo.cos, geo.sin, 2 * H, hd, backward=True, lead_heads=H, lead_scale=hd**-0.5 * LOG2E)
     g_wqkv = torch.empty(3 * C, C, dtype=gdt["attn.q_proj.weight"], device=dev)
     g_bqkv = off_chain(lambda: weight_grad(dqkv, n1, g_wqkv, gdt["attn.q_proj.bias"]))
-    if together and side is not None:
-        ev = torch.cuda.Event()
-        ev.record(main)
-        with torch.cuda.stream(side):
-            side.wait_event(ev)
-            ops.weight_grads(later)
-    elif together:
-        ops.weight_grads(later)
     dn1 = d_o
     ops.gemm(dqkv, W.wqkv, dn1, trans_b=True, overlapped=beside)
     dx, g_n1 = ops.rmsnorm_bwd(dn1, x, W.norm1.view(-1), rstd1, dx_add=dx1, w_grad_dtype=gdt["norm1.weight"])

@@ -431,43 +431,6 @@ def weight_grad(dy: torch.Tensor, act: torch.Tensor, out: torch.Tensor, bias_dty
     return bias
 
 
-@functools.lru_cache(maxsize=None)
-def block_wgrads_together(dtype: torch.dtype, grad_dtype: Optional[torch.dtype], S: int, channels: int, inner: int, padded: int) -> bool:
-    """Whether a block's weight gradients over S rows are faster dealt out evenly in one launch (``weight_grads``)."""
-    if dtype not in _DT or grad_dtype not in _DT:
-        return False
-    a = _lib.BlockArgs()
-    a.dtype, a.grad_dtype, a.S, a.C, a.I, a.Ipad = _DT[dtype], _DT[grad_dtype], S, channels, inner, padded
-    return bool(_lib.load().mvit_block_bwd_wgrads_together(C.byref(a)))
-
-
-def weight_grads(products) -> None:
-    """Weight gradients over the same rows in one launch that deals their work out evenly.  Each of one to four products is
-    (dy, act, out, n, bias): out[:, :n] = dy^T act[:, :n], all of them bf16, and, where `bias` is given, the column sums of dy."""
-    args = (GemmArgs * len(products))()
-    K = products[0][0].shape[0]
-    for a, (dy, act, out, n, bias) in zip(args, products):
-        for t, name in ((dy, "dy"), (act, "act"), (out, "out")):
-            _rowmajor(t, f"weight_grads {name}")
-            if t.dtype != torch.bfloat16 or t.device != dy.device:
-                raise ValueError("weight_grads: bf16 operands and results on one device")
-        M = dy.shape[1]
-        if dy.shape[0] != K or act.shape[0] != K or act.shape[1] < n or out.shape[0] != M or out.shape[1] < n:
-            raise ValueError(f"weight_grads: dy {tuple(dy.shape)}, act {tuple(act.shape)}, out {tuple(out.shape)}, n={n}")
-        if bias is not None and (bias.dtype != out.dtype or bias.shape != (M,) or not bias.is_contiguous() or bias.device != dy.device):
-            raise ValueError(f"weight_grads: a bias gradient must be contiguous [{M}] of out's dtype")
-        a.dtype = a.out_dtype = _lib.BF16
-        a.trans_a = a.trans_b = a.split_k = 1
-        a.M, a.N, a.K = M, n, K
-        a.A, a.lda, a.B, a.ldb, a.C, a.ldc = dy.data_ptr(), dy.stride(0), act.data_ptr(), act.stride(0), out.data_ptr(), out.stride(0)
-        a.row_sums = _p(bias)
-    lib, st = _lib.load(), _stream(products[0][0])
-    nbytes = lib.mvit_gemm_wgrads_workspace_bytes(args, len(args))
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=products[0][0].device) if nbytes else None
-    info = {"products": [(a.M, a.N) for a in args], "K": K}
-    _lib.check(_launch("gemm_tt_together", info, lambda: lib.mvit_gemm_wgrads(args, len(args), _p(ws), nbytes, st)), "mvit_gemm_wgrads")
-
-
 # ------------------------------------------------------------------------------ attention
 
 

@@ -492,53 +492,6 @@ def test_weight_gradients_leave_the_second_stream_where_a_block_has_little_work(
     assert side(256, 1280, 3420, dtype=_lib.F32, grad=_lib.F32) == side(256, 1280, 3420, grad=_lib.F32) == side(256, 1280, 3420, split=2) == 1
 
 
-def test_weight_gradients_are_dealt_out_evenly_where_a_block_has_much_work():
-    """The line, the workspace of the pieces and what the call refuses; made-up addresses, nothing is launched."""
-    import ctypes
-
-    import torch
-
-    from mi355_vit import _lib, ops
-
-    together = lambda S, C, I, dtype=torch.bfloat16, grad=torch.bfloat16: ops.block_wgrads_together(dtype, grad, S, C, I, -(-I // 64) * 64)  # noqa: E731
-    assert [together(S, 1280, 3420) for S in (4096, 11999, 12000, 65536)] == [False, False, True, True]
-    assert [together(S, 2560, 6840) for S in (2048, 2999, 3001)] == [False, False, True] and not together(2047, 5120, 13680) and together(2048, 5120, 13680)
-    assert not together(65536, 1280, 3420, grad=torch.float32) and not together(65536, 1280, 3420, torch.float32, torch.float32)
-    assert not together(65536, 1280, 3420, grad=None) and not together(65536, 1284, 3420)
-
-    lib, fake = _lib.load(), 0x10000000
-
-    def products(shapes, K):
-        args = (_lib.GemmArgs * len(shapes))()
-        for a, (M, N) in zip(args, shapes):
-            a.dtype = a.out_dtype = _lib.BF16
-            a.trans_a = a.trans_b = a.split_k = 1
-            a.M, a.N, a.K, a.lda, a.ldb, a.ldc = M, N, K, -(-M // 8) * 8, -(-N // 8) * 8, N
-            a.A = a.B = a.C = fake
-        return args
-
-    nbytes = lambda shapes, K: lib.mvit_gemm_wgrads_workspace_bytes(products(shapes, K), len(shapes))  # noqa: E731
-    piece = (256 * 256 + 256) * 4
-    block = [(1280, 3420), (6912, 1280), (1280, 1280), (3840, 1280)]  # 305 tiles: 256 whole and 49 in slices
-    assert nbytes(block, 25524) == 49 * 5 * piece
-    assert nbytes([(4096, 4096)], 8192) == 0 and nbytes([(4096, 4096), (256, 256)], 65536) % piece == 0 != nbytes([(4096, 4096), (256, 256)], 65536)
-    assert nbytes(block, 128) == 0  # not such products
-    args, need = products(block, 25524), nbytes(block, 25524)
-    call = lambda n=4, ws=fake, size=need: lib.mvit_gemm_wgrads(args, n, ws, size, None)  # noqa: E731
-    assert lib.mvit_gemm_wgrads(None, 1, None, 0, None) == call(n=0) == call(n=5) == -1 and b"one to 4 products" in lib.mvit_last_error()
-    assert call(ws=None) == call(size=need - 1) == call(ws=fake + 8) == -1 and b"workspace" in lib.mvit_last_error()
-    for field, value in (("K", 25523), ("dtype", _lib.F32), ("out_dtype", _lib.F32), ("trans_b", 0), ("epilogue", 1), ("M", 0)):
-        old = getattr(args[1], field)
-        setattr(args[1], field, value)
-        assert call() == -1 and b"plain bf16 products" in lib.mvit_last_error(), field
-        setattr(args[1], field, old)
-    for field, value in (("A", None), ("B", fake + 8), ("C", None), ("lda", 6908), ("ldb", 1272), ("ldc", 1279), ("lda", (1 << 22) + 8)):
-        old = getattr(args[1], field)
-        setattr(args[1], field, value)
-        assert call() == -1 and b"product 1" in lib.mvit_last_error(), field
-        setattr(args[1], field, old)
-
-
 def test_windowed_backward_behind_one_call_refuses_gradients_that_share_memory():
     """Windows of head_dim 80, whose dq and dk are turned back on their way out, refuse what mvit_attn_bwd refuses; nothing is launched."""
     import ctypes

@@ -935,48 +935,6 @@ def test_gemm_wgrad_row_sums(odt, split_k, S, No, Ni):
     assert bool(((sums.cpu().double() - want).abs() <= bound).all())
 
 
-_EVEN = [
-    (129, [(8, 8)]),  # three K tiles, the last of one row; a piece of a tile and nothing else
-    (192, [(256, 256), (257, 264), (130, 72), (8, 3000)]),
-    (1000, [(520, 261), (256, 1280)]),  # a row pitch that takes 8-byte stores, one that takes single ones
-    (2056, [(1280, 3420), (6912, 1280), (1280, 1280), (3840, 1280)]),  # a round of whole tiles and 49 in slices
-    (700, [(4096, 4096)]),  # one round of whole tiles
-    (3000, [(4096, 4096), (264, 256)]),  # two tiles in many slices
-    (160, [(5120, 3584)]),  # whole tiles only, the last round not full
-]
-
-
-@pytest.mark.parametrize("S,shapes", _EVEN)
-def test_weight_gradients_dealt_out_evenly(S, shapes):
-    """One launch for several weight gradients: whole tiles, pieces of tiles, edges, every kind of store; with and without sums of the rows,
-    and with infinities and NaNs of one channel, which reach no other."""
-    _announce(f"weight gradients dealt out evenly S={S} {shapes}")
-    ops = _ops()
-    products, wants = [], []
-    for i, (No, Ni) in enumerate(shapes):
-        dy, act = _rand((S, -(-No // 8) * 8), torch.bfloat16, 2 * i).to(DEV), _rand((S, -(-Ni // 8) * 8), torch.bfloat16, 2 * i + 1).to(DEV)
-        dy[:, No:] = float("nan")  # padding of a row to 16 bytes
-        out = torch.full((No, Ni), float("nan"), dtype=torch.bfloat16, device=DEV)
-        bias = torch.full((No,), float("nan"), dtype=torch.bfloat16, device=DEV) if i % 2 == 0 else None
-        products.append((dy[:, :No], act, out, Ni, bias))
-        x, y = dy[:, :No].double(), act[:, :Ni].double()
-        wants.append((x.T @ y, x.abs().T @ y.abs(), x.sum(0), x.abs().sum(0)))
-    ops.weight_grads(products)
-    # S - 1 fp32 additions in some order, then one rounding to bf16
-    within = lambda got, want, size: bool(((got.double() - want).abs() <= size * (S * 2.0**-24) + want.abs() * 2.0**-8).all())  # noqa: E731
-    for (_, _, out, _, bias), (want, size, sums, sums_size) in zip(products, wants):
-        assert within(out, want, size)
-        assert bias is None or within(bias, sums, sums_size)
-    again = [(dy, act, torch.empty_like(out), n, None if b is None else torch.empty_like(b)) for dy, act, out, n, b in products]
-    dy, _, _, _, bias = again[0]
-    dy[S - 1, 0] = float("inf")
-    ops.weight_grads(again)
-    for i, ((_, _, out, _, b), (_, _, out2, _, b2)) in enumerate(zip(products, again)):
-        first = 1 if i == 0 else 0
-        assert torch.equal(out[first:], out2[first:]) and (b is None or torch.equal(b[first:], b2[first:])), i
-    assert bias[0] == float("inf")
-
-
 @pytest.mark.parametrize("full_tiles", [False, True])
 @pytest.mark.parametrize("S,No,split_k", [(200, 130, 1), (1000, 386, 1), (1000, 386, 3), (20011, 3834, 3)])
 def test_gemm_wgrad_row_sums_read_their_own_row_only(S, No, split_k, full_tiles, monkeypatch):
