@@ -486,13 +486,13 @@ __global__ __launch_bounds__(64 * ND, LOOP ? 3 : 5) void attn_fwd_window_rope(co
   constexpr int HD = G::HD, NT = 64 * ND, KT = 4, KK = 2, HALF = HD / 2;
   __shared__ __attribute__((aligned(16))) bf16_t lds_q[64 * G::PK], lds_k[64 * G::PK], lds_v[64 * G::PV];
 
-  // work items are dealt so that all heads of a window meet on one XCD (seg_and_head)
-  int seg = blockIdx.x / w.parts, part = blockIdx.x % w.parts;
+  // grid (parts, windows): in one dimension 65,535 windows of 205 heads would be 2^32 threads.  Work items are dealt so that all heads of a window meet on one XCD (seg_and_head)
+  int seg = blockIdx.y, part = blockIdx.x;
   const unsigned items = (unsigned)w.n_seg * (unsigned)w.parts;
   if (items % 8 == 0) {
-    const unsigned item = (blockIdx.x & 7) * (items >> 3) + (blockIdx.x >> 3);
-    seg = item / w.parts;
-    part = item % w.parts;
+    const unsigned at = blockIdx.y * (unsigned)w.parts + blockIdx.x, item = (at & 7) * (items >> 3) + (at >> 3);
+    seg = item / (unsigned)w.parts;
+    part = item % (unsigned)w.parts;
   }
   if (p.order) {
     const int listed = p.order[seg];
@@ -2350,9 +2350,9 @@ int mvit_attn_fwd_window_rope(const mvit_window_rope& w, hipStream_t stream) {
   const int most = !loop ? 1 : w.keep ? 2 : 4;
   while (2 * r.heads <= most && w.nheads % (2 * r.heads) == 0) r.heads *= 2;
   r.parts = w.nheads / r.heads;
-  const unsigned items = (unsigned)w.n_seg * (unsigned)r.parts;
-  if (r.heads > 1) hipLaunchKernelGGL((attn_fwd_window_rope<5, true>), items, 320, 0, stream, p, r);
-  else hipLaunchKernelGGL((attn_fwd_window_rope<5, false>), items, 320, 0, stream, p, r);
+  const dim3 grid((unsigned)r.parts, (unsigned)w.n_seg);
+  if (r.heads > 1) hipLaunchKernelGGL((attn_fwd_window_rope<5, true>), grid, 320, 0, stream, p, r);
+  else hipLaunchKernelGGL((attn_fwd_window_rope<5, false>), grid, 320, 0, stream, p, r);
   MVIT_CHECK_LAUNCH("attn_fwd_window_rope");
   return MVIT_OK;
 }

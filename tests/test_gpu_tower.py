@@ -276,6 +276,29 @@ def test_weight_gradients_of_many_rows_are_summed_in_the_slices_of_their_product
         F.BLOCK_CALLS, ops.OVERLAP_WGRAD = old
 
 
+def test_windowed_block_takes_as_many_windows_and_heads_as_the_two_passes():
+    """65,535 windows, all but one of them empty, of 205 heads: together more threads than one dimension of a grid holds."""
+    from mi355_vit import functional as F
+
+    H, rows, I = 205, 64, 8
+    C, g = 80 * H, torch.Generator(device=DEV).manual_seed(3)
+    cu = torch.full((65536,), rows, dtype=torch.int32, device=DEV)
+    cu[:40000] = 0
+    angle = torch.randn(rows, 40, generator=g, device=DEV).repeat(1, 2)
+    geo = F.AttnGeometry(cu, 64, H, 80, angle.cos().contiguous(), angle.sin().contiguous())
+    r = lambda *shape: (torch.randn(*shape, generator=g, device=DEV) * 0.02).to(torch.bfloat16)  # noqa: E731
+    Ipad = F.padded_inner(I)
+    W = F.BlockWeights(r(1, C) + 1, r(1, C) + 1, r(3 * C, C), r(1, 3 * C), r(C, C), r(1, C), r(2 * Ipad, C), r(1, 2 * Ipad), r(C, Ipad), r(1, C), C, I, Ipad)
+    x, old, got = r(rows, C) * 50, F.BLOCK_CALLS, {}
+    try:
+        for F.BLOCK_CALLS in (False, True):
+            y, saved = F._block_forward(x, W, geo, 1e-6)
+            got[F.BLOCK_CALLS] = [y] + [saved[i] for i in (2, 3, 4)]
+    finally:
+        F.BLOCK_CALLS = old
+    assert torch.isfinite(got[True][0]).all() and all(torch.equal(a, b) for a, b in zip(got[True], got[False]))
+
+
 _FEW_ROWS = ([[1, 2, 2]], [[1, 6, 10]], [[1, 16, 16], [1, 2, 6]], [[1, 32, 40]], [[1, 32, 40], [1, 2, 2]])
 
 
