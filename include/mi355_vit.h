@@ -252,7 +252,7 @@ int mvit_attn_bwd(const void* q, const void* k, const void* v, const void* o, co
  *   weights  norm1, norm2 [C]; wqkv [3C, C], bqkv [3C] (q | k | v stacked); wproj [C, C], bproj [C];
  *            wgu [2*Ipad, C], bgu [2*Ipad] (gate rows [0, I), up rows [Ipad, Ipad+I), padding rows zero);
  *            wdown [C, Ipad] (padding columns zero), bdown [C]
- *   geometry cu / seg_order / n_seg / max_seqlen as for mvit_attn_fwd; cos, sin fp32 [S, head_dim];
+ *   geometry cu / seg_order / n_seg / max_seqlen as for mvit_attn_fwd (windows that rotate inside do not look at seg_order); cos, sin fp32 [S, head_dim];
  *            q_lead_scale = head_dim^-1/2 * log2 e applied to the queries in the rotary pass, attn_scale = 1 / log2 e
  *   forward  x [S,C] in; written: n1 [S,C], rstd1 [S], qkv [S,3C], o [S,C] and lse [nheads,S] (read instead when
  *            skip_attention != 0: the re-run of a checkpointed block that kept them), x1 [S,C], n2 [S,C], rstd2 [S],

@@ -494,10 +494,6 @@ __global__ __launch_bounds__(64 * ND, LOOP ? 3 : 5) void attn_fwd_window_rope(co
     seg = item / (unsigned)w.parts;
     part = item % (unsigned)w.parts;
   }
-  if (p.order) {
-    const int listed = p.order[seg];
-    if ((unsigned)listed < (unsigned)w.n_seg) seg = listed;  // an entry outside the list never becomes an address
-  }
   const int s0 = p.cu[seg], L = min(p.cu[seg + 1] - s0, 64);
   if (L <= 0) return;
   const int t = threadIdx.x, l = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), g = l >> 4, r = l & 15;
@@ -2342,7 +2338,7 @@ int mvit_attn_fwd_window_rope(const mvit_window_rope& w, hipStream_t stream) {
   const int64_t C = (int64_t)w.nheads * 80;
   AttnParams p = {};
   bf16_t* qkv = static_cast<bf16_t*>(w.qkv);
-  p.q = qkv; p.k = qkv + C; p.v = qkv + 2 * C; p.out = w.o; p.lse = w.lse; p.cu = w.cu; p.order = w.order; p.total = w.S; p.nheads = w.nheads;
+  p.q = qkv; p.k = qkv + C; p.v = qkv + 2 * C; p.out = w.o; p.lse = w.lse; p.cu = w.cu; p.total = w.S; p.nheads = w.nheads;
   p.q_stride = p.k_stride = p.v_stride = 3 * C; p.o_stride = C; p.scale = w.attn_scale;
   WindowRope r{w.cos, w.sin, w.q_gain, 1, w.keep ? 1 : 0, w.n_seg, w.nheads};
   // LOOP once q, k and v are more than stays in the memory-side cache (256 MB) between the product that writes them and this
@@ -2363,7 +2359,7 @@ int mvit_attn_bwd_window_rope(const mvit_window_rope& w, const void* d_o, void* 
   const bf16_t* qkv = static_cast<const bf16_t*>(w.qkv);
   bf16_t* d = static_cast<bf16_t*>(dqkv);
   p.q = qkv; p.k = qkv + C; p.v = qkv + 2 * C; p.d_o = d_o; p.lse = w.lse; p.delta = delta; p.dq = d; p.dk = d + C; p.dv = d + 2 * C;
-  p.cu = w.cu; p.order = w.order; p.total = w.S; p.nheads = w.nheads;
+  p.cu = w.cu; p.total = w.S; p.nheads = w.nheads;
   p.q_stride = p.k_stride = p.v_stride = p.dq_stride = p.dk_stride = p.dv_stride = 3 * C; p.o_stride = p.do_stride = C; p.scale = w.attn_scale;
   if (((int64_t)w.n_seg * w.nheads) % 8 == 0) p.seg_major = 2;  // heads of a segment together on one XCD
   hipLaunchKernelGGL((attn_bwd_window_mfma<5, 4, 2, true>), dim3(1, (unsigned)w.n_seg, (unsigned)w.nheads), 256, 0, stream, p, WindowRope{w.cos, w.sin, w.q_gain, 1, 0, w.n_seg, w.nheads});

@@ -124,7 +124,7 @@ extern "C" int mvit_block_fwd(const mvit_block_args* a, mvit_stream_t stream) {
     STEP(mvit_gemm(&g, stream));
   }
   // rotary embedding of q and k in place; the queries also take the softmax scale in base-2 units.  Windows: inside their attention
-  const mvit_window_rope rotated{a->qkv, a->o, a->lse, a->cu, a->seg_order, a->cos, a->sin, a->n_seg, H, S, a->q_lead_scale, a->attn_scale, a->gu != nullptr};
+  const mvit_window_rope rotated{a->qkv, a->o, a->lse, a->cu, a->cos, a->sin, a->n_seg, H, S, a->q_lead_scale, a->attn_scale, a->gu != nullptr};
   const bool inside = !a->skip_attention && mvit_window_rope_takes(rotated, hd, a->max_seqlen, dt);
   if (inside) STEP(mvit_attn_fwd_window_rope(rotated, reinterpret_cast<hipStream_t>(stream)));
   else STEP(mvit_rope_scaled(a->qkv, a->cos, a->sin, S, 2 * H, hd, 3 * C, 0, H, a->q_lead_scale, dt, stream));
@@ -183,7 +183,7 @@ extern "C" int mvit_block_bwd(const mvit_block_args* a, mvit_stream_t stream) {
   const int64_t S = a->S, C = a->C, I = a->I, Ipad = a->Ipad;
   const int H = a->nheads, hd = a->head_dim;
   // windows: the inverse rotation of dq and dk is in their attention's backward
-  const mvit_window_rope rotated{a->qkv, a->o, a->lse, a->cu, a->seg_order, a->cos, a->sin, a->n_seg, H, S, a->q_lead_scale, a->attn_scale, true};
+  const mvit_window_rope rotated{a->qkv, a->o, a->lse, a->cu, a->cos, a->sin, a->n_seg, H, S, a->q_lead_scale, a->attn_scale, true};
   const bool inside = mvit_window_rope_takes(rotated, hd, a->max_seqlen, dt) && mvit_aligned16(a->dqkv) && mvit_aligned16(a->dn);
   if (inside) {  // as mvit_attn_bwd asks of its outputs
     const struct { const void* ptr; int64_t cols; const char* name; } ins[] = {{a->qkv, 3 * C, "qkv"}, {a->o, C, "o"}, {a->dn, C, "d_o"}};

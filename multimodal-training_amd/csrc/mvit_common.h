@@ -43,11 +43,12 @@ static inline bool mvit_aligned16(const void* p) { return (reinterpret_cast<uint
 
 // Launches that several steps of a block share (block.cpp).
 // Attention over windows of at most 64 tokens with the rotary embedding of q and k inside (bf16, head_dim 80; qkv [S, 3 * nheads * 80]).  The rotated
-// q and k replace the others in qkv where `keep` is set.  `mvit_window_rope_takes`: whether a block's tensors suit it.
+// q and k replace the others in qkv where `keep` is set, so every window is taken once, in its own place: an order of segments (windows are about
+// alike) is not looked at, since one that names a window twice would have it rotated twice.  `mvit_window_rope_takes`: whether a block's tensors suit it.
 struct mvit_window_rope {
   void *qkv, *o;
   float* lse;
-  const int32_t *cu, *order;
+  const int32_t* cu;
   const float *cos, *sin;
   int n_seg, nheads;
   int64_t S;

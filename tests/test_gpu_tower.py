@@ -276,6 +276,35 @@ def test_weight_gradients_of_many_rows_are_summed_in_the_slices_of_their_product
         F.BLOCK_CALLS, ops.OVERLAP_WGRAD = old
 
 
+@pytest.mark.parametrize("kind", ["permuted", "named twice", "outside the list"])
+def test_windows_that_rotate_are_taken_once_each_whatever_the_order_of_segments_says(kind):
+    """q and k are rotated in place inside the windows' attention: an order that names a window twice must not have it rotated twice."""
+    from mi355_vit import functional as F
+
+    H, C, I, g = 16, 1280, 64, torch.Generator().manual_seed(5)
+    lengths = torch.randint(1, 65, (97,), generator=g)
+    cu = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)]).to(torch.int32).to(DEV)
+    rows, n = int(lengths.sum()), lengths.numel()
+    order = torch.randperm(n, generator=g) if kind == "permuted" else torch.randint(0, n, (n,), generator=g)
+    if kind == "outside the list":
+        order[::2] = n + order[::2]
+    angle = torch.randn(rows, 40, generator=g).repeat(1, 2).to(DEV)
+    tables = angle.cos().contiguous(), angle.sin().contiguous()
+    r = lambda *shape: (torch.randn(*shape, generator=g) * 0.05).to(torch.bfloat16).to(DEV)  # noqa: E731
+    Ipad = F.padded_inner(I)
+    W = F.BlockWeights(r(1, C) + 1, r(1, C) + 1, r(3 * C, C), r(1, 3 * C), r(C, C), r(1, C), r(2 * Ipad, C), r(1, 2 * Ipad), r(C, Ipad), r(1, C), C, I, Ipad)
+    x, dy = r(rows, C) * 20, r(rows, C) * 20
+
+    def run(order):
+        geo = F.AttnGeometry(cu, 64, H, 80, *tables, order)
+        y, saved = F._block_forward(x, W, geo, 1e-6)
+        kept = [saved[i].clone() for i in (2, 3, 4)]
+        dx, grads = F._block_backward(dy, x, saved, W, geo, torch.bfloat16)
+        return [y, *kept, F._block_forward(x, W, geo, 1e-6, for_backward=False)[0], dx, *grads]
+
+    assert all(torch.equal(a, b) for a, b in zip(run(order.to(torch.int32).to(DEV)), run(None)))
+
+
 def test_windowed_block_takes_as_many_windows_and_heads_as_the_two_passes():
     """65,535 windows, all but one of them empty, of 205 heads: together more threads than one dimension of a grid holds."""
     from mi355_vit import functional as F
