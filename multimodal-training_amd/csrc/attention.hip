@@ -1983,17 +1983,22 @@ __global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const Attn
   const int l = threadIdx.x & 63, wv = threadIdx.x >> 6, g = l >> 4, r = l & 15;
   const float c = p.scale * LOG2E;
   static_assert(NB == 1, "a wave's sixteen rows of the k and v tiles are its own behind pass A");
+  // lanes hand rows of LDS to each other within a wave, in both directions: what was read before the rows change, what was written before it is read
+  auto lanes_meet = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
   // results leave as whole chunks of rows: turned in the wave's own rows of a tile that no other wave reads any more
   auto turn_in = [&](bf16_t* tile, const bf16x4 (&v)[ND]) {
+    lanes_meet();
 #pragma unroll
     for (int d = 0; d < ND; ++d) *reinterpret_cast<bf16x4*>(tile + (wv * 16 + r) * PK + 16 * d + 4 * g) = v[d];
   };
   auto leave = [&](bf16_t* tile, const bf16x4 (&v)[ND], bf16_t* dst, int64_t stride) {
     const bf16_t* turn = tile + wv * 16 * PK;
     turn_in(tile, v);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    lanes_meet();
 #pragma unroll
     for (int i = 0; i < (16 * G::CH + 63) / 64; ++i) {
       const int at = l + 64 * i, rr = at / G::CH, cc = at % G::CH;
@@ -2183,9 +2188,7 @@ __global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const Attn
       leave(lds_k, a, DK, p.dk_stride);
     } else {
       turn_in(lds_k, a);
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      lanes_meet();
 #pragma unroll
       for (int i = 0; i < PAIRS; ++i) {
         const int at = l + 64 * i, rr = at / ND, cc = at % ND, row = wv * 16 + rr;
