@@ -1964,10 +1964,10 @@ __global__ __launch_bounds__(64 * NWAVES) void attn_bwd_dq_mfma(const AttnParams
 // ROPE: dQ and dK are turned back by the rotary embedding's angles on their way out (with the roundings of the pass of its own, which read and wrote both
 // once more); dQ waits in LDS for the tables, which are fetched once for both and travel while dK and dV are rounded.  ms per step, pass of its own /
 // inside: 1,024 rows 12.0 / 11.6, 4,096 checkpointed 27.9 / 27.6, 14,336 62.2 / 61.0, 25,524 104.9 / 104.3, 36,864 239.6 / 238.3.
-template <int ND, int NW, int MINW = 1, bool ROPE = false>  // NW waves share the staged tiles; wave w owns query / key blocks [w*4/NW, (w+1)*4/NW)
-__global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const AttnParams p, const WindowRope rope) {
+template <int ND, bool ROPE = false>  // four waves share the staged tiles; wave w owns queries and keys [16 w, 16 w + 16)
+__global__ __launch_bounds__(256, 2) void attn_bwd_window_mfma(const AttnParams p, const WindowRope rope) {
   using G = Geo<ND>;
-  constexpr int HD = G::HD, R = 64, PK = G::PK, NB = 4 / NW;  // NB 16-row blocks per wave
+  constexpr int HD = G::HD, R = 64, PK = G::PK;
   __shared__ __attribute__((aligned(16))) bf16_t lds_q[R * PK];
   __shared__ __attribute__((aligned(16))) bf16_t lds_k[R * PK];
   __shared__ __attribute__((aligned(16))) bf16_t lds_v[R * PK];
@@ -1982,14 +1982,13 @@ __global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const Attn
   if (L <= 0) return;
   const int l = threadIdx.x & 63, wv = threadIdx.x >> 6, g = l >> 4, r = l & 15;
   const float c = p.scale * LOG2E;
-  static_assert(NB == 1, "a wave's sixteen rows of the k and v tiles are its own behind pass A");
   // lanes hand rows of LDS to each other within a wave, in both directions: what was read before the rows change, what was written before it is read
   auto lanes_meet = [] {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
-  // results leave as whole chunks of rows: turned in the wave's own rows of a tile that no other wave reads any more
+  // results leave as whole chunks of rows: turned in the wave's own sixteen rows of the k or v tile, which no other wave reads behind pass A
   auto turn_in = [&](bf16_t* tile, const bf16x4 (&v)[ND]) {
     lanes_meet();
 #pragma unroll
@@ -2008,7 +2007,7 @@ __global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const Attn
   bf16x4 dq_out[ND];
   bf16_t* DQ = static_cast<bf16_t*>(p.dq) + (int64_t)s0 * p.dq_stride + (int64_t)h * HD;
   {
-    TileStager<ND, R, PK, 64 * NW> sq, sk, sv, sdo;
+    TileStager<ND, R, PK, 256> sq, sk, sv, sdo;
     sq.init(p.q_stride);
     sk.init(p.k_stride);
     sv.init(p.v_stride);
@@ -2044,10 +2043,8 @@ __global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const Attn
       }
     }
     float* DELTA = p.delta + (int64_t)h * p.total + s0;
-#pragma unroll 1
-    for (int qb = wv * NB; qb < (wv + 1) * NB; ++qb) {
-      if (qb * 16 >= L) break;
-      const int qi = qb * 16 + r;
+    if (wv * 16 < L) {
+      const int qi = wv * 16 + r;
       RowFrag<ND> qf, dof;
       load_rowfrag_lds<ND, PK>(qf, lds_q, qi, g);
       load_rowfrag_lds<ND, PK>(dof, lds_do, qi, g);
@@ -2058,7 +2055,7 @@ __global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const Attn
       for (int kc = 0; kc < 2; ++kc)
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-          const f32x4 sc = dot_frag<ND>(ka[kc][t], qf);  // S[q = qb*16+r][key = kc*32+t*16+4g+i]
+          const f32x4 sc = dot_frag<ND>(ka[kc][t], qf);  // S[q = wv*16+r][key = kc*32+t*16+4g+i]
           dp[kc][t] = dot_frag<ND>(va[kc][t], dof);      // dP, same layout
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
@@ -2069,7 +2066,7 @@ __global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const Attn
           }
         }
       part += __shfl_xor(part, 16);
-      part += __shfl_xor(part, 32);  // lanes r, r+16, r+32, r+48 share query qb*16+r
+      part += __shfl_xor(part, 32);  // lanes r, r+16, r+32, r+48 share query wv*16+r
       if (g == 0) {
         lds_delta[qi] = part;
         if (qi < L) DELTA[qi] = part;
@@ -2093,24 +2090,20 @@ __global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const Attn
 #pragma unroll
         for (int i = 0; i < 4; ++i) dq_out[d][i] = (bf16_t)(dq[d][i] * p.scale);
     }
-    for (int q = 16 * ((L + 15) / 16) + (int)threadIdx.x; q < R; q += 64 * NW) lds_delta[q] = 0.f;  // query blocks that were skipped
+    for (int q = 16 * ((L + 15) / 16) + (int)threadIdx.x; q < R; q += 256) lds_delta[q] = 0.f;  // query blocks that were skipped
   }
   __syncthreads();
 
   // ---- pass B: dV^T += dO^T P, dK^T += Q^T dS per 16-key block, queries in two tiles of 32
   {
-    RowFrag<ND> kf[NB], vf[NB];
-    f32x4 dk[NB][ND], dv[NB][ND];
-    const int key0 = wv * NB * 16;  // this wave's first key
+    RowFrag<ND> kf, vf;
+    f32x4 dk[ND], dv[ND];
+    load_rowfrag_lds<ND, PK>(kf, lds_k, wv * 16 + r, g);
+    load_rowfrag_lds<ND, PK>(vf, lds_v, wv * 16 + r, g);
 #pragma unroll
-    for (int kb = 0; kb < NB; ++kb) {
-      load_rowfrag_lds<ND, PK>(kf[kb], lds_k, key0 + kb * 16 + r, g);
-      load_rowfrag_lds<ND, PK>(vf[kb], lds_v, key0 + kb * 16 + r, g);
-#pragma unroll
-      for (int d = 0; d < ND; ++d) {
-        dk[kb][d] = f32x4{0.f, 0.f, 0.f, 0.f};
-        dv[kb][d] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
+    for (int d = 0; d < ND; ++d) {
+      dk[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+      dv[d] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     if (!ROPE && wv * 16 < L) leave(lds_v, dq_out, DQ, p.dq_stride);
     if (ROPE) turn_in(lds_v, dq_out);  // stays there until the tables are fetched, once for both
@@ -2134,27 +2127,24 @@ __global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const Attn
         qt[d] = tr_pair(tq + off, tq + off + 16 * PK);
         dt_[d] = tr_pair(tdo + off, tdo + off + 16 * PK);
       }
+      f32x4 pv[2], ds[2];
 #pragma unroll
-      for (int kb = 0; kb < NB; ++kb) {
-        f32x4 pv[2], ds[2];
+      for (int t = 0; t < 2; ++t) {
+        const f32x4 sc = dot_frag<ND>(qa[t], kf);   // S[q = qs+t*16+4g+i][key = wv*16+r]
+        const f32x4 dpp = dot_frag<ND>(da[t], vf);  // dP, same layout
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const f32x4 sc = dot_frag<ND>(qa[t], kf[kb]);   // S[q = qs+t*16+4g+i][key = kb*16+r]
-          const f32x4 dpp = dot_frag<ND>(da[t], vf[kb]);  // dP, same layout
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float x = __builtin_amdgcn_exp2f(sc[i] - lse2[t][i]);
-            pv[t][i] = x;
-            ds[t][i] = x * (dpp[i] - dl[t][i]);
-          }
+        for (int i = 0; i < 4; ++i) {
+          const float x = __builtin_amdgcn_exp2f(sc[i] - lse2[t][i]);
+          pv[t][i] = x;
+          ds[t][i] = x * (dpp[i] - dl[t][i]);
         }
-        const bf16x8 pb = pack8(pv[0], pv[1]);
-        const bf16x8 dsb = pack8(ds[0], ds[1]);
+      }
+      const bf16x8 pb = pack8(pv[0], pv[1]);
+      const bf16x8 dsb = pack8(ds[0], ds[1]);
 #pragma unroll
-        for (int d = 0; d < ND; ++d) {
-          dv[kb][d] = mfma32(dt_[d], pb, dv[kb][d]);
-          dk[kb][d] = mfma32(qt[d], dsb, dk[kb][d]);
-        }
+      for (int d = 0; d < ND; ++d) {
+        dv[d] = mfma32(dt_[d], pb, dv[d]);
+        dk[d] = mfma32(qt[d], dsb, dk[d]);
       }
     }
     bf16_t* DK = static_cast<bf16_t*>(p.dk) + (int64_t)s0 * p.dk_stride + (int64_t)h * HD;
@@ -2181,8 +2171,8 @@ __global__ __launch_bounds__(64 * NW, MINW) void attn_bwd_window_mfma(const Attn
     for (int d = 0; d < ND; ++d)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        a[d][i] = (bf16_t)(dk[0][d][i] * LN2);  // dS^T (Q scale log2e) / log2e
-        b[d][i] = (bf16_t)dv[0][d][i];
+        a[d][i] = (bf16_t)(dk[d][i] * LN2);  // dS^T (Q scale log2e) / log2e
+        b[d][i] = (bf16_t)dv[d][i];
       }
     if constexpr (!ROPE) {
       leave(lds_k, a, DK, p.dk_stride);
@@ -2263,7 +2253,7 @@ int launch_bwd_mfma(const AttnParams& p, int n_seg, int max_seqlen, hipStream_t 
       // four waves x 16 rows: ~160 registers, three work-groups (12 waves) per CU to cover the load -> MFMA -> store latency
       AttnParams pw = p;
       if (((int64_t)n_seg * p.nheads) % 8 == 0) pw.seg_major = 2;  // heads of a segment together on one XCD
-      hipLaunchKernelGGL((attn_bwd_window_mfma<ND, 4, 2>), grid, 256, 0, s, pw, WindowRope{});  // computes delta itself
+      hipLaunchKernelGGL((attn_bwd_window_mfma<ND>), grid, 256, 0, s, pw, WindowRope{});  // computes delta itself
     } else {
       hipLaunchKernelGGL((attn_bwd_dkdv_mfma<ND, 1, 4>), grid, 64, 0, s, p);
       hipLaunchKernelGGL((attn_bwd_dq_mfma<ND, 1, 4>), grid, 64, 0, s, p);
@@ -2365,7 +2355,7 @@ int mvit_attn_bwd_window_rope(const mvit_window_rope& w, const void* d_o, void* 
   p.cu = w.cu; p.total = w.S; p.nheads = w.nheads;
   p.q_stride = p.k_stride = p.v_stride = p.dq_stride = p.dk_stride = p.dv_stride = 3 * C; p.o_stride = p.do_stride = C; p.scale = w.attn_scale;
   if (((int64_t)w.n_seg * w.nheads) % 8 == 0) p.seg_major = 2;  // heads of a segment together on one XCD
-  hipLaunchKernelGGL((attn_bwd_window_mfma<5, 4, 2, true>), dim3(1, (unsigned)w.n_seg, (unsigned)w.nheads), 256, 0, stream, p, WindowRope{w.cos, w.sin, w.q_gain, 1, 0, w.n_seg, w.nheads});
+  hipLaunchKernelGGL((attn_bwd_window_mfma<5, true>), dim3(1, (unsigned)w.n_seg, (unsigned)w.nheads), 256, 0, stream, p, WindowRope{w.cos, w.sin, w.q_gain, 1, 0, w.n_seg, w.nheads});
   MVIT_CHECK_LAUNCH("attn_bwd_window_rope");
   return MVIT_OK;
 }
