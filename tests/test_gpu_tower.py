@@ -305,6 +305,51 @@ def test_windows_that_rotate_are_taken_once_each_whatever_the_order_of_segments_
     assert all(torch.equal(a, b) for a, b in zip(run(order.to(torch.int32).to(DEV)), run(None)))
 
 
+@pytest.mark.parametrize("where", ["a token", "a channel of v", "a channel of q", "a gradient"])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_windows_with_the_rotation_inside_keep_infinities_and_nans_where_two_passes_do(value, where):
+    """One token's row (NaN behind its norm), one channel of one head, one row of the incoming gradient; ragged windows."""
+    from mi355_vit import functional as F
+
+    H, C, I, g = 3, 240, 64, torch.Generator().manual_seed(9)
+    lengths = torch.tensor([64, 17, 1, 50, 33, 64, 16])
+    cu = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)]).to(torch.int32).to(DEV)
+    rows = int(lengths.sum())
+    angle = torch.randn(rows, 40, generator=g).repeat(1, 2).to(DEV)
+    geo = F.AttnGeometry(cu, 64, H, 80, angle.cos().contiguous(), angle.sin().contiguous())
+    r = lambda *shape: (torch.randn(*shape, generator=g) * 0.05).to(torch.bfloat16).to(DEV)  # noqa: E731
+    Ipad = F.padded_inner(I)
+    W = F.BlockWeights(r(1, C) + 1, r(1, C) + 1, r(3 * C, C), r(1, 3 * C), r(C, C), r(1, C), r(2 * Ipad, C), r(1, 2 * Ipad), r(C, Ipad), r(1, C), C, I, Ipad)
+    x, dy = r(rows, C) * 20, r(rows, C) * 20
+    if where == "a token":
+        x[70, 11] = value  # in the second window
+    elif where == "a gradient":
+        dy[70, 11] = value
+    else:
+        W.bqkv[0, (2 * C if where == "a channel of v" else 0) + 80 + 7] = value  # of the second head
+    old = F.BLOCK_CALLS
+    same = lambda a, b: torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))  # noqa: E731
+    try:
+        got = {}
+        for one_call in (True, False):
+            F.BLOCK_CALLS = one_call
+            y0, saved0 = F._block_forward(x, W, geo, 1e-6, for_backward=False)
+            y, saved = F._block_forward(x, W, geo, 1e-6)
+            kept = [saved[i].clone() for i in (2, 3, 4)]
+            dx, grads = F._block_backward(dy, x, tuple(saved), W, geo, torch.bfloat16)
+            got[one_call] = [y0, saved0[3], saved0[4], y, *kept, dx, *grads]
+    finally:
+        F.BLOCK_CALLS = old
+    assert all(same(a, b) for a, b in zip(got[True], got[False]))
+    y, o = got[True][3], got[True][5]
+    if where == "a token":  # its window and no other
+        hit = torch.isnan(y).any(1).cpu()
+        assert hit[64:81].any() and not hit[:64].any() and not hit[81:].any()
+    elif where != "a gradient":  # its head and no other
+        hit = (~torch.isfinite(o.view(rows, H, 80))).any(2).cpu()
+        assert hit[:, 1].all() and not hit[:, 0].any() and not hit[:, 2].any()
+
+
 def test_windowed_block_takes_as_many_windows_and_heads_as_the_two_passes():
     """65,535 windows, all but one of them empty, of 205 heads: together more threads than one dimension of a grid holds."""
     from mi355_vit import functional as F
