@@ -2325,7 +2325,7 @@ bool strided_rows_overlap(const void* a, int64_t pa, const void* b, int64_t pb, 
 
 bool mvit_window_rope_takes(const mvit_window_rope& w, int head_dim, int max_seqlen, int dtype) {
   return dtype == MVIT_BF16 && head_dim == 80 && max_seqlen > 0 && max_seqlen <= 64 && w.n_seg > 0 && w.n_seg <= 65535 && w.nheads > 0 && w.nheads <= 65535 && w.S > 0 &&
-         mvit_aligned16(w.qkv) && mvit_aligned16(w.o) && mvit_aligned16(w.cos) && mvit_aligned16(w.sin);
+         mvit_aligned16(w.qkv) && mvit_aligned16(w.o) && mvit_aligned16(w.lse) && mvit_aligned16(w.cos) && mvit_aligned16(w.sin);
 }
 int mvit_attn_fwd_window_rope(const mvit_window_rope& w, hipStream_t stream) {
   const int64_t C = (int64_t)w.nheads * 80;

@@ -350,6 +350,37 @@ def test_windows_with_the_rotation_inside_keep_infinities_and_nans_where_two_pas
         assert hit[:, 1].all() and not hit[:, 0].any() and not hit[:, 2].any()
 
 
+def test_windowed_block_refuses_the_tensors_that_the_attention_calls_refuse():
+    """A log-sum-exp that does not start at a 16-byte address, in both directions, as mvit_attn_fwd and mvit_attn_bwd answer it."""
+    import ctypes
+
+    from mi355_vit import _lib
+    from mi355_vit import functional as F
+    from mi355_vit import ops
+
+    H, C, I, rows, g = 2, 160, 64, 100, torch.Generator().manual_seed(2)
+    cu = torch.tensor([0, 64, 100], dtype=torch.int32, device=DEV)
+    angle = torch.randn(rows, 40, generator=g).repeat(1, 2).to(DEV)
+    geo = F.AttnGeometry(cu, 64, H, 80, angle.cos().contiguous(), angle.sin().contiguous())
+    r = lambda *shape: (torch.randn(*shape, generator=g) * 0.05).to(torch.bfloat16).to(DEV)  # noqa: E731
+    Ipad = F.padded_inner(I)
+    W = F.BlockWeights(r(1, C) + 1, r(1, C) + 1, r(3 * C, C), r(1, 3 * C), r(C, C), r(1, C), r(2 * Ipad, C), r(1, 2 * Ipad), r(C, Ipad), r(1, C), C, I, Ipad)
+    x, dy = r(rows, C) * 20, r(rows, C) * 20
+    _, saved = F._block_forward(x, W, geo, 1e-6)
+    kept = [t.clone() for t in saved]
+    moved = torch.empty(H * rows + 1, dtype=torch.float32, device=DEV)[1:].view(H, rows)
+    moved.copy_(kept[4])
+    F._block_backward(dy, x, tuple(kept), W, geo, torch.bfloat16)
+    with pytest.raises(RuntimeError, match="unaligned"):
+        F._block_backward(dy, x, tuple(kept[:4] + [moved] + kept[5:]), W, geo, torch.bfloat16)
+    a = F._block_args(x, W, geo, 1e-6)
+    a.rstd1, a.n1, a.qkv, a.o, a.lse, a.x1, a.rstd2, a.n2, a.gu, a.h = (t.data_ptr() for t in kept)
+    y = torch.empty_like(x)
+    a.x2, a.lse = y.data_ptr(), moved.data_ptr()
+    with pytest.raises(RuntimeError, match="unaligned"):
+        _lib.check(_lib.load().mvit_block_fwd(ctypes.byref(a), ops._stream(x)), "mvit_block_fwd")
+
+
 def test_windowed_block_takes_as_many_windows_and_heads_as_the_two_passes():
     """65,535 windows, all but one of them empty, of 205 heads: together more threads than one dimension of a grid holds."""
     from mi355_vit import functional as F
