@@ -33,7 +33,7 @@ typedef void* mvit_stream_t; /* hipStream_t */
 enum { MVIT_F32 = 0, MVIT_BF16 = 1 };
 enum { MVIT_OK = 0, MVIT_ERR_ARG = -1, MVIT_ERR_LAUNCH = -2, MVIT_ERR_UNSUPPORTED = -3 };
 
-/* 205: without 204's mvit_gemm_wgrads, whose sums were further from the exact ones than those of slices.
+/* 205: without 204's mvit_gemm_wgrads, whose sums were further from the exact ones than those of slices; mvit_gemm_full_round_rows.
  * 203: mvit_gemm_args ends with overlapped; mvit_gemm_wgrad_split_k answers for a product that has the GPU to itself.
  * 202: mvit_gemm_args ends with colsum_rows.
  * 201: mvit_gemm_args has row_sums at its end.
@@ -203,9 +203,12 @@ typedef struct mvit_gemm_args {
 int mvit_gemm(const mvit_gemm_args* args, mvit_stream_t stream);
 
 /* Host-only: the tile with which a bf16 product of this form and shape is computed on n_cu compute units, biases given, operands
- * aligned, neither K slices nor column sums: tile[0] x tile[1] (rows x columns; 0: no tile fits, a kernel of 256 rows), tile[2]
+ * aligned, neither K slices nor column sums, where it is one launch: tile[0] x tile[1] (rows x columns; 0: no tile fits, a kernel of 256 rows), tile[2]
  * work-groups to a unit, tile[3] whether a wave of each reads B ahead of the main loop. */
 int mvit_gemm_tile(int trans_a, int trans_b, int epilogue, int64_t M, int64_t N, int64_t K, int overlapped, int n_cu, int32_t* tile);
+/* Host-only: the rows of such a product that go in a launch of their own, full rounds of 256 x 256 tiles, before the rest, whose tile is
+ * that of a product of M minus these rows (0: one launch; -1: no such product). */
+int64_t mvit_gemm_full_round_rows(int trans_a, int trans_b, int epilogue, int64_t M, int64_t N, int64_t K, int overlapped, int n_cu);
 /* Host-only: the split_k to ask for when C[out_rows, out_cols] is a weight gradient contracted over k tokens (bf16). */
 int mvit_gemm_wgrad_split_k(int64_t out_rows, int64_t out_cols, int64_t k);
 /* Host-only: the same for a product that shares the GPU with another stream's (`overlapped`). */

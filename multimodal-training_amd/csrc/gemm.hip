@@ -1189,7 +1189,8 @@ bool pp_takes(GemmTiledKind kind, int64_t k_chunk, int64_t k_last) {  // at leas
 // of the launch (clock, and operands that the L2s and the memory-side cache no longer hold): a launch of r rounds takes 5 % longer per round beyond the
 // first on 128 x 128 tiles, 15 % on 64-row ones.  us, input gradients of 1280 columns, the mean above -> this: K = 6912 13,312 rows 268 -> 215,
 // 14,336 267 -> 223, 16,384 282 -> 294 (4 % off the best), 18,432 and 27,648 284 and 432 (328 and 540 without the growth); K = 3840 13,312 rows
-// 155 -> 129, 16,384 160 -> 148; 5120 columns, K = 5120 (the merger) 3,584 rows 202 -> 171.  Over 107 sizes from 1,024 to 65,536 rows the
+// 155 -> 129, 16,384 160 -> 148; 5120 columns, K = 5120 (the merger) 3,584 rows 202 -> 171.  (One launch each; rows_in_full_rounds then cuts some in two: K = 6912,
+// 14,336 rows 194.)  Over 107 sizes from 1,024 to 65,536 rows the
 // choice is 0.1 % off the fastest tile on average.
 constexpr double PP_STEP_US = 1.15, PP_TILE_US = 7., PP_SWIGLU_TILE_US = 11.;
 struct TileChoice {
@@ -1560,12 +1561,22 @@ static int wgrad_split_k(int64_t out_rows, int64_t out_cols, int64_t k, bool ove
   return best;
 }
 
-extern "C" int mvit_gemm_tile(int trans_a, int trans_b, int epilogue, int64_t M, int64_t N, int64_t K, int overlapped, int n_cu, int32_t* tile) {
-  MVIT_REQUIRE(tile && M > 0 && N > 0 && K > 0 && n_cu > 0, "gemm_tile: null pointer or bad shape");
+static GemmTiledKind bf16_kind(int trans_a, int trans_b, int epilogue, int64_t N) {
   GemmParams p{};
   p.N = N;
   p.bias = p.bias2 = &p;  // as a product with biases has them
-  const GemmTiledKind kind = tiled_kind(MVIT_BF16, MVIT_BF16, trans_a, trans_b, epilogue, p);
+  return tiled_kind(MVIT_BF16, MVIT_BF16, trans_a, trans_b, epilogue, p);
+}
+
+extern "C" int64_t mvit_gemm_full_round_rows(int trans_a, int trans_b, int epilogue, int64_t M, int64_t N, int64_t K, int overlapped, int n_cu) {
+  const GemmTiledKind kind = bf16_kind(trans_a, trans_b, epilogue, N);
+  if (M <= 0 || N <= 0 || K <= 0 || n_cu <= 0 || kind == TILED_NONE) return -1;
+  return rows_in_full_rounds(kind, M, N, K, n_cu, overlapped != 0);
+}
+
+extern "C" int mvit_gemm_tile(int trans_a, int trans_b, int epilogue, int64_t M, int64_t N, int64_t K, int overlapped, int n_cu, int32_t* tile) {
+  MVIT_REQUIRE(tile && M > 0 && N > 0 && K > 0 && n_cu > 0, "gemm_tile: null pointer or bad shape");
+  const GemmTiledKind kind = bf16_kind(trans_a, trans_b, epilogue, N);
   if (kind == TILED_NONE) return mvit_set_error(MVIT_ERR_UNSUPPORTED, "gemm_tile: trans_a=%d trans_b=%d epilogue %d of %lld columns has no choice of tiles", trans_a, trans_b, epilogue, (long long)N);
   const TileChoice c = choose_tile(kind, M, N, K, K, 1, n_cu, overlapped != 0);
   tile[0] = c.bm; tile[1] = c.bn;

@@ -116,7 +116,7 @@ PROTOTYPES = {
     "mvit_block_bwd_uses_side_stream": [C.POINTER(BlockArgs)],
     "mvit_attn_bwd": [_vp] * 10 + [_i64, _vp, _vp] + [_i32, _i32, _i64, _i32, _i32] + [_i64] * 8 + [_f32, _i32, _vp],
 }
-EXPORTS = sorted(list(PROTOTYPES) + ["mvit_version", "mvit_last_error", "mvit_attn_bwd_delta_elems", "mvit_block_bwd_workspace_bytes"])
+EXPORTS = sorted(list(PROTOTYPES) + ["mvit_version", "mvit_last_error", "mvit_attn_bwd_delta_elems", "mvit_block_bwd_workspace_bytes", "mvit_gemm_full_round_rows"])
 HEADER_VERSION = 205  # MVIT_VERSION of include/mi355_vit.h these prototypes were written for
 
 _lib = None
@@ -144,6 +144,8 @@ def load() -> C.CDLL:
         lib.mvit_attn_bwd_delta_elems.restype = _i64
         lib.mvit_block_bwd_workspace_bytes.argtypes = [C.POINTER(BlockArgs)]
         lib.mvit_block_bwd_workspace_bytes.restype = _i64
+        lib.mvit_gemm_full_round_rows.argtypes = [_i32, _i32, _i32, _i64, _i64, _i64, _i32, _i32]
+        lib.mvit_gemm_full_round_rows.restype = _i64
         if lib.mvit_version() != HEADER_VERSION:
             raise RuntimeError(f"{LIB_PATH} reports interface version {lib.mvit_version()}, these bindings are written for {HEADER_VERSION}: rebuild the library")
         _lib = lib

@@ -511,6 +511,17 @@ def test_windowed_backward_behind_one_call_refuses_gradients_that_share_memory()
         assert lib.mvit_block_bwd(ctypes.byref(a), None) == -1 and b"dqkv overlaps " + shared.encode() in lib.mvit_last_error()
 
 
+def test_rows_in_full_rounds_are_named_for_forward_products_and_lone_input_gradients():
+    from mi355_vit import _lib
+
+    rows = _lib.load().mvit_gemm_full_round_rows
+    assert rows(0, 1, 0, 14336, 1280, 6912, 0, 256) == rows(0, 1, 0, 14336, 1280, 3840, 0, 256) == rows(0, 0, 2, 14336, 1280, 1280, 0, 256) == 51 * 256
+    assert rows(0, 1, 6, 3584, 5120, 3584, 0, 256) == 12 * 256 and rows(0, 0, 2, 14336, 1280, 1280, 1, 256) == 51 * 256
+    assert rows(0, 1, 0, 14336, 1280, 6912, 1, 256) == rows(0, 1, 5, 14336, 3456, 1280, 0, 256) == rows(1, 1, 0, 14336, 1280, 6912, 0, 256) == 0
+    assert rows(0, 1, 0, 13056, 1280, 6912, 0, 256) == rows(0, 1, 0, 1000, 1280, 6912, 0, 256) == rows(0, 1, 0, 14336, 1280, 128, 0, 256) == 0
+    assert rows(1, 0, 0, 14336, 1280, 6912, 0, 256) == rows(0, 1, 0, 0, 1280, 6912, 0, 256) == rows(0, 1, 0, 14336, 1280, 6912, 0, 0) == -1
+
+
 def _tile(rows, cols, k, trans_b=1, epilogue=0, overlapped=0):
     import ctypes
 

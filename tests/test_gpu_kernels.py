@@ -500,6 +500,8 @@ def test_gemm_input_gradient_in_full_rounds_and_the_rest_has_the_bits_of_one_lau
     from mi355_vit import _lib as E
 
     K, dtype = 520, torch.bfloat16
+    head = E.load().mvit_gemm_full_round_rows(0, 1, E.EPI_GELU_BWD if gelu else E.EPI_NONE, M, N, K, 0, torch.cuda.get_device_properties(0).multi_processor_count)
+    assert 0 < head < M and head % 256 == 0
     dy, w, x = _rand((M, K), dtype, 1).to(DEV), _rand((K, N), dtype, 2, K**-0.5).to(DEV), _rand((M, N), dtype, 3).to(DEV)
 
     def run():
@@ -526,6 +528,9 @@ def test_gemm_rows_in_full_rounds_and_the_rest_give_the_same_bits_as_one_launch(
     K, dtype = 1280, torch.bfloat16
     if epi.startswith("swiglu"):
         N //= 2
+    which = {"none": E.EPI_NONE, "bias": E.EPI_BIAS, "bias_res": E.EPI_BIAS_RES, "gelu": E.EPI_BIAS_GELU}.get(epi, E.EPI_SWIGLU)
+    head = E.load().mvit_gemm_full_round_rows(0, 0, which, M, N, K, 0, torch.cuda.get_device_properties(0).multi_processor_count)
+    assert 0 < head < M and head % 256 == 0
     a, b, b2 = (_rand(s, dtype, i, sc).to(DEV) for i, (s, sc) in enumerate((((M, K), 1.0), ((N, K), K**-0.5), ((N, K), K**-0.5))))
     bias, bias2, res = _rand((N,), dtype, 3).to(DEV), _rand((N,), dtype, 4).to(DEV), _rand((M, N), dtype, 5).to(DEV)
     kw = {"none": {}, "bias": dict(epilogue=E.EPI_BIAS, bias=bias), "bias_res": dict(epilogue=E.EPI_BIAS_RES, bias=bias, residual=res),
