@@ -136,6 +136,7 @@ def measured_traffic_bytes(workload: str, tag: str):
     return None
 
 
+# The trace issues a block's launches one by one; names of what it times
 KERNEL_NAMES = {
     "gemm_nn_epi0": "gemm_pp_kernel / gemm_small_kernel<TO, TA=false, TB=false, EPI=NONE>",
     "gemm_nn_epi1": "gemm_pp_kernel / gemm_small_kernel<TO, TA=false, TB=false, EPI=BIAS>",
@@ -143,14 +144,17 @@ KERNEL_NAMES = {
     "gemm_nn_epi3": "gemm_pp_kernel / gemm_small_kernel<TO, TA=false, TB=false, EPI=BIAS_GELU>",
     "gemm_nn_epi4": "gemm_pp_kernel / gemm_small_kernel<TO, TA=false, TB=false, EPI=SWIGLU>",
     "gemm_nt_epi0": "gemm_pp_kernel / gemm_small_kernel<TO, TA=false, TB=true, EPI=NONE>",
-    "gemm_nt_epi5": "gemm_dl_kernel<TO, TA=false, TB=true, EPI=SWIGLU_BWD>",
+    "gemm_nt_epi5": "gemm_pp_kernel / gemm_small_kernel<TO, TA=false, TB=true, EPI=SWIGLU_BWD>",
     "gemm_nt_epi6": "gemm_pp_kernel / gemm_small_kernel<TO, TA=false, TB=true, EPI=GELU_BWD>",
     "gemm_tt_epi0": "gemm_pp_kernel / gemm_small_kernel<TO, TA=true, TB=true, EPI=NONE> + splitk_reduce_kernel",
     "attn_fwd_full": "attn_fwd_x32<5> (segments >= 512 tokens), attn_fwd_mfma<5, 8, 32, true, 2, 4> (shorter)",
     "attn_bwd_full": "attn_delta_rows_kernel + attn_bwd_prepare_kernel + attn_bwd_dkdv_wide<5> + attn_bwd_dq_wide<5>",
-    "attn_fwd_window": "attn_fwd_mfma<5, 2, 64, false, 2, 4>",
+    "attn_fwd_window": "attn_fwd_mfma<5, 4, 64, false, 1, 5>",
     "attn_bwd_window": "attn_bwd_window_mfma<5>",
 }
+BREAKDOWN_NOTE = ("traced launch by launch, in a step of its own. The timed step issues each block with one call, whose windowed layers rotate inside their "
+                  "attention (attn_fwd_window_rope, attn_bwd_window_mfma<5, true>): of the rope launches here it runs those of the full layers, and its "
+                  "attn_*_window kernels move and compute what these and the other rope launches do together")
 
 
 def optimizer_leg(model, step, iters: int = 5):
@@ -630,6 +634,7 @@ def main() -> None:
         "vision_text_handoff": handoff,
         "input_side": input_side,
         "kernel_breakdown": breakdown,
+        "kernel_breakdown_note": BREAKDOWN_NOTE if breakdown and dtype == torch.bfloat16 else None,
     }
     print(json.dumps(result))
 
