@@ -34,6 +34,7 @@ enum { MVIT_F32 = 0, MVIT_BF16 = 1 };
 enum { MVIT_OK = 0, MVIT_ERR_ARG = -1, MVIT_ERR_LAUNCH = -2, MVIT_ERR_UNSUPPORTED = -3 };
 
 /* 205: without 204's mvit_gemm_wgrads, whose sums were further from the exact ones than those of slices; mvit_gemm_full_round_rows.
+ *      Since 204 mvit_block_fwd without gu may leave q and k in qkv without their rotation.
  * 203: mvit_gemm_args ends with overlapped; mvit_gemm_wgrad_split_k answers for a product that has the GPU to itself.
  * 202: mvit_gemm_args ends with colsum_rows.
  * 201: mvit_gemm_args has row_sums at its end.
