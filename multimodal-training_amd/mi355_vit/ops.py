@@ -397,7 +397,7 @@ def gemm(
     return out
 
 
-@functools.lru_cache(maxsize=None)
+@functools.lru_cache(maxsize=4096)  # ragged batches bring a row count each
 def wgrad_split_k(out_rows: int, out_cols: int, k: int, overlapped: bool = False) -> int:
     """K slices for a GEMM with few output tiles and a long contraction: the weight gradients (contraction over the
     tokens).  The model uses it for those only: on a forward or input-gradient GEMM a slice count chosen from the batch
@@ -407,7 +407,7 @@ def wgrad_split_k(out_rows: int, out_cols: int, k: int, overlapped: bool = False
     return (lib.mvit_gemm_wgrad_split_k_overlapped if overlapped else lib.mvit_gemm_wgrad_split_k)(out_rows, out_cols, k)
 
 
-@functools.lru_cache(maxsize=None)
+@functools.lru_cache(maxsize=4096)  # ragged batches bring a row count each
 def swiglu_bwd_colsum_rows(rows: int, cols: int, k: int) -> int:
     """Rows per row of column sums (256 or 64) with which the bf16 SwiGLU-backward product of this shape is fastest."""
     return _lib.load().mvit_gemm_swiglu_bwd_colsum_rows(rows, cols, k)

@@ -511,6 +511,16 @@ def test_windowed_backward_behind_one_call_refuses_gradients_that_share_memory()
         assert lib.mvit_block_bwd(ctypes.byref(a), None) == -1 and b"dqkv overlaps " + shared.encode() in lib.mvit_last_error()
 
 
+def test_what_is_remembered_by_the_number_of_rows_is_bounded():
+    from mi355_vit import ops
+
+    for fn in (ops.wgrad_split_k, ops.swiglu_bwd_colsum_rows):
+        assert fn.cache_info().maxsize is not None
+    for rows in range(64, 64 + 5000):
+        ops.swiglu_bwd_colsum_rows(rows, 3456, 1280)
+    assert ops.swiglu_bwd_colsum_rows.cache_info().currsize <= 4096 and ops.swiglu_bwd_colsum_rows(12000, 3456, 1280) == 256
+
+
 def test_rows_in_full_rounds_are_named_for_forward_products_and_lone_input_gradients():
     from mi355_vit import _lib
 
