@@ -2323,8 +2323,11 @@ bool strided_rows_overlap(const void* a, int64_t pa, const void* b, int64_t pb, 
 
 }  // namespace
 
+// Not windows of fewer than ten tokens on average: a work-group costs the same for four tokens as for 64, and the two passes hold more of them.  us of a
+// block's forward (kept) and backward, 65,536 rows x 16 heads, two passes / inside: windows of 4 tokens 1,840 / 1,945, 3,673 / 3,857; 6 1,608 / 1,649,
+// 3,110 / 3,140; 8 1,489 / 1,509, 2,844 / 2,839; 10 1,424 / 1,426, 2,672 / 2,640; 12 1,377 / 1,366, 2,542 / 2,475; 14,336 rows, 4 426 / 444, 882 / 898; 8 361 / 356, 719 / 705
 bool mvit_window_rope_takes(const mvit_window_rope& w, int head_dim, int max_seqlen, int dtype) {
-  return dtype == MVIT_BF16 && head_dim == 80 && max_seqlen > 0 && max_seqlen <= 64 && w.n_seg > 0 && w.n_seg <= 65535 && w.nheads > 0 && w.nheads <= 65535 && w.S > 0 &&
+  return w.S >= 10 * (int64_t)w.n_seg && dtype == MVIT_BF16 && head_dim == 80 && max_seqlen > 0 && max_seqlen <= 64 && w.n_seg > 0 && w.n_seg <= 65535 && w.nheads > 0 && w.nheads <= 65535 && w.S > 0 &&
          mvit_aligned16(w.qkv) && mvit_aligned16(w.o) && mvit_aligned16(w.lse) && mvit_aligned16(w.cos) && mvit_aligned16(w.sin);
 }
 int mvit_attn_fwd_window_rope(const mvit_window_rope& w, hipStream_t stream) {
@@ -2334,8 +2337,10 @@ int mvit_attn_fwd_window_rope(const mvit_window_rope& w, hipStream_t stream) {
   p.q = qkv; p.k = qkv + C; p.v = qkv + 2 * C; p.out = w.o; p.lse = w.lse; p.cu = w.cu; p.total = w.S; p.nheads = w.nheads;
   p.q_stride = p.k_stride = p.v_stride = 3 * C; p.o_stride = C; p.scale = w.attn_scale;
   WindowRope r{w.cos, w.sin, w.q_gain, 1, w.keep ? 1 : 0, w.n_seg, w.nheads};
-  // LOOP once q, k and v are more than stays in the memory-side cache (256 MB) between the product that writes them and this
-  const bool loop = w.S * 3 * C * 2 > (160ll << 20);
+  // LOOP once q, k and v are more than stays in the memory-side cache (256 MB) between the product that writes them and this, and windows long
+  // enough for two work-groups to keep a unit's loads coming: us of a block's forward, 65,536 rows x 16 heads, one head / LOOP, kept and not kept:
+  // windows of 16 tokens 1,311 / 1,410, 1,234 / 1,359; 32 1,247 / 1,251, +31; 40 1,250 / 1,233, +4; 48 1,248 / 1,219, -10; 64 1,246 / 1,211, -12
+  const bool loop = w.S * 3 * C * 2 > (160ll << 20) && w.S >= (w.keep ? 40 : 48) * (int64_t)w.n_seg;
   const int most = !loop ? 1 : w.keep ? 2 : 4;
   while (2 * r.heads <= most && w.nheads % (2 * r.heads) == 0) r.heads *= 2;
   r.parts = w.nheads / r.heads;

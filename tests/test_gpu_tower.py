@@ -276,6 +276,31 @@ def test_weight_gradients_of_many_rows_are_summed_in_the_slices_of_their_product
         F.BLOCK_CALLS, ops.OVERLAP_WGRAD = old
 
 
+@pytest.mark.parametrize("rows,window", [(1000, 4), (999, 9), (1000, 10), (1001, 11), (22000, 4), (22003, 16), (22016, 39), (22000, 40), (22008, 47), (22032, 48)])
+def test_windows_give_the_bits_of_two_passes_on_both_sides_of_the_lines(rows, window):
+    """Short windows are rotated by a pass of their own; many rows of long ones take several heads to a work-group."""
+    from mi355_vit import functional as F
+
+    H, C, I, g = 16, 1280, 64, torch.Generator().manual_seed(rows)
+    cu = torch.tensor(list(range(0, rows, window)) + [rows], dtype=torch.int32).to(DEV)
+    angle = torch.randn(rows, 40, generator=g).repeat(1, 2).to(DEV)
+    geo = F.AttnGeometry(cu, window, H, 80, angle.cos().contiguous(), angle.sin().contiguous())
+    r = lambda *shape: (torch.randn(*shape, generator=g) * 0.05).to(torch.bfloat16).to(DEV)  # noqa: E731
+    Ipad = F.padded_inner(I)
+    W = F.BlockWeights(r(1, C) + 1, r(1, C) + 1, r(3 * C, C), r(1, 3 * C), r(C, C), r(1, C), r(2 * Ipad, C), r(1, 2 * Ipad), r(C, Ipad), r(1, C), C, I, Ipad)
+    x, dy, old, got = r(rows, C) * 20, r(rows, C) * 20, F.BLOCK_CALLS, {}
+    try:
+        for F.BLOCK_CALLS in (True, False):
+            y0, saved0 = F._block_forward(x, W, geo, 1e-6, for_backward=False)
+            y, saved = F._block_forward(x, W, geo, 1e-6)
+            kept = [saved[i].clone() for i in (2, 3, 4)]
+            dx, grads = F._block_backward(dy, x, tuple(saved), W, geo, torch.bfloat16)
+            got[F.BLOCK_CALLS] = [y0, saved0[3], saved0[4], y, *kept, dx, *grads]
+    finally:
+        F.BLOCK_CALLS = old
+    assert all(torch.equal(a, b) for a, b in zip(got[True], got[False]))
+
+
 @pytest.mark.parametrize("kind", ["permuted", "named twice", "outside the list"])
 def test_windows_that_rotate_are_taken_once_each_whatever_the_order_of_segments_says(kind):
     """q and k are rotated in place inside the windows' attention: an order that names a window twice must not have it rotated twice."""
