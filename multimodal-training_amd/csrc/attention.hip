@@ -1960,7 +1960,8 @@ __global__ __launch_bounds__(64 * NWAVES) void attn_bwd_dq_mfma(const AttnParams
 // pass B repeats the dK/dV kernel's tile loop on the staged tiles.  HBM traffic: four tiles in, three out.
 // Results are turned in LDS and leave as 16-byte chunks, a row's 160 bytes together: as 8-byte pieces of 32 bytes a row, straight from the accumulators,
 // they took twice the write requests.  us before / now, operands from HBM: 4,096 rows x 16 heads 27.8 / 25.0, 14,336 80 / 68, 25,524 128 / 108, 65,536 307 / 259
-// (4.5 TB/s).
+// (4.5 TB/s).  Waves without rows leave before pass B; while they turned nothing but zeros, short windows were slower than with the pieces: 65,536 rows x 16 heads, pieces /
+// all waves / this, windows of 16 tokens 506 / 515 / 491, of 4 1,592 / 1,710 / 1,541, head_dim 32 190 / 219 / 175, 627 / 738 / 558.
 // ROPE: dQ and dK are turned back by the rotary embedding's angles on their way out (with the roundings of the pass of its own, which read and wrote both
 // once more); dQ waits in LDS for the tables, which are fetched once for both and travel while dK and dV are rounded.  ms per step, pass of its own /
 // inside: 1,024 rows 12.0 / 11.6, 4,096 checkpointed 27.9 / 27.6, 14,336 62.2 / 61.0, 25,524 104.9 / 104.3, 36,864 239.6 / 238.3.
@@ -2093,6 +2094,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_window_mfma(const AttnParams 
     for (int q = 16 * ((L + 15) / 16) + (int)threadIdx.x; q < R; q += 256) lds_delta[q] = 0.f;  // query blocks that were skipped
   }
   __syncthreads();
+  if (wv * 16 >= L) return;  // the waves meet no more
 
   // ---- pass B: dV^T += dO^T P, dK^T += Q^T dS per 16-key block, queries in two tiles of 32
   {
@@ -2105,7 +2107,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_window_mfma(const AttnParams 
       dk[d] = f32x4{0.f, 0.f, 0.f, 0.f};
       dv[d] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    if (!ROPE && wv * 16 < L) leave(lds_v, dq_out, DQ, p.dq_stride);
+    if (!ROPE) leave(lds_v, dq_out, DQ, p.dq_stride);
     if (ROPE) turn_in(lds_v, dq_out);  // stays there until the tables are fetched, once for both
 #pragma unroll 1
     for (int qs = 0; qs < L; qs += 32) {
