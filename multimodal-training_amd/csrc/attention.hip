@@ -2326,8 +2326,8 @@ bool strided_rows_overlap(const void* a, int64_t pa, const void* b, int64_t pb, 
 }  // namespace
 
 // Not windows of fewer than ten tokens on average: a work-group costs the same for four tokens as for 64, and the two passes hold more of them.  us of a
-// block's forward (kept) and backward, 65,536 rows x 16 heads, two passes / inside: windows of 4 tokens 1,840 / 1,945, 3,673 / 3,857; 6 1,608 / 1,649,
-// 3,110 / 3,140; 8 1,489 / 1,509, 2,844 / 2,839; 10 1,424 / 1,426, 2,672 / 2,640; 12 1,377 / 1,366, 2,542 / 2,475; 14,336 rows, 4 426 / 444, 882 / 898; 8 361 / 356, 719 / 705
+// block's forward (kept), 65,536 rows x 16 heads, two passes / inside: windows of 4 tokens 1,840 / 1,945, 6 1,608 / 1,649, 8 1,489 / 1,509, 10 1,424 / 1,426,
+// 12 1,377 / 1,366; 14,336 rows, 4 426 / 444, 8 361 / 356.  The backward goes the same way (65,536 rows, 12 2,451 / 2,349, 16 2,342 / 2,285).
 bool mvit_window_rope_takes(const mvit_window_rope& w, int head_dim, int max_seqlen, int dtype) {
   return w.S >= 10 * (int64_t)w.n_seg && dtype == MVIT_BF16 && head_dim == 80 && max_seqlen > 0 && max_seqlen <= 64 && w.n_seg > 0 && w.n_seg <= 65535 && w.nheads > 0 && w.nheads <= 65535 && w.S > 0 &&
          mvit_aligned16(w.qkv) && mvit_aligned16(w.o) && mvit_aligned16(w.lse) && mvit_aligned16(w.cos) && mvit_aligned16(w.sin);

@@ -1189,8 +1189,7 @@ bool pp_takes(GemmTiledKind kind, int64_t k_chunk, int64_t k_last) {  // at leas
 // of the launch (clock, and operands that the L2s and the memory-side cache no longer hold): a launch of r rounds takes 5 % longer per round beyond the
 // first on 128 x 128 tiles, 15 % on 64-row ones.  us, input gradients of 1280 columns, the mean above -> this: K = 6912 13,312 rows 268 -> 215,
 // 14,336 267 -> 223, 16,384 282 -> 294 (4 % off the best), 18,432 and 27,648 284 and 432 (328 and 540 without the growth); K = 3840 13,312 rows
-// 155 -> 129, 16,384 160 -> 148; 5120 columns, K = 5120 (the merger) 3,584 rows 202 -> 171.  (One launch each; rows_in_full_rounds then cuts some in two: K = 6912,
-// 14,336 rows 194.)  Over 107 sizes from 1,024 to 65,536 rows the
+// 155 -> 129, 16,384 160 -> 148; 5120 columns, K = 5120 (the merger) 3,584 rows 202 -> 171.  (One launch each; rows_in_full_rounds then cuts some in two.)  Over 107 sizes from 1,024 to 65,536 rows the
 // choice is 0.1 % off the fastest tile on average.
 constexpr double PP_STEP_US = 1.15, PP_TILE_US = 7., PP_SWIGLU_TILE_US = 11.;
 struct TileChoice {
@@ -1265,8 +1264,9 @@ TileChoice choose_tile(GemmTiledKind kind, int64_t M, int64_t N, int64_t k_chunk
 // tiles that suit it (0: one launch for all).  14,336 rows are 56 x 5 tiles of 1280 columns, 1.09 rounds of 256 units: a second
 // round for 24 tiles, or 2.2 rounds of 128 x 128 tiles at two thirds of the rate.  255 tiles in one round and 1,280 rows on small
 // tiles are faster than either (forward products of the tower, time alone of the step: 14,336 rows 71.6 -> 69.6 ms, 9,600 51.7 ->
-// 50.2, 4,360 without gradients 8.92 -> 8.61).  Input gradients, us in one launch / head and rest: 14,336 x 1280, K = 6912 219 / 194, K = 3840
-// 130 / 114; 3,584 x 5120, K = 3584, GELU backward 168 / 144; 4,096 x 5120 190 / 170; the model errs at 6,381 x 5120, K = 3584, 166 / 170.  In the backward the second stream fills the last round, see choose_tile.
+// 50.2, 4,360 without gradients 8.92 -> 8.61).  Input gradients, us in one launch / head and rest: 14,336 x 1280, K = 6912 211 / 200, K = 3840
+// 126 / 115; 16,384 x 1280, K = 6912, GELU backward 318 / 260; 3,584 x 5120, K = 3584, GELU backward 166 / 144; 4,096 x 5120, K = 5120 187 / 169.  Over 126 drawn sizes that it cuts
+// (1,340 to 60,000 rows) 10 % less on average and nowhere more than 0.2 % more; 16,384 x 1280, K = 1280, GELU backward 88 / 89.  In the backward the second stream fills the last round, see choose_tile.
 int64_t rows_in_full_rounds(GemmTiledKind kind, int64_t M, int64_t N, int64_t K, int n_cu, bool overlapped) {
   if (!(kind == NN_NONE || kind == NN_BIAS || kind == NN_BIAS_RES || kind == NN_BIAS_GELU || kind == NN_SWIGLU || ((kind == NT_NONE || kind == NT_GELU_BWD) && !overlapped)) || !pp_takes(kind, K, K)) return 0;
   const int64_t tn = (N * (kind == NN_SWIGLU ? 2 : 1) + 255) / 256, rounds = (M + 255) / 256 * tn / n_cu, rows = rounds * n_cu / tn * 256;
