@@ -407,7 +407,8 @@ def test_windowed_block_refuses_the_tensors_that_the_attention_calls_refuse():
 
 
 def test_windowed_block_takes_as_many_windows_and_heads_as_the_two_passes():
-    """65,535 windows, all but one of them empty, of 205 heads: together more threads than one dimension of a grid holds."""
+    """65,535 windows, all but one of them empty, of 205 heads: together more threads than one dimension of a grid holds.  Of so few tokens on
+    average they go as two passes too; inside, windows and heads have a grid dimension each."""
     from mi355_vit import functional as F
 
     H, rows, I = 205, 64, 8
